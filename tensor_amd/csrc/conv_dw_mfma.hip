@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(256) conv_dw3x3_mfma_kernel(const int8_t* __re
                 const v4i res = dw_dequant4(ep, cur[t], si[t], bi[t]);
                 // the second set's channels 4..7: the next Float4 pack is one plane further, in Float8 they follow
                 const unsigned vo_t = (t == 0 || !row_ok) ? v_o : v_o + (EPI == EPI_F32_P4 ? OHW * 16u : 16u);
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u_store, res), rout, (int)vo_t, (int)s_row, 0);
+                store_b128_row(res, rout, vo_t, s_row);
             }
         } else {
             constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
                 for (int t = 0; t < T; ++t) {
                     const v4i res = dw_dequant4(ep, cur[c][t], si[t], bi[t]);
                     const unsigned vo_t = (t == 0 || v_out[c] == DW_OOB) ? v_out[c] : v_out[c] + (EPI == EPI_F32_P4 ? OHW * 16u : 16u);
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u_store, res), rout, (int)vo_t, (int)s_row, 0);
+                    store_b128_row(res, rout, vo_t, s_row);
                 }
             } else {
                 constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;

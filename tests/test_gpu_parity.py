@@ -464,6 +464,22 @@ def test_depthwise5x5_and_wide_padding(hip, oracle, family, s):
                 assert_f32_close(out, want)
 
 
+@pytest.mark.parametrize("k,s,src_f32", [(3, 1, False), (5, 1, False), (3, 2, False), (3, 1, True)])
+def test_depthwise_fp32_result_at_a_full_machine(hip, oracle, k, s, src_f32):
+    """Enough workgroups to keep every store unit busy: a 16-byte row store whose data registers were overwritten by the
+    next row's conversion gave one wrong value in some 50 000 here and none in smaller launches."""
+    rng = np.random.default_rng(70 + k + s)
+    x, wq, ws, bias = _rand_problem(rng, 128, 128, k, 128, 16, 52, 52)
+    if src_f32:
+        x = x.astype(np.float32) / 20
+    want = oracle.conv_layer_forward(x, wq, ws, 20.0, stride=(s, s), pad=(k // 2, k // 2), groups=128, bias=bias, act_type=2,
+                                     act_params=[0.1], int8_out=False)
+    out, kind = run_conv(hip, oracle, x, wq, ws, 20.0, stride=s, pad=k // 2, groups=128, bias=bias, act=2, act_p0=0.1,
+                         out_kind=capi.OUT_F32)
+    assert kind == 2
+    assert_f32_close(out, want)
+
+
 @pytest.mark.parametrize("C,K,k,s,p,g,N,H,W,kind", [
     (64, 96, 3, 1, 1, 1, 2, 14, 16, 3),     # 3x3 LDS-halo kernel
     (80, 72, 1, 1, 0, 1, 2, 13, 11, 1),     # 1x1 implicit GEMM
