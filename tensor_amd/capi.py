@@ -1,12 +1,15 @@
 """ctypes binding of include/otter_hip_int8.h. Fails loudly when the library or the GPU is missing:
 there is no CPU fallback anywhere in this package."""
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 import numpy as np
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libotter_hip_int8.so")
+BINDING_PATH = os.path.join(HERE, "lib", "_otter_binding.so")
 
 # otter_hip_layout
 F32, F32_P4, F32_P8, I8, I8_P8, I32, I32_P4, I32_P8 = range(8)
@@ -88,6 +91,18 @@ def load_cdll():
     return C.CDLL(LIB_PATH)
 
 
+def load_binding():
+    """The native per-call path (tensor_amd/binding): allocation, stream and C ABI call of one layer in one native call."""
+    if not os.path.exists(BINDING_PATH):
+        raise OSError("%s is not built: run `python -c 'import __graft_entry__ as g; g.build()'` "
+                      "(tensor_amd/binding/build.sh)" % BINDING_PATH)
+    loader = importlib.machinery.ExtensionFileLoader("_otter_binding", BINDING_PATH)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_otter_binding", loader))
+    loader.exec_module(mod)
+    mod.set_error(HipError)
+    return mod
+
+
 class Library:
     """The GPU library on cuda:0. Tensors are torch CUDA tensors holding the reference's packed storage."""
 
@@ -103,6 +118,7 @@ class Library:
         L.otter_hip_conv_block_workspace_bytes.restype = C.c_size_t
         L.otter_hip_conv_avgpool_workspace_bytes.restype = C.c_size_t
         self.device = torch.device("cuda", device)
+        self.native, self.device_index = load_binding(), device
         self._check(L.otter_hip_init(C.c_int(device)))
 
     # -- plumbing -------------------------------------------------------------------------------------
@@ -111,7 +127,7 @@ class Library:
             raise HipError(rc, self.lib.otter_hip_last_error().decode(errors="replace"))
 
     def stream(self):
-        return C.c_void_p(self.torch.cuda.current_stream().cuda_stream)
+        return C.c_void_p(self.native.current_stream())
 
     def to_device(self, a):
         return self.torch.from_numpy(np.ascontiguousarray(a)).to(self.device)
@@ -264,42 +280,15 @@ class Library:
 
     def conv_chain(self, convs, x, n, h, w, out=None, workspace=None):
         """otter_hip_conv_chain_forward: x (int8 Byte8) through the layers `convs`, intermediate blobs in `workspace`."""
-        hs = (C.c_void_p * len(convs))(*[c.h for c in convs])
-        ws_bytes = self.lib.otter_hip_conv_chain_workspace_bytes(hs, len(convs), n, h, w)
-        if ws_bytes and workspace is None:
-            workspace = self.empty(ws_bytes, np.int8)
-        oh, ow = h, w
-        for c in convs:
-            oh, ow = c.out_hw(oh, ow)
-        if out is None:
-            out = self.empty(n * convs[-1].K * oh * ow, np.int8)
-        ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0  # what the buffer really holds
-        self._check(self.lib.otter_hip_conv_chain_forward(hs, len(convs), self.ptr(x), n, h, w, self.ptr(out),
-                                                          self.ptr(workspace) if workspace is not None else None,
-                                                          C.c_size_t(ws_bytes), self.stream()))
-        return out
+        return self.native.conv_chain([c._hp for c in convs], convs[-1].K, x, n, h, w, out, workspace, self.device_index)
 
     def conv_block(self, expand, dw, project, x, n, h, w, residual=None, q_scale=None, q_round_mode=ROUND_SSE, out=None,
                    q=None, workspace=None):
         """otter_hip_conv_block_forward: x (int8 Byte8) through expand -> depthwise -> project (+ residual), and with
         q_scale the Byte8 quantization of the result. Returns (out, q or None)."""
-        oh, ow = dw.out_hw(*expand.out_hw(h, w))
-        oh, ow = project.out_hw(oh, ow)
-        f32 = project.out_kind == OUT_F32
-        out_layout = F32_P4 if f32 else I8_P8
-        if out is None:
-            out = self.empty(n * project.K * oh * ow, np.float32 if f32 else np.int8)
-        if q is None and q_scale is not None:
-            q = self.empty(n * project.K * oh * ow, np.int8)
-        ws_bytes = self.lib.otter_hip_conv_block_workspace_bytes(expand.h, dw.h, project.h, n, h, w)
-        if ws_bytes and workspace is None:
-            workspace = self.empty(ws_bytes, np.int8)
-        ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0  # what the buffer really holds
-        self._check(self.lib.otter_hip_conv_block_forward(
-            expand.h, dw.h, project.h, self.ptr(x), n, h, w, self.ptr(residual) if residual is not None else None,
-            self.ptr(out), out_layout, self.ptr(q) if q is not None else None, C.c_float(q_scale or 0.0), q_round_mode,
-            self.ptr(workspace) if workspace is not None else None, C.c_size_t(ws_bytes), self.stream()))
-        return out, q
+        out_layout = F32_P4 if project.out_kind == OUT_F32 else I8_P8
+        return self.native.conv_block(expand._hp, dw._hp, project._hp, project.K, out_layout, x, n, h, w, residual, q_scale,
+                                      q_round_mode, out, q, workspace, self.device_index)
 
     def conv_block_set_always(self, on):
         """otter_hip_conv_block_set_always: returns the previous setting."""
@@ -364,6 +353,7 @@ class Conv:
             b.ctypes.data_as(f32p) if b is not None else None, C.c_float(in_scale),
             so.ctypes.data_as(f32p) if so is not None else None, C.c_int(0 if so is None else so.size),
             C.byref(self.h)))
+        self._hp = self.h.value  # the handle as the native call path takes it
 
     def out_hw(self, h, w):
         oh, ow = C.c_int(), C.c_int()
@@ -383,18 +373,8 @@ class Conv:
         self.L._check(self.L.lib.otter_hip_conv_block_set_plan(self.h, rows_per_band, slice_channels, split))
 
     def forward(self, x, in_layout, n, h, w, out_layout=None, out=None, workspace=None):
-        out_layout = self.default_out_layout() if out_layout is None else out_layout
-        oh, ow = self.out_hw(h, w)
-        if out is None:
-            out = self.L.empty(n * self.K * oh * ow, layout_dtype(out_layout))
-        ws_bytes = self.L.lib.otter_hip_conv_workspace_bytes(self.h, in_layout, n, h, w)
-        if ws_bytes and workspace is None:
-            workspace = self.L.empty(ws_bytes, np.int8)
-        ws_bytes = workspace.numel() * workspace.element_size() if workspace is not None else 0  # what the buffer really holds
-        self.L._check(self.L.lib.otter_hip_conv_forward(
-            self.h, self.L.ptr(x), in_layout, n, h, w, self.L.ptr(out), out_layout,
-            self.L.ptr(workspace) if workspace is not None else None, C.c_size_t(ws_bytes), self.L.stream()))
-        return out
+        return self.L.native.conv_forward(self._hp, self.K, x, in_layout, n, h, w, out_layout, out, workspace,
+                                          self.L.device_index)
 
     def avgpool_launches(self, in_layout, n, h, w):
         r = self.L.lib.otter_hip_conv_avgpool_launches(self.h, in_layout, n, h, w)
@@ -453,7 +433,7 @@ class Conv:
     def close(self):
         if self.h:
             self.L.lib.otter_hip_conv_destroy(self.h)
-            self.h = None
+            self.h = self._hp = None
 
     def __del__(self):
         try:
