@@ -65,7 +65,8 @@ class HipError(RuntimeError):
 
 EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otter_hip_device_info",
            "otter_hip_shader_clock_mhz", "otter_hip_malloc",
-           "otter_hip_free", "otter_hip_memcpy_h2d", "otter_hip_memcpy_d2h", "otter_hip_stream_create",
+           "otter_hip_free", "otter_hip_memcpy_h2d", "otter_hip_memcpy_d2h", "otter_hip_upload",
+           "otter_hip_download", "otter_hip_host_malloc", "otter_hip_host_free", "otter_hip_copy", "otter_hip_stream_create",
            "otter_hip_stream_destroy", "otter_hip_stream_synchronize", "otter_hip_conv_create",
            "otter_hip_conv_destroy", "otter_hip_conv_output_shape", "otter_hip_conv_default_out_layout",
            "otter_hip_conv_workspace_bytes", "otter_hip_conv_forward", "otter_hip_conv_kernel_kind",

@@ -178,6 +178,24 @@ int otter_hip_free(void* ptr) {
     return OTTER_HIP_OK;
 }
 
+int otter_hip_host_malloc(void** ptr, size_t bytes) {
+    if (!ptr) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_host_malloc: null");
+    OHIP_CHECK(hipHostMalloc(ptr, bytes ? bytes : 1, hipHostMallocDefault));
+    return OTTER_HIP_OK;
+}
+
+int otter_hip_host_free(void* ptr) {
+    if (ptr) OHIP_CHECK(hipHostFree(ptr));
+    return OTTER_HIP_OK;
+}
+
+int otter_hip_copy(void* dst, const void* src, size_t bytes, void* stream) {
+    if (bytes && (!dst || !src || (((uintptr_t)dst | (uintptr_t)src) & 15)))
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_copy: null or not 16-byte aligned");
+    if (bytes) OHIP_CHECK(run_copy_bytes(src, dst, bytes, (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
 int otter_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream) {
     OHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, (hipStream_t)stream));
     return OTTER_HIP_OK;
@@ -185,6 +203,132 @@ int otter_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream)
 
 int otter_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream) {
     OHIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
+// ---- pinned staging ------------------------------------------------------------------------------------------
+// A copy between pageable host memory and the device goes through the driver's own staging and costs 21-26 us for 4 to
+// 256 KB including the wait (and 2.2 ms for 38 MB down); through a pinned buffer the same copies take 11-13 us (0.7 ms).
+// A buffer is 1 MiB: a chunk's host copy (10-30 us) then covers the cost of enqueueing it, and the transfer of one chunk
+// runs under the host copy of the next.
+}  // extern "C"
+
+namespace {
+
+struct Staging {
+    char* host = nullptr;
+    hipEvent_t busy = nullptr;  // recorded behind the last copy that uses the buffer
+    bool pending = false;
+};
+constexpr size_t kStagingBytes = 1u << 20;
+constexpr int kStagingMax = 16;
+std::mutex g_staging_mutex;
+std::vector<Staging> g_staging_free;  // (of all devices: pinned memory is visible to every GPU, the events are per process)
+int g_staging_made = 0;
+
+// a buffer nobody else holds; its last copy may still be on its way when `pending`
+hipError_t staging_get(Staging* out) {
+    {
+        std::lock_guard<std::mutex> lock(g_staging_mutex);
+        // the buffer used last if its copy is over (it is in the caches), else the oldest
+        for (size_t i : {g_staging_free.size() - 1, (size_t)0}) {
+            if (g_staging_free.empty()) break;
+            Staging& s = g_staging_free[i];
+            if (g_staging_made < kStagingMax && s.pending && hipEventQuery(s.busy) != hipSuccess) continue;
+            *out = s;
+            g_staging_free.erase(g_staging_free.begin() + i);
+            return hipSuccess;
+        }
+        (void)hipGetLastError();  // (hipErrorNotReady of the query)
+        ++g_staging_made;         // beyond the bound only while as many threads copy at once; such a buffer is not kept
+    }
+    *out = Staging{};
+    hipError_t e = hipHostMalloc((void**)&out->host, kStagingBytes, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&out->busy, hipEventDisableTiming);
+    if (e != hipSuccess) {
+        if (out->host) (void)hipHostFree(out->host);
+        std::lock_guard<std::mutex> lock(g_staging_mutex);
+        --g_staging_made;
+    }
+    return e;
+}
+
+hipError_t staging_wait(Staging& s) {
+    if (!s.pending) return hipSuccess;
+    s.pending = false;
+    return hipEventSynchronize(s.busy);
+}
+
+void staging_put(Staging& s) {
+    if (!s.host) return;
+    {
+        std::lock_guard<std::mutex> lock(g_staging_mutex);
+        if (g_staging_made <= kStagingMax) {
+            g_staging_free.push_back(s);
+            return;
+        }
+        --g_staging_made;
+    }
+    (void)staging_wait(s);
+    (void)hipEventDestroy(s.busy);
+    (void)hipHostFree(s.host);
+}
+
+}  // namespace
+
+extern "C" {
+
+int otter_hip_upload(void* dst, const void* src, size_t bytes, void* stream_) {
+    if (bytes && (!dst || !src)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_upload: null");
+    hipStream_t stream = (hipStream_t)stream_;
+    for (size_t at = 0; at < bytes; at += kStagingBytes) {
+        const size_t n = bytes - at < kStagingBytes ? bytes - at : kStagingBytes;
+        Staging s;
+        hipError_t e = staging_get(&s);
+        if (e == hipSuccess) e = staging_wait(s);
+        if (e == hipSuccess) {
+            std::memcpy(s.host, (const char*)src + at, n);
+            e = hipMemcpyAsync((char*)dst + at, s.host, n, hipMemcpyHostToDevice, stream);
+            s.pending = e == hipSuccess;
+            if (e == hipSuccess) e = hipEventRecord(s.busy, stream);
+        }
+        staging_put(s);
+        OHIP_CHECK(e);
+    }
+    return OTTER_HIP_OK;
+}
+
+int otter_hip_download(void* dst, const void* src, size_t bytes, void* stream_) {
+    if (bytes && (!dst || !src)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_download: null");
+    hipStream_t stream = (hipStream_t)stream_;
+    Staging s[2];
+    hipError_t e = hipSuccess;
+    const size_t chunks = (bytes + kStagingBytes - 1) / kStagingBytes;
+    for (size_t i = 0; i < 2 && i < chunks && e == hipSuccess; ++i) {
+        e = staging_get(&s[i]);
+        if (e == hipSuccess) e = staging_wait(s[i]);
+    }
+    // chunk c travels while chunk c - 1 is copied out
+    auto length = [&](size_t c) { return c + 1 < chunks ? kStagingBytes : bytes - c * kStagingBytes; };
+    for (size_t c = 0; c <= chunks && e == hipSuccess; ++c) {
+        if (c < chunks) {
+            Staging& b = s[c & 1];
+            e = hipMemcpyAsync(b.host, (const char*)src + c * kStagingBytes, length(c), hipMemcpyDeviceToHost, stream);
+            if (e == hipSuccess && chunks > 1) {
+                e = hipEventRecord(b.busy, stream);
+                b.pending = e == hipSuccess;
+            }
+        }
+        if (c > 0 && e == hipSuccess) {
+            Staging& b = s[(c - 1) & 1];
+            e = chunks > 1 ? staging_wait(b) : hipStreamSynchronize(stream);
+            if (e == hipSuccess) std::memcpy((char*)dst + (c - 1) * kStagingBytes, b.host, length(c - 1));
+        }
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(stream);  // nothing may still write into a buffer that goes back
+    staging_put(s[0]);
+    staging_put(s[1]);
+    OHIP_CHECK(e);
     return OTTER_HIP_OK;
 }
 

@@ -107,6 +107,22 @@ __global__ void __launch_bounds__(256) inner_product_kernel(const float* __restr
     if (q == 0 && o < OUT && n < N) y[(size_t)n * OUT + o] = s + (b ? b[o] : 0.f);
 }
 
+// 16 bytes per thread and trip. For an image in pinned host memory the link is the bound (600 KB: 12 us); 256 workgroups
+// keep enough reads of it in flight.
+__global__ void __launch_bounds__(256) copy_bytes_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n16,
+                                                         size_t bytes) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) dst[i] = src[i];
+    if (blockIdx.x == 0 && threadIdx.x < bytes - n16 * 16)
+        reinterpret_cast<char*>(dst)[n16 * 16 + threadIdx.x] = reinterpret_cast<const char*>(src)[n16 * 16 + threadIdx.x];
+}
+
+hipError_t run_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream) {
+    const size_t n16 = bytes / 16;
+    const unsigned blocks = (unsigned)(n16 < 256 * 256 ? (n16 + 255) / 256 : 256);
+    hipLaunchKernelGGL(copy_bytes_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, stream, (const uint4*)src, (uint4*)dst, n16, bytes);
+    return hipGetLastError();
+}
+
 hipError_t run_eltwise_add(const float* a, const float* b, float* out, size_t n, hipStream_t stream) {
     if (n == 0) return hipSuccess;
     const size_t n4 = n / 4;

@@ -2,6 +2,7 @@
 // benchmark drive the Net through it). Options are "key=value;key=value" strings with the reference's own keys.
 #include <chrono>
 #include <cstring>
+#include <memory>
 #include <string>
 
 #include "../../include/otter_hip_int8.h"
@@ -29,6 +30,18 @@ LayerOption parse_options(const char* opts) {
         pos = e + 1;
     }
     return lo;
+}
+// a pass's result, unpacked: what it is, and its values in host memory where the caller has room for them
+void fetched(const Tensor& top, void* out, size_t capacity, int* dtype, int64_t* shape4) {
+    const Tensor f = top.dim() == 4 && top.elempack() != 1 ? top.packing(1) : top;
+    const ScalarType b = base_of(f.scalar_type());
+    if (dtype) *dtype = b == ScalarType::Float ? 0 : (b == ScalarType::Byte ? 1 : 2);
+    if (shape4)
+        for (int i = 0; i < 4; ++i) shape4[i] = i < f.dim() ? f.size(i) : 1;
+    if (out) {
+        OTTER_CHECK(f.nbytes() <= capacity, "output buffer too small");
+        f.download(out);
+    }
 }
 Tensor f32_vec(const float* p, int n) { return Tensor::from_blob(p, {n}, ScalarType::Float); }
 }  // namespace
@@ -147,8 +160,8 @@ int otter_host_net_run(void* net, const char* in_name, const void* x, int x_is_i
                        int repeat, double* seconds) {
     try {
         Net* N = static_cast<Net*>(net);
-        Tensor in = Tensor::from_blob(x, {n, c, h, w}, x_is_int8 ? ScalarType::Byte : ScalarType::Float);
-        in.device_ptr();  // resident before the timed region
+        // resident before the timed region
+        const Tensor in = Tensor::from_host(x, {n, c, h, w}, x_is_int8 ? ScalarType::Byte : ScalarType::Float);
         Tensor feat;
         auto pass = [&]() -> int {
             Extractor ex = N->create_extractor();
@@ -165,15 +178,7 @@ int otter_host_net_run(void* net, const char* in_name, const void* x, int x_is_i
             otter_hip_stream_synchronize(nullptr);
             if (seconds) *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() / repeat;
         }
-        if (feat.dim() == 4 && feat.elempack() != 1) feat = feat.packing(1);
-        const ScalarType b = base_of(feat.scalar_type());
-        if (out_dtype) *out_dtype = b == ScalarType::Float ? 0 : (b == ScalarType::Byte ? 1 : 2);
-        if (out_shape4)
-            for (int i = 0; i < 4; ++i) out_shape4[i] = i < feat.dim() ? feat.size(i) : 1;
-        if (out) {
-            if (feat.nbytes() > out_capacity_bytes) return fail("output buffer too small");
-            std::memcpy(out, feat.data_ptr(), feat.nbytes());
-        }
+        fetched(feat, out, out_capacity_bytes, out_dtype, out_shape4);
         return 0;
     } catch (const std::exception& e) {
         return fail(e.what());
@@ -196,8 +201,7 @@ void* otter_host_session_create(void* net, const char* in_name, const void* x, i
         s->net = static_cast<Net*>(net);
         s->in_name = in_name;
         s->out_name = out_name;
-        s->in = Tensor::from_blob(x, {n, c, h, w}, x_is_int8 ? ScalarType::Byte : ScalarType::Float);
-        s->in.device_ptr();
+        s->in = Tensor::from_host(x, {n, c, h, w}, x_is_int8 ? ScalarType::Byte : ScalarType::Float);
         return s;
     } catch (const std::exception& e) {
         g_err = e.what();
@@ -229,10 +233,8 @@ long otter_host_session_fetch(void* session, void* out, size_t capacity) {
     try {
         auto* s = static_cast<otter_host_session*>(session);
         if (!s->out.defined()) return fail("no pass has run");
-        Tensor f = (s->out.dim() == 4 && s->out.elempack() != 1) ? s->out.packing(1) : s->out;
-        if (f.nbytes() > capacity) return fail("output buffer too small");
-        std::memcpy(out, f.data_ptr(), f.nbytes());
-        return (long)f.nbytes();
+        fetched(s->out, out, capacity, nullptr, nullptr);
+        return (long)s->out.nbytes();
     } catch (const std::exception& e) {
         return fail(e.what());
     }
@@ -314,25 +316,21 @@ int otter_host_net_eval(void* net, int n_inputs, const char* const* in_names, co
                         size_t out_capacity_bytes, int* out_dtype, int64_t* out_shape4) {
     try {
         Net* N = static_cast<Net*>(net);
+        std::vector<std::unique_ptr<HostInput>> ins;
         Extractor ex = N->create_extractor();
         ex.set_lightmode(false);
         for (int i = 0; i < n_inputs; ++i) {
             const int64_t* s = shapes4 + 4 * i;
-            Tensor in = Tensor::from_blob(in_ptrs[i], {s[0], s[1], s[2], s[3]}, in_is_int8[i] ? ScalarType::Byte : ScalarType::Float);
-            if (ex.input(in_names[i], in)) return fail(std::string("unknown blob ") + in_names[i]);
+            ins.push_back(std::make_unique<HostInput>(in_ptrs[i], std::vector<int64_t>(s, s + 4),
+                                                      in_is_int8[i] ? ScalarType::Byte : ScalarType::Float));
+            if (ex.input(in_names[i], ins.back()->blob)) return fail(std::string("unknown blob ") + in_names[i]);
         }
         Tensor feat;
         const int rc = ex.extract(out_name, feat, 0);
         if (rc) return fail("forward failed with code " + std::to_string(rc) + ": " + otter_hip_last_error());
-        if (feat.dim() == 4 && feat.elempack() != 1) feat = feat.packing(1);
-        const ScalarType b = base_of(feat.scalar_type());
-        if (out_dtype) *out_dtype = b == ScalarType::Float ? 0 : (b == ScalarType::Byte ? 1 : 2);
-        if (out_shape4)
-            for (int i = 0; i < 4; ++i) out_shape4[i] = i < feat.dim() ? feat.size(i) : 1;
-        if (out) {
-            if (feat.nbytes() > out_capacity_bytes) return fail("output buffer too small");
-            std::memcpy(out, feat.data_ptr(), feat.nbytes());
-        }
+        fetched(feat, out, out_capacity_bytes, out_dtype, out_shape4);
+        if (out)  // the download has waited for the pass
+            for (auto& in : ins) in->pass_done();
         return 0;
     } catch (const std::exception& e) {
         return fail(e.what());

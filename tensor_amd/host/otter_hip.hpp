@@ -46,6 +46,7 @@ public:
     static Tensor empty(const std::vector<int64_t>& sizes, ScalarType dtype);        // host storage
     static Tensor empty_device(const std::vector<int64_t>& sizes, ScalarType dtype); // device storage only
     static Tensor from_blob(const void* data, const std::vector<int64_t>& sizes, ScalarType dtype);  // copies
+    static Tensor from_host(const void* data, const std::vector<int64_t>& sizes, ScalarType dtype);  // copies to the device
 
     bool defined() const { return (bool)st_; }
     int64_t dim() const { return (int64_t)sizes_.size(); }
@@ -69,6 +70,7 @@ public:
     const T* data_ptr() const { return static_cast<const T*>(data_ptr()); }
 
     void* device_ptr() const;       // device pointer; uploads first if the fresh copy is on the host
+    void download(void* dst) const; // copies the tensor to host memory, with no host copy of its own
     bool on_device() const;         // a valid device copy exists
     void mark_device_written();     // the device copy is now the fresh one
 
@@ -82,6 +84,23 @@ private:
     std::shared_ptr<Storage> st_;
     std::vector<int64_t> sizes_;
     ScalarType dtype_ = ScalarType::Undefined;
+};
+
+// A device blob made from host data for one pass, through pinned memory that is free for the next pass when this object
+// goes. The caller says so when it has waited for the pass (a download did); otherwise the destructor waits.
+class HostInput {
+public:
+    HostInput(const void* data, const std::vector<int64_t>& sizes, ScalarType dtype);
+    ~HostInput();
+    HostInput(const HostInput&) = delete;
+    HostInput& operator=(const HostInput&) = delete;
+    void pass_done() { done_ = true; }
+    Tensor blob;
+
+private:
+    size_t bytes_;
+    void* buffer_ = nullptr;
+    bool done_ = false;
 };
 
 // Tensor/NetOption.hpp

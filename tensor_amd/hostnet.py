@@ -56,6 +56,7 @@ class Net:
 
     def __init__(self, use_packing_layout=True, lightmode=True):
         self.lib = load_cdll()
+        self._eval_args = {}
         self.h = C.c_void_p(self.lib.otter_host_net_create(int(use_packing_layout), int(lightmode)))
         if not self.h:
             raise HostError(self.lib.otter_host_last_error().decode())
@@ -143,21 +144,28 @@ class Net:
     def eval(self, inputs, out_name):
         """One pass with the blobs of `inputs` (name -> NCHW fp32 / int8 array) set beforehand; returns `out_name`
         unpacked (Extractor::input + Extractor::extract(name, type 0))."""
-        names = [k.encode() for k in inputs]
         arrs = [np.ascontiguousarray(v) for v in inputs.values()]
-        n = len(arrs)
-        c_names = (C.c_char_p * n)(*names)
+        key = (out_name,) + tuple((k, a.shape, a.dtype.char) for k, a in zip(inputs, arrs))
+        args = self._eval_args.get(key)
+        if args is None:  # everything but the addresses stays the same from call to call
+            n = len(arrs)
+            args = (n, (C.c_char_p * n)(*[k.encode() for k in inputs]), (C.c_int * n)(*[int(a.dtype == np.int8) for a in arrs]),
+                    (C.c_int64 * (4 * n))(*[d for a in arrs for d in a.shape]), out_name.encode())
+        n, c_names, c_i8, c_shapes, c_out = args[:5]
         c_ptrs = (C.c_void_p * n)(*[a.ctypes.data for a in arrs])
-        c_i8 = (C.c_int * n)(*[int(a.dtype == np.int8) for a in arrs])
-        c_shapes = (C.c_int64 * (4 * n))(*[d for a in arrs for d in a.shape])
         dtype, shape = C.c_int(), (C.c_int64 * 4)()
-        cap = 1 << 28
-        buf = np.empty(cap, np.uint8)
-        self._check(self.lib.otter_host_net_eval(self.h, n, c_names, c_ptrs, c_i8, c_shapes, out_name.encode(),
-                                                 buf.ctypes.data_as(C.c_void_p), C.c_size_t(cap), C.byref(dtype), shape))
-        np_dt = [np.float32, np.int8, np.int32][dtype.value]
-        count = int(np.prod(tuple(shape)))
-        return buf[:count * np.dtype(np_dt).itemsize].view(np_dt).reshape(tuple(shape)).copy()
+        # the result of a call seen before has the size it had then; else room for any blob, of which only the part that is
+        # written is ever touched
+        out = np.empty(args[5], args[6]) if len(args) > 5 else np.empty(1 << 28, np.uint8)
+        self._check(self.lib.otter_host_net_eval(self.h, n, c_names, c_ptrs, c_i8, c_shapes, c_out,
+                                                 C.c_void_p(out.ctypes.data), C.c_size_t(out.nbytes), C.byref(dtype), shape))
+        got, np_dt = tuple(shape), [np.float32, np.int8, np.int32][dtype.value]
+        if len(args) > 5 and got == args[5] and np_dt is args[6]:
+            return out
+        if len(args) == 5 and len(self._eval_args) < 64:
+            self._eval_args[key] = args + (got, np_dt)
+        count = int(np.prod(got))
+        return out.reshape(-1).view(np.uint8)[:count * np.dtype(np_dt).itemsize].view(np_dt).reshape(got).copy()
 
     def close(self):
         if self.h:
