@@ -282,8 +282,9 @@ int otter_hip_conv_block_set_plan(otter_hip_conv_t* expand, int rows_per_band, i
  * GEMM, 2 depthwise, 3 MFMA 3x3 halo kernel, 4 few-channel 3x3 kernel (an image stem read straight from the unpacked
  * blob), 5 streamed 1x1 kernel (int8 -> int8 over at most 64 input channels), 6 pointwise layer on an fp32 Float8 blob
  * of 64..256 channels, quantize and convolution in one launch that reads the blob once. (Other pointwise and depthwise 3x3
- * layers on an fp32 Float8 blob also quantize inside the convolution's launch; they report 1 and 2.) For tests and
- * profiling. */
+ * layers on an fp32 Float8 blob also quantize inside the convolution's launch; they report 1 and 2. Families 1, 3 and 6
+ * have a second kernel for layers that it is measured faster on, mostly those that leave the machine idle; the family
+ * stays what is reported.) For tests and profiling. */
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w,
                                int out_layout);
 
@@ -300,7 +301,9 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * (2 or 4) and the slices the output channels are cut into (0 = automatic for either). tm == -6: quantize an fp32 blob
  * in a launch of its own (the two launches of the reference's order) where the convolution's launch would do it.
  * tm == -7 on a pointwise layer: kernel 6 above wherever it can run, tn = groups | pairs << 3 forcing the 16-pixel
- * groups a wave owns (1 or 2) and the pairs of 16 output channels per LDS round (0 = automatic for either). */
+ * groups a wave owns (1 or 2) and the pairs of 16 output channels per LDS round (0 = automatic for either).
+ * tm == -8: the launch of families 1 and 3 that reads both operands straight from memory and deals the reduction to the waves
+ * of a workgroup, tn = 0..4 its tile. */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 
 /* Test hook with no counterpart in the reference, host arithmetic only (no GPU needed): the launch plan of the 3x3

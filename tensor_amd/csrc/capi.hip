@@ -93,6 +93,7 @@ struct otter_hip_conv {
     bool depthwise = false;
     int8_t* w_raw = nullptr;     // [K, C/g, kh, kw]           (direct kernel)
     int8_t* w_igemm = nullptr;   // MFMA lane order            (groups == 1, C % 8 == 0)
+    int8_t* w_tap = nullptr;     // the same in the order of conv_tap.hip; w_igemm itself where the two agree
     int8_t* w_stem = nullptr;    // MFMA lane order of the few-channel 3x3 kernel (C <= 5, K <= 64)
     int32_t* w_dw = nullptr;     // dot4 weight words          (depthwise, C % 8 == 0)
     int8_t* w_dw_mfma = nullptr; // block-diagonal MFMA operands (depthwise 3x3, C % 8 == 0)
@@ -356,6 +357,7 @@ int otter_hip_stream_synchronize(void* stream) {
 int otter_hip_conv_destroy(otter_hip_conv_t* h) {
     if (!h) return OTTER_HIP_OK;
     (void)hipFree(h->w_raw);
+    if (h->w_tap != h->w_igemm) (void)hipFree(h->w_tap);
     (void)hipFree(h->w_igemm);
     (void)hipFree(h->w_stem);
     (void)hipFree(h->w_dw);
@@ -489,6 +491,15 @@ int otter_hip_conv_create(const otter_hip_conv_desc* desc, const int8_t* weight,
                 if ((rc = upload<int8_t>(&h->w_stem, wsv.data(), wsv.size(), wsv.size(), 0))) break;
             }
         }
+        if (h->w_igemm && !h->c_pad && maxk <= 31) {
+            if (tap_weights_are_igemm(C / g, d.kernel_h, d.kernel_w, g > 1 ? igemm_tap_pack(C / g, d.kernel_h, d.kernel_w) : 1)) {
+                h->w_tap = h->w_igemm;
+            } else {
+                std::vector<int8_t> wt(tap_grouped_weight_bytes(K, C, g, d.kernel_h, d.kernel_w));
+                tap_pack_weights_grouped(weight, K, C, g, d.kernel_h, d.kernel_w, wt.data());
+                if ((rc = upload<int8_t>(&h->w_tap, wt.data(), wt.size(), wt.size(), 0))) break;
+            }
+        }
     } while (0);
     if (rc != OTTER_HIP_OK) {
         std::string keep = g_last_error;
@@ -618,6 +629,24 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
     return h->force_tm == -7 || (g.C >= 64 && g.K >= 128);
 }
 
+// The tile of the kernel whose workgroups deal the reduction to their waves (conv_tap.hip), for a layer that the kernels of
+// `family` (1 or 3; with an fp32 blob the launches of families 1 and 6) would run otherwise, or -1 where those are faster by
+// the two cost models. They have to be slower by 15 %: below that the models' errors decide. An fp32 blob may also be
+// quantized by a pass of its own, 2 us and 0.5 us per million values, in front of whichever int8 kernel is faster.
+// set_tile(-8, tile) forces it.
+static int tap_config(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, bool f32in, int family) {
+    if (!h->w_tap || (h->force_tm != 0 && h->force_tm != -8) || !conv_tap_supported(g, ep, f32in)) return -1;
+    if (h->force_tm == -8) return h->force_tn;
+    if (family != 1 && family != 3 && !(f32in && family == 6)) return -1;
+    const int ob = layout_elem_bytes(ep.out_layout);
+    int config, config_i8;
+    const float cost = conv_tap_cost(g, f32in, &config);
+    const float other = f32in && g.kh * g.kw > 1 ? 2.f + 0.5e-6f * (float)g.N * g.C * g.H * g.W +
+                                                       fminf(conv_tap_cost(g, false, &config_i8), conv_family_cost(g, family, false, ob))
+                                                 : conv_family_cost(g, family, f32in, ob);
+    return cost < 0.85f * other ? config : -1;
+}
+
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w, int out_layout) {
     if (!h || !valid_layout(in_layout)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_kernel_kind: bad argument");
     int l = in_layout;
@@ -700,6 +729,23 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
         return quantize_twin();
     }
 
+    auto fuse = [&](Epilogue& ep) {  // the sum and the twin by the convolution itself
+        ep.twin = twin, ep.twin_scale = twin_scale;
+        ep.twin_half = twin_round == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+        ep.residual = residual;
+        twin = nullptr, residual = nullptr;
+    };
+    if (in_layout == OTTER_HIP_F32_P8 && h->w_tap && !h->c_pad) {
+        Epilogue ep = make_epilogue(h, out_layout);
+        const int kind = use_pw_f32in(h, in_layout, g, ep) ? 6 : use_igemm_f32in(h, in_layout, g, ep) ? 1 : pick_kernel(h, OTTER_HIP_I8_P8, g, ep);
+        const int config = tap_config(h, g, ep, true, kind);
+        if (config >= 0) {
+            if ((twin || residual) && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) fuse(ep);
+            OHIP_CHECK(run_conv_tap(in, true, h->w_tap, out, g, ep, config, h->in_scale, d.in_round_mode, stream));
+            return quantize_twin();
+        }
+    }
+
     // A pointwise layer on an fp32 Float8 blob: quantize_to_int8 inside the convolution's launch.
     {
         Epilogue ep = make_epilogue(h, out_layout);
@@ -746,6 +792,14 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
 
     Epilogue ep = make_epilogue(h, out_layout);
     const int kind = pick_kernel(h, q_layout, g, ep);
+    if (q_layout == OTTER_HIP_I8_P8 && !h->c_pad && (kind == 1 || kind == 3 || h->force_tm == -8)) {
+        const int config = tap_config(h, g, ep, false, kind);
+        if (config >= 0) {
+            if ((twin || residual) && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) fuse(ep);
+            OHIP_CHECK(run_conv_tap(xq, false, h->w_tap, out, g, ep, config, h->in_scale, d.in_round_mode, stream));
+            return quantize_twin();
+        }
+    }
     if ((twin || residual) && kind == 1 && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) {
         ep.twin = twin, ep.twin_scale = twin_scale;
         ep.twin_half = twin_round == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;

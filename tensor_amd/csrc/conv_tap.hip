@@ -1,0 +1,442 @@
+// Dense and grouped int8 convolution with both matrix operands straight from memory and the reduction dealt to the waves
+// of a workgroup: the kernel for launches that do not fill the machine, and for reductions that the 64-channel steps of the
+// implicit-GEMM kernel pad heavily.
+//
+// What bounds those launches is not bandwidth or operations but one chain of dependent latencies per workgroup. The
+// implicit-GEMM kernel walks its k-chunks one barrier and one LDS round trip after the other (264 -> 24 5x5 stride 2 on
+// twelve 7x7 images: 125 chunks, three workgroups, 46 us); the LDS-halo kernel stages whole rows before its first
+// multiplication. Here
+//  * WK waves of a workgroup take every WK-th reduction step each, hold their loads DEPTH steps ahead in registers and
+//    meet once, in LDS, to add up their int32 accumulators (integers: the same result in any order);
+//  * the reduction runs over (tap, channel octet) pairs in that order, eight to a 64-deep matrix step, with no padding but
+//    at its end: 8 channels of a 5x5 layer are 4 steps instead of 25, 104 channels of a 3x3 layer 15 instead of 18. A
+//    lane's 16-byte operand is two consecutive pairs of its pixel, two 8-byte loads (16 lanes: 128 contiguous bytes each);
+//  * the byte offset of a pair and the bit of its tap come from a table in LDS, the taps that fall outside the image from a
+//    bit mask per pixel: three vector instructions per load, an invalid one gets an offset beyond the buffer and reads zero.
+// The same operands are re-read per tap from L1 / L2, which is why large launches with long reductions stay with the
+// kernels that stage them in LDS (conv_tap_cost against conv_family_cost).
+//
+// Measured, us per launch before / after: 336 -> 184 3x3, one 13x13 image 22.7 / 4.5; 400 -> 216 3x3 stride 2, thirteen 23x23
+// 29.1 / 8.1; 160 -> 8 5x5 @184x224 43.0 / 17.7; 16 -> 184 5x5 @168x168 x4 56.4 / 30.9; 720 -> 384 1x1 from fp32, one 13x13
+// image 9.2 / 3.7; 64 -> 128 3x3 in 8 groups @32x32 x13 8.8 / 6.2.
+//
+// INF: the input is a Float8 blob ([N][C/8][H*W][8 floats]); a lane quantizes the pairs it loads (quantize_to_int8,
+// Tensor/ConvolutionLayer.cpp:770-775). Every value is quantized once per tap that reads it, which a launch that leaves
+// most of the vector ALU idle has room for; it saves the quantize launch and its blob.
+#include "common.hpp"
+#include "conv_igemm.hpp"
+
+#include <cmath>
+
+namespace ohip {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+namespace {
+
+constexpr int TAP_MAX_TAPS = 31;      // bit 31 of a pixel's mask stands for "past the end of the reduction"
+constexpr int TAP_MAX_PAIRS = 2048;   // table entries: 16 KB of LDS
+
+// n / d for 0 <= n < 2^31 as a multiplication: with 2^(l-1) < d <= 2^l and m = ceil(2^(31+l) / d) the error m d - 2^(31+l) is
+// below 2^l, so that n times it stays below 2^(31+l)
+struct FastDiv {
+    unsigned m, s, d;
+};
+FastDiv fast_div(unsigned d) {
+    FastDiv f{0, 0, d};
+    if (d <= 1) return f;
+    unsigned l = 1;
+    while ((1ull << l) < d) ++l;
+    f.m = (unsigned)(((1ull << (31 + l)) + d - 1) / d);
+    f.s = l - 1;
+    return f;
+}
+__device__ __forceinline__ unsigned div_by(unsigned n, const FastDiv& f) { return f.m ? __umulhi(n, f.m) >> f.s : n; }
+
+struct TapArgs {
+    ConvGeom g;           // one group's channels; g.Cs / g.Ks the tensors'
+    FastDiv ohw, ow, c8, kw;
+    int steps, pairs;     // reduction steps and (tap, octet) pairs of them
+    int m_tiles16;        // 16-row tiles of one group's packed weights
+    int n_pix_tiles;
+    unsigned in_bytes, w_bytes;
+    const float* in_scale;
+    float in_half;
+};
+
+__device__ __forceinline__ int tap_quant4(const v4i& f, float scale, float half) {
+    int k[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float t = __fmul_rn(__int_as_float(f[e]), scale);
+        k[e] = (int)__fadd_rn(t, __builtin_copysignf(half, t));  // toward zero, saturating
+    }
+    const ohip_v2s top = {127, 127}, bot = {-127, -127};
+    ohip_v2s a = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[0], k[1]));
+    ohip_v2s b = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[2], k[3]));
+    a = __builtin_elementwise_max(__builtin_elementwise_min(a, top), bot);
+    b = __builtin_elementwise_max(__builtin_elementwise_min(b, top), bot);
+    return (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x06040200u);
+}
+
+}  // namespace
+
+template <int FM, int FN, int WK, int WN, int DEPTH, int EPI, bool INF>
+__global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
+                                                                void* __restrict__ out, TapArgs ta, Epilogue ep) {
+    constexpr int UNITS = FM / 2 * FN;  // (row-tile pair, pixel fragment) accumulators of a wave
+    constexpr int OOB = (int)0x80000000;  // beyond any buffer here (below 2 GiB)
+    extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+    v2i* const table = reinterpret_cast<v2i*>(lds);  // [pairs, rounded up to whole steps]: {byte offset, bit number of the tap}
+    v4i* const red = reinterpret_cast<v4i*>(lds + (size_t)ta.steps * 64);  // [wn][wk][unit][half][lane]
+    const ConvGeom& g = ta.g;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, p = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave % WK, wn = wave / WK;
+    int pt = blockIdx.x;
+    {  // a contiguous run of pixel tiles per XCD (workgroups go to the 8 XCDs round-robin)
+        const int per = ta.n_pix_tiles / 8;
+        if (pt < per * 8) pt = (pt % 8) * per + pt / 8;
+    }
+    const int mt0 = blockIdx.y * FM;
+    const int HW = g.H * g.W, OHW = g.OH * g.OW, C8 = g.C / 8, Cs8 = g.Cs / 8;
+    const int grp = blockIdx.z;
+    const unsigned total_pix = (unsigned)g.N * (unsigned)OHW;
+
+    // ---- weights: the first steps are on their way before anything else happens ------------------------------------------
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(wpk + (size_t)grp * ta.w_bytes), 0, (int)ta.w_bytes, 0x00020000);
+    v4i a[DEPTH][FM];
+    auto load_a = [&](int d, int s) {  // step s (uniform); past the end: zeros
+        const int v = s < ta.steps ? lane * 16 : OOB, so = s < ta.steps ? (s * ta.m_tiles16 + mt0) * 1024 : 0;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) a[d][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, v + i * 1024, so, 0));
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) load_a(d, wk + d * WK);
+
+    // ---- the table of pairs ---------------------------------------------------------------------------------------------------
+    for (int e = tid; e < ta.steps * 8; e += 64 * WK * WN) {
+        const unsigned tap = div_by((unsigned)e, ta.c8), oct = (unsigned)e - tap * (unsigned)C8;
+        const unsigned dy = div_by(tap, ta.kw), dx = tap - dy * (unsigned)g.kw;
+        table[e] = e < ta.pairs ? v2i{(int)(oct * (unsigned)HW + dy * (unsigned)(g.dh * g.W) + dx * (unsigned)g.dw) * 8, (int)tap}
+                                : v2i{0, 31};
+    }
+
+    // ---- this lane's pixels ---------------------------------------------------------------------------------------------------
+    unsigned px_ofs[FN], mask[FN], out_n[FN], out_pix[FN];
+    bool px_ok[FN];
+    const bool pointwise = g.kh == 1 && g.kw == 1 && g.sh == 1 && g.sw == 1 && g.ph == 0 && g.pw == 0;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const unsigned gp = ((unsigned)pt * WN + wn) * (16 * FN) + 16 * j + p;
+        px_ok[j] = gp < total_pix;
+        const unsigned n = div_by(gp, ta.ohw), pix = gp - n * (unsigned)OHW;
+        out_n[j] = n, out_pix[j] = pix;
+        const unsigned img = (n * (unsigned)Cs8 + (unsigned)(grp * C8)) * (unsigned)HW * 8u;
+        if (pointwise) {
+            px_ofs[j] = img + pix * 8u, mask[j] = 0x80000000u;
+        } else {
+            const unsigned oy = div_by(pix, ta.ow), ox = pix - oy * (unsigned)g.OW;
+            const int iy0 = (int)oy * g.sh - g.ph, ix0 = (int)ox * g.sw - g.pw;
+            px_ofs[j] = img + (unsigned)((iy0 * g.W + ix0) * 8);  // (modulo 2^32: the pair's offset brings it back)
+            unsigned cols = 0, all = (1u << g.kw) - 1, m = 0x80000000u;
+            for (int dx = 0; dx < g.kw; ++dx) {
+                const int ix = ix0 + dx * g.dw;
+                cols |= (ix < 0 || ix >= g.W ? 1u : 0u) << dx;
+            }
+            for (int dy = 0; dy < g.kh; ++dy) {
+                const int iy = iy0 + dy * g.dh;
+                m |= (iy < 0 || iy >= g.H ? all : cols) << (dy * g.kw);
+            }
+            mask[j] = m;
+        }
+        if (!px_ok[j]) mask[j] = 0xffffffffu;
+    }
+
+    // ---- the reduction --------------------------------------------------------------------------------------------------------
+    const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(x), 0, (int)ta.in_bytes, 0x00020000);
+    v2i b[INF ? 1 : DEPTH][FN][2];
+    v4i bf[INF ? DEPTH : 1][FN][4];
+    float in_scale = 0.f;
+    if constexpr (INF) in_scale = ta.in_scale[0];
+    __syncthreads();
+    auto load_b = [&](int d, int s) {
+        // steps past the end keep the bit of the last table row's padding out of reach: they read the table's first step
+        // with every pair invalid
+        const bool in = s < ta.steps;
+        const v4i t = reinterpret_cast<const v4i*>(table)[(in ? s : 0) * 4 + q];
+        const int b0 = in ? t[1] : 31, b1 = in ? t[3] : 31;
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            // the tap's invalid bit becomes bit 31 of the offset: beyond the buffer, whatever the rest of it is
+            const unsigned i0 = __builtin_amdgcn_ubfe(mask[j], (unsigned)b0, 1) << 31;
+            const unsigned i1 = __builtin_amdgcn_ubfe(mask[j], (unsigned)b1, 1) << 31;
+            const unsigned o0 = px_ofs[j] + (unsigned)t[0], o1 = px_ofs[j] + (unsigned)t[2];
+            if constexpr (INF) {  // (the fp32 element of a pixel's octet lies at four times the int8 element's offset)
+                const int f0 = (int)(o0 * 4u | i0), f1 = (int)(o1 * 4u | i1);
+                bf[d][j][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, f0, 0, 0));
+                bf[d][j][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, f0 + 16, 0, 0));
+                bf[d][j][2] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, f1, 0, 0));
+                bf[d][j][3] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, f1 + 16, 0, 0));
+            } else {
+                b[d][j][0] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)(o0 | i0), 0, 0));
+                b[d][j][1] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)(o1 | i1), 0, 0));
+            }
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) load_b(d, wk + d * WK);
+    v4i acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+    for (int s0 = wk; s0 < ta.steps; s0 += DEPTH * WK) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            v4i bb[FN];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (INF)
+                    bb[j] = v4i{tap_quant4(bf[d][j][0], in_scale, ta.in_half), tap_quant4(bf[d][j][1], in_scale, ta.in_half),
+                                tap_quant4(bf[d][j][2], in_scale, ta.in_half), tap_quant4(bf[d][j][3], in_scale, ta.in_half)};
+                else
+                    bb[j] = v4i{b[d][j][0][0], b[d][j][0][1], b[d][j][1][0], b[d][j][1][1]};
+            }
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[d][i], bb[j], acc[i][j], 0, 0, 0);
+            const int nx = s0 + (DEPTH + d) * WK;  // the step this stage holds next
+            if (nx < ta.steps) {                   // (uniform)
+                load_a(d, nx);
+                load_b(d, nx);
+            } else {
+#pragma unroll
+                for (int i = 0; i < FM; ++i) a[d][i] = v4i{0, 0, 0, 0};
+            }
+        }
+    }
+
+    // ---- the waves' sums meet: unit u of a pixel group is finished by its wave u % WK ---------------------------------------------
+    if constexpr (WK > 1) {
+        v4i* const mine = red + (size_t)((wn * WK + wk) * UNITS) * 128 + lane;
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            if (u % WK == wk) continue;
+            mine[u * 128] = acc[2 * (u / FN)][u % FN];
+            mine[u * 128 + 64] = acc[2 * (u / FN) + 1][u % FN];
+        }
+        __syncthreads();
+    }
+    const size_t ch_base = (size_t)grp * g.K;
+    ep.scale_in += ch_base, ep.bias += ch_base;
+    if (ep.scale_out) ep.scale_out += ch_base;
+    const int Ks = g.Ks;
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+        if (WK > 1 && u % WK != wk) continue;  // (uniform)
+        const int pair = u / FN, j = u % FN;
+        v4i lo = acc[2 * pair][j], hi = acc[2 * pair + 1][j];
+        if constexpr (WK > 1) {
+            const v4i* const r = red + (size_t)(wn * WK * UNITS + u) * 128 + lane;
+#pragma unroll
+            for (int k = 0; k < WK; ++k) {
+                if (k == u % WK) continue;
+                lo += r[k * UNITS * 128];
+                hi += r[k * UNITS * 128 + 64];
+            }
+        }
+        const int ch0 = 16 * mt0 + 32 * pair + 8 * q;  // this lane's 8 consecutive output channels of the group
+        if (!px_ok[j] || ch0 >= g.K) continue;
+        const int a8[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        const unsigned n = out_n[j], pix = out_pix[j];
+        if constexpr (EPI == EPI_GENERIC) {
+            epilogue_store8_generic(out, &ep, (int)n, ch0, (int)pix, g.K, OHW, a8[0], a8[1], a8[2], a8[3], a8[4], a8[5], a8[6], a8[7]);
+        } else {
+            Epi8 prm;
+            epi8_load<EPI>(prm, ep, ch0);
+            const unsigned ch = (unsigned)ch_base + (unsigned)ch0;  // in the tensor
+            if constexpr (EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
+                const size_t o = ((size_t)(n * (unsigned)(Ks / 8) + ch / 8) * (unsigned)OHW + pix) * 8;
+                epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm, o, a8);
+            } else {
+                constexpr bool FUSED = EPI == EPI_F32_P4_FUSED;
+                const size_t e = ((size_t)(n * (unsigned)(Ks / 4) + ch / 4) * (unsigned)OHW + pix) * 4;
+                ohip_v2i tw = {0, 0};
+                tw[0] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si, prm.bi, e, a8[0], a8[1], a8[2], a8[3]);
+                if (ch0 + 4 < g.K)
+                    tw[1] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si + 4, prm.bi + 4, e + (size_t)OHW * 4, a8[4], a8[5],
+                                                         a8[6], a8[7]);
+                if constexpr (FUSED)
+                    if (ep.twin != nullptr)  // K % 8 == 0 then: the lane's 8 channels are one Byte8 element
+                        *reinterpret_cast<ohip_v2i*>(ep.twin + ((size_t)(n * (unsigned)(Ks / 8) + ch / 8) * (unsigned)OHW + pix) * 8) = tw;
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------------------------------------------------------------
+
+static int tap_pairs(int C, int kh, int kw) { return kh * kw * (C / 8); }
+static int tap_steps(int C, int kh, int kw) { return (tap_pairs(C, kh, kw) + 7) / 8; }
+
+// whether the implicit-GEMM packing of these weights already is this kernel's: a step is then whole taps, or one tap's part
+bool tap_weights_are_igemm(int C, int kh, int kw, int tap_pack) {
+    if (kh * kw == 1 || C % 64 == 0) return true;
+    return tap_pack > 1 && C * tap_pack == 64;
+}
+
+size_t tap_packed_weight_bytes(int K, int C, int kh, int kw) {
+    return (size_t)tap_steps(C, kh, kw) * (igemm_padded_rows(K) / 16) * 1024;
+}
+
+// weight [K, C, kh, kw] int8 -> [step][16-row tile][lane][16 bytes]: bytes 0-7 / 8-15 of lane (r, q) are the octets of pairs
+// 8 step + 2 q and + 1, pair e = (tap e / (C/8), octet e % (C/8))
+void tap_pack_weights(const int8_t* w, int K, int C, int kh, int kw, int8_t* dst) {
+    const int mt16 = igemm_padded_rows(K) / 16, taps = kh * kw, C8 = C / 8, pairs = tap_pairs(C, kh, kw);
+    size_t o = 0;
+    for (int s = 0; s < tap_steps(C, kh, kw); ++s)
+        for (int mt = 0; mt < mt16; ++mt)
+            for (int lane = 0; lane < 64; ++lane) {
+                const int ch = igemm_row_channel(mt * 16 + (lane & 15));
+                for (int h = 0; h < 2; ++h) {
+                    const int e = 8 * s + 2 * (lane >> 4) + h, tap = e / C8, c0 = e % C8 * 8;
+                    for (int b = 0; b < 8; ++b, ++o)
+                        dst[o] = ch < K && e < pairs ? w[((size_t)ch * C + c0 + b) * taps + tap] : 0;
+                }
+            }
+}
+
+size_t tap_grouped_weight_bytes(int K, int C, int groups, int kh, int kw) {
+    return (size_t)groups * tap_packed_weight_bytes(K / groups, C / groups, kh, kw);
+}
+void tap_pack_weights_grouped(const int8_t* w, int K, int C, int groups, int kh, int kw, int8_t* dst) {
+    const int kg = K / groups, cg = C / groups;
+    const size_t per = tap_packed_weight_bytes(kg, cg, kh, kw);
+    for (int grp = 0; grp < groups; ++grp)
+        tap_pack_weights(w + (size_t)grp * kg * cg * kh * kw, kg, cg, kh, kw, dst + grp * per);
+}
+
+bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
+    if (g.OH < 1 || g.OW < 1 || g.C % g.groups || g.K % g.groups) return false;
+    const int cg = g.C / g.groups, kg = g.K / g.groups;
+    if (cg % 8 || g.kh * g.kw > TAP_MAX_TAPS || tap_pairs(cg, g.kh, g.kw) > TAP_MAX_PAIRS || g.groups > 65535) return false;
+    const int epi = pick_epilogue(ep, kg);
+    if (g.groups > 1 && (epi == EPI_GENERIC || ep.twin != nullptr || ep.residual != nullptr)) return false;
+    if ((ep.twin != nullptr || ep.residual != nullptr) && epi != EPI_F32_P4) return false;
+    if (f32in && epi == EPI_GENERIC) return false;
+    return (size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1) < ((size_t)1 << 31);  // 32-bit byte offsets
+}
+
+namespace {
+// A tile is 16 fm output channels x 16 fn wn pixels. The cost of a launch in microseconds (measured inside a graph of
+// launches, warm) is start + chain * S + c * (waves * S * step + group), with S the reduction steps of one wave and c the
+// workgroups per compute unit, at least 1: fitted to 420 layers drawn over 8..512 channels, 1x1 to 5x5, 50 to 600 000
+// pixels; the median error is 8 %, the choice by it costs 4 % against the best tile of each layer. Second row: fp32 input.
+struct TapConfig {
+    int fm, fn, wk, wn;
+    float start, chain, step, group;
+    float start_f32, chain_f32, step_f32, group_f32;
+};
+constexpr TapConfig kTapConfigs[] = {
+    {2, 1, 8, 1, 2.42f, 0.097f, 0.020f, 0.72f, 2.42f, 0.284f, 0.050f, 0.48f},
+    {2, 2, 4, 1, 2.59f, 0.066f, 0.033f, 0.57f, 2.80f, 0.238f, 0.099f, 0.38f},
+    {4, 2, 4, 1, 2.49f, 0.087f, 0.049f, 0.50f, 2.61f, 0.225f, 0.111f, 0.69f},
+    {4, 2, 2, 2, 2.64f, 0.027f, 0.056f, 0.60f, 2.76f, 0.114f, 0.127f, 0.93f},
+    {4, 4, 1, 4, 2.78f, 0.000f, 0.103f, 1.82f, 0.f, 0.f, 0.f, 0.f},  // (no fp32 input: registers)
+};
+constexpr int kTapConfigCount = (int)(sizeof(kTapConfigs) / sizeof(kTapConfigs[0]));
+
+template <int FM, int FN, int WK, int WN, int DEPTH, int EPI, bool INF>
+hipError_t launch_tap(const void* x, const int8_t* wpk, void* out, const TapArgs& ta, const Epilogue& ep, int groups, hipStream_t stream) {
+    const size_t lds = (size_t)ta.steps * 64 + (WK > 1 ? (size_t)WN * WK * (FM / 2) * FN * 2048 : 0);
+    const dim3 grid((unsigned)ta.n_pix_tiles, (unsigned)((ta.g.K + 16 * FM - 1) / (16 * FM)), (unsigned)groups);
+    hipLaunchKernelGGL((conv_tap_kernel<FM, FN, WK, WN, DEPTH, EPI, INF>), grid, dim3(64 * WK * WN), lds, stream, (const int8_t*)x,
+                       wpk, out, ta, ep);
+    return hipGetLastError();
+}
+}  // namespace
+
+float conv_tap_cost(const ConvGeom& g, bool f32in, int* config) {
+    const int C = g.C / g.groups, K = g.K / g.groups, steps = tap_steps(C, g.kh, g.kw);
+    const float px = (float)g.N * g.OH * g.OW;
+    float best = __builtin_inff();
+    *config = -1;
+    for (int i = 0; i < kTapConfigCount; ++i) {
+        const TapConfig& c = kTapConfigs[i];
+        if (f32in && c.step_f32 == 0.f) continue;
+        // whole reductions in one wave: the tile's input no longer fits L1 between two taps (measured twice the model's time)
+        if (c.wk == 1 && steps > (g.sh == 2 ? 8 : 16)) continue;
+        const float groups = ceilf(px / (16 * c.fn * c.wn)) * (float)((K + 16 * c.fm - 1) / (16 * c.fm)) * g.groups;
+        const float s = (float)((steps + c.wk - 1) / c.wk), cu = fmaxf(1.f, groups / 256), w = (float)(c.wk * c.wn) * s;
+        const float t = f32in ? c.start_f32 + c.chain_f32 * s + cu * (w * c.step_f32 + c.group_f32)
+                              : c.start + c.chain * s + cu * (w * c.step + c.group);
+        if (t < best) best = t, *config = i;
+    }
+    return best;
+}
+
+// The same for the launches that the kernel above competes with (families of otter_hip_conv_kernel_kind): the
+// implicit-GEMM kernel (1; with fp32 input for pointwise layers), the LDS-halo kernel (3), the fp32 pointwise kernel (6).
+// Fitted to the same layers: start + chain * chunks + matrix work + epilogue + bytes in + bytes out, median error 4 to 9 %.
+float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes) {
+    const int C = g.C / g.groups, K = g.K / g.groups, taps = g.kh * g.kw, tp = g.groups > 1 ? igemm_tap_pack(C, g.kh, g.kw) : 1;
+    const float chunks = tp > 1 ? (float)((taps + tp - 1) / tp) : (float)(taps * igemm_channel_groups(C));
+    const float px = (float)g.N * g.OH * g.OW * g.groups, rows = K <= 32 ? 32.f : (float)((K + 63) / 64 * 64);
+    const float in_mb = (float)g.N * g.C * g.H * g.W * 1e-6f, out_mb = (float)g.N * g.OH * g.OW * g.K * out_bytes * 1e-6f;
+    const float mac = px * rows * chunks * 1e-9f, epi = px * rows * 1e-8f;
+    if (family == 6) return 2.35f + 1.52f * chunks + 53.7f * epi + 0.07f * out_mb;
+    if (family == 3) return 2.97f + 0.27f * chunks + 25.2f * mac + 39.6f * epi + 0.055f * out_mb;
+    if (taps > 1) return 3.0f + 0.32f * chunks + 62.5f * mac + 50.f * epi + 0.26f * in_mb + 0.02f * out_mb;
+    if (f32in) return 2.37f + 0.50f * chunks + 201.f * mac + 18.f * epi + 0.33f * in_mb + 0.09f * out_mb;
+    return 2.46f + 0.34f * chunks + 94.f * mac + 26.f * epi + 0.03f * in_mb + 0.07f * out_mb;
+}
+
+hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g_in, const Epilogue& ep, int config,
+                        const float* in_scale, int in_round_mode, hipStream_t stream) {
+    if (!conv_tap_supported(g_in, ep, f32in) || config < 0 || config >= kTapConfigCount) return hipErrorInvalidValue;
+    TapArgs ta;
+    ta.g = g_in;
+    ta.g.Cs = g_in.C, ta.g.Ks = g_in.K;
+    ta.g.C = g_in.C / g_in.groups, ta.g.K = g_in.K / g_in.groups;
+    const ConvGeom& g = ta.g;
+    ta.ohw = fast_div((unsigned)(g.OH * g.OW)), ta.ow = fast_div((unsigned)g.OW);
+    ta.c8 = fast_div((unsigned)(g.C / 8)), ta.kw = fast_div((unsigned)g.kw);
+    ta.steps = tap_steps(g.C, g.kh, g.kw), ta.pairs = tap_pairs(g.C, g.kh, g.kw);
+    ta.m_tiles16 = igemm_padded_rows(g.K) / 16;
+    ta.in_bytes = (unsigned)((size_t)g.N * g.Cs * g.H * g.W * (f32in ? 4 : 1));
+    ta.w_bytes = (unsigned)tap_packed_weight_bytes(g.K, g.C, g.kh, g.kw);
+    ta.in_scale = in_scale;
+    ta.in_half = in_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+    const TapConfig c = kTapConfigs[config];
+    const long px = (long)g.N * g.OH * g.OW, per = 16l * c.fn * c.wn;
+    ta.n_pix_tiles = (int)((px + per - 1) / per);
+    int epi = pick_epilogue(ep, g.K);
+    if (epi == EPI_F32_P4 && (ep.twin != nullptr || ep.residual != nullptr)) epi = EPI_F32_P4_FUSED;
+#define OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, E_)                                                                           \
+    if (config == I_ && epi == E_) {                                                                                        \
+        if (!f32in) return launch_tap<FM_, FN_, WK_, WN_, D_, E_, false>(x, wpk, out, ta, ep, g_in.groups, stream);         \
+        if constexpr (E_ != EPI_GENERIC && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g_in.groups, stream); \
+    }
+#define OHIP_TAP(I_, FM_, FN_, WK_, WN_, D_)                 \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8)         \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8_NONNEG)  \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4)        \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4_FUSED)  \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_GENERIC)
+    OHIP_TAP(0, 2, 1, 8, 1, 4)
+    OHIP_TAP(1, 2, 2, 4, 1, 4)
+    OHIP_TAP(2, 4, 2, 4, 1, 2)
+    OHIP_TAP(3, 4, 2, 2, 2, 2)
+    OHIP_TAP(4, 4, 4, 1, 4, 2)
+#undef OHIP_TAP
+#undef OHIP_TAP2
+    return hipErrorInvalidValue;
+}
+
+}  // namespace ohip

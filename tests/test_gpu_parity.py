@@ -899,3 +899,69 @@ def test_error_codes(hip):
     with pytest.raises(capi.HipError) as e:
         hip.conv(wq=wq, scale_in=np.ones(8, np.float32), out_kind=capi.OUT_I8)  # int8 output without output scale
     assert e.value.code == -2
+
+
+@pytest.mark.parametrize("config", range(5))
+@pytest.mark.parametrize("C,K,kh,s,p,d,g,N,H,W", [
+    (8, 8, 5, 1, 2, 1, 1, 1, 7, 7),        # 25 taps of one octet: four steps, the last nearly empty
+    (24, 40, 3, 2, 1, 1, 1, 2, 13, 10),    # steps that end inside a tap
+    (104, 72, 3, 1, 1, 1, 1, 1, 5, 3),     # fewer pixels than a fragment, rows past one pair of tiles
+    (64, 136, 3, 1, 2, 2, 1, 2, 9, 11),    # dilation
+    (528, 20, 1, 1, 0, 1, 1, 1, 9, 8),     # a long pointwise reduction; K a multiple of four only (fp32 result)
+    (16, 16, 1, 1, 0, 1, 1, 3, 16, 16),    # one step: most waves have none
+    (64, 96, 3, 1, 1, 1, 4, 2, 12, 17),    # groups of 16 -> 24
+    (32, 64, 3, 1, 0, 1, 2, 1, 40, 33),    # no padding
+    (72, 33, 3, 1, 1, 1, 1, 1, 8, 8),      # K odd: the generic epilogue
+])
+def test_reduction_dealt_to_waves(hip, oracle, config, C, K, kh, s, p, d, g, N, H, W):
+    """The kernel that reads both operands straight from memory, every tile of it: raw accumulators, int8 results of both
+    epilogues and fp32 results with LeakyReLU, from int8 and from fp32 blobs."""
+    rng = np.random.default_rng(1000 + C + K)
+    x, wq, ws, bias = _rand_problem(rng, C, K, kh, g, N, H, W)
+    geo = dict(stride=s, pad=p, dil=d, groups=g)
+    ogeo = dict(stride=(s, s), pad=(p, p), dil=(d, d), groups=g)
+    xf = (x.astype(np.float32) / 20 + rng.uniform(-0.02, 0.02, x.shape)).astype(np.float32)
+    for src in (x, xf):
+        if src is xf and (config == 4 or K % 4):
+            continue  # that tile takes int8 only, the generic epilogue as well
+        for act, int8_out in ((1, True), (0, True), (2, False)):
+            if int8_out and (K // g) % 8 and g > 1:
+                continue
+            want = oracle.conv_layer_forward(src, wq, ws, 20.0, bias=bias, top_scale=9.0, int8_out=int8_out, act_type=act,
+                                             act_params=[0.1] if act == 2 else None, **ogeo)
+            if src is xf and int8_out and K % 8:
+                continue
+            out, _ = run_conv(hip, oracle, src, wq, ws, 20.0, bias=bias, top_scale=9.0, act=act, act_p0=0.1,
+                              out_kind=capi.OUT_I8 if int8_out else capi.OUT_F32, tile=(-8, config), **geo)
+            if int8_out:
+                np.testing.assert_array_equal(out, want)
+            else:
+                assert_f32_close(out, want)
+    if g == 1:
+        _, acc_want = oracle.conv_layer_forward(x, wq, ws, 20.0, want_acc=True, int8_out=False, **ogeo)
+        acc, _ = run_conv(hip, oracle, x, wq, ws, 20.0, out_kind=capi.OUT_I32, tile=(-8, config), **geo)
+        np.testing.assert_array_equal(acc, acc_want)
+
+
+@pytest.mark.parametrize("config", range(4))
+@pytest.mark.parametrize("f32in", [False, True])
+def test_reduction_dealt_to_waves_with_sum_and_twin(hip, oracle, config, f32in):
+    rng = np.random.default_rng(77)
+    C, K, N, H, W = 96, 40, 2, 9, 7
+    _, wq, ws, bias = _rand_problem(rng, C, K, 1, 1, N, H, W)
+    x = rng.uniform(-5, 5, (N, C, H, W)).astype(np.float32)
+    layout = capi.F32_P8 if f32in else capi.I8_P8
+    if not f32in:
+        x = rng.integers(-127, 128, x.shape).astype(np.int8)
+    conv = hip.conv(wq=wq, scale_in=host_scale_in(ws, 20.0), bias=bias, in_scale=20.0, out_kind=capi.OUT_F32, act=1)
+    conv.set_tile(-4, 0)
+    xd = hip.to_device(capi.pack_np(x, 8))
+    res = hip.to_device(capi.pack_np(rng.normal(0, 1, (N, K, H, W)).astype(np.float32), 4))
+    want, wantq = conv.forward_residual(xd, layout, N, H, W, res, q_scale=11.0)
+    plain, twin = conv.forward_twin(xd, layout, N, H, W, 11.0, capi.ROUND_EXACT)
+    conv.set_tile(-8, config)
+    got, gotq = conv.forward_residual(xd, layout, N, H, W, res, q_scale=11.0)
+    assert hip.torch.equal(got.view(hip.torch.int32), want.view(hip.torch.int32)) and hip.torch.equal(gotq, wantq)
+    got, gotq = conv.forward_twin(xd, layout, N, H, W, 11.0, capi.ROUND_EXACT)
+    assert hip.torch.equal(got.view(hip.torch.int32), plain.view(hip.torch.int32)) and hip.torch.equal(gotq, twin)
+    conv.close()
