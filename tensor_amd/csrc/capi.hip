@@ -631,7 +631,7 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 
 // The tile of the kernel whose workgroups deal the reduction to their waves (conv_tap.hip), for a layer that the kernels of
 // `family` (1 or 3; with an fp32 blob the launches of families 1 and 6) would run otherwise, or -1 where those are faster by
-// the two cost models. They have to be slower by 15 %: below that the models' errors decide. An fp32 blob may also be
+// the two cost models. They have to be slower by 5 % (pointwise layers: 15 %): below that the models' errors decide. An fp32 blob may also be
 // quantized by a pass of its own, 2 us and 0.5 us per million values, in front of whichever int8 kernel is faster.
 // set_tile(-8, tile) forces it.
 static int tap_config(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, bool f32in, int family) {
@@ -644,7 +644,7 @@ static int tap_config(const otter_hip_conv* h, const ConvGeom& g, const Epilogue
     const float other = f32in && g.kh * g.kw > 1 ? 2.f + 0.5e-6f * (float)g.N * g.C * g.H * g.W +
                                                        fminf(conv_tap_cost(g, false, &config_i8), conv_family_cost(g, family, false, ob))
                                                  : conv_family_cost(g, family, f32in, ob);
-    return cost < 0.85f * other ? config : -1;
+    return cost < (g.kh * g.kw > 1 ? 0.95f : 0.85f) * other ? config : -1;
 }
 
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w, int out_layout) {

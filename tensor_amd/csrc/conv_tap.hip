@@ -336,19 +336,19 @@ bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
 namespace {
 // A tile is 16 fm output channels x 16 fn wn pixels. The cost of a launch in microseconds (measured inside a graph of
 // launches, warm) is start + chain * S + c * (waves * S * step + group), with S the reduction steps of one wave and c the
-// workgroups per compute unit, at least 1: fitted to 420 layers drawn over 8..512 channels, 1x1 to 5x5, 50 to 600 000
-// pixels; the median error is 8 %, the choice by it costs 4 % against the best tile of each layer. Second row: fp32 input.
+// workgroups of the busiest compute unit: fitted to 420 layers drawn over 8..512 channels, 1x1 to 5x5, 50 to 600 000
+// pixels; the median error is 7 %, the choice by it costs 2 % against the best tile of each layer. Last four: fp32 input.
 struct TapConfig {
     int fm, fn, wk, wn;
     float start, chain, step, group;
     float start_f32, chain_f32, step_f32, group_f32;
 };
 constexpr TapConfig kTapConfigs[] = {
-    {2, 1, 8, 1, 2.42f, 0.097f, 0.020f, 0.72f, 2.42f, 0.284f, 0.050f, 0.48f},
-    {2, 2, 4, 1, 2.59f, 0.066f, 0.033f, 0.57f, 2.80f, 0.238f, 0.099f, 0.38f},
-    {4, 2, 4, 1, 2.49f, 0.087f, 0.049f, 0.50f, 2.61f, 0.225f, 0.111f, 0.69f},
-    {4, 2, 2, 2, 2.64f, 0.027f, 0.056f, 0.60f, 2.76f, 0.114f, 0.127f, 0.93f},
-    {4, 4, 1, 4, 2.78f, 0.000f, 0.103f, 1.82f, 0.f, 0.f, 0.f, 0.f},  // (no fp32 input: registers)
+    {2, 1, 8, 1, 2.31f, 0.067f, 0.019f, 0.72f, 2.31f, 0.242f, 0.048f, 0.47f},
+    {2, 2, 4, 1, 2.50f, 0.056f, 0.032f, 0.56f, 2.66f, 0.245f, 0.095f, 0.38f},
+    {4, 2, 4, 1, 2.44f, 0.075f, 0.047f, 0.49f, 2.40f, 0.251f, 0.104f, 0.68f},
+    {4, 2, 2, 2, 2.56f, 0.042f, 0.051f, 0.59f, 2.41f, 0.165f, 0.113f, 0.92f},
+    {4, 4, 1, 4, 2.93f, 0.000f, 0.098f, 1.63f, 0.f, 0.f, 0.f, 0.f},  // (no fp32 input: registers)
 };
 constexpr int kTapConfigCount = (int)(sizeof(kTapConfigs) / sizeof(kTapConfigs[0]));
 
@@ -370,10 +370,8 @@ float conv_tap_cost(const ConvGeom& g, bool f32in, int* config) {
     for (int i = 0; i < kTapConfigCount; ++i) {
         const TapConfig& c = kTapConfigs[i];
         if (f32in && c.step_f32 == 0.f) continue;
-        // whole reductions in one wave: the tile's input no longer fits L1 between two taps (measured twice the model's time)
-        if (c.wk == 1 && steps > (g.sh == 2 ? 8 : 16)) continue;
         const float groups = ceilf(px / (16 * c.fn * c.wn)) * (float)((K + 16 * c.fm - 1) / (16 * c.fm)) * g.groups;
-        const float s = (float)((steps + c.wk - 1) / c.wk), cu = fmaxf(1.f, groups / 256), w = (float)(c.wk * c.wn) * s;
+        const float s = (float)((steps + c.wk - 1) / c.wk), cu = ceilf(groups / 256), w = (float)(c.wk * c.wn) * s;
         const float t = f32in ? c.start_f32 + c.chain_f32 * s + cu * (w * c.step_f32 + c.group_f32)
                               : c.start + c.chain * s + cu * (w * c.step + c.group);
         if (t < best) best = t, *config = i;
