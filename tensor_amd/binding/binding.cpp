@@ -8,7 +8,7 @@
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
-#include <ATen/ops/empty.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 
 #include "../../include/otter_hip_int8.h"
@@ -59,7 +59,8 @@ struct Args {
 };
 
 at::Tensor device_empty(int64_t count, at::ScalarType dt, long device) {
-    return at::empty({count}, at::TensorOptions().dtype(dt).device(c10::DeviceType::CUDA, (c10::DeviceIndex)device));
+    // (what at::empty comes to behind the dispatcher)
+    return at::detail::empty_cuda({count}, dt, c10::Device(c10::DeviceType::CUDA, (c10::DeviceIndex)device), std::nullopt);
 }
 at::ScalarType type_of_layout(int layout) {
     return layout <= OTTER_HIP_F32_P8 ? at::kFloat : layout <= OTTER_HIP_I8_P8 ? at::kChar : at::kInt;
