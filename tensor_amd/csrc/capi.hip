@@ -94,6 +94,7 @@ struct otter_hip_conv {
     int8_t* w_raw = nullptr;     // [K, C/g, kh, kw]           (direct kernel)
     int8_t* w_igemm = nullptr;   // MFMA lane order            (groups == 1, C % 8 == 0)
     int8_t* w_tap = nullptr;     // the same in the order of conv_tap.hip; w_igemm itself where the two agree
+    int8_t* w_rows = nullptr;    // the same in the order of conv_rows.hip (k x k layers)
     int8_t* w_stem = nullptr;    // MFMA lane order of the few-channel 3x3 kernel (C <= 5, K <= 64)
     int32_t* w_dw = nullptr;     // dot4 weight words          (depthwise, C % 8 == 0)
     int8_t* w_dw_mfma = nullptr; // block-diagonal MFMA operands (depthwise 3x3, C % 8 == 0)
@@ -358,6 +359,7 @@ int otter_hip_conv_destroy(otter_hip_conv_t* h) {
     if (!h) return OTTER_HIP_OK;
     (void)hipFree(h->w_raw);
     if (h->w_tap != h->w_igemm) (void)hipFree(h->w_tap);
+    (void)hipFree(h->w_rows);
     (void)hipFree(h->w_igemm);
     (void)hipFree(h->w_stem);
     (void)hipFree(h->w_dw);
@@ -500,6 +502,11 @@ int otter_hip_conv_create(const otter_hip_conv_desc* desc, const int8_t* weight,
                 if ((rc = upload<int8_t>(&h->w_tap, wt.data(), wt.size(), wt.size(), 0))) break;
             }
         }
+        if (h->w_igemm && !h->c_pad && maxk > 1 && maxk <= 25) {
+            std::vector<int8_t> wr(rows_grouped_weight_bytes(K, C, g, d.kernel_h, d.kernel_w));
+            rows_pack_weights_grouped(weight, K, C, g, d.kernel_h, d.kernel_w, wr.data());
+            if ((rc = upload<int8_t>(&h->w_rows, wr.data(), wr.size(), wr.size(), 0))) break;
+        }
     } while (0);
     if (rc != OTTER_HIP_OK) {
         std::string keep = g_last_error;
@@ -629,22 +636,32 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
     return h->force_tm == -7 || (g.C >= 64 && g.K >= 128);
 }
 
-// The tile of the kernel whose workgroups deal the reduction to their waves (conv_tap.hip), for a layer that the kernels of
-// `family` (1 or 3; with an fp32 blob the launches of families 1 and 6) would run otherwise, or -1 where those are faster by
-// the two cost models. They have to be slower by 5 % (pointwise layers: 15 %): below that the models' errors decide. An fp32 blob may also be
-// quantized by a pass of its own, 2 us and 0.5 us per million values, in front of whichever int8 kernel is faster.
-// set_tile(-8, tile) forces it.
-static int tap_config(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, bool f32in, int family) {
-    if (!h->w_tap || (h->force_tm != 0 && h->force_tm != -8) || !conv_tap_supported(g, ep, f32in)) return -1;
-    if (h->force_tm == -8) return h->force_tn;
-    if (family != 1 && family != 3 && !(f32in && family == 6)) return -1;
+// The launches beside those of `family` (1 or 3; with an fp32 blob also 6) that a layer may take, by the cost models: the kernel
+// whose workgroups deal the reduction to their waves (conv_tap.hip) and, for k x k layers without a sum or a twin, the one on
+// staged rows (conv_rows.hip). They have to be faster than the family's launch by 5 % and 10 % (pointwise layers: 15 %): below
+// that the models' errors decide. An fp32 blob may also be quantized by a pass of its own, 2 us and 0.5 us per million
+// values, in front of whichever int8 kernel is faster. set_tile(-8, tile) and set_tile(-9, tile) force them.
+enum AltKernel { ALT_NONE, ALT_TAP, ALT_ROWS };
+static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, bool f32in, int family, bool fused, int* config) {
+    *config = h->force_tn;
+    const bool kxk = g.kh * g.kw > 1, tap = h->w_tap && conv_tap_supported(g, ep, f32in);
+    const bool rows = h->w_rows && !fused && conv_rows_supported(g, ep, f32in);
+    if (h->force_tm == -9) return rows ? ALT_ROWS : ALT_NONE;
+    if (h->force_tm == -8) return tap ? ALT_TAP : ALT_NONE;
+    if (h->force_tm != 0 || (family != 1 && family != 3 && !(f32in && family == 6))) return ALT_NONE;
+    // the staged rows are worth a look where even the fastest such launch (3.5 us) would win
+    auto rows_cost = [&](bool f32, float other, int* c) { return rows && other > 3.9f ? conv_rows_cost(g, f32, c) : __builtin_inff(); };
     const int ob = layout_elem_bytes(ep.out_layout);
-    int config, config_i8;
-    const float cost = conv_tap_cost(g, f32in, &config);
-    const float other = f32in && g.kh * g.kw > 1 ? 2.f + 0.5e-6f * (float)g.N * g.C * g.H * g.W +
-                                                       fminf(conv_tap_cost(g, false, &config_i8), conv_family_cost(g, family, false, ob))
-                                                 : conv_family_cost(g, family, f32in, ob);
-    return cost < (g.kh * g.kw > 1 ? 0.95f : 0.85f) * other ? config : -1;
+    int tap_tile = -1, rows_tile = -1, unused;
+    const float tap_t = tap ? conv_tap_cost(g, f32in, &tap_tile) : __builtin_inff();
+    float other = conv_family_cost(g, family, f32in && !kxk, ob);
+    if (f32in && kxk) {
+        if (tap) other = fminf(other, conv_tap_cost(g, false, &unused));
+        other = 2.f + 0.5e-6f * (float)g.N * g.C * g.H * g.W + fminf(other, rows_cost(false, other, &unused));
+    }
+    const float best = tap_t < (kxk ? 0.95f : 0.85f) * other ? tap_t : other;
+    if (rows_cost(f32in, best, &rows_tile) < 0.9f * best) return *config = rows_tile, ALT_ROWS;
+    return *config = tap_tile, best < other ? ALT_TAP : ALT_NONE;
 }
 
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w, int out_layout) {
@@ -735,15 +752,23 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
         ep.residual = residual;
         twin = nullptr, residual = nullptr;
     };
-    if (in_layout == OTTER_HIP_F32_P8 && h->w_tap && !h->c_pad) {
+    // the launches of conv_tap.hip and conv_rows.hip, where they are the faster ones
+    auto run_alt = [&](const void* src, bool f32in, int family, bool* ran) {
+        Epilogue ep = make_epilogue(h, out_layout);
+        int config;
+        const AltKernel alt = alt_kernel(h, g, ep, f32in, family, twin || residual, &config);
+        *ran = alt != ALT_NONE;
+        if (alt == ALT_ROWS) return run_conv_rows(src, f32in, h->w_rows, out, g, ep, config, h->in_scale, d.in_round_mode, stream);
+        if (alt == ALT_NONE) return hipSuccess;
+        if ((twin || residual) && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) fuse(ep);
+        return run_conv_tap(src, f32in, h->w_tap, out, g, ep, config, h->in_scale, d.in_round_mode, stream);
+    };
+    bool ran;
+    if (in_layout == OTTER_HIP_F32_P8 && (h->w_tap || h->w_rows) && !h->c_pad) {
         Epilogue ep = make_epilogue(h, out_layout);
         const int kind = use_pw_f32in(h, in_layout, g, ep) ? 6 : use_igemm_f32in(h, in_layout, g, ep) ? 1 : pick_kernel(h, OTTER_HIP_I8_P8, g, ep);
-        const int config = tap_config(h, g, ep, true, kind);
-        if (config >= 0) {
-            if ((twin || residual) && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) fuse(ep);
-            OHIP_CHECK(run_conv_tap(in, true, h->w_tap, out, g, ep, config, h->in_scale, d.in_round_mode, stream));
-            return quantize_twin();
-        }
+        OHIP_CHECK(run_alt(in, true, kind, &ran));
+        if (ran) return quantize_twin();
     }
 
     // A pointwise layer on an fp32 Float8 blob: quantize_to_int8 inside the convolution's launch.
@@ -792,13 +817,9 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
 
     Epilogue ep = make_epilogue(h, out_layout);
     const int kind = pick_kernel(h, q_layout, g, ep);
-    if (q_layout == OTTER_HIP_I8_P8 && !h->c_pad && (kind == 1 || kind == 3 || h->force_tm == -8)) {
-        const int config = tap_config(h, g, ep, false, kind);
-        if (config >= 0) {
-            if ((twin || residual) && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) fuse(ep);
-            OHIP_CHECK(run_conv_tap(xq, false, h->w_tap, out, g, ep, config, h->in_scale, d.in_round_mode, stream));
-            return quantize_twin();
-        }
+    if (q_layout == OTTER_HIP_I8_P8 && !h->c_pad) {
+        OHIP_CHECK(run_alt(xq, false, kind, &ran));
+        if (ran) return quantize_twin();
     }
     if ((twin || residual) && kind == 1 && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) {
         ep.twin = twin, ep.twin_scale = twin_scale;

@@ -407,4 +407,36 @@ __device__ __forceinline__ unsigned epi4_store_f32p4(float* __restrict__ out, co
     return q;
 }
 
+// float2int8 of four values into the four bytes of a dword (quantize_to_int8)
+__device__ __forceinline__ int quantize4(const ohip_v4i& f, float scale, float half) {
+    int k[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float t = __fmul_rn(__int_as_float(f[e]), scale);
+        k[e] = (int)__fadd_rn(t, __builtin_copysignf(half, t));  // toward zero, saturating
+    }
+    const ohip_v2s top = {127, 127}, bot = {-127, -127};
+    ohip_v2s a = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[0], k[1]));
+    ohip_v2s b = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[2], k[3]));
+    a = __builtin_elementwise_max(__builtin_elementwise_min(a, top), bot);
+    b = __builtin_elementwise_max(__builtin_elementwise_min(b, top), bot);
+    return (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x06040200u);
+}
+
+// n / d for 0 <= n < 2^31 as a multiplication: with 2^(l-1) < d <= 2^l and m = ceil(2^(31+l) / d) the error m d - 2^(31+l) is
+// below 2^l, so that n times it stays below 2^(31+l)
+struct FastDiv {
+    unsigned m, s, d;
+};
+inline FastDiv fast_div(unsigned d) {
+    FastDiv f{0, 0, d};
+    if (d <= 1) return f;
+    unsigned l = 1;
+    while ((1ull << l) < d) ++l;
+    f.m = (unsigned)(((1ull << (31 + l)) + d - 1) / d);
+    f.s = l - 1;
+    return f;
+}
+__device__ __forceinline__ unsigned div_by(unsigned n, const FastDiv& f) { return f.m ? __umulhi(n, f.m) >> f.s : n; }
+
 }  // namespace ohip

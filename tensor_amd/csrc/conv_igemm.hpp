@@ -29,6 +29,14 @@ float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes)
 hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep, int config,
                         const float* in_scale, int in_round_mode, hipStream_t stream);
 
+// conv_rows.hip: k x k layers on input rows staged in LDS
+size_t rows_grouped_weight_bytes(int K, int C, int groups, int kh, int kw);
+void rows_pack_weights_grouped(const int8_t* w, int K, int C, int groups, int kh, int kw, int8_t* dst);
+bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in);
+float conv_rows_cost(const ConvGeom& g, bool f32in, int* config);
+hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep, int config,
+                         const float* in_scale, int in_round_mode, hipStream_t stream);
+
 // conv_pw.hip: 1x1 stride-1 int8 -> int8 over at most 64 input channels, streamed (reads the implicit-GEMM weight packing)
 bool conv_pw_stream_applicable(const ConvGeom& g, const Epilogue& ep);
 void conv_pw_stream_plan(const ConvGeom& g, int* groups, int* slices);

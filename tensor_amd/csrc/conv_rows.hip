@@ -1,0 +1,452 @@
+// Dense and grouped k x k int8 convolution (k up to 5, any stride and dilation) on input rows staged in LDS: the kernel for
+// large launches that conv3x3_halo_kernel does not take or pads heavily -- 5x5 windows, groups, few input or output channels --
+// and for k x k layers on an fp32 blob, which is quantized once per value on its way into LDS.
+//
+// What bounds the implicit-GEMM kernel on these layers is the supply of the pixel operand from L1: a lane's 16 bytes are two
+// 8-byte loads, a wave's load four 128-byte segments on odd lines, and one such load occupies the compute unit's memory pipe
+// for about 54 cycles (256 -> 256 3x3 in 8 groups @28x28 b64: 250 880 of them, 22.8 us, whatever the kernel around them).
+// The same read from LDS takes 8 to 16, and every input byte crosses the memory pipe once per tile instead of once per tap.
+//
+// A workgroup of four waves owns PT = 64 FN consecutive output pixels and FM 16-row tiles of output channels (all of them, one
+// block after the other, where the input channels fit one stage). Wide images are cut into column strips first, and a strip
+// then counts as an image of its own: pixels are numbered (image, strip, row, column in strip), so that a tile may run over
+// the end of a small image into the next and no lane is idle but in the last tile. The rows of such a sequence of images lie
+// in LDS one after the other with their padding rows and columns as zeros: virtual row v of the tile is row v % VH - pad of
+// image v / VH, VH the padded height. A reduction step is eight (tap, channel octet) pairs of the stage; a lane's two pairs are
+// byte offsets added to its pixel's address. The channel octets come in stages of at most 8; octet planes are 64 bytes off a
+// multiple of 128, which puts the pairs of neighbouring lane quarters into different halves of the banks.
+//
+// Measured, us per launch before / after: 256 -> 256 3x3 in 8 groups @28x28 b64 22.6 / 13.9; 384 -> 64 5x5 in 4 groups
+// @67x67 b9 73 / 20; 272 -> 24 3x3 @157x157 b16 129 / 60; 24 -> 32 5x5 @162x162 b13 51.5 / 16.8; 16 -> 16 3x3 dilated
+// @204x204 b55 107 / 56; 8 -> 344 5x5 @113x113 b24 96 / 62; from fp32 128 -> 64 5x5 in 8 groups @75x89 b32 48.6 / 28.9.
+// What is left above the floor is the chain of a tile (rows in, barrier, steps, stores), which three or four workgroups per
+// compute unit hide in part; keeping eight octets or four weight steps in flight instead cost registers and was slower.
+#include "common.hpp"
+#include "conv_igemm.hpp"
+
+#include <cmath>
+
+namespace ohip {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+namespace {
+
+constexpr int ROWS_OCTETS = 8;             // channel octets of a stage
+constexpr int ROWS_LDS = 64 * 1024;        // what a workgroup may use: two to a compute unit
+
+struct RowsArgs {
+    ConvGeom g;                            // one group's channels; g.Cs / g.Ks the tensors'
+    FastDiv img, tw, vh, vw, ntx, kw;      // dividers: pixels of a strip, its width, VH, VW2, strips per image, kernel width
+    int strips, strip_w, VH, VW2;          // column strips per image, output columns of one, padded height, pixel pairs of a row
+    int rows_max, pitch, plane;            // LDS rows of an octet plane, bytes of a row and of a plane
+    int stages, blocks_per_wg;             // stages of the channels; row blocks that a workgroup walks
+    int m_tiles16, n_tiles;
+    unsigned total_pix;                    // numbered as above, ragged strips included
+    unsigned in_bytes, w_bytes;
+    const float* in_scale;
+    float in_half;
+};
+
+// octets [first, first + count) of stage c: the C/8 octets dealt to the stages as evenly as whole octets allow
+__host__ __device__ inline void rows_stage(int C8, int stages, int c, int* first, int* count) {
+    const int base = C8 / stages, more = C8 % stages;
+    *first = c * base + (c < more ? c : more);
+    *count = base + (c < more ? 1 : 0);
+}
+
+}  // namespace
+
+static int rows_stages(int C) { return (C / 8 + ROWS_OCTETS - 1) / ROWS_OCTETS; }
+static int rows_steps(int C, int taps) {
+    int steps = 0;
+    for (int c = 0, n = rows_stages(C); c < n; ++c) {
+        int first, count;
+        rows_stage(C / 8, n, c, &first, &count);
+        steps += (taps * count + 7) / 8;
+    }
+    return steps;
+}
+
+template <int FM, int FN, int EPI, bool INF>
+__global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
+                                                           void* __restrict__ out, RowsArgs ra, Epilogue ep) {
+    constexpr int OOB = (int)0x80000000;  // beyond any buffer here (below 2 GiB)
+    extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+    const ConvGeom& g = ra.g;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, p = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int pt = blockIdx.x;
+    {  // a contiguous run of tiles per XCD: neighbours share input rows and weights
+        const int per = ra.n_tiles / 8;
+        if (pt < per * 8) pt = (pt % 8) * per + pt / 8;
+    }
+    const int grp = blockIdx.z;
+    const int HW = g.H * g.W, OHW = g.OH * g.OW, C8 = g.C / 8, Cs8 = g.Cs / 8;
+    const int taps = g.kh * g.kw;
+    v2i* const table = reinterpret_cast<v2i*>(lds);            // [pair / 2]: the byte offsets of two pairs
+    v2i* const row_tab = table + (taps * ROWS_OCTETS + 7) / 8 * 4;  // [row]: {byte offset of its column 0, first | last + 1 << 16 valid}
+    int8_t* const data = reinterpret_cast<int8_t*>(row_tab + (ra.rows_max + 1) / 2 * 2);
+
+    // ---- the tile: its first pixel (uniform), its virtual rows ---------------------------------------------------------------------
+    const unsigned t0 = (unsigned)pt * (64 * FN), t1 = min(t0 + 64 * FN, ra.total_pix) - 1;
+    const unsigned m0 = div_by(t0, ra.img), m1 = div_by(t1, ra.img);
+    const unsigned r0 = div_by(t0 - m0 * ra.img.d, ra.tw), r1 = div_by(t1 - m1 * ra.img.d, ra.tw);
+    const int v0 = (int)r0 * g.sh;
+    const int rows = (int)(m1 - m0) * ra.VH + (int)r1 * g.sh + (g.kh - 1) * g.dh + 1 - v0;  // at most rows_max
+
+    // ---- this lane's pixels: LDS address of tap (0, 0), place in the output -----------------------------------------------------------
+    int px[FN];
+    unsigned out_n[FN], out_pix[FN], out_at[FN];  // (the first two for the generic epilogue only)
+    bool px_ok[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const unsigned t = t0 + (wave * FN + j) * 16 + p;
+        const unsigned m = div_by(t, ra.img), in = t - m * ra.img.d, oy = div_by(in, ra.tw), oxs = in - oy * ra.tw.d;
+        const unsigned n = div_by(m, ra.ntx), ox = (m - n * ra.ntx.d) * (unsigned)ra.strip_w + oxs;
+        px_ok[j] = t < ra.total_pix && ox < (unsigned)g.OW;
+        px[j] = t < ra.total_pix ? ((int)(m - m0) * ra.VH + (int)oy * g.sh - v0) * ra.pitch +
+                                       ((int)oxs * g.sw + (((int)(m - n * ra.ntx.d) * ra.strip_w * g.sw - g.pw) & 1)) * 8
+                                 : 0;
+        out_n[j] = n, out_pix[j] = oy * (unsigned)g.OW + ox;
+        out_at[j] = n * (unsigned)(g.Ks * OHW) + out_pix[j] * (EPI == EPI_F32_P4 ? 4u : 8u);
+    }
+
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int8_t*>(wpk + (size_t)grp * ra.w_bytes), 0, (int)ra.w_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(x), 0, (int)ra.in_bytes, 0x00020000);
+    float in_scale = 0.f;
+    if constexpr (INF) in_scale = ra.in_scale[0];
+    ep.scale_in += grp * g.K, ep.bias += grp * g.K;
+    if (ep.scale_out) ep.scale_out += grp * g.K;
+
+    // the rows: a strip's columns start at an even one (the one before its first where that is odd), so that a pixel pair never
+    // lies across the left edge of the image
+    for (int r = tid; r < rows; r += 256) {
+        const unsigned v = (unsigned)(r + v0), im = div_by(v, ra.vh), m = m0 + im, n = div_by(m, ra.ntx);
+        const int iy = (int)(v - im * (unsigned)ra.VH) - g.ph;
+        const int c0 = ((int)(m - n * ra.ntx.d) * ra.strip_w * g.sw - g.pw) & ~1;
+        const bool in = iy >= 0 && iy < g.H && n < (unsigned)g.N;
+        const int first = c0 < 0 ? -c0 : 0, last = g.W - c0 < 2 * ra.VW2 ? g.W - c0 : 2 * ra.VW2;
+        row_tab[r] = v2i{(int)(((n * (unsigned)Cs8 + (unsigned)(grp * C8)) * (unsigned)HW + (unsigned)(iy * g.W + c0)) * 8u),
+                         in && last > first ? first | last << 16 : 0};
+    }
+
+    const int HW8 = HW * 8;
+    const bool even = (g.W & 1) == 0;    // then no pair lies across the right edge either
+    constexpr int UN = INF ? 2 : 4;      // octets in flight per thread
+    constexpr int D = 2;    // weight steps in flight
+    constexpr int INS = INF ? 4 : 1;     // bytes of an input value
+
+    v4i acc[FM][FN];
+    int block = blockIdx.y * ra.blocks_per_wg;
+    const int block_end = min(block + ra.blocks_per_wg, (g.K + 16 * FM - 1) / (16 * FM));
+    auto load_a = [&](v4i (&a)[FM], int step) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+            a[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16 + i * 1024,
+                                                                                (step * ra.m_tiles16 + block * FM) * 1024, 0));
+    };
+
+    for (int c = 0, step0 = 0; c < ra.stages; ++c) {
+        int first, count;
+        rows_stage(C8, ra.stages, c, &first, &count);
+        const int steps = (taps * count + 7) / 8;
+        v4i a[D][FM];
+#pragma unroll
+        for (int d = 0; d + 1 < D; ++d)
+            if (d < steps) load_a(a[d], step0 + d);
+        __syncthreads();  // the row table stands / everyone has read the stage before
+        // the table of this stage's pairs e = (tap e / count, octet e % count); pairs past the end meet zero weights
+        for (int e = tid; e < steps * 8; e += 256) {
+            const unsigned tap = (unsigned)e / (unsigned)count, oct = (unsigned)e - tap * (unsigned)count;
+            const unsigned dy = div_by(tap, ra.kw), dx = tap - dy * (unsigned)g.kw;
+            reinterpret_cast<int*>(table)[e] =
+                e < taps * count ? (int)oct * ra.plane + (int)dy * g.dh * ra.pitch + (int)dx * g.dw * 8 : 0;
+        }
+        // the stage's rows, zeros outside the image, as pixel pairs. A thread keeps one place of the octet planes and walks the
+        // octets, so that an octet costs it a load and a write and no address arithmetic; planes of at most 128 pairs are dealt to
+        // 256 / pairs threads each
+        const int pairs = rows * ra.VW2, sub = pairs > 128 ? 1 : 256 / pairs;
+        const int oct0 = sub == 1 ? 0 : tid / pairs;
+        if (oct0 < sub) {
+            for (int pos = tid - oct0 * pairs; pos < pairs; pos += 256) {
+                const int row = (int)div_by((unsigned)pos, ra.vw), c0 = 2 * (pos - row * ra.VW2);
+                const v2i rt = row_tab[row];
+                const int lo = rt[1] & 0xffff, hi = rt[1] >> 16;
+                const bool in0 = c0 >= lo && c0 < hi, in1 = c0 + 1 >= lo && c0 + 1 < hi;
+                const int o = rt[0] + c0 * 8 + oct0 * HW8;
+                const int o0 = in0 ? o * INS : OOB, o1 = in1 ? (o + 8) * INS : OOB;
+                int8_t* at = data + oct0 * ra.plane + pos * 16;  // (rows are VW2 pairs long)
+                for (int oct = oct0, so = first * HW8 * INS; oct < count; oct += UN * sub) {
+                    v4i v[UN];
+                    v4i f[INF ? UN : 1][4];
+#pragma unroll
+                    for (int u = 0; u < UN; ++u) {
+                        const bool there = u == 0 || oct + u * sub < count;
+                        const int a0 = there ? o0 + so : OOB, a1 = there ? o1 + so : OOB;  // (OOB + so stays beyond any buffer)
+                        if constexpr (INF) {
+                            f[u][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, 0, 0));
+                            f[u][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0 + 16, 0, 0));
+                            f[u][2] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1, 0, 0));
+                            f[u][3] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1 + 16, 0, 0));
+                        } else if (even) {
+                            v[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, 0, 0));
+                        } else {
+                            const v2i l = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a0, 0, 0));
+                            const v2i h = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a1, 0, 0));
+                            v[u] = v4i{l[0], l[1], h[0], h[1]};
+                        }
+                        so += sub * HW8 * INS;
+                    }
+#pragma unroll
+                    for (int u = 0; u < UN; ++u) {
+                        if constexpr (INF)
+                            v[u] = v4i{quantize4(f[u][0], in_scale, ra.in_half), quantize4(f[u][1], in_scale, ra.in_half),
+                                       quantize4(f[u][2], in_scale, ra.in_half), quantize4(f[u][3], in_scale, ra.in_half)};
+                        if (u == 0 || oct + u * sub < count) *reinterpret_cast<v4i*>(at + u * sub * ra.plane) = v[u];
+                    }
+                    at += UN * sub * ra.plane;
+                }
+            }
+        }
+        __syncthreads();
+        // one block of output channels per pass over the stage; several only when there is one stage
+        for (;;) {
+            if (c == 0) {
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+            }
+            auto multiply = [&](int s, const v4i (&aa)[FM]) {
+                const v2i t = table[s * 4 + q];
+                v4i b[FN];
+#pragma unroll
+                for (int j = 0; j < FN; ++j) {
+                    const v2i lo = *reinterpret_cast<const v2i*>(data + px[j] + t[0]);
+                    const v2i hi = *reinterpret_cast<const v2i*>(data + px[j] + t[1]);
+                    b[j] = v4i{lo[0], lo[1], hi[0], hi[1]};
+                }
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(aa[i], b[j], acc[i][j], 0, 0, 0);
+            };
+            for (int s = 0; s < steps; s += D) {
+#pragma unroll
+                for (int d = 0; d < D; ++d)
+                    if (s + d < steps) {
+                        if (s + d + D - 1 < steps) load_a(a[(d + D - 1) % D], step0 + s + d + D - 1);
+                        multiply(s + d, a[d]);
+                    }
+            }
+            if (c + 1 < ra.stages) break;
+            // ---- epilogue of the block -------------------------------------------------------------------------------------------
+            const int mt0 = block * FM;
+            ++block;
+            if (block < block_end)
+#pragma unroll
+                for (int d = 0; d + 1 < D; ++d)
+                    if (d < steps) load_a(a[d], d);  // (one stage: step0 == 0)
+#pragma unroll
+            for (int pair = 0; pair < FM / 2; ++pair) {
+                const int ch0 = 16 * mt0 + 32 * pair + 8 * q;  // this lane's 8 consecutive output channels of the group
+                if (ch0 < g.K) {
+                    Epi8 prm;
+                    if constexpr (EPI != EPI_GENERIC) epi8_load<EPI>(prm, ep, ch0);
+                    const unsigned ch = (unsigned)(grp * g.K + ch0);
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) {
+                        const v4i lo = acc[2 * pair][j], hi = acc[2 * pair + 1][j];
+                        const int a8[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                        if (!px_ok[j]) continue;
+                        if constexpr (EPI == EPI_GENERIC) {
+                            epilogue_store8_generic(out, &ep, (int)out_n[j], ch0, (int)out_pix[j], g.K, OHW, a8[0], a8[1], a8[2], a8[3],
+                                                    a8[4], a8[5], a8[6], a8[7]);
+                        } else if constexpr (EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
+                            const size_t o = out_at[j] + ch * (unsigned)OHW;
+                            epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm, o, a8);
+                        } else {
+                            const size_t e = out_at[j] + ch * (unsigned)OHW;
+                            epi4_store_f32p4<false>((float*)out, ep, prm.si, prm.bi, e, a8[0], a8[1], a8[2], a8[3]);
+                            if (ch0 + 4 < g.K)
+                                epi4_store_f32p4<false>((float*)out, ep, prm.si + 4, prm.bi + 4, e + (size_t)OHW * 4, a8[4], a8[5], a8[6], a8[7]);
+                        }
+                    }
+                }
+            }
+            if (block >= block_end) break;
+        }
+        step0 += steps;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------------------------------------------------------------
+
+static size_t rows_packed_weight_bytes(int K, int C, int taps) { return (size_t)rows_steps(C, taps) * (igemm_padded_rows(K) / 16) * 1024; }
+size_t rows_grouped_weight_bytes(int K, int C, int groups, int kh, int kw) {
+    return (size_t)groups * rows_packed_weight_bytes(K / groups, C / groups, kh * kw);
+}
+
+// weight [K, C / groups, kh, kw] int8 -> per group [stage][step][16-row tile][lane][16 bytes]: bytes 0-7 / 8-15 of lane (r, q) are
+// the octets of the stage's pairs 8 step + 2 q and + 1
+void rows_pack_weights_grouped(const int8_t* w, int K, int C, int groups, int kh, int kw, int8_t* dst) {
+    const int kg = K / groups, cg = C / groups, taps = kh * kw, mt16 = igemm_padded_rows(kg) / 16, stages = rows_stages(cg);
+    size_t o = 0;
+    for (int grp = 0; grp < groups; ++grp)
+        for (int c = 0; c < stages; ++c) {
+            int first, count;
+            rows_stage(cg / 8, stages, c, &first, &count);
+            for (int s = 0; s < (taps * count + 7) / 8; ++s)
+                for (int mt = 0; mt < mt16; ++mt)
+                    for (int lane = 0; lane < 64; ++lane) {
+                        const int ch = igemm_row_channel(mt * 16 + (lane & 15));
+                        for (int h = 0; h < 2; ++h) {
+                            const int e = 8 * s + 2 * (lane >> 4) + h, tap = e / count, c0 = (first + e % count) * 8;
+                            for (int b = 0; b < 8; ++b, ++o)
+                                dst[o] = ch < kg && e < taps * count ? w[(((size_t)grp * kg + ch) * cg + c0 + b) * taps + tap] : 0;
+                        }
+                    }
+        }
+}
+
+static bool rows_plan(const ConvGeom& g_in, int fn, RowsArgs* ra, size_t* lds) {
+    ra->g = g_in;
+    ra->g.Cs = g_in.C, ra->g.Ks = g_in.K;
+    ra->g.C = g_in.C / g_in.groups, ra->g.K = g_in.K / g_in.groups;
+    const ConvGeom& g = ra->g;
+    const int pt = 64 * fn, taps = g.kh * g.kw;
+    ra->VH = (g.OH - 1) * g.sh + (g.kh - 1) * g.dh + 1;
+    // the number of strips that makes a tile stage the fewest bytes: wide strips read padding rows, narrow ones padding columns
+    long best = 0;
+    const long max_px = (1l << 31) - pt;
+    for (int strips = (g.OW + 79) / 80; strips <= (g.OW + 15) / 16; ++strips) {
+        const int w = (g.OW + strips - 1) / strips, vw2 = ((w - 1) * g.sw + (g.kw - 1) * g.dw + 1 + 2) / 2;  // (one column more in front)
+        const long total = (long)g.N * g.OH * strips * w;
+        if (total >= max_px || (long)g.OH * w >= max_px) break;
+        const int strip_px = g.OH * w, tiles = (int)((unsigned)(total + pt - 1) / (unsigned)pt);
+        // rows of a tile: the output rows it can touch, and the padding rows between the images it can run over
+        const int out_rows = (pt - 1) / w + 2, crossings = (pt - 1) / strip_px + 1;
+        const int between = ra->VH - g.OH * g.sh;  // virtual rows an image has more than its output rows' share (may be negative)
+        const int rows = (out_rows - 1) * g.sh + (between > 0 ? crossings * between : 0) + (g.kh - 1) * g.dh + 1;
+        const long cost = (long)tiles * (rows * vw2 + 64);
+        if (best == 0 || cost < best) {
+            best = cost;
+            ra->strips = strips, ra->strip_w = w, ra->VW2 = vw2, ra->rows_max = rows;
+            ra->total_pix = (unsigned)total, ra->n_tiles = tiles;
+        }
+    }
+    if (best == 0) return false;
+    const long strip_px = (long)g.OH * ra->strip_w;
+    ra->pitch = ra->VW2 * 16;
+    ra->plane = (ra->rows_max * ra->pitch + 63) / 128 * 128 + 64;
+    ra->stages = rows_stages(g.C);
+    const int oct = (g.C / 8 + ra->stages - 1) / ra->stages;
+    *lds = (size_t)(taps * ROWS_OCTETS + 7) / 8 * 32 + (size_t)(ra->rows_max + 1) / 2 * 16 + (size_t)oct * ra->plane;
+    ra->img = fast_div((unsigned)strip_px), ra->tw = fast_div((unsigned)ra->strip_w), ra->vh = fast_div((unsigned)ra->VH);
+    ra->vw = fast_div((unsigned)ra->VW2), ra->ntx = fast_div((unsigned)ra->strips), ra->kw = fast_div((unsigned)g.kw);
+    ra->m_tiles16 = igemm_padded_rows(g.K) / 16;
+    ra->w_bytes = (unsigned)rows_packed_weight_bytes(g.K, g.C, taps);
+    return *lds <= (size_t)ROWS_LDS;
+}
+
+bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
+    if (g.OH < 1 || g.OW < 1 || g.C % g.groups || g.K % g.groups || g.kh * g.kw < 2 || g.kh * g.kw > 25 || g.groups > 65535) return false;
+    if ((g.C / g.groups) % 8 || ep.twin != nullptr || ep.residual != nullptr) return false;
+    const int epi = pick_epilogue(ep, g.K / g.groups);
+    if (epi == EPI_GENERIC && (g.groups > 1 || f32in)) return false;
+    return (size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1) < ((size_t)1 << 31) && (size_t)g.N * g.K * g.OH * g.OW < ((size_t)1 << 31);
+}
+
+// one stage: a workgroup walks row blocks over its staged pixels, as many as leave two workgroups per compute unit
+static int rows_blocks_per_workgroup(const RowsArgs& ra, int blocks) {
+    if (ra.stages > 1) return 1;
+    const long tiles = (long)ra.n_tiles * ra.g.groups;
+    const int want = (int)((512 + tiles - 1) / tiles), slices = want > blocks ? blocks : want;
+    return (blocks + slices - 1) / slices;
+}
+
+namespace {
+// A tile, and the coefficients of its duration in us for int8 and fp32 input: start + step * steps + stage * stages of a
+// workgroup's serial chain, and per workgroup of the busiest compute unit each its start, steps, staged places (pixel pairs
+// of a thread) and row blocks. Fitted to 260 layers (k 3 and 5, 8..512 channels, 100..2.3 million pixels), median error 7 %.
+struct RowsCost {
+    float start, step, stage, cu_start, cu_step, cu_place, cu_block;
+};
+struct RowsConfig {
+    int fm, fn;
+    RowsCost i8, f32;
+};
+constexpr RowsConfig kRowsConfigs[] = {
+    {2, 2, {2.65f, 0.114f, 0.55f, 0.32f, 0.040f, 0.058f, 0.34f}, {2.16f, 0.135f, 1.04f, 0.f, 0.013f, 0.205f, 0.57f}},
+    {2, 4, {2.61f, 0.180f, 0.82f, 0.39f, 0.040f, 0.082f, 0.64f}, {2.21f, 0.202f, 1.27f, 0.f, 0.000f, 0.247f, 0.89f}},
+    {4, 2, {2.74f, 0.118f, 0.53f, 0.08f, 0.081f, 0.075f, 0.77f}, {2.52f, 0.154f, 0.91f, 0.f, 0.068f, 0.232f, 0.59f}},
+    {4, 4, {2.63f, 0.188f, 0.77f, 0.30f, 0.085f, 0.105f, 1.19f}, {2.40f, 0.236f, 1.27f, 0.f, 0.051f, 0.286f, 1.16f}},
+};
+constexpr int kRowsConfigCount = (int)(sizeof(kRowsConfigs) / sizeof(kRowsConfigs[0]));
+}  // namespace
+
+float conv_rows_cost(const ConvGeom& g_in, bool f32in, int* config) {
+    float best = __builtin_inff();
+    *config = -1;
+    RowsArgs ra;
+    size_t lds;
+    bool fits = false;
+    const int steps = rows_steps(g_in.C / g_in.groups, g_in.kh * g_in.kw);
+    for (const int i : {0, 2, 1, 3}) {  // by pixels of a tile: one plan for two
+        const RowsConfig& c = kRowsConfigs[i];
+        if (i == 0 || i == 1) fits = rows_plan(g_in, c.fn, &ra, &lds);
+        if (!fits) continue;
+        const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm), bpw = rows_blocks_per_workgroup(ra, blocks);
+        const int pairs = ra.rows_max * ra.VW2, oct = (ra.g.C / 8 + ra.stages - 1) / ra.stages;
+        const float places = (float)(ra.stages * oct) * (pairs > 128 ? (float)((pairs + 255) / 256) : 1.f / (float)(256 / pairs));
+        const float cu = ceilf((float)ra.n_tiles * (float)((blocks + bpw - 1) / bpw) * (float)ra.g.groups / 256);
+        const RowsCost& k = f32in ? c.f32 : c.i8;
+        const float t = k.start + k.step * (float)(bpw * steps) + k.stage * (float)ra.stages +
+                        cu * (k.cu_start + k.cu_step * (float)(bpw * steps) + k.cu_place * places + k.cu_block * (float)bpw);
+        if (t < best) best = t, *config = i;
+    }
+    return best;
+}
+
+hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g_in, const Epilogue& ep, int config,
+                         const float* in_scale, int in_round_mode, hipStream_t stream) {
+    if (!conv_rows_supported(g_in, ep, f32in) || config < 0 || config >= kRowsConfigCount) return hipErrorInvalidValue;
+    const RowsConfig c = kRowsConfigs[config];
+    RowsArgs ra;
+    size_t lds;
+    if (!rows_plan(g_in, c.fn, &ra, &lds)) return hipErrorInvalidValue;
+    ra.in_bytes = (unsigned)((size_t)ra.g.N * ra.g.Cs * ra.g.H * ra.g.W * (f32in ? 4 : 1));
+    ra.in_scale = in_scale;
+    ra.in_half = in_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+    const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm);
+    ra.blocks_per_wg = rows_blocks_per_workgroup(ra, blocks);
+    const dim3 grid((unsigned)ra.n_tiles, (unsigned)((blocks + ra.blocks_per_wg - 1) / ra.blocks_per_wg), (unsigned)g_in.groups);
+    const int epi = pick_epilogue(ep, ra.g.K);
+#define OHIP_ROWS2(I_, FM_, FN_, E_)                                                                                         \
+    if (config == I_ && epi == E_) {                                                                                         \
+        if (!f32in) {                                                                                                        \
+            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, false>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, ep); \
+            return hipGetLastError();                                                                                        \
+        }                                                                                                                    \
+        if constexpr (E_ != EPI_GENERIC) {                                                                                   \
+            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, true>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, ep); \
+            return hipGetLastError();                                                                                        \
+        }                                                                                                                    \
+    }
+#define OHIP_ROWS(I_, FM_, FN_) \
+    OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8) OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8_NONNEG) OHIP_ROWS2(I_, FM_, FN_, EPI_F32_P4) OHIP_ROWS2(I_, FM_, FN_, EPI_GENERIC)
+    OHIP_ROWS(0, 2, 2)
+    OHIP_ROWS(1, 2, 4)
+    OHIP_ROWS(2, 4, 2)
+    OHIP_ROWS(3, 4, 4)
+#undef OHIP_ROWS
+#undef OHIP_ROWS2
+    return hipErrorInvalidValue;
+}
+
+}  // namespace ohip

@@ -38,22 +38,6 @@ namespace {
 constexpr int TAP_MAX_TAPS = 31;      // bit 31 of a pixel's mask stands for "past the end of the reduction"
 constexpr int TAP_MAX_PAIRS = 2048;   // table entries: 16 KB of LDS
 
-// n / d for 0 <= n < 2^31 as a multiplication: with 2^(l-1) < d <= 2^l and m = ceil(2^(31+l) / d) the error m d - 2^(31+l) is
-// below 2^l, so that n times it stays below 2^(31+l)
-struct FastDiv {
-    unsigned m, s, d;
-};
-FastDiv fast_div(unsigned d) {
-    FastDiv f{0, 0, d};
-    if (d <= 1) return f;
-    unsigned l = 1;
-    while ((1ull << l) < d) ++l;
-    f.m = (unsigned)(((1ull << (31 + l)) + d - 1) / d);
-    f.s = l - 1;
-    return f;
-}
-__device__ __forceinline__ unsigned div_by(unsigned n, const FastDiv& f) { return f.m ? __umulhi(n, f.m) >> f.s : n; }
-
 struct TapArgs {
     ConvGeom g;           // one group's channels; g.Cs / g.Ks the tensors'
     FastDiv ohw, ow, c8, kw;
@@ -64,21 +48,6 @@ struct TapArgs {
     const float* in_scale;
     float in_half;
 };
-
-__device__ __forceinline__ int tap_quant4(const v4i& f, float scale, float half) {
-    int k[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const float t = __fmul_rn(__int_as_float(f[e]), scale);
-        k[e] = (int)__fadd_rn(t, __builtin_copysignf(half, t));  // toward zero, saturating
-    }
-    const ohip_v2s top = {127, 127}, bot = {-127, -127};
-    ohip_v2s a = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[0], k[1]));
-    ohip_v2s b = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[2], k[3]));
-    a = __builtin_elementwise_max(__builtin_elementwise_min(a, top), bot);
-    b = __builtin_elementwise_max(__builtin_elementwise_min(b, top), bot);
-    return (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x06040200u);
-}
 
 }  // namespace
 
@@ -200,8 +169,8 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
                 if constexpr (INF)
-                    bb[j] = v4i{tap_quant4(bf[d][j][0], in_scale, ta.in_half), tap_quant4(bf[d][j][1], in_scale, ta.in_half),
-                                tap_quant4(bf[d][j][2], in_scale, ta.in_half), tap_quant4(bf[d][j][3], in_scale, ta.in_half)};
+                    bb[j] = v4i{quantize4(bf[d][j][0], in_scale, ta.in_half), quantize4(bf[d][j][1], in_scale, ta.in_half),
+                                quantize4(bf[d][j][2], in_scale, ta.in_half), quantize4(bf[d][j][3], in_scale, ta.in_half)};
                 else
                     bb[j] = v4i{b[d][j][0][0], b[d][j][0][1], b[d][j][1][0], b[d][j][1][1]};
             }

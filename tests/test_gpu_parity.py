@@ -944,6 +944,42 @@ def test_reduction_dealt_to_waves(hip, oracle, config, C, K, kh, s, p, d, g, N, 
 
 
 @pytest.mark.parametrize("config", range(4))
+@pytest.mark.parametrize("C,K,kh,s,p,d,g,N,H,W", [
+    (8, 16, 3, 1, 1, 1, 1, 1, 1, 1),        # one pixel; less than a tile, a pair and a row block
+    (24, 40, 3, 1, 1, 1, 1, 9, 5, 7),       # a tile over several images, odd width
+    (72, 24, 3, 1, 1, 1, 1, 1, 6, 163),     # three ragged column strips; two stages of 5 and 4 octets
+    (16, 72, 5, 1, 2, 1, 1, 2, 19, 82),     # one stage walked by several row blocks, odd columns in front of a strip
+    (32, 8, 5, 2, 0, 1, 1, 2, 40, 33),      # stride 2 without padding
+    (136, 24, 3, 1, 4, 3, 1, 2, 17, 21),    # dilation, padding wider than it, three stages
+    (64, 96, 3, 1, 1, 1, 4, 3, 14, 18),     # groups with a ragged row block
+    (16, 20, 3, 3, 1, 1, 1, 2, 26, 23),     # output channels not a multiple of 8, stride 3
+])
+def test_rows_staged_in_lds(hip, oracle, config, C, K, kh, s, p, d, g, N, H, W):
+    """The kernel on staged input rows, every tile of it, from int8 and from fp32 blobs."""
+    rng = np.random.default_rng(2000 + C + K)
+    x, wq, ws, bias = _rand_problem(rng, C, K, kh, g, N, H, W)
+    geo = dict(stride=s, pad=p, dil=d, groups=g)
+    ogeo = dict(stride=(s, s), pad=(p, p), dil=(d, d), groups=g)
+    xf = (x.astype(np.float32) / 20 + rng.uniform(-0.02, 0.02, x.shape)).astype(np.float32)
+    for src in (x, xf):
+        for act, int8_out in ((1, True), (0, True), (2, False)):
+            if src is xf and int8_out and K % 8:
+                continue  # (the generic epilogue reads int8 only)
+            want = oracle.conv_layer_forward(src, wq, ws, 20.0, bias=bias, top_scale=9.0, int8_out=int8_out, act_type=act,
+                                             act_params=[0.1] if act == 2 else None, **ogeo)
+            out, _ = run_conv(hip, oracle, src, wq, ws, 20.0, bias=bias, top_scale=9.0, act=act, act_p0=0.1,
+                              out_kind=capi.OUT_I8 if int8_out else capi.OUT_F32, tile=(-9, config), **geo)
+            if int8_out:
+                np.testing.assert_array_equal(out, want)
+            else:
+                assert_f32_close(out, want)
+    if g == 1:
+        _, acc_want = oracle.conv_layer_forward(x, wq, ws, 20.0, want_acc=True, int8_out=False, **ogeo)
+        acc, _ = run_conv(hip, oracle, x, wq, ws, 20.0, out_kind=capi.OUT_I32, tile=(-9, config), **geo)
+        np.testing.assert_array_equal(acc, acc_want)
+
+
+@pytest.mark.parametrize("config", range(4))
 @pytest.mark.parametrize("f32in", [False, True])
 def test_reduction_dealt_to_waves_with_sum_and_twin(hip, oracle, config, f32in):
     rng = np.random.default_rng(77)
