@@ -189,6 +189,20 @@ int otter_hip_conv_forward_residual(const otter_hip_conv_t* handle, const void* 
                                     float q_scale, int q_round_mode, void* workspace, size_t workspace_bytes,
                                     void* stream);
 
+/* An int8 convolution with an fp32 result whose only reader is Concat(2 blobs of K channels) -> ChannelShuffle(2 groups)
+ * (Tensor/ConcatLayer.cpp:54-67, Tensor/ChannelShuffleKernel.cpp:19-55), in one launch: the result's channels alternate with
+ * those of `other` (Float4 or Float8, the layer's output shape), which takes the odd channels if other_odd, else the even
+ * ones. The 2 K shuffled channels come in two halves as Float8 blobs (what the two half Crop layers behind it make), or with
+ * `joined` as one blob of 2 K channels in first_half. first_half_q / second_half_q: the quantize_to_int8 of each with q_scale
+ * for the int8 convolutions that read it, Byte8. Any of the four may be NULL: it is not written. Needs an int8 Byte8 input,
+ * K % 8 == 0 and otter_hip_conv_shuffle_launches(...) == 1 (2: the layer and the shuffle are separate calls); refused
+ * otherwise. No workspace. */
+int otter_hip_conv_shuffle_launches(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w);
+int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w,
+                                   const float* other, int other_layout, int other_odd, float* first_half, float* second_half,
+                                   int8_t* first_half_q, int8_t* second_half_q, int joined, float q_scale, int q_round_mode,
+                                   void* stream);
+
 /* A chain of layers that each map an int8 Byte8 blob to an int8 Byte8 blob (consecutive Convolution layers of a
  * Net, Tensor/Net.cpp:413-505 runs them one after the other): out = layer[n-1](... layer[0](in)). The result is what
  * n calls of otter_hip_conv_forward give. The intermediate blobs live in `workspace`

@@ -82,7 +82,7 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_chain_set_min_tiles", "otter_hip_conv_block_launches", "otter_hip_conv_block_workspace_bytes",
            "otter_hip_conv_block_forward", "otter_hip_conv_block_set_plan", "otter_hip_conv_block_set_always", "otter_hip_conv_block_set_pair",
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
-           "otter_hip_conv_block_plan"]
+           "otter_hip_conv_block_plan", "otter_hip_conv_shuffle_launches", "otter_hip_conv_forward_shuffle"]
 
 
 def load_cdll():
@@ -401,6 +401,27 @@ class Conv:
         self.L._check(self.L.lib.otter_hip_conv_forward_static(
             self.h, self.L.ptr(x), in_layout, n, h, w, self.L.ptr(out), out_layout, self.L.stream()))
         return out
+
+    def shuffle_launches(self, in_layout, n, h, w):
+        return self.L.lib.otter_hip_conv_shuffle_launches(self.h, in_layout, n, h, w)
+
+    def forward_shuffle(self, x, n, h, w, other, other_layout, other_odd=False, joined=False, q_scale=None,
+                        q_round_mode=ROUND_SSE, whole=True):
+        """The layer and the Concat -> ChannelShuffle(2) with `other` behind it (otter_hip_conv_forward_shuffle). Returns
+        (first half, second half, their Byte8 quantizations), flat, None where not made; joined: (blob, None, q, None)."""
+        oh, ow = self.out_hw(h, w)
+        count = n * self.K * oh * ow * (2 if joined else 1)
+
+        def new(want, dtype):
+            return self.L.empty(count, dtype) if want else None
+
+        out = [new(whole, np.float32), new(whole and not joined, np.float32), new(q_scale is not None, np.int8),
+               new(q_scale is not None and not joined, np.int8)]
+        self.L._check(self.L.lib.otter_hip_conv_forward_shuffle(
+            self.h, self.L.ptr(x), I8_P8, n, h, w, self.L.ptr(other), other_layout, int(other_odd),
+            *[self.L.ptr(t) if t is not None else None for t in out], int(joined), C.c_float(q_scale or 0.0), q_round_mode,
+            self.L.stream()))
+        return tuple(out)
 
     def forward_twin(self, x, in_layout, n, h, w, q_scale, q_round_mode, out_layout=None):
         """fp32 result and its Byte8 quantization for the int8 convolutions that read it (otter_hip_conv_forward_twin)"""

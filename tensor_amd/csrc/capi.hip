@@ -1375,6 +1375,69 @@ int otter_hip_global_avgpool(const float* src, int src_layout, int n, int c, int
 
 // ---- a convolution with an fp32 result and the global average pooling that is its only reader ----------------------
 
+// ---- a layer and the Concat -> ChannelShuffle(2) behind it -------------------------------------------------------------
+
+// The kernels that carry the shuffled epilogue, for an int8 Byte8 input: conv_tap_kernel and the implicit-GEMM kernel, as the
+// plain layer would choose between them. The other families' layers (depthwise, LDS-halo, streamed) stay two launches.
+static AltKernel shuffle_kernel(const otter_hip_conv* h, int in_layout, const ConvGeom& g, const Epilogue& ep, int* config, bool* ok) {
+    *ok = false;
+    if (in_layout != OTTER_HIP_I8_P8 || h->d.out_kind != OTTER_HIP_OUT_F32 || h->c_pad || g.groups != 1 || g.K % 8) return ALT_NONE;
+    if (pick_epilogue(ep, g.K) != EPI_F32_P4) return ALT_NONE;
+    const int kind = pick_kernel(h, in_layout, g, ep);
+    const AltKernel alt = alt_kernel(h, g, ep, false, kind, true, config);
+    *ok = alt == ALT_TAP || kind == 1;
+    return alt;
+}
+
+int otter_hip_conv_shuffle_launches(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w) {
+    if (!h || !valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_shuffle_launches: bad argument");
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_shuffle_launches: empty output");
+    int config;
+    bool ok;
+    shuffle_kernel(h, in_layout, g, make_epilogue(h, OTTER_HIP_F32_P4), &config, &ok);
+    return ok ? 1 : 2;
+}
+
+int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w,
+                                   const float* other, int other_layout, int other_odd, float* first_half, float* second_half,
+                                   int8_t* first_half_q, int8_t* second_half_q, int joined, float q_scale, int q_round_mode,
+                                   void* stream_) {
+    if (!h || !in || !other) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_shuffle: null");
+    if (!valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_shuffle: bad argument");
+    if (other_layout != OTTER_HIP_F32_P4 && other_layout != OTTER_HIP_F32_P8)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_shuffle: the other blob must be Float4 or Float8");
+    if (joined && (second_half || second_half_q))
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_shuffle: a joined result is one blob");
+    if ((first_half_q || second_half_q) && q_round_mode != OTTER_HIP_ROUND_EXACT && q_round_mode != OTTER_HIP_ROUND_SSE)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_shuffle: unknown rounding mode");
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_shuffle: empty output");
+    if ((size_t)n * g.C * in_h * in_w >= (1ull << 31) || (size_t)n * g.K * 2 * g.OH * g.OW >= (1ull << 31))
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: tensor exceeds 2^31 elements");
+    Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
+    int config;
+    bool ok;
+    const AltKernel alt = shuffle_kernel(h, in_layout, g, ep, &config, &ok);
+    if (!ok) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: not a single launch (otter_hip_conv_shuffle_launches)");
+    if (n == 0) return OTTER_HIP_OK;
+    const size_t half = (size_t)g.K * g.OH * g.OW;  // elements of one half of one image
+    ep.other = other, ep.other_pack = layout_pack(other_layout), ep.other_odd = other_odd != 0;
+    ep.twin_scale = q_scale, ep.twin_half = q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+    ep.sh_image = joined ? 2 * half : half;
+    ep.sh_out0 = first_half, ep.sh_q0 = first_half_q;
+    ep.sh_out1 = joined ? (first_half ? first_half + half : nullptr) : second_half;
+    ep.sh_q1 = joined ? (first_half_q ? first_half_q + half : nullptr) : second_half_q;
+    if (alt == ALT_TAP)
+        OHIP_CHECK(run_conv_tap(in, false, h->w_tap, nullptr, g, ep, config, h->in_scale, h->d.in_round_mode, (hipStream_t)stream_));
+    else
+        OHIP_CHECK(run_conv_igemm((const int8_t*)in, h->w_igemm, nullptr, g, ep, h->force_tm > 0 ? h->force_tm : 0,
+                                  h->force_tm > 0 ? h->force_tn : 0, (hipStream_t)stream_));
+    return OTTER_HIP_OK;
+}
+
 static bool conv_avgpool_one_launch(const otter_hip_conv_t* h, int in_layout, const ConvGeom& g) {
     if (in_layout != OTTER_HIP_I8_P8 || !h->w_igemm || h->c_pad || h->force_tm || h->d.out_kind != OTTER_HIP_OUT_F32) return false;
     return conv_pw_avgpool_applicable(g, make_epilogue(h, otter_hip_conv_default_out_layout(h)));

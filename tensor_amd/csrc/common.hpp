@@ -123,6 +123,17 @@ struct Epilogue {
     // fp32 output only: a blob in the output's layout that is added to the activated result (the Eltwise sum of a
     // residual block; null: none). The twin, if any, is the quantization of the sum. Float4 epilogue only.
     const float* residual = nullptr;
+    // fp32 output only: the layer is one half of Concat -> ChannelShuffle(2) and writes the shuffled blob, its channels
+    // alternating with those of `other` (K channels too, Float4 or Float8: other_pack; null: no shuffle). The 2 K channels are
+    // two halves of K, each an fp32 blob sh_out and a Byte8 blob sh_q (quantized with twin_scale), null where not wanted;
+    // sh_image: elements from one image to the next in all four. Float4 output layout and K % 8 == 0 only.
+    const float* other = nullptr;
+    int other_pack = 0;
+    bool other_odd = false;  // `other` takes the odd channels of the shuffled blob, else the even ones
+    float *sh_out0 = nullptr, *sh_out1 = nullptr;
+    int8_t *sh_q0 = nullptr, *sh_q1 = nullptr;
+    size_t sh_image = 0;
+    bool fused() const { return twin != nullptr || residual != nullptr || other != nullptr; }
 };
 
 // which epilogue code a kernel instance carries
@@ -132,7 +143,8 @@ enum {
     EPI_F32_P4 = 2,
     EPI_I8_P8_NONNEG = 3,
     EPI_F32_P8 = 4,       // depthwise only
-    EPI_F32_P4_FUSED = 5  // implicit GEMM only: EPI_F32_P4 plus the residual addend and / or the int8 twin
+    EPI_F32_P4_FUSED = 5,  // implicit GEMM only: EPI_F32_P4 plus the residual addend and / or the int8 twin
+    EPI_F32_SHUFFLE = 6    // the same kernels: the channels interleaved with another blob's (Epilogue::other)
 };
 
 // The fast epilogues need: activation in {none, ReLU, clip, LeakyReLU with a slope in [0, 1]}, and (I8_P8) int8
@@ -371,6 +383,48 @@ __device__ __forceinline__ ohip_v4i epi4_dequant_f32p4(const Epilogue& ep, const
         r[e] = __float_as_int(v);
     }
     return r;
+}
+
+// Channels ch0 .. ch0 + 7 of one pixel into the shuffled blob: with the same channels of Epilogue::other they are its
+// channels 2 ch0 .. 2 ch0 + 15, two packs of 8 that a lane writes whole (32 bytes fp32, 8 bytes int8 each). Bound by the bytes of
+// the two fp32 blobs; the layer's own result is neither written nor read back. Layer and shuffle as two launches / as one, in the
+// detection network at batch 16: 88 channels @52x52 23 / 14.5 us, 176 @26x26 15.6 / 10.2 us, 352 @13x13 11.8 / 7.5 us.
+template <int LRELU>
+__device__ __forceinline__ void epi8_store_shuffle(const Epilogue& ep, const float* si, const float* bi, const int (&a8)[8], unsigned n,
+                                                   unsigned pix, int ch0, int K, int OHW) {
+    const size_t plane = (size_t)OHW * ep.other_pack;
+    const float* o = ep.other + ((size_t)n * (unsigned)(K / ep.other_pack) + (unsigned)(ch0 / ep.other_pack)) * plane +
+                     (size_t)pix * (unsigned)ep.other_pack;
+    const ohip_v4i x0 = *reinterpret_cast<const ohip_v4i*>(o);
+    const ohip_v4i x1 = *reinterpret_cast<const ohip_v4i*>(o + (ep.other_pack == 8 ? 4 : plane));
+    const ohip_v4i v0 = epi4_dequant_f32p4<LRELU>(ep, si, bi, a8[0], a8[1], a8[2], a8[3]);
+    const ohip_v4i v1 = epi4_dequant_f32p4<LRELU>(ep, si + 4, bi + 4, a8[4], a8[5], a8[6], a8[7]);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const ohip_v4i x = h ? x1 : x0, v = h ? v1 : v0;
+        const ohip_v4i even = ep.other_odd ? v : x, odd = ep.other_odd ? x : v;  // wave-uniform
+        const int f[8] = {even[0], odd[0], even[1], odd[1], even[2], odd[2], even[3], odd[3]};
+        const int pack = ch0 / 4 + h, half = K / 8;  // pack of the 2 K channels, packs in each half
+        const bool second = pack >= half;
+        const size_t e = (size_t)n * ep.sh_image + ((size_t)(unsigned)(second ? pack - half : pack) * (unsigned)OHW + pix) * 8;
+        float* out = second ? ep.sh_out1 : ep.sh_out0;
+        int8_t* q = second ? ep.sh_q1 : ep.sh_q0;
+        if (out != nullptr) {
+            const ohip_v4i lo = {f[0], f[1], f[2], f[3]}, hi = {f[4], f[5], f[6], f[7]};
+            *reinterpret_cast<ohip_v4i*>(out + e) = lo;
+            *reinterpret_cast<ohip_v4i*>(out + e + 4) = hi;
+        }
+        if (q != nullptr) {
+            ohip_v2i pk = {0, 0};
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const float t = __fmul_rn(__int_as_float(f[b]), ep.twin_scale);
+                const int k = (int)__fadd_rn(t, __builtin_copysignf(ep.twin_half, t));
+                pk[b / 4] |= (min(max(k, -127), 127) & 0xff) << (8 * (b % 4));
+            }
+            *reinterpret_cast<ohip_v2i*>(q + e) = pk;
+        }
+    }
 }
 
 // dequantize (+clamp activation) 4 channels and store one Float4 element. FUSED: first add the residual blob's element

@@ -299,18 +299,20 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
     unsigned n0, pix0;
     locate((unsigned)(wn * (TN / WN) + (lane & 15)), n0, pix0);
     const bool wide = (unsigned)OHW >= 16u * FN;  // then a column is at most one image further than the first
-    if constexpr (EPI == EPI_F32_P4 || EPI == EPI_F32_P4_FUSED || EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
+    if constexpr (EPI == EPI_F32_P4 || EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_SHUFFLE || EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
         // Packed outputs. A lane's stores differ by a column offset (image, pixel) and a row
         // offset (channel group): each computed once, one 64-bit addition per store. LeakyReLU is decided once, in
         // front of the unrolled loops, not per value.
         constexpr bool FUSED = EPI == EPI_F32_P4_FUSED;  // plus the residual addend and / or the int8 twin
-        constexpr bool F32 = EPI == EPI_F32_P4 || FUSED;
+        constexpr bool SHUF = EPI == EPI_F32_SHUFFLE;    // interleaved with another blob's channels
+        constexpr bool F32 = EPI == EPI_F32_P4 || FUSED || SHUF;
         constexpr int EB = F32 ? 16 : 8;       // bytes of one (pixel, channel group) element
         constexpr int CG = F32 ? 4 : 8;        // channels per group
         const size_t plane = (size_t)OHW * EB;  // one channel group of one image
         const size_t image = plane * (size_t)(Ks / CG);
         size_t col_ofs[FN];
         unsigned col_twin[FUSED ? FN : 1];  // the same for the Byte8 twin (below 2 GiB)
+        unsigned col_n[SHUF ? FN : 1], col_pix[SHUF ? FN : 1];
         bool col_ok[FN];
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
@@ -324,6 +326,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
             }
             col_ok[j] = gpo < total_pix;
             col_ofs[j] = (size_t)nn * image + (size_t)pp * EB;
+            if constexpr (SHUF) col_n[j] = nn, col_pix[j] = pp;
             if constexpr (FUSED) col_twin[j] = (nn * (unsigned)(Ks / 8) * (unsigned)OHW + pp) * 8u;
         }
         auto rows = [&](auto lrelu_c) {
@@ -347,7 +350,9 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
                     }
                     if (ch_ok && col_ok[j]) {
                         char* o = row + col_ofs[j];
-                        if constexpr (FUSED) {
+                        if constexpr (SHUF) {
+                            epi8_store_shuffle<LRELU ? 1 : 0>(ep, prm.si, prm.bi, a8, col_n[j], col_pix[j], ch0, g.K, OHW);
+                        } else if constexpr (FUSED) {
                             const size_t elem = (row_ofs + col_ofs[j]) >> 2;  // in floats, for the result and the addend
                             ohip_v2i tw = {0, 0};
                             tw[0] = (int)epi4_store_f32p4<true, LRELU ? 1 : 0>((float*)out, ep, prm.si, prm.bi, elem, a8[0], a8[1],
@@ -503,7 +508,8 @@ static hipError_t launch_igemm_f32in(const float* x, const int8_t* wpk, void* ou
     case EPI_I8_P8: OHIP_IGF(EPI_I8_P8); break;
     case EPI_I8_P8_NONNEG: OHIP_IGF(EPI_I8_P8_NONNEG); break;
     case EPI_F32_P4:
-        if (ep.twin != nullptr || ep.residual != nullptr) OHIP_IGF(EPI_F32_P4_FUSED);
+        if (ep.other != nullptr) return hipErrorInvalidValue;
+        if (ep.fused()) OHIP_IGF(EPI_F32_P4_FUSED);
         else OHIP_IGF(EPI_F32_P4);
         break;
     default: return hipErrorInvalidValue;
@@ -540,7 +546,8 @@ static hipError_t launch_igemm(const int8_t* x, const int8_t* wpk, void* out, co
     case EPI_I8_P8_NONNEG:
         return launch_igemm_e<TM, TN, WM, WN, EPI_I8_P8_NONNEG>(x, wpk, out, g, ep, stage, stream);
     case EPI_F32_P4:
-        if (ep.twin != nullptr || ep.residual != nullptr)
+        if (ep.other != nullptr) return launch_igemm_e<TM, TN, WM, WN, EPI_F32_SHUFFLE>(x, wpk, out, g, ep, stage, stream);
+        if (ep.fused())
             return launch_igemm_e<TM, TN, WM, WN, EPI_F32_P4_FUSED>(x, wpk, out, g, ep, stage, stream);
         return launch_igemm_e<TM, TN, WM, WN, EPI_F32_P4>(x, wpk, out, g, ep, stage, stream);
     default:
@@ -587,7 +594,7 @@ bool igemm_grouped_applicable(const ConvGeom& g, const Epilogue& ep) {
     if (cg % 8) return false;
     const int epi = pick_epilogue(ep, kg);
     if (epi == EPI_GENERIC) return false;
-    if (ep.twin != nullptr || ep.residual != nullptr) return false;
+    if (ep.fused()) return false;
     return (epi == EPI_F32_P4) ? kg % 4 == 0 : kg % 8 == 0;
 }
 

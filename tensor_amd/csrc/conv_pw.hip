@@ -437,7 +437,7 @@ static int pw_f32in_pairs_per_round(int cgs, int pairs) { return std::max(1, std
 bool conv_pw_f32in_applicable(const ConvGeom& g, const Epilogue& ep) {
     if (g.groups != 1 || g.kh != 1 || g.kw != 1 || g.sh != 1 || g.sw != 1 || g.ph != 0 || g.pw != 0) return false;
     if (g.Cs || g.Ks || g.C % 8 || g.C > 64 * PW_MAX_CG || g.N < 1 || g.N > 65535) return false;
-    if (ep.twin != nullptr || ep.residual != nullptr) return false;
+    if (ep.fused()) return false;
     const int epi = pick_epilogue(ep, g.K);
     if (epi != EPI_I8_P8 && epi != EPI_I8_P8_NONNEG && epi != EPI_F32_P4) return false;
     if (g.K % (epi == EPI_F32_P4 ? 4 : 8)) return false;

@@ -356,7 +356,7 @@ static bool rows_plan(const ConvGeom& g_in, int fn, RowsArgs* ra, size_t* lds) {
 
 bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
     if (g.OH < 1 || g.OW < 1 || g.C % g.groups || g.K % g.groups || g.kh * g.kw < 2 || g.kh * g.kw > 25 || g.groups > 65535) return false;
-    if ((g.C / g.groups) % 8 || ep.twin != nullptr || ep.residual != nullptr) return false;
+    if ((g.C / g.groups) % 8 || ep.fused()) return false;
     const int epi = pick_epilogue(ep, g.K / g.groups);
     if (epi == EPI_GENERIC && (g.groups > 1 || f32in)) return false;
     return (size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1) < ((size_t)1 << 31) && (size_t)g.N * g.K * g.OH * g.OW < ((size_t)1 << 31);

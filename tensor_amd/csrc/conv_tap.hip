@@ -231,6 +231,9 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
             if constexpr (EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
                 const size_t o = ((size_t)(n * (unsigned)(Ks / 8) + ch / 8) * (unsigned)OHW + pix) * 8;
                 epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm, o, a8);
+            } else if constexpr (EPI == EPI_F32_SHUFFLE) {
+                if (ep.lrelu) epi8_store_shuffle<1>(ep, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
+                else epi8_store_shuffle<0>(ep, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
             } else {
                 constexpr bool FUSED = EPI == EPI_F32_P4_FUSED;
                 const size_t e = ((size_t)(n * (unsigned)(Ks / 4) + ch / 4) * (unsigned)OHW + pix) * 4;
@@ -296,9 +299,9 @@ bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
     const int cg = g.C / g.groups, kg = g.K / g.groups;
     if (cg % 8 || g.kh * g.kw > TAP_MAX_TAPS || tap_pairs(cg, g.kh, g.kw) > TAP_MAX_PAIRS || g.groups > 65535) return false;
     const int epi = pick_epilogue(ep, kg);
-    if (g.groups > 1 && (epi == EPI_GENERIC || ep.twin != nullptr || ep.residual != nullptr)) return false;
-    if ((ep.twin != nullptr || ep.residual != nullptr) && epi != EPI_F32_P4) return false;
-    if (f32in && epi == EPI_GENERIC) return false;
+    if (g.groups > 1 && (epi == EPI_GENERIC || ep.fused())) return false;
+    if (ep.fused() && epi != EPI_F32_P4) return false;
+    if (f32in && (epi == EPI_GENERIC || ep.other != nullptr)) return false;
     return (size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1) < ((size_t)1 << 31);  // 32-bit byte offsets
 }
 
@@ -384,17 +387,18 @@ hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out,
     const long px = (long)g.N * g.OH * g.OW, per = 16l * c.fn * c.wn;
     ta.n_pix_tiles = (int)((px + per - 1) / per);
     int epi = pick_epilogue(ep, g.K);
-    if (epi == EPI_F32_P4 && (ep.twin != nullptr || ep.residual != nullptr)) epi = EPI_F32_P4_FUSED;
+    if (epi == EPI_F32_P4 && ep.fused()) epi = ep.other != nullptr ? EPI_F32_SHUFFLE : EPI_F32_P4_FUSED;
 #define OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, E_)                                                                           \
     if (config == I_ && epi == E_) {                                                                                        \
         if (!f32in) return launch_tap<FM_, FN_, WK_, WN_, D_, E_, false>(x, wpk, out, ta, ep, g_in.groups, stream);         \
-        if constexpr (E_ != EPI_GENERIC && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g_in.groups, stream); \
+        if constexpr (E_ != EPI_GENERIC && E_ != EPI_F32_SHUFFLE && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g_in.groups, stream); \
     }
 #define OHIP_TAP(I_, FM_, FN_, WK_, WN_, D_)                 \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8)         \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8_NONNEG)  \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4)        \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4_FUSED)  \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_SHUFFLE)   \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_GENERIC)
     OHIP_TAP(0, 2, 1, 8, 1, 4)
     OHIP_TAP(1, 2, 2, 4, 1, 4)

@@ -780,6 +780,51 @@ int ConvolutionLayer::forward_int8(const Tensor& bottom_in, const Tensor* shortc
     return 0;
 }
 
+int ConvolutionLayer::forward_shuffle(const Tensor& bottom_in, const Tensor& other, bool other_odd, bool joined, float q_scale,
+                                      int q_round, Tensor& first, Tensor& second, const NetOption& opt) const {
+    if (!handle_ || !int8_scale_term || int8_scale_term > 100 || force_out_layout >= 0 || !opt.use_packing_layout) return 1;
+    if (!bottom_in.defined() || bottom_in.dim() != 4 || out_channels % 8) return 1;
+    Tensor bottom = bottom_in, twin;
+    if (base_of(bottom_in.scalar_type()) == ScalarType::Float && in_channels % 8 == 0 &&
+        bottom_in.quantized_twin(bottom_blob_int8_scales.data_ptr<float>()[0], input_round_mode(opt), twin))
+        bottom = twin;
+    if (bottom.scalar_type() != ScalarType::Byte8 || bottom.channels() != in_channels) return 1;
+    const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3);
+    int oh = 0, ow = 0;
+    if (otter_hip_conv_output_shape(handle_, H, W, &oh, &ow)) return 1;
+    if (!other.defined() || other.dim() != 4 || base_of(other.scalar_type()) != ScalarType::Float || other.elempack() == 1 ||
+        other.channels() != out_channels || other.size(0) != N || other.size(2) != oh || other.size(3) != ow)
+        return 1;
+    if (otter_hip_conv_shuffle_launches(handle_, OTTER_HIP_I8_P8, N, H, W) != 1) return 1;
+    try {
+        const std::vector<int64_t> sizes = {N, (joined ? 2 : 1) * out_channels / 8, oh, ow};
+        first = Tensor::empty_device(sizes, ScalarType::Float8);
+        if (!joined) second = Tensor::empty_device(sizes, ScalarType::Float8);
+        Tensor q;
+        if (q_scale > 0.f) q = Tensor::empty_device(sizes, ScalarType::Byte8);
+        int8_t* qp = q.defined() ? (int8_t*)q.device_ptr() : nullptr;
+        const int rc = otter_hip_conv_forward_shuffle(
+            handle_, bottom.device_ptr(), OTTER_HIP_I8_P8, N, H, W, (const float*)other.device_ptr(), hip_layout_of(other.scalar_type()),
+            other_odd, (float*)first.device_ptr(), joined ? nullptr : (float*)second.device_ptr(), joined ? qp : nullptr,
+            joined ? nullptr : qp, joined, q_scale, q_round, nullptr);
+        if (rc) return rc;
+        first.mark_device_written();
+        if (!joined) second.mark_device_written();
+        if (q.defined()) {
+            q.mark_device_written();
+            (joined ? first : second).attach_quantized(q, q_scale, q_round);
+        }
+    } catch (const Error&) {
+        return -100;
+    }
+    return 0;
+}
+
+int ConvolutionLayer::block_launches(const ConvolutionLayer* e, const ConvolutionLayer* d, const ConvolutionLayer* p, int n, int h,
+                                     int w) {
+    return e->handle_ && d->handle_ && p->handle_ ? otter_hip_conv_block_launches(e->handle_, d->handle_, p->handle_, n, h, w) : 3;
+}
+
 static std::atomic<long> g_chain_forwards{0};
 long ConvolutionLayer::chain_forward_count() { return g_chain_forwards.load(); }
 
@@ -1908,6 +1953,16 @@ void Net::plan_fused_quantize() const {
         const int si = sole_reader(cat->tops[0]);
         const auto* sh = si < 0 ? nullptr : dynamic_cast<const ChannelShuffleLayer*>(layers_[si]);
         if (!sh || sh->groups() != 2) continue;
+        // the later of the two layers in front, if it is an int8 convolution with an fp32 result: the other's is ready by then
+        int conv = -1, conv_k = 0;
+        for (int k = 0; k < 2 && cat->bottoms[0] != cat->bottoms[1]; ++k) {
+            const int b = cat->bottoms[k], pi = blobs_[b].producer;
+            const auto* pc = pi < 0 ? nullptr : dynamic_cast<const ConvolutionLayer*>(layers_[pi]);
+            if (!pc || !pc->int8_scale_term || pc->int8_scale_term > 100 || pc->force_out_layout >= 0 || pc->bottoms.size() != 1) continue;
+            if (blobs_[b].consumers.size() == 1 && pi > conv) conv = pi, conv_k = k;
+        }
+        const ShuffleUnit whole{(int)ci, si, -1, -1, sh->fuse_scale, sh->fuse_round, conv, conv_k};
+        if (conv >= 0) shuffle_units_[si] = whole;
         int sp = sole_reader(sh->tops[0]);
         if (sp < 0 || layers_[sp]->type() != "Split" || layers_[sp]->tops.size() != 2) continue;
         int lo = -1, hi = -1;
@@ -1934,7 +1989,7 @@ void Net::plan_fused_quantize() const {
             if (hs != 0.f && (sc != hs || r != hr)) agree = false;
             hs = sc, hr = r;
         }
-        const ShuffleUnit u{(int)ci, si, lo, hi, agree && hs > 0.f ? hs : 0.f, hr};
+        const ShuffleUnit u{(int)ci, si, lo, hi, agree && hs > 0.f ? hs : 0.f, hr, conv, conv_k};
         shuffle_units_[lo] = u;
         shuffle_units_[hi] = u;
     }
@@ -2068,9 +2123,53 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
     return 0;
 }
 
+// The unit in the launch of the convolution in front of it. Returns 1 when the blobs at hand do not allow it.
+int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const {
+    const auto* conv = static_cast<const ConvolutionLayer*>(layers_[u.conv]);
+    const int other = layers_[u.concat]->bottoms[1 - u.conv_k], in_blob = conv->bottoms[0];
+    const auto bu = block_units_.find(u.conv);
+    if (bu != block_units_.end() && !blobs[layers_[bu->second.expand]->tops[0]].defined() && !blobs[in_blob].defined()) {
+        // the layer may be the last of an inverted-residual block: the block's shared launch saves more
+        const auto* ec = static_cast<const ConvolutionLayer*>(layers_[bu->second.expand]);
+        const int b = ec->bottoms[0];
+        if (!blobs[b].defined()) {
+            const int rc = forward_layer(blobs_[b].producer, blobs, opt);
+            if (rc) return rc;
+        }
+        if (blobs[b].dim() == 4 &&
+            ConvolutionLayer::block_launches(ec, static_cast<const ConvolutionLayer*>(layers_[bu->second.depthwise]), conv,
+                                             (int)blobs[b].size(0), (int)blobs[b].size(2), (int)blobs[b].size(3)) < 3)
+            return 1;
+    }
+    for (int b : {other, in_blob})
+        if (!blobs[b].defined()) {
+            const int rc = forward_layer(blobs_[b].producer, blobs, opt);
+            if (rc) return rc;
+        }
+    const bool joined = u.crop_lo < 0;
+    Tensor first, second;
+    const int rc = conv->forward_shuffle(blobs[in_blob], blobs[other], u.conv_k == 0, joined, u.hi_scale, u.hi_round, first, second, opt);
+    if (rc) return rc;
+    if (joined) {
+        blobs[layers_[u.shuffle]->tops[0]] = first;
+    } else {
+        blobs[layers_[u.crop_lo]->tops[0]] = first;
+        blobs[layers_[u.crop_hi]->tops[0]] = second;
+    }
+    if (opt.lightmode)
+        for (int b : {other, in_blob})
+            if (blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+    return 0;
+}
+
 // One kernel for a whole unit (otter_hip_shuffle2_split) when the blobs between its ends are not wanted by anybody else.
 int Net::forward_shuffle_unit(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const {
     const Layer* cat = layers_[u.concat];
+    if (u.conv >= 0 && !blobs[layers_[u.conv]->tops[0]].defined()) {
+        const int rc = forward_conv_shuffle(u, blobs, opt);
+        if (rc <= 0) return rc;
+    }
+    if (u.crop_lo < 0) return 1;
     for (int b : cat->bottoms)
         if (!blobs[b].defined()) {
             const int rc = forward_layer(blobs_[b].producer, blobs, opt);

@@ -237,6 +237,14 @@ public:
     // otter_hip_conv_forward_avgpool, when that is one launch for this input; `mean` is [N, K, 1, 1]. Returns 1, and does
     // nothing, otherwise (the caller then runs the two layers one after the other).
     int forward_avgpool(const Tensor& bottom_blob, Tensor& mean, const NetOption& opt) const;
+    // This layer (fp32 result) and the Concat with `other` -> ChannelShuffle(2) that is its only reader, in one launch
+    // (otter_hip_conv_forward_shuffle): the shuffled channels' two halves, or with `joined` the whole blob in `first`; q_scale
+    // > 0 also quantizes the second half (joined: the blob). Returns 1, and does nothing, when that is not one launch here.
+    int forward_shuffle(const Tensor& bottom_blob, const Tensor& other, bool other_odd, bool joined, float q_scale, int q_round,
+                        Tensor& first, Tensor& second, const NetOption& opt) const;
+    // what otter_hip_conv_block_launches says of the three layers on an input of this size
+    static int block_launches(const ConvolutionLayer* expand, const ConvolutionLayer* depthwise, const ConvolutionLayer* project,
+                              int n, int h, int w);
     // A run of int8 -> int8 convolution layers, each reading the one before, as one call of the C ABI's chain entry point
     // when that takes the run as a single launch (otter_hip_conv_chain_launches == 1); `top` is the last layer's blob,
     // the blobs in between are not made. Returns 1, and does nothing, for any other run or input.
@@ -329,13 +337,17 @@ private:
     std::vector<LayerOption> layer_options_;
     mutable bool planned_ = false;
     // Concat(a, b) -> ChannelShuffle(2) -> Crop(first half) + Crop(second half), found by the plan: either Crop layer's
-    // index -> the unit; forward_layer runs the whole unit in one kernel when none of its inner blobs exists yet
+    // index -> the unit; forward_layer runs the whole unit in one kernel when none of its inner blobs exists yet. Without
+    // the Crops (-1) the unit is the ChannelShuffle layer's and needs a convolution to run in.
     struct ShuffleUnit {
         int concat, shuffle, crop_lo, crop_hi;
         float hi_scale;  // > 0: the second half is read by int8 convolutions with this input scale ...
         int hi_round;    // ... and this rounding primitive: quantize it on the way
+        int conv;        // the int8 convolution whose fp32 result is bottom conv_k of the Concat and read by nothing else, or -1
+        int conv_k;
     };
     mutable std::map<int, ShuffleUnit> shuffle_units_;
+    int forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_shuffle_unit(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const;
     // The tail of a residual block, found by the plan: an Eltwise sum of two blobs, one of them the fp32 result of an
     // int8 convolution that nothing else reads. Eltwise layer's index -> the unit; forward_layer runs convolution and

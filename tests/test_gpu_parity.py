@@ -642,6 +642,54 @@ def test_forward_residual_equals_forward_then_add(hip, oracle, C, K, k, s, p, g,
     conv.close()
 
 
+@pytest.mark.parametrize("C,K,k,s,N,H,W,act,tile", [
+    (88, 88, 1, 1, 3, 14, 13, 2, 0),      # a branch's last layer (LeakyReLU), the automatic choice
+    (88, 88, 1, 1, 2, 26, 26, 2, -4),     # the same on the implicit-GEMM kernel
+    (176, 176, 1, 1, 1, 13, 13, 0, 0),
+    (24, 8, 1, 1, 2, 5, 7, 1, 0),         # one pack each: the halves split inside a lane's two packs
+    (24, 40, 1, 1, 2, 9, 5, 3, -4),       # an odd number of packs in each half
+    (48, 136, 1, 1, 1, 1, 1, 0, -4),      # one pixel
+    (16, 24, 3, 2, 3, 11, 9, 1, -8),      # k x k with a stride, forced onto conv_tap_kernel
+    (16, 24, 5, 1, 1, 7, 40, 2, -4),
+    (64, 520, 1, 1, 5, 7, 7, 1, -4),      # wide row tiles
+])
+@pytest.mark.parametrize("other_pack,other_odd,joined", [(8, False, False), (4, True, False), (4, False, True), (8, True, True)])
+def test_forward_shuffle_equals_forward_concat_shuffle(hip, oracle, C, K, k, s, N, H, W, act, tile, other_pack, other_odd, joined):
+    """otter_hip_conv_forward_shuffle: the channels of otter_hip_conv_forward's blob and of the other one in turn, bit for bit,
+    and the oracle's quantize_to_int8 of them; blobs that are not asked for are not needed for the rest."""
+    rng = np.random.default_rng(C * 3 + K + k + act)
+    x, wq, ws, bias = _rand_problem(rng, C, K, k, 1, N, H, W)
+    conv = hip.conv(wq=wq, scale_in=host_scale_in(ws, 20.0), bias=bias, in_scale=20.0, out_scale=None, stride=(s, s),
+                    pad=(k // 2, k // 2), dil=(1, 1), groups=1, act=act, act_p0=0.1, out_kind=capi.OUT_F32, out_round=0,
+                    in_round=oracle.quantize_round_mode(C, True))
+    xd = hip.to_device(capi.pack_np(x, 8))
+    if tile:
+        conv.set_tile(tile, 0)
+    oh, ow = conv.out_hw(H, W)
+    plain = capi.unpack_np(conv.forward(xd, capi.I8_P8, N, H, W, capi.F32_P4).cpu().numpy(), 4, (N, K, oh, ow))
+    other = (rng.normal(0, 1, plain.shape) * np.abs(plain).mean()).astype(np.float32)
+    pair = (plain, other) if other_odd else (other, plain)
+    want = np.stack(pair, 2).reshape(N, 2 * K, oh, ow)
+    q_scale = 127.0 / float(np.abs(want).max()) * 1.3  # some values saturate
+    want_q = oracle.quantize(want, np.float32(q_scale), capi.ROUND_SSE)
+    od = hip.to_device(capi.pack_np(other, other_pack))
+    layout = capi.F32_P8 if other_pack == 8 else capi.F32_P4
+    assert conv.shuffle_launches(capi.I8_P8, N, H, W) == 1
+    for whole in (True, False):
+        out = conv.forward_shuffle(xd, N, H, W, od, layout, other_odd, joined, q_scale, capi.ROUND_SSE, whole=whole)
+        hip.torch.cuda.synchronize()
+        parts = [slice(0, 2 * K)] if joined else [slice(0, K), slice(K, 2 * K)]
+        for i, part in enumerate(parts):
+            shape = want[:, part].shape
+            if whole:
+                got = capi.unpack_np(out[i].cpu().numpy(), 8, shape)
+                np.testing.assert_array_equal(got.view(np.uint32), np.ascontiguousarray(want[:, part]).view(np.uint32))
+            np.testing.assert_array_equal(capi.unpack_np(out[2 + i].cpu().numpy(), 8, shape), want_q[:, part])
+    with pytest.raises(capi.HipError):
+        conv.forward_shuffle(xd, N, H, W, od, capi.F32, other_odd, joined)  # an unpacked other blob
+    conv.close()
+
+
 @pytest.mark.parametrize("s", [1, 2])
 def test_depthwise3x3_from_an_fp32_blob_in_one_launch(hip, oracle, s):
     """A depthwise 3x3 layer on an fp32 Float8 blob of 17..128 columns runs quantize_to_int8 and the convolution as ONE
