@@ -195,13 +195,22 @@ int otter_hip_conv_forward_residual(const otter_hip_conv_t* handle, const void* 
  * ones. The 2 K shuffled channels come in two halves as Float8 blobs (what the two half Crop layers behind it make), or with
  * `joined` as one blob of 2 K channels in first_half. first_half_q / second_half_q: the quantize_to_int8 of each with q_scale
  * for the int8 convolutions that read it, Byte8. Any of the four may be NULL: it is not written. Needs an int8 Byte8 input,
- * K % 8 == 0 and otter_hip_conv_shuffle_launches(...) == 1 (2: the layer and the shuffle are separate calls); refused
+ * K % 8 == 0 and otter_hip_conv_join_launches(...) == 1 (2: the layer and the shuffle are separate calls); refused
  * otherwise. No workspace. */
-int otter_hip_conv_shuffle_launches(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w);
+int otter_hip_conv_join_launches(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w);
 int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w,
                                    const float* other, int other_layout, int other_odd, float* first_half, float* second_half,
                                    int8_t* first_half_q, int8_t* second_half_q, int joined, float q_scale, int q_round_mode,
                                    void* stream);
+
+/* otter_hip_conv_forward_residual where the shortcut is Concat(part0, part1) that nothing else reads (Tensor/ConcatLayer.cpp:54-67,
+ * Tensor/ShortCutLayer.cpp): out (Float4) = activation(convolution) + [part0 | part1], one launch, the concatenated blob not made.
+ * part0 has part0_channels channels, part1 the other K - part0_channels; Float4 or Float8 each. out_q (or NULL) as there.
+ * Needs an int8 Byte8 input, whole channel octets throughout and otter_hip_conv_join_launches(...) == 1. No workspace. */
+int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w,
+                                           const float* part0, int part0_layout, int part0_channels, const float* part1,
+                                           int part1_layout, float* out, int8_t* out_q, float q_scale, int q_round_mode,
+                                           void* stream);
 
 /* A chain of layers that each map an int8 Byte8 blob to an int8 Byte8 blob (consecutive Convolution layers of a
  * Net, Tensor/Net.cpp:413-505 runs them one after the other): out = layer[n-1](... layer[0](in)). The result is what

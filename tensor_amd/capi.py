@@ -82,7 +82,8 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_chain_set_min_tiles", "otter_hip_conv_block_launches", "otter_hip_conv_block_workspace_bytes",
            "otter_hip_conv_block_forward", "otter_hip_conv_block_set_plan", "otter_hip_conv_block_set_always", "otter_hip_conv_block_set_pair",
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
-           "otter_hip_conv_block_plan", "otter_hip_conv_shuffle_launches", "otter_hip_conv_forward_shuffle"]
+           "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
+           "otter_hip_conv_forward_residual_concat"]
 
 
 def load_cdll():
@@ -402,8 +403,8 @@ class Conv:
             self.h, self.L.ptr(x), in_layout, n, h, w, self.L.ptr(out), out_layout, self.L.stream()))
         return out
 
-    def shuffle_launches(self, in_layout, n, h, w):
-        return self.L.lib.otter_hip_conv_shuffle_launches(self.h, in_layout, n, h, w)
+    def join_launches(self, in_layout, n, h, w):
+        return self.L.lib.otter_hip_conv_join_launches(self.h, in_layout, n, h, w)
 
     def forward_shuffle(self, x, n, h, w, other, other_layout, other_odd=False, joined=False, q_scale=None,
                         q_round_mode=ROUND_SSE, whole=True):
@@ -422,6 +423,18 @@ class Conv:
             *[self.L.ptr(t) if t is not None else None for t in out], int(joined), C.c_float(q_scale or 0.0), q_round_mode,
             self.L.stream()))
         return tuple(out)
+
+    def forward_residual_concat(self, x, n, h, w, part0, part0_layout, part0_channels, part1, part1_layout, q_scale=None,
+                                q_round_mode=ROUND_SSE):
+        """activation(convolution) + [part0 | part1] and, with q_scale, its Byte8 quantization
+        (otter_hip_conv_forward_residual_concat). Returns (Float4 sum, q or None)."""
+        oh, ow = self.out_hw(h, w)
+        out = self.L.empty(n * self.K * oh * ow, np.float32)
+        q = self.L.empty(n * self.K * oh * ow, np.int8) if q_scale is not None else None
+        self.L._check(self.L.lib.otter_hip_conv_forward_residual_concat(
+            self.h, self.L.ptr(x), I8_P8, n, h, w, self.L.ptr(part0), part0_layout, part0_channels, self.L.ptr(part1), part1_layout,
+            self.L.ptr(out), self.L.ptr(q) if q is not None else None, C.c_float(q_scale or 0.0), q_round_mode, self.L.stream()))
+        return out, q
 
     def forward_twin(self, x, in_layout, n, h, w, q_scale, q_round_mode, out_layout=None):
         """fp32 result and its Byte8 quantization for the int8 convolutions that read it (otter_hip_conv_forward_twin)"""

@@ -1375,11 +1375,11 @@ int otter_hip_global_avgpool(const float* src, int src_layout, int n, int c, int
 
 // ---- a convolution with an fp32 result and the global average pooling that is its only reader ----------------------
 
-// ---- a layer and the Concat -> ChannelShuffle(2) behind it -------------------------------------------------------------
+// ---- a layer and the Concat -> ChannelShuffle(2), or the sum with a Concat, behind it ----------------------------------
 
-// The kernels that carry the shuffled epilogue, for an int8 Byte8 input: conv_tap_kernel and the implicit-GEMM kernel, as the
+// The kernels that carry these epilogues, for an int8 Byte8 input: conv_tap_kernel and the implicit-GEMM kernel, as the
 // plain layer would choose between them. The other families' layers (depthwise, LDS-halo, streamed) stay two launches.
-static AltKernel shuffle_kernel(const otter_hip_conv* h, int in_layout, const ConvGeom& g, const Epilogue& ep, int* config, bool* ok) {
+static AltKernel join_kernel(const otter_hip_conv* h, int in_layout, const ConvGeom& g, const Epilogue& ep, int* config, bool* ok) {
     *ok = false;
     if (in_layout != OTTER_HIP_I8_P8 || h->d.out_kind != OTTER_HIP_OUT_F32 || h->c_pad || g.groups != 1 || g.K % 8) return ALT_NONE;
     if (pick_epilogue(ep, g.K) != EPI_F32_P4) return ALT_NONE;
@@ -1389,14 +1389,24 @@ static AltKernel shuffle_kernel(const otter_hip_conv* h, int in_layout, const Co
     return alt;
 }
 
-int otter_hip_conv_shuffle_launches(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w) {
+static int join_run(const otter_hip_conv* h, const void* in, void* out, const ConvGeom& g, const Epilogue& ep, AltKernel alt,
+                    int config, hipStream_t stream) {
+    if (alt == ALT_TAP)
+        OHIP_CHECK(run_conv_tap(in, false, h->w_tap, out, g, ep, config, h->in_scale, h->d.in_round_mode, stream));
+    else
+        OHIP_CHECK(run_conv_igemm((const int8_t*)in, h->w_igemm, out, g, ep, h->force_tm > 0 ? h->force_tm : 0,
+                                  h->force_tm > 0 ? h->force_tn : 0, stream));
+    return OTTER_HIP_OK;
+}
+
+int otter_hip_conv_join_launches(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w) {
     if (!h || !valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1)
-        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_shuffle_launches: bad argument");
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_join_launches: bad argument");
     const ConvGeom g = make_geom(h->d, n, in_h, in_w);
-    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_shuffle_launches: empty output");
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_join_launches: empty output");
     int config;
     bool ok;
-    shuffle_kernel(h, in_layout, g, make_epilogue(h, OTTER_HIP_F32_P4), &config, &ok);
+    join_kernel(h, in_layout, g, make_epilogue(h, OTTER_HIP_F32_P4), &config, &ok);
     return ok ? 1 : 2;
 }
 
@@ -1420,8 +1430,8 @@ int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* h, const void* in, in
     Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
     int config;
     bool ok;
-    const AltKernel alt = shuffle_kernel(h, in_layout, g, ep, &config, &ok);
-    if (!ok) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: not a single launch (otter_hip_conv_shuffle_launches)");
+    const AltKernel alt = join_kernel(h, in_layout, g, ep, &config, &ok);
+    if (!ok) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: not a single launch (otter_hip_conv_join_launches)");
     if (n == 0) return OTTER_HIP_OK;
     const size_t half = (size_t)g.K * g.OH * g.OW;  // elements of one half of one image
     ep.other = other, ep.other_pack = layout_pack(other_layout), ep.other_odd = other_odd != 0;
@@ -1430,12 +1440,39 @@ int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* h, const void* in, in
     ep.sh_out0 = first_half, ep.sh_q0 = first_half_q;
     ep.sh_out1 = joined ? (first_half ? first_half + half : nullptr) : second_half;
     ep.sh_q1 = joined ? (first_half_q ? first_half_q + half : nullptr) : second_half_q;
-    if (alt == ALT_TAP)
-        OHIP_CHECK(run_conv_tap(in, false, h->w_tap, nullptr, g, ep, config, h->in_scale, h->d.in_round_mode, (hipStream_t)stream_));
-    else
-        OHIP_CHECK(run_conv_igemm((const int8_t*)in, h->w_igemm, nullptr, g, ep, h->force_tm > 0 ? h->force_tm : 0,
-                                  h->force_tm > 0 ? h->force_tn : 0, (hipStream_t)stream_));
-    return OTTER_HIP_OK;
+    return join_run(h, in, nullptr, g, ep, alt, config, (hipStream_t)stream_);
+}
+
+int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w,
+                                           const float* part0, int part0_layout, int part0_channels, const float* part1,
+                                           int part1_layout, float* out, int8_t* out_q, float q_scale, int q_round_mode, void* stream_) {
+    if (!h || !in || !part0 || !part1 || !out) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: null");
+    if (!valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: bad argument");
+    for (int l : {part0_layout, part1_layout})
+        if (l != OTTER_HIP_F32_P4 && l != OTTER_HIP_F32_P8)
+            return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: the parts must be Float4 or Float8");
+    if (part0_channels < 8 || part0_channels % 8 || part0_channels >= h->d.out_channels)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: parts of whole channel octets expected");
+    if (out_q && q_round_mode != OTTER_HIP_ROUND_EXACT && q_round_mode != OTTER_HIP_ROUND_SSE)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: unknown rounding mode");
+    if (out == part0 || out == part1)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: out must not be a part");
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: empty output");
+    if ((size_t)n * g.C * in_h * in_w >= (1ull << 31) || (size_t)n * g.K * g.OH * g.OW >= (1ull << 31))
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_residual_concat: tensor exceeds 2^31 elements");
+    Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
+    int config;
+    bool ok;
+    const AltKernel alt = join_kernel(h, in_layout, g, ep, &config, &ok);
+    if (!ok)
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_residual_concat: not a single launch (otter_hip_conv_join_launches)");
+    if (n == 0) return OTTER_HIP_OK;
+    ep.residual = part0, ep.residual1 = part1, ep.res_split = part0_channels;
+    ep.res_pack0 = layout_pack(part0_layout), ep.res_pack1 = layout_pack(part1_layout);
+    ep.twin = out_q, ep.twin_scale = q_scale, ep.twin_half = q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+    return join_run(h, in, out, g, ep, alt, config, (hipStream_t)stream_);
 }
 
 static bool conv_avgpool_one_launch(const otter_hip_conv_t* h, int in_layout, const ConvGeom& g) {

@@ -312,7 +312,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
         const size_t image = plane * (size_t)(Ks / CG);
         size_t col_ofs[FN];
         unsigned col_twin[FUSED ? FN : 1];  // the same for the Byte8 twin (below 2 GiB)
-        unsigned col_n[SHUF ? FN : 1], col_pix[SHUF ? FN : 1];
+        unsigned col_n[SHUF || FUSED ? FN : 1], col_pix[SHUF || FUSED ? FN : 1];
         bool col_ok[FN];
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
             }
             col_ok[j] = gpo < total_pix;
             col_ofs[j] = (size_t)nn * image + (size_t)pp * EB;
-            if constexpr (SHUF) col_n[j] = nn, col_pix[j] = pp;
+            if constexpr (SHUF || FUSED) col_n[j] = nn, col_pix[j] = pp;
             if constexpr (FUSED) col_twin[j] = (nn * (unsigned)(Ks / 8) * (unsigned)OHW + pp) * 8u;
         }
         auto rows = [&](auto lrelu_c) {
@@ -354,12 +354,17 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
                             epi8_store_shuffle<LRELU ? 1 : 0>(ep, prm.si, prm.bi, a8, col_n[j], col_pix[j], ch0, g.K, OHW);
                         } else if constexpr (FUSED) {
                             const size_t elem = (row_ofs + col_ofs[j]) >> 2;  // in floats, for the result and the addend
+                            const float *r0 = nullptr, *r1 = nullptr;
+                            if (ep.residual1 != nullptr) {  // wave-uniform
+                                r0 = epi4_residual_at(ep, col_n[j], col_pix[j], ch0, g.K, OHW);
+                                r1 = epi4_residual_at(ep, col_n[j], col_pix[j], ch0 + 4, g.K, OHW);
+                            }
                             ohip_v2i tw = {0, 0};
                             tw[0] = (int)epi4_store_f32p4<true, LRELU ? 1 : 0>((float*)out, ep, prm.si, prm.bi, elem, a8[0], a8[1],
-                                                                              a8[2], a8[3]);
+                                                                              a8[2], a8[3], r0);
                             if (ch0 + 4 < g.K)
                                 tw[1] = (int)epi4_store_f32p4<true, LRELU ? 1 : 0>((float*)out, ep, prm.si + 4, prm.bi + 4,
-                                                                                  elem + (plane >> 2), a8[4], a8[5], a8[6], a8[7]);
+                                                                                  elem + (plane >> 2), a8[4], a8[5], a8[6], a8[7], r1);
                             if (ep.twin != nullptr)  // K % 8 == 0 then: the lane's 8 channels are one Byte8 element
                                 *reinterpret_cast<ohip_v2i*>(ep.twin + (size_t)(ch0 / 8) * OHW * 8 + col_twin[j]) = tw;
                         } else if constexpr (F32) {

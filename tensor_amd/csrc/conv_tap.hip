@@ -237,11 +237,16 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
             } else {
                 constexpr bool FUSED = EPI == EPI_F32_P4_FUSED;
                 const size_t e = ((size_t)(n * (unsigned)(Ks / 4) + ch / 4) * (unsigned)OHW + pix) * 4;
+                const float *r0 = nullptr, *r1 = nullptr;
+                if (FUSED && ep.residual1 != nullptr) {  // wave-uniform; one group then
+                    r0 = epi4_residual_at(ep, n, pix, ch0, g.K, OHW);
+                    r1 = epi4_residual_at(ep, n, pix, ch0 + 4, g.K, OHW);
+                }
                 ohip_v2i tw = {0, 0};
-                tw[0] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si, prm.bi, e, a8[0], a8[1], a8[2], a8[3]);
+                tw[0] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si, prm.bi, e, a8[0], a8[1], a8[2], a8[3], r0);
                 if (ch0 + 4 < g.K)
                     tw[1] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si + 4, prm.bi + 4, e + (size_t)OHW * 4, a8[4], a8[5],
-                                                         a8[6], a8[7]);
+                                                         a8[6], a8[7], r1);
                 if constexpr (FUSED)
                     if (ep.twin != nullptr)  // K % 8 == 0 then: the lane's 8 channels are one Byte8 element
                         *reinterpret_cast<ohip_v2i*>(ep.twin + ((size_t)(n * (unsigned)(Ks / 8) + ch / 8) * (unsigned)OHW + pix) * 8) = tw;

@@ -780,22 +780,60 @@ int ConvolutionLayer::forward_int8(const Tensor& bottom_in, const Tensor* shortc
     return 0;
 }
 
+bool ConvolutionLayer::join_input(const Tensor& bottom, const NetOption& opt, Tensor& input, int& oh, int& ow) const {
+    if (!handle_ || !int8_scale_term || int8_scale_term > 100 || force_out_layout >= 0 || !opt.use_packing_layout) return false;
+    if (!bottom.defined() || bottom.dim() != 4 || out_channels % 8) return false;
+    Tensor twin;
+    input = bottom;
+    if (base_of(bottom.scalar_type()) == ScalarType::Float && in_channels % 8 == 0 &&
+        bottom.quantized_twin(bottom_blob_int8_scales.data_ptr<float>()[0], input_round_mode(opt), twin))
+        input = twin;
+    if (input.scalar_type() != ScalarType::Byte8 || input.channels() != in_channels) return false;
+    const int N = (int)input.size(0), H = (int)input.size(2), W = (int)input.size(3);
+    return !otter_hip_conv_output_shape(handle_, H, W, &oh, &ow) && otter_hip_conv_join_launches(handle_, OTTER_HIP_I8_P8, N, H, W) == 1;
+}
+
+int ConvolutionLayer::forward_residual_concat(const Tensor& bottom_in, const Tensor& part0, const Tensor& part1, float q_scale,
+                                              int q_round, Tensor& sum, const NetOption& opt) const {
+    Tensor bottom;
+    int oh = 0, ow = 0;
+    if (!join_input(bottom_in, opt, bottom, oh, ow)) return 1;
+    const int N = (int)bottom.size(0);
+    for (const Tensor* t : {&part0, &part1})
+        if (!t->defined() || t->dim() != 4 || base_of(t->scalar_type()) != ScalarType::Float || t->elempack() == 1 ||
+            t->channels() % 8 || t->size(0) != N || t->size(2) != oh || t->size(3) != ow)
+            return 1;
+    if (part0.channels() + part1.channels() != out_channels) return 1;
+    try {
+        sum = Tensor::empty_device({N, out_channels / 4, oh, ow}, ScalarType::Float4);
+        Tensor q;
+        if (q_scale > 0.f) q = Tensor::empty_device({N, out_channels / 8, oh, ow}, ScalarType::Byte8);
+        const int rc = otter_hip_conv_forward_residual_concat(
+            handle_, bottom.device_ptr(), OTTER_HIP_I8_P8, N, (int)bottom.size(2), (int)bottom.size(3), (const float*)part0.device_ptr(),
+            hip_layout_of(part0.scalar_type()), (int)part0.channels(), (const float*)part1.device_ptr(),
+            hip_layout_of(part1.scalar_type()), (float*)sum.device_ptr(), q.defined() ? (int8_t*)q.device_ptr() : nullptr, q_scale,
+            q_round, nullptr);
+        if (rc) return rc;
+        sum.mark_device_written();
+        if (q.defined()) {
+            q.mark_device_written();
+            sum.attach_quantized(q, q_scale, q_round);
+        }
+    } catch (const Error&) {
+        return -100;
+    }
+    return 0;
+}
+
 int ConvolutionLayer::forward_shuffle(const Tensor& bottom_in, const Tensor& other, bool other_odd, bool joined, float q_scale,
                                       int q_round, Tensor& first, Tensor& second, const NetOption& opt) const {
-    if (!handle_ || !int8_scale_term || int8_scale_term > 100 || force_out_layout >= 0 || !opt.use_packing_layout) return 1;
-    if (!bottom_in.defined() || bottom_in.dim() != 4 || out_channels % 8) return 1;
-    Tensor bottom = bottom_in, twin;
-    if (base_of(bottom_in.scalar_type()) == ScalarType::Float && in_channels % 8 == 0 &&
-        bottom_in.quantized_twin(bottom_blob_int8_scales.data_ptr<float>()[0], input_round_mode(opt), twin))
-        bottom = twin;
-    if (bottom.scalar_type() != ScalarType::Byte8 || bottom.channels() != in_channels) return 1;
-    const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3);
+    Tensor bottom;
     int oh = 0, ow = 0;
-    if (otter_hip_conv_output_shape(handle_, H, W, &oh, &ow)) return 1;
+    if (!join_input(bottom_in, opt, bottom, oh, ow)) return 1;
+    const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3);
     if (!other.defined() || other.dim() != 4 || base_of(other.scalar_type()) != ScalarType::Float || other.elempack() == 1 ||
         other.channels() != out_channels || other.size(0) != N || other.size(2) != oh || other.size(3) != ow)
         return 1;
-    if (otter_hip_conv_shuffle_launches(handle_, OTTER_HIP_I8_P8, N, H, W) != 1) return 1;
     try {
         const std::vector<int64_t> sizes = {N, (joined ? 2 : 1) * out_channels / 8, oh, ow};
         first = Tensor::empty_device(sizes, ScalarType::Float8);
@@ -1929,7 +1967,10 @@ void Net::plan_fused_quantize() const {
             if (e->bottoms[0] == e->bottoms[1]) continue;
             if (best < 0 || pi > blobs_[e->bottoms[best]].producer) best = k;  // the later one: the other is ready by then
         }
-        if (best >= 0) residual_units_[(int)ei] = ResidualUnit{blobs_[e->bottoms[best]].producer, (int)ei, e->bottoms[1 - best]};
+        if (best < 0) continue;
+        const int other = e->bottoms[1 - best], oi = blobs_[other].producer;
+        const bool concat = oi >= 0 && layers_[oi]->type() == "Concat" && layers_[oi]->bottoms.size() == 2 && blobs_[other].consumers.size() == 1;
+        residual_units_[(int)ei] = ResidualUnit{blobs_[e->bottoms[best]].producer, (int)ei, other, concat ? oi : -1};
     }
     // Classifier tails: a GlobalAvgPool layer on the fp32 result of an int8 convolution read by nothing else
     pool_units_.clear();
@@ -2108,12 +2149,30 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
             if (rc <= 0) return rc;
         }
     }
+    Tensor sum;
+    if (u.concat >= 0 && !blobs[u.shortcut].defined()) {
+        // the sum straight from the two blobs that the Concat would copy
+        const int p0 = layers_[u.concat]->bottoms[0], p1 = layers_[u.concat]->bottoms[1];
+        for (int b : {p0, p1, conv->bottoms[0]})
+            if (!blobs[b].defined()) {
+                const int rc = forward_layer(blobs_[b].producer, blobs, opt);
+                if (rc) return rc;
+            }
+        const int rc = conv->forward_residual_concat(blobs[conv->bottoms[0]], blobs[p0], blobs[p1], e->fuse_scale, e->fuse_round, sum, opt);
+        if (rc < 0) return rc;
+        if (rc == 0) {
+            blobs[e->tops[0]] = sum;
+            if (opt.lightmode)
+                for (int b : {p0, p1, conv->bottoms[0]})
+                    if (blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+            return 0;
+        }
+    }
     for (int b : {u.shortcut, conv->bottoms[0]})
         if (!blobs[b].defined()) {
             const int rc = forward_layer(blobs_[b].producer, blobs, opt);
             if (rc) return rc;
         }
-    Tensor sum;
     const int rc = conv->forward_residual(blobs[conv->bottoms[0]], blobs[u.shortcut], e->fuse_scale, e->fuse_round, sum, opt);
     if (rc) return rc;
     blobs[e->tops[0]] = sum;

@@ -242,6 +242,9 @@ public:
     // > 0 also quantizes the second half (joined: the blob). Returns 1, and does nothing, when that is not one launch here.
     int forward_shuffle(const Tensor& bottom_blob, const Tensor& other, bool other_odd, bool joined, float q_scale, int q_round,
                         Tensor& first, Tensor& second, const NetOption& opt) const;
+    // forward_residual where the shortcut is the concatenation of two blobs (otter_hip_conv_forward_residual_concat)
+    int forward_residual_concat(const Tensor& bottom_blob, const Tensor& part0, const Tensor& part1, float q_scale, int q_round,
+                                Tensor& sum, const NetOption& opt) const;
     // what otter_hip_conv_block_launches says of the three layers on an input of this size
     static int block_launches(const ConvolutionLayer* expand, const ConvolutionLayer* depthwise, const ConvolutionLayer* project,
                               int n, int h, int w);
@@ -259,6 +262,8 @@ public:
     static long block_forward_count();  // blocks executed that way so far in this process (for tests)
 
 private:
+    // the int8 blob that a launch with another layer's work in its epilogue reads, and that launch's output size; false: no such launch
+    bool join_input(const Tensor& bottom_blob, const NetOption& opt, Tensor& input, int& out_h, int& out_w) const;
     int create_pipeline_int8(const NetOption& opt);
     int forward_int8(const Tensor& bottom_blob, const Tensor* shortcut, float q_scale, int q_round, Tensor& top_blob,
                      const NetOption& opt) const;
@@ -355,6 +360,7 @@ private:
     struct ResidualUnit {
         int conv, eltwise;
         int shortcut;  // blob index of the other operand
+        int concat;    // the Concat layer of two blobs that makes the other operand, which nothing else reads, or -1
     };
     mutable std::map<int, ResidualUnit> residual_units_;
     int forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const;

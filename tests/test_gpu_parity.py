@@ -674,7 +674,7 @@ def test_forward_shuffle_equals_forward_concat_shuffle(hip, oracle, C, K, k, s, 
     want_q = oracle.quantize(want, np.float32(q_scale), capi.ROUND_SSE)
     od = hip.to_device(capi.pack_np(other, other_pack))
     layout = capi.F32_P8 if other_pack == 8 else capi.F32_P4
-    assert conv.shuffle_launches(capi.I8_P8, N, H, W) == 1
+    assert conv.join_launches(capi.I8_P8, N, H, W) == 1
     for whole in (True, False):
         out = conv.forward_shuffle(xd, N, H, W, od, layout, other_odd, joined, q_scale, capi.ROUND_SSE, whole=whole)
         hip.torch.cuda.synchronize()
@@ -687,6 +687,47 @@ def test_forward_shuffle_equals_forward_concat_shuffle(hip, oracle, C, K, k, s, 
             np.testing.assert_array_equal(capi.unpack_np(out[2 + i].cpu().numpy(), 8, shape), want_q[:, part])
     with pytest.raises(capi.HipError):
         conv.forward_shuffle(xd, N, H, W, od, capi.F32, other_odd, joined)  # an unpacked other blob
+    conv.close()
+
+
+@pytest.mark.parametrize("C,K,split,k,N,H,W,act,tile", [
+    (128, 128, 64, 1, 2, 13, 13, 0, 0),
+    (128, 128, 64, 1, 2, 26, 26, 2, -4),
+    (24, 16, 8, 1, 3, 5, 7, 1, 0),         # one octet each
+    (24, 72, 56, 1, 2, 9, 5, 3, -4),       # parts of unequal size, remainders in both
+    (16, 24, 16, 3, 1, 11, 9, 0, -8),
+    (64, 520, 8, 1, 5, 1, 1, 0, -4),       # one pixel, wide row tiles
+])
+@pytest.mark.parametrize("packs", [(4, 4), (8, 4), (4, 8)])
+def test_forward_residual_concat_equals_forward_then_add(hip, oracle, C, K, split, k, N, H, W, act, tile, packs):
+    """otter_hip_conv_forward_residual_concat: otter_hip_conv_forward's blob plus the concatenation of the two parts, one fp32
+    addition per element, and the oracle's quantize_to_int8 of it."""
+    rng = np.random.default_rng(C * 3 + K + k + act)
+    x, wq, ws, bias = _rand_problem(rng, C, K, k, 1, N, H, W)
+    conv = hip.conv(wq=wq, scale_in=host_scale_in(ws, 20.0), bias=bias, in_scale=20.0, out_scale=None, stride=(1, 1),
+                    pad=(k // 2, k // 2), dil=(1, 1), groups=1, act=act, act_p0=0.1, out_kind=capi.OUT_F32, out_round=0,
+                    in_round=oracle.quantize_round_mode(C, True))
+    xd = hip.to_device(capi.pack_np(x, 8))
+    if tile:
+        conv.set_tile(tile, 0)
+    plain = capi.unpack_np(conv.forward(xd, capi.I8_P8, N, H, W, capi.F32_P4).cpu().numpy(), 4, (N, K, H, W))
+    short = (rng.normal(0, 1, plain.shape) * np.abs(plain).mean()).astype(np.float32)
+    want = plain + short
+    q_scale = 127.0 / float(np.abs(want).max()) * 1.3  # some values saturate
+    layouts = [capi.F32_P8 if p == 8 else capi.F32_P4 for p in packs]
+    parts = [hip.to_device(capi.pack_np(np.ascontiguousarray(a), p)) for a, p in zip((short[:, :split], short[:, split:]), packs)]
+    assert conv.join_launches(capi.I8_P8, N, H, W) == 1
+    for scale in (q_scale, None):
+        out, q = conv.forward_residual_concat(xd, N, H, W, parts[0], layouts[0], split, parts[1], layouts[1], scale)
+        hip.torch.cuda.synchronize()
+        got = capi.unpack_np(out.cpu().numpy(), 4, want.shape)
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+        if scale:
+            np.testing.assert_array_equal(capi.unpack_np(q.cpu().numpy(), 8, want.shape),
+                                          oracle.quantize(want, np.float32(scale), capi.ROUND_SSE))
+    for bad in (0, K, 4):
+        with pytest.raises(capi.HipError):
+            conv.forward_residual_concat(xd, N, H, W, parts[0], layouts[0], bad, parts[1], layouts[1])
     conv.close()
 
 
