@@ -172,7 +172,8 @@ int otter_hip_conv_forward_static(const otter_hip_conv_t* handle, const void* in
  * blob (Tensor/ConvolutionLayer.cpp:770-775), out_q = float2int8(out * q_scale) as Byte8 [N][K/8][OH*OW][8].
  * q_scale = the readers' bottom_blob_int8_scales[0], q_round_mode = their input rounding primitive. The implicit-GEMM
  * kernel writes out_q from its own epilogue (Float4 output, clamp-type activation); every other case runs the
- * quantize pass after the convolution, with the same result. */
+ * quantize pass after the convolution, with the same result. `out` may be NULL (the fp32 blob has no other reader) where
+ * out_layout is F32_P4 and otter_hip_conv_join_launches(...) == 1; the same holds for otter_hip_conv_forward_residual. */
 int otter_hip_conv_forward_twin(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h,
                                 int in_w, void* out, int out_layout, void* out_q, float q_scale, int q_round_mode,
                                 void* workspace, size_t workspace_bytes, void* stream);
@@ -206,7 +207,7 @@ int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* handle, const void* i
 /* otter_hip_conv_forward_residual where the shortcut is Concat(part0, part1) that nothing else reads (Tensor/ConcatLayer.cpp:54-67,
  * Tensor/ShortCutLayer.cpp): out (Float4) = activation(convolution) + [part0 | part1], one launch, the concatenated blob not made.
  * part0 has part0_channels channels, part1 the other K - part0_channels; Float4 or Float8 each. out_q (or NULL) as there.
- * Needs an int8 Byte8 input, whole channel octets throughout and otter_hip_conv_join_launches(...) == 1. No workspace. */
+ * Needs an int8 Byte8 input, whole channel octets throughout and otter_hip_conv_join_launches(...) == 1. No workspace. out may be NULL with out_q. */
 int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w,
                                            const float* part0, int part0_layout, int part0_channels, const float* part1,
                                            int part1_layout, float* out, int8_t* out_q, float q_scale, int q_round_mode,
@@ -427,7 +428,8 @@ int otter_hip_copy_channels_quantize(const float* src, int src_layout, int src_c
  * size and image size, src_channels[i] channels each in layout src_layouts[i], one after the other along the channel
  * axis of dst. Packed layouts only (F32_P4 / F32_P8 on every side; otter_hip_copy_channels covers the rest). With dst_q
  * (or NULL; needs a channel sum divisible by 8) also the quantize_to_int8 of dst that an int8 convolution reading it
- * would compute first (Tensor/ConvolutionLayer.cpp:770-775): dst_q = float2int8(dst * scale) as Byte8. */
+ * would compute first (Tensor/ConvolutionLayer.cpp:770-775): dst_q = float2int8(dst * scale) as Byte8. dst may
+ * be NULL with dst_q. */
 int otter_hip_concat_channels(const float* const* srcs, const int* src_layouts, const int* src_channels, int count,
                               float* dst, int dst_layout, int n, int h, int w, int8_t* dst_q, float scale,
                               int round_mode, void* stream);

@@ -695,7 +695,7 @@ int otter_hip_conv3x3_halo_plan(int in_channels, int out_channels, int pad, int 
 static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w, void* out,
                         int out_layout, void* workspace, size_t workspace_bytes, void* stream_, int8_t* twin,
                         float twin_scale, int twin_round, const float* residual = nullptr) {
-    if (!h || !in || !out) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: null");
+    if (!h || !in || (!out && !twin)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: null");
     if (!valid_layout(in_layout) || !valid_layout(out_layout))
         return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: unknown layout");
     const otter_hip_conv_desc& d = h->d;
@@ -714,6 +714,9 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
     if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: empty output");
     if ((size_t)n * g.C * in_h * in_w >= (1ull << 31) || (size_t)n * g.K * g.OH * g.OW >= (1ull << 31))
         return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward: tensor exceeds 2^31 elements; split the batch");
+    if (!out && (out_layout != OTTER_HIP_F32_P4 || in_h < 1 || otter_hip_conv_join_launches(h, in_layout, n, in_h, in_w) != 1))
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: the int8 result alone needs a Float4 layer that is one launch with "
+                                           "it (otter_hip_conv_join_launches)");
     if (n == 0) return OTTER_HIP_OK;
 
     // the sum and the twin as a pass of their own, for the kernels that do not write them
@@ -1053,6 +1056,7 @@ int otter_hip_conv_forward_residual(const otter_hip_conv_t* h, const void* in, i
         return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual: the quantized sum needs K % 8 == 0");
     if (out_q && q_round_mode != OTTER_HIP_ROUND_SSE && q_round_mode != OTTER_HIP_ROUND_EXACT)
         return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual: unknown rounding mode");
+    if (!out && !out_q) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual: null");
     if (residual == out) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual: out must not be the residual");
     return conv_forward(h, in, in_layout, n, in_h, in_w, out, out_layout, workspace, workspace_bytes, stream, (int8_t*)out_q,
                         q_scale, q_round_mode, residual);
@@ -1434,19 +1438,21 @@ int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* h, const void* in, in
     if (!ok) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: not a single launch (otter_hip_conv_join_launches)");
     if (n == 0) return OTTER_HIP_OK;
     const size_t half = (size_t)g.K * g.OH * g.OW;  // elements of one half of one image
-    ep.other = other, ep.other_pack = layout_pack(other_layout), ep.other_odd = other_odd != 0;
+    JoinArgs ja;
+    ep.join = &ja;
+    ja.other = other, ja.other_pack = layout_pack(other_layout), ja.other_odd = other_odd != 0;
     ep.twin_scale = q_scale, ep.twin_half = q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
-    ep.sh_image = joined ? 2 * half : half;
-    ep.sh_out0 = first_half, ep.sh_q0 = first_half_q;
-    ep.sh_out1 = joined ? (first_half ? first_half + half : nullptr) : second_half;
-    ep.sh_q1 = joined ? (first_half_q ? first_half_q + half : nullptr) : second_half_q;
+    ja.sh_image = joined ? 2 * half : half;
+    ja.sh_out0 = first_half, ja.sh_q0 = first_half_q;
+    ja.sh_out1 = joined ? (first_half ? first_half + half : nullptr) : second_half;
+    ja.sh_q1 = joined ? (first_half_q ? first_half_q + half : nullptr) : second_half_q;
     return join_run(h, in, nullptr, g, ep, alt, config, (hipStream_t)stream_);
 }
 
 int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w,
                                            const float* part0, int part0_layout, int part0_channels, const float* part1,
                                            int part1_layout, float* out, int8_t* out_q, float q_scale, int q_round_mode, void* stream_) {
-    if (!h || !in || !part0 || !part1 || !out) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: null");
+    if (!h || !in || !part0 || !part1 || (!out && !out_q)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: null");
     if (!valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1)
         return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_residual_concat: bad argument");
     for (int l : {part0_layout, part1_layout})
@@ -1469,8 +1475,10 @@ int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* h, const void
     if (!ok)
         return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_residual_concat: not a single launch (otter_hip_conv_join_launches)");
     if (n == 0) return OTTER_HIP_OK;
-    ep.residual = part0, ep.residual1 = part1, ep.res_split = part0_channels;
-    ep.res_pack0 = layout_pack(part0_layout), ep.res_pack1 = layout_pack(part1_layout);
+    JoinArgs ja;
+    ep.join = &ja;
+    ep.residual = part0, ja.residual1 = part1, ja.res_split = part0_channels;
+    ja.res_pack0 = layout_pack(part0_layout), ja.res_pack1 = layout_pack(part1_layout);
     ep.twin = out_q, ep.twin_scale = q_scale, ep.twin_half = q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     return join_run(h, in, out, g, ep, alt, config, (hipStream_t)stream_);
 }
@@ -1591,7 +1599,7 @@ int otter_hip_channel_shuffle(const float* src, int src_layout, float* dst, int 
 int otter_hip_concat_channels(const float* const* srcs, const int* src_layouts, const int* src_channels, int count,
                               float* dst, int dst_layout, int n, int h, int w, int8_t* dst_q, float scale, int round_mode,
                               void* stream) {
-    if (!srcs || !src_layouts || !src_channels || !dst) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_concat_channels: null");
+    if (!srcs || !src_layouts || !src_channels || (!dst && !dst_q)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_concat_channels: null");
     if (count < 1 || count > CONCAT_MAX)
         return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_concat_channels: 1 to 8 sources (use otter_hip_copy_channels for more)");
     if (n < 0 || h < 1 || w < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_concat_channels: bad shape");

@@ -123,21 +123,28 @@ struct Epilogue {
     // fp32 output only: a blob in the output's layout that is added to the activated result (the Eltwise sum of a
     // residual block; null: none). The twin, if any, is the quantization of the sum. Float4 epilogue only.
     const float* residual = nullptr;
-    // The addend may be a concatenation that nobody else reads: channels below res_split come from `residual`, the rest from
-    // residual1 (null: one blob in the output's layout), each Float4 or Float8. K and res_split are multiples of 8 then.
+    // host side only: what the EPI_F32_SHUFFLE and EPI_F32_P4_PARTS instances take beside this struct (null: neither)
+    const struct JoinArgs* join = nullptr;
+    bool fused() const { return twin != nullptr || residual != nullptr || join != nullptr; }
+};
+
+// Other layers' work in the epilogue of a Float4 layer (K % 8 == 0). An argument of its own: with it inside Epilogue every launch
+// of the library carried 100 to 300 bytes more of arguments, 0.1 us each.
+struct JoinArgs {
+    // The addend is a concatenation that nobody else reads: channels below res_split come from Epilogue::residual, the rest from
+    // residual1, each Float4 or Float8; res_split is a multiple of 8.
     const float* residual1 = nullptr;
     int res_split = 0, res_pack0 = 4, res_pack1 = 4;
-    // fp32 output only: the layer is one half of Concat -> ChannelShuffle(2) and writes the shuffled blob, its channels
-    // alternating with those of `other` (K channels too, Float4 or Float8: other_pack; null: no shuffle). The 2 K channels are
-    // two halves of K, each an fp32 blob sh_out and a Byte8 blob sh_q (quantized with twin_scale), null where not wanted;
-    // sh_image: elements from one image to the next in all four. Float4 output layout and K % 8 == 0 only.
-    const float* other = nullptr;
+    // The layer is one half of Concat -> ChannelShuffle(2) and writes the shuffled blob, its channels alternating with those of
+    // `other` (K channels too, Float4 or Float8: other_pack; null: no shuffle). The 2 K channels are two halves of K, each an fp32
+    // blob sh_out and a Byte8 blob sh_q (quantized with twin_scale), null where not wanted; sh_image: elements from one image to
+    // the next in all four.
     int other_pack = 0;
+    const float* other = nullptr;
     bool other_odd = false;  // `other` takes the odd channels of the shuffled blob, else the even ones
     float *sh_out0 = nullptr, *sh_out1 = nullptr;
     int8_t *sh_q0 = nullptr, *sh_q1 = nullptr;
     size_t sh_image = 0;
-    bool fused() const { return twin != nullptr || residual != nullptr || other != nullptr; }
 };
 
 // which epilogue code a kernel instance carries
@@ -148,8 +155,31 @@ enum {
     EPI_I8_P8_NONNEG = 3,
     EPI_F32_P8 = 4,       // depthwise only
     EPI_F32_P4_FUSED = 5,  // implicit GEMM only: EPI_F32_P4 plus the residual addend and / or the int8 twin
-    EPI_F32_SHUFFLE = 6    // the same kernels: the channels interleaved with another blob's (Epilogue::other)
+    EPI_F32_SHUFFLE = 6,   // the same kernels: the channels interleaved with another blob's (JoinArgs::other)
+    EPI_F32_P4_PARTS = 7   // EPI_F32_P4_FUSED with the addend in two parts (JoinArgs::residual1)
 };
+
+// the argument that an instance takes for them
+struct NoJoin {
+    static NoJoin of(const Epilogue&) { return {}; }
+};
+struct WithJoin : JoinArgs {
+    static WithJoin of(const Epilogue& ep) { return {*ep.join}; }
+};
+template <int EPI>
+struct JoinOf {
+    using Type = NoJoin;
+};
+template <>
+struct JoinOf<EPI_F32_SHUFFLE> {
+    using Type = WithJoin;
+};
+template <>
+struct JoinOf<EPI_F32_P4_PARTS> {
+    using Type = WithJoin;
+};
+template <int EPI>
+using JoinParam = typename JoinOf<EPI>::Type;
 
 // The fast epilogues need: activation in {none, ReLU, clip, LeakyReLU with a slope in [0, 1]}, and (I8_P8) int8
 // output in Byte8 with K % 8 == 0 or (F32_P4) fp32 output in Float4 with K % 4 == 0.
@@ -389,30 +419,30 @@ __device__ __forceinline__ ohip_v4i epi4_dequant_f32p4(const Epilogue& ep, const
     return r;
 }
 
-// Channels ch0 .. ch0 + 7 of one pixel into the shuffled blob: with the same channels of Epilogue::other they are its
+// Channels ch0 .. ch0 + 7 of one pixel into the shuffled blob: with the same channels of JoinArgs::other they are its
 // channels 2 ch0 .. 2 ch0 + 15, two packs of 8 that a lane writes whole (32 bytes fp32, 8 bytes int8 each). Bound by the bytes of
 // the two fp32 blobs; the layer's own result is neither written nor read back. Layer and shuffle as two launches / as one, in the
 // detection network at batch 16: 88 channels @52x52 23 / 14.5 us, 176 @26x26 15.6 / 10.2 us, 352 @13x13 11.8 / 7.5 us.
 template <int LRELU>
-__device__ __forceinline__ void epi8_store_shuffle(const Epilogue& ep, const float* si, const float* bi, const int (&a8)[8], unsigned n,
+__device__ __forceinline__ void epi8_store_shuffle(const Epilogue& ep, const JoinArgs& ja, const float* si, const float* bi, const int (&a8)[8], unsigned n,
                                                    unsigned pix, int ch0, int K, int OHW) {
-    const size_t plane = (size_t)OHW * ep.other_pack;
-    const float* o = ep.other + ((size_t)n * (unsigned)(K / ep.other_pack) + (unsigned)(ch0 / ep.other_pack)) * plane +
-                     (size_t)pix * (unsigned)ep.other_pack;
+    const size_t plane = (size_t)OHW * ja.other_pack;
+    const float* o = ja.other + ((size_t)n * (unsigned)(K / ja.other_pack) + (unsigned)(ch0 / ja.other_pack)) * plane +
+                     (size_t)pix * (unsigned)ja.other_pack;
     const ohip_v4i x0 = *reinterpret_cast<const ohip_v4i*>(o);
-    const ohip_v4i x1 = *reinterpret_cast<const ohip_v4i*>(o + (ep.other_pack == 8 ? 4 : plane));
+    const ohip_v4i x1 = *reinterpret_cast<const ohip_v4i*>(o + (ja.other_pack == 8 ? 4 : plane));
     const ohip_v4i v0 = epi4_dequant_f32p4<LRELU>(ep, si, bi, a8[0], a8[1], a8[2], a8[3]);
     const ohip_v4i v1 = epi4_dequant_f32p4<LRELU>(ep, si + 4, bi + 4, a8[4], a8[5], a8[6], a8[7]);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const ohip_v4i x = h ? x1 : x0, v = h ? v1 : v0;
-        const ohip_v4i even = ep.other_odd ? v : x, odd = ep.other_odd ? x : v;  // wave-uniform
+        const ohip_v4i even = ja.other_odd ? v : x, odd = ja.other_odd ? x : v;  // wave-uniform
         const int f[8] = {even[0], odd[0], even[1], odd[1], even[2], odd[2], even[3], odd[3]};
         const int pack = ch0 / 4 + h, half = K / 8;  // pack of the 2 K channels, packs in each half
         const bool second = pack >= half;
-        const size_t e = (size_t)n * ep.sh_image + ((size_t)(unsigned)(second ? pack - half : pack) * (unsigned)OHW + pix) * 8;
-        float* out = second ? ep.sh_out1 : ep.sh_out0;
-        int8_t* q = second ? ep.sh_q1 : ep.sh_q0;
+        const size_t e = (size_t)n * ja.sh_image + ((size_t)(unsigned)(second ? pack - half : pack) * (unsigned)OHW + pix) * 8;
+        float* out = second ? ja.sh_out1 : ja.sh_out0;
+        int8_t* q = second ? ja.sh_q1 : ja.sh_q0;
         if (out != nullptr) {
             const ohip_v4i lo = {f[0], f[1], f[2], f[3]}, hi = {f[4], f[5], f[6], f[7]};
             *reinterpret_cast<ohip_v4i*>(out + e) = lo;
@@ -431,14 +461,14 @@ __device__ __forceinline__ void epi8_store_shuffle(const Epilogue& ep, const flo
     }
 }
 
-// Four channels of one pixel of an addend in two parts (Epilogue::residual1). Saves the copies that brought the two blobs
+// Four channels of one pixel of an addend in two parts (JoinArgs::residual1). Saves the copies that brought the two blobs
 // together and into the result's layout, and the pass that added them: 128 channels @52x52, batch 16, concatenation + layer +
 // repack + sum 45.6 us as four launches, 14.4 us as one.
-__device__ __forceinline__ const float* epi4_residual_at(const Epilogue& ep, unsigned n, unsigned pix, int ch, int K, int OHW) {
-    const bool second = ch >= ep.res_split;
-    const int c = second ? ch - ep.res_split : ch, channels = second ? K - ep.res_split : ep.res_split;
-    const int pack = second ? ep.res_pack1 : ep.res_pack0, at = c & (pack - 1);
-    return (second ? ep.residual1 : ep.residual) + (size_t)(n * (unsigned)channels + (unsigned)(c - at)) * (unsigned)OHW +
+__device__ __forceinline__ const float* epi4_residual_at(const Epilogue& ep, const JoinArgs& ja, unsigned n, unsigned pix, int ch, int K, int OHW) {
+    const bool second = ch >= ja.res_split;
+    const int c = second ? ch - ja.res_split : ch, channels = second ? K - ja.res_split : ja.res_split;
+    const int pack = second ? ja.res_pack1 : ja.res_pack0, at = c & (pack - 1);
+    return (second ? ja.residual1 : ep.residual) + (size_t)(n * (unsigned)channels + (unsigned)(c - at)) * (unsigned)OHW +
            (size_t)pix * (unsigned)pack + (unsigned)at;
 }
 
@@ -457,7 +487,7 @@ __device__ __forceinline__ unsigned epi4_store_f32p4(float* __restrict__ out, co
     ohip_v4i res = {0, 0, 0, 0};
     if constexpr (FUSED)
         if (ep.residual != nullptr)  // wave-uniform
-            res = *reinterpret_cast<const ohip_v4i*>(ep.residual1 != nullptr ? res_at : ep.residual + elem);
+            res = *reinterpret_cast<const ohip_v4i*>(res_at != nullptr ? res_at : ep.residual + elem);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         float v = __fmaf_rn((float)a[e], si[e], bi[e]);
@@ -475,7 +505,7 @@ __device__ __forceinline__ unsigned epi4_store_f32p4(float* __restrict__ out, co
         }
         r[e] = __float_as_int(v);
     }
-    *reinterpret_cast<ohip_v4i*>(out + elem) = r;
+    if (!FUSED || out != nullptr) *reinterpret_cast<ohip_v4i*>(out + elem) = r;  // (null: the twin alone)
     return q;
 }
 

@@ -46,7 +46,7 @@ template <int TM, int TN, int WM, int WN, int EPI, int KC, bool INF = false>
 __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
                                                          void* __restrict__ out, ConvGeom g, Epilogue ep, int m_tiles16,
                                                          int c_groups, int n_pix_tiles, const float* __restrict__ in_scale_p,
-                                                         float in_half) {
+                                                         float in_half, JoinParam<EPI> ja) {
     using Cfg = IgemmCfg<TM, TN, WM, WN>;
     constexpr int FM = Cfg::FM, FN = Cfg::FN;
     constexpr int NBUF = KC == 1 ? 2 : KC;
@@ -299,11 +299,12 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
     unsigned n0, pix0;
     locate((unsigned)(wn * (TN / WN) + (lane & 15)), n0, pix0);
     const bool wide = (unsigned)OHW >= 16u * FN;  // then a column is at most one image further than the first
-    if constexpr (EPI == EPI_F32_P4 || EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_SHUFFLE || EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
+    if constexpr (EPI == EPI_F32_P4 || EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_SHUFFLE || EPI == EPI_F32_P4_PARTS || EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
         // Packed outputs. A lane's stores differ by a column offset (image, pixel) and a row
         // offset (channel group): each computed once, one 64-bit addition per store. LeakyReLU is decided once, in
         // front of the unrolled loops, not per value.
-        constexpr bool FUSED = EPI == EPI_F32_P4_FUSED;  // plus the residual addend and / or the int8 twin
+        constexpr bool PARTS = EPI == EPI_F32_P4_PARTS;
+        constexpr bool FUSED = EPI == EPI_F32_P4_FUSED || PARTS;  // plus the residual addend and / or the int8 twin
         constexpr bool SHUF = EPI == EPI_F32_SHUFFLE;    // interleaved with another blob's channels
         constexpr bool F32 = EPI == EPI_F32_P4 || FUSED || SHUF;
         constexpr int EB = F32 ? 16 : 8;       // bytes of one (pixel, channel group) element
@@ -312,7 +313,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
         const size_t image = plane * (size_t)(Ks / CG);
         size_t col_ofs[FN];
         unsigned col_twin[FUSED ? FN : 1];  // the same for the Byte8 twin (below 2 GiB)
-        unsigned col_n[SHUF || FUSED ? FN : 1], col_pix[SHUF || FUSED ? FN : 1];
+        unsigned col_n[SHUF || PARTS ? FN : 1], col_pix[SHUF || PARTS ? FN : 1];
         bool col_ok[FN];
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
@@ -326,7 +327,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
             }
             col_ok[j] = gpo < total_pix;
             col_ofs[j] = (size_t)nn * image + (size_t)pp * EB;
-            if constexpr (SHUF || FUSED) col_n[j] = nn, col_pix[j] = pp;
+            if constexpr (SHUF || PARTS) col_n[j] = nn, col_pix[j] = pp;
             if constexpr (FUSED) col_twin[j] = (nn * (unsigned)(Ks / 8) * (unsigned)OHW + pp) * 8u;
         }
         auto rows = [&](auto lrelu_c) {
@@ -351,13 +352,13 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
                     if (ch_ok && col_ok[j]) {
                         char* o = row + col_ofs[j];
                         if constexpr (SHUF) {
-                            epi8_store_shuffle<LRELU ? 1 : 0>(ep, prm.si, prm.bi, a8, col_n[j], col_pix[j], ch0, g.K, OHW);
+                            epi8_store_shuffle<LRELU ? 1 : 0>(ep, ja, prm.si, prm.bi, a8, col_n[j], col_pix[j], ch0, g.K, OHW);
                         } else if constexpr (FUSED) {
                             const size_t elem = (row_ofs + col_ofs[j]) >> 2;  // in floats, for the result and the addend
                             const float *r0 = nullptr, *r1 = nullptr;
-                            if (ep.residual1 != nullptr) {  // wave-uniform
-                                r0 = epi4_residual_at(ep, col_n[j], col_pix[j], ch0, g.K, OHW);
-                                r1 = epi4_residual_at(ep, col_n[j], col_pix[j], ch0 + 4, g.K, OHW);
+                            if constexpr (PARTS) {
+                                r0 = epi4_residual_at(ep, ja, col_n[j], col_pix[j], ch0, g.K, OHW);
+                                r1 = epi4_residual_at(ep, ja, col_n[j], col_pix[j], ch0 + 4, g.K, OHW);
                             }
                             ohip_v2i tw = {0, 0};
                             tw[0] = (int)epi4_store_f32p4<true, LRELU ? 1 : 0>((float*)out, ep, prm.si, prm.bi, elem, a8[0], a8[1],
@@ -494,7 +495,7 @@ static hipError_t launch_igemm_k(const int8_t* x, const int8_t* wpk, void* out, 
     const int m_tiles = (g.K + TM - 1) / TM;  // row blocks that hold at least one real channel (the rows are padded further)
     const int grid_z = g.Cs ? g.Cs / g.C : 1;  // groups of a grouped convolution
     hipLaunchKernelGGL((conv_igemm_kernel<TM, TN, WM, WN, EPI, KC>), dim3(n_pix_tiles, m_tiles, grid_z), dim3(256), 0,
-                       stream, x, wpk, out, g, ep, mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, (const float*)nullptr, 0.f);
+                       stream, x, wpk, out, g, ep, mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, (const float*)nullptr, 0.f, JoinParam<EPI>::of(ep));
     return hipGetLastError();
 }
 
@@ -508,12 +509,12 @@ static hipError_t launch_igemm_f32in(const float* x, const int8_t* wpk, void* ou
     const dim3 grid(n_pix_tiles, (g.K + TM - 1) / TM, 1);
 #define OHIP_IGF(E_)                                                                                                        \
     hipLaunchKernelGGL((conv_igemm_kernel<TM, TN, WM, WN, E_, 1, true>), grid, dim3(256), 0, stream, (const int8_t*)x, wpk, out, g, ep, \
-                       mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, in_scale, in_half)
+                       mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, in_scale, in_half, NoJoin{})
     switch (pick_epilogue(ep, g.K)) {
     case EPI_I8_P8: OHIP_IGF(EPI_I8_P8); break;
     case EPI_I8_P8_NONNEG: OHIP_IGF(EPI_I8_P8_NONNEG); break;
     case EPI_F32_P4:
-        if (ep.other != nullptr) return hipErrorInvalidValue;
+        if (ep.join != nullptr) return hipErrorInvalidValue;
         if (ep.fused()) OHIP_IGF(EPI_F32_P4_FUSED);
         else OHIP_IGF(EPI_F32_P4);
         break;
@@ -551,7 +552,8 @@ static hipError_t launch_igemm(const int8_t* x, const int8_t* wpk, void* out, co
     case EPI_I8_P8_NONNEG:
         return launch_igemm_e<TM, TN, WM, WN, EPI_I8_P8_NONNEG>(x, wpk, out, g, ep, stage, stream);
     case EPI_F32_P4:
-        if (ep.other != nullptr) return launch_igemm_e<TM, TN, WM, WN, EPI_F32_SHUFFLE>(x, wpk, out, g, ep, stage, stream);
+        if (ep.join != nullptr && ep.join->other != nullptr) return launch_igemm_e<TM, TN, WM, WN, EPI_F32_SHUFFLE>(x, wpk, out, g, ep, stage, stream);
+        if (ep.join != nullptr) return launch_igemm_e<TM, TN, WM, WN, EPI_F32_P4_PARTS>(x, wpk, out, g, ep, stage, stream);
         if (ep.fused())
             return launch_igemm_e<TM, TN, WM, WN, EPI_F32_P4_FUSED>(x, wpk, out, g, ep, stage, stream);
         return launch_igemm_e<TM, TN, WM, WN, EPI_F32_P4>(x, wpk, out, g, ep, stage, stream);

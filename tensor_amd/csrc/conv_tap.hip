@@ -53,7 +53,8 @@ struct TapArgs {
 
 template <int FM, int FN, int WK, int WN, int DEPTH, int EPI, bool INF>
 __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
-                                                                void* __restrict__ out, TapArgs ta, Epilogue ep) {
+                                                                void* __restrict__ out, TapArgs ta, Epilogue ep,
+                                                                JoinParam<EPI> ja) {
     constexpr int UNITS = FM / 2 * FN;  // (row-tile pair, pixel fragment) accumulators of a wave
     constexpr int OOB = (int)0x80000000;  // beyond any buffer here (below 2 GiB)
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
@@ -232,15 +233,15 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
                 const size_t o = ((size_t)(n * (unsigned)(Ks / 8) + ch / 8) * (unsigned)OHW + pix) * 8;
                 epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm, o, a8);
             } else if constexpr (EPI == EPI_F32_SHUFFLE) {
-                if (ep.lrelu) epi8_store_shuffle<1>(ep, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
-                else epi8_store_shuffle<0>(ep, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
+                if (ep.lrelu) epi8_store_shuffle<1>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
+                else epi8_store_shuffle<0>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
             } else {
-                constexpr bool FUSED = EPI == EPI_F32_P4_FUSED;
+                constexpr bool FUSED = EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_P4_PARTS;
                 const size_t e = ((size_t)(n * (unsigned)(Ks / 4) + ch / 4) * (unsigned)OHW + pix) * 4;
                 const float *r0 = nullptr, *r1 = nullptr;
-                if (FUSED && ep.residual1 != nullptr) {  // wave-uniform; one group then
-                    r0 = epi4_residual_at(ep, n, pix, ch0, g.K, OHW);
-                    r1 = epi4_residual_at(ep, n, pix, ch0 + 4, g.K, OHW);
+                if constexpr (EPI == EPI_F32_P4_PARTS) {  // (one group)
+                    r0 = epi4_residual_at(ep, ja, n, pix, ch0, g.K, OHW);
+                    r1 = epi4_residual_at(ep, ja, n, pix, ch0 + 4, g.K, OHW);
                 }
                 ohip_v2i tw = {0, 0};
                 tw[0] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si, prm.bi, e, a8[0], a8[1], a8[2], a8[3], r0);
@@ -306,7 +307,7 @@ bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
     const int epi = pick_epilogue(ep, kg);
     if (g.groups > 1 && (epi == EPI_GENERIC || ep.fused())) return false;
     if (ep.fused() && epi != EPI_F32_P4) return false;
-    if (f32in && (epi == EPI_GENERIC || ep.other != nullptr)) return false;
+    if (f32in && (epi == EPI_GENERIC || ep.join != nullptr)) return false;
     return (size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1) < ((size_t)1 << 31);  // 32-bit byte offsets
 }
 
@@ -334,7 +335,7 @@ hipError_t launch_tap(const void* x, const int8_t* wpk, void* out, const TapArgs
     const size_t lds = (size_t)ta.steps * 64 + (WK > 1 ? (size_t)WN * WK * (FM / 2) * FN * 2048 : 0);
     const dim3 grid((unsigned)ta.n_pix_tiles, (unsigned)((ta.g.K + 16 * FM - 1) / (16 * FM)), (unsigned)groups);
     hipLaunchKernelGGL((conv_tap_kernel<FM, FN, WK, WN, DEPTH, EPI, INF>), grid, dim3(64 * WK * WN), lds, stream, (const int8_t*)x,
-                       wpk, out, ta, ep);
+                       wpk, out, ta, ep, JoinParam<EPI>::of(ep));
     return hipGetLastError();
 }
 }  // namespace
@@ -392,11 +393,11 @@ hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out,
     const long px = (long)g.N * g.OH * g.OW, per = 16l * c.fn * c.wn;
     ta.n_pix_tiles = (int)((px + per - 1) / per);
     int epi = pick_epilogue(ep, g.K);
-    if (epi == EPI_F32_P4 && ep.fused()) epi = ep.other != nullptr ? EPI_F32_SHUFFLE : EPI_F32_P4_FUSED;
+    if (epi == EPI_F32_P4 && ep.fused()) epi = ep.join == nullptr ? EPI_F32_P4_FUSED : ep.join->other != nullptr ? EPI_F32_SHUFFLE : EPI_F32_P4_PARTS;
 #define OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, E_)                                                                           \
     if (config == I_ && epi == E_) {                                                                                        \
         if (!f32in) return launch_tap<FM_, FN_, WK_, WN_, D_, E_, false>(x, wpk, out, ta, ep, g_in.groups, stream);         \
-        if constexpr (E_ != EPI_GENERIC && E_ != EPI_F32_SHUFFLE && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g_in.groups, stream); \
+        if constexpr (E_ != EPI_GENERIC && E_ < EPI_F32_SHUFFLE && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g_in.groups, stream); \
     }
 #define OHIP_TAP(I_, FM_, FN_, WK_, WN_, D_)                 \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8)         \
@@ -404,6 +405,7 @@ hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out,
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4)        \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4_FUSED)  \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_SHUFFLE)   \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4_PARTS)  \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_GENERIC)
     OHIP_TAP(0, 2, 1, 8, 1, 4)
     OHIP_TAP(1, 2, 2, 4, 1, 4)

@@ -95,7 +95,8 @@ __global__ void __launch_bounds__(256) copy_channels4_kernel(const float* __rest
 
 // A whole Concat over channels in one launch: up to CONCAT_MAX packed fp32 sources, every channel count a multiple of
 // 4, into a packed destination; one thread per channel quad of one destination pixel, in destination memory order.
-// With qdst also the Byte8 quantization of the result (Cd % 8 == 0), as in copy_channels4_kernel.
+// With qdst also the Byte8 quantization of the result (Cd % 8 == 0), as in copy_channels4_kernel; dst may be null then.
+// Bound by its bytes. 256 channels @52x52, batch 16: 23.1 us with both results, 19.1 us with the int8 one alone.
 __global__ void __launch_bounds__(256) concat_channels4_kernel(ConcatSources srcs, float* __restrict__ dst, int Cd, int pd,
                                                                int H, int W, unsigned total4, int8_t* __restrict__ qdst,
                                                                float scale, float half) {
@@ -118,7 +119,7 @@ __global__ void __launch_bounds__(256) concat_channels4_kernel(ConcatSources src
         if (j < srcs.count && c >= srcs.first[j]) k = j;
     const float4 v = *reinterpret_cast<const float4*>(srcs.ptr[k] +
                                                       packed_off(n, c - srcs.first[k], y, x, srcs.channels[k], H, W, srcs.pack[k]));
-    *reinterpret_cast<float4*>(dst + packed_off(n, c, y, x, Cd, H, W, pd)) = v;
+    if (dst != nullptr) *reinterpret_cast<float4*>(dst + packed_off(n, c, y, x, Cd, H, W, pd)) = v;  // uniform
     if (qdst != nullptr) {  // uniform
         const float f[4] = {v.x, v.y, v.z, v.w};
         unsigned pk = 0;

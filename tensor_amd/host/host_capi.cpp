@@ -1,5 +1,6 @@
 // extern "C" facade over the C++ host layer, for hosts that cannot include otter_hip.hpp (the python tests and the
 // benchmark drive the Net through it). Options are "key=value;key=value" strings with the reference's own keys.
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 #include <memory>
@@ -190,7 +191,8 @@ int otter_host_net_run(void* net, const char* in_name, const void* x, int x_is_i
 // detection network): a pass extracts every one of them from the same Extractor, the fetch returns the last.
 struct otter_host_session {
     Net* net;
-    std::string in_name, out_name;
+    std::string in_name;
+    std::vector<std::string> out_names;
     Tensor in, out;
 };
 
@@ -200,7 +202,11 @@ void* otter_host_session_create(void* net, const char* in_name, const void* x, i
         auto* s = new otter_host_session();
         s->net = static_cast<Net*>(net);
         s->in_name = in_name;
-        s->out_name = out_name;
+        std::string names(out_name);
+        for (size_t at = 0, e; at <= names.size(); at = e + 1) {
+            e = std::min(names.find(',', at), names.size());
+            s->out_names.push_back(names.substr(at, e - at));
+        }
         s->in = Tensor::from_host(x, {n, c, h, w}, x_is_int8 ? ScalarType::Byte : ScalarType::Float);
         return s;
     } catch (const std::exception& e) {
@@ -214,13 +220,10 @@ int otter_host_session_pass(void* session) {
         auto* s = static_cast<otter_host_session*>(session);
         Extractor ex = s->net->create_extractor();
         if (ex.input(s->in_name, s->in)) return fail("no such input blob");
-        size_t pos = 0;
-        while (pos <= s->out_name.size()) {
-            size_t e = s->out_name.find(',', pos);
-            if (e == std::string::npos) e = s->out_name.size();
-            const int rc = ex.extract(s->out_name.substr(pos, e - pos), s->out, 1);
+        ex.only(s->out_names);
+        for (const std::string& name : s->out_names) {
+            const int rc = ex.extract(name, s->out, 1);
             if (rc) return fail("forward failed with code " + std::to_string(rc) + ": " + otter_hip_last_error());
-            pos = e + 1;
         }
         return 0;
     } catch (const std::exception& e) {
@@ -325,6 +328,7 @@ int otter_host_net_eval(void* net, int n_inputs, const char* const* in_names, co
                                                       in_is_int8[i] ? ScalarType::Byte : ScalarType::Float));
             if (ex.input(in_names[i], ins.back()->blob)) return fail(std::string("unknown blob ") + in_names[i]);
         }
+        ex.only({out_name});
         Tensor feat;
         const int rc = ex.extract(out_name, feat, 0);
         if (rc) return fail("forward failed with code " + std::to_string(rc) + ": " + otter_hip_last_error());

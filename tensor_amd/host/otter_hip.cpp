@@ -684,14 +684,14 @@ int ConvolutionLayer::create_pipeline_int8(const NetOption& opt) {
 }
 
 int ConvolutionLayer::forward(const Tensor& bottom, Tensor& top, const NetOption& opt) const {
-    if (int8_scale_term) return forward_int8(bottom, nullptr, fuse_scale, fuse_round, top, opt);
+    if (int8_scale_term) return forward_int8(bottom, nullptr, fuse_scale, fuse_round, top, opt, int8_only(opt));
     return -1;
 }
 
 int ConvolutionLayer::forward_residual(const Tensor& bottom, const Tensor& shortcut, float q_scale, int q_round, Tensor& sum,
-                                       const NetOption& opt) const {
+                                       const NetOption& opt, bool int8_only) const {
     if (!int8_scale_term || int8_scale_term > 100 || !shortcut.defined()) return 1;
-    return forward_int8(bottom, &shortcut, q_scale, q_round, sum, opt);
+    return forward_int8(bottom, &shortcut, q_scale, q_round, sum, opt, int8_only);
 }
 
 int ConvolutionLayer::forward_avgpool(const Tensor& bottom_in, Tensor& mean, const NetOption& opt) const {
@@ -718,7 +718,7 @@ int ConvolutionLayer::forward_avgpool(const Tensor& bottom_in, Tensor& mean, con
 
 // Tensor/ConvolutionLayer.cpp:754-847, whole batch in one launch; with `shortcut` the Eltwise sum behind it as well
 int ConvolutionLayer::forward_int8(const Tensor& bottom_in, const Tensor* shortcut, float q_scale, int q_round, Tensor& top,
-                                   const NetOption& opt) const {
+                                   const NetOption& opt, bool int8_only) const {
     if (!handle_ || !bottom_in.defined() || bottom_in.dim() != 4) return -1;
     // the producer may already have quantized this blob with this layer's scale (see Net::plan_fused_quantize)
     Tensor bottom = bottom_in, twin;
@@ -741,33 +741,37 @@ int ConvolutionLayer::forward_int8(const Tensor& bottom_in, const Tensor* shortc
             shortcut->channels() != out_channels || shortcut->size(2) != oh || shortcut->size(3) != ow)
             return 1;
     }
+    const bool with_q = q_scale > 0.f && out_layout == OTTER_HIP_F32_P4 && out_channels % 8 == 0;
+    const bool no_f32 = int8_only && with_q && otter_hip_conv_join_launches(handle_, in_layout, N, H, W) == 1;
     try {
-        top = Tensor::empty_device({N, out_channels / elempack_of(odt), oh, ow}, odt);
+        if (!no_f32) top = Tensor::empty_device({N, out_channels / elempack_of(odt), oh, ow}, odt);
         Tensor ws;
         const size_t ws_bytes = otter_hip_conv_workspace_bytes(handle_, in_layout, N, H, W);
         if (ws_bytes) ws = Tensor::empty_device({(int64_t)ws_bytes}, ScalarType::Byte);
         int rc;
-        const bool with_q = q_scale > 0.f && out_layout == OTTER_HIP_F32_P4 && out_channels % 8 == 0;
+        void* const out = no_f32 ? nullptr : top.device_ptr();
         if (shortcut) {
             Tensor q;
             if (with_q) q = Tensor::empty_device({N, out_channels / 8, oh, ow}, ScalarType::Byte8);
             rc = otter_hip_conv_forward_residual(handle_, bottom.device_ptr(), in_layout, N, H, W,
-                                                 (const float*)shortcut->device_ptr(), top.device_ptr(), out_layout,
+                                                 (const float*)shortcut->device_ptr(), out, out_layout,
                                                  with_q ? q.device_ptr() : nullptr, q_scale, q_round,
                                                  ws_bytes ? ws.device_ptr() : nullptr, ws_bytes, nullptr);
             if (rc) return rc;
             if (with_q) {
                 q.mark_device_written();
-                top.attach_quantized(q, q_scale, q_round);
+                if (no_f32) top = q;
+                else top.attach_quantized(q, q_scale, q_round);
             }
         } else if (with_q) {
             Tensor q = Tensor::empty_device({N, out_channels / 8, oh, ow}, ScalarType::Byte8);
-            rc = otter_hip_conv_forward_twin(handle_, bottom.device_ptr(), in_layout, N, H, W, top.device_ptr(), out_layout,
+            rc = otter_hip_conv_forward_twin(handle_, bottom.device_ptr(), in_layout, N, H, W, out, out_layout,
                                              q.device_ptr(), q_scale, q_round, ws_bytes ? ws.device_ptr() : nullptr,
                                              ws_bytes, nullptr);
             if (rc) return rc;
             q.mark_device_written();
-            top.attach_quantized(q, q_scale, q_round);
+            if (no_f32) top = q;
+            else top.attach_quantized(q, q_scale, q_round);
         } else {
             rc = otter_hip_conv_forward(handle_, bottom.device_ptr(), in_layout, N, H, W, top.device_ptr(), out_layout,
                                         ws_bytes ? ws.device_ptr() : nullptr, ws_bytes, nullptr);
@@ -794,7 +798,7 @@ bool ConvolutionLayer::join_input(const Tensor& bottom, const NetOption& opt, Te
 }
 
 int ConvolutionLayer::forward_residual_concat(const Tensor& bottom_in, const Tensor& part0, const Tensor& part1, float q_scale,
-                                              int q_round, Tensor& sum, const NetOption& opt) const {
+                                              int q_round, Tensor& sum, const NetOption& opt, bool int8_only) const {
     Tensor bottom;
     int oh = 0, ow = 0;
     if (!join_input(bottom_in, opt, bottom, oh, ow)) return 1;
@@ -805,19 +809,22 @@ int ConvolutionLayer::forward_residual_concat(const Tensor& bottom_in, const Ten
             return 1;
     if (part0.channels() + part1.channels() != out_channels) return 1;
     try {
-        sum = Tensor::empty_device({N, out_channels / 4, oh, ow}, ScalarType::Float4);
+        const bool no_f32 = int8_only && q_scale > 0.f;
+        if (!no_f32) sum = Tensor::empty_device({N, out_channels / 4, oh, ow}, ScalarType::Float4);
         Tensor q;
         if (q_scale > 0.f) q = Tensor::empty_device({N, out_channels / 8, oh, ow}, ScalarType::Byte8);
         const int rc = otter_hip_conv_forward_residual_concat(
             handle_, bottom.device_ptr(), OTTER_HIP_I8_P8, N, (int)bottom.size(2), (int)bottom.size(3), (const float*)part0.device_ptr(),
             hip_layout_of(part0.scalar_type()), (int)part0.channels(), (const float*)part1.device_ptr(),
-            hip_layout_of(part1.scalar_type()), (float*)sum.device_ptr(), q.defined() ? (int8_t*)q.device_ptr() : nullptr, q_scale,
+            hip_layout_of(part1.scalar_type()), no_f32 ? nullptr : (float*)sum.device_ptr(), q.defined() ? (int8_t*)q.device_ptr() : nullptr, q_scale,
             q_round, nullptr);
         if (rc) return rc;
-        sum.mark_device_written();
-        if (q.defined()) {
-            q.mark_device_written();
-            sum.attach_quantized(q, q_scale, q_round);
+        if (q.defined()) q.mark_device_written();
+        if (no_f32) {
+            sum = q;
+        } else {
+            sum.mark_device_written();
+            if (q.defined()) sum.attach_quantized(q, q_scale, q_round);
         }
     } catch (const Error&) {
         return -100;
@@ -826,7 +833,7 @@ int ConvolutionLayer::forward_residual_concat(const Tensor& bottom_in, const Ten
 }
 
 int ConvolutionLayer::forward_shuffle(const Tensor& bottom_in, const Tensor& other, bool other_odd, bool joined, float q_scale,
-                                      int q_round, Tensor& first, Tensor& second, const NetOption& opt) const {
+                                      int q_round, Tensor& first, Tensor& second, const NetOption& opt, bool int8_only) const {
     Tensor bottom;
     int oh = 0, ow = 0;
     if (!join_input(bottom_in, opt, bottom, oh, ow)) return 1;
@@ -836,21 +843,24 @@ int ConvolutionLayer::forward_shuffle(const Tensor& bottom_in, const Tensor& oth
         return 1;
     try {
         const std::vector<int64_t> sizes = {N, (joined ? 2 : 1) * out_channels / 8, oh, ow};
-        first = Tensor::empty_device(sizes, ScalarType::Float8);
-        if (!joined) second = Tensor::empty_device(sizes, ScalarType::Float8);
-        Tensor q;
+        Tensor q, &last = joined ? first : second;  // `last`: the blob that is quantized
         if (q_scale > 0.f) q = Tensor::empty_device(sizes, ScalarType::Byte8);
+        const bool no_f32 = int8_only && q.defined();
+        if (!no_f32) last = Tensor::empty_device(sizes, ScalarType::Float8);
+        if (!joined) first = Tensor::empty_device(sizes, ScalarType::Float8);
         int8_t* qp = q.defined() ? (int8_t*)q.device_ptr() : nullptr;
+        float *p1 = last.defined() ? (float*)last.device_ptr() : nullptr, *p0 = joined ? p1 : (float*)first.device_ptr();
         const int rc = otter_hip_conv_forward_shuffle(
             handle_, bottom.device_ptr(), OTTER_HIP_I8_P8, N, H, W, (const float*)other.device_ptr(), hip_layout_of(other.scalar_type()),
-            other_odd, (float*)first.device_ptr(), joined ? nullptr : (float*)second.device_ptr(), joined ? qp : nullptr,
-            joined ? nullptr : qp, joined, q_scale, q_round, nullptr);
+            other_odd, p0, joined ? nullptr : p1, joined ? qp : nullptr, joined ? nullptr : qp, joined, q_scale, q_round, nullptr);
         if (rc) return rc;
-        first.mark_device_written();
-        if (!joined) second.mark_device_written();
-        if (q.defined()) {
-            q.mark_device_written();
-            (joined ? first : second).attach_quantized(q, q_scale, q_round);
+        if (!joined) first.mark_device_written();
+        if (q.defined()) q.mark_device_written();
+        if (no_f32) {
+            last = q;
+        } else {
+            last.mark_device_written();
+            if (q.defined()) last.attach_quantized(q, q_scale, q_round);
         }
     } catch (const Error&) {
         return -100;
@@ -1300,37 +1310,43 @@ public:
         top_shapes = {s};
         return 0;
     }
-    int forward(const std::vector<Tensor>& b, std::vector<Tensor>& tops, const NetOption&) const override {
+    int forward(const std::vector<Tensor>& b, std::vector<Tensor>& tops, const NetOption& opt) const override {
         if (b.empty()) return -1;
         int64_t C = 0;
         for (const Tensor& t : b) {
             if (!f32_4d(t) || t.size(0) != b[0].size(0) || t.size(2) != b[0].size(2) || t.size(3) != b[0].size(3)) return -1;
             C += t.channels();
         }
-        Tensor out = empty_f32_device(b[0].size(0), C, b[0].size(2), b[0].size(3));
         // the readers are int8 convolutions: every copy also writes its channels of the quantized blob, when all of
         // them move whole quads of channels
-        bool with_q = fuse_scale > 0.f && C % 8 == 0 && out.elempack() % 4 == 0;
+        const int pack = best_pack(C);
+        bool with_q = fuse_scale > 0.f && C % 8 == 0;
         for (const Tensor& t : b) with_q = with_q && t.channels() % 4 == 0 && t.elempack() % 4 == 0;
         Tensor q;
         if (with_q) q = Tensor::empty_device({b[0].size(0), C / 8, b[0].size(2), b[0].size(3)}, ScalarType::Byte8);
-        bool quads = b.size() <= 8 && out.elempack() % 4 == 0;
+        bool quads = b.size() <= 8 && pack % 4 == 0;
         for (const Tensor& t : b) quads = quads && t.elempack() % 4 == 0;
+        const bool no_f32 = quads && with_q && int8_only(opt);
+        Tensor out;
+        if (!no_f32) out = empty_f32_device(b[0].size(0), C, b[0].size(2), b[0].size(3));
         if (quads) {  // every blob packed: the whole layer is one launch
             const float* ptrs[8];
             int layouts[8], channels[8];
             for (size_t i = 0; i < b.size(); ++i)
                 ptrs[i] = (const float*)b[i].device_ptr(), layouts[i] = hip_layout_of(b[i].scalar_type()), channels[i] = (int)b[i].channels();
-            if (otter_hip_concat_channels(ptrs, layouts, channels, (int)b.size(), (float*)out.device_ptr(),
-                                          hip_layout_of(out.scalar_type()), (int)b[0].size(0), (int)b[0].size(2),
+            if (otter_hip_concat_channels(ptrs, layouts, channels, (int)b.size(),
+                                          no_f32 ? nullptr : (float*)out.device_ptr(),
+                                          pack == 8 ? OTTER_HIP_F32_P8 : OTTER_HIP_F32_P4, (int)b[0].size(0), (int)b[0].size(2),
                                           (int)b[0].size(3), with_q ? (int8_t*)q.device_ptr() : nullptr, fuse_scale, fuse_round,
                                           nullptr))
                 return -1;
-            out.mark_device_written();
-            if (with_q) {
-                q.mark_device_written();
-                out.attach_quantized(q, fuse_scale, fuse_round);
+            if (with_q) q.mark_device_written();
+            if (no_f32) {
+                tops.assign(1, q);
+                return 0;
             }
+            out.mark_device_written();
+            if (with_q) out.attach_quantized(q, fuse_scale, fuse_round);
             tops.assign(1, out);
             return 0;
         }
@@ -1925,32 +1941,42 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
 // -- an element-wise sum, a channel concatenation, an int8 convolution with an fp32 result -- does it on the way (one
 // pass over the blob instead of two, one launch less per reader). Readers behind the automatic Split layers count.
 void Net::plan_fused_quantize() const {
+    root_.resize(blobs_.size());
+    for (size_t b = 0; b < root_.size(); ++b) root_[b] = (int)b;
     for (Layer* l : layers_) {
         l->fuse_scale = 0.f;
+        l->fuse_only = false;
         if (l->tops.size() != 1 || l->type() == "Split" || l->type() == "Input") continue;
         if (const auto* pc = dynamic_cast<const ConvolutionLayer*>(l))
             if (!pc->int8_scale_term || pc->int8_scale_term > 100) continue;  // fp32 results only
         std::vector<int> pending(l->tops.begin(), l->tops.end());
         float scale = 0.f;
         int round = 0;
-        bool agree = true;
+        bool agree = true, all = true;  // all: every reader is one of those convolutions
         while (!pending.empty()) {
             const int b = pending.back();
             pending.pop_back();
+            all = all && !blobs_[b].consumers.empty();
             for (int ci : blobs_[b].consumers) {
                 const Layer* c = layers_[ci];
                 if (c->type() == "Split") {
+                    for (int t : c->tops) root_[t] = l->tops[0];
                     pending.insert(pending.end(), c->tops.begin(), c->tops.end());
                 } else if (const auto* conv = dynamic_cast<const ConvolutionLayer*>(c)) {
-                    if (!conv->int8_scale_term || !conv->bottom_blob_int8_scales.defined() || conv->in_channels % 8) continue;
+                    if (!conv->int8_scale_term || !conv->bottom_blob_int8_scales.defined() || conv->in_channels % 8) {
+                        all = false;
+                        continue;
+                    }
                     const float s = conv->bottom_blob_int8_scales.data_ptr<float>()[0];
                     const int r = conv->input_round_mode(option);
                     if (scale != 0.f && (s != scale || r != round)) agree = false;
                     scale = s, round = r;
+                } else {
+                    all = false;
                 }
             }
         }
-        if (agree && scale > 0.f) l->fuse_scale = scale, l->fuse_round = round;
+        if (agree && scale > 0.f) l->fuse_scale = scale, l->fuse_round = round, l->fuse_only = all;
     }
     // Residual block tails: Eltwise / ShortCut sum of two blobs, one the fp32 result of an int8 convolution read by
     // nothing else
@@ -2002,7 +2028,7 @@ void Net::plan_fused_quantize() const {
             if (!pc || !pc->int8_scale_term || pc->int8_scale_term > 100 || pc->force_out_layout >= 0 || pc->bottoms.size() != 1) continue;
             if (blobs_[b].consumers.size() == 1 && pi > conv) conv = pi, conv_k = k;
         }
-        const ShuffleUnit whole{(int)ci, si, -1, -1, sh->fuse_scale, sh->fuse_round, conv, conv_k};
+        const ShuffleUnit whole{(int)ci, si, -1, -1, sh->fuse_scale, sh->fuse_round, sh->fuse_only, conv, conv_k};
         if (conv >= 0) shuffle_units_[si] = whole;
         int sp = sole_reader(sh->tops[0]);
         if (sp < 0 || layers_[sp]->type() != "Split" || layers_[sp]->tops.size() != 2) continue;
@@ -2030,7 +2056,7 @@ void Net::plan_fused_quantize() const {
             if (hs != 0.f && (sc != hs || r != hr)) agree = false;
             hs = sc, hr = r;
         }
-        const ShuffleUnit u{(int)ci, si, lo, hi, agree && hs > 0.f ? hs : 0.f, hr, conv, conv_k};
+        const ShuffleUnit u{(int)ci, si, lo, hi, agree && hs > 0.f ? hs : 0.f, hr, agree && hs > 0.f, conv, conv_k};
         shuffle_units_[lo] = u;
         shuffle_units_[hi] = u;
     }
@@ -2158,7 +2184,8 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
                 const int rc = forward_layer(blobs_[b].producer, blobs, opt);
                 if (rc) return rc;
             }
-        const int rc = conv->forward_residual_concat(blobs[conv->bottoms[0]], blobs[p0], blobs[p1], e->fuse_scale, e->fuse_round, sum, opt);
+        const int rc = conv->forward_residual_concat(blobs[conv->bottoms[0]], blobs[p0], blobs[p1], e->fuse_scale, e->fuse_round, sum, opt,
+                                                     e->int8_only(opt));
         if (rc < 0) return rc;
         if (rc == 0) {
             blobs[e->tops[0]] = sum;
@@ -2173,7 +2200,8 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
             const int rc = forward_layer(blobs_[b].producer, blobs, opt);
             if (rc) return rc;
         }
-    const int rc = conv->forward_residual(blobs[conv->bottoms[0]], blobs[u.shortcut], e->fuse_scale, e->fuse_round, sum, opt);
+    const int rc = conv->forward_residual(blobs[conv->bottoms[0]], blobs[u.shortcut], e->fuse_scale, e->fuse_round, sum, opt,
+                                          e->int8_only(opt));
     if (rc) return rc;
     blobs[e->tops[0]] = sum;
     if (opt.lightmode)
@@ -2207,7 +2235,10 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
         }
     const bool joined = u.crop_lo < 0;
     Tensor first, second;
-    const int rc = conv->forward_shuffle(blobs[in_blob], blobs[other], u.conv_k == 0, joined, u.hi_scale, u.hi_round, first, second, opt);
+    const int last = joined ? layers_[u.shuffle]->tops[0] : layers_[u.crop_hi]->tops[0];
+    const bool int8_only = u.hi_only && opt.wanted && !(*opt.wanted)[last];
+    const int rc = conv->forward_shuffle(blobs[in_blob], blobs[other], u.conv_k == 0, joined, u.hi_scale, u.hi_round, first, second, opt,
+                                         int8_only);
     if (rc) return rc;
     if (joined) {
         blobs[layers_[u.shuffle]->tops[0]] = first;
@@ -2276,6 +2307,15 @@ Extractor Net::create_extractor() const {
 Extractor::Extractor(const Net* net, size_t blob_count) : option(net->option), net_(net), blob_tensors_(blob_count) {}
 
 void Extractor::clear() { blob_tensors_.assign(blob_tensors_.size(), Tensor()); }
+
+void Extractor::only(const std::vector<std::string>& names) {
+    auto wanted = std::make_shared<std::vector<char>>(blob_tensors_.size());
+    for (const std::string& name : names) {
+        const int i = net_->find_blob_index_by_name(name);
+        if (i >= 0) (*wanted)[i] = (*wanted)[net_->root_[i]] = 1;
+    }
+    option.wanted = wanted;
+}
 
 int Extractor::input(const std::string& name, const Tensor& in) {
     const int i = net_->find_blob_index_by_name(name);

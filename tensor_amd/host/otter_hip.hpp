@@ -112,6 +112,9 @@ public:
     bool use_packing_layout = true;
     bool use_fp16_storage = true;
     int openmp_blocktime = 20;
+    // set by Extractor::only: by blob, whether it (or a Split of it) will be asked for. Null: any blob may be, so every fp32 blob
+    // is made; else one that only int8 convolutions read may exist as their common int8 input alone.
+    std::shared_ptr<const std::vector<char>> wanted;
 };
 enum class CompileMode { Inference, Initial };
 
@@ -183,6 +186,10 @@ public:
     // int8 blob to its top blob (Tensor::attach_quantized); one that cannot ignores the two.
     float fuse_scale = 0.f;
     int fuse_round = 0;
+    bool fuse_only = false;  // with fuse_scale > 0: nothing but those convolutions reads the blob
+    bool int8_only(const NetOption& opt) const {
+        return fuse_only && fuse_scale > 0.f && opt.use_packing_layout && opt.wanted && !(*opt.wanted)[tops[0]];
+    }
 };
 
 // Tensor/LayerRegistry.hpp:17-85: string-keyed factory; a later AddCreator overrides an earlier one
@@ -232,7 +239,7 @@ public:
     // with q_scale (> 0) for the int8 convolutions that read the sum. Returns 1, and does nothing, when the blobs do not
     // have the layouts that takes (the caller then runs the two layers one after the other).
     int forward_residual(const Tensor& bottom_blob, const Tensor& shortcut, float q_scale, int q_round, Tensor& sum,
-                         const NetOption& opt) const;
+                         const NetOption& opt, bool int8_only = false) const;
     // This layer (fp32 result) and the global average pooling that is its only reader through
     // otter_hip_conv_forward_avgpool, when that is one launch for this input; `mean` is [N, K, 1, 1]. Returns 1, and does
     // nothing, otherwise (the caller then runs the two layers one after the other).
@@ -241,10 +248,10 @@ public:
     // (otter_hip_conv_forward_shuffle): the shuffled channels' two halves, or with `joined` the whole blob in `first`; q_scale
     // > 0 also quantizes the second half (joined: the blob). Returns 1, and does nothing, when that is not one launch here.
     int forward_shuffle(const Tensor& bottom_blob, const Tensor& other, bool other_odd, bool joined, float q_scale, int q_round,
-                        Tensor& first, Tensor& second, const NetOption& opt) const;
+                        Tensor& first, Tensor& second, const NetOption& opt, bool int8_only) const;
     // forward_residual where the shortcut is the concatenation of two blobs (otter_hip_conv_forward_residual_concat)
     int forward_residual_concat(const Tensor& bottom_blob, const Tensor& part0, const Tensor& part1, float q_scale, int q_round,
-                                Tensor& sum, const NetOption& opt) const;
+                                Tensor& sum, const NetOption& opt, bool int8_only) const;
     // what otter_hip_conv_block_launches says of the three layers on an input of this size
     static int block_launches(const ConvolutionLayer* expand, const ConvolutionLayer* depthwise, const ConvolutionLayer* project,
                               int n, int h, int w);
@@ -265,8 +272,9 @@ private:
     // the int8 blob that a launch with another layer's work in its epilogue reads, and that launch's output size; false: no such launch
     bool join_input(const Tensor& bottom_blob, const NetOption& opt, Tensor& input, int& out_h, int& out_w) const;
     int create_pipeline_int8(const NetOption& opt);
+    // int8_only: top_blob is the int8 blob itself where the launch can leave the fp32 one out
     int forward_int8(const Tensor& bottom_blob, const Tensor* shortcut, float q_scale, int q_round, Tensor& top_blob,
-                     const NetOption& opt) const;
+                     const NetOption& opt, bool int8_only) const;
     otter_hip_conv* handle_ = nullptr;
 };
 
@@ -341,6 +349,7 @@ private:
     std::vector<Blob> blobs_;
     std::vector<LayerOption> layer_options_;
     mutable bool planned_ = false;
+    mutable std::vector<int> root_;  // by blob: the blob that it is a Split's share of (itself otherwise)
     // Concat(a, b) -> ChannelShuffle(2) -> Crop(first half) + Crop(second half), found by the plan: either Crop layer's
     // index -> the unit; forward_layer runs the whole unit in one kernel when none of its inner blobs exists yet. Without
     // the Crops (-1) the unit is the ChannelShuffle layer's and needs a convolution to run in.
@@ -348,6 +357,7 @@ private:
         int concat, shuffle, crop_lo, crop_hi;
         float hi_scale;  // > 0: the second half is read by int8 convolutions with this input scale ...
         int hi_round;    // ... and this rounding primitive: quantize it on the way
+        bool hi_only;    // ... and by nothing else
         int conv;        // the int8 convolution whose fp32 result is bottom conv_k of the Concat and read by nothing else, or -1
         int conv_k;
     };
@@ -395,6 +405,8 @@ public:
     int input(const std::string& blob_name, const Tensor& in);
     // type 0: unpacked (elempack 1) host-visible result, as the reference; type 1: whatever layout the layer left
     int extract(const std::string& blob_name, Tensor& feat, int type);
+    // Promises that no blob but these will be extracted, which spares the pass fp32 blobs that nothing else reads.
+    void only(const std::vector<std::string>& blob_names);
     NetOption option;
 
 private:
