@@ -1,5 +1,6 @@
 """The fp32 glue entry points of the C ABI called directly, with every combination of source and destination layout
 (elempack 1, 4, 8), against numpy / torch definitions: the host layer only ever uses a few of these combinations."""
+import ctypes
 import itertools
 
 import numpy as np
@@ -142,6 +143,29 @@ def test_concat_channels_in_one_launch(hip, oracle, packs, with_q):
     np.testing.assert_array_equal(_host(dst, packs[3], want.shape), want)
     if with_q:
         np.testing.assert_array_equal(_host(q, 8, want.shape), oracle.quantize(want, [scale], capi.ROUND_SSE))
+
+
+@pytest.mark.parametrize("N,H,W,channels", [(1, 1, 1, (8, 8)), (3, 9, 14, (8, 40)), (2, 1, 128, (16, 8)), (2, 7, 73, (8, 16)),
+                                            (1, 16, 32, (24, 8)), (2, 27, 19, (8, 8, 8, 8, 8, 8, 8, 8)), (2, 33, 31, (40,)),
+                                            (2, 9, 7, (12, 4))], ids=str)
+def test_concat_image_sizes(hip, oracle, N, H, W, channels):
+    """Around the pixels that a workgroup moves (128 and 512, and where the two sizes meet), with and without the fp32 blob."""
+    rng = np.random.default_rng(H * W)
+    parts = [rng.normal(0, 1, (N, c, H, W)).astype(np.float32) for c in channels]
+    want = np.concatenate(parts, axis=1)
+    want_q = oracle.quantize(want, [37.5], capi.ROUND_EXACT)
+    packs = [8 if c % 8 == 0 and i % 2 else 4 for i, c in enumerate(channels)]
+    srcs, layouts = [_dev(hip, a, p) for a, p in zip(parts, packs)], [F32[p] for p in packs]
+    for pack in (4, 8):
+        dst, q = hip.concat_channels(srcs, layouts, list(channels), N, H, W, F32[pack], 37.5, capi.ROUND_EXACT)
+        np.testing.assert_array_equal(_host(dst, pack, want.shape), want)
+        np.testing.assert_array_equal(_host(q, 8, want.shape), want_q)
+    ptrs = (ctypes.c_void_p * len(srcs))(*[t.data_ptr() for t in srcs])
+    q = hip.empty(want.size, np.int8)
+    ints = ctypes.c_int * len(srcs)
+    hip._check(hip.lib.otter_hip_concat_channels(ptrs, ints(*layouts), ints(*channels), len(srcs), None, F32[8], N, H, W, hip.ptr(q),
+                                                 ctypes.c_float(37.5), capi.ROUND_EXACT, hip.stream()))
+    np.testing.assert_array_equal(_host(q, 8, want.shape), want_q)
 
 
 @pytest.mark.parametrize("mode", [capi.ROUND_SSE, capi.ROUND_EXACT])
