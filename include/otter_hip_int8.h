@@ -262,15 +262,14 @@ int otter_hip_conv_chain_set_min_tiles(int tiles);
  * calls give, bit for bit. Where the depthwise layer is stride 1 pad 1 on an image at most 64 pixels wide, the first
  * layer reads at most 192 channels and the activations are none / ReLU / clip, the block can run as ONE launch that
  * keeps the expanded tensor in LDS; it does (otter_hip_conv_block_launches says 1) for the
- * shapes where that was measured faster than the three launches (images up to 28 pixels wide, 128..512 workgroups
- * over the batch, at most 24 tiles of 32 channels x 16 pixels of the last layer per band), or for every shape that qualifies after
+ * shapes where a cost model fitted to measured blocks says that it is the fastest form, or for every shape that qualifies after
  * otter_hip_conv_block_set_always(1) / a forced plan. Where a batch has fewer bands than half the compute units, the
  * expanded channels of a band are dealt to several workgroups whose accumulators meet in `workspace` (the last to
  * arrive adds them up: integer sums, the same result). Otherwise, where the first layer reads at most 128 channels and
  * writes a multiple of 16, the depthwise layer is 3x3 stride 1 / 2 on an image at most 128 pixels wide (64 when the first
  * layer reads more than 32 channels) and both clamp at zero or neither clamps, the first two layers can run as ONE
  * launch that keeps the expanded rows in LDS, the last layer by itself; they do (otter_hip_conv_block_launches says 2)
- * where that was measured faster, or wherever they can after otter_hip_conv_block_set_pair(1); any other block makes
+ * where the model says so, or wherever they can after otter_hip_conv_block_set_pair(1); any other block makes
  * three launches. The blobs between the launches live in `workspace`;
  * otter_hip_conv_block_workspace_bytes gives the size either way (0 for a single launch with one workgroup per band). */
 int otter_hip_conv_block_launches(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise,

@@ -1102,6 +1102,55 @@ static bool block_geoms(const otter_hip_conv_t* e, const otter_hip_conv_t* d, co
 
 static int g_block_always = 0;  // see block_single_launch
 
+// The three forms of a block, in microseconds a call: three launches, the first two layers as one (conv_xdw.hip) and the last
+// by itself, the whole block as one (conv_block.hip). Fitted to 770 blocks drawn over 16..160 input channels, 7x7..112x112,
+// batch 1..64, the calls queued behind one another; median errors 5, 6 and 6 %. The form chosen by them is 0.9 % slower than
+// the fastest of each block on average. Small blocks gain most, being launch latency: 24 -> 144 -> 24 @12x17 b9 11.5 us as three
+// launches, 8.8 as two, 8.0 as one; 29x29 48 -> 288 -> 48 b29 24.5, 23.8, 14.2; but 23x23 152 -> 912 -> 152 b14 24.8 as three,
+// 35.6 as one, and 36x36 stride 2 112 -> 672 -> 232 b38 48.7 as three, 60.0 as two.
+static float block_cost_three(const ConvGeom g[3]) {
+    const float px = (float)g[0].N * g[0].H * g[0].W * 1e-6f, opx = (float)g[2].N * g[2].OH * g[2].OW * 1e-6f;
+    const float ce = (float)g[0].K, mac_e = px * ce * igemm_channel_groups(g[0].C);
+    const float mac_p = opx * igemm_channel_groups(g[2].C) * (float)((g[2].K + 31) / 32 * 32);
+    return 12.6f + 0.22f * px * ce + 0.41f * opx * ce + 0.78f * opx * g[2].K + 0.198f * mac_e + 0.194f * mac_p;
+}
+static float block_cost_pair(const ConvGeom g[3]) {
+    float rows;  // of the busiest SIMD
+    xdw_strip_rows(g[1], &rows);
+    const float opx = (float)g[2].N * g[2].OH * g[2].OW * 1e-6f, groups = (float)xdw_pixel_groups(g[0].W);
+    const float mac_p = opx * igemm_channel_groups(g[2].C) * (float)((g[2].K + 31) / 32 * 32);
+    return 8.6f + 0.01f * rows * (1.43f + groups * (g[0].C > 32 ? 0.43f : 0.2f)) + 0.44f * opx * g[2].C + 0.2f * opx * g[2].K +
+           0.433f * mac_p;
+}
+static float block_cost_single(const ConvGeom g[3], const int plan[6]) {
+    const int rb = plan[0], sl = plan[2], split = plan[4], W = g[0].W;
+    const long wgs = (long)g[0].N * plan[1] * split;
+    // one workgroup per compute unit, or two that hide part of each other
+    const float rounds = plan[3] > 80 * 1024 ? (float)((wgs + 255) / 256) : wgs <= 256 ? 1.f : fmaxf(1.f, 0.7f * (float)((wgs + 255) / 256));
+    const float slices = (float)(((g[0].K + sl - 1) / sl + split - 1) / split);
+    const float tiles_e = (float)((std::min(rb + 2, g[0].H) * W + 15) / 16) * sl * 1e-3f;
+    const float items = (float)((g[2].K + 31) / 32 * ((rb * W + 15) / 16));
+    return 3.56f + rounds * (slices * (1.59f + tiles_e * (1.39f + 0.3f * igemm_channel_groups(g[0].C))) + 0.096f * items) +
+           (split > 1 ? 1.f + 0.056f * items * split : 0.f);
+}
+
+// What a stride-1 block of 64 input channels or more has to gain where its three launches are launch latency throughout: such a
+// block of the dispatch's test stays three launches at a small batch (64 -> 384 -> 64 @14x14 b4: 11.3 us, 8.8 as one). Over
+// the drawn blocks the choice costs 2 % against the best form with it, 0.9 % without.
+static float block_margin(const ConvGeom g[3], float us) { return g[0].C >= 64 && block_cost_three(g) < 14.f ? us : 0.f; }
+
+// The first two layers of a block as one launch (conv_xdw.hip), the last by itself. 0: where the cost models say so; 1: wherever
+// the kernel takes the shapes; -1: never.
+static int g_block_pair = 0;
+
+static bool block_pair_takes(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const ConvGeom g[3]) {
+    if (!e->w_xdw || e->c_pad || e->force_tm || !d->w_dw_mfma || d->c_pad || d->force_tm) return false;
+    const Epilogue e1 = make_epilogue(e, OTTER_HIP_I8_P8), e2 = make_epilogue(d, OTTER_HIP_I8_P8);
+    if (!xdw_applicable(g[0], e1, pick_epilogue(e1, g[0].K), e->so_positive, g[1], e2, dw_mfma_epilogue(e2, g[1].K), d->so_positive))
+        return false;
+    return g[0].C <= 32 || g[0].W <= 64;  // (the other instances of the kernel do not fit the register file)
+}
+
 static bool block_single_launch(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
                                 const ConvGeom g[3], int out_layout, int plan[6]) {
     if (g_block_always == 2) return false;  // (tuning hook: never)
@@ -1112,36 +1161,16 @@ static bool block_single_launch(const otter_hip_conv_t* e, const otter_hip_conv_
     if (!conv_block_applicable(g[0], e1, g[1], e2, g[2], e3)) return false;
     if (!conv_block_plan(g[0], g[2], e->block_rb, e->block_sl, e->block_split, plan)) return false;
     if (g_block_always == 1 || e->block_rb || e->block_sl || e->block_split) return true;
-    // The single launch pays where the three layers are short, latency-bound launches and its workgroups (a band of
-    // rows of one image each, or a share of a band's expanded channels) about fill the 256 compute units once.
-    // Measured at batch 64 against the three launches (kernel trace; in brackets the three launches inside a network,
-    // where each starts on cold inputs): 14x14 64 -> 384 -> 64 13.2 us against 17.8, 14x14 96 -> 576 -> 96 21.8 against
-    // 23.5 (29.8), 28x28 32 -> 192 -> 32 15.2 against 21.8, 7x7 160 -> 960 -> 160 with the slices of an image dealt to
-    // four workgroups 18.5 against 20 (23.4), 7x7 160 -> 960 -> 320 as two bands of 20 project tiles, each dealt to two
-    // workgroups, 20.8 against 20.3 (24.4). Not taken: 56x56 24 -> 144 -> 24 (896 workgroups of 13 us each on 256
-    // compute units) 53 against 45.
-    const long wgs = (long)g[0].N * plan[1] * plan[4];
-    const int items = ((g[2].K + 31) / 32) * ((plan[0] * g[0].W + 15) / 16);
-    return g[0].C <= 192 && g[0].W <= 28 && wgs >= 128 && wgs <= 512 && items <= 24;
+    const float single = block_cost_single(g, plan);
+    return single < block_cost_three(g) - block_margin(g, 3.8f) && (!block_pair_takes(e, d, g) || single < block_cost_pair(g));
 }
 
-// The first two layers of a block as one launch (conv_xdw.hip), the last by itself: where the single launch of the
-// whole block is not taken. 0: where it was measured faster than the two layers one by one; 1: wherever the kernel
-// takes the shapes; -1: never.
-static int g_block_pair = 0;
-
 static bool block_pair_launch(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const ConvGeom g[3]) {
-    if (g_block_pair < 0 || !e->w_xdw || e->c_pad || e->force_tm || !d->w_dw_mfma || d->c_pad || d->force_tm) return false;
-    const Epilogue e1 = make_epilogue(e, OTTER_HIP_I8_P8), e2 = make_epilogue(d, OTTER_HIP_I8_P8);
-    if (!xdw_applicable(g[0], e1, pick_epilogue(e1, g[0].K), e->so_positive, g[1], e2, dw_mfma_epilogue(e2, g[1].K), d->so_positive))
-        return false;
-    if (g[0].C > 32 && g[0].W > 64) return false;  // (those instances of the kernel do not fit the register file)
-    if (g_block_pair > 0) return true;
-    // Measured at batch 64 against the two layers one by one (kernel trace): with a stride-2 depthwise layer, where the
-    // expanded blob is four times what the launch writes, 16 -> 96 @112x112 29.5 us against 46, 24 -> 144 @56x56 17.9
-    // against 27, 32 -> 192 @28x28 9.7 against 15, 96 -> 576 @14x14 13.2 against 15; with stride 1 24 -> 144 @56x56 28.6
-    // against 31, and the 88 / 176-channel units of the detection model at 52x52 .. 13x13 (batch 16) no gain.
-    return g[1].sh == 2 || (size_t)g[0].N * g[0].K * g[0].OH * g[0].OW >= ((size_t)16 << 20);
+    if (g_block_pair < 0 || !block_pair_takes(e, d, g)) return false;
+    // (10 %: inside a network each of three launches starts on a blob that the last one has just written, which the calls that
+    // were fitted do not show: 96 -> 576 @14x14 stride 2 b64, first two layers, 13.2 us as one launch there, 15 as two)
+    const float three = block_cost_three(g);
+    return g_block_pair > 0 || block_cost_pair(g) < (g[1].sh == 2 ? 1.1f * three : three - block_margin(g, 2.8f));
 }
 
 static int block_default_out_layout(const otter_hip_conv_t* p) {

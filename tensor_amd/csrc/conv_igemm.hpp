@@ -99,6 +99,8 @@ hipError_t run_conv_pw_avgpool(const int8_t* x, const int8_t* wpk, float* out, c
 // pointwise int8 -> int8 convolution + depthwise 3x3 int8 -> int8 convolution as one launch (conv_xdw.hip)
 size_t xdw_weight_bytes(int Cin, int K);
 void xdw_pack_weights(const int8_t* w, int Cin, int K, int8_t* dst);
+int xdw_strip_rows(const ConvGeom& g, float* cost);
+int xdw_pixel_groups(int W);
 bool xdw_applicable(const ConvGeom& gx, const Epilogue& epx, int epi_x, bool sox_positive, const ConvGeom& gd, const Epilogue& ep,
                     int epi_d, bool so_positive);
 hipError_t run_conv_xdw(const int8_t* x, const int8_t* wx, const int8_t* wa, void* out, const ConvGeom& gx, const Epilogue& epx,

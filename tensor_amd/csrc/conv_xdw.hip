@@ -289,34 +289,39 @@ bool xdw_applicable(const ConvGeom& gx, const Epilogue& epx, int epi_x, bool sox
     return (long)gd.N * (gd.C / 16) <= 65535;
 }
 
+// Strips of equal height. The kernel is bound by the vector instructions of its rows, so the launch lasts about as
+// long as the busiest of the chip's 1024 SIMDs: (waves per SIMD, rounded up) x (input rows a wave walks + about two
+// rows' worth of set-up). More strips balance the SIMDs better and recompute more halo rows; take the count that
+// minimises the product, the fewest strips among equals.
+int xdw_strip_rows(const ConvGeom& g, float* cost_out) {
+    const long planes = (long)g.N * (g.C / 16);
+    long best = -1;
+    int rps = g.OH;
+    for (int r = g.OH; r >= 1; --r) {
+        const int ns = (g.OH + r - 1) / r;
+        const long per_simd = (planes * ns + 1023) / 1024;
+        // (a lone wave issues a vector instruction every 6 cycles where two or more reach the pipe's 4)
+        const long cost = per_simd * ((r - 1) * g.sh + 3 + 2) * (per_simd == 1 ? 15 : per_simd == 2 ? 11 : 10);
+        if (best < 0 || cost < best) best = cost, rps = r;
+    }
+    if (cost_out) *cost_out = (float)best;
+    return rps;
+}
+int xdw_pixel_groups(int W) {
+    const int ng = (W + 15) / 16;
+    return ng <= 1 ? 1 : (ng <= 2 ? 2 : (ng <= 4 ? 4 : (ng <= 7 ? 7 : 8)));
+}
+
 hipError_t run_conv_xdw(const int8_t* x, const int8_t* wx, const int8_t* wa, void* out, const ConvGeom& gx, const Epilogue& epx,
                         const ConvGeom& g, const Epilogue& ep, int epi_d, int strip_rows, hipStream_t stream) {
     if (g.N == 0 || g.OH * g.OW == 0) return hipSuccess;
     const long planes = (long)g.N * (g.C / 16);
     if (planes > 65535) return hipErrorInvalidValue;
-    // Strips of equal height. The kernel is bound by the vector instructions of its rows, so the launch lasts about as
-    // long as the busiest of the chip's 1024 SIMDs: (waves per SIMD, rounded up) x (input rows a wave walks + about two
-    // rows' worth of set-up). More strips balance the SIMDs better and recompute more halo rows; take the count that
-    // minimises the product, the fewest strips among equals.
-    int rps;
-    if (strip_rows > 0) {
-        rps = std::min(strip_rows, g.OH);
-    } else {
-        long best = -1;
-        rps = g.OH;
-        for (int r = g.OH; r >= 1; --r) {
-            const int ns = (g.OH + r - 1) / r;
-            const long per_simd = (planes * ns + 1023) / 1024;
-            // (a lone wave issues a vector instruction every 6 cycles where two or more reach the pipe's 4)
-            const long cost = per_simd * ((r - 1) * g.sh + 3 + 2) * (per_simd == 1 ? 15 : per_simd == 2 ? 11 : 10);
-            if (best < 0 || cost < best) best = cost, rps = r;
-        }
-    }
+    const int rps = strip_rows > 0 ? std::min(strip_rows, g.OH) : xdw_strip_rows(g, nullptr);
     const int n_strips = (g.OH + rps - 1) / rps;
     const int wpb = n_strips % 4 == 0 ? 4 : (n_strips % 2 == 0 ? 2 : 1);
     const dim3 grid((unsigned)(n_strips / wpb), (unsigned)planes), block(64 * wpb);
-    const int ng = (g.W + 15) / 16;
-    const int NG = ng <= 1 ? 1 : (ng <= 2 ? 2 : (ng <= 4 ? 4 : (ng <= 7 ? 7 : 8)));
+    const int NG = xdw_pixel_groups(g.W);
     const int nch = (NG + 3) / 4;
     const unsigned lds_bytes = (unsigned)wpb * 2u * (4u * (64u * nch + 8u) * 8u + 128u);
     const unsigned in_bytes = (unsigned)((size_t)gx.N * gx.C * gx.H * gx.W);
