@@ -288,13 +288,14 @@ int otter_hip_conv_block_forward(const otter_hip_conv_t* expand, const otter_hip
 int otter_hip_conv_block_plan(int in_channels, int expanded_channels, int out_channels, int n, int in_h, int in_w,
                               int rows_per_band, int slice_channels, int split, int plan[6]);
 /* Tuning / test hook with no counterpart in the reference: 1 = every block that qualifies by shape runs as the single
- * launch, 0 = only the shapes measured faster that way (default), 2 = none does. Process-wide; returns the previous
+ * launch, 0 = those for which the cost models say that it is the fastest form (default), 2 = none does. Process-wide; returns the previous
  * value; a negative argument only queries. */
 int otter_hip_conv_block_set_always(int on);
-/* Tuning / test hook with no counterpart in the reference: how a block that does not run as the single launch runs its
- * first two layers: 0 = as one launch where that was measured faster (a stride-2 depthwise layer, or an expanded blob
- * of 16 MiB or more; default), 1 = wherever the kernel takes the shapes, -1 = always one by one. Process-wide; returns
- * the previous value; any other argument only queries. */
+/* Tuning / test hook with no counterpart in the reference: how a block runs its first two layers: 0 = as the cost models say
+ * (default), 1 = as one launch, the last layer by itself, wherever the kernel takes the shapes, -1 = one by one, three launches.
+ * 1 and -1 come before the models' choice of the single launch of the whole block, but not before a single launch that
+ * otter_hip_conv_block_set_always(1) or a forced plan asks for. Process-wide; returns the previous value; any other argument only
+ * queries. */
 int otter_hip_conv_block_set_pair(int mode);
 /* Tuning / test hook with no counterpart in the reference: force the single launch's output rows per band, the
  * expanded channels per LDS slice (64 or 128) and the workgroups a band's slices are dealt to, for blocks whose first

@@ -1140,7 +1140,7 @@ static float block_cost_single(const ConvGeom g[3], const int plan[6]) {
 static float block_margin(const ConvGeom g[3], float us) { return g[0].C >= 64 && block_cost_three(g) < 14.f ? us : 0.f; }
 
 // The first two layers of a block as one launch (conv_xdw.hip), the last by itself. 0: where the cost models say so; 1: wherever
-// the kernel takes the shapes; -1: never.
+// the kernel takes the shapes; -1: never. 1 and -1 come before the models' choice of the single launch, not before a forced one.
 static int g_block_pair = 0;
 
 static bool block_pair_takes(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const ConvGeom g[3]) {
@@ -1161,6 +1161,7 @@ static bool block_single_launch(const otter_hip_conv_t* e, const otter_hip_conv_
     if (!conv_block_applicable(g[0], e1, g[1], e2, g[2], e3)) return false;
     if (!conv_block_plan(g[0], g[2], e->block_rb, e->block_sl, e->block_split, plan)) return false;
     if (g_block_always == 1 || e->block_rb || e->block_sl || e->block_split) return true;
+    if (g_block_pair < 0 || (g_block_pair > 0 && block_pair_takes(e, d, g))) return false;
     const float single = block_cost_single(g, plan);
     return single < block_cost_three(g) - block_margin(g, 3.8f) && (!block_pair_takes(e, d, g) || single < block_cost_pair(g));
 }

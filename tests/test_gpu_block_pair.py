@@ -146,3 +146,28 @@ def test_pair_launch_random_shapes(hip):
         hip.conv_block_set_always(always)
         hip.conv_block_set_pair(pair)
     assert taken >= 30
+
+
+@pytest.mark.parametrize("cin,ce,cout,N,H,W", [(8, 16, 8, 1, 1, 1), (40, 144, 24, 2, 11, 13), (32, 192, 32, 64, 28, 28)])
+def test_forced_pair_setting_comes_before_the_automatic_single_launch(hip, cin, ce, cout, N, H, W):
+    """Blocks that run as the single launch by themselves: the setting gives the shared launch or three launches, and a single
+    launch that was asked for still wins over it."""
+    layers = make_block(hip, np.random.default_rng(1), cin, ce, cout, 3, True)
+    e, d, p = (l["conv"] for l in layers)
+    always, pair = hip.conv_block_set_always(0), hip.conv_block_set_pair(0)
+    try:
+        assert hip.conv_block_launches(e, d, p, N, H, W) == 1
+        for mode, want in ((1, 2), (-1, 3)):
+            hip.conv_block_set_pair(mode)
+            assert hip.conv_block_launches(e, d, p, N, H, W) == want
+            hip.conv_block_set_always(1)
+            assert hip.conv_block_launches(e, d, p, N, H, W) == 1
+            hip.conv_block_set_always(0)
+            e.set_block_plan(0, 64, 0)
+            assert hip.conv_block_launches(e, d, p, N, H, W) == 1
+            e.set_block_plan(0, 0, 0)
+    finally:
+        hip.conv_block_set_always(always)
+        hip.conv_block_set_pair(pair)
+    for l in layers:
+        l["conv"].close()
