@@ -32,9 +32,11 @@ LayerOption parse_options(const char* opts) {
     }
     return lo;
 }
-// a pass's result, unpacked: what it is, and its values in host memory where the caller has room for them
-void fetched(const Tensor& top, void* out, size_t capacity, int* dtype, int64_t* shape4) {
+// a pass's result, unpacked: what it is, and its values in host memory where the caller has room for them. `unpacked` (or
+// null) receives the blob itself first.
+void fetched(const Tensor& top, void* out, size_t capacity, int* dtype, int64_t* shape4, Tensor* unpacked = nullptr) {
     const Tensor f = top.dim() == 4 && top.elempack() != 1 ? top.packing(1) : top;
+    if (unpacked) *unpacked = f;
     const ScalarType b = base_of(f.scalar_type());
     if (dtype) *dtype = b == ScalarType::Float ? 0 : (b == ScalarType::Byte ? 1 : 2);
     if (shape4)
@@ -313,12 +315,17 @@ long otter_host_net_describe(void* net, char* buf, size_t capacity) {
 }
 
 // One pass with any number of blobs set beforehand (Extractor::input on each), e.g. a layer's bottoms when a test
-// drives a single layer: inputs are NCHW fp32 / int8 on the host, shapes4 holds 4 entries per input.
+// drives a single layer: inputs are NCHW fp32 / int8 on the host, shapes4 holds 4 entries per input. out_dtype and
+// out_shape4 are known even where out holds too little (status -1) or is null; the result is then still to be had, once, from
+// otter_host_net_eval_fetch on the same thread.
+static thread_local Tensor t_eval_result;
+
 int otter_host_net_eval(void* net, int n_inputs, const char* const* in_names, const void* const* in_ptrs,
                         const int* in_is_int8, const int64_t* shapes4, const char* out_name, void* out,
                         size_t out_capacity_bytes, int* out_dtype, int64_t* out_shape4) {
     try {
         Net* N = static_cast<Net*>(net);
+        t_eval_result = Tensor();
         std::vector<std::unique_ptr<HostInput>> ins;
         Extractor ex = N->create_extractor();
         ex.set_lightmode(false);
@@ -332,9 +339,24 @@ int otter_host_net_eval(void* net, int n_inputs, const char* const* in_names, co
         Tensor feat;
         const int rc = ex.extract(out_name, feat, 0);
         if (rc) return fail("forward failed with code " + std::to_string(rc) + ": " + otter_hip_last_error());
-        fetched(feat, out, out_capacity_bytes, out_dtype, out_shape4);
-        if (out)  // the download has waited for the pass
+        fetched(feat, out, out_capacity_bytes, out_dtype, out_shape4, &t_eval_result);
+        if (out) {  // the download has waited for the pass
+            t_eval_result = Tensor();
             for (auto& in : ins) in->pass_done();
+        }
+        return 0;
+    } catch (const std::exception& e) {
+        return fail(e.what());
+    }
+}
+
+// the result that the last otter_host_net_eval of this thread had no room for
+int otter_host_net_eval_fetch(void* out, size_t capacity) {
+    try {
+        if (!t_eval_result.defined()) return fail("no result is waiting");
+        OTTER_CHECK(out && t_eval_result.nbytes() <= capacity, "output buffer too small");
+        t_eval_result.download(out);
+        t_eval_result = Tensor();
         return 0;
     } catch (const std::exception& e) {
         return fail(e.what());

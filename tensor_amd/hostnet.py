@@ -13,7 +13,8 @@ EXPORTS = ["otter_host_last_error", "otter_host_net_create", "otter_host_net_des
            "otter_host_net_set_inner_product", "otter_host_net_run", "otter_host_session_create",
            "otter_host_session_pass", "otter_host_session_fetch", "otter_host_session_destroy",
            "otter_host_functional_chain", "otter_host_net_load_otter", "otter_host_net_load_weight",
-           "otter_host_net_describe", "otter_host_net_conv_fp32_probe", "otter_host_net_eval", "otter_host_otter_dump", "otter_host_ncnn_read",
+           "otter_host_net_describe", "otter_host_net_conv_fp32_probe", "otter_host_net_eval", "otter_host_net_eval_fetch",
+           "otter_host_otter_dump", "otter_host_ncnn_read",
            "otter_host_chain_forward_count", "otter_host_block_forward_count"]
 
 
@@ -153,19 +154,27 @@ class Net:
                     (C.c_int64 * (4 * n))(*[d for a in arrs for d in a.shape]), out_name.encode())
         n, c_names, c_i8, c_shapes, c_out = args[:5]
         c_ptrs = (C.c_void_p * n)(*[a.ctypes.data for a in arrs])
-        dtype, shape = C.c_int(), (C.c_int64 * 4)()
-        # the result of a call seen before has the size it had then; else room for any blob, of which only the part that is
-        # written is ever touched
-        out = np.empty(args[5], args[6]) if len(args) > 5 else np.empty(1 << 28, np.uint8)
-        self._check(self.lib.otter_host_net_eval(self.h, n, c_names, c_ptrs, c_i8, c_shapes, c_out,
-                                                 C.c_void_p(out.ctypes.data), C.c_size_t(out.nbytes), C.byref(dtype), shape))
-        got, np_dt = tuple(shape), [np.float32, np.int8, np.int32][dtype.value]
-        if len(args) > 5 and got == args[5] and np_dt is args[6]:
-            return out
-        if len(args) == 5 and len(self._eval_args) < 64:
-            self._eval_args[key] = args + (got, np_dt)
-        count = int(np.prod(got))
-        return out.reshape(-1).view(np.uint8)[:count * np.dtype(np_dt).itemsize].view(np_dt).reshape(got).copy()
+        dtype, shape = C.c_int(-1), (C.c_int64 * 4)()
+        # the result of a call seen before most likely is what it was then; anything else is fetched once its size is known
+        out = np.empty(args[5], args[6]) if len(args) > 5 else None
+        rc = self.lib.otter_host_net_eval(self.h, n, c_names, c_ptrs, c_i8, c_shapes, c_out,
+                                          C.c_void_p(out.ctypes.data) if out is not None else None,
+                                          C.c_size_t(out.nbytes if out is not None else 0), C.byref(dtype), shape)
+        got, np_dt = tuple(shape), [np.float32, np.int8, np.int32, None][dtype.value]
+        if np_dt is None:  # the pass itself failed
+            self._check(rc)
+        need = int(np.prod(got)) * np.dtype(np_dt).itemsize
+        if out is None or need > out.nbytes:
+            out = np.empty(got, np_dt)
+            self._check(self.lib.otter_host_net_eval_fetch(C.c_void_p(out.ctypes.data), C.c_size_t(out.nbytes)))
+        else:
+            self._check(rc)
+            if got == args[5] and np_dt is args[6]:
+                return out
+            out = out.reshape(-1).view(np.uint8)[:need].view(np_dt).reshape(got).copy()
+        if key in self._eval_args or len(self._eval_args) < 64:
+            self._eval_args[key] = args[:5] + (got, np_dt)
+        return out
 
     def close(self):
         if self.h:
