@@ -224,33 +224,60 @@ struct Staging {
 };
 constexpr size_t kStagingBytes = 1u << 20;
 constexpr int kStagingMax = 16;
+// One pool per GPU: an event can only be recorded on a stream of the GPU that it was created on.
+struct StagingPool {
+    std::vector<Staging> free;
+    int made = 0;
+};
 std::mutex g_staging_mutex;
-std::vector<Staging> g_staging_free;  // (of all devices: pinned memory is visible to every GPU, the events are per process)
-int g_staging_made = 0;
+StagingPool g_staging[kMaxDevices];
+
+// the pool of the stream's GPU (the null stream's: the current one)
+hipError_t staging_pool(hipStream_t stream, StagingPool** out) {
+    int dev = -1;
+    const hipError_t e = stream ? hipStreamGetDevice(stream, &dev) : hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+    *out = &g_staging[dev];
+    return hipSuccess;
+}
+
+hipError_t staging_make(int device, Staging* s) {
+    int before = device;
+    hipError_t e = hipGetDevice(&before);
+    if (e == hipSuccess && before != device) e = hipSetDevice(device);
+    if (e != hipSuccess) return e;
+    *s = Staging{};
+    e = hipHostMalloc((void**)&s->host, kStagingBytes, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&s->busy, hipEventDisableTiming);
+    if (e != hipSuccess && s->host) {
+        (void)hipHostFree(s->host);
+        *s = Staging{};
+    }
+    if (before != device) (void)hipSetDevice(before);
+    return e;
+}
 
 // a buffer nobody else holds; its last copy may still be on its way when `pending`
-hipError_t staging_get(Staging* out) {
+hipError_t staging_get(StagingPool& pool, Staging* out) {
     {
         std::lock_guard<std::mutex> lock(g_staging_mutex);
         // the buffer used last if its copy is over (it is in the caches), else the oldest
-        for (size_t i : {g_staging_free.size() - 1, (size_t)0}) {
-            if (g_staging_free.empty()) break;
-            Staging& s = g_staging_free[i];
-            if (g_staging_made < kStagingMax && s.pending && hipEventQuery(s.busy) != hipSuccess) continue;
+        for (size_t i : {pool.free.size() - 1, (size_t)0}) {
+            if (pool.free.empty()) break;
+            Staging& s = pool.free[i];
+            if (pool.made < kStagingMax && s.pending && hipEventQuery(s.busy) != hipSuccess) continue;
             *out = s;
-            g_staging_free.erase(g_staging_free.begin() + i);
+            pool.free.erase(pool.free.begin() + i);
             return hipSuccess;
         }
         (void)hipGetLastError();  // (hipErrorNotReady of the query)
-        ++g_staging_made;         // beyond the bound only while as many threads copy at once; such a buffer is not kept
+        ++pool.made;              // beyond the bound only while as many threads copy at once; such a buffer is not kept
     }
-    *out = Staging{};
-    hipError_t e = hipHostMalloc((void**)&out->host, kStagingBytes, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&out->busy, hipEventDisableTiming);
+    const hipError_t e = staging_make((int)(&pool - g_staging), out);
     if (e != hipSuccess) {
-        if (out->host) (void)hipHostFree(out->host);
         std::lock_guard<std::mutex> lock(g_staging_mutex);
-        --g_staging_made;
+        --pool.made;
     }
     return e;
 }
@@ -261,15 +288,23 @@ hipError_t staging_wait(Staging& s) {
     return hipEventSynchronize(s.busy);
 }
 
-void staging_put(Staging& s) {
-    if (!s.host) return;
+// the event behind the copy just enqueued; without one the copy is waited for, so that the buffer is never reused under it
+hipError_t staging_record(Staging& s, hipStream_t stream) {
+    const hipError_t e = hipEventRecord(s.busy, stream);
+    s.pending = e == hipSuccess;
+    if (e != hipSuccess) (void)hipStreamSynchronize(stream);
+    return e;
+}
+
+void staging_put(StagingPool& pool, Staging& s) {
+    if (!s.host) return;  // (none could be made)
     {
         std::lock_guard<std::mutex> lock(g_staging_mutex);
-        if (g_staging_made <= kStagingMax) {
-            g_staging_free.push_back(s);
+        if (pool.made <= kStagingMax) {
+            pool.free.push_back(s);
             return;
         }
-        --g_staging_made;
+        --pool.made;
     }
     (void)staging_wait(s);
     (void)hipEventDestroy(s.busy);
@@ -283,18 +318,19 @@ extern "C" {
 int otter_hip_upload(void* dst, const void* src, size_t bytes, void* stream_) {
     if (bytes && (!dst || !src)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_upload: null");
     hipStream_t stream = (hipStream_t)stream_;
+    StagingPool* pool = nullptr;
+    if (bytes) OHIP_CHECK(staging_pool(stream, &pool));
     for (size_t at = 0; at < bytes; at += kStagingBytes) {
         const size_t n = bytes - at < kStagingBytes ? bytes - at : kStagingBytes;
         Staging s;
-        hipError_t e = staging_get(&s);
+        hipError_t e = staging_get(*pool, &s);
         if (e == hipSuccess) e = staging_wait(s);
         if (e == hipSuccess) {
             std::memcpy(s.host, (const char*)src + at, n);
             e = hipMemcpyAsync((char*)dst + at, s.host, n, hipMemcpyHostToDevice, stream);
-            s.pending = e == hipSuccess;
-            if (e == hipSuccess) e = hipEventRecord(s.busy, stream);
+            if (e == hipSuccess) e = staging_record(s, stream);
         }
-        staging_put(s);
+        staging_put(*pool, s);
         OHIP_CHECK(e);
     }
     return OTTER_HIP_OK;
@@ -303,11 +339,13 @@ int otter_hip_upload(void* dst, const void* src, size_t bytes, void* stream_) {
 int otter_hip_download(void* dst, const void* src, size_t bytes, void* stream_) {
     if (bytes && (!dst || !src)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_download: null");
     hipStream_t stream = (hipStream_t)stream_;
+    StagingPool* pool = nullptr;
+    if (bytes) OHIP_CHECK(staging_pool(stream, &pool));
     Staging s[2];
     hipError_t e = hipSuccess;
     const size_t chunks = (bytes + kStagingBytes - 1) / kStagingBytes;
     for (size_t i = 0; i < 2 && i < chunks && e == hipSuccess; ++i) {
-        e = staging_get(&s[i]);
+        e = staging_get(*pool, &s[i]);
         if (e == hipSuccess) e = staging_wait(s[i]);
     }
     // chunk c travels while chunk c - 1 is copied out
@@ -316,10 +354,7 @@ int otter_hip_download(void* dst, const void* src, size_t bytes, void* stream_) 
         if (c < chunks) {
             Staging& b = s[c & 1];
             e = hipMemcpyAsync(b.host, (const char*)src + c * kStagingBytes, length(c), hipMemcpyDeviceToHost, stream);
-            if (e == hipSuccess && chunks > 1) {
-                e = hipEventRecord(b.busy, stream);
-                b.pending = e == hipSuccess;
-            }
+            if (e == hipSuccess && chunks > 1) e = staging_record(b, stream);
         }
         if (c > 0 && e == hipSuccess) {
             Staging& b = s[(c - 1) & 1];
@@ -328,8 +363,8 @@ int otter_hip_download(void* dst, const void* src, size_t bytes, void* stream_) 
         }
     }
     if (e != hipSuccess) (void)hipStreamSynchronize(stream);  // nothing may still write into a buffer that goes back
-    staging_put(s[0]);
-    staging_put(s[1]);
+    if (pool)
+        for (Staging& b : s) staging_put(*pool, b);
     OHIP_CHECK(e);
     return OTTER_HIP_OK;
 }
