@@ -85,7 +85,8 @@ int otter_hip_memcpy_h2d(void* dst_dev, const void* src_host, size_t bytes, void
 int otter_hip_memcpy_d2h(void* dst_host, const void* src_dev, size_t bytes, void* stream);
 /* Copies of pageable host memory through pinned staging buffers that the library keeps (at most 16 of 1 MiB per GPU,
  * safe with several threads, streams and GPUs). upload: returns when `src_host` has been read; the copy is ordered on `stream`
- * like a launch. download: ordered behind what `stream` holds, returns when `dst_host` is written. Stand in for the
+ * like a launch. download: ordered behind what `stream` holds, returns when `dst_host` is written. Both are refused on a stream
+ * that is being captured. Stand in for the
  * host <-> blob copies of the reference's Extractor (Tensor/Net.cpp:668-736), which have no device to cross to. */
 int otter_hip_upload(void* dst_dev, const void* src_host, size_t bytes, void* stream);
 int otter_hip_download(void* dst_host, const void* src_dev, size_t bytes, void* stream);

@@ -232,10 +232,14 @@ struct StagingPool {
 std::mutex g_staging_mutex;
 StagingPool g_staging[kMaxDevices];
 
-// the pool of the stream's GPU (the null stream's: the current one)
+// the pool of the stream's GPU (the null stream's: the current one). A stream that is being captured has none: a replay would
+// read or write the buffer when it holds another copy's bytes.
 hipError_t staging_pool(hipStream_t stream, StagingPool** out) {
     int dev = -1;
-    const hipError_t e = stream ? hipStreamGetDevice(stream, &dev) : hipGetDevice(&dev);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    hipError_t e = stream ? hipStreamIsCapturing(stream, &capturing) : hipSuccess;  // (the null stream is never captured)
+    if (e == hipSuccess && capturing != hipStreamCaptureStatusNone) e = hipErrorStreamCaptureUnsupported;
+    if (e == hipSuccess) e = stream ? hipStreamGetDevice(stream, &dev) : hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
     *out = &g_staging[dev];

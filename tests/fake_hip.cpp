@@ -25,7 +25,7 @@ struct Event {
 };
 constexpr int kDevices = 3;
 Stream g_null[kDevices] = {{0, {}}, {1, {}}, {2, {}}};
-int g_current = 0, g_fail_records = 0, g_pinned = 0;
+int g_current = 0, g_fail_records = 0, g_pinned = 0, g_capturing = 0;
 Stream* of(void* s) { return s ? static_cast<Stream*>(s) : &g_null[g_current]; }
 constexpr int kInvalidHandle = 400, kNotReady = 600, kInvalidDevice = 101;
 }  // namespace
@@ -34,7 +34,7 @@ extern "C" {
 int hipGetDevice(int* d) { return *d = g_current, 0; }
 int hipSetDevice(int d) { return d < 0 || d >= kDevices ? kInvalidDevice : (g_current = d, 0); }
 int hipStreamGetDevice(void* s, int* d) { return *d = of(s)->device, 0; }
-int hipStreamIsCapturing(void*, int* status) { return *status = 0, 0; }
+int hipStreamIsCapturing(void*, int* status) { return *status = g_capturing, 0; }
 int hipHostMalloc(void** p, size_t n, unsigned) { return *p = std::malloc(n), ++g_pinned, 0; }
 int hipHostFree(void* p) { return std::free(p), --g_pinned, 0; }
 int hipEventCreateWithFlags(void** e, unsigned) { return *e = new Event{g_current, nullptr}, 0; }
@@ -54,6 +54,7 @@ int hipStreamSynchronize(void* s) { return of(s)->run(), 0; }
 int hipGetLastError() { return 0; }
 
 void fake_fail_records(int n) { g_fail_records = n; }
+void fake_capture(int on) { g_capturing = on; }
 void* fake_stream(int device) { return new Stream{device, {}}; }
 int fake_pinned() { return g_pinned; }
 }

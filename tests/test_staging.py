@@ -60,6 +60,17 @@ second = upload(1000)
 good(*second)
 assert (first[2] == first[1]).all()
 """,
+    # a replay of the copy would read a buffer that holds something else by then
+    "a stream under capture": """
+s = fake.fake_stream(0)
+fake.fake_capture(1)
+rc, src, dst = upload(100, s)
+assert rc != 0 and b"captur" in lib.otter_hip_last_error()
+assert lib.otter_hip_download(C.c_void_p(dst.ctypes.data), C.c_void_p(src.ctypes.data), C.c_size_t(100), C.c_void_p(s)) != 0
+good(*upload(100))
+fake.fake_capture(0)
+good(*upload(100, s), s)
+""",
     # buffers are kept up to 16 per GPU
     "what is kept": """
 for device in (0, 1):
