@@ -271,12 +271,15 @@ int otter_hip_conv_chain_set_min_tiles(int tiles);
  * layer reads more than 32 channels) and both clamp at zero or neither clamps, the first two layers can run as ONE
  * launch that keeps the expanded rows in LDS, the last layer by itself; they do (otter_hip_conv_block_launches says 2)
  * where the model says so, or wherever they can after otter_hip_conv_block_set_pair(1); any other block makes
- * three launches. The blobs between the launches live in `workspace`;
- * otter_hip_conv_block_workspace_bytes gives the size either way (0 for a single launch with one workgroup per band). */
+ * three launches. Any other layout of out runs as two or three launches. The blobs between the launches live in `workspace`:
+ * otter_hip_conv_block_workspace_bytes covers every out_layout, otter_hip_conv_block_layout_workspace_bytes is what the call with
+ * that layout needs (0 for a single launch with one workgroup per band). */
 int otter_hip_conv_block_launches(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise,
                                   const otter_hip_conv_t* project, int n, int in_h, int in_w);
 size_t otter_hip_conv_block_workspace_bytes(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise,
                                             const otter_hip_conv_t* project, int n, int in_h, int in_w);
+size_t otter_hip_conv_block_layout_workspace_bytes(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise,
+                                                   const otter_hip_conv_t* project, int out_layout, int n, int in_h, int in_w);
 int otter_hip_conv_block_forward(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise,
                                  const otter_hip_conv_t* project, const void* in, int n, int in_h, int in_w,
                                  const float* residual, void* out, int out_layout, void* out_q, float q_scale,

@@ -188,7 +188,7 @@ PyObject* conv_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (!out) out = &(made = device_empty(count, type_of_layout(out_layout), device));
         if (!q && with_q) q = &(made_q = device_empty(count, at::kChar, device));
         if (!ws) {
-            const size_t need = otter_hip_conv_block_workspace_bytes(e, d, p, n, ih, iw);
+            const size_t need = otter_hip_conv_block_layout_workspace_bytes(e, d, p, out_layout, n, ih, iw);
             if (need) ws = &(made_ws = device_empty((int64_t)need, at::kChar, device));
         }
         void* stream = stream_now();

@@ -80,6 +80,7 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_chain_forward", "otter_hip_conv_chain_status", "otter_hip_conv_chain_launches",
            "otter_hip_conv_chain_last_launches", "otter_hip_conv_chain_clock_mhz",
            "otter_hip_conv_chain_set_min_tiles", "otter_hip_conv_block_launches", "otter_hip_conv_block_workspace_bytes",
+           "otter_hip_conv_block_layout_workspace_bytes",
            "otter_hip_conv_block_forward", "otter_hip_conv_block_set_plan", "otter_hip_conv_block_set_always", "otter_hip_conv_block_set_pair",
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
            "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
@@ -118,6 +119,7 @@ class Library:
         L.otter_hip_conv_workspace_bytes.restype = C.c_size_t
         L.otter_hip_conv_chain_workspace_bytes.restype = C.c_size_t
         L.otter_hip_conv_block_workspace_bytes.restype = C.c_size_t
+        L.otter_hip_conv_block_layout_workspace_bytes.restype = C.c_size_t
         L.otter_hip_conv_avgpool_workspace_bytes.restype = C.c_size_t
         self.device = torch.device("cuda", device)
         self.native, self.device_index = load_binding(), device

@@ -1,5 +1,6 @@
 // extern "C" boundary of the library (include/otter_hip_int8.h): argument checking, handle management,
 // weight re-layout at create time and kernel dispatch. No kernels live here.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -1228,16 +1229,32 @@ int otter_hip_conv_block_launches(const otter_hip_conv_t* e, const otter_hip_con
     return n >= 1 && block_pair_launch(e, d, g) ? 2 : 3;
 }
 
+// the two blobs between the launches of a block that is not one
+static size_t block_blob_bytes(const ConvGeom g[3], size_t* second) {
+    const size_t b0 = (size_t)g[0].N * g[0].K * g[0].OH * g[0].OW, b1 = (size_t)g[1].N * g[1].K * g[1].OH * g[1].OW;
+    if (second) *second = (b0 + 255) / 256 * 256;
+    return (b0 + 255) / 256 * 256 + (b1 + 255) / 256 * 256;
+}
+
+size_t otter_hip_conv_block_layout_workspace_bytes(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
+                                                   int out_layout, int n, int in_h, int in_w) {
+    if (!e || !d || !p || n < 1 || in_h < 1 || in_w < 1) return 0;
+    ConvGeom g[3];
+    if (!block_geoms(e, d, p, n, in_h, in_w, g)) return 0;
+    int plan[6];
+    if (p->d.out_channels % 8 == 0 && out_layout == block_default_out_layout(p) && block_single_launch(e, d, p, g, out_layout, plan))
+        return (size_t)plan[5] * sizeof(int);  // the accumulators of a band's workgroups, when there are several
+    return block_blob_bytes(g, nullptr);
+}
+
 size_t otter_hip_conv_block_workspace_bytes(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
                                             int n, int in_h, int in_w) {
     if (!e || !d || !p || n < 1 || in_h < 1 || in_w < 1) return 0;
     ConvGeom g[3];
     if (!block_geoms(e, d, p, n, in_h, in_w, g)) return 0;
-    int plan[6];
-    if (p->d.out_channels % 8 == 0 && block_single_launch(e, d, p, g, block_default_out_layout(p), plan))
-        return (size_t)plan[5] * sizeof(int);  // the accumulators of a band's workgroups, when there are several
-    const size_t b0 = (size_t)n * g[0].K * g[0].OH * g[0].OW, b1 = (size_t)n * g[1].K * g[1].OH * g[1].OW;
-    return (b0 + 255) / 256 * 256 + (b1 + 255) / 256 * 256;
+    // (only the default layout can take the single launch)
+    return std::max(block_blob_bytes(g, nullptr),
+                    otter_hip_conv_block_layout_workspace_bytes(e, d, p, block_default_out_layout(p), n, in_h, in_w));
 }
 
 int otter_hip_conv_block_plan(int in_channels, int expanded_channels, int out_channels, int n, int in_h, int in_w,
@@ -1317,13 +1334,13 @@ int otter_hip_conv_block_forward(const otter_hip_conv_t* e, const otter_hip_conv
         return OTTER_HIP_OK;
     }
     // the layers one after the other, the intermediate blobs in the workspace
-    const size_t b0 = (size_t)n * g[0].K * g[0].OH * g[0].OW, b1 = (size_t)n * g[1].K * g[1].OH * g[1].OW;
-    const size_t need = (b0 + 255) / 256 * 256 + (b1 + 255) / 256 * 256;
+    size_t second;
+    const size_t need = block_blob_bytes(g, &second);
     if (!workspace || workspace_bytes < need)
         return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_block_forward: needs the workspace reported by "
                                            "otter_hip_conv_block_workspace_bytes");
     void* t0 = workspace;
-    void* t1 = (char*)workspace + (b0 + 255) / 256 * 256;
+    void* t1 = (char*)workspace + second;
     if (block_pair_launch(e, d, g)) {
         // the pointwise layer and its depthwise reader in one launch: the expanded blob is not made
         const Epilogue e1 = make_epilogue(e, OTTER_HIP_I8_P8), e2 = make_epilogue(d, OTTER_HIP_I8_P8);

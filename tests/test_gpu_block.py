@@ -290,3 +290,27 @@ def test_block_random_shapes(hip):
         for l in layers:
             l["conv"].close()
     assert taken >= 20
+
+
+@pytest.mark.parametrize("f32_out,layout", [(True, capi.F32_P8), (True, capi.F32), (True, capi.F32_P4), (False, capi.I8), (False, capi.I8_P8)])
+@pytest.mark.parametrize("cin,ce,cout,n,h,w", [(32, 192, 32, 64, 28, 28), (48, 288, 48, 29, 29, 29), (160, 960, 160, 64, 7, 7)])
+def test_reported_workspace_is_enough_for_every_layout(hip, cin, ce, cout, n, h, w, f32_out, layout):
+    """Blocks that run as the single launch by default, which only writes the default layout: the size that
+    otter_hip_conv_block_workspace_bytes reports is enough for any of them, the other function's is for the one it is asked for."""
+    hip.conv_block_set_always(0)
+    rng = np.random.default_rng(cin)
+    layers = make_block(hip, rng, cin, ce, cout, 3, f32_out)
+    e, d, p = (l["conv"] for l in layers)
+    assert hip.conv_block_launches(e, d, p, n, h, w) == 1
+    xd = hip.to_device(capi.pack_np(rng.integers(-127, 128, (n, cin, h, w)).astype(np.int8), 8))
+    t = e.forward(xd, capi.I8_P8, n, h, w, capi.I8_P8)
+    t = d.forward(t, capi.I8_P8, n, h, w, capi.I8_P8)
+    want = p.forward(t, capi.I8_P8, n, h, w, layout)
+    for size in (hip.lib.otter_hip_conv_block_workspace_bytes(e.h, d.h, p.h, n, h, w),
+                 hip.lib.otter_hip_conv_block_layout_workspace_bytes(e.h, d.h, p.h, layout, n, h, w)):
+        ws = hip.empty(max(size, 1), np.int8)[:size]
+        got, _ = hip.native.conv_block(e._hp, d._hp, p._hp, cout, layout, xd, n, h, w, None, None, capi.ROUND_SSE, None, None, ws,
+                                       hip.device_index)
+        assert hip.torch.equal(got, want)
+    for l in layers:
+        l["conv"].close()
