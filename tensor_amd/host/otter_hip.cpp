@@ -205,14 +205,21 @@ HostInput::HostInput(const void* data, const std::vector<int64_t>& sizes, Scalar
     constexpr size_t kPiece = 768u << 10;
     buffer_ = pinned().get(bytes_);
     char *const dev = static_cast<char*>(blob.device_ptr()), *const pin = static_cast<char*>(buffer_);
-    for (size_t at = 0; at < bytes_; at += kPiece) {
-        const size_t n = std::min(kPiece, bytes_ - at);
-        std::memcpy(pin + at, static_cast<const char*>(data) + at, n);
-        hip_check(otter_hip_copy(dev + at, pin + at, n, nullptr), "upload");
+    try {
+        for (size_t at = 0; at < bytes_; at += kPiece) {
+            const size_t n = std::min(kPiece, bytes_ - at);
+            std::memcpy(pin + at, static_cast<const char*>(data) + at, n);
+            hip_check(otter_hip_copy(dev + at, pin + at, n, nullptr), "upload");
+        }
+    } catch (...) {  // (no destructor runs for an object that was not finished)
+        release();
+        throw;
     }
 }
 
-HostInput::~HostInput() {
+HostInput::~HostInput() { release(); }
+
+void HostInput::release() {
     if (!done_) otter_hip_stream_synchronize(nullptr);
     pinned().put(bytes_, buffer_);
 }

@@ -98,6 +98,7 @@ public:
     Tensor blob;
 
 private:
+    void release();
     size_t bytes_;
     void* buffer_ = nullptr;
     bool done_ = false;
