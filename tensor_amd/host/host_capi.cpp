@@ -145,10 +145,12 @@ int otter_host_net_get_scale_in(void* net, const char* layer_name, float* out) {
 
 int otter_host_net_set_inner_product(void* net, const char* layer_name, const float* weight, const float* bias) {
     try {
-        auto* L = dynamic_cast<InnerProductLayer*>(static_cast<Net*>(net)->layer_by_name(layer_name));
+        Net* n = static_cast<Net*>(net);
+        auto* L = dynamic_cast<InnerProductLayer*>(n->layer_by_name(layer_name));
         if (!L) return fail(std::string("no InnerProduct layer named ") + layer_name);
         L->weight_data = Tensor::from_blob(weight, {L->out_features, L->in_features}, ScalarType::Float);
         if (L->bias_term && bias) L->bias_data = f32_vec(bias, L->out_features);
+        if (L->create_pipeline(n->option)) return fail(std::string("create_pipeline: ") + otter_hip_last_error());
         return 0;
     } catch (const std::exception& e) {
         return fail(e.what());

@@ -288,6 +288,7 @@ public:
     int load_param(const ParamDict& pd) override;
     int init_model() override;
     int load_model(const Initializer& initializer) override;
+    int create_pipeline(const NetOption& opt) override;
     int forward(const Tensor& bottom_blob, Tensor& top_blob, const NetOption& opt) const override;
     std::string type() const override { return "InnerProduct"; }
     int in_features = 0, out_features = 0, bias_term = 1;
