@@ -99,7 +99,7 @@ public:
 
 private:
     void release();
-    size_t bytes_;
+    size_t held_;  // bytes of the pinned buffer
     void* buffer_ = nullptr;
     bool done_ = false;
 };

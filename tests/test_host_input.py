@@ -90,3 +90,14 @@ for k in range(2):  # set once, and again
     assert (n.eval({"data": x}, "fc").ravel() == x.ravel() @ w.T + b).all()
     assert fake.fake_uploads() == before
 """)
+
+
+def test_an_input_of_another_size_reuses_a_buffer_that_holds_it(tmp_path):
+    run(tmp_path, r"""
+rng = np.random.default_rng(2)
+n = net(40, 40)
+for h, w, new in ((40, 40, 1), (40, 39, 1), (20, 40, 1), (40, 40, 1), (20, 39, 2), (40, 40, 2), (41, 40, 3), (40, 40, 3)):
+    x = rng.random((1, 3, h, w), dtype=np.float32)
+    assert (n.eval({"data": x}, "data") == x).all()
+    assert fake.fake_allocated() == new, (h, w, fake.fake_allocated())
+""")
