@@ -344,6 +344,13 @@ int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 int otter_hip_conv3x3_halo_plan(int in_channels, int out_channels, int pad, int n, int in_h, int in_w, int force_fn,
                                 int plan[8]);
 
+/* Test hook with no counterpart in the reference, host arithmetic only (no GPU needed): what the launch that stages input rows
+ * in LDS (set_tile(-9, ...)) keeps of a k x k layer's input for a tile of 128 or 256 output pixels. plan = { column strips per
+ * image, output columns of a strip, LDS rows of an octet plane (the most that a tile can touch, padding rows between images
+ * included), pixel pairs of a row, bytes of an octet plane, LDS bytes of a workgroup }. Refused where the launch does not take
+ * the shape; `desc` as for otter_hip_conv_create. */
+int otter_hip_conv_rows_plan(const otter_hip_conv_desc* desc, int n, int in_h, int in_w, int pixels, int plan[6]);
+
 /* ------------------------------------------------------------------------------------------------ */
 /* standalone quantize / dequantize / requantize                                                    */
 /* ------------------------------------------------------------------------------------------------ */

@@ -729,6 +729,19 @@ int otter_hip_conv3x3_halo_plan(int in_channels, int out_channels, int pad, int 
     return OTTER_HIP_OK;
 }
 
+int otter_hip_conv_rows_plan(const otter_hip_conv_desc* desc, int n, int in_h, int in_w, int pixels, int plan[6]) {
+    if (!desc || !plan || n < 1 || in_h < 1 || in_w < 1 || (pixels != 128 && pixels != 256) || desc->kernel_h < 1 ||
+        desc->kernel_w < 1 || desc->stride_h < 1 || desc->stride_w < 1 || desc->dilation_h < 1 || desc->dilation_w < 1 ||
+        desc->pad_h < 0 || desc->pad_w < 0 || desc->groups < 1 || desc->in_channels < 1 || desc->out_channels < 1)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_rows_plan: bad argument");
+    Epilogue ep{};
+    ep.out_kind = OTTER_HIP_OUT_I8, ep.out_layout = OTTER_HIP_I8_P8;
+    const ConvGeom g = make_geom(*desc, n, in_h, in_w);
+    if (!conv_rows_supported(g, ep, false) || !conv_rows_plan(g, pixels, plan))
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_rows_plan: the kernel on staged rows does not take this shape");
+    return OTTER_HIP_OK;
+}
+
 // the convolution; `twin` (or null) receives the Byte8 quantization of an fp32 result, from the convolution's own
 // epilogue where that kernel can write it and from a quantize pass after it otherwise
 // `residual` (or null): a blob in the output's layout added to the fp32 result; the twin is then made of the sum

@@ -32,6 +32,7 @@ hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out,
 // conv_rows.hip: k x k layers on input rows staged in LDS
 size_t rows_grouped_weight_bytes(int K, int C, int groups, int kh, int kw);
 void rows_pack_weights_grouped(const int8_t* w, int K, int C, int groups, int kh, int kw, int8_t* dst);
+bool conv_rows_plan(const ConvGeom& g, int pixels, int plan[6]);  // pixels of a tile: 128 or 256
 bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in);
 float conv_rows_cost(const ConvGeom& g, bool f32in, int* config);
 hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep, int config,

@@ -320,28 +320,29 @@ static bool rows_plan(const ConvGeom& g_in, int fn, RowsArgs* ra, size_t* lds) {
     ra->g.C = g_in.C / g_in.groups, ra->g.K = g_in.K / g_in.groups;
     const ConvGeom& g = ra->g;
     const int pt = 64 * fn, taps = g.kh * g.kw;
-    ra->VH = (g.OH - 1) * g.sh + (g.kh - 1) * g.dh + 1;
-    // the number of strips that makes a tile stage the fewest bytes: wide strips read padding rows, narrow ones padding columns
-    long best = 0;
-    const long max_px = (1l << 31) - pt;
+    // the number of strips that makes a tile stage the fewest bytes: wide strips read padding rows, narrow ones padding columns.
+    // (Rows and columns in 64 bits: with dilations in the thousands their product passes 2^32.)
+    const long vh = (long)(g.OH - 1) * g.sh + (long)(g.kh - 1) * g.dh + 1, max_px = (1l << 31) - pt;
+    long best = 0, best_rows = 0, best_vw2 = 0;
     for (int strips = (g.OW + 79) / 80; strips <= (g.OW + 15) / 16; ++strips) {
-        const int w = (g.OW + strips - 1) / strips, vw2 = ((w - 1) * g.sw + (g.kw - 1) * g.dw + 1 + 2) / 2;  // (one column more in front)
-        const long total = (long)g.N * g.OH * strips * w;
-        if (total >= max_px || (long)g.OH * w >= max_px) break;
-        const int strip_px = g.OH * w, tiles = (int)((unsigned)(total + pt - 1) / (unsigned)pt);
+        const int w = (g.OW + strips - 1) / strips;
+        const long vw2 = ((long)(w - 1) * g.sw + (long)(g.kw - 1) * g.dw + 1 + 2) / 2;  // (one column more in front)
+        const long total = (long)g.N * g.OH * strips * w, strip_px = (long)g.OH * w;
+        if (total >= max_px || strip_px >= max_px) break;
+        const int tiles = (int)((unsigned)(total + pt - 1) / (unsigned)pt);
         // rows of a tile: the output rows it can touch, and the padding rows between the images it can run over
-        const int out_rows = (pt - 1) / w + 2, crossings = (pt - 1) / strip_px + 1;
-        const int between = ra->VH - g.OH * g.sh;  // virtual rows an image has more than its output rows' share (may be negative)
-        const int rows = (out_rows - 1) * g.sh + (between > 0 ? crossings * between : 0) + (g.kh - 1) * g.dh + 1;
+        const long out_rows = (pt - 1) / w + 2, crossings = (pt - 1) / strip_px + 1;
+        const long between = vh - (long)g.OH * g.sh;  // virtual rows an image has more than its output rows' share (may be negative)
+        const long rows = (out_rows - 1) * g.sh + (between > 0 ? crossings * between : 0) + (long)(g.kh - 1) * g.dh + 1;
         const long cost = (long)tiles * (rows * vw2 + 64);
         if (best == 0 || cost < best) {
-            best = cost;
-            ra->strips = strips, ra->strip_w = w, ra->VW2 = vw2, ra->rows_max = rows;
-            ra->total_pix = (unsigned)total, ra->n_tiles = tiles;
+            best = cost, best_rows = rows, best_vw2 = vw2;
+            ra->strips = strips, ra->strip_w = w, ra->total_pix = (unsigned)total, ra->n_tiles = tiles;
         }
     }
-    if (best == 0) return false;
+    if (best == 0 || best_rows * best_vw2 * 16 > ROWS_LDS) return false;  // (one octet plane alone)
     const long strip_px = (long)g.OH * ra->strip_w;
+    ra->VH = (int)vh, ra->rows_max = (int)best_rows, ra->VW2 = (int)best_vw2;
     ra->pitch = ra->VW2 * 16;
     ra->plane = (ra->rows_max * ra->pitch + 63) / 128 * 128 + 64;
     ra->stages = rows_stages(g.C);
@@ -352,6 +353,14 @@ static bool rows_plan(const ConvGeom& g_in, int fn, RowsArgs* ra, size_t* lds) {
     ra->m_tiles16 = igemm_padded_rows(g.K) / 16;
     ra->w_bytes = (unsigned)rows_packed_weight_bytes(g.K, g.C, taps);
     return *lds <= (size_t)ROWS_LDS;
+}
+
+bool conv_rows_plan(const ConvGeom& g, int pixels, int plan[6]) {
+    RowsArgs ra;
+    size_t lds;
+    if (g.OH < 1 || g.OW < 1 || !rows_plan(g, pixels / 64, &ra, &lds)) return false;
+    plan[0] = ra.strips, plan[1] = ra.strip_w, plan[2] = ra.rows_max, plan[3] = ra.VW2, plan[4] = ra.plane, plan[5] = (int)lds;
+    return true;
 }
 
 bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
