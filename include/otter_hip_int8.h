@@ -335,6 +335,12 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * tn = 0..3 its tile. */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 
+/* Test hook with no counterpart in the reference: which of the launches of its family a dense or grouped layer takes on a packed
+ * blob (no sum, no twin): choice = { 8 or 9 as set_tile(-8, ...) and set_tile(-9, ...) name them, or 0, the family's own launch (on
+ * an fp32 blob that may also be a quantize pass and the choice for its int8 copy), tile }. */
+int otter_hip_conv_launch_choice(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w, int out_layout,
+                                 int choice[2]);
+
 /* Test hook with no counterpart in the reference, host arithmetic only (no GPU needed): the launch plan of the 3x3
  * stride-1 LDS-halo kernel for a dense layer of this shape. plan = { pixel fragments per wave, pixels per tile, tiles
  * per image, persistent workgroups (grid.x), row blocks (grid.y), 1 if a workgroup reuses the per-lane LDS offsets of

@@ -678,9 +678,12 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 
 // The launches beside those of `family` (1 or 3; with an fp32 blob also 6) that a layer may take, by the cost models: the kernel
 // whose workgroups deal the reduction to their waves (conv_tap.hip) and, for k x k layers without a sum or a twin, the one on
-// staged rows (conv_rows.hip). They have to be faster than the family's launch by 5 % and 10 % (pointwise layers: 15 %): below
-// that the models' errors decide. An fp32 blob may also be quantized by a pass of its own, 2 us and 0.5 us per million
-// values, in front of whichever int8 kernel is faster. set_tile(-8, tile) and set_tile(-9, tile) force them.
+// staged rows (conv_rows.hip). They have to be faster than the family's launch by 5 % (pointwise layers on an fp32 blob: 10 %):
+// below that the models' errors decide. An fp32 blob may also be quantized by a pass of its own, 2 us and 0.65 us per million
+// values (0.85 beyond 50 million), in front of whichever int8 kernel is faster. Over 2000 drawn layers that the fits had not seen,
+// each on an int8 and on an fp32 blob, the choice takes 53 % of the time of the families' launches alone (k x k; pointwise 88 and
+// 86 %); it is over 6 % slower than those for 13 of the 2400 k x k launches and 9 of the 1600 pointwise ones, 1.28 times at worst.
+// set_tile(-8, tile) and set_tile(-9, tile) force them.
 enum AltKernel { ALT_NONE, ALT_TAP, ALT_ROWS };
 static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, bool f32in, int family, bool fused, int* config) {
     *config = h->force_tn;
@@ -689,18 +692,19 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
     if (h->force_tm == -9) return rows ? ALT_ROWS : ALT_NONE;
     if (h->force_tm == -8) return tap ? ALT_TAP : ALT_NONE;
     if (h->force_tm != 0 || (family != 1 && family != 3 && !(f32in && family == 6))) return ALT_NONE;
-    // the staged rows are worth a look where even the fastest such launch (3.5 us) would win
-    auto rows_cost = [&](bool f32, float other, int* c) { return rows && other > 3.9f ? conv_rows_cost(g, f32, c) : __builtin_inff(); };
     const int ob = layout_elem_bytes(ep.out_layout);
+    // the staged rows are worth a look where even the fastest such launch (3.5 us) would win
+    auto rows_cost = [&](bool f32, float other, int* c) { return rows && other > 3.9f ? conv_rows_cost(g, f32, ob, c) : __builtin_inff(); };
     int tap_tile = -1, rows_tile = -1, unused;
-    const float tap_t = tap ? conv_tap_cost(g, f32in, &tap_tile) : __builtin_inff();
+    const float tap_t = tap ? conv_tap_cost(g, f32in, ob, &tap_tile) : __builtin_inff();
     float other = conv_family_cost(g, family, f32in && !kxk, ob);
     if (f32in && kxk) {
-        if (tap) other = fminf(other, conv_tap_cost(g, false, &unused));
-        other = 2.f + 0.5e-6f * (float)g.N * g.C * g.H * g.W + fminf(other, rows_cost(false, other, &unused));
+        if (tap) other = fminf(other, conv_tap_cost(g, false, ob, &unused));
+        const float millions = (float)g.N * g.C * g.H * g.W * 1e-6f;
+        other = 2.f + 0.65f * millions + 0.2f * fmaxf(0.f, millions - 50.f) + fminf(other, rows_cost(false, other, &unused));
     }
-    const float best = tap_t < (kxk ? 0.95f : 0.85f) * other ? tap_t : other;
-    if (rows_cost(f32in, best, &rows_tile) < 0.9f * best) return *config = rows_tile, ALT_ROWS;
+    const float best = tap_t < (f32in && !kxk ? 0.9f : 0.95f) * other ? tap_t : other;
+    if (rows_cost(f32in, best, &rows_tile) < 0.95f * best) return *config = rows_tile, ALT_ROWS;
     return *config = tap_tile, best < other ? ALT_TAP : ALT_NONE;
 }
 
@@ -714,6 +718,19 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* h, int in_layout, int n, 
     if (layout_elem(l) == 0) l = h->d.in_channels % 8 == 0 ? OTTER_HIP_I8_P8 : OTTER_HIP_I8;
     if (h->c_pad) l = OTTER_HIP_I8_P8, g.C = h->c_pad;
     return pick_kernel(h, l, g, make_epilogue(h, out_layout));
+}
+
+int otter_hip_conv_launch_choice(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w, int out_layout, int choice[2]) {
+    if (!h || !choice || (in_layout != OTTER_HIP_F32_P8 && in_layout != OTTER_HIP_I8_P8) || !valid_layout(out_layout) || n < 1 || in_h < 1 || in_w < 1)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_launch_choice: bad argument");
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1 || h->c_pad) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_launch_choice: not a layer of this choice");
+    const Epilogue ep = make_epilogue(h, out_layout);
+    const int family = otter_hip_conv_kernel_kind(h, in_layout, n, in_h, in_w, out_layout);
+    const AltKernel alt = alt_kernel(h, g, ep, in_layout == OTTER_HIP_F32_P8, family, false, &choice[1]);
+    choice[0] = alt == ALT_TAP ? 8 : alt == ALT_ROWS ? 9 : 0;
+    if (alt == ALT_NONE) choice[1] = 0;
+    return OTTER_HIP_OK;
 }
 
 int otter_hip_conv3x3_halo_plan(int in_channels, int out_channels, int pad, int n, int in_h, int in_w, int force_fn,

@@ -24,7 +24,7 @@ bool tap_weights_are_igemm(int C, int kh, int kw, int tap_pack);
 size_t tap_grouped_weight_bytes(int K, int C, int groups, int kh, int kw);
 void tap_pack_weights_grouped(const int8_t* w, int K, int C, int groups, int kh, int kw, int8_t* dst);
 bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in);
-float conv_tap_cost(const ConvGeom& g, bool f32in, int* config);
+float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config);
 float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes);
 hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep, int config,
                         const float* in_scale, int in_round_mode, hipStream_t stream);
@@ -34,7 +34,7 @@ size_t rows_grouped_weight_bytes(int K, int C, int groups, int kh, int kw);
 void rows_pack_weights_grouped(const int8_t* w, int K, int C, int groups, int kh, int kw, int8_t* dst);
 bool conv_rows_plan(const ConvGeom& g, int pixels, int plan[6]);  // pixels of a tile: 128 or 256
 bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in);
-float conv_rows_cost(const ConvGeom& g, bool f32in, int* config);
+float conv_rows_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config);
 hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep, int config,
                          const float* in_scale, int in_round_mode, hipStream_t stream);
 

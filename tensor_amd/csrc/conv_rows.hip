@@ -24,6 +24,7 @@
 #include "common.hpp"
 #include "conv_igemm.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace ohip {
@@ -380,32 +381,37 @@ static int rows_blocks_per_workgroup(const RowsArgs& ra, int blocks) {
 }
 
 namespace {
-// A tile, and the coefficients of its duration in us for int8 and fp32 input: start + step * steps + stage * stages of a
-// workgroup's serial chain, and per workgroup of the busiest compute unit each its start, steps, staged places (pixel pairs
-// of a thread) and row blocks. Fitted to 260 layers (k 3 and 5, 8..512 channels, 100..2.3 million pixels), median error 7 %.
+// A tile, the workgroups of it that the register file holds per compute unit, and the coefficients of its duration in us (inside
+// a graph of launches, warm) for int8 and fp32 input. A workgroup's chain is step * steps + stage * stages, and a compute unit
+// runs as many of them one after the other as its workgroups do not fit side by side; per workgroup of the busiest compute unit
+// comes what they share: steps, staged places (pixel pairs of a thread) and row blocks; per launch the megabytes in and out. With
+// a stride the lanes of a pixel read lie on every other 8 bytes, and a step costs 1 + strided of what it does else. Fitted to 3000
+// drawn layers (k 3 and 5, 8..512 channels, 600..2.5 million pixels): median error 4 to 7 %, 9 in 10 below 12 to 18 %.
 struct RowsCost {
-    float start, step, stage, cu_start, cu_step, cu_place, cu_block;
+    float start, step, stage, cu_step, cu_place, cu_block, strided, in_mb, out_mb;
 };
 struct RowsConfig {
-    int fm, fn;
+    int fm, fn, resident;
     RowsCost i8, f32;
 };
 constexpr RowsConfig kRowsConfigs[] = {
-    {2, 2, {2.65f, 0.114f, 0.55f, 0.32f, 0.040f, 0.058f, 0.34f}, {2.16f, 0.135f, 1.04f, 0.f, 0.013f, 0.205f, 0.57f}},
-    {2, 4, {2.61f, 0.180f, 0.82f, 0.39f, 0.040f, 0.082f, 0.64f}, {2.21f, 0.202f, 1.27f, 0.f, 0.000f, 0.247f, 0.89f}},
-    {4, 2, {2.74f, 0.118f, 0.53f, 0.08f, 0.081f, 0.075f, 0.77f}, {2.52f, 0.154f, 0.91f, 0.f, 0.068f, 0.232f, 0.59f}},
-    {4, 4, {2.63f, 0.188f, 0.77f, 0.30f, 0.085f, 0.105f, 1.19f}, {2.40f, 0.236f, 1.27f, 0.f, 0.051f, 0.286f, 1.16f}},
+    {2, 2, 5, {2.648f, 0.103f, 1.02f, 0.031f, 0.037f, 0.31f, 0.504f, 0.028f, 0.084f}, {2.228f, 0.126f, 1.373f, 0.027f, 0.133f, 0.252f, 0.858f, 0.053f, 0.097f}},
+    {2, 4, 4, {2.918f, 0.188f, 1.113f, 0.029f, 0.055f, 0.494f, 0.436f, 0.037f, 0.088f}, {2.53f, 0.26f, 1.306f, 0.f, 0.176f, 0.456f, 0.535f, 0.064f, 0.095f}},
+    {4, 2, 4, {2.723f, 0.12f, 1.003f, 0.072f, 0.043f, 0.458f, 0.366f, 0.f, 0.105f}, {2.446f, 0.181f, 1.174f, 0.056f, 0.147f, 0.355f, 0.627f, 0.045f, 0.112f}},
+    {4, 4, 3, {3.078f, 0.24f, 1.033f, 0.055f, 0.067f, 0.789f, 0.352f, 0.f, 0.115f}, {2.79f, 0.35f, 1.117f, 0.f, 0.21f, 0.701f, 0.375f, 0.049f, 0.121f}},
 };
 constexpr int kRowsConfigCount = (int)(sizeof(kRowsConfigs) / sizeof(kRowsConfigs[0]));
 }  // namespace
 
-float conv_rows_cost(const ConvGeom& g_in, bool f32in, int* config) {
+float conv_rows_cost(const ConvGeom& g_in, bool f32in, int out_bytes, int* config) {
     float best = __builtin_inff();
     *config = -1;
     RowsArgs ra;
     size_t lds;
     bool fits = false;
     const int steps = rows_steps(g_in.C / g_in.groups, g_in.kh * g_in.kw);
+    const float in_mb = (float)g_in.N * g_in.C * g_in.H * g_in.W * (f32in ? 4e-6f : 1e-6f);
+    const float out_mb = (float)g_in.N * g_in.K * g_in.OH * g_in.OW * 1e-6f * out_bytes;
     for (const int i : {0, 2, 1, 3}) {  // by pixels of a tile: one plan for two
         const RowsConfig& c = kRowsConfigs[i];
         if (i == 0 || i == 1) fits = rows_plan(g_in, c.fn, &ra, &lds);
@@ -414,9 +420,11 @@ float conv_rows_cost(const ConvGeom& g_in, bool f32in, int* config) {
         const int pairs = ra.rows_max * ra.VW2, oct = (ra.g.C / 8 + ra.stages - 1) / ra.stages;
         const float places = (float)(ra.stages * oct) * (pairs > 128 ? (float)((pairs + 255) / 256) : 1.f / (float)(256 / pairs));
         const float cu = ceilf((float)ra.n_tiles * (float)((blocks + bpw - 1) / bpw) * (float)ra.g.groups / 256);
+        const float rounds = ceilf(cu / (float)std::min(c.resident, (int)(160 * 1024 / lds)));
         const RowsCost& k = f32in ? c.f32 : c.i8;
-        const float t = k.start + k.step * (float)(bpw * steps) + k.stage * (float)ra.stages +
-                        cu * (k.cu_start + k.cu_step * (float)(bpw * steps) + k.cu_place * places + k.cu_block * (float)bpw);
+        const float s = (float)(bpw * steps) * (g_in.sw > 1 ? 1.f + k.strided : 1.f);
+        const float t = k.start + rounds * (k.step * s + k.stage * (float)ra.stages) +
+                        cu * (k.cu_step * s + k.cu_place * places + k.cu_block * (float)bpw) + k.in_mb * in_mb + k.out_mb * out_mb;
         if (t < best) best = t, *config = i;
     }
     return best;

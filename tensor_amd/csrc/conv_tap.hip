@@ -312,21 +312,28 @@ bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
 }
 
 namespace {
-// A tile is 16 fm output channels x 16 fn wn pixels. The cost of a launch in microseconds (measured inside a graph of
-// launches, warm) is start + chain * S + c * (waves * S * step + group), with S the reduction steps of one wave and c the
-// workgroups of the busiest compute unit: fitted to 420 layers drawn over 8..512 channels, 1x1 to 5x5, 50 to 600 000
-// pixels; the median error is 7 %, the choice by it costs 2 % against the best tile of each layer. Last four: fp32 input.
+// A tile is 16 fm output channels x 16 fn wn pixels, `resident` workgroups of it a compute unit's registers hold. The cost of a
+// launch in microseconds (measured inside a graph of launches, warm) is start + chain * S + c * (waves * S * step + group) +
+// out_mb per megabyte of results, with S the reduction steps of one wave and c the workgroups of the busiest compute unit. Chain
+// and step grow by `strided` where the stride is not 1, a load then using every second 8 bytes of its lines, and by up to `far`
+// where the pixels of the workgroups side by side on a compute unit are more than its share of an XCD's L2 (128 KB: 4 MB over 32)
+// holds from one tap, or one row block, to the next: from the whole share (fp32 blobs, the widest tile) or half of it on, fully at
+// twice that, and only as far as the blob is over 4 MB, fully at 16. Fitted to 5800 layers drawn over 8..960 channels, 1x1 to 5x5,
+// 50 to 2.5 million pixels; the median error is 5 to 7 %. (Without these two, 3x3 stride 2 232 -> 344 @57x66 b30 took the last tile
+// at 112 us; the implicit-GEMM kernel takes 64.)
+struct TapCost {
+    float start, chain, step, group, out_mb, strided, far;
+};
 struct TapConfig {
-    int fm, fn, wk, wn;
-    float start, chain, step, group;
-    float start_f32, chain_f32, step_f32, group_f32;
+    int fm, fn, wk, wn, resident, resident_f32;
+    TapCost i8, f32;
 };
 constexpr TapConfig kTapConfigs[] = {
-    {2, 1, 8, 1, 2.31f, 0.067f, 0.019f, 0.72f, 2.31f, 0.242f, 0.048f, 0.47f},
-    {2, 2, 4, 1, 2.50f, 0.056f, 0.032f, 0.56f, 2.66f, 0.245f, 0.095f, 0.38f},
-    {4, 2, 4, 1, 2.44f, 0.075f, 0.047f, 0.49f, 2.40f, 0.251f, 0.104f, 0.68f},
-    {4, 2, 2, 2, 2.56f, 0.042f, 0.051f, 0.59f, 2.41f, 0.165f, 0.113f, 0.92f},
-    {4, 4, 1, 4, 2.93f, 0.000f, 0.098f, 1.63f, 0.f, 0.f, 0.f, 0.f},  // (no fp32 input: registers)
+    {2, 1, 8, 1, 3, 3, {2.382f, 0.041f, 0.021f, 0.747f, 0.005f, 0.145f, 2.2f}, {2.332f, 0.069f, 0.051f, 0.576f, 0.f, 0.37f, 2.224f}},
+    {2, 2, 4, 1, 5, 4, {2.605f, 0.048f, 0.033f, 0.552f, 0.029f, 0.157f, 0.364f}, {2.754f, 0.158f, 0.087f, 0.509f, 0.006f, 0.354f, 1.091f}},
+    {4, 2, 4, 1, 4, 3, {2.517f, 0.062f, 0.048f, 0.466f, 0.041f, 0.137f, 0.346f}, {2.702f, 0.129f, 0.103f, 0.694f, 0.061f, 0.346f, 1.079f}},
+    {4, 2, 2, 2, 5, 3, {2.719f, 0.041f, 0.05f, 0.485f, 0.083f, 0.104f, 0.229f}, {2.862f, 0.122f, 0.101f, 0.754f, 0.089f, 0.266f, 0.918f}},
+    {4, 4, 1, 4, 3, 0, {3.568f, 0.036f, 0.084f, 1.238f, 0.096f, 0.101f, 0.8f}, {}},  // (no fp32 input: registers)
 };
 constexpr int kTapConfigCount = (int)(sizeof(kTapConfigs) / sizeof(kTapConfigs[0]));
 
@@ -340,18 +347,25 @@ hipError_t launch_tap(const void* x, const int8_t* wpk, void* out, const TapArgs
 }
 }  // namespace
 
-float conv_tap_cost(const ConvGeom& g, bool f32in, int* config) {
+float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config) {
     const int C = g.C / g.groups, K = g.K / g.groups, steps = tap_steps(C, g.kh, g.kw);
-    const float px = (float)g.N * g.OH * g.OW;
+    const float bytes = f32in ? 4.f : 1.f, in_mb = (float)g.N * g.C * g.H * g.W * 1e-6f * bytes;
+    const float px = (float)g.N * g.OH * g.OW, out_mb = px * (float)g.K * 1e-6f * (float)out_bytes;
+    auto clamp01 = [](float v) { return fminf(fmaxf(v, 0.f), 1.f); };
     float best = __builtin_inff();
     *config = -1;
     for (int i = 0; i < kTapConfigCount; ++i) {
         const TapConfig& c = kTapConfigs[i];
-        if (f32in && c.step_f32 == 0.f) continue;
-        const float groups = ceilf(px / (16 * c.fn * c.wn)) * (float)((K + 16 * c.fm - 1) / (16 * c.fm)) * g.groups;
+        const TapCost& k = f32in ? c.f32 : c.i8;
+        if (k.step == 0.f) continue;
+        const int blocks = (K + 16 * c.fm - 1) / (16 * c.fm);
+        const float groups = ceilf(px / (16 * c.fn * c.wn)) * (float)blocks * g.groups;
         const float s = (float)((steps + c.wk - 1) / c.wk), cu = ceilf(groups / 256), w = (float)(c.wk * c.wn) * s;
-        const float t = f32in ? c.start_f32 + c.chain_f32 * s + cu * (w * c.step_f32 + c.group_f32)
-                              : c.start + c.chain * s + cu * (w * c.step + c.group);
+        const float side = fminf(cu, (float)(f32in ? c.resident_f32 : c.resident)) * (float)(16 * c.fn * c.wn * g.sw) * (float)C * bytes;
+        const float beyond = clamp01(side / (f32in || c.fn == 4 ? 131072.f : 65536.f) - 1.f) * clamp01((in_mb - 4.f) / 12.f);
+        const bool again = g.kh * g.kw * blocks > 1;  // the pixels are read more than once
+        const float slow = (g.sw > 1 ? 1.f + k.strided : 1.f) * (again ? 1.f + k.far * beyond : 1.f);
+        const float t = k.start + k.chain * s * slow + cu * (w * k.step * slow + k.group) + k.out_mb * out_mb;
         if (t < best) best = t, *config = i;
     }
     return best;
@@ -359,16 +373,21 @@ float conv_tap_cost(const ConvGeom& g, bool f32in, int* config) {
 
 // The same for the launches that the kernel above competes with (families of otter_hip_conv_kernel_kind): the
 // implicit-GEMM kernel (1; with fp32 input for pointwise layers), the LDS-halo kernel (3), the fp32 pointwise kernel (6).
-// Fitted to the same layers: start + chain * chunks + matrix work + epilogue + bytes in + bytes out, median error 4 to 9 %.
+// Start + chain * chunks + matrix work + epilogue + bytes in + bytes out, fitted to drawn layers; median error 4 to 11 %. The fp32
+// pointwise kernel walks all output channels per workgroup of 64 pixels, so that its chain grows with them (128 -> 1280 on one
+// 29x29 image: 15.6 us, where the kernel above takes 5.8).
 float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes) {
     const int C = g.C / g.groups, K = g.K / g.groups, taps = g.kh * g.kw, tp = g.groups > 1 ? igemm_tap_pack(C, g.kh, g.kw) : 1;
     const float chunks = tp > 1 ? (float)((taps + tp - 1) / tp) : (float)(taps * igemm_channel_groups(C));
     const float px = (float)g.N * g.OH * g.OW * g.groups, rows = K <= 32 ? 32.f : (float)((K + 63) / 64 * 64);
     const float in_mb = (float)g.N * g.C * g.H * g.W * 1e-6f, out_mb = (float)g.N * g.OH * g.OW * g.K * out_bytes * 1e-6f;
     const float mac = px * rows * chunks * 1e-9f, epi = px * rows * 1e-8f;
-    if (family == 6) return 2.35f + 1.52f * chunks + 53.7f * epi + 0.07f * out_mb;
+    if (family == 6) {
+        const float cu = ceilf((float)g.N * (float)((g.H * g.W + 63) / 64) / 256), k = 0.01f * (float)K;
+        return 2.18f + 0.5f * cu + 0.2f * chunks + k * (0.336f + 0.333f * cu + chunks * (0.063f + 0.096f * cu)) + 0.39f * in_mb + 0.048f * out_mb;
+    }
     if (family == 3) return 2.97f + 0.27f * chunks + 25.2f * mac + 39.6f * epi + 0.055f * out_mb;
-    if (taps > 1) return 3.0f + 0.32f * chunks + 62.5f * mac + 50.f * epi + 0.26f * in_mb + 0.02f * out_mb;
+    if (taps > 1) return 3.08f + 0.327f * chunks + 62.1f * mac + 44.2f * epi + px * (6.5e-6f + 1.71e-6f * chunks) + 0.061f * in_mb + 0.052f * out_mb;
     if (f32in) return 2.37f + 0.50f * chunks + 201.f * mac + 18.f * epi + 0.33f * in_mb + 0.09f * out_mb;
     return 2.46f + 0.34f * chunks + 94.f * mac + 26.f * epi + 0.03f * in_mb + 0.07f * out_mb;
 }
