@@ -8,7 +8,11 @@
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <ATen/Context.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/empty.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include "../../include/otter_hip_int8.h"
@@ -58,9 +62,14 @@ struct Args {
     }
 };
 
+// An allocation. The dispatcher in front of it costs 0.5 us of a call's 4.6, so it is left out where nothing can be listening: no
+// dispatch mode or transform of this thread, no profiler, and no deterministic filling of new memory.
 at::Tensor device_empty(int64_t count, at::ScalarType dt, long device) {
-    // (what at::empty comes to behind the dispatcher)
-    return at::detail::empty_cuda({count}, dt, c10::Device(c10::DeviceType::CUDA, (c10::DeviceIndex)device), std::nullopt);
+    const c10::Device where(c10::DeviceType::CUDA, (c10::DeviceIndex)device);
+    if (c10::impl::tls_local_dispatch_key_set().included_ == c10::default_included_set && !at::hasCallbacks() &&
+        !at::globalContext().deterministicAlgorithms())
+        return at::detail::empty_cuda({count}, dt, where, std::nullopt);
+    return at::empty({count}, at::TensorOptions().dtype(dt).device(where));
 }
 at::ScalarType type_of_layout(int layout) {
     return layout <= OTTER_HIP_F32_P8 ? at::kFloat : layout <= OTTER_HIP_I8_P8 ? at::kChar : at::kInt;
