@@ -693,15 +693,17 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
     if (h->force_tm == -8) return tap ? ALT_TAP : ALT_NONE;
     if (h->force_tm != 0 || (family != 1 && family != 3 && !(f32in && family == 6))) return ALT_NONE;
     const int ob = layout_elem_bytes(ep.out_layout);
-    // the staged rows are worth a look where even the fastest such launch (3.5 us) would win
-    auto rows_cost = [&](bool f32, float other, int* c) { return rows && other > 3.9f ? conv_rows_cost(g, f32, ob, c) : __builtin_inff(); };
+    // the staged rows are worth a look where even the fastest such launch would win
+    constexpr float least = 3.9f;
+    auto rows_cost = [&](bool f32, float other, int* c) { return rows && other > least ? conv_rows_cost(g, f32, ob, c) : __builtin_inff(); };
     int tap_tile = -1, rows_tile = -1, unused;
     const float tap_t = tap ? conv_tap_cost(g, f32in, ob, &tap_tile) : __builtin_inff();
     float other = conv_family_cost(g, family, f32in && !kxk, ob);
     if (f32in && kxk) {
         if (tap) other = fminf(other, conv_tap_cost(g, false, ob, &unused));
-        const float millions = (float)g.N * g.C * g.H * g.W * 1e-6f;
-        other = 2.f + 0.65f * millions + 0.2f * fmaxf(0.f, millions - 50.f) + fminf(other, rows_cost(false, other, &unused));
+        const float millions = (float)g.N * g.C * g.H * g.W * 1e-6f, pass = 2.f + 0.65f * millions + 0.2f * fmaxf(0.f, millions - 50.f);
+        // (the rows behind the pass are only looked at where they could still be faster than the launch without it)
+        other = pass + (tap_t < 0.95f * (pass + fminf(other, least)) ? other : fminf(other, rows_cost(false, other, &unused)));
     }
     const float best = tap_t < (f32in && !kxk ? 0.9f : 0.95f) * other ? tap_t : other;
     if (rows_cost(f32in, best, &rows_tile) < 0.95f * best) return *config = rows_tile, ALT_ROWS;

@@ -342,15 +342,12 @@ static bool rows_plan(const ConvGeom& g_in, int fn, RowsArgs* ra, size_t* lds) {
         }
     }
     if (best == 0 || best_rows * best_vw2 * 16 > ROWS_LDS) return false;  // (one octet plane alone)
-    const long strip_px = (long)g.OH * ra->strip_w;
     ra->VH = (int)vh, ra->rows_max = (int)best_rows, ra->VW2 = (int)best_vw2;
     ra->pitch = ra->VW2 * 16;
     ra->plane = (ra->rows_max * ra->pitch + 63) / 128 * 128 + 64;
     ra->stages = rows_stages(g.C);
     const int oct = (g.C / 8 + ra->stages - 1) / ra->stages;
     *lds = (size_t)(taps * ROWS_OCTETS + 7) / 8 * 32 + (size_t)(ra->rows_max + 1) / 2 * 16 + (size_t)oct * ra->plane;
-    ra->img = fast_div((unsigned)strip_px), ra->tw = fast_div((unsigned)ra->strip_w), ra->vh = fast_div((unsigned)ra->VH);
-    ra->vw = fast_div((unsigned)ra->VW2), ra->ntx = fast_div((unsigned)ra->strips), ra->kw = fast_div((unsigned)g.kw);
     ra->m_tiles16 = igemm_padded_rows(g.K) / 16;
     ra->w_bytes = (unsigned)rows_packed_weight_bytes(g.K, g.C, taps);
     return *lds <= (size_t)ROWS_LDS;
@@ -419,8 +416,9 @@ float conv_rows_cost(const ConvGeom& g_in, bool f32in, int out_bytes, int* confi
         const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm), bpw = rows_blocks_per_workgroup(ra, blocks);
         const int pairs = ra.rows_max * ra.VW2, oct = (ra.g.C / 8 + ra.stages - 1) / ra.stages;
         const float places = (float)(ra.stages * oct) * (pairs > 128 ? (float)((pairs + 255) / 256) : 1.f / (float)(256 / pairs));
-        const float cu = ceilf((float)ra.n_tiles * (float)((blocks + bpw - 1) / bpw) * (float)ra.g.groups / 256);
-        const float rounds = ceilf(cu / (float)std::min(c.resident, (int)(160 * 1024 / lds)));
+        const int wgs = (int)std::min(((long)ra.n_tiles * ((blocks + bpw - 1) / bpw) * ra.g.groups + 255) / 256, 1l << 24);
+        const int side = std::min(c.resident, (int)(160 * 1024 / lds));
+        const float cu = (float)wgs, rounds = (float)((wgs + side - 1) / side);
         const RowsCost& k = f32in ? c.f32 : c.i8;
         const float s = (float)(bpw * steps) * (g_in.sw > 1 ? 1.f + k.strided : 1.f);
         const float t = k.start + rounds * (k.step * s + k.stage * (float)ra.stages) +
@@ -437,6 +435,8 @@ hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out
     RowsArgs ra;
     size_t lds;
     if (!rows_plan(g_in, c.fn, &ra, &lds)) return hipErrorInvalidValue;
+    ra.img = fast_div((unsigned)(ra.g.OH * ra.strip_w)), ra.tw = fast_div((unsigned)ra.strip_w), ra.vh = fast_div((unsigned)ra.VH);
+    ra.vw = fast_div((unsigned)ra.VW2), ra.ntx = fast_div((unsigned)ra.strips), ra.kw = fast_div((unsigned)ra.g.kw);
     ra.in_bytes = (unsigned)((size_t)ra.g.N * ra.g.Cs * ra.g.H * ra.g.W * (f32in ? 4 : 1));
     ra.in_scale = in_scale;
     ra.in_half = in_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;

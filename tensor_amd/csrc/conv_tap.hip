@@ -350,7 +350,8 @@ hipError_t launch_tap(const void* x, const int8_t* wpk, void* out, const TapArgs
 float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config) {
     const int C = g.C / g.groups, K = g.K / g.groups, steps = tap_steps(C, g.kh, g.kw);
     const float bytes = f32in ? 4.f : 1.f, in_mb = (float)g.N * g.C * g.H * g.W * 1e-6f * bytes;
-    const float px = (float)g.N * g.OH * g.OW, out_mb = px * (float)g.K * 1e-6f * (float)out_bytes;
+    const long px = (long)g.N * g.OH * g.OW;
+    const float out_mb = (float)px * (float)g.K * 1e-6f * (float)out_bytes;
     auto clamp01 = [](float v) { return fminf(fmaxf(v, 0.f), 1.f); };
     float best = __builtin_inff();
     *config = -1;
@@ -359,8 +360,8 @@ float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config) {
         const TapCost& k = f32in ? c.f32 : c.i8;
         if (k.step == 0.f) continue;
         const int blocks = (K + 16 * c.fm - 1) / (16 * c.fm);
-        const float groups = ceilf(px / (16 * c.fn * c.wn)) * (float)blocks * g.groups;
-        const float s = (float)((steps + c.wk - 1) / c.wk), cu = ceilf(groups / 256), w = (float)(c.wk * c.wn) * s;
+        const long groups = (px + 16 * c.fn * c.wn - 1) / (16 * c.fn * c.wn) * blocks * g.groups;
+        const float s = (float)((steps + c.wk - 1) / c.wk), cu = (float)((groups + 255) / 256), w = (float)(c.wk * c.wn) * s;
         const float side = fminf(cu, (float)(f32in ? c.resident_f32 : c.resident)) * (float)(16 * c.fn * c.wn * g.sw) * (float)C * bytes;
         const float beyond = clamp01(side / (f32in || c.fn == 4 ? 131072.f : 65536.f) - 1.f) * clamp01((in_mb - 4.f) / 12.f);
         const bool again = g.kh * g.kw * blocks > 1;  // the pixels are read more than once
