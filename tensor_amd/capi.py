@@ -371,6 +371,12 @@ class Conv:
     def kernel_kind(self, in_layout, n, h, w, out_layout):
         return self.L.lib.otter_hip_conv_kernel_kind(self.h, in_layout, n, h, w, out_layout)
 
+    def launch_choice(self, in_layout, n, h, w, out_layout):
+        """otter_hip_conv_launch_choice: (8, tile), (9, tile) or (0, 0), the family's own launch."""
+        c = (C.c_int * 2)()
+        self.L._check(self.L.lib.otter_hip_conv_launch_choice(self.h, in_layout, n, h, w, out_layout, c))
+        return tuple(c)
+
     def set_tile(self, tm, tn):
         self.L._check(self.L.lib.otter_hip_conv_set_tile(self.h, tm, tn))
 

@@ -1,8 +1,6 @@
 """The launch that the cost models choose for a layer, at shapes where each form was measured well ahead of the others (us: the
 family's own launch / the one that deals the reduction to its waves / the one on staged rows, best tile of each) and where an
 earlier fit chose a slow one."""
-import ctypes as C
-
 import numpy as np
 import pytest
 
@@ -32,10 +30,8 @@ def test_launch_choice(hip, cin, cout, k, stride, groups, n, h, w, f32in, f32out
                     scale_in=np.full(cout, 1e-3, np.float32), bias=np.zeros(cout, np.float32), in_scale=40.0,
                     out_scale=None if f32out else [20.0], stride=(stride, stride), pad=(k // 2, k // 2), groups=groups, act=1,
                     out_kind=capi.OUT_F32 if f32out else capi.OUT_I8)
-    choice = (C.c_int * 2)()
-    hip._check(hip.lib.otter_hip_conv_launch_choice(conv.h, capi.F32_P8 if f32in else capi.I8_P8, n, h, w,
-                                                    capi.F32_P4 if f32out else capi.I8_P8, choice))
-    assert choice[0] in right, tuple(choice)
+    choice = conv.launch_choice(capi.F32_P8 if f32in else capi.I8_P8, n, h, w, capi.F32_P4 if f32out else capi.I8_P8)
+    assert choice[0] in right, choice
     if choice[0] == TAP and stride == 2:
         assert choice[1] != 4, "the widest tile reads such a blob from beyond the L2 for every tap"
     conv.close()
