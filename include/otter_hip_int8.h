@@ -86,8 +86,8 @@ int otter_hip_memcpy_d2h(void* dst_host, const void* src_dev, size_t bytes, void
 /* Copies of pageable host memory through pinned staging buffers that the library keeps (at most 16 of 1 MiB per GPU,
  * safe with several threads, streams and GPUs). upload: returns when `src_host` has been read; the copy is ordered on `stream`
  * like a launch. download: ordered behind what `stream` holds, returns when `dst_host` is written. Both are refused on a stream
- * that is being captured. Stand in for the
- * host <-> blob copies of the reference's Extractor (Tensor/Net.cpp:668-736), which have no device to cross to. */
+ * that is being captured. Stand in for the host <-> blob copies of the reference's Extractor (Tensor/Net.cpp:668-736), which
+ * have no device to cross to. */
 int otter_hip_upload(void* dst_dev, const void* src_host, size_t bytes, void* stream);
 int otter_hip_download(void* dst_host, const void* src_dev, size_t bytes, void* stream);
 /* Pinned host memory, and a copy between two places the GPU can address (device or pinned host memory; 16-byte aligned)
@@ -311,8 +311,8 @@ int otter_hip_conv_block_set_plan(otter_hip_conv_t* expand, int rows_per_band, i
  * blob), 5 streamed 1x1 kernel (int8 -> int8 over at most 64 input channels), 6 pointwise layer on an fp32 Float8 blob
  * of 64..256 channels, quantize and convolution in one launch that reads the blob once. (Other pointwise and depthwise 3x3
  * layers on an fp32 Float8 blob also quantize inside the convolution's launch; they report 1 and 2. Families 1, 3 and 6
- * have a second kernel for layers that it is measured faster on, mostly those that leave the machine idle; the family
- * stays what is reported.) For tests and profiling. */
+ * have other kernels for layers that those are faster on, see otter_hip_conv_launch_choice; the family stays what is
+ * reported.) For tests and profiling. */
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w,
                                int out_layout);
 
