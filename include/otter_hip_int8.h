@@ -310,7 +310,7 @@ int otter_hip_conv_block_set_plan(otter_hip_conv_t* expand, int rows_per_band, i
  * GEMM, 2 depthwise, 3 MFMA 3x3 halo kernel, 4 few-channel 3x3 kernel (an image stem read straight from the unpacked
  * blob), 5 streamed 1x1 kernel (int8 -> int8 over at most 64 input channels), 6 pointwise layer on an fp32 Float8 blob
  * of 64..256 channels, quantize and convolution in one launch that reads the blob once. (Other pointwise and depthwise 3x3
- * layers on an fp32 Float8 blob also quantize inside the convolution's launch; they report 1 and 2. Families 1, 3 and 6
+ * layers on an fp32 Float8 blob also quantize inside the convolution's launch; they report 1 and 2. Families 1, 3, 5 and 6
  * have other kernels for layers that those are faster on, see otter_hip_conv_launch_choice; the family stays what is
  * reported.) For tests and profiling. */
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w,
@@ -332,11 +332,13 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * groups a wave owns (1 or 2) and the pairs of 16 output channels per LDS round (0 = automatic for either).
  * tm == -8: the launch of families 1 and 3 that reads both operands straight from memory and deals the reduction to the waves
  * of a workgroup, tn = 0..4 its tile. tm == -9 on a k x k layer: the launch of those families that stages input rows in LDS,
- * tn = 0..3 its tile. */
+ * tn = 0..3 its tile. tm == -10 on a pointwise layer with an int8 blob: the launch that keeps its operands in registers wherever it
+ * can run, tn = groups | pairs << 3 forcing the 16-pixel groups a wave owns (1, 2, or 4 with at most 256 input channels and a result
+ * without a sum, a twin or a shuffle) and the pairs of 16 output channels it walks (0 = automatic for both). */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 
 /* Test hook with no counterpart in the reference: which of the launches of its family a dense or grouped layer takes on a packed
- * blob (no sum, no twin): choice = { 8 or 9 as set_tile(-8, ...) and set_tile(-9, ...) name them, or 0, the family's own launch (on
+ * blob (no sum, no twin): choice = { 8, 9 or 10 as set_tile(-8, ...), set_tile(-9, ...) and set_tile(-10, ...) name them, or 0, the family's own launch (on
  * an fp32 blob that may also be a quantize pass and the choice for its int8 copy), tile }. */
 int otter_hip_conv_launch_choice(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w, int out_layout,
                                  int choice[2]);

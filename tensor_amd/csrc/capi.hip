@@ -102,6 +102,8 @@ struct otter_hip_conv {
     int8_t* w_xdw = nullptr;     // MFMA operands of a pointwise int8 -> int8 layer for the launch it shares with its depthwise reader
     int32_t* blk_consts = nullptr; // the layer's constants (and depthwise 3x3 weights) as the fused block launch keeps them in LDS
     bool so_positive = true;     // every output scale is finite and > 0
+    bool so_same = true;         // the output scales are all so_one
+    float so_one = 1.f;
     float* scale_in = nullptr;   // [Kpad]
     float* bias = nullptr;       // [Kpad]; -0.0f everywhere when the layer has no bias
     float* scale_out = nullptr;  // [Kpad] or null
@@ -451,7 +453,9 @@ int otter_hip_conv_create(const otter_hip_conv_desc* desc, const int8_t* weight,
             for (int i = 0; i < K; ++i) {
                 so[i] = n_out_scale == 1 ? out_scale[0] : out_scale[i];
                 if (!(so[i] > 0.f) || std::isinf(so[i])) h->so_positive = false;
+                if (so[i] != so[0]) h->so_same = false;
             }
+            h->so_one = so[0];
             if ((rc = upload<float>(&h->scale_out, so.data(), K, kpad, 1.f))) break;
             if (g == 1 && h->so_positive && (d.activation_type == 1 || d.activation_type == 3)) {
                 // the streamed 1x1 kernel reads the clamps of its ReLU / clip epilogue instead of deriving them per wave
@@ -676,6 +680,8 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
     return h->force_tm == -7 || (g.C >= 64 && g.K >= 128);
 }
 
+// A pointwise layer on an int8 blob takes the launch with its operands in registers (conv_pw_reg.hip) wherever that can run: at
+// most 384 input channels, one output scale for all channels, a packed result.
 // The launches beside those of `family` (1 or 3; with an fp32 blob also 6) that a layer may take, by the cost models: the kernel
 // whose workgroups deal the reduction to their waves (conv_tap.hip) and, for k x k layers without a sum or a twin, the one on
 // staged rows (conv_rows.hip). They have to be faster than the family's launch by 5 % (pointwise layers on an fp32 blob: 10 %):
@@ -683,10 +689,12 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 // values (0.85 beyond 50 million), in front of whichever int8 kernel is faster. Over 2000 drawn layers that the fits had not seen,
 // each on an int8 and on an fp32 blob, the choice takes 53 % of the time of the families' launches alone (k x k; pointwise 88 and
 // 86 %); it is over 6 % slower than those for 13 of the 2400 k x k launches and 9 of the 1600 pointwise ones, 1.28 times at worst.
-// set_tile(-8, tile) and set_tile(-9, tile) force them.
-enum AltKernel { ALT_NONE, ALT_TAP, ALT_ROWS };
+// set_tile(-8, tile), set_tile(-9, tile) and set_tile(-10, ...) force them.
+enum AltKernel { ALT_NONE, ALT_TAP, ALT_ROWS, ALT_PW_REG };
 static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, bool f32in, int family, bool fused, int* config) {
     *config = h->force_tn;
+    if (!f32in && (h->force_tm == 0 || h->force_tm == -10) && h->w_igemm && !h->c_pad && h->so_same && conv_pw_reg_applicable(g, ep))
+        return ALT_PW_REG;
     const bool kxk = g.kh * g.kw > 1, tap = h->w_tap && conv_tap_supported(g, ep, f32in);
     const bool rows = h->w_rows && !fused && conv_rows_supported(g, ep, f32in);
     if (h->force_tm == -9) return rows ? ALT_ROWS : ALT_NONE;
@@ -730,7 +738,7 @@ int otter_hip_conv_launch_choice(const otter_hip_conv_t* h, int in_layout, int n
     const Epilogue ep = make_epilogue(h, out_layout);
     const int family = otter_hip_conv_kernel_kind(h, in_layout, n, in_h, in_w, out_layout);
     const AltKernel alt = alt_kernel(h, g, ep, in_layout == OTTER_HIP_F32_P8, family, false, &choice[1]);
-    choice[0] = alt == ALT_TAP ? 8 : alt == ALT_ROWS ? 9 : 0;
+    choice[0] = alt == ALT_TAP ? 8 : alt == ALT_ROWS ? 9 : alt == ALT_PW_REG ? 10 : 0;
     if (alt == ALT_NONE) choice[1] = 0;
     return OTTER_HIP_OK;
 }
@@ -836,6 +844,7 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
         if (alt == ALT_ROWS) return run_conv_rows(src, f32in, h->w_rows, out, g, ep, config, h->in_scale, d.in_round_mode, stream);
         if (alt == ALT_NONE) return hipSuccess;
         if ((twin || residual) && g.groups == 1 && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) fuse(ep);
+        if (alt == ALT_PW_REG) return run_conv_pw_reg((const int8_t*)src, h->w_igemm, h->so_one, out, g, ep, config, stream);
         return run_conv_tap(src, f32in, h->w_tap, out, g, ep, config, h->in_scale, d.in_round_mode, stream);
     };
     bool ran;
@@ -1507,7 +1516,7 @@ static AltKernel join_kernel(const otter_hip_conv* h, int in_layout, const ConvG
     if (pick_epilogue(ep, g.K) != EPI_F32_P4) return ALT_NONE;
     const int kind = pick_kernel(h, in_layout, g, ep);
     const AltKernel alt = alt_kernel(h, g, ep, false, kind, true, config);
-    *ok = alt == ALT_TAP || kind == 1;
+    *ok = alt == ALT_TAP || alt == ALT_PW_REG || kind == 1;
     return alt;
 }
 
@@ -1515,6 +1524,8 @@ static int join_run(const otter_hip_conv* h, const void* in, void* out, const Co
                     int config, hipStream_t stream) {
     if (alt == ALT_TAP)
         OHIP_CHECK(run_conv_tap(in, false, h->w_tap, out, g, ep, config, h->in_scale, h->d.in_round_mode, stream));
+    else if (alt == ALT_PW_REG)
+        OHIP_CHECK(run_conv_pw_reg((const int8_t*)in, h->w_igemm, h->so_one, out, g, ep, config, stream));
     else
         OHIP_CHECK(run_conv_igemm((const int8_t*)in, h->w_igemm, out, g, ep, h->force_tm > 0 ? h->force_tm : 0,
                                   h->force_tm > 0 ? h->force_tn : 0, stream));

@@ -525,6 +525,18 @@ __device__ __forceinline__ int quantize4(const ohip_v4i& f, float scale, float h
     return (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x06040200u);
 }
 
+typedef unsigned ohip_v4u __attribute__((__vector_size__(4 * sizeof(unsigned))));
+// A 16-byte buffer store whose row offset sits in a scalar register. The store unit reads the four data registers over
+// several cycles, and a vector instruction right behind the store that overwrites one of them can get there first: the
+// compiler separates the two behind a store with a constant offset, but takes a scalar-register offset to be safe, which
+// on this GPU it is not (seen in the fp32 depthwise epilogue at 16x128x52x52, where the next row's conversion follows the
+// store at once: 1 value in 50 000 was the next row's raw accumulator). The data registers are therefore kept live across
+// two wait states behind the store.
+__device__ __forceinline__ void store_b128_row(ohip_v4i data, __amdgpu_buffer_rsrc_t dst, unsigned v_off, unsigned s_off) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ohip_v4u, data), dst, (int)v_off, (int)s_off, 0);
+    asm volatile("s_nop 1" ::"v"(data) : "memory");
+}
+
 // n / d for 0 <= n < 2^31 as a multiplication: with 2^(l-1) < d <= 2^l and m = ceil(2^(31+l) / d) the error m d - 2^(31+l) is
 // below 2^l, so that n times it stays below 2^(31+l)
 struct FastDiv {

@@ -45,6 +45,13 @@ void conv_pw_stream_clamps(float act_hi, float round_half, const float* scale_ou
 hipError_t run_conv_pw_stream(const int8_t* x, const int8_t* wpk, const unsigned* qh, void* out, const ConvGeom& g,
                               const Epilogue& ep, int force_groups, int force_slices, hipStream_t stream);
 
+// conv_pw_reg.hip: pointwise int8 layers of at most 64 PW_REG_STEPS input channels, operands in registers
+constexpr int PW_REG_STEPS = 6;
+bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep);
+void conv_pw_reg_plan(const ConvGeom& g, bool wide, bool f32out, int* groups, int* per);
+hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* out, const ConvGeom& g, const Epilogue& ep, int force,
+                           hipStream_t stream);
+
 // conv_block.hip: 1x1 expand -> depthwise 3x3 -> 1x1 project (+ shortcut sum, + int8 twin) as one launch
 bool conv_block_applicable(const ConvGeom& ge, const Epilogue& e1, const ConvGeom& gd, const Epilogue& e2, const ConvGeom& gp,
                            const Epilogue& e3);

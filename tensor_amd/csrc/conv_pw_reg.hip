@@ -1,0 +1,349 @@
+// Pointwise (1x1, stride 1) int8 convolution with every operand in registers: no LDS, no barrier, no loop over the reduction.
+//
+// The pointwise layers of a network are short: a wave's whole reduction is CG <= 6 matrix steps, and what their launches cost is
+// the instructions around those and the latency of the first loads. The implicit-GEMM kernel spends 750 to 1500 vector and 640 to
+// 1700 scalar instructions per wave on 16 results a lane (its tap and column arithmetic, divisions, the way through LDS, 64-bit
+// addresses), where the requantization itself is 110 to 140. Here
+//  * a wave owns FN groups of 16 consecutive pixels (of the whole batch) and requests all their channels at once: the octets of a
+//    reduction step differ by a uniform offset, so a load is one instruction with no address arithmetic;
+//  * it walks `per` pairs of 16-row tiles of the output channels. The weights of a pair are refilled in place behind its last
+//    multiplication, its constants (and the elements of an addend) are requested one pair ahead;
+//  * the pixels of an XCD's workgroups are one contiguous run of the batch, the same for every slice of the output channels, so that
+//    a layer finds in its L2 what the layer before it wrote there.
+// Epilogues: int8 Byte8 and fp32 Float4 results, the latter with the addend, the int8 twin and the shuffle of the implicit-GEMM
+// kernel (common.hpp).
+#include "common.hpp"
+#include "conv_igemm.hpp"
+
+#include <algorithm>
+#include <cmath>
+
+namespace ohip {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef unsigned v2u_store __attribute__((__vector_size__(2 * sizeof(unsigned))));
+
+namespace {
+
+constexpr unsigned PR_OOB = 0x80000000u;  // past any buffer here: a load returns zero, a store is dropped
+
+struct PwRegArgs {
+    FastDiv hw;
+    int C8, K, HW, tiles, per, mt;  // tiles: workgroups along the pixels; mt: 16-row tiles of the packed weights per step
+    unsigned total_pix, in_bytes;
+    float so;     // the output scale of every channel
+    unsigned qh;  // upper clamp of the rounded result, in both halves (EPI_I8_P8_NONNEG)
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ v4i load16(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
+    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, (int)v, (int)s, 0));
+}
+__device__ __forceinline__ v2i load8(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
+    return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, (int)s, 0));
+}
+__device__ __forceinline__ void store16(__amdgpu_buffer_rsrc_t r, v4i d, unsigned v, unsigned s) { store_b128_row(d, r, v, s); }
+__device__ __forceinline__ void store8(__amdgpu_buffer_rsrc_t r, v2i d, unsigned v, unsigned s) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, d), r, (int)v, (int)s, 0);
+}
+
+}  // namespace
+
+template <int FN, int CG, int EPI>
+__global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
+                                                          PwRegArgs pa, Epilogue ep, JoinParam<EPI> ja) {
+    constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
+    constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
+    constexpr bool ADD = SHUF || FUSED;  // reads elements of another fp32 blob
+    const unsigned lane = threadIdx.x & 63, q = lane >> 4, p = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int xcd = blockIdx.x & 7, first = xcd * pa.tiles >> 3, tile = first + (int)(blockIdx.x >> 3);  // (grid.x is a multiple of 8)
+    const unsigned gp0 = (unsigned)(tile * 4 + wave) * (16 * FN);
+    if (tile >= (xcd + 1) * pa.tiles >> 3 || gp0 >= pa.total_pix) return;  // (uniform)
+    const int pairs = (pa.K + 31) / 32, pr0 = blockIdx.y * pa.per, pr1 = min(pr0 + pa.per, pairs);
+    const unsigned HW = pa.HW, K = pa.K, C8 = pa.C8;
+    const unsigned kpad = (unsigned)pa.mt * 16u;
+
+    // ---- weights and constants of a channel pair -------------------------------------------------------------------------------
+    const __amdgpu_buffer_rsrc_t rw = rsrc(wpk, (unsigned)(CG * pa.mt) * 1024u);
+    const __amdgpu_buffer_rsrc_t rsi = rsrc(ep.scale_in, kpad * 4), rbi = rsrc(ep.bias, kpad * 4);
+    v4i a[CG][2];
+    auto load_a = [&](int pr) {
+#pragma unroll
+        for (int cg = 0; cg < CG; ++cg)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) a[cg][h] = load16(rw, lane * 16 + h * 1024, (unsigned)(cg * pa.mt + 2 * pr) * 1024u);
+    };
+    struct Pair {
+        v4i si[2], bi[2];
+        v4i add[ADD ? FN : 1][2];
+    };
+
+    load_a(pr0);
+
+    // ---- the pixels: every channel of them requested now ---------------------------------------------------------------------------
+    const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.in_bytes);
+    unsigned n[FN], pix[FN];
+    bool ok[FN];
+    v4i b[FN][CG];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const unsigned gp = gp0 + 16 * j + p;
+        ok[j] = gp < pa.total_pix;
+        n[j] = div_by(gp, pa.hw), pix[j] = gp - n[j] * HW;
+        const unsigned v = ok[j] ? ((n[j] * C8 + 2 * q) * HW + pix[j]) * 8u : PR_OOB;
+#pragma unroll
+        for (int cg = 0; cg < CG; ++cg) {
+            const bool last = cg == CG - 1;  // only the last step may end in octets that do not exist
+            const v2i lo = load8(rin, !last || 8 * cg + 2 * q < C8 ? v : PR_OOB, (unsigned)cg * 64u * HW);
+            const v2i hi = load8(rin, !last || 8 * cg + 2 * q + 1 < C8 ? v : PR_OOB, ((unsigned)cg * 64u + 8u) * HW);
+            b[j][cg] = v4i{lo[0], lo[1], hi[0], hi[1]};
+        }
+    }
+
+    // byte offset of (image, this lane's channels of a pair, pixel) in a blob of K channels: Byte8, Float4, Float8; a pair is 32 HW
+    // (Byte8) or 128 HW (fp32) bytes further
+    auto at_b8 = [&](int j) { return ((n[j] * (K / 8) + q) * HW + pix[j]) * 8u; };
+    auto at_f4 = [&](int j) { return ((n[j] * (K / 4) + 2 * q) * HW + pix[j]) * 16u; };
+    auto at_f8 = [&](int j) { return ((n[j] * (K / 8) + q) * HW + pix[j]) * 32u; };
+    const unsigned f_bytes = pa.total_pix * K * 4u;
+    unsigned vo[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) vo[j] = ok[j] ? (I8 ? at_b8(j) : at_f4(j)) : PR_OOB;
+
+    auto load_pair = [&](Pair& k, int pr) {
+        const unsigned s = (unsigned)pr * 128u;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            k.si[h] = load16(rsi, q * 32 + h * 16, s), k.bi[h] = load16(rbi, q * 32 + h * 16, s);
+        if constexpr (SHUF) {
+            const __amdgpu_buffer_rsrc_t r = rsrc(ja.other, f_bytes);
+            const bool live = 32u * pr + 8 * q < K;
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const unsigned v = ok[j] && live ? (ja.other_pack == 8 ? at_f8(j) : at_f4(j)) : PR_OOB;  // (uniform choice)
+                k.add[j][0] = load16(r, v, s * HW);
+                k.add[j][1] = load16(r, v, s * HW + (ja.other_pack == 8 ? 16u : HW * 16u));
+            }
+        }
+        if constexpr (PARTS) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                if (ok[j] && 32u * pr + 8 * q < K)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        k.add[j][h] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep, ja, n[j], pix[j], (int)(32u * pr + 8 * q + 4 * h), (int)K, (int)HW));
+        } else if constexpr (FUSED) {
+            if (ep.residual != nullptr) {  // (uniform)
+                const __amdgpu_buffer_rsrc_t r = rsrc(ep.residual, f_bytes);
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) k.add[j][h] = load16(r, 32u * pr + 8 * q + 4 * h < K ? vo[j] : PR_OOB, s * HW + h * HW * 16u);
+            }
+        }
+    };
+
+    const __amdgpu_buffer_rsrc_t rout = rsrc(out, I8 ? pa.total_pix * K : f_bytes);
+    auto finish = [&](const Pair& k, int pr, v4i (&c0)[FN], v4i (&c1)[FN], auto lrelu_c) {
+        constexpr bool LRELU = decltype(lrelu_c)::value;
+        const unsigned ch0 = 32u * pr + 8 * q;
+        float si[8], bi[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) si[e] = __int_as_float(k.si[e / 4][e % 4]), bi[e] = __int_as_float(k.bi[e / 4][e % 4]);
+        if constexpr (I8) {
+            Epi8 prm;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) prm.si[e] = si[e], prm.bi[e] = bi[e], prm.so[e] = pa.so;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) prm.qh[e] = pa.qh;
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                const int a8[8] = {c0[j][0], c0[j][1], c0[j][2], c0[j][3], c1[j][0], c1[j][1], c1[j][2], c1[j][3]};
+                store8(rout, epi8_quant_i8p8<NONNEG, LRELU ? 1 : 0>(ep, prm, a8), ch0 < K ? vo[j] : PR_OOB, (unsigned)pr * 32u * HW);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                v4i r[2] = {epi4_dequant_f32p4<LRELU>(ep, si, bi, c0[j][0], c0[j][1], c0[j][2], c0[j][3]),
+                            epi4_dequant_f32p4<LRELU>(ep, si + 4, bi + 4, c1[j][0], c1[j][1], c1[j][2], c1[j][3])};
+                if constexpr (SHUF) {
+                    // with the same channels of the other blob these are channels 2 ch0 .. 2 ch0 + 15 of the shuffled one: two packs of 8
+                    const unsigned half = K / 8;  // packs of 8 in each half
+#pragma unroll
+                    for (int w = 0; w < 2; ++w) {
+                        float* const f = w ? ja.sh_out1 : ja.sh_out0;
+                        int8_t* const b8 = w ? ja.sh_q1 : ja.sh_q0;
+                        if (w ? 8u * pr + 8 <= half : 8u * pr >= half) continue;  // (uniform: none of the pair's packs is in this half)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const v4i o = k.add[j][h];
+                            const v4i even = ja.other_odd ? r[h] : o, odd = ja.other_odd ? o : r[h];  // (uniform)
+                            const v4i lo = {even[0], odd[0], even[1], odd[1]}, hi = {even[2], odd[2], even[3], odd[3]};
+                            const unsigned pack = ch0 / 4 + h - (w ? half : 0u);  // in this half; beyond it on either side: the other half's
+                            const unsigned e = n[j] * (unsigned)ja.sh_image + (pack * HW + pix[j]) * 8u;
+                            const bool live = ok[j] && pack < half;  // (a channel past the last one is a pack past the second half)
+                            if (f != nullptr) {
+                                const __amdgpu_buffer_rsrc_t rf = rsrc(f, PR_OOB);
+                                store16(rf, lo, live ? e * 4u : PR_OOB, 0), store16(rf, hi, (live ? e * 4u : PR_OOB) + 16u, 0);
+                            }
+                            if (b8 != nullptr)
+                                store8(rsrc(b8, PR_OOB), v2i{quantize4(lo, ep.twin_scale, ep.twin_half), quantize4(hi, ep.twin_scale, ep.twin_half)},
+                                       live ? e : PR_OOB, 0);
+                        }
+                    }
+                } else {
+                    v2i tw;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        if constexpr (FUSED) {
+                            if (PARTS || ep.residual != nullptr)
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) r[h][e] = __float_as_int(__fadd_rn(__int_as_float(r[h][e]), __int_as_float(k.add[j][h][e])));
+                            if (ep.twin != nullptr) tw[h] = quantize4(r[h], ep.twin_scale, ep.twin_half);
+                        }
+                        if (!FUSED || out != nullptr) store16(rout, r[h], ch0 + 4 * h < K ? vo[j] : PR_OOB, (unsigned)pr * 128u * HW + h * HW * 16u);
+                    }
+                    if constexpr (FUSED)
+                        if (ep.twin != nullptr)  // K % 8 == 0 then: the lane's 8 channels are one Byte8 element
+                            store8(rsrc(ep.twin, pa.total_pix * K), tw, ok[j] && ch0 < K ? at_b8(j) : PR_OOB, (unsigned)pr * 32u * HW);
+                }
+            }
+        }
+    };
+    auto step = [&](const Pair& k, Pair& next, int pr) {
+        if (pr + 1 < pr1) load_pair(next, pr + 1);
+        v4i c0[FN], c1[FN];
+#pragma unroll
+        for (int cg = 0; cg < CG; ++cg)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) {
+                c0[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[cg][0], b[j][cg], cg ? c0[j] : v4i{0, 0, 0, 0}, 0, 0, 0);
+                c1[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[cg][1], b[j][cg], cg ? c1[j] : v4i{0, 0, 0, 0}, 0, 0, 0);
+            }
+        if (pr + 1 < pr1) load_a(pr + 1);
+        if (!NONNEG && ep.lrelu) finish(k, pr, c0, c1, std::true_type{});  // (uniform)
+        else finish(k, pr, c0, c1, std::false_type{});
+    };
+    Pair k0, k1;
+    load_pair(k0, pr0);
+    for (int pr = pr0;;) {
+        step(k0, k1, pr);
+        if (++pr >= pr1) break;
+        step(k1, k0, pr);
+        if (++pr >= pr1) break;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------------------------------------------------------------
+
+static int pw_reg_epilogue(const Epilogue& ep, int K) {
+    const int epi = pick_epilogue(ep, K);
+    if (epi != EPI_F32_P4 || !ep.fused()) return epi;
+    return ep.join == nullptr ? EPI_F32_P4_FUSED : ep.join->other != nullptr ? EPI_F32_SHUFFLE : EPI_F32_P4_PARTS;
+}
+
+bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep) {
+    if (g.groups != 1 || g.kh != 1 || g.kw != 1 || g.sh != 1 || g.sw != 1 || g.ph != 0 || g.pw != 0) return false;
+    if (g.C % 8 || g.C > 64 * PW_REG_STEPS || g.N < 1) return false;
+    const int epi = pw_reg_epilogue(ep, g.K);
+    if (epi == EPI_GENERIC || ((ep.twin != nullptr || ep.join != nullptr) && g.K % 8)) return false;
+    const size_t px = (size_t)g.N * g.H * g.W;
+    // 32-bit byte offsets into every blob
+    return px * g.C < ((size_t)1 << 31) && px * g.K * (epi == EPI_F32_SHUFFLE ? 8 : layout_elem_bytes(ep.out_layout)) < ((size_t)1 << 31);
+}
+
+template <int FN, int CG, int EPI>
+static hipError_t launch_pw_reg(const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
+                                hipStream_t stream) {
+    hipLaunchKernelGGL((conv_pw_reg_kernel<FN, CG, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa, ep,
+                       JoinParam<EPI>::of(ep));
+    return hipGetLastError();
+}
+
+template <int FN, int CG>
+static hipError_t launch_pw_reg_e(int epi, const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
+                                  hipStream_t stream) {
+    switch (epi) {
+    case EPI_I8_P8: return launch_pw_reg<FN, CG, EPI_I8_P8>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_I8_P8_NONNEG: return launch_pw_reg<FN, CG, EPI_I8_P8_NONNEG>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_P4: return launch_pw_reg<FN, CG, EPI_F32_P4>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_P4_FUSED: return launch_pw_reg<FN, CG, EPI_F32_P4_FUSED>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_SHUFFLE: return launch_pw_reg<FN, CG, EPI_F32_SHUFFLE>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_P4_PARTS: return launch_pw_reg<FN, CG, EPI_F32_P4_PARTS>(x, wpk, out, pa, ep, slices, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+template <int CG>
+static hipError_t launch_pw_reg_wide(int epi, const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
+                                     hipStream_t stream) {
+    switch (epi) {
+    case EPI_I8_P8: return launch_pw_reg<4, CG, EPI_I8_P8>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_I8_P8_NONNEG: return launch_pw_reg<4, CG, EPI_I8_P8_NONNEG>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_P4: return launch_pw_reg<4, CG, EPI_F32_P4>(x, wpk, out, pa, ep, slices, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+// so: the output scale of every channel (int8 results); force: 0 = automatic, else pixel groups | pairs per wave << 3
+hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* out, const ConvGeom& g, const Epilogue& ep, int force,
+                           hipStream_t stream) {
+    if (!conv_pw_reg_applicable(g, ep)) return hipErrorInvalidValue;
+    const int epi = pw_reg_epilogue(ep, g.K), steps = igemm_channel_groups(g.C), pairs = (g.K + 31) / 32;
+    PwRegArgs pa;
+    pa.HW = g.H * g.W, pa.hw = fast_div((unsigned)pa.HW), pa.C8 = g.C / 8, pa.K = g.K, pa.mt = igemm_padded_rows(g.K) / 16, pa.so = so, pa.qh = 0;
+    const float both[2] = {so, so};
+    if (epi == EPI_I8_P8_NONNEG) conv_pw_stream_clamps(ep.act_hi, ep.round_half, both, 2, &pa.qh);
+    pa.total_pix = (unsigned)g.N * (unsigned)pa.HW, pa.in_bytes = pa.total_pix * (unsigned)g.C;
+    const bool wide = steps <= 4 && (epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG);  // (registers)
+    int fn = 1, per = 1;
+    conv_pw_reg_plan(g, wide, layout_elem_bytes(ep.out_layout) == 4, &fn, &per);
+    if (force) fn = force & 7, per = force >> 3;
+    if ((fn != 1 && fn != 2 && !(fn == 4 && wide)) || per < 1) return hipErrorInvalidValue;
+    per = std::min(per, pairs);
+    pa.per = per, pa.tiles = (int)((pa.total_pix + 64u * fn - 1) / (64u * fn));
+    const int slices = (pairs + per - 1) / per;
+    if (slices > 65535) return hipErrorInvalidValue;
+#define OHIP_PWR(CG_)                                                                                      \
+    if constexpr (CG_ <= 4)                                                                                \
+        if (steps == CG_ && fn == 4) return launch_pw_reg_wide<CG_>(epi, x, wpk, out, pa, ep, slices, stream); \
+    if (steps == CG_) return fn == 1 ? launch_pw_reg_e<1, CG_>(epi, x, wpk, out, pa, ep, slices, stream)    \
+                                     : launch_pw_reg_e<2, CG_>(epi, x, wpk, out, pa, ep, slices, stream);
+    OHIP_PWR(1)
+    OHIP_PWR(2)
+    OHIP_PWR(3)
+    OHIP_PWR(4)
+    OHIP_PWR(5)
+    OHIP_PWR(6)
+#undef OHIP_PWR
+    return hipErrorInvalidValue;
+}
+
+// Pixel groups of a wave (1, 2 or 4) and channel pairs that it walks. A pair costs a wave `pair` microseconds of latency whatever
+// else runs, a launch the cycles of its waves' loads and stores on the address unit of a compute unit (ta) and of their vector
+// instructions (va). More pairs per wave share the loads of the pixels and the prologue: with the pairs cut into slices the sum
+// is least at the square root below. Fitted to 150 drawn layers of 16 .. 384 input channels, 49 to 800 000 pixels: 2.7 % above
+// the best measured split on average. Against the launches of the other kernels (streamed, implicit GEMM, dealt reduction; the
+// faster one by their cost models) 80 % of the time; slower for 5 of the 150, by 14 % at worst (344 -> 448 @56x56 x2).
+void conv_pw_reg_plan(const ConvGeom& g, bool wide, bool f32out, int* groups, int* per) {
+    const int pairs = (g.K + 31) / 32, cg = igemm_channel_groups(g.C);
+    const float px = (float)g.N * (float)g.H * (float)g.W;
+    float best = __builtin_inff();
+    for (int fn = 1; fn <= (wide ? 4 : 2); fn *= 2) {
+        const float pair = 0.008f + 0.296f * (float)fn + 0.017f * (float)cg, waves = px / (float)(4096 * fn);  // per compute unit
+        const float once = (0.933f * (float)(fn * cg * 16) + 24.2f) / 2300.f;
+        const int want = std::clamp((int)(sqrtf(waves * (float)pairs * once / pair) + 0.5f), 1, pairs);
+        const int slices = (pairs + want - 1) / want, p = (pairs + slices - 1) / slices;
+        const float ta = (float)(p * (cg * 32 + 64 + fn * (f32out ? 32 : 8))), va = (float)p * (20.f + (float)fn * (f32out ? 36.f : 64.f));
+        const float t = (float)p * pair + waves * (float)slices * (once + (0.933f * ta + 0.404f * va) / 2300.f);
+        if (t < best) best = t, *groups = fn, *per = p;
+    }
+}
+
+}  // namespace ohip

@@ -1,0 +1,92 @@
+"""Pointwise layers on the launch that keeps its operands in registers (set_tile(-10, groups | pairs << 3)) against the implicit-GEMM
+kernel (set_tile(-4, 0)), bit for bit: ends of reduction steps, of pixel groups and of channel pairs, every split and epilogue."""
+import numpy as np
+import pytest
+
+from gpu_util import host_scale_in
+from tensor_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # C, K, N, H, W
+    (8, 8, 1, 1, 1),
+    (64, 40, 3, 5, 7),       # the last pair ends in its second octet; pixel groups across images
+    (72, 96, 2, 9, 13),      # the second reduction step holds one octet
+    (136, 264, 5, 4, 4),     # more pairs than a wave walks, images of one pixel group
+    (256, 32, 9, 16, 17),
+    (312, 72, 17, 3, 11),
+    (384, 24, 2, 13, 13),
+]
+SPLITS = [(1, 1), (2, 1), (1, 3), (2, 2), (4, 1), (4, 3), (0, 0)]
+
+
+def _layer(hip, rng, C, K, act, i8):
+    wq = rng.integers(-127, 128, (K, C, 1, 1)).astype(np.int8)
+    return hip.conv(wq=wq, scale_in=host_scale_in(np.full(K, 60.0, np.float32) + rng.uniform(0, 1, K).astype(np.float32), 20.0),
+                    bias=rng.normal(0, 1, K).astype(np.float32), in_scale=20.0, out_scale=[7.0] if i8 else None, act=act, act_p0=0.1,
+                    out_kind=capi.OUT_I8 if i8 else capi.OUT_F32)
+
+
+def _same(hip, got, want):
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert hip.torch.equal(a.view(hip.torch.uint8), b.view(hip.torch.uint8))
+
+
+@pytest.mark.parametrize("C,K,N,H,W", SHAPES)
+@pytest.mark.parametrize("i8", [True, False])
+def test_splits_and_activations(hip, C, K, N, H, W, i8):
+    rng = np.random.default_rng(C + K)
+    x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
+    for act in (0, 1, 2, 3):
+        conv = _layer(hip, rng, C, K if i8 else K - 4, act, i8)  # (fp32: a last octet of which half exists)
+        conv.set_tile(-4, 0)
+        want = conv.forward(x, capi.I8_P8, N, H, W)
+        for groups, pairs in SPLITS:
+            if groups == 4 and C > 256:
+                continue
+            conv.set_tile(-10, groups | pairs << 3)
+            assert conv.launch_choice(capi.I8_P8, N, H, W, conv.default_out_layout())[0] == 10
+            _same(hip, [conv.forward(x, capi.I8_P8, N, H, W)], [want])
+        conv.close()
+
+
+@pytest.mark.parametrize("C,K,N,H,W", SHAPES)
+@pytest.mark.parametrize("act", [1, 2])
+def test_sum_twin_and_joins(hip, C, K, N, H, W, act):
+    rng = np.random.default_rng(C * 2 + K)
+    x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
+    other = hip.to_device(rng.normal(0, 3, N * K * H * W).astype(np.float32))
+    conv = _layer(hip, rng, C, K, act, False)
+
+    def everything():
+        yield conv.forward_residual(x, capi.I8_P8, N, H, W, other, q_scale=9.0)
+        yield conv.forward_residual(x, capi.I8_P8, N, H, W, other)
+        yield conv.forward_twin(x, capi.I8_P8, N, H, W, 9.0, capi.ROUND_EXACT)
+        for layout, odd, joined in ((capi.F32_P8, False, False), (capi.F32_P4, True, True)):
+            for whole in (True, False):
+                yield conv.forward_shuffle(x, N, H, W, other, layout, odd, joined, 9.0, capi.ROUND_SSE, whole=whole)
+        if K > 8:
+            yield conv.forward_residual_concat(x, N, H, W, other[:N * 8 * H * W], capi.F32_P8, 8, other[N * 8 * H * W:], capi.F32_P4, 9.0)
+
+    conv.set_tile(-4, 0)
+    want = list(everything())
+    for groups, pairs in SPLITS:
+        if groups == 4:
+            continue
+        conv.set_tile(-10, groups | pairs << 3)
+        for got, w in zip(everything(), want):
+            _same(hip, got, w)
+    conv.set_tile(-10, 4 | 1 << 3)  # four groups with a sum: refused, as more registers than there are
+    with pytest.raises(capi.HipError):
+        conv.forward_residual(x, capi.I8_P8, N, H, W, other)
+    conv.close()
+
+
+def test_a_scale_per_output_channel_stays_with_the_other_kernels(hip):
+    rng = np.random.default_rng(5)
+    conv = hip.conv(wq=rng.integers(-127, 128, (16, 24, 1, 1)).astype(np.int8), scale_in=np.full(16, 1e-3, np.float32), in_scale=20.0,
+                    out_scale=list(rng.uniform(5, 9, 16)), out_kind=capi.OUT_I8)
+    assert conv.launch_choice(capi.I8_P8, 1, 7, 7, capi.I8_P8)[0] != 10
+    conv.close()
