@@ -322,7 +322,7 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * variant that stages several, tn alone leaves that choice automatic). tm < 0: keep the 3x3 halo kernel where it applies and force its pixel-fragment count to tn
  * (4..7, 0 = automatic; set on the first layer of a chain it also applies to otter_hip_conv_chain_forward's single
  * launch). tm == -2 on a depthwise 3x3 layer: force the matrix-core kernel's strip height to tn
- * steps of 8 / stride output rows (0 = automatic). tm == -3: use the vector-ALU depthwise kernels instead, with a
+ * steps of 8 / stride output rows, or with tn < 0 to -tn rows (0 = automatic). tm == -3: use the vector-ALU depthwise kernels instead, with a
  * strip height of (8 >> tn) output rows for stride 1 and (4 >> tn) for stride 2, tn in 0..2. tm == -4: the generic
  * implicit-GEMM kernel with its automatic tile choice, where the LDS-halo or the streamed 1x1 kernel would be picked.
  * tm == -5 on a layer the streamed 1x1 kernel takes: tn = groups | slices << 3 forces the 16-pixel groups a wave owns

@@ -930,7 +930,7 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
             gs.N = (n - b < per) ? n - b : per;
             const int8_t* xs = xq + (size_t)b * g.C * in_h * in_w;
             void* os = (char*)out + (size_t)b * g.K * g.OH * g.OW * layout_elem_bytes(out_layout);
-            if (mfma) OHIP_CHECK(run_conv_dw_mfma(xs, h->w_dw_mfma, os, gs, ep, epi, dw_shift, stream));
+            if (mfma) OHIP_CHECK(run_conv_dw_mfma(xs, h->w_dw_mfma, os, gs, ep, epi, h->force_tm == -2 ? h->force_tn : 0, stream));
             else OHIP_CHECK(run_conv_dw(xs, h->w_dw, os, gs, ep, dw_shift, stream));
         }
         break;

@@ -19,6 +19,7 @@
 // Image borders cost no instructions: loads and stores go through buffer descriptors, a lane that falls outside
 // the image carries an out-of-range offset, reads zero and writes nothing.
 #include <algorithm>
+#include <cmath>
 
 #include "common.hpp"
 #include "conv_dw_common.hpp"
@@ -72,71 +73,41 @@ __device__ __forceinline__ v4i dw_dequant4(const Epilogue& ep, const v4i& acc, c
     return res;
 }
 
+// What a launch is cut into, and the divisions of its indices (a division by a kernel argument is some 40 scalar instructions, and
+// a short strip's wave issues few others).
+struct DwPlan {
+    FastDiv gx, c8, chunks, lpi;  // by the workgroups along x, the octets, the column chunks of a row, the lane columns of an image
+    int rps, ipw;                 // output rows of a strip, images of a wave
+    unsigned total, in_bytes, out_bytes;
+};
+
 // A wave owns one channel octet x 16 lane columns (64 output pixels of a row at stride 1, 32 at stride 2) and walks
 // down `rps` output rows. The input rows live in a ring of 8 register fragments: a step computes 8/S output rows
 // from the ring and refills every slot as soon as its last reader has issued, so the loads run 5 input rows ahead of
 // the matrix instructions for the whole walk. Narrow images sit side by side in the wave (`lpi` lane columns each).
 template <int S, int EPI, bool ODDW, int KS>
-__global__ void __launch_bounds__(256) conv_dw3x3_mfma_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wa,
-                                                              void* __restrict__ out, ConvGeom g, Epilogue ep,
-                                                              int n_strips, int rps, int col_chunks, int lpi, int ipw,
-                                                              unsigned in_bytes, unsigned out_bytes) {
+__global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wa,
+                                                              void* __restrict__ out, ConvGeom g, Epilogue ep, DwPlan pl) {
     constexpr int RING = 8, U = RING / S;  // U output rows per step
     constexpr int PH = 4 / S;              // output pixels per lane column
     constexpr int T = S == 1 ? 2 : 1;      // A sets
-    const int C8 = g.C / 8;
+    const int C8 = (int)pl.c8.d, ipw = pl.ipw, rps = pl.rps;
     // Workgroups go to the 8 XCDs round-robin in launch order. Work items that share input cache lines - the column
     // chunks of a row (a 128-byte line straddles the chunk border), the strip groups of a plane (halo rows), the
     // octets of an image - get consecutive indices on ONE XCD, so that a shared line comes from memory once.
-    unsigned bx = blockIdx.x, by = blockIdx.y;
-    {
-        const unsigned id = by * gridDim.x + bx, total = gridDim.x * gridDim.y, per = total / 8;
-        if (id < per * 8) {
-            const unsigned w = (id % 8) * per + id / 8;
-            bx = w % gridDim.x, by = w / gridDim.x;
-        }
-    }
-    const int o = by % C8;
-    const int n0 = (by / C8) * ipw;
-    const int chunk = bx % col_chunks;
-    const int strip = __builtin_amdgcn_readfirstlane((bx / col_chunks) * (blockDim.x >> 6) + (threadIdx.x >> 6));
-    if (strip >= n_strips) return;  // whole wave
-    const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
+    unsigned w = blockIdx.y * pl.gx.d + blockIdx.x;
+    const unsigned per = pl.total / 8;
+    if (w < per * 8) w = (w % 8) * per + w / 8;
+    const unsigned by = div_by(w, pl.gx), bx = w - by * pl.gx.d, img = div_by(by, pl.c8), sg = div_by(bx, pl.chunks);
+    const int o = (int)(by - img * pl.c8.d), n0 = (int)img * ipw, chunk = (int)(bx - sg * pl.chunks.d);
+    const int strip = (int)sg;
+    const int lane = threadIdx.x, n = lane & 15, q = lane >> 4;
     int di = 0, nl = chunk * 16 + n;  // image within the wave, lane column within the image
     if (ipw > 1) {
-        di = n / lpi;
-        nl = n - di * lpi;
+        di = (int)div_by((unsigned)n, pl.lpi);
+        nl = n - di * (int)pl.lpi.d;
     }
     const bool lane_ok = di < ipw && n0 + di < g.N;
-
-    // ---- input: one 16-byte load per lane and row; per-lane byte offset fixed for the walk + per-row scalar offset --
-    const unsigned HW8 = (unsigned)(g.H * g.W * 8);
-    const int ic = 4 * nl - 2 + 2 * q;  // first input pixel of this lane's pair
-    const bool in_ok = lane_ok && ic >= 0 && ic < g.W;
-    const unsigned v_in = in_ok ? (unsigned)di * (unsigned)C8 * HW8 + (unsigned)ic * 8u : DW_OOB;
-    const unsigned v_in2 = (in_ok && ic + 1 < g.W) ? v_in + 8u : DW_OOB;  // second pixel of the pair (odd widths only)
-    const unsigned s_in = (unsigned)(n0 * C8 + o) * HW8;
-    const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, in_bytes);
-
-    const int oy0 = strip * rps;
-    const int iy0 = oy0 * S - g.ph;
-    const int rows_needed = (min(rps, g.OH - oy0) - 1) * S + KS;  // input rows this strip really reads
-    auto load_row = [&](int j) -> v4i {  // j: input row relative to iy0; rows outside the image or the strip read zero
-        const int iy = iy0 + j;
-        const bool ok = iy >= 0 && iy < g.H && j < rows_needed;  // wave-uniform
-        const unsigned s_row = ok ? s_in + (unsigned)(iy * g.W * 8) : 0u;
-        if constexpr (ODDW) {  // odd width: a row ends on half a pair, which is loaded as 8 bytes + zero
-            const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)(ok ? v_in : DW_OOB), (int)s_row, 0));
-            const v2i hi = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)(ok ? v_in2 : DW_OOB), (int)s_row, 0));
-            return v4i{lo[0], lo[1], hi[0], hi[1]};
-        }
-        const v4i f = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, (int)(ok ? v_in : DW_OOB), (int)s_row, 0));
-        return f;
-    };
-
-    v4i frag[RING];
-#pragma unroll
-    for (int j = 0; j < RING; ++j) frag[j] = load_row(j);
 
     v4i a[KS][T];
     {
@@ -146,6 +117,34 @@ __global__ void __launch_bounds__(256) conv_dw3x3_mfma_kernel(const int8_t* __re
 #pragma unroll
             for (int t = 0; t < T; ++t) a[dy][t] = ap[(dy * T + t) * 64];
     }
+
+    // ---- input: one 16-byte load per lane and row; per-lane byte offset fixed for the walk + per-row scalar offset --
+    const unsigned HW8 = (unsigned)(g.H * g.W * 8);
+    const int ic = 4 * nl - 2 + 2 * q;  // first input pixel of this lane's pair
+    const bool in_ok = lane_ok && ic >= 0 && ic < g.W;
+    const unsigned v_in = in_ok ? (unsigned)di * (unsigned)C8 * HW8 + (unsigned)ic * 8u : DW_OOB;
+    const unsigned v_in2 = (in_ok && ic + 1 < g.W) ? v_in + 8u : DW_OOB;  // second pixel of the pair (odd widths only)
+    const unsigned s_in = (unsigned)(n0 * C8 + o) * HW8;
+    const int oy0 = strip * rps;
+    const int iy0 = oy0 * S - g.ph;
+    const int rows_needed = (min(rps, g.OH - oy0) - 1) * S + KS;  // input rows this strip really reads
+    const unsigned row_end = (unsigned)min(g.H, iy0 + rows_needed);
+    // j: input row relative to iy0; rows outside the image or the strip read zero, through a descriptor of no bytes
+    auto load_row = [&](int j) -> v4i {
+        const int iy = iy0 + j;
+        const bool ok = (unsigned)iy < row_end;  // wave-uniform
+        const __amdgpu_buffer_rsrc_t r = dw_rsrc(x, ok ? pl.in_bytes : 0u);
+        const unsigned s_row = ok ? s_in + (unsigned)(iy * g.W * 8) : 0u;
+        if constexpr (ODDW) {  // odd width: a row ends on half a pair, which is loaded as 8 bytes + zero
+            const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v_in, (int)s_row, 0));
+            const v2i hi = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v_in2, (int)s_row, 0));
+            return v4i{lo[0], lo[1], hi[0], hi[1]};
+        }
+        return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, (int)v_in, (int)s_row, 0));
+    };
+    v4i frag[RING];
+#pragma unroll
+    for (int j = 0; j < RING; ++j) frag[j] = load_row(j);
 
     // ---- epilogue constants: stride 1 -> the octet's 8 channels (same for every lane); stride 2 -> this lane's 4 ----
     const int ch = 8 * o + (S == 1 ? 0 : 4 * (q & 1));
@@ -191,7 +190,7 @@ __global__ void __launch_bounds__(256) conv_dw3x3_mfma_kernel(const int8_t* __re
         s_out = (unsigned)(n0 * C8 + o) * OHW * 8u;
         row_bytes = (unsigned)g.OW * 8u;
     }
-    const __amdgpu_buffer_rsrc_t rout = dw_rsrc(out, out_bytes);
+    const __amdgpu_buffer_rsrc_t rout = dw_rsrc(out, pl.out_bytes);
 
     // Software pipeline, one output row deep: a step issues the matrix instructions of row r+1, refills the ring slots
     // they free, and then runs the epilogue of row r while those instructions execute. The scheduling barriers keep
@@ -207,9 +206,6 @@ __global__ void __launch_bounds__(256) conv_dw3x3_mfma_kernel(const int8_t* __re
     };
     v4i cur[T], nxt[T];
     row_mfma(0, cur);
-#pragma unroll
-    for (int k = 0; k < S; ++k) frag[k % RING] = load_row(k + RING);
-    __builtin_amdgcn_sched_barrier(0);
 
     auto epilogue_store = [&](unsigned v_o, unsigned s_row, bool row_ok) {
         if constexpr (EPI == EPI_F32_P4 || EPI == EPI_F32_P8) {
@@ -234,54 +230,74 @@ __global__ void __launch_bounds__(256) conv_dw3x3_mfma_kernel(const int8_t* __re
         }
     };
 
-    // A step of U rows is "interior" when every row it stores lies inside the strip and every row it loads inside
-    // the image: then the per-row scalar offsets just advance and nothing is predicated. The steps at the
-    // end of a strip take the checked path, which also leaves as soon as the strip's last row is stored (a strip need
-    // not be a whole number of steps).
     const int nrows = min(rps, g.OH - oy0);
+    unsigned s_st = s_out + (unsigned)oy0 * row_bytes;
+    if (rows_needed <= RING) {  // (wave-uniform) a short strip: every input row is in the ring already
+#pragma unroll
+        for (int u = 0; u < (RING - KS) / S + 1; ++u) {
+            if (u + 1 < nrows) row_mfma(u + 1, nxt);
+            epilogue_store(v_out, s_st, true);
+            if (u + 1 >= nrows) return;
+            s_st += row_bytes;
+#pragma unroll
+            for (int t = 0; t < T; ++t) cur[t] = nxt[t];
+        }
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k) frag[k % RING] = load_row(k + RING);
+    __builtin_amdgcn_sched_barrier(0);
+    // A step of U rows is "interior" when every row it stores lies inside the strip and every row it loads inside
+    // the image: then the per-row scalar offsets just advance and nothing is predicated. The step at the end of a strip takes the
+    // checked path (a strip need not be a whole number of steps). There, too, every load is in the main flow, only sent to nowhere:
+    // behind a return between the rows the compiler moves the loads down to their first use, a row's latency each.
     // loads of rows [RING, in_rows_ok) stay inside the image (iy0 + RING > 0); the few an interior step fetches past
     // the strip's own last row are rows the next strip reads anyway
+    const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, pl.in_bytes);
     const int in_rows_ok = g.H - iy0;
     const unsigned in_row_bytes = (unsigned)(g.W * 8);
-    for (int rb = 0; rb < nrows; rb += U) {
-        if (rb + U <= nrows && (rb + U) * S + S - 1 + RING < in_rows_ok) {
-            unsigned s_ld = s_in + (unsigned)(iy0 + (rb + 1) * S + RING) * in_row_bytes;
-            unsigned s_st = s_out + (unsigned)(oy0 + rb) * row_bytes;
+    // (two loops and not one with two paths: a ring slot that either path may refill is refilled elsewhere and copied at the end of a
+    // step, which waits for every load in flight)
+    int rb = 0;
+    for (; rb + U <= nrows && (rb + U) * S + S - 1 + RING < in_rows_ok; rb += U) {
+        unsigned s_ld = s_in + (unsigned)(iy0 + (rb + 1) * S + RING) * in_row_bytes;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                row_mfma((u + 1) % U, nxt);
+        for (int u = 0; u < U; ++u) {
+            row_mfma((u + 1) % U, nxt);
 #pragma unroll
-                for (int k = 0; k < S; ++k) {
-                    v4i& f = frag[((u + 1) * S + k) % RING];
-                    if constexpr (ODDW) {
-                        const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)v_in, (int)s_ld, 0));
-                        const v2i hi = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)v_in2, (int)s_ld, 0));
-                        f = v4i{lo[0], lo[1], hi[0], hi[1]};
-                    } else {
-                        f = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, (int)v_in, (int)s_ld, 0));
-                    }
-                    s_ld += in_row_bytes;
+            for (int k = 0; k < S; ++k) {
+                v4i& f = frag[((u + 1) * S + k) % RING];
+                if constexpr (ODDW) {
+                    const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)v_in, (int)s_ld, 0));
+                    const v2i hi = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)v_in2, (int)s_ld, 0));
+                    f = v4i{lo[0], lo[1], hi[0], hi[1]};
+                } else {
+                    f = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, (int)v_in, (int)s_ld, 0));
                 }
-                epilogue_store(v_out, s_st, true);
-                s_st += row_bytes;
-#pragma unroll
-                for (int t = 0; t < T; ++t) cur[t] = nxt[t];
-                __builtin_amdgcn_sched_barrier(0);
+                s_ld += in_row_bytes;
             }
-        } else {
+            epilogue_store(v_out, s_st, true);
+            s_st += row_bytes;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int r = rb + u;  // output row of the strip whose epilogue runs now
-                if (r >= nrows) return;  // wave-uniform
+            for (int t = 0; t < T; ++t) cur[t] = nxt[t];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    for (; rb < nrows; rb += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int r = rb + u;  // output row of the strip whose epilogue runs now
+            if (r < nrows) {       // wave-uniform
                 // row r+1: its input rows start (r+1)*S rows into the strip; the ring phase repeats every U rows
                 row_mfma((u + 1) % U, nxt);
-#pragma unroll
-                for (int k = 0; k < S; ++k) frag[((u + 1) * S + k) % RING] = load_row((r + 1) * S + k + RING);
-                epilogue_store(v_out, s_out + (unsigned)(oy0 + r) * row_bytes, true);
-#pragma unroll
-                for (int t = 0; t < T; ++t) cur[t] = nxt[t];
-                __builtin_amdgcn_sched_barrier(0);
+                epilogue_store(v_out, s_st, true);
             }
+#pragma unroll
+            for (int k = 0; k < S; ++k) frag[((u + 1) * S + k) % RING] = load_row((r + 1) * S + k + RING);
+            s_st += row_bytes;
+#pragma unroll
+            for (int t = 0; t < T; ++t) cur[t] = nxt[t];
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
@@ -618,6 +634,30 @@ bool dw_mfma_applicable(const ConvGeom& g, const Epilogue& ep, int epi, bool sca
     return in_bytes < ((size_t)1 << 31) && out_bytes < ((size_t)1 << 31);  // 32-bit buffer offsets
 }
 
+// Output rows of a strip. Its wave takes `row` microseconds per row whatever else runs, and as much as `extra` rows more where the
+// strip is longer than the ring of input rows holds; a SIMD with several waves takes their instructions one after the other, and up
+// to six of them the fullest SIMD (ceil) counts. columns: waves side by side at one strip per image. Fitted to 260 drawn layers of
+// 16 .. 960 channels, 7x7 to 208x208, 1 .. 64 images: the chosen height is 0.5 % slower than the best on average, 9 % at worst.
+// With the rule and kernel before (the tallest strips that leave 2048 waves, 8 / stride rows at least; seven divisions per wave)
+// 128 channels 5x5 LeakyReLU @13x13 x16 took 4.4 us (now 3.1), 384 @14x14 x1 3.6 (2.8), 88 @52x52 x16 6.0 (5.1).
+static int dw_strip_rows(const ConvGeom& g, int epi, float columns) {
+    const float row = 0.139f * (g.sh == 2 ? 0.624f : 1.f) * (g.kh == 5 ? 0.763f : 1.f) *
+                      (epi == EPI_I8_P8_NONNEG ? 0.89f : epi == EPI_I8_P8 ? 1.f : 0.596f);
+    const int step = 8 / g.sh, ring = (8 - g.kh) / g.sh + 1;  // output rows of a step, and those that the first input rows make
+    float best = __builtin_inff();
+    int rows = g.OH;
+    for (int r = g.OH;;) {
+        const int strips = (g.OH + r - 1) / r;
+        const float extra = r <= ring ? 0.f : r % step ? 4.258f : 2.865f, walk = row * ((float)r + extra);
+        const float m = columns * (float)strips / 1024.f, full = m <= 6.f ? ceilf(m) : m + 0.311f;
+        const float t = 0.788f * walk + (0.88f * fmaxf(m, 1.f) + 0.443f * full) * (0.306f + 0.55f * walk);
+        if (t < best) best = t, rows = r;
+        if (r == 1) return rows;
+        r = std::min(r - 1, (g.OH + strips) / (strips + 1));  // the height of the next number of strips
+    }
+}
+
+// strip_blocks: 0 = automatic, > 0: steps of 8 / stride output rows of a strip, < 0: rows of it
 hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const ConvGeom& g, const Epilogue& ep, int epi,
                             int strip_blocks, hipStream_t stream) {
     if (g.N == 0 || g.OH * g.OW == 0) return hipSuccess;
@@ -633,40 +673,24 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     }
     const long groups = (long)((g.N + ipw - 1) / ipw) * C8;
     if (groups > 65535) return hipErrorInvalidValue;  // grid.y limit; the caller splits the batch
-    // strip height: the tallest strips (setup and halo rows amortised over the longest walk) that still give about two
-    // waves per SIMD (measured: fewer, longer waves win), all of the same height so that the waves finish together
     const int U = 8 / g.sh;
-    const int blocks_total = (g.OH + U - 1) / U;
-    int rps;
-    if (strip_blocks > 0) {
-        rps = std::min(strip_blocks, blocks_total) * U;
-    } else {
-        int ns = 1;
-        while (ns < blocks_total && (long)col_chunks * ns * groups < 2048) ++ns;
-        rps = (g.OH + ns - 1) / ns;
-    }
+    const int rps = strip_blocks > 0   ? std::min(strip_blocks, (g.OH + U - 1) / U) * U
+                    : strip_blocks < 0 ? std::min(-strip_blocks, g.OH)
+                                       : dw_strip_rows(g, epi, (float)(col_chunks * groups));
     const int n_strips = (g.OH + rps - 1) / rps;
-    const int wpb = n_strips % 4 == 0 ? 4 : (n_strips % 2 == 0 ? 2 : 1);
-    const dim3 grid((unsigned)(col_chunks * (n_strips / wpb)), (unsigned)groups), block(64 * wpb);
-    // A grid of at most a few workgroups per CU is resident all at once, and the dispatcher is free to give one CU
-    // three of them and another one: the kernel then lasts as long as the fullest CU. Reserving a share of the CU's
-    // 160 KB of LDS per workgroup (the kernel uses none) caps the workgroups per CU at the even share.
-    constexpr long kCUs = 256;
-    const long wgs = (long)grid.x * grid.y;
-    const long per_cu = (wgs + kCUs - 1) / kCUs;
-    unsigned lds_reserve = 0;
-    if (wpb == 4 && per_cu >= 2 && per_cu <= 4) lds_reserve = (unsigned)(160 * 1024 / per_cu) / 1024 * 1024;
-    if (lds_reserve > 64 * 1024) lds_reserve = 64 * 1024;  // the default limit of dynamic LDS; still two per CU
+    // a workgroup is one strip: with two and four strips a workgroup, and shares of LDS reserved to even them out over the compute
+    // units, 140 drawn layers were 2 % and 5 % slower at their best strip height
+    const dim3 grid((unsigned)(col_chunks * n_strips), (unsigned)groups), block(64);
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW * (epi == EPI_F32_P4 || epi == EPI_F32_P8 ? 4 : 1));
+    const DwPlan pl = {fast_div(grid.x), fast_div((unsigned)C8), fast_div((unsigned)col_chunks), fast_div((unsigned)lpi),
+                       rps, ipw, grid.x * grid.y, in_bytes, out_bytes};
 #define OHIP_DWM_K(S_, E_, O_)                                                                                         \
     do {                                                                                                               \
         if (g.kh == 3)                                                                                                 \
-            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 3>), grid, block, lds_reserve, stream, x, wa, out, g, ep, \
-                               n_strips, rps, col_chunks, lpi, ipw, in_bytes, out_bytes);                              \
+            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 3>), grid, block, 0, stream, x, wa, out, g, ep, pl); \
         else                                                                                                           \
-            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 5>), grid, block, lds_reserve, stream, x, wa, out, g, ep, \
-                               n_strips, rps, col_chunks, lpi, ipw, in_bytes, out_bytes);                              \
+            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 5>), grid, block, 0, stream, x, wa, out, g, ep, pl); \
     } while (0)
 #define OHIP_DWM(S_, E_) \
     do {                                                                                                               \
