@@ -681,7 +681,7 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 }
 
 // A pointwise layer on an int8 blob takes the launch with its operands in registers (conv_pw_reg.hip) wherever that can run: at
-// most 384 input channels, one output scale for all channels, a packed result.
+// most 1024 input channels, one output scale for all channels, a packed result.
 // The launches beside those of `family` (1 or 3; with an fp32 blob also 6) that a layer may take, by the cost models: the kernel
 // whose workgroups deal the reduction to their waves (conv_tap.hip) and, for k x k layers without a sum or a twin, the one on
 // staged rows (conv_rows.hip). They have to be faster than the family's launch by 5 % (pointwise layers on an fp32 blob: 10 %):

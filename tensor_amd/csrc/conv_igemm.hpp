@@ -45,10 +45,10 @@ void conv_pw_stream_clamps(float act_hi, float round_half, const float* scale_ou
 hipError_t run_conv_pw_stream(const int8_t* x, const int8_t* wpk, const unsigned* qh, void* out, const ConvGeom& g,
                               const Epilogue& ep, int force_groups, int force_slices, hipStream_t stream);
 
-// conv_pw_reg.hip: pointwise int8 layers of at most 64 PW_REG_STEPS input channels, operands in registers
-constexpr int PW_REG_STEPS = 6;
+// conv_pw_reg.hip: pointwise int8 layers with their operands in registers; over 64 PW_REG_STEPS input channels the reduction is split
+constexpr int PW_REG_STEPS = 4, PW_REG_STEPS_SPLIT = 16;
 bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep);
-void conv_pw_reg_plan(const ConvGeom& g, bool wide, bool f32out, int* groups, int* per);
+void conv_pw_reg_plan(const ConvGeom& g, bool split, int max_groups, bool f32out, int* groups, int* per);
 hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* out, const ConvGeom& g, const Epilogue& ep, int force,
                            hipStream_t stream);
 

@@ -1,6 +1,6 @@
 // Pointwise (1x1, stride 1) int8 convolution with every operand in registers: no LDS, no barrier, no loop over the reduction.
 //
-// The pointwise layers of a network are short: a wave's whole reduction is CG <= 6 matrix steps, and what their launches cost is
+// The pointwise layers of a network are short: a wave's whole reduction is CG <= 4 matrix steps, and what their launches cost is
 // the instructions around those and the latency of the first loads. The implicit-GEMM kernel spends 750 to 1500 vector and 640 to
 // 1700 scalar instructions per wave on 16 results a lane (its tap and column arithmetic, divisions, the way through LDS, 64-bit
 // addresses), where the requantization itself is 110 to 140. Here
@@ -13,6 +13,7 @@
 // Epilogues: int8 Byte8 and fp32 Float4 results, the latter with the addend, the int8 twin and the shuffle of the implicit-GEMM
 // kernel (common.hpp).
 #include "common.hpp"
+#include "conv_dw_common.hpp"
 #include "conv_igemm.hpp"
 
 #include <algorithm>
@@ -20,9 +21,6 @@
 
 namespace ohip {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef unsigned v2u_store __attribute__((__vector_size__(2 * sizeof(unsigned))));
 
 namespace {
 
@@ -238,6 +236,183 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
     }
 }
 
+// The same for longer reductions (up to 64 PW_REG_STEPS_SPLIT input channels): the four waves of a workgroup own the same pixels and
+// take every fourth reduction step each, NS at most. Per channel pair their partial sums meet in LDS (integers: the same in any
+// order), and each wave finishes the half pairs (four channels of a lane's pixel) that are its own. One barrier per pair: the
+// sums of consecutive pairs lie in two buffers.
+template <int FN, int NS, int EPI>
+__global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
+                                                            PwRegArgs pa, Epilogue ep, JoinParam<EPI> ja) {
+    constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
+    constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
+    constexpr int OWN = FN < 2 ? 1 : FN / 2;  // half pairs that a wave finishes (of 2 FN; with FN == 1 waves 0 and 1 have one each)
+    __shared__ v4i red[2][2 * FN][3][64];     // [buffer][half pair][the other waves][lane]
+    const unsigned lane = threadIdx.x & 63, q = lane >> 4, p = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int xcd = blockIdx.x & 7, first = xcd * pa.tiles >> 3, tile = first + (int)(blockIdx.x >> 3);  // (grid.x is a multiple of 8)
+    if (tile >= (xcd + 1) * pa.tiles >> 3) return;  // (uniform over the workgroup)
+    const int pairs = (pa.K + 31) / 32, pr0 = blockIdx.y * pa.per, pr1 = min(pr0 + pa.per, pairs), steps = (pa.C8 + 7) / 8;
+    const unsigned HW = pa.HW, K = pa.K, C8 = pa.C8, kpad = (unsigned)pa.mt * 16u, f_bytes = pa.total_pix * K * 4u;
+
+    const __amdgpu_buffer_rsrc_t rw = rsrc(wpk, (unsigned)(steps * pa.mt) * 1024u);
+    const __amdgpu_buffer_rsrc_t rsi = rsrc(ep.scale_in, kpad * 4), rbi = rsrc(ep.bias, kpad * 4);
+    v4i a[NS][2];
+    auto load_a = [&](int pr) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const int s = wave + 4 * i;
+            if (i < NS - 1 || s < steps)  // (uniform; only a wave's last step may not exist)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) a[i][h] = load16(rw, lane * 16 + h * 1024, (unsigned)(s * pa.mt + 2 * pr) * 1024u);
+        }
+    };
+    load_a(pr0);
+
+    const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.in_bytes);
+    unsigned n[FN], pix[FN];
+    bool ok[FN];
+    v4i b[FN][NS];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const unsigned gp = (unsigned)tile * (16 * FN) + 16 * j + p;
+        ok[j] = gp < pa.total_pix;
+        n[j] = div_by(gp, pa.hw), pix[j] = gp - n[j] * HW;
+        const unsigned v = ok[j] ? ((n[j] * C8 + 2 * q) * HW + pix[j]) * 8u : PR_OOB;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const unsigned s = (unsigned)(wave + 4 * i);
+            if (i < NS - 1 || (int)s < steps) {  // (uniform) the last one may end in octets that do not exist
+                const v2i lo = load8(rin, 8 * s + 2 * q < C8 ? v : PR_OOB, s * 64u * HW);
+                const v2i hi = load8(rin, 8 * s + 2 * q + 1 < C8 ? v : PR_OOB, (s * 64u + 8u) * HW);
+                b[j][i] = v4i{lo[0], lo[1], hi[0], hi[1]};
+            } else {
+                b[j][i] = v4i{0, 0, 0, 0}, a[i][0] = a[i][1] = v4i{0, 0, 0, 0};
+            }
+        }
+    }
+    // this wave's half pairs: pixel group jo[o], channels 4 h .. 4 h + 3 of a lane's eight
+    const bool finishes = FN > 1 || wave < 2;  // (uniform)
+    struct Half {
+        v4i si, bi, add[OWN];
+    };
+    const unsigned h = wave & 1;
+    unsigned vo[OWN];  // byte offset of the half pair's element in the result; a pair is 32 HW (Byte8) or 128 HW (fp32) bytes further
+    unsigned no[OWN], po[OWN];
+    bool oko[OWN];
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+        const int jo = FN == 1 ? 0 : (wave >> 1) + 2 * o;
+        // (selected without an index into registers)
+        no[o] = n[0], po[o] = pix[0], oko[o] = ok[0];
+#pragma unroll
+        for (int j = 1; j < FN; ++j)
+            if (j == jo) no[o] = n[j], po[o] = pix[j], oko[o] = ok[j];
+        vo[o] = !oko[o] ? PR_OOB : I8 ? ((no[o] * (K / 8) + q) * HW + po[o]) * 8u + 4 * h : ((no[o] * (K / 4) + 2 * q + h) * HW + po[o]) * 16u;
+    }
+    auto load_half = [&](Half& k, int pr) {
+        const unsigned s = (unsigned)pr * 128u, ch = 32u * pr + 8 * q + 4 * h;
+        k.si = load16(rsi, q * 32 + h * 16, s), k.bi = load16(rbi, q * 32 + h * 16, s);
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            if constexpr (SHUF) {
+                const unsigned v = ja.other_pack == 8 ? ((no[o] * (K / 8) + q) * HW + po[o]) * 32u + 16 * h : vo[o];  // (uniform choice)
+                k.add[o] = load16(rsrc(ja.other, f_bytes), oko[o] && ch < K ? v : PR_OOB, s * HW);
+            }
+            if constexpr (PARTS) {
+                if (oko[o] && ch < K) k.add[o] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep, ja, no[o], po[o], (int)ch, (int)K, (int)HW));
+            } else if constexpr (FUSED) {
+                if (ep.residual != nullptr) k.add[o] = load16(rsrc(ep.residual, f_bytes), ch < K ? vo[o] : PR_OOB, s * HW);  // (uniform)
+            }
+        }
+    };
+    const __amdgpu_buffer_rsrc_t rout = rsrc(out, I8 ? pa.total_pix * K : f_bytes);
+    auto finish = [&](const Half& k, int pr, const v4i (&c)[OWN]) {
+        const unsigned ch = 32u * pr + 8 * q + 4 * h;
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            if constexpr (I8) {
+                const v4i so = v4i{1, 1, 1, 1} * __float_as_int(pa.so);
+                const unsigned w = dw_requant4<NONNEG>(ep, c[o], k.si, k.bi, so, pa.qh, pa.qh);
+                __builtin_amdgcn_raw_buffer_store_b32(w, rout, (int)(ch < K ? vo[o] : PR_OOB), (int)((unsigned)pr * 32u * HW), 0);
+                continue;
+            }
+            float si[4], bi[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) si[e] = __int_as_float(k.si[e]), bi[e] = __int_as_float(k.bi[e]);
+            v4i r = ep.lrelu ? epi4_dequant_f32p4<true>(ep, si, bi, c[o][0], c[o][1], c[o][2], c[o][3])  // (uniform)
+                             : epi4_dequant_f32p4<false>(ep, si, bi, c[o][0], c[o][1], c[o][2], c[o][3]);
+            if constexpr (SHUF) {
+                // with the same channels of the other blob these are channels 2 ch .. 2 ch + 7 of the shuffled one: a pack of 8
+                const v4i even = ja.other_odd ? r : k.add[o], odd = ja.other_odd ? k.add[o] : r;  // (uniform)
+                const v4i lo = {even[0], odd[0], even[1], odd[1]}, hi = {even[2], odd[2], even[3], odd[3]};
+                const unsigned half = K / 8;  // packs of 8 in each half of the 2 K channels
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    float* const f = w ? ja.sh_out1 : ja.sh_out0;
+                    int8_t* const b8 = w ? ja.sh_q1 : ja.sh_q0;
+                    const unsigned pack = ch / 4 - (w ? half : 0u);  // beyond this half on either side: the other half's
+                    const unsigned e = no[o] * (unsigned)ja.sh_image + (pack * HW + po[o]) * 8u;
+                    const bool live = oko[o] && pack < half;
+                    if (f != nullptr) {
+                        const __amdgpu_buffer_rsrc_t rf = rsrc(f, PR_OOB);
+                        store16(rf, lo, live ? e * 4u : PR_OOB, 0), store16(rf, hi, (live ? e * 4u : PR_OOB) + 16u, 0);
+                    }
+                    if (b8 != nullptr)
+                        store8(rsrc(b8, PR_OOB), v2i{quantize4(lo, ep.twin_scale, ep.twin_half), quantize4(hi, ep.twin_scale, ep.twin_half)},
+                               live ? e : PR_OOB, 0);
+                }
+            } else {
+                if constexpr (FUSED)
+                    if (PARTS || ep.residual != nullptr)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) r[e] = __float_as_int(__fadd_rn(__int_as_float(r[e]), __int_as_float(k.add[o][e])));
+                if (!FUSED || out != nullptr) store16(rout, r, ch < K ? vo[o] : PR_OOB, (unsigned)pr * 128u * HW);
+                if constexpr (FUSED)
+                    if (ep.twin != nullptr)
+                        __builtin_amdgcn_raw_buffer_store_b32((unsigned)quantize4(r, ep.twin_scale, ep.twin_half), rsrc(ep.twin, pa.total_pix * K),
+                                                              (int)(oko[o] && ch < K ? ((no[o] * (K / 8) + q) * HW + po[o]) * 8u + 4 * h : PR_OOB),
+                                                              (int)((unsigned)pr * 32u * HW), 0);
+            }
+        }
+    };
+    Half k0, k1;
+    if (finishes) load_half(k0, pr0);
+    for (int pr = pr0; pr < pr1; ++pr) {
+        v4i c[FN][2];
+#pragma unroll
+        for (int i = 0; i < NS; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) c[j][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i][t], b[j][i], i ? c[j][t] : v4i{0, 0, 0, 0}, 0, 0, 0);
+        if (pr + 1 < pr1) {
+            load_a(pr + 1);
+            if (finishes) load_half(k1, pr + 1);
+        }
+        // half pair u = 2 j + t belongs to wave (j % 2) * 2 + t (FN == 1: wave t)
+        v4i own[OWN];
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int w = FN == 1 ? t : (j & 1) * 2 + t;
+                if (wave == w) own[j >> 1] = c[j][t];
+                else red[pr & 1][2 * j + t][wave < w ? wave : wave - 1][lane] = c[j][t];
+            }
+        __syncthreads();
+        if (finishes) {
+#pragma unroll
+            for (int o = 0; o < OWN; ++o) {
+                const int u = FN == 1 ? wave : 2 * ((wave >> 1) + 2 * o) + (wave & 1);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) own[o] += red[pr & 1][u][i][lane];
+            }
+            finish(k0, pr, own);
+            k0 = k1;
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------------------------------------------------
@@ -250,7 +425,7 @@ static int pw_reg_epilogue(const Epilogue& ep, int K) {
 
 bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep) {
     if (g.groups != 1 || g.kh != 1 || g.kw != 1 || g.sh != 1 || g.sw != 1 || g.ph != 0 || g.pw != 0) return false;
-    if (g.C % 8 || g.C > 64 * PW_REG_STEPS || g.N < 1) return false;
+    if (g.C % 8 || g.C > 64 * PW_REG_STEPS_SPLIT || g.N < 1) return false;
     const int epi = pw_reg_epilogue(ep, g.K);
     if (epi == EPI_GENERIC || ((ep.twin != nullptr || ep.join != nullptr) && g.K % 8)) return false;
     const size_t px = (size_t)g.N * g.H * g.W;
@@ -291,7 +466,29 @@ static hipError_t launch_pw_reg_wide(int epi, const int8_t* x, const int8_t* wpk
     return hipErrorInvalidValue;
 }
 
-// so: the output scale of every channel (int8 results); force: 0 = automatic, else pixel groups | pairs per wave << 3
+template <int FN, int NS, int EPI>
+static hipError_t launch_pw_split(const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
+                                  hipStream_t stream) {
+    hipLaunchKernelGGL((conv_pw_split_kernel<FN, NS, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa, ep,
+                       JoinParam<EPI>::of(ep));
+    return hipGetLastError();
+}
+
+template <int FN, int NS>
+static hipError_t launch_pw_split_e(int epi, const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
+                                    hipStream_t stream) {
+    switch (epi) {
+    case EPI_I8_P8: return launch_pw_split<FN, NS, EPI_I8_P8>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_I8_P8_NONNEG: return launch_pw_split<FN, NS, EPI_I8_P8_NONNEG>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_P4: return launch_pw_split<FN, NS, EPI_F32_P4>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_P4_FUSED: return launch_pw_split<FN, NS, EPI_F32_P4_FUSED>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_SHUFFLE: return launch_pw_split<FN, NS, EPI_F32_SHUFFLE>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_P4_PARTS: return launch_pw_split<FN, NS, EPI_F32_P4_PARTS>(x, wpk, out, pa, ep, slices, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+// so: the output scale of every channel (int8 results); force: 0 = automatic, else pixel groups | 64 if the reduction is split | pairs per wave << 7
 hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* out, const ConvGeom& g, const Epilogue& ep, int force,
                            hipStream_t stream) {
     if (!conv_pw_reg_applicable(g, ep)) return hipErrorInvalidValue;
@@ -301,47 +498,64 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
     const float both[2] = {so, so};
     if (epi == EPI_I8_P8_NONNEG) conv_pw_stream_clamps(ep.act_hi, ep.round_half, both, 2, &pa.qh);
     pa.total_pix = (unsigned)g.N * (unsigned)pa.HW, pa.in_bytes = pa.total_pix * (unsigned)g.C;
-    const bool wide = steps <= 4 && (epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG);  // (registers)
     int fn = 1, per = 1;
-    conv_pw_reg_plan(g, wide, layout_elem_bytes(ep.out_layout) == 4, &fn, &per);
-    if (force) fn = force & 7, per = force >> 3;
-    if ((fn != 1 && fn != 2 && !(fn == 4 && wide)) || per < 1) return hipErrorInvalidValue;
+    const bool split = force ? (force & 64) != 0 : steps > PW_REG_STEPS;
+    const bool wide = split || epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG;  // (registers)
+    conv_pw_reg_plan(g, split, wide ? 4 : 2, layout_elem_bytes(ep.out_layout) == 4, &fn, &per);
+    if (force) fn = force & 7, per = force >> 7;
+    if ((fn != 1 && fn != 2 && !(fn == 4 && wide)) || per < 1 || (split ? steps < 2 : steps > PW_REG_STEPS)) return hipErrorInvalidValue;
     per = std::min(per, pairs);
-    pa.per = per, pa.tiles = (int)((pa.total_pix + 64u * fn - 1) / (64u * fn));
+    const unsigned wg_pix = (split ? 16u : 64u) * (unsigned)fn;
+    pa.per = per, pa.tiles = (int)((pa.total_pix + wg_pix - 1) / wg_pix);
     const int slices = (pairs + per - 1) / per;
     if (slices > 65535) return hipErrorInvalidValue;
+    if (split) {
+#define OHIP_PWS(NS_)                                                                                             \
+    if ((steps + 3) / 4 == NS_) return fn == 1   ? launch_pw_split_e<1, NS_>(epi, x, wpk, out, pa, ep, slices, stream) \
+                                       : fn == 2 ? launch_pw_split_e<2, NS_>(epi, x, wpk, out, pa, ep, slices, stream) \
+                                                 : launch_pw_split_e<4, NS_>(epi, x, wpk, out, pa, ep, slices, stream);
+        OHIP_PWS(1)
+        OHIP_PWS(2)
+        OHIP_PWS(3)
+        OHIP_PWS(4)
+#undef OHIP_PWS
+        return hipErrorInvalidValue;
+    }
 #define OHIP_PWR(CG_)                                                                                      \
-    if constexpr (CG_ <= 4)                                                                                \
-        if (steps == CG_ && fn == 4) return launch_pw_reg_wide<CG_>(epi, x, wpk, out, pa, ep, slices, stream); \
+    if (steps == CG_ && fn == 4) return launch_pw_reg_wide<CG_>(epi, x, wpk, out, pa, ep, slices, stream); \
     if (steps == CG_) return fn == 1 ? launch_pw_reg_e<1, CG_>(epi, x, wpk, out, pa, ep, slices, stream)    \
                                      : launch_pw_reg_e<2, CG_>(epi, x, wpk, out, pa, ep, slices, stream);
     OHIP_PWR(1)
     OHIP_PWR(2)
     OHIP_PWR(3)
     OHIP_PWR(4)
-    OHIP_PWR(5)
-    OHIP_PWR(6)
 #undef OHIP_PWR
     return hipErrorInvalidValue;
 }
 
 // Pixel groups of a wave (1, 2 or 4) and channel pairs that it walks. A pair costs a wave `pair` microseconds of latency whatever
 // else runs, a launch the cycles of its waves' loads and stores on the address unit of a compute unit (ta) and of their vector
-// instructions (va). More pairs per wave share the loads of the pixels and the prologue: with the pairs cut into slices the sum
-// is least at the square root below. Fitted to 150 drawn layers of 16 .. 384 input channels, 49 to 800 000 pixels: 2.7 % above
-// the best measured split on average. Against the launches of the other kernels (streamed, implicit GEMM, dealt reduction; the
-// faster one by their cost models) 80 % of the time; slower for 5 of the 150, by 14 % at worst (344 -> 448 @56x56 x2).
-void conv_pw_reg_plan(const ConvGeom& g, bool wide, bool f32out, int* groups, int* per) {
+// instructions (va). More pairs per wave share the loads of the pixels and the prologue (once): with the pairs cut into slices the
+// sum is least at the square root below.
+// Whole reductions (at most 256 channels): fitted to 150 drawn layers of 16 .. 384 channels, 49 to 800 000 pixels, 2.7 % above the
+// best measured split on average, 80 % of the time of the launches before (streamed, implicit GEMM, dealt reduction; the faster
+// by their cost models). Split reductions: 138 layers of 257 .. 960 channels, 2.3 % above the best, 85 % of the best of the
+// implicit-GEMM kernel and every tile of the dealt reduction. Where both can run: 257 .. 384 channels 5 % faster split, 193 .. 256 2 %
+// and up to 192 8 % slower.
+void conv_pw_reg_plan(const ConvGeom& g, bool split, int max_groups, bool f32out, int* groups, int* per) {
     const int pairs = (g.K + 31) / 32, cg = igemm_channel_groups(g.C);
     const float px = (float)g.N * (float)g.H * (float)g.W;
     float best = __builtin_inff();
-    for (int fn = 1; fn <= (wide ? 4 : 2); fn *= 2) {
-        const float pair = 0.008f + 0.296f * (float)fn + 0.017f * (float)cg, waves = px / (float)(4096 * fn);  // per compute unit
-        const float once = (0.933f * (float)(fn * cg * 16) + 24.2f) / 2300.f;
+    for (int fn = 1; fn <= max_groups; fn *= 2) {
+        const float f = (float)fn, c = (float)cg;
+        const float waves = px / (4096.f * f) * (split ? 16.f : 1.f);  // per compute unit (split: workgroups)
+        const float pair = split ? 0.11f + 0.203f * f + 0.051f * c : 0.008f + 0.296f * f + 0.017f * c;
+        const float once = (split ? 0.27f * f * c + 142.f : 14.9f * f * c + 24.2f) / 2300.f;
         const int want = std::clamp((int)(sqrtf(waves * (float)pairs * once / pair) + 0.5f), 1, pairs);
         const int slices = (pairs + want - 1) / want, p = (pairs + slices - 1) / slices;
-        const float ta = (float)(p * (cg * 32 + 64 + fn * (f32out ? 32 : 8))), va = (float)p * (20.f + (float)fn * (f32out ? 36.f : 64.f));
-        const float t = (float)p * pair + waves * (float)slices * (once + (0.933f * ta + 0.404f * va) / 2300.f);
+        const float ta = 32.f * c + 64.f + f * (f32out ? 32.f : 8.f), va = 20.f + f * (f32out ? 36.f : 64.f);
+        const float each = (split ? 0.017f * ta + 6.5f + 1.6f * f : 0.933f * ta + 0.404f * va) / 2300.f;
+        const float t = (float)p * pair + (split ? 1.21f * f : 0.f) + waves * (float)slices * (once + (float)p * each);
         if (t < best) best = t, *groups = fn, *per = p;
     }
 }

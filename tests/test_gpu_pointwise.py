@@ -1,4 +1,4 @@
-"""Pointwise layers on the launch that keeps its operands in registers (set_tile(-10, groups | pairs << 3)) against the implicit-GEMM
+"""Pointwise layers on the launch that keeps its operands in registers (set_tile(-10, groups | pairs << 7)) against the implicit-GEMM
 kernel (set_tile(-4, 0)), bit for bit: ends of reduction steps, of pixel groups and of channel pairs, every split and epilogue."""
 import numpy as np
 import pytest
@@ -16,8 +16,14 @@ SHAPES = [  # C, K, N, H, W
     (256, 32, 9, 16, 17),
     (312, 72, 17, 3, 11),
     (384, 24, 2, 13, 13),
+    (968, 136, 1, 5, 9),     # sixteen reduction steps, the last of one octet
 ]
-SPLITS = [(1, 1), (2, 1), (1, 3), (2, 2), (4, 1), (4, 3), (0, 0)]
+# groups, pairs, and whether the waves of a workgroup share the reduction (needs two steps of 64 channels; otherwise at most four)
+SPLITS = [(1, 1, 0), (2, 1, 0), (1, 3, 0), (2, 2, 0), (4, 1, 0), (4, 3, 0), (1, 1, 64), (1, 3, 64), (2, 1, 64), (2, 2, 64), (4, 3, 64), (0, 0, 0)]
+
+
+def _can(C, groups, split):
+    return groups == 0 or (C > 64 if split else C <= 256)
 
 
 def _layer(hip, rng, C, K, act, i8):
@@ -43,10 +49,10 @@ def test_splits_and_activations(hip, C, K, N, H, W, i8):
         conv = _layer(hip, rng, C, K if i8 else K - 4, act, i8)  # (fp32: a last octet of which half exists)
         conv.set_tile(-4, 0)
         want = conv.forward(x, capi.I8_P8, N, H, W)
-        for groups, pairs in SPLITS:
-            if groups == 4 and C > 256:
+        for groups, pairs, split in SPLITS:
+            if not _can(C, groups, split):
                 continue
-            conv.set_tile(-10, groups | pairs << 3)
+            conv.set_tile(-10, groups | split | pairs << 7)
             assert conv.launch_choice(capi.I8_P8, N, H, W, conv.default_out_layout())[0] == 10
             _same(hip, [conv.forward(x, capi.I8_P8, N, H, W)], [want])
         conv.close()
@@ -72,13 +78,13 @@ def test_sum_twin_and_joins(hip, C, K, N, H, W, act):
 
     conv.set_tile(-4, 0)
     want = list(everything())
-    for groups, pairs in SPLITS:
-        if groups == 4:
+    for groups, pairs, split in SPLITS:
+        if not _can(C, groups, split) or (groups == 4 and not split):
             continue
-        conv.set_tile(-10, groups | pairs << 3)
+        conv.set_tile(-10, groups | split | pairs << 7)
         for got, w in zip(everything(), want):
             _same(hip, got, w)
-    conv.set_tile(-10, 4 | 1 << 3)  # four groups with a sum: refused, as more registers than there are
+    conv.set_tile(-10, 4 | 1 << 7)  # four groups with a sum: refused, as more registers than there are
     with pytest.raises(capi.HipError):
         conv.forward_residual(x, capi.I8_P8, N, H, W, other)
     conv.close()
