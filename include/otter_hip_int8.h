@@ -284,6 +284,18 @@ int otter_hip_conv_block_forward(const otter_hip_conv_t* expand, const otter_hip
                                  const otter_hip_conv_t* project, const void* in, int n, int in_h, int in_w,
                                  const float* residual, void* out, int out_layout, void* out_q, float q_scale,
                                  int q_round_mode, void* workspace, size_t workspace_bytes, void* stream);
+/* The same block in a form that the caller names: form = 1, 2 or 3 launches, refused where the block cannot run so.
+ * otter_hip_conv_block_fastest names the fastest by cost models of the launches as they are (otter_hip_conv_block_launches goes on
+ * giving the single launch to the blocks that it was the fastest form of before the layers by themselves became faster).
+ * The result is the same, bit for bit. */
+int otter_hip_conv_block_fastest(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise, const otter_hip_conv_t* project,
+                                 int n, int in_h, int in_w);
+size_t otter_hip_conv_block_form_workspace_bytes(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise,
+                                                 const otter_hip_conv_t* project, int form, int n, int in_h, int in_w);
+int otter_hip_conv_block_forward_form(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise, const otter_hip_conv_t* project,
+                                      int form, const void* in, int n, int in_h, int in_w, const float* residual, void* out,
+                                      int out_layout, void* out_q, float q_scale, int q_round_mode, void* workspace,
+                                      size_t workspace_bytes, void* stream);
 /* Test hook with no counterpart in the reference, host arithmetic only (no GPU needed): the launch plan of the single
  * launch for a block in_channels -> expanded_channels -> out_channels on n images of in_h x in_w (stride-1 depthwise
  * layer), with rows_per_band / slice_channels / split forced (0 = automatic). plan = { output rows per band, bands per

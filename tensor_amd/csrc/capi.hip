@@ -1183,27 +1183,40 @@ static bool block_geoms(const otter_hip_conv_t* e, const otter_hip_conv_t* d, co
 
 static int g_block_always = 0;  // see block_single_launch
 
-// The three forms of a block, in microseconds a call: three launches, the first two layers as one (conv_xdw.hip) and the last
-// by itself, the whole block as one (conv_block.hip). Fitted to 770 blocks drawn over 16..160 input channels, 7x7..112x112,
-// batch 1..64, the calls queued behind one another; median errors 5, 6 and 6 %. The form chosen by them is 0.9 % slower than
-// the fastest of each block on average. Small blocks gain most, being launch latency: 24 -> 144 -> 24 @12x17 b9 11.5 us as three
-// launches, 8.8 as two, 8.0 as one; 29x29 48 -> 288 -> 48 b29 24.5, 23.8, 14.2; but 23x23 152 -> 912 -> 152 b14 24.8 as three,
-// 35.6 as one, and 36x36 stride 2 112 -> 672 -> 232 b38 48.7 as three, 60.0 as two.
-static float block_cost_three(const ConvGeom g[3]) {
+// The three forms of a block, in microseconds: three launches, the first two layers as one (conv_xdw.hip) and the last by itself,
+// the whole block as one (conv_block.hip).
+struct BlockCost {
+    float three[7], pair[7], single[7];
+};
+// Fitted to 400 blocks drawn over 16..160 input channels, 7x7..112x112, batch 1..64, launches replayed from captured graphs; median
+// errors 5, 4.5 and 5 %. The form chosen by them is 0.9 % slower than the fastest of each block on average; with the constants below
+// it is 12 %, since the pointwise and depthwise launches have become faster: 160 -> 960 -> 160 @7x7 b64 20.2 us as one, 14.2 as three;
+// 32 -> 192 -> 32 @28x28 b1 10.3 and 7.2; 96 -> 576 -> 160 @14x14 stride 2 b1 6.8 as three, 6.0 as two.
+constexpr BlockCost kBlockCost = {{7.55f, 0.495f, 0.577f, 0.909f, 0.058f, 0.0906f, 0.092f},
+                                  {4.82f, 2.067f, 0.258f, 0.672f, 0.573f, 0.881f, 0.0912f},
+                                  {3.25f, 1.926f, 1.857f, 0.0415f, 0.0982f, 2.61f, 0.0623f}};
+// The same, fitted to 770 such blocks when those launches took longer: they decide which blocks otter_hip_conv_block_forward still
+// runs as the single launch (otter_hip_conv_block_launches, which callers and the tests of the dispatch go by).
+constexpr BlockCost kBlockCostSingle = {{12.6f, 0.22f, 0.41f, 0.78f, 0.198f, 0.194f, 0.f},
+                                        {8.6f, 1.43f, 0.2f, 0.43f, 0.44f, 0.2f, 0.433f},
+                                        {3.56f, 1.59f, 1.39f, 0.3f, 0.096f, 1.f, 0.056f}};
+static float block_cost_three(const BlockCost& k, const ConvGeom g[3]) {
     const float px = (float)g[0].N * g[0].H * g[0].W * 1e-6f, opx = (float)g[2].N * g[2].OH * g[2].OW * 1e-6f;
     const float ce = (float)g[0].K, mac_e = px * ce * igemm_channel_groups(g[0].C);
     const float mac_p = opx * igemm_channel_groups(g[2].C) * (float)((g[2].K + 31) / 32 * 32);
-    return 12.6f + 0.22f * px * ce + 0.41f * opx * ce + 0.78f * opx * g[2].K + 0.198f * mac_e + 0.194f * mac_p;
+    const float sum = g[1].sh == 1 && g[0].C == g[2].K ? opx * g[2].K : 0.f;  // (most such blocks have a shortcut)
+    return k.three[0] + k.three[1] * px * ce + k.three[2] * opx * ce + k.three[3] * opx * g[2].K + k.three[4] * mac_e + k.three[5] * mac_p +
+           k.three[6] * sum;
 }
-static float block_cost_pair(const ConvGeom g[3]) {
+static float block_cost_pair(const BlockCost& k, const ConvGeom g[3]) {
     float rows;  // of the busiest SIMD
     xdw_strip_rows(g[1], &rows);
     const float opx = (float)g[2].N * g[2].OH * g[2].OW * 1e-6f, groups = (float)xdw_pixel_groups(g[0].W);
     const float mac_p = opx * igemm_channel_groups(g[2].C) * (float)((g[2].K + 31) / 32 * 32);
-    return 8.6f + 0.01f * rows * (1.43f + groups * (g[0].C > 32 ? 0.43f : 0.2f)) + 0.44f * opx * g[2].C + 0.2f * opx * g[2].K +
-           0.433f * mac_p;
+    return k.pair[0] + 0.01f * rows * (k.pair[1] + groups * (g[0].C > 32 ? k.pair[3] : k.pair[2])) + k.pair[4] * opx * g[2].C +
+           k.pair[5] * opx * g[2].K + k.pair[6] * mac_p;
 }
-static float block_cost_single(const ConvGeom g[3], const int plan[6]) {
+static float block_cost_single(const BlockCost& k, const ConvGeom g[3], const int plan[6]) {
     const int rb = plan[0], sl = plan[2], split = plan[4], W = g[0].W;
     const long wgs = (long)g[0].N * plan[1] * split;
     // one workgroup per compute unit, or two that hide part of each other
@@ -1211,14 +1224,13 @@ static float block_cost_single(const ConvGeom g[3], const int plan[6]) {
     const float slices = (float)(((g[0].K + sl - 1) / sl + split - 1) / split);
     const float tiles_e = (float)((std::min(rb + 2, g[0].H) * W + 15) / 16) * sl * 1e-3f;
     const float items = (float)((g[2].K + 31) / 32 * ((rb * W + 15) / 16));
-    return 3.56f + rounds * (slices * (1.59f + tiles_e * (1.39f + 0.3f * igemm_channel_groups(g[0].C))) + 0.096f * items) +
-           (split > 1 ? 1.f + 0.056f * items * split : 0.f);
+    return k.single[0] + rounds * (slices * (k.single[1] + tiles_e * (k.single[2] + k.single[3] * igemm_channel_groups(g[0].C))) + k.single[4] * items) +
+           (split > 1 ? k.single[5] + k.single[6] * items * split : 0.f);
 }
 
-// What a stride-1 block of 64 input channels or more has to gain where its three launches are launch latency throughout: such a
-// block of the dispatch's test stays three launches at a small batch (64 -> 384 -> 64 @14x14 b4: 11.3 us, 8.8 as one). Over
-// the drawn blocks the choice costs 2 % against the best form with it, 0.9 % without.
-static float block_margin(const ConvGeom g[3], float us) { return g[0].C >= 64 && block_cost_three(g) < 14.f ? us : 0.f; }
+// What a stride-1 block of 64 input channels or more has to gain over its three launches where those are launch latency throughout:
+// such a block of the dispatch's test stays three launches at a small batch (64 -> 384 -> 64 @14x14 b4).
+static float block_margin(const ConvGeom g[3], float us) { return g[0].C >= 64 && block_cost_three(kBlockCostSingle, g) < 14.f ? us : 0.f; }
 
 // The first two layers of a block as one launch (conv_xdw.hip), the last by itself. 0: where the cost models say so; 1: wherever
 // the kernel takes the shapes; -1: never. 1 and -1 come before the models' choice of the single launch, not before a forced one.
@@ -1232,27 +1244,44 @@ static bool block_pair_takes(const otter_hip_conv_t* e, const otter_hip_conv_t* 
     return g[0].C <= 32 || g[0].W <= 64;  // (the other instances of the kernel do not fit the register file)
 }
 
-static bool block_single_launch(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
-                                const ConvGeom g[3], int out_layout, int plan[6]) {
+static bool block_single_takes(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p, const ConvGeom g[3],
+                               int out_layout, int plan[6]) {
     if (g_block_always == 2) return false;  // (tuning hook: never)
     if (!e->w_igemm || e->c_pad || e->force_tm || !e->blk_consts || !d->depthwise || !d->blk_consts || d->c_pad || d->force_tm || !p->w_igemm ||
-        p->c_pad || p->force_tm)
+        p->c_pad || p->force_tm || p->d.out_channels % 8)
         return false;
     const Epilogue e1 = make_epilogue(e, OTTER_HIP_I8_P8), e2 = make_epilogue(d, OTTER_HIP_I8_P8), e3 = make_epilogue(p, out_layout);
-    if (!conv_block_applicable(g[0], e1, g[1], e2, g[2], e3)) return false;
-    if (!conv_block_plan(g[0], g[2], e->block_rb, e->block_sl, e->block_split, plan)) return false;
-    if (g_block_always == 1 || e->block_rb || e->block_sl || e->block_split) return true;
-    if (g_block_pair < 0 || (g_block_pair > 0 && block_pair_takes(e, d, g))) return false;
-    const float single = block_cost_single(g, plan);
-    return single < block_cost_three(g) - block_margin(g, 3.8f) && (!block_pair_takes(e, d, g) || single < block_cost_pair(g));
+    return conv_block_applicable(g[0], e1, g[1], e2, g[2], e3) && conv_block_plan(g[0], g[2], e->block_rb, e->block_sl, e->block_split, plan);
 }
+
+static bool block_single_forced(const otter_hip_conv_t* e) { return g_block_always == 1 || e->block_rb || e->block_sl || e->block_split; }
+
+static bool block_single_launch(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
+                                const ConvGeom g[3], int out_layout, int plan[6]) {
+    if (!block_single_takes(e, d, p, g, out_layout, plan)) return false;
+    if (block_single_forced(e)) return true;
+    if (g_block_pair < 0 || (g_block_pair > 0 && block_pair_takes(e, d, g))) return false;
+    const BlockCost& k = kBlockCostSingle;
+    const float single = block_cost_single(k, g, plan);
+    return single < block_cost_three(k, g) - block_margin(g, 3.8f) && (!block_pair_takes(e, d, g) || single < block_cost_pair(k, g));
+}
+
+static bool block_pair_faster(const ConvGeom g[3]) { return block_cost_pair(kBlockCost, g) < block_cost_three(kBlockCost, g); }
 
 static bool block_pair_launch(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const ConvGeom g[3]) {
     if (g_block_pair < 0 || !block_pair_takes(e, d, g)) return false;
-    // (10 %: inside a network each of three launches starts on a blob that the last one has just written, which the calls that
-    // were fitted do not show: 96 -> 576 @14x14 stride 2 b64, first two layers, 13.2 us as one launch there, 15 as two)
-    const float three = block_cost_three(g);
-    return g_block_pair > 0 || block_cost_pair(g) < (g[1].sh == 2 ? 1.1f * three : three - block_margin(g, 2.8f));
+    return g_block_pair > 0 || (block_pair_faster(g) && (g[1].sh == 2 || block_margin(g, 1.f) == 0.f));
+}
+
+// the fastest of the three forms by the newer constants; what the hooks force comes first
+static int block_fastest(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p, const ConvGeom g[3],
+                         int out_layout, int plan[6]) {
+    const bool single = block_single_takes(e, d, p, g, out_layout, plan);
+    if (single && block_single_forced(e)) return 1;
+    const int others = g_block_pair >= 0 && block_pair_takes(e, d, g) && (g_block_pair > 0 || block_pair_faster(g)) ? 2 : 3;
+    if (!single || g_block_pair < 0 || (g_block_pair > 0 && others == 2)) return others;
+    const float t = others == 2 ? block_cost_pair(kBlockCost, g) : block_cost_three(kBlockCost, g);
+    return block_cost_single(kBlockCost, g, plan) < t ? 1 : others;
 }
 
 static int block_default_out_layout(const otter_hip_conv_t* p) {
@@ -1266,8 +1295,17 @@ int otter_hip_conv_block_launches(const otter_hip_conv_t* e, const otter_hip_con
     ConvGeom g[3];
     if (!block_geoms(e, d, p, n, in_h, in_w, g)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_block_launches: empty output");
     int plan[6];
-    if (n >= 1 && p->d.out_channels % 8 == 0 && block_single_launch(e, d, p, g, block_default_out_layout(p), plan)) return 1;
+    if (n >= 1 && block_single_launch(e, d, p, g, block_default_out_layout(p), plan)) return 1;
     return n >= 1 && block_pair_launch(e, d, g) ? 2 : 3;
+}
+
+int otter_hip_conv_block_fastest(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p, int n, int in_h, int in_w) {
+    int rc = block_check(e, d, p, n, in_h, in_w, "otter_hip_conv_block_fastest");
+    if (rc) return rc;
+    ConvGeom g[3];
+    if (!block_geoms(e, d, p, n, in_h, in_w, g)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_block_fastest: empty output");
+    int plan[6];
+    return n >= 1 ? block_fastest(e, d, p, g, block_default_out_layout(p), plan) : 3;
 }
 
 // the two blobs between the launches of a block that is not one
@@ -1283,8 +1321,18 @@ size_t otter_hip_conv_block_layout_workspace_bytes(const otter_hip_conv_t* e, co
     ConvGeom g[3];
     if (!block_geoms(e, d, p, n, in_h, in_w, g)) return 0;
     int plan[6];
-    if (p->d.out_channels % 8 == 0 && out_layout == block_default_out_layout(p) && block_single_launch(e, d, p, g, out_layout, plan))
+    if (out_layout == block_default_out_layout(p) && block_single_launch(e, d, p, g, out_layout, plan))
         return (size_t)plan[5] * sizeof(int);  // the accumulators of a band's workgroups, when there are several
+    return block_blob_bytes(g, nullptr);
+}
+
+size_t otter_hip_conv_block_form_workspace_bytes(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p, int form,
+                                                 int n, int in_h, int in_w) {
+    if (!e || !d || !p || n < 1 || in_h < 1 || in_w < 1) return 0;
+    ConvGeom g[3];
+    if (!block_geoms(e, d, p, n, in_h, in_w, g)) return 0;
+    int plan[6];
+    if (form == 1) return block_single_takes(e, d, p, g, block_default_out_layout(p), plan) ? (size_t)plan[5] * sizeof(int) : 0;
     return block_blob_bytes(g, nullptr);
 }
 
@@ -1334,7 +1382,8 @@ int otter_hip_conv_block_set_plan(otter_hip_conv_t* e, int rows_per_band, int sl
     return OTTER_HIP_OK;
 }
 
-int otter_hip_conv_block_forward(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
+// form: 1, 2 or 3 launches; 0 = as otter_hip_conv_block_launches says
+static int block_forward(int form, const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
                                  const void* in, int n, int in_h, int in_w, const float* residual, void* out, int out_layout,
                                  void* out_q, float q_scale, int q_round_mode, void* workspace, size_t workspace_bytes,
                                  void* stream_) {
@@ -1360,7 +1409,12 @@ int otter_hip_conv_block_forward(const otter_hip_conv_t* e, const otter_hip_conv
     hipStream_t stream = (hipStream_t)stream_;
 
     int plan[6];
-    if (p->d.out_channels % 8 == 0 && out_layout == block_default_out_layout(p) && block_single_launch(e, d, p, g, out_layout, plan)) {
+    const bool single = out_layout == block_default_out_layout(p) &&
+                        (form == 0 ? block_single_launch(e, d, p, g, out_layout, plan) : form == 1 && block_single_takes(e, d, p, g, out_layout, plan));
+    const bool pair = form == 0 ? block_pair_launch(e, d, g) : form == 2 && block_pair_takes(e, d, g);
+    if ((form == 1 && !single) || (form == 2 && !pair))
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_block_forward_form: the block does not run in this form");
+    if (single) {
         const size_t need1 = (size_t)plan[5] * sizeof(int);
         if (need1 && (!workspace || workspace_bytes < need1))
             return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_block_forward: needs the workspace reported by "
@@ -1382,7 +1436,7 @@ int otter_hip_conv_block_forward(const otter_hip_conv_t* e, const otter_hip_conv
                                            "otter_hip_conv_block_workspace_bytes");
     void* t0 = workspace;
     void* t1 = (char*)workspace + second;
-    if (block_pair_launch(e, d, g)) {
+    if (pair) {
         // the pointwise layer and its depthwise reader in one launch: the expanded blob is not made
         const Epilogue e1 = make_epilogue(e, OTTER_HIP_I8_P8), e2 = make_epilogue(d, OTTER_HIP_I8_P8);
         OHIP_CHECK(run_conv_xdw((const int8_t*)in, e->w_xdw, d->w_dw_mfma, t1, g[0], e1, g[1], e2, dw_mfma_epilogue(e2, g[1].K),
@@ -1395,6 +1449,21 @@ int otter_hip_conv_block_forward(const otter_hip_conv_t* e, const otter_hip_conv
     }
     return conv_forward(p, t1, OTTER_HIP_I8_P8, n, g[2].H, g[2].W, out, out_layout, nullptr, 0, stream_, (int8_t*)out_q, q_scale,
                         q_round_mode, residual);
+}
+
+int otter_hip_conv_block_forward(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,
+                                 const void* in, int n, int in_h, int in_w, const float* residual, void* out, int out_layout,
+                                 void* out_q, float q_scale, int q_round_mode, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+    return block_forward(0, e, d, p, in, n, in_h, in_w, residual, out, out_layout, out_q, q_scale, q_round_mode, workspace, workspace_bytes, stream);
+}
+
+int otter_hip_conv_block_forward_form(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p, int form,
+                                      const void* in, int n, int in_h, int in_w, const float* residual, void* out, int out_layout,
+                                      void* out_q, float q_scale, int q_round_mode, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+    if (form < 1 || form > 3) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_block_forward_form: 1, 2 or 3 launches");
+    return block_forward(form, e, d, p, in, n, in_h, in_w, residual, out, out_layout, out_q, q_scale, q_round_mode, workspace, workspace_bytes, stream);
 }
 
 // -----------------------------------------------------------------------------------------------------

@@ -880,7 +880,7 @@ int ConvolutionLayer::forward_shuffle(const Tensor& bottom_in, const Tensor& oth
 
 int ConvolutionLayer::block_launches(const ConvolutionLayer* e, const ConvolutionLayer* d, const ConvolutionLayer* p, int n, int h,
                                      int w) {
-    return e->handle_ && d->handle_ && p->handle_ ? otter_hip_conv_block_launches(e->handle_, d->handle_, p->handle_, n, h, w) : 3;
+    return e->handle_ && d->handle_ && p->handle_ ? otter_hip_conv_block_fastest(e->handle_, d->handle_, p->handle_, n, h, w) : 3;
 }
 
 static std::atomic<long> g_chain_forwards{0};
@@ -934,10 +934,9 @@ int ConvolutionLayer::forward_block(const ConvolutionLayer* e, const Convolution
     if (e->force_out_layout >= 0 || d->force_out_layout >= 0 || p->force_out_layout >= 0) return 1;
     const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3);
     if (bottom.channels() != e->in_channels || p->out_channels % 8) return 1;
-    {  // one launch for the block, or one for its first two layers and one for the last; three are the layers one by one
-        const int launches = otter_hip_conv_block_launches(e->handle_, d->handle_, p->handle_, N, H, W);
-        if (launches != 1 && launches != 2) return 1;
-    }
+    // one launch for the block, or one for its first two layers and one for the last; three are the layers one by one
+    const int form = otter_hip_conv_block_fastest(e->handle_, d->handle_, p->handle_, N, H, W);
+    if (form != 1 && form != 2) return 1;
     int oh = H, ow = W;
     for (const ConvolutionLayer* c : {e, d, p}) {
         int h2 = 0, w2 = 0;
@@ -957,14 +956,13 @@ int ConvolutionLayer::forward_block(const ConvolutionLayer* e, const Convolution
         Tensor q;
         if (with_q) q = Tensor::empty_device({N, p->out_channels / 8, oh, ow}, ScalarType::Byte8);
         const int out_layout = f32 ? OTTER_HIP_F32_P4 : OTTER_HIP_I8_P8;
-        const size_t ws_bytes =
-            otter_hip_conv_block_layout_workspace_bytes(e->handle_, d->handle_, p->handle_, out_layout, N, H, W);
+        const size_t ws_bytes = otter_hip_conv_block_form_workspace_bytes(e->handle_, d->handle_, p->handle_, form, N, H, W);
         Tensor ws;
         if (ws_bytes) ws = Tensor::empty_device({(int64_t)ws_bytes}, ScalarType::Byte);
-        const int rc = otter_hip_conv_block_forward(e->handle_, d->handle_, p->handle_, bottom.device_ptr(), N, H, W,
-                                                    shortcut ? (const float*)shortcut->device_ptr() : nullptr, top.device_ptr(),
-                                                    out_layout, with_q ? q.device_ptr() : nullptr,
-                                                    q_scale, q_round, ws_bytes ? ws.device_ptr() : nullptr, ws_bytes, nullptr);
+        const int rc = otter_hip_conv_block_forward_form(e->handle_, d->handle_, p->handle_, form, bottom.device_ptr(), N, H, W,
+                                                         shortcut ? (const float*)shortcut->device_ptr() : nullptr, top.device_ptr(),
+                                                         out_layout, with_q ? q.device_ptr() : nullptr,
+                                                         q_scale, q_round, ws_bytes ? ws.device_ptr() : nullptr, ws_bytes, nullptr);
         if (rc) return rc;
         top.mark_device_written();
         if (with_q) {

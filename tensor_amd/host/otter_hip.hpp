@@ -253,7 +253,7 @@ public:
     // forward_residual where the shortcut is the concatenation of two blobs (otter_hip_conv_forward_residual_concat)
     int forward_residual_concat(const Tensor& bottom_blob, const Tensor& part0, const Tensor& part1, float q_scale, int q_round,
                                 Tensor& sum, const NetOption& opt, bool int8_only) const;
-    // what otter_hip_conv_block_launches says of the three layers on an input of this size
+    // what otter_hip_conv_block_fastest says of the three layers on an input of this size
     static int block_launches(const ConvolutionLayer* expand, const ConvolutionLayer* depthwise, const ConvolutionLayer* project,
                               int n, int h, int w);
     // A run of int8 -> int8 convolution layers, each reading the one before, as one call of the C ABI's chain entry point
