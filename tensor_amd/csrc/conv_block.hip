@@ -628,7 +628,7 @@ static unsigned* g_counter_ptr[64] = {};
 static unsigned g_counter_next[64][2] = {};
 
 __global__ void blk_zero_counters_kernel(unsigned* p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = 0u;
 }
 

@@ -17,6 +17,23 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t dw_rsrc(const void* p, unsigne
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
 }
 
+// The workgroups of a launch over strips (x) and planes (y): consecutive strips of a plane and consecutive planes on one XCD, which
+// workgroups go to round-robin in launch order. Divisions as multiplications (some 40 scalar instructions each otherwise), and no
+// use of gridDim or blockDim: those bring 256 bytes of hidden launch arguments along, 0.3 us of the host's time per launch.
+struct DwGrid {
+    FastDiv gx, planes;  // workgroups along x, planes per image
+    unsigned total;
+    int wpb;             // strips of a workgroup
+    static DwGrid of(unsigned gx, unsigned gy, unsigned planes, int wpb) { return {fast_div(gx), fast_div(planes), gx * gy, wpb}; }
+    __device__ __forceinline__ void locate(unsigned* bx, unsigned* plane, unsigned* img) const {
+        unsigned w = blockIdx.y * gx.d + blockIdx.x;
+        const unsigned per = total / 8;
+        if (w < per * 8) w = (w % 8) * per + w / 8;
+        const unsigned by = div_by(w, gx);
+        *bx = w - by * gx.d, *img = div_by(by, planes), *plane = by - *img * planes.d;
+    }
+};
+
 // Requantize four accumulators into four saturated bytes of one dword.
 // The activation clamp [0, hi] is applied AFTER scaling and rounding, on the packed int16 values, instead of on the
 // float before them: x -> trunc(fl(fl(x * so) + half)) is monotone for so > 0, so clamping its argument to [0, hi]

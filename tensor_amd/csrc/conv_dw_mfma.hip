@@ -73,12 +73,24 @@ __device__ __forceinline__ v4i dw_dequant4(const Epilogue& ep, const v4i& acc, c
     return res;
 }
 
-// What a launch is cut into, and the divisions of its indices (a division by a kernel argument is some 40 scalar instructions, and
-// a short strip's wave issues few others).
-struct DwPlan {
-    FastDiv gx, c8, chunks, lpi;  // by the workgroups along x, the octets, the column chunks of a row, the lane columns of an image
-    int rps, ipw;                 // output rows of a strip, images of a wave
+// What the kernel reads of a layer and what its launch is cut into, with the divisions of its indices (a division by a kernel
+// argument is some 40 scalar instructions, and a short strip's wave issues few others). 152 bytes, where ConvGeom and Epilogue
+// made 268: the host writes launch arguments to device memory one by one (3.85 us a launch with 180 bytes, 3.35 with 96).
+struct DwArgs {
+    const float *scale_in, *bias, *scale_out;
+    unsigned gx_m, gx, c8_m, chunks_m, chunks;  // divisions (FastDiv) by the workgroups along x, the octets, the column chunks of a row
+    int N, H, W, OH, OW, rps;           // rps: output rows of a strip
     unsigned total, in_bytes, out_bytes;
+    float p0, lo, hi, half;             // LeakyReLU slope, clamp of an fp32 result, rounding constant
+    unsigned short c8, lpi_m;           // octets; 1 / lane columns of an image, for lanes below 16 (16.8 fixed point)
+    unsigned char gx_s, c8_s, chunks_s, lpi, ipw, ph, lrelu;  // ipw: images of a wave
+
+    __device__ Epilogue epilogue() const {
+        Epilogue ep{};
+        ep.scale_in = scale_in, ep.bias = bias, ep.scale_out = scale_out;
+        ep.act_p0 = p0, ep.act_lo = lo, ep.act_hi = hi, ep.round_half = half, ep.lrelu = lrelu != 0;
+        return ep;
+    }
 };
 
 // A wave owns one channel octet x 16 lane columns (64 output pixels of a row at stride 1, 32 at stride 2) and walks
@@ -87,25 +99,27 @@ struct DwPlan {
 // the matrix instructions for the whole walk. Narrow images sit side by side in the wave (`lpi` lane columns each).
 template <int S, int EPI, bool ODDW, int KS>
 __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wa,
-                                                              void* __restrict__ out, ConvGeom g, Epilogue ep, DwPlan pl) {
+                                                              void* __restrict__ out, DwArgs g) {
     constexpr int RING = 8, U = RING / S;  // U output rows per step
     constexpr int PH = 4 / S;              // output pixels per lane column
     constexpr int T = S == 1 ? 2 : 1;      // A sets
-    const int C8 = (int)pl.c8.d, ipw = pl.ipw, rps = pl.rps;
+    const Epilogue ep = g.epilogue();
+    const int C8 = g.c8, ipw = g.ipw, rps = g.rps;
     // Workgroups go to the 8 XCDs round-robin in launch order. Work items that share input cache lines - the column
     // chunks of a row (a 128-byte line straddles the chunk border), the strip groups of a plane (halo rows), the
     // octets of an image - get consecutive indices on ONE XCD, so that a shared line comes from memory once.
-    unsigned w = blockIdx.y * pl.gx.d + blockIdx.x;
-    const unsigned per = pl.total / 8;
+    unsigned w = blockIdx.y * g.gx + blockIdx.x;
+    const unsigned per = g.total / 8;
     if (w < per * 8) w = (w % 8) * per + w / 8;
-    const unsigned by = div_by(w, pl.gx), bx = w - by * pl.gx.d, img = div_by(by, pl.c8), sg = div_by(bx, pl.chunks);
-    const int o = (int)(by - img * pl.c8.d), n0 = (int)img * ipw, chunk = (int)(bx - sg * pl.chunks.d);
+    const unsigned by = div_by(w, FastDiv{g.gx_m, g.gx_s, g.gx}), bx = w - by * g.gx;
+    const unsigned img = div_by(by, FastDiv{g.c8_m, g.c8_s, g.c8}), sg = div_by(bx, FastDiv{g.chunks_m, g.chunks_s, g.chunks});
+    const int o = (int)(by - img * (unsigned)C8), n0 = (int)img * ipw, chunk = (int)(bx - sg * g.chunks);
     const int strip = (int)sg;
     const int lane = threadIdx.x, n = lane & 15, q = lane >> 4;
     int di = 0, nl = chunk * 16 + n;  // image within the wave, lane column within the image
     if (ipw > 1) {
-        di = (int)div_by((unsigned)n, pl.lpi);
-        nl = n - di * (int)pl.lpi.d;
+        di = n * g.lpi_m >> 8;
+        nl = n - di * g.lpi;
     }
     const bool lane_ok = di < ipw && n0 + di < g.N;
 
@@ -133,7 +147,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
     auto load_row = [&](int j) -> v4i {
         const int iy = iy0 + j;
         const bool ok = (unsigned)iy < row_end;  // wave-uniform
-        const __amdgpu_buffer_rsrc_t r = dw_rsrc(x, ok ? pl.in_bytes : 0u);
+        const __amdgpu_buffer_rsrc_t r = dw_rsrc(x, ok ? g.in_bytes : 0u);
         const unsigned s_row = ok ? s_in + (unsigned)(iy * g.W * 8) : 0u;
         if constexpr (ODDW) {  // odd width: a row ends on half a pair, which is loaded as 8 bytes + zero
             const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v_in, (int)s_row, 0));
@@ -175,9 +189,9 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
     const bool st_ok = lane_ok && ox < g.OW;
     unsigned v_out, s_out, row_bytes;
     if constexpr (EPI == EPI_F32_P4) {  // Float4: [N][C/4][OH*OW][4 floats]; packs 2o and 2o+1
-        v_out = st_ok ? ((unsigned)di * (unsigned)(g.C / 4) + (S == 1 ? 0u : (unsigned)(q & 1))) * OHW * 16u + (unsigned)ox * 16u
+        v_out = st_ok ? ((unsigned)di * (unsigned)(2 * C8) + (S == 1 ? 0u : (unsigned)(q & 1))) * OHW * 16u + (unsigned)ox * 16u
                       : DW_OOB;
-        s_out = (unsigned)(n0 * (g.C / 4) + 2 * o) * OHW * 16u;
+        s_out = (unsigned)(n0 * (2 * C8) + 2 * o) * OHW * 16u;
         row_bytes = (unsigned)g.OW * 16u;
     } else if constexpr (EPI == EPI_F32_P8) {  // Float8: [N][C/8][OH*OW][8 floats]; a lane's sets are the pixel's halves
         v_out = st_ok ? (unsigned)di * (unsigned)C8 * OHW * 32u + (unsigned)ox * 32u + (S == 1 ? 0u : (unsigned)(q & 1) * 16u)
@@ -190,7 +204,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
         s_out = (unsigned)(n0 * C8 + o) * OHW * 8u;
         row_bytes = (unsigned)g.OW * 8u;
     }
-    const __amdgpu_buffer_rsrc_t rout = dw_rsrc(out, pl.out_bytes);
+    const __amdgpu_buffer_rsrc_t rout = dw_rsrc(out, g.out_bytes);
 
     // Software pipeline, one output row deep: a step issues the matrix instructions of row r+1, refills the ring slots
     // they free, and then runs the epilogue of row r while those instructions execute. The scheduling barriers keep
@@ -253,7 +267,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
     // behind a return between the rows the compiler moves the loads down to their first use, a row's latency each.
     // loads of rows [RING, in_rows_ok) stay inside the image (iy0 + RING > 0); the few an interior step fetches past
     // the strip's own last row are rows the next strip reads anyway
-    const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, pl.in_bytes);
+    const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, g.in_bytes);
     const int in_rows_ok = g.H - iy0;
     const unsigned in_row_bytes = (unsigned)(g.W * 8);
     // (two loops and not one with two paths: a ring slot that either path may refill is refilled elsewhere and copied at the end of a
@@ -323,7 +337,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
 template <int S, int EPI, int NL>
 __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* __restrict__ x, const int8_t* __restrict__ wa,
                                                                void* __restrict__ out, ConvGeom g, Epilogue ep,
-                                                               const float* __restrict__ in_scale_p, float in_half,
+                                                               const float* __restrict__ in_scale_p, float in_half, DwGrid dg,
                                                                int n_strips, int rps, unsigned in_bytes, unsigned out_bytes) {
     constexpr int RL = 4, PF = 4;      // LDS lines / register stages per wave
     constexpr int NCH = (NL + 1) / 2;  // column chunks of 64 pixels (a matrix operand covers 4 x 16 of them)
@@ -333,17 +347,11 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
     constexpr int LINE = (64 * NCH + 8) * 8;
     __shared__ __attribute__((aligned(16))) int8_t lds_all[4][RL][LINE];
     const int C8 = g.C / 8;
-    unsigned bx = blockIdx.x, by = blockIdx.y;
-    {  // consecutive strips of a plane and consecutive planes on one XCD (see conv_dw3x3_mfma_kernel)
-        const unsigned id = by * gridDim.x + bx, total = gridDim.x * gridDim.y, per = total / 8;
-        if (id < per * 8) {
-            const unsigned w = (id % 8) * per + id / 8;
-            bx = w % gridDim.x, by = w / gridDim.x;
-        }
-    }
-    const int o = by % C8, img = by / C8;
+    unsigned bx, o_u, img_u;
+    dg.locate(&bx, &o_u, &img_u);
+    const int o = (int)o_u, img = (int)img_u;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int strip = __builtin_amdgcn_readfirstlane(bx * (blockDim.x >> 6) + wave);
+    const int strip = __builtin_amdgcn_readfirstlane(bx * dg.wpb + wave);
     if (strip >= n_strips) return;  // whole wave
     const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
     int8_t* const lds = &lds_all[wave][0][0];
@@ -589,7 +597,7 @@ hipError_t run_conv_dw_f32in(const float* x, const int8_t* wa, void* out, const 
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW * (epi == EPI_F32_P4 || epi == EPI_F32_P8 ? 4 : 1));
 #define OHIP_DWF_L(S_, E_, L_)                                                                                           \
     hipLaunchKernelGGL((conv_dw3x3_f32in_kernel<S_, E_, L_>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
-                       n_strips, rps, in_bytes, out_bytes)
+                       DwGrid::of(grid.x, grid.y, (unsigned)C8, wpb), n_strips, rps, in_bytes, out_bytes)
 #define OHIP_DWF_N(S_, E_)                       \
     do {                                         \
         switch ((g.W + 31) / 32) {               \
@@ -683,14 +691,21 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     const dim3 grid((unsigned)(col_chunks * n_strips), (unsigned)groups), block(64);
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW * (epi == EPI_F32_P4 || epi == EPI_F32_P8 ? 4 : 1));
-    const DwPlan pl = {fast_div(grid.x), fast_div((unsigned)C8), fast_div((unsigned)col_chunks), fast_div((unsigned)lpi),
-                       rps, ipw, grid.x * grid.y, in_bytes, out_bytes};
+    const FastDiv gx = fast_div(grid.x), c8 = fast_div((unsigned)C8), ch = fast_div((unsigned)col_chunks);
+    DwArgs pl{};
+    pl.scale_in = ep.scale_in, pl.bias = ep.bias, pl.scale_out = ep.scale_out;
+    pl.gx_m = gx.m, pl.gx_s = (unsigned char)gx.s, pl.gx = grid.x, pl.c8_m = c8.m, pl.c8_s = (unsigned char)c8.s, pl.c8 = (unsigned short)C8;
+    pl.chunks_m = ch.m, pl.chunks_s = (unsigned char)ch.s, pl.chunks = (unsigned)col_chunks;
+    pl.lpi = (unsigned char)lpi, pl.lpi_m = (unsigned short)(256 / lpi + 1), pl.ipw = (unsigned char)ipw;
+    pl.N = g.N, pl.H = g.H, pl.W = g.W, pl.OH = g.OH, pl.OW = g.OW, pl.ph = (unsigned char)g.ph, pl.rps = rps;
+    pl.total = grid.x * grid.y, pl.in_bytes = in_bytes, pl.out_bytes = out_bytes;
+    pl.p0 = ep.act_p0, pl.lo = ep.act_lo, pl.hi = ep.act_hi, pl.half = ep.round_half, pl.lrelu = ep.lrelu;
 #define OHIP_DWM_K(S_, E_, O_)                                                                                         \
     do {                                                                                                               \
         if (g.kh == 3)                                                                                                 \
-            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 3>), grid, block, 0, stream, x, wa, out, g, ep, pl); \
+            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 3>), grid, block, 0, stream, x, wa, out, pl); \
         else                                                                                                           \
-            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 5>), grid, block, 0, stream, x, wa, out, g, ep, pl); \
+            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 5>), grid, block, 0, stream, x, wa, out, pl); \
     } while (0)
 #define OHIP_DWM(S_, E_) \
     do {                                                                                                               \

@@ -26,13 +26,82 @@ namespace {
 
 constexpr unsigned PR_OOB = 0x80000000u;  // past any buffer here: a load returns zero, a store is dropped
 
+// What these kernels read of a layer. Launch arguments are written to device memory one by one: on the host a launch with 32 bytes
+// of them takes 3.1 us, with 96 3.35, with 180 (ConvGeom and Epilogue as they are) 3.85, and such a layer's kernel is done in less.
 struct PwRegArgs {
-    FastDiv hw;
-    int C8, K, HW, tiles, per, mt;  // tiles: workgroups along the pixels; mt: 16-row tiles of the packed weights per step
-    unsigned total_pix, in_bytes;
-    float so;     // the output scale of every channel
-    unsigned qh;  // upper clamp of the rounded result, in both halves (EPI_I8_P8_NONNEG)
+    const float *scale_in, *bias;
+    unsigned hw_m, total_pix;    // hw_m, hw_s: division by HW (FastDiv)
+    int HW, K, tiles, per, mt;   // tiles: workgroups along the pixels; mt: 16-row tiles of the packed weights per step
+    unsigned short C8;
+    unsigned char hw_s, lrelu;
+    float p0;                    // slope of LeakyReLU
+    float scale, half;           // int8 result: the output scale of every channel, the rounding constant; fp32: act_lo, act_hi
+    unsigned qh;                 // upper clamp of the rounded result, in both halves (EPI_I8_P8_NONNEG)
+
+    __device__ FastDiv hw() const { return {hw_m, hw_s, (unsigned)HW}; }
 };
+// the rest of an epilogue that needs more
+struct PwFused {
+    const float* residual;
+    int8_t* twin;
+    float twin_scale, twin_half;
+    static PwFused of(const Epilogue& ep) { return {ep.residual, ep.twin, ep.twin_scale, ep.twin_half}; }
+};
+struct PwParts : PwFused {  // JoinArgs::residual1 and the like
+    const float* residual1;
+    int split;
+    short pack0, pack1;
+    static PwParts of(const Epilogue& ep) {
+        return {PwFused::of(ep), ep.join->residual1, ep.join->res_split, (short)ep.join->res_pack0, (short)ep.join->res_pack1};
+    }
+    __device__ JoinArgs join() const {
+        JoinArgs ja{};
+        ja.residual1 = residual1, ja.res_split = split, ja.res_pack0 = pack0, ja.res_pack1 = pack1;
+        return ja;
+    }
+};
+struct PwShuffle {  // JoinArgs::other and the like
+    const float* other;
+    float *sh_out0, *sh_out1;
+    int8_t *sh_q0, *sh_q1;
+    float twin_scale, twin_half;
+    unsigned sh_image;
+    short other_pack, other_odd;
+    static PwShuffle of(const Epilogue& ep) {
+        const JoinArgs& j = *ep.join;
+        return {j.other, j.sh_out0, j.sh_out1, j.sh_q0, j.sh_q1, ep.twin_scale, ep.twin_half, (unsigned)j.sh_image, (short)j.other_pack, (short)j.other_odd};
+    }
+};
+template <int EPI>
+struct PwAddOf {
+    using Type = NoJoin;
+};
+template <>
+struct PwAddOf<EPI_F32_P4_FUSED> {
+    using Type = PwFused;
+};
+template <>
+struct PwAddOf<EPI_F32_SHUFFLE> {
+    using Type = PwShuffle;
+};
+template <>
+struct PwAddOf<EPI_F32_P4_PARTS> {
+    using Type = PwParts;
+};
+template <int EPI>
+using PwAdd = typename PwAddOf<EPI>::Type;
+
+template <int EPI>
+__device__ __forceinline__ Epilogue pw_epilogue(const PwRegArgs& pa, const PwAdd<EPI>& ja) {
+    constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG;
+    Epilogue ep{};
+    ep.lrelu = pa.lrelu != 0, ep.act_p0 = pa.p0;
+    if (I8) ep.round_half = pa.half;
+    else ep.act_lo = pa.scale, ep.act_hi = pa.half;
+    if constexpr (!I8 && EPI != EPI_F32_P4) ep.twin_scale = ja.twin_scale, ep.twin_half = ja.twin_half;
+    if constexpr (EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_P4_PARTS) ep.residual = ja.residual, ep.twin = ja.twin;
+    return ep;
+}
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
@@ -52,10 +121,11 @@ __device__ __forceinline__ void store8(__amdgpu_buffer_rsrc_t r, v2i d, unsigned
 
 template <int FN, int CG, int EPI>
 __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
-                                                          PwRegArgs pa, Epilogue ep, JoinParam<EPI> ja) {
+                                                          PwRegArgs pa, PwAdd<EPI> ja) {
     constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
     constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
     constexpr bool ADD = SHUF || FUSED;  // reads elements of another fp32 blob
+    const Epilogue ep = pw_epilogue<EPI>(pa, ja);
     const unsigned lane = threadIdx.x & 63, q = lane >> 4, p = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int xcd = blockIdx.x & 7, first = xcd * pa.tiles >> 3, tile = first + (int)(blockIdx.x >> 3);  // (grid.x is a multiple of 8)
@@ -67,7 +137,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
 
     // ---- weights and constants of a channel pair -------------------------------------------------------------------------------
     const __amdgpu_buffer_rsrc_t rw = rsrc(wpk, (unsigned)(CG * pa.mt) * 1024u);
-    const __amdgpu_buffer_rsrc_t rsi = rsrc(ep.scale_in, kpad * 4), rbi = rsrc(ep.bias, kpad * 4);
+    const __amdgpu_buffer_rsrc_t rsi = rsrc(pa.scale_in, kpad * 4), rbi = rsrc(pa.bias, kpad * 4);
     v4i a[CG][2];
     auto load_a = [&](int pr) {
 #pragma unroll
@@ -83,7 +153,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
     load_a(pr0);
 
     // ---- the pixels: every channel of them requested now ---------------------------------------------------------------------------
-    const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.in_bytes);
+    const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.total_pix * C8 * 8u);
     unsigned n[FN], pix[FN];
     bool ok[FN];
     v4i b[FN][CG];
@@ -91,7 +161,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
     for (int j = 0; j < FN; ++j) {
         const unsigned gp = gp0 + 16 * j + p;
         ok[j] = gp < pa.total_pix;
-        n[j] = div_by(gp, pa.hw), pix[j] = gp - n[j] * HW;
+        n[j] = div_by(gp, pa.hw()), pix[j] = gp - n[j] * HW;
         const unsigned v = ok[j] ? ((n[j] * C8 + 2 * q) * HW + pix[j]) * 8u : PR_OOB;
 #pragma unroll
         for (int cg = 0; cg < CG; ++cg) {
@@ -133,7 +203,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
                 if (ok[j] && 32u * pr + 8 * q < K)
 #pragma unroll
                     for (int h = 0; h < 2; ++h)
-                        k.add[j][h] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep, ja, n[j], pix[j], (int)(32u * pr + 8 * q + 4 * h), (int)K, (int)HW));
+                        k.add[j][h] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep, ja.join(), n[j], pix[j], (int)(32u * pr + 8 * q + 4 * h), (int)K, (int)HW));
         } else if constexpr (FUSED) {
             if (ep.residual != nullptr) {  // (uniform)
                 const __amdgpu_buffer_rsrc_t r = rsrc(ep.residual, f_bytes);
@@ -155,7 +225,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
         if constexpr (I8) {
             Epi8 prm;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) prm.si[e] = si[e], prm.bi[e] = bi[e], prm.so[e] = pa.so;
+            for (int e = 0; e < 8; ++e) prm.si[e] = si[e], prm.bi[e] = bi[e], prm.so[e] = pa.scale;
 #pragma unroll
             for (int e = 0; e < 4; ++e) prm.qh[e] = pa.qh;
 #pragma unroll
@@ -182,7 +252,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
                             const v4i even = ja.other_odd ? r[h] : o, odd = ja.other_odd ? o : r[h];  // (uniform)
                             const v4i lo = {even[0], odd[0], even[1], odd[1]}, hi = {even[2], odd[2], even[3], odd[3]};
                             const unsigned pack = ch0 / 4 + h - (w ? half : 0u);  // in this half; beyond it on either side: the other half's
-                            const unsigned e = n[j] * (unsigned)ja.sh_image + (pack * HW + pix[j]) * 8u;
+                            const unsigned e = n[j] * ja.sh_image + (pack * HW + pix[j]) * 8u;
                             const bool live = ok[j] && pack < half;  // (a channel past the last one is a pack past the second half)
                             if (f != nullptr) {
                                 const __amdgpu_buffer_rsrc_t rf = rsrc(f, PR_OOB);
@@ -242,11 +312,12 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
 // sums of consecutive pairs lie in two buffers.
 template <int FN, int NS, int EPI>
 __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
-                                                            PwRegArgs pa, Epilogue ep, JoinParam<EPI> ja) {
+                                                            PwRegArgs pa, PwAdd<EPI> ja) {
     constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
     constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
     constexpr int OWN = FN < 2 ? 1 : FN / 2;  // half pairs that a wave finishes (of 2 FN; with FN == 1 waves 0 and 1 have one each)
     __shared__ v4i red[2][2 * FN][3][64];     // [buffer][half pair][the other waves][lane]
+    const Epilogue ep = pw_epilogue<EPI>(pa, ja);
     const unsigned lane = threadIdx.x & 63, q = lane >> 4, p = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int xcd = blockIdx.x & 7, first = xcd * pa.tiles >> 3, tile = first + (int)(blockIdx.x >> 3);  // (grid.x is a multiple of 8)
@@ -255,7 +326,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
     const unsigned HW = pa.HW, K = pa.K, C8 = pa.C8, kpad = (unsigned)pa.mt * 16u, f_bytes = pa.total_pix * K * 4u;
 
     const __amdgpu_buffer_rsrc_t rw = rsrc(wpk, (unsigned)(steps * pa.mt) * 1024u);
-    const __amdgpu_buffer_rsrc_t rsi = rsrc(ep.scale_in, kpad * 4), rbi = rsrc(ep.bias, kpad * 4);
+    const __amdgpu_buffer_rsrc_t rsi = rsrc(pa.scale_in, kpad * 4), rbi = rsrc(pa.bias, kpad * 4);
     v4i a[NS][2];
     auto load_a = [&](int pr) {
 #pragma unroll
@@ -268,7 +339,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
     };
     load_a(pr0);
 
-    const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.in_bytes);
+    const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.total_pix * C8 * 8u);
     unsigned n[FN], pix[FN];
     bool ok[FN];
     v4i b[FN][NS];
@@ -276,7 +347,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
     for (int j = 0; j < FN; ++j) {
         const unsigned gp = (unsigned)tile * (16 * FN) + 16 * j + p;
         ok[j] = gp < pa.total_pix;
-        n[j] = div_by(gp, pa.hw), pix[j] = gp - n[j] * HW;
+        n[j] = div_by(gp, pa.hw()), pix[j] = gp - n[j] * HW;
         const unsigned v = ok[j] ? ((n[j] * C8 + 2 * q) * HW + pix[j]) * 8u : PR_OOB;
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
@@ -319,7 +390,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
                 k.add[o] = load16(rsrc(ja.other, f_bytes), oko[o] && ch < K ? v : PR_OOB, s * HW);
             }
             if constexpr (PARTS) {
-                if (oko[o] && ch < K) k.add[o] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep, ja, no[o], po[o], (int)ch, (int)K, (int)HW));
+                if (oko[o] && ch < K) k.add[o] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep, ja.join(), no[o], po[o], (int)ch, (int)K, (int)HW));
             } else if constexpr (FUSED) {
                 if (ep.residual != nullptr) k.add[o] = load16(rsrc(ep.residual, f_bytes), ch < K ? vo[o] : PR_OOB, s * HW);  // (uniform)
             }
@@ -331,7 +402,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
 #pragma unroll
         for (int o = 0; o < OWN; ++o) {
             if constexpr (I8) {
-                const v4i so = v4i{1, 1, 1, 1} * __float_as_int(pa.so);
+                const v4i so = v4i{1, 1, 1, 1} * __float_as_int(pa.scale);
                 const unsigned w = dw_requant4<NONNEG>(ep, c[o], k.si, k.bi, so, pa.qh, pa.qh);
                 __builtin_amdgcn_raw_buffer_store_b32(w, rout, (int)(ch < K ? vo[o] : PR_OOB), (int)((unsigned)pr * 32u * HW), 0);
                 continue;
@@ -351,7 +422,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
                     float* const f = w ? ja.sh_out1 : ja.sh_out0;
                     int8_t* const b8 = w ? ja.sh_q1 : ja.sh_q0;
                     const unsigned pack = ch / 4 - (w ? half : 0u);  // beyond this half on either side: the other half's
-                    const unsigned e = no[o] * (unsigned)ja.sh_image + (pack * HW + po[o]) * 8u;
+                    const unsigned e = no[o] * ja.sh_image + (pack * HW + po[o]) * 8u;
                     const bool live = oko[o] && pack < half;
                     if (f != nullptr) {
                         const __amdgpu_buffer_rsrc_t rf = rsrc(f, PR_OOB);
@@ -436,8 +507,8 @@ bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep) {
 template <int FN, int CG, int EPI>
 static hipError_t launch_pw_reg(const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
                                 hipStream_t stream) {
-    hipLaunchKernelGGL((conv_pw_reg_kernel<FN, CG, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa, ep,
-                       JoinParam<EPI>::of(ep));
+    hipLaunchKernelGGL((conv_pw_reg_kernel<FN, CG, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa,
+                       PwAdd<EPI>::of(ep));
     return hipGetLastError();
 }
 
@@ -469,8 +540,8 @@ static hipError_t launch_pw_reg_wide(int epi, const int8_t* x, const int8_t* wpk
 template <int FN, int NS, int EPI>
 static hipError_t launch_pw_split(const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
                                   hipStream_t stream) {
-    hipLaunchKernelGGL((conv_pw_split_kernel<FN, NS, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa, ep,
-                       JoinParam<EPI>::of(ep));
+    hipLaunchKernelGGL((conv_pw_split_kernel<FN, NS, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa,
+                       PwAdd<EPI>::of(ep));
     return hipGetLastError();
 }
 
@@ -493,11 +564,14 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
                            hipStream_t stream) {
     if (!conv_pw_reg_applicable(g, ep)) return hipErrorInvalidValue;
     const int epi = pw_reg_epilogue(ep, g.K), steps = igemm_channel_groups(g.C), pairs = (g.K + 31) / 32;
-    PwRegArgs pa;
-    pa.HW = g.H * g.W, pa.hw = fast_div((unsigned)pa.HW), pa.C8 = g.C / 8, pa.K = g.K, pa.mt = igemm_padded_rows(g.K) / 16, pa.so = so, pa.qh = 0;
+    const FastDiv hw = fast_div((unsigned)(g.H * g.W));
+    const bool i8 = epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG;
+    PwRegArgs pa{};
+    pa.scale_in = ep.scale_in, pa.bias = ep.bias, pa.hw_m = hw.m, pa.hw_s = (unsigned char)hw.s, pa.HW = g.H * g.W, pa.K = g.K;
+    pa.total_pix = (unsigned)g.N * (unsigned)pa.HW, pa.C8 = (unsigned short)(g.C / 8), pa.mt = igemm_padded_rows(g.K) / 16;
+    pa.lrelu = ep.lrelu, pa.p0 = ep.act_p0, pa.scale = i8 ? so : ep.act_lo, pa.half = i8 ? ep.round_half : ep.act_hi;
     const float both[2] = {so, so};
     if (epi == EPI_I8_P8_NONNEG) conv_pw_stream_clamps(ep.act_hi, ep.round_half, both, 2, &pa.qh);
-    pa.total_pix = (unsigned)g.N * (unsigned)pa.HW, pa.in_bytes = pa.total_pix * (unsigned)g.C;
     int fn = 1, per = 1;
     const bool split = force ? (force & 64) != 0 : steps > PW_REG_STEPS;
     const bool wide = split || epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG;  // (registers)

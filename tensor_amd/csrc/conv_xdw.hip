@@ -40,7 +40,7 @@ void xdw_pack_weights(const int8_t* w, int Cin, int K, int8_t* dst) {
 template <int S, int EPI, bool XNN, int NG, int CK>
 __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S == 2 && NG <= 4)) ? 3 : 2) conv_xdw_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wx,
                                                        const int8_t* __restrict__ wa, void* __restrict__ out, ConvGeom g, int cin,
-                                                       Epilogue epx, Epilogue ep, int n_strips, int rps, unsigned in_bytes,
+                                                       Epilogue epx, Epilogue ep, DwGrid dg, int n_strips, int rps, unsigned in_bytes,
                                                        unsigned out_bytes) {
     constexpr int RL = 4, PF = 2;      // LDS lines per octet / rows of loads in flight
     constexpr int NCH = (NG + 3) / 4;  // column chunks of 64 pixels of the depthwise operand
@@ -50,18 +50,12 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
     constexpr int LINE = (64 * NCH + 8) * 8;
     constexpr int OCT = RL * LINE + 128;  // the second octet's lines, off the first one's banks
     extern __shared__ __attribute__((aligned(16))) int8_t lds_all[];  // [waves of the workgroup][2 octets][RL lines]
-    const int C8 = g.C / 8, P = g.C / 16;
-    unsigned bx = blockIdx.x, by = blockIdx.y;
-    {  // consecutive strips of a plane and consecutive planes on one XCD (see conv_dw3x3_mfma_kernel)
-        const unsigned id = by * gridDim.x + bx, total = gridDim.x * gridDim.y, per = total / 8;
-        if (id < per * 8) {
-            const unsigned w = (id % 8) * per + id / 8;
-            bx = w % gridDim.x, by = w / gridDim.x;
-        }
-    }
-    const int pr = by % P, img = by / P;
+    const int C8 = g.C / 8;
+    unsigned bx, pr_u, img_u;
+    dg.locate(&bx, &pr_u, &img_u);
+    const int pr = (int)pr_u, img = (int)img_u;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int strip = __builtin_amdgcn_readfirstlane(bx * (blockDim.x >> 6) + wave);
+    const int strip = __builtin_amdgcn_readfirstlane(bx * dg.wpb + wave);
     if (strip >= n_strips) return;  // whole wave
     const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
     int8_t* const lds = lds_all + wave * (2 * OCT);
@@ -329,7 +323,7 @@ hipError_t run_conv_xdw(const int8_t* x, const int8_t* wx, const int8_t* wa, voi
     const bool nn = epi_d == EPI_I8_P8_NONNEG;
 #define OHIP_XDW_L(S_, NN_, G_, CK_)                                                                                              \
     hipLaunchKernelGGL((conv_xdw_kernel<S_, NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8, NN_, G_, CK_>), grid, block, lds_bytes, stream, x, wx, wa, \
-                       out, g, gx.C, epx, ep, n_strips, rps, in_bytes, out_bytes)
+                       out, g, gx.C, epx, ep, DwGrid::of(grid.x, grid.y, (unsigned)(g.C / 16), wpb), n_strips, rps, in_bytes, out_bytes)
 #define OHIP_XDW_G(S_, NN_, CK_)                 \
     do {                                         \
         switch (NG) {                            \

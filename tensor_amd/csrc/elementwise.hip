@@ -110,12 +110,12 @@ struct CopyOp {
 
 template <typename TI, typename TO, int SP, int DP, int V, class Op>
 __global__ void __launch_bounds__(256) ew_kernel(const TI* __restrict__ src, TO* __restrict__ dst, int N, int C, int HW,
-                                                 Op op) {
+                                                 unsigned stride, Op op) {
     // 32-bit indices (the C ABI refuses tensors of 2^31 elements or more): 64-bit divisions would cost more vector
     // instructions than the operation itself
     const unsigned cv_count = (unsigned)(C / V);
     const unsigned total = (unsigned)N * cv_count * (unsigned)HW;
-    for (unsigned idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
+    for (unsigned idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += stride) {  // (no gridDim: 256 bytes of hidden arguments)
         const unsigned r = idx / (unsigned)HW;
         const int pix = (int)(idx - r * (unsigned)HW);
         const int n = (int)(r / cv_count);
@@ -136,7 +136,7 @@ static hipError_t launch_ew(const TI* src, TO* dst, int N, int C, int HW, Op op,
     size_t blocks = (total + 255) / 256;
     if (blocks > (1u << 20)) blocks = 1u << 20;
     hipLaunchKernelGGL((ew_kernel<TI, TO, SP, DP, V, Op>), dim3((unsigned)blocks), dim3(256), 0, stream, src, dst, N, C,
-                       HW, op);
+                       HW, (unsigned)blocks * 256u, op);
     return hipGetLastError();
 }
 

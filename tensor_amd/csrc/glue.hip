@@ -110,8 +110,8 @@ __global__ void __launch_bounds__(256) inner_product_kernel(const float* __restr
 // 16 bytes per thread and trip. For an image in pinned host memory the link is the bound (600 KB: 12 us); 256 workgroups
 // keep enough reads of it in flight.
 __global__ void __launch_bounds__(256) copy_bytes_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n16,
-                                                         size_t bytes) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) dst[i] = src[i];
+                                                         size_t bytes, unsigned threads) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += threads) dst[i] = src[i];
     if (blockIdx.x == 0 && threadIdx.x < bytes - n16 * 16)
         reinterpret_cast<char*>(dst)[n16 * 16 + threadIdx.x] = reinterpret_cast<const char*>(src)[n16 * 16 + threadIdx.x];
 }
@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(256) copy_bytes_kernel(const uint4* __restrict
 hipError_t run_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream) {
     const size_t n16 = bytes / 16;
     const unsigned blocks = (unsigned)(n16 < 256 * 256 ? (n16 + 255) / 256 : 256);
-    hipLaunchKernelGGL(copy_bytes_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, stream, (const uint4*)src, (uint4*)dst, n16, bytes);
+    hipLaunchKernelGGL(copy_bytes_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, stream, (const uint4*)src, (uint4*)dst, n16, bytes, blocks * 256);
     return hipGetLastError();
 }
 
