@@ -39,7 +39,7 @@ template <int FM, int FN, int WM, int WN, int EPI, int LOGP, int S = 1, int D = 
 __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
                                                            void* __restrict__ out, ConvGeom g, Epilogue ep, int m_tiles16,
                                                            int c_groups, int r_max, int cb, int tiles_per_img, int prm_ofs,
-                                                           int total_tiles, unsigned in_bytes, int tile_inv, int grid_x) {
+                                                           int total_tiles, unsigned in_bytes, int tile_inv) {
     static_assert(WM * WN == 4 && FM % 2 == 0, "four waves, row fragments in pairs");
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     constexpr int PT = WN * FN * 16;
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
 
     // Persistent workgroups: the grid holds at most two workgroups per CU and each walks over tiles.
     int bcc[FN];
-    for (int wg0 = blockIdx.x; wg0 < total_tiles; wg0 += grid_x) {
+    for (int wg0 = blockIdx.x; wg0 < total_tiles; wg0 += gridDim.x) {
         tile_of(wg0, n, p0);
         const int r_lo = p0 / g.OW;
 
@@ -285,9 +285,9 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
             // transfers run under the rest of this tile's work (the epilogue, for the last block)
             if (cb0 + cb < c_groups * 64) {
                 stage(n, p0, cb0 + cb);
-            } else if (wg0 + grid_x < total_tiles) {
+            } else if (wg0 + (int)gridDim.x < total_tiles) {
                 int n2, p2;
-                tile_of(wg0 + grid_x, n2, p2);
+                tile_of(wg0 + gridDim.x, n2, p2);
                 stage(n2, p2, 0);
             }
         }
@@ -418,7 +418,7 @@ hipError_t launch_halo_w(const int8_t* x, const int8_t* wpk, void* out, const Co
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W);
     hipLaunchKernelGGL(kern, dim3(grid_x, m_blocks), dim3(256), prm_ofs + 3 * WM * FM * 16 * sizeof(float), stream, x, wpk,
                        out, g, ep, mpad / 16, igemm_channel_groups(g.C), pl.r_max, pl.cb, pl.tiles_per_img, prm_ofs,
-                       total_tiles, in_bytes, halo_tile_invariant(WN * FN * 16, g.OW, g.OH * g.OW) ? 1 : 0, (int)grid_x);
+                       total_tiles, in_bytes, halo_tile_invariant(WN * FN * 16, g.OW, g.OH * g.OW) ? 1 : 0);
     return hipGetLastError();
 }
 
