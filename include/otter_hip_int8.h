@@ -343,7 +343,7 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * tm == -7 on a pointwise layer: kernel 6 above wherever it can run, tn = groups | pairs << 3 forcing the 16-pixel
  * groups a wave owns (1 or 2) and the pairs of 16 output channels per LDS round (0 = automatic for either).
  * tm == -8: the launch of families 1 and 3 that reads both operands straight from memory and deals the reduction to the waves
- * of a workgroup, tn = 0..4 its tile. tm == -9 on a k x k layer: the launch of those families that stages input rows in LDS,
+ * of a workgroup, tn = 0..6 its tile. tm == -9 on a k x k layer: the launch of those families that stages input rows in LDS,
  * tn = 0..3 its tile. tm == -10 on a pointwise layer with an int8 blob: the launch that keeps its operands in registers wherever it
  * can run, tn = groups | 64 if the reduction is split among the waves of a workgroup | pairs << 7 forcing the 16-pixel groups a wave owns (1, 2, or 4 with at most 256 input channels and a result
  * without a sum, a twin or a shuffle) and the pairs of 16 output channels it walks (0 = automatic for both). */

@@ -372,7 +372,7 @@ class Conv:
         return self.L.lib.otter_hip_conv_kernel_kind(self.h, in_layout, n, h, w, out_layout)
 
     def launch_choice(self, in_layout, n, h, w, out_layout):
-        """otter_hip_conv_launch_choice: (8, tile), (9, tile) or (0, 0), the family's own launch."""
+        """otter_hip_conv_launch_choice: (8, tile), (9, tile), (10, ...) or (0, 0), the family's own launch."""
         c = (C.c_int * 2)()
         self.L._check(self.L.lib.otter_hip_conv_launch_choice(self.h, in_layout, n, h, w, out_layout, c))
         return tuple(c)

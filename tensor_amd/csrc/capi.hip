@@ -684,9 +684,10 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 // most 1024 input channels, one output scale for all channels, a packed result.
 // The launches beside those of `family` (1 or 3; with an fp32 blob also 6) that a layer may take, by the cost models: the kernel
 // whose workgroups deal the reduction to their waves (conv_tap.hip) and, for k x k layers without a sum or a twin, the one on
-// staged rows (conv_rows.hip). They have to be faster than the family's launch by 5 % (pointwise layers on an fp32 blob: 10 %):
-// below that the models' errors decide. An fp32 blob may also be quantized by a pass of its own, 2 us and 0.65 us per million
-// values (0.85 beyond 50 million), in front of whichever int8 kernel is faster. Over 2000 drawn layers that the fits had not seen,
+// staged rows (conv_rows.hip). They have to be faster than the family's launch by 5 % (pointwise layers on an fp32 blob with a launch
+// of their own there: 10 %): below that the models' errors decide. An fp32 blob is otherwise quantized by a pass of its own, 2 us and
+// 0.65 us per million values (0.85 beyond 50 million), in front of whichever int8 kernel is faster (strided pointwise layers, 32 -> 56
+// on three 24x24 images: 5.9 us with that pass, 3.7 without). Over 2000 drawn layers that the fits had not seen,
 // each on an int8 and on an fp32 blob, the choice takes 53 % of the time of the families' launches alone (k x k; pointwise 88 and
 // 86 %); it is over 6 % slower than those for 13 of the 2400 k x k launches and 9 of the 1600 pointwise ones, 1.28 times at worst.
 // set_tile(-8, tile), set_tile(-9, tile) and set_tile(-10, ...) force them.
@@ -706,14 +707,16 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
     auto rows_cost = [&](bool f32, float other, int* c) { return rows && other > least ? conv_rows_cost(g, f32, ob, c) : __builtin_inff(); };
     int tap_tile = -1, rows_tile = -1, unused;
     const float tap_t = tap ? conv_tap_cost(g, f32in, ob, &tap_tile) : __builtin_inff();
-    float other = conv_family_cost(g, family, f32in && !kxk, ob);
-    if (f32in && kxk) {
+    // (without a launch of its own on fp32: k x k, strided or padded)
+    const bool own = f32in && (family == 6 || use_igemm_f32in(h, OTTER_HIP_F32_P8, g, ep));
+    float other = conv_family_cost(g, family, own, ob);
+    if (f32in && !own) {
         if (tap) other = fminf(other, conv_tap_cost(g, false, ob, &unused));
         const float millions = (float)g.N * g.C * g.H * g.W * 1e-6f, pass = 2.f + 0.65f * millions + 0.2f * fmaxf(0.f, millions - 50.f);
         // (the rows behind the pass are only looked at where they could still be faster than the launch without it)
         other = pass + (tap_t < 0.95f * (pass + fminf(other, least)) ? other : fminf(other, rows_cost(false, other, &unused)));
     }
-    const float best = tap_t < (f32in && !kxk ? 0.9f : 0.95f) * other ? tap_t : other;
+    const float best = tap_t < (own ? 0.9f : 0.95f) * other ? tap_t : other;
     if (rows_cost(f32in, best, &rows_tile) < 0.95f * best) return *config = rows_tile, ALT_ROWS;
     return *config = tap_tile, best < other ? ALT_TAP : ALT_NONE;
 }

@@ -19,6 +19,10 @@
 // Measured, us per launch before / after: 336 -> 184 3x3, one 13x13 image 22.7 / 4.5; 400 -> 216 3x3 stride 2, thirteen 23x23
 // 29.1 / 8.1; 160 -> 8 5x5 @184x224 43.0 / 17.7; 16 -> 184 5x5 @168x168 x4 56.4 / 30.9; 720 -> 384 1x1 from fp32, one 13x13
 // image 9.2 / 3.7; 64 -> 128 3x3 in 8 groups @32x32 x13 8.8 / 6.2.
+// The small launches are bound by what surrounds the loop: 64 -> 64 3x3 on one 56x56 image from fp32 spent 1.8 of 5.1 us before its
+// first step, 2.4 in the loop, 0.9 behind it. A window's mask in closed form, a loop whose loads are waited for one by one and tiles
+// of one fragment took it to 3.6 (from int8 4.0 / 3.0; 32 -> 64 stride 2 @112x112 x4 from fp32 5.4 / 4.8). 900 drawn k x k layers
+// under a million pixels: 0.915 of the time.
 //
 // INF: the input is a Float8 blob ([N][C/8][H*W][8 floats]); a lane quantizes the pairs it loads (quantize_to_int8,
 // Tensor/ConvolutionLayer.cpp:770-775). Every value is quantized once per tap that reads it, which a launch that leaves
@@ -26,6 +30,7 @@
 #include "common.hpp"
 #include "conv_igemm.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace ohip {
@@ -38,29 +43,32 @@ namespace {
 constexpr int TAP_MAX_TAPS = 31;      // bit 31 of a pixel's mask stands for "past the end of the reduction"
 constexpr int TAP_MAX_PAIRS = 2048;   // table entries: 16 KB of LDS
 
-struct TapArgs {
-    ConvGeom g;           // one group's channels; g.Cs / g.Ks the tensors'
-    FastDiv ohw, ow, c8, kw;
-    int steps, pairs;     // reduction steps and (tap, octet) pairs of them
-    int m_tiles16;        // 16-row tiles of one group's packed weights
+struct TapArgs {  // (a launch costs the host about 0.1 us more for every 32 bytes of arguments)
+    int H, W, OW, OHW, K, Ks, Cs8;        // K: one group's channels; Ks, Cs8: the tensors' channels, and octets
+    int sh, sw, ph, pw, dh, dw;
+    unsigned total_pix, in_bytes, w_bytes;
+    unsigned ohw_m, ow_m, c8_m, kw_m;     // divisions (FastDiv): multipliers, and the shifts below
+    unsigned char ohw_s, ow_s, c8_s, kw_s;
+    unsigned char kh, kw;
+    unsigned short C8, steps, pairs;      // one group's octets; reduction steps and (tap, octet) pairs of them
+    int m_tiles16;                        // 16-row tiles of one group's packed weights
     int n_pix_tiles;
-    unsigned in_bytes, w_bytes;
-    const float* in_scale;
+    unsigned row_ones;                    // bit kw * dy of each kernel row
     float in_half;
+    const float* in_scale;
 };
 
 }  // namespace
 
 template <int FM, int FN, int WK, int WN, int DEPTH, int EPI, bool INF>
 __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
-                                                                void* __restrict__ out, TapArgs ta, Epilogue ep,
+                                                                void* __restrict__ out, TapArgs ta, EpiArgs<EPI> ea,
                                                                 JoinParam<EPI> ja) {
     constexpr int UNITS = FM / 2 * FN;  // (row-tile pair, pixel fragment) accumulators of a wave
     constexpr int OOB = (int)0x80000000;  // beyond any buffer here (below 2 GiB)
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     v2i* const table = reinterpret_cast<v2i*>(lds);  // [pairs, rounded up to whole steps]: {byte offset, bit number of the tap}
     v4i* const red = reinterpret_cast<v4i*>(lds + (size_t)ta.steps * 64);  // [wn][wk][unit][half][lane]
-    const ConvGeom& g = ta.g;
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, p = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = wave % WK, wn = wave / WK;
@@ -70,16 +78,16 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
         if (pt < per * 8) pt = (pt % 8) * per + pt / 8;
     }
     const int mt0 = blockIdx.y * FM;
-    const int HW = g.H * g.W, OHW = g.OH * g.OW, C8 = g.C / 8, Cs8 = g.Cs / 8;
+    const int HW = ta.H * ta.W, OHW = ta.OHW, C8 = ta.C8, steps = ta.steps;
     const int grp = blockIdx.z;
-    const unsigned total_pix = (unsigned)g.N * (unsigned)OHW;
+    const FastDiv d_ohw{ta.ohw_m, ta.ohw_s, 0}, d_ow{ta.ow_m, ta.ow_s, 0}, d_c8{ta.c8_m, ta.c8_s, 0}, d_kw{ta.kw_m, ta.kw_s, 0};
 
     // ---- weights: the first steps are on their way before anything else happens ------------------------------------------
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int8_t*>(wpk + (size_t)grp * ta.w_bytes), 0, (int)ta.w_bytes, 0x00020000);
     v4i a[DEPTH][FM];
     auto load_a = [&](int d, int s) {  // step s (uniform); past the end: zeros
-        const int v = s < ta.steps ? lane * 16 : OOB, so = s < ta.steps ? (s * ta.m_tiles16 + mt0) * 1024 : 0;
+        const int v = s < steps ? lane * 16 : OOB, so = s < steps ? (s * ta.m_tiles16 + mt0) * 1024 : 0;
 #pragma unroll
         for (int i = 0; i < FM; ++i) a[d][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, v + i * 1024, so, 0));
     };
@@ -87,40 +95,51 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
     for (int d = 0; d < DEPTH; ++d) load_a(d, wk + d * WK);
 
     // ---- the table of pairs ---------------------------------------------------------------------------------------------------
-    for (int e = tid; e < ta.steps * 8; e += 64 * WK * WN) {
-        const unsigned tap = div_by((unsigned)e, ta.c8), oct = (unsigned)e - tap * (unsigned)C8;
-        const unsigned dy = div_by(tap, ta.kw), dx = tap - dy * (unsigned)g.kw;
-        table[e] = e < ta.pairs ? v2i{(int)(oct * (unsigned)HW + dy * (unsigned)(g.dh * g.W) + dx * (unsigned)g.dw) * 8, (int)tap}
+    for (int e = tid; e < steps * 8; e += 64 * WK * WN) {
+        const unsigned tap = div_by((unsigned)e, d_c8), oct = (unsigned)e - tap * (unsigned)C8;
+        const unsigned dy = div_by(tap, d_kw), dx = tap - dy * (unsigned)ta.kw;
+        table[e] = e < ta.pairs ? v2i{(int)(oct * (unsigned)HW + dy * (unsigned)(ta.dh * ta.W) + dx * (unsigned)ta.dw) * 8, (int)tap}
                                 : v2i{0, 31};
     }
 
     // ---- this lane's pixels ---------------------------------------------------------------------------------------------------
     unsigned px_ofs[FN], mask[FN], out_n[FN], out_pix[FN];
     bool px_ok[FN];
-    const bool pointwise = g.kh == 1 && g.kw == 1 && g.sh == 1 && g.sw == 1 && g.ph == 0 && g.pw == 0;
+    const int kh = ta.kh, kw = ta.kw;
+    const bool pointwise = kh == 1 && kw == 1 && ta.sh == 1 && ta.sw == 1 && ta.ph == 0 && ta.pw == 0;
+    const bool dilated = ta.dh != 1 || ta.dw != 1;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
         const unsigned gp = ((unsigned)pt * WN + wn) * (16 * FN) + 16 * j + p;
-        px_ok[j] = gp < total_pix;
-        const unsigned n = div_by(gp, ta.ohw), pix = gp - n * (unsigned)OHW;
+        px_ok[j] = gp < ta.total_pix;
+        const unsigned n = div_by(gp, d_ohw), pix = gp - n * (unsigned)OHW;
         out_n[j] = n, out_pix[j] = pix;
-        const unsigned img = (n * (unsigned)Cs8 + (unsigned)(grp * C8)) * (unsigned)HW * 8u;
+        const unsigned img = (n * (unsigned)ta.Cs8 + (unsigned)(grp * C8)) * (unsigned)HW * 8u;
         if (pointwise) {
             px_ofs[j] = img + pix * 8u, mask[j] = 0x80000000u;
         } else {
-            const unsigned oy = div_by(pix, ta.ow), ox = pix - oy * (unsigned)g.OW;
-            const int iy0 = (int)oy * g.sh - g.ph, ix0 = (int)ox * g.sw - g.pw;
-            px_ofs[j] = img + (unsigned)((iy0 * g.W + ix0) * 8);  // (modulo 2^32: the pair's offset brings it back)
-            unsigned cols = 0, all = (1u << g.kw) - 1, m = 0x80000000u;
-            for (int dx = 0; dx < g.kw; ++dx) {
-                const int ix = ix0 + dx * g.dw;
-                cols |= (ix < 0 || ix >= g.W ? 1u : 0u) << dx;
+            const unsigned oy = div_by(pix, d_ow), ox = pix - oy * (unsigned)ta.OW;
+            const int iy0 = (int)oy * ta.sh - ta.ph, ix0 = (int)ox * ta.sw - ta.pw;
+            px_ofs[j] = img + (unsigned)((iy0 * ta.W + ix0) * 8);  // (modulo 2^32: the pair's offset brings it back)
+            if (dilated) {
+                unsigned cols = 0, all = (1u << kw) - 1, m = 0x80000000u;
+                for (int dx = 0; dx < kw; ++dx) {
+                    const int ix = ix0 + dx * ta.dw;
+                    cols |= (ix < 0 || ix >= ta.W ? 1u : 0u) << dx;
+                }
+                for (int dy = 0; dy < kh; ++dy) {
+                    const int iy = iy0 + dy * ta.dh;
+                    m |= (iy < 0 || iy >= ta.H ? all : cols) << (dy * kw);
+                }
+                mask[j] = m;
+            } else {
+                // the taps inside the image are columns x0..x1 of rows y0..y1: the columns' bits, repeated per kernel row, under the
+                // rows' bits (the loops above take 100 instructions of a wave that has few others: 0.2 to 0.5 us of a launch)
+                const int x1 = min(max(ta.W - ix0, 0), kw), x0 = min(max(-ix0, 0), x1);
+                const int y1 = min(max(ta.H - iy0, 0), kh), y0 = min(max(-iy0, 0), y1);
+                const unsigned cols = (1u << x1) - (1u << x0), rows = (1u << (y1 * kw)) - (1u << (y0 * kw));
+                mask[j] = ~(cols * ta.row_ones & rows);
             }
-            for (int dy = 0; dy < g.kh; ++dy) {
-                const int iy = iy0 + dy * g.dh;
-                m |= (iy < 0 || iy >= g.H ? all : cols) << (dy * g.kw);
-            }
-            mask[j] = m;
         }
         if (!px_ok[j]) mask[j] = 0xffffffffu;
     }
@@ -135,7 +154,7 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
     auto load_b = [&](int d, int s) {
         // steps past the end keep the bit of the last table row's padding out of reach: they read the table's first step
         // with every pair invalid
-        const bool in = s < ta.steps;
+        const bool in = s < steps;
         const v4i t = reinterpret_cast<const v4i*>(table)[(in ? s : 0) * 4 + q];
         const int b0 = in ? t[1] : 31, b1 = in ? t[3] : 31;
 #pragma unroll
@@ -163,31 +182,55 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
-    for (int s0 = wk; s0 < ta.steps; s0 += DEPTH * WK) {
+    auto multiply = [&](int d) {
+        v4i bb[FN];
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            v4i bb[FN];
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                if constexpr (INF)
-                    bb[j] = v4i{quantize4(bf[d][j][0], in_scale, ta.in_half), quantize4(bf[d][j][1], in_scale, ta.in_half),
-                                quantize4(bf[d][j][2], in_scale, ta.in_half), quantize4(bf[d][j][3], in_scale, ta.in_half)};
-                else
-                    bb[j] = v4i{b[d][j][0][0], b[d][j][0][1], b[d][j][1][0], b[d][j][1][1]};
-            }
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[d][i], bb[j], acc[i][j], 0, 0, 0);
-            const int nx = s0 + (DEPTH + d) * WK;  // the step this stage holds next
-            if (nx < ta.steps) {                   // (uniform)
-                load_a(d, nx);
-                load_b(d, nx);
-            } else {
-#pragma unroll
-                for (int i = 0; i < FM; ++i) a[d][i] = v4i{0, 0, 0, 0};
-            }
+        for (int j = 0; j < FN; ++j) {
+            if constexpr (INF)
+                bb[j] = v4i{quantize4(bf[d][j][0], in_scale, ta.in_half), quantize4(bf[d][j][1], in_scale, ta.in_half),
+                            quantize4(bf[d][j][2], in_scale, ta.in_half), quantize4(bf[d][j][3], in_scale, ta.in_half)};
+            else
+                bb[j] = v4i{b[d][j][0][0], b[d][j][0][1], b[d][j][1][0], b[d][j][1][1]};
         }
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[d][i], bb[j], acc[i][j], 0, 0, 0);
+    };
+    // No load of the loop is conditional: behind a conditional one the compiler waits for every load in flight (which made the
+    // stages ahead worthless). The last trip's 1 to DEPTH - 1 loads are code of their own (EXACT); where that takes too
+    // many registers (from fp32, the widest tile) they go beyond the buffer where a step is missing.
+    constexpr bool EXACT = !INF && FM * FN < 16;
+    constexpr int WHOLE = EXACT ? 2 * DEPTH : DEPTH + 1;
+    int s = wk, left = (steps - wk + WK - 1) / WK;  // this wave's next step, and how many it has from there on
+    for (; left >= WHOLE; left -= DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d, s += WK) {
+            multiply(d);
+            load_a(d, s + DEPTH * WK);
+            load_b(d, s + DEPTH * WK);
+        }
+    }
+    bool done = false;
+    if constexpr (EXACT) {
+#pragma unroll
+        for (int r = 1; r < DEPTH; ++r)
+            if (left == DEPTH + r) {
+#pragma unroll
+                for (int d = 0; d < r; ++d, s += WK) {
+                    multiply(d);
+                    load_a(d, s + DEPTH * WK);
+                    load_b(d, s + DEPTH * WK);
+                }
+#pragma unroll
+                for (int d = r; d < DEPTH + r; ++d) multiply(d % DEPTH);
+                done = true;
+            }
+    }
+    if (!done) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+            if (d < left) multiply(d);
     }
 
     // ---- the waves' sums meet: unit u of a pixel group is finished by its wave u % WK ---------------------------------------------
@@ -201,10 +244,11 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
         }
         __syncthreads();
     }
-    const size_t ch_base = (size_t)grp * g.K;
+    const int K = ta.K, Ks = ta.Ks;
+    const size_t ch_base = (size_t)grp * K;
+    Epilogue ep = ea.epilogue();
     ep.scale_in += ch_base, ep.bias += ch_base;
     if (ep.scale_out) ep.scale_out += ch_base;
-    const int Ks = g.Ks;
 #pragma unroll
     for (int u = 0; u < UNITS; ++u) {
         if (WK > 1 && u % WK != wk) continue;  // (uniform)
@@ -220,11 +264,11 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
             }
         }
         const int ch0 = 16 * mt0 + 32 * pair + 8 * q;  // this lane's 8 consecutive output channels of the group
-        if (!px_ok[j] || ch0 >= g.K) continue;
+        if (!px_ok[j] || ch0 >= K) continue;
         const int a8[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         const unsigned n = out_n[j], pix = out_pix[j];
         if constexpr (EPI == EPI_GENERIC) {
-            epilogue_store8_generic(out, &ep, (int)n, ch0, (int)pix, g.K, OHW, a8[0], a8[1], a8[2], a8[3], a8[4], a8[5], a8[6], a8[7]);
+            epilogue_store8_generic(out, &ep, (int)n, ch0, (int)pix, K, OHW, a8[0], a8[1], a8[2], a8[3], a8[4], a8[5], a8[6], a8[7]);
         } else {
             Epi8 prm;
             epi8_load<EPI>(prm, ep, ch0);
@@ -233,19 +277,19 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
                 const size_t o = ((size_t)(n * (unsigned)(Ks / 8) + ch / 8) * (unsigned)OHW + pix) * 8;
                 epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm, o, a8);
             } else if constexpr (EPI == EPI_F32_SHUFFLE) {
-                if (ep.lrelu) epi8_store_shuffle<1>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
-                else epi8_store_shuffle<0>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, g.K, OHW);
+                if (ep.lrelu) epi8_store_shuffle<1>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, K, OHW);
+                else epi8_store_shuffle<0>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, K, OHW);
             } else {
                 constexpr bool FUSED = EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_P4_PARTS;
                 const size_t e = ((size_t)(n * (unsigned)(Ks / 4) + ch / 4) * (unsigned)OHW + pix) * 4;
                 const float *r0 = nullptr, *r1 = nullptr;
                 if constexpr (EPI == EPI_F32_P4_PARTS) {  // (one group)
-                    r0 = epi4_residual_at(ep, ja, n, pix, ch0, g.K, OHW);
-                    r1 = epi4_residual_at(ep, ja, n, pix, ch0 + 4, g.K, OHW);
+                    r0 = epi4_residual_at(ep, ja, n, pix, ch0, K, OHW);
+                    r1 = epi4_residual_at(ep, ja, n, pix, ch0 + 4, K, OHW);
                 }
                 ohip_v2i tw = {0, 0};
                 tw[0] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si, prm.bi, e, a8[0], a8[1], a8[2], a8[3], r0);
-                if (ch0 + 4 < g.K)
+                if (ch0 + 4 < K)
                     tw[1] = (int)epi4_store_f32p4<FUSED>((float*)out, ep, prm.si + 4, prm.bi + 4, e + (size_t)OHW * 4, a8[4], a8[5],
                                                          a8[6], a8[7], r1);
                 if constexpr (FUSED)
@@ -313,36 +357,47 @@ bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
 
 namespace {
 // A tile is 16 fm output channels x 16 fn wn pixels, `resident` workgroups of it a compute unit's registers hold. The cost of a
-// launch in microseconds (measured inside a graph of launches, warm) is start + chain * S + c * (waves * S * step + group) +
-// out_mb per megabyte of results, with S the reduction steps of one wave and c the workgroups of the busiest compute unit. Chain
-// and step grow by `strided` where the stride is not 1, a load then using every second 8 bytes of its lines, and by up to `far`
-// where the pixels of the workgroups side by side on a compute unit are more than its share of an XCD's L2 (128 KB: 4 MB over 32)
-// holds from one tap, or one row block, to the next: from the whole share (fp32 blobs, the widest tile) or half of it on, fully at
-// twice that, and only as far as the blob is over 4 MB, fully at 16. Fitted to 5800 layers drawn over 8..960 channels, 1x1 to 5x5,
-// 50 to 2.5 million pixels; the median error is 5 to 7 %. (Without these two, 3x3 stride 2 232 -> 344 @57x66 b30 took the last tile
-// at 112 us; the implicit-GEMM kernel takes 64.)
+// launch in microseconds (measured inside a graph of launches, warm) is start + chain * S + c * (waves * S * step + group, with
+// `quant` more where the result is int8) + round for every time the compute unit fills up again + in_mb and out_mb per megabyte,
+// with S the reduction steps of one wave and c the workgroups of the busiest compute unit. Chain and step grow by `strided` where the
+// stride is not 1, a load then using every second 8 bytes of its lines, and by up to `far` where the pixels of the workgroups side by
+// side on a compute unit are more than its share of an XCD's L2 (128 KB: 4 MB over 32) holds from one tap, or one row block, to the
+// next: from the whole share (fp32 blobs, the widest tile) or half of it on, fully at twice that, and only as far as the blob is over
+// 4 MB, fully at 16. Fitted to 2900 layers drawn over 8..800 channels, 1x1 to 5x5, 50 to 2.5 million pixels, errors below the
+// measurement counted 1.6 times; the median error is 3 to 5 %. (The widest tile keeps an older fit: this one called strided layers of
+// 300 channels and more on it 2 times too fast.) The tile that the costs name is 1.1 % slower than the fastest one on average.
+// Tiles of one pixel fragment per wave (the last two) are the fastest for 45 % of the layers from fp32 and 30 % of those from int8:
+// they fill the machine with half the pixels. 64 -> 64 3x3 on one 56x56 image from fp32 3.6 us, 4.0 to 5.0 with the others.
 struct TapCost {
-    float start, chain, step, group, out_mb, strided, far;
+    float start, chain, step, group, out_mb, strided, far, in_mb, quant, round;
 };
 struct TapConfig {
     int fm, fn, wk, wn, resident, resident_f32;
     TapCost i8, f32;
 };
 constexpr TapConfig kTapConfigs[] = {
-    {2, 1, 8, 1, 3, 3, {2.382f, 0.041f, 0.021f, 0.747f, 0.005f, 0.145f, 2.2f}, {2.332f, 0.069f, 0.051f, 0.576f, 0.f, 0.37f, 2.224f}},
-    {2, 2, 4, 1, 5, 4, {2.605f, 0.048f, 0.033f, 0.552f, 0.029f, 0.157f, 0.364f}, {2.754f, 0.158f, 0.087f, 0.509f, 0.006f, 0.354f, 1.091f}},
-    {4, 2, 4, 1, 4, 3, {2.517f, 0.062f, 0.048f, 0.466f, 0.041f, 0.137f, 0.346f}, {2.702f, 0.129f, 0.103f, 0.694f, 0.061f, 0.346f, 1.079f}},
-    {4, 2, 2, 2, 5, 3, {2.719f, 0.041f, 0.05f, 0.485f, 0.083f, 0.104f, 0.229f}, {2.862f, 0.122f, 0.101f, 0.754f, 0.089f, 0.266f, 0.918f}},
-    {4, 4, 1, 4, 3, 0, {3.568f, 0.036f, 0.084f, 1.238f, 0.096f, 0.101f, 0.8f}, {}},  // (no fp32 input: registers)
+    {2, 1, 8, 1, 3, 3, {2.53f, 0.005f, 0.024f, 0.52f, 0.3f, 0.139f, 4.f, 0.f, 0.064f, 0.581f},
+                       {2.497f, 0.043f, 0.049f, 0.222f, 0.3f, 0.295f, 0.875f, 0.051f, 0.097f, 0.626f}},
+    {2, 2, 4, 1, 5, 4, {2.717f, 0.028f, 0.034f, 0.251f, 0.207f, 0.132f, 0.666f, 0.f, 0.07f, 1.082f},
+                       {2.833f, 0.122f, 0.082f, 0.159f, 0.191f, 0.195f, 0.955f, 0.06f, 0.076f, 0.919f}},
+    {4, 2, 4, 1, 4, 3, {2.745f, 0.031f, 0.052f, 0.082f, 0.158f, 0.16f, 0.497f, 0.f, 0.074f, 0.696f},
+                       {2.929f, 0.177f, 0.097f, 0.05f, 0.178f, 0.187f, 0.906f, 0.051f, 0.087f, 1.476f}},
+    {4, 2, 2, 2, 4, 3, {2.787f, 0.043f, 0.05f, 0.058f, 0.166f, 0.126f, 0.472f, 0.005f, 0.168f, 0.718f},
+                       {3.026f, 0.145f, 0.098f, 0.05f, 0.193f, 0.223f, 0.84f, 0.062f, 0.17f, 1.221f}},
+    {4, 4, 1, 4, 3, 0, {3.568f, 0.036f, 0.084f, 1.238f, 0.096f, 0.101f, 0.8f, 0.f, 0.f, 0.f}, {}},  // (no fp32 input: registers)
+    {4, 1, 4, 1, 6, 5, {2.611f, 0.016f, 0.041f, 0.081f, 0.188f, 0.082f, 0.501f, 0.f, 0.04f, 0.355f},
+                       {2.604f, 0.078f, 0.055f, 0.093f, 0.267f, 0.197f, 1.033f, 0.046f, 0.08f, 0.642f}},
+    {4, 1, 8, 1, 3, 2, {2.537f, 0.012f, 0.04f, 0.244f, 0.262f, 0.125f, 4.f, 0.001f, 0.143f, 0.447f},
+                       {2.666f, 0.018f, 0.06f, 0.12f, 0.3f, 0.323f, 2.149f, 0.056f, 0.136f, 0.957f}},
 };
 constexpr int kTapConfigCount = (int)(sizeof(kTapConfigs) / sizeof(kTapConfigs[0]));
 
 template <int FM, int FN, int WK, int WN, int DEPTH, int EPI, bool INF>
 hipError_t launch_tap(const void* x, const int8_t* wpk, void* out, const TapArgs& ta, const Epilogue& ep, int groups, hipStream_t stream) {
     const size_t lds = (size_t)ta.steps * 64 + (WK > 1 ? (size_t)WN * WK * (FM / 2) * FN * 2048 : 0);
-    const dim3 grid((unsigned)ta.n_pix_tiles, (unsigned)((ta.g.K + 16 * FM - 1) / (16 * FM)), (unsigned)groups);
+    const dim3 grid((unsigned)ta.n_pix_tiles, (unsigned)((ta.K + 16 * FM - 1) / (16 * FM)), (unsigned)groups);
     hipLaunchKernelGGL((conv_tap_kernel<FM, FN, WK, WN, DEPTH, EPI, INF>), grid, dim3(64 * WK * WN), lds, stream, (const int8_t*)x,
-                       wpk, out, ta, ep, JoinParam<EPI>::of(ep));
+                       wpk, out, ta, EpiArgs<EPI>::of(ep), JoinParam<EPI>::of(ep));
     return hipGetLastError();
 }
 }  // namespace
@@ -352,6 +407,7 @@ float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config) {
     const float bytes = f32in ? 4.f : 1.f, in_mb = (float)g.N * g.C * g.H * g.W * 1e-6f * bytes;
     const long px = (long)g.N * g.OH * g.OW;
     const float out_mb = (float)px * (float)g.K * 1e-6f * (float)out_bytes;
+    const float rows_read = fminf(1.f, (float)g.kh / (float)g.sh);
     auto clamp01 = [](float v) { return fminf(fmaxf(v, 0.f), 1.f); };
     float best = __builtin_inff();
     *config = -1;
@@ -361,12 +417,14 @@ float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config) {
         if (k.step == 0.f) continue;
         const int blocks = (K + 16 * c.fm - 1) / (16 * c.fm);
         const long groups = (px + 16 * c.fn * c.wn - 1) / (16 * c.fn * c.wn) * blocks * g.groups;
-        const float s = (float)((steps + c.wk - 1) / c.wk), cu = (float)((groups + 255) / 256), w = (float)(c.wk * c.wn) * s;
+        const float s = (float)((steps + c.wk - 1) / c.wk), cu = (float)std::min((groups + 255) / 256, 1l << 24), w = (float)(c.wk * c.wn) * s;
         const float side = fminf(cu, (float)(f32in ? c.resident_f32 : c.resident)) * (float)(16 * c.fn * c.wn * g.sw) * (float)C * bytes;
         const float beyond = clamp01(side / (f32in || c.fn == 4 ? 131072.f : 65536.f) - 1.f) * clamp01((in_mb - 4.f) / 12.f);
         const bool again = g.kh * g.kw * blocks > 1;  // the pixels are read more than once
         const float slow = (g.sw > 1 ? 1.f + k.strided : 1.f) * (again ? 1.f + k.far * beyond : 1.f);
-        const float t = k.start + k.chain * s * slow + cu * (w * k.step * slow + k.group) + k.out_mb * out_mb;
+        const float rounds = (float)(((int)cu - 1) / (f32in ? c.resident_f32 : c.resident));  // behind the first
+        const float t = k.start + k.chain * s * slow + cu * (w * k.step * slow + k.group + (out_bytes == 1 ? k.quant : 0.f)) +
+                        rounds * k.round + k.in_mb * in_mb * rows_read + k.out_mb * out_mb;
         if (t < best) best = t, *config = i;
     }
     return best;
@@ -393,31 +451,36 @@ float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes)
     return 2.46f + 0.34f * chunks + 94.f * mac + 26.f * epi + 0.03f * in_mb + 0.07f * out_mb;
 }
 
-hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g_in, const Epilogue& ep, int config,
+hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep, int config,
                         const float* in_scale, int in_round_mode, hipStream_t stream) {
-    if (!conv_tap_supported(g_in, ep, f32in) || config < 0 || config >= kTapConfigCount) return hipErrorInvalidValue;
+    if (!conv_tap_supported(g, ep, f32in) || config < 0 || config >= kTapConfigCount) return hipErrorInvalidValue;
+    const int C = g.C / g.groups, K = g.K / g.groups;
+    const FastDiv ohw = fast_div((unsigned)(g.OH * g.OW)), ow = fast_div((unsigned)g.OW), c8 = fast_div((unsigned)(C / 8)),
+                  kw = fast_div((unsigned)g.kw);
     TapArgs ta;
-    ta.g = g_in;
-    ta.g.Cs = g_in.C, ta.g.Ks = g_in.K;
-    ta.g.C = g_in.C / g_in.groups, ta.g.K = g_in.K / g_in.groups;
-    const ConvGeom& g = ta.g;
-    ta.ohw = fast_div((unsigned)(g.OH * g.OW)), ta.ow = fast_div((unsigned)g.OW);
-    ta.c8 = fast_div((unsigned)(g.C / 8)), ta.kw = fast_div((unsigned)g.kw);
-    ta.steps = tap_steps(g.C, g.kh, g.kw), ta.pairs = tap_pairs(g.C, g.kh, g.kw);
-    ta.m_tiles16 = igemm_padded_rows(g.K) / 16;
-    ta.in_bytes = (unsigned)((size_t)g.N * g.Cs * g.H * g.W * (f32in ? 4 : 1));
-    ta.w_bytes = (unsigned)tap_packed_weight_bytes(g.K, g.C, g.kh, g.kw);
+    ta.H = g.H, ta.W = g.W, ta.OW = g.OW, ta.OHW = g.OH * g.OW, ta.K = K, ta.Ks = g.K, ta.Cs8 = g.C / 8;
+    ta.sh = g.sh, ta.sw = g.sw, ta.ph = g.ph, ta.pw = g.pw, ta.dh = g.dh, ta.dw = g.dw;
+    ta.total_pix = (unsigned)g.N * (unsigned)ta.OHW;
+    ta.ohw_m = ohw.m, ta.ow_m = ow.m, ta.c8_m = c8.m, ta.kw_m = kw.m;
+    ta.ohw_s = (unsigned char)ohw.s, ta.ow_s = (unsigned char)ow.s, ta.c8_s = (unsigned char)c8.s, ta.kw_s = (unsigned char)kw.s;
+    ta.kh = (unsigned char)g.kh, ta.kw = (unsigned char)g.kw, ta.C8 = (unsigned short)(C / 8);  // (conv_tap_supported bounds them)
+    ta.steps = (unsigned short)tap_steps(C, g.kh, g.kw), ta.pairs = (unsigned short)tap_pairs(C, g.kh, g.kw);
+    ta.m_tiles16 = igemm_padded_rows(K) / 16;
+    ta.in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1));
+    ta.w_bytes = (unsigned)tap_packed_weight_bytes(K, C, g.kh, g.kw);
+    ta.row_ones = 0;
+    for (int dy = 0; dy < g.kh; ++dy) ta.row_ones |= 1u << (dy * g.kw);
     ta.in_scale = in_scale;
     ta.in_half = in_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     const TapConfig c = kTapConfigs[config];
     const long px = (long)g.N * g.OH * g.OW, per = 16l * c.fn * c.wn;
     ta.n_pix_tiles = (int)((px + per - 1) / per);
-    int epi = pick_epilogue(ep, g.K);
+    int epi = pick_epilogue(ep, K);
     if (epi == EPI_F32_P4 && ep.fused()) epi = ep.join == nullptr ? EPI_F32_P4_FUSED : ep.join->other != nullptr ? EPI_F32_SHUFFLE : EPI_F32_P4_PARTS;
 #define OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, E_)                                                                           \
     if (config == I_ && epi == E_) {                                                                                        \
-        if (!f32in) return launch_tap<FM_, FN_, WK_, WN_, D_, E_, false>(x, wpk, out, ta, ep, g_in.groups, stream);         \
-        if constexpr (E_ != EPI_GENERIC && E_ < EPI_F32_SHUFFLE && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g_in.groups, stream); \
+        if (!f32in) return launch_tap<FM_, FN_, WK_, WN_, D_, E_, false>(x, wpk, out, ta, ep, g.groups, stream);         \
+        if constexpr (E_ != EPI_GENERIC && E_ < EPI_F32_SHUFFLE && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g.groups, stream); \
     }
 #define OHIP_TAP(I_, FM_, FN_, WK_, WN_, D_)                 \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8)         \
@@ -432,6 +495,8 @@ hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out,
     OHIP_TAP(2, 4, 2, 4, 1, 2)
     OHIP_TAP(3, 4, 2, 2, 2, 2)
     OHIP_TAP(4, 4, 4, 1, 4, 2)
+    OHIP_TAP(5, 4, 1, 4, 1, 2)
+    OHIP_TAP(6, 4, 1, 8, 1, 2)
 #undef OHIP_TAP
 #undef OHIP_TAP2
     return hipErrorInvalidValue;
