@@ -157,6 +157,13 @@ size_t otter_hip_conv_workspace_bytes(const otter_hip_conv_t* handle, int in_lay
 int otter_hip_conv_forward(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w,
                            void* out, int out_layout, void* workspace, size_t workspace_bytes, void* stream);
 
+/* otter_hip_conv_forward with the workspace made by the call, at most once and only where the chosen launches use one: make returns
+ * device memory of at least that many bytes, on the calling thread, or null (the call then fails as without a workspace). It is the
+ * caller's to free, after the stream's work up to here; make must not throw. */
+typedef void* (*otter_hip_workspace_fn)(void* ctx, size_t bytes);
+int otter_hip_conv_forward_making(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w, void* out,
+                                  int out_layout, otter_hip_workspace_fn make, void* ctx, void* stream);
+
 /* No counterpart in the reference. For callers that cannot allocate device memory -- code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc: otter_hip_conv_forward with the workspace (the quantized copy
  * of an fp32 input, or the channel-padded copy of a blob with C % 8 != 0) taken from a static device array of

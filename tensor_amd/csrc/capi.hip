@@ -711,9 +711,9 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
     const bool own = f32in && (family == 6 || use_igemm_f32in(h, OTTER_HIP_F32_P8, g, ep));
     float other = conv_family_cost(g, family, own, ob);
     if (f32in && !own) {
-        if (tap) other = fminf(other, conv_tap_cost(g, false, ob, &unused));
         const float millions = (float)g.N * g.C * g.H * g.W * 1e-6f, pass = 2.f + 0.65f * millions + 0.2f * fmaxf(0.f, millions - 50.f);
-        // (the rows behind the pass are only looked at where they could still be faster than the launch without it)
+        // (the launches behind the pass are only looked at where they could still be faster than the one without it; 2.2: none costs less)
+        if (tap && tap_t >= 0.95f * (pass + 2.2f)) other = fminf(other, conv_tap_cost(g, false, ob, &unused));
         other = pass + (tap_t < 0.95f * (pass + fminf(other, least)) ? other : fminf(other, rows_cost(false, other, &unused)));
     }
     const float best = tap_t < (own ? 0.9f : 0.95f) * other ? tap_t : other;
@@ -777,7 +777,14 @@ int otter_hip_conv_rows_plan(const otter_hip_conv_desc* desc, int n, int in_h, i
 // `residual` (or null): a blob in the output's layout added to the fp32 result; the twin is then made of the sum
 static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w, void* out,
                         int out_layout, void* workspace, size_t workspace_bytes, void* stream_, int8_t* twin,
-                        float twin_scale, int twin_round, const float* residual = nullptr) {
+                        float twin_scale, int twin_round, const float* residual = nullptr,
+                        otter_hip_workspace_fn make_workspace = nullptr, void* make_ctx = nullptr) {
+    // the caller's workspace, or one that it makes now: most launches on an fp32 blob quantize for themselves and need none
+    auto workspace_of = [&](size_t need) {
+        if (make_workspace && need) workspace = make_workspace(make_ctx, need), workspace_bytes = workspace ? need : 0;
+        return workspace && workspace_bytes >= need;
+    };
+
     if (!h || !in || (!out && !twin)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: null");
     if (!valid_layout(in_layout) || !valid_layout(out_layout))
         return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: unknown layout");
@@ -884,7 +891,7 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
     if (h->c_pad) {
         // (quantize and) zero-pad the channels into a Byte8 copy; the MFMA kernels then see C = c_pad
         const size_t need = (size_t)n * h->c_pad * in_h * in_w;
-        if (!workspace || workspace_bytes < need)
+        if (!workspace_of(need))
             return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: this layer needs the workspace reported by "
                                                "otter_hip_conv_workspace_bytes");
         OHIP_CHECK(run_pad_pack8(in, layout_elem(in_layout) == 0, layout_pack(in_layout), (int8_t*)workspace, n, g.C,
@@ -894,7 +901,7 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
         g.C = h->c_pad;
     } else if (layout_elem(in_layout) == 0) {
         const size_t need = (size_t)n * g.C * in_h * in_w;
-        if (!workspace || workspace_bytes < need)
+        if (!workspace_of(need))
             return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward: fp32 input needs a workspace of N*C*H*W bytes");
         q_layout = g.C % 8 == 0 ? OTTER_HIP_I8_P8 : OTTER_HIP_I8;
         OHIP_CHECK(run_quantize((const float*)in, layout_pack(in_layout), (int8_t*)workspace, layout_pack(q_layout), n,
@@ -958,6 +965,11 @@ int otter_hip_conv_forward(const otter_hip_conv_t* h, const void* in, int in_lay
                            void* out, int out_layout, void* workspace, size_t workspace_bytes, void* stream) {
     return conv_forward(h, in, in_layout, n, in_h, in_w, out, out_layout, workspace, workspace_bytes, stream, nullptr, 0.f,
                         0);
+}
+
+int otter_hip_conv_forward_making(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w, void* out, int out_layout,
+                                  otter_hip_workspace_fn make_workspace, void* ctx, void* stream) {
+    return conv_forward(h, in, in_layout, n, in_h, in_w, out, out_layout, nullptr, 0, stream, nullptr, 0.f, 0, nullptr, make_workspace, ctx);
 }
 
 int otter_hip_conv_forward_static(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w,

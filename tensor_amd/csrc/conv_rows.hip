@@ -332,7 +332,7 @@ static bool rows_plan(const ConvGeom& g_in, int fn, RowsArgs* ra, size_t* lds) {
         if (total >= max_px || strip_px >= max_px) break;
         const int tiles = (int)((unsigned)(total + pt - 1) / (unsigned)pt);
         // rows of a tile: the output rows it can touch, and the padding rows between the images it can run over
-        const long out_rows = (pt - 1) / w + 2, crossings = (pt - 1) / strip_px + 1;
+        const long out_rows = (pt - 1) / w + 2, crossings = (pt - 1) / (int)strip_px + 1;
         const long between = vh - (long)g.OH * g.sh;  // virtual rows an image has more than its output rows' share (may be negative)
         const long rows = (out_rows - 1) * g.sh + (between > 0 ? crossings * between : 0) + (long)(g.kh - 1) * g.dh + 1;
         const long cost = (long)tiles * (rows * vw2 + 64);

@@ -1,0 +1,36 @@
+"""A layer call without a workspace of the caller's: one is made only where the chosen launches use it, with the results unchanged."""
+import numpy as np
+import pytest
+
+from gpu_util import host_scale_in
+from tensor_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _allocations(torch, f):
+    f()
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    out = f()
+    return out, torch.cuda.memory_stats()["allocation.all.allocated"] - before
+
+
+@pytest.mark.parametrize("C,K,k,hw,tile,made", [
+    (64, 64, 3, 14, (-8, 5), 1),   # quantized by the launch itself: the output alone
+    (64, 64, 3, 14, (-4, 0), 2),   # a quantize pass in front
+    (20, 24, 3, 9, (0, 0), 2),     # channels padded to a multiple of 8
+    (64, 64, 1, 14, (0, 0), 1),
+])
+def test_workspace_only_where_used(hip, C, K, k, hw, tile, made):
+    rng = np.random.default_rng(C)
+    conv = hip.conv(wq=rng.integers(-127, 128, (K, C, k, k)).astype(np.int8), scale_in=host_scale_in(np.full(K, 60.0, np.float32), 20.0),
+                    bias=rng.normal(0, 1, K).astype(np.float32), in_scale=20.0, pad=(k // 2, k // 2), out_kind=capi.OUT_F32)
+    conv.set_tile(*tile)
+    layout = capi.F32_P8 if C % 8 == 0 else capi.F32_P4
+    x = hip.to_device(rng.uniform(-5, 5, 2 * C * hw * hw).astype(np.float32))
+    need = hip.lib.otter_hip_conv_workspace_bytes(conv.h, layout, 2, hw, hw)
+    want = conv.forward(x, layout, 2, hw, hw, workspace=hip.empty(need, np.int8))
+    got, count = _allocations(hip.torch, lambda: conv.forward(x, layout, 2, hw, hw))
+    assert hip.torch.equal(got.view(hip.torch.int32), want.view(hip.torch.int32))
+    assert count == made
+    conv.close()
