@@ -21,6 +21,13 @@ namespace ohip {
 // LDS lines of their octet. Rows outside the image and pixels past the row's end are written as zeros: they are the
 // depthwise layer's padding, not the pointwise layer's result on a zero input. The depthwise layer then reads its
 // operands from those lines, octet by octet, exactly as conv_dw3x3_f32in_kernel does.
+//
+// What bounds it: the vector instructions of the rows (the cost of a strip below), and in launches of a few hundred waves the chain in
+// front of the first row and the memory latency of each row that is requested late. There every row of a short strip is requested
+// before the first is waited for, narrow lines are cleared by 5 stores instead of 7 with a division each, behind the requests, and a
+// row outside the image goes through an empty descriptor, not through a branch around each load. Pointwise + depthwise, us per launch
+// before / after: 64 -> 384 @14x14 b1 4.8 / 4.3, 32 -> 192 @28x28 b1 5.0 / 4.7, 24 -> 144 @56x56 b1 6.0 / 5.1, 16 -> 96 @112x112
+// stride 2 b64 27.6 / 26.7, 24 -> 144 @56x56 b64 24.4 / 23.3.
 size_t xdw_weight_bytes(int Cin, int K) { return (size_t)(K / 16) * (Cin <= 32 ? 64 * 8 : 2 * 64 * 16); }
 
 // weight [K][Cin] int8 -> A operands [K/16][reduction step][lane 64][16 bytes] (8 bytes for at most 32 input channels):
@@ -37,12 +44,20 @@ void xdw_pack_weights(const int8_t* w, int Cin, int K, int8_t* dst) {
                 }
 }
 
+struct XdwArgs {  // (a launch costs the host 0.1 us more for every 32 bytes of arguments: 200 instead of 350)
+    int H, W, OH, OW, K, cin, ph;  // K: expanded channels
+    int n_strips, rps;             // strips of an image, output rows of a strip
+    unsigned in_bytes, out_bytes;
+    DwGrid dg;
+};
+
 template <int S, int EPI, bool XNN, int NG, int CK>
-__global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S == 2 && NG <= 4)) ? 3 : 2) conv_xdw_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wx,
-                                                       const int8_t* __restrict__ wa, void* __restrict__ out, ConvGeom g, int cin,
-                                                       Epilogue epx, Epilogue ep, DwGrid dg, int n_strips, int rps, unsigned in_bytes,
-                                                       unsigned out_bytes) {
-    constexpr int RL = 4, PF = 2;      // LDS lines per octet / rows of loads in flight
+__global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S == 2 && NG <= 2)) ? 3 : 2) conv_xdw_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wx,
+                                                       const int8_t* __restrict__ wa, void* __restrict__ out, XdwArgs g,
+                                                       EpiArgs<EPI> eax, EpiArgs<EPI> ea) {
+    // LDS lines per octet / rows of loads in flight: four where they take few registers, so that a strip of one or two output rows
+    // has every input row requested before it waits for one
+    constexpr int RL = 4, PF = NG == 1 || (NG == 2 && CK == 32) ? 4 : 2;
     constexpr int NCH = (NG + 3) / 4;  // column chunks of 64 pixels of the depthwise operand
     constexpr int T = S == 1 ? 2 : 1;  // A sets of the depthwise layer
     constexpr int PH = 4 / S;          // output pixels per lane column
@@ -50,29 +65,19 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
     constexpr int LINE = (64 * NCH + 8) * 8;
     constexpr int OCT = RL * LINE + 128;  // the second octet's lines, off the first one's banks
     extern __shared__ __attribute__((aligned(16))) int8_t lds_all[];  // [waves of the workgroup][2 octets][RL lines]
-    const int C8 = g.C / 8;
+    const Epilogue epx = eax.epilogue(), ep = ea.epilogue();
+    const int C8 = g.K / 8;
     unsigned bx, pr_u, img_u;
-    dg.locate(&bx, &pr_u, &img_u);
+    g.dg.locate(&bx, &pr_u, &img_u);
     const int pr = (int)pr_u, img = (int)img_u;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int strip = __builtin_amdgcn_readfirstlane(bx * dg.wpb + wave);
-    if (strip >= n_strips) return;  // whole wave
+    const int strip = __builtin_amdgcn_readfirstlane(bx * g.dg.wpb + wave);
+    if (strip >= g.n_strips) return;  // whole wave
     const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
     int8_t* const lds = lds_all + wave * (2 * OCT);
 
-    // the padding slots of every line: pixels -2, -1 and 16 NG .. 64 NCH + 5 (the pixels from W to 16 NG - 1 are written
-    // as zeros with every row)
-    {
-        constexpr int PADS = 64 * NCH + 8 - 16 * NG;
-        for (int i = lane; i < PADS * RL * 2; i += 64) {
-            const int line = i / PADS, k = i % PADS;
-            const int slot = k < 2 ? k : 16 * NG + k;
-            *reinterpret_cast<v2i*>(lds + (line / RL) * OCT + (line % RL) * LINE + slot * 8) = v2i{0, 0};
-        }
-    }
-
     // ---- pointwise layer: weights, this lane's input octet(s) of every pixel group, its four channels' constants -------
-    const int Cin8 = cin / 8;
+    const int Cin8 = g.cin / 8;
     const unsigned HW8 = (unsigned)(g.H * g.W) * 8u;
     const unsigned s_in = (unsigned)(img * Cin8) * HW8;
     const int oct0 = CK == 32 ? q : 2 * q;  // first input octet of this lane's reduction bytes
@@ -81,19 +86,20 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
     for (int p = 0; p < NG; ++p) v_in[p] = (16 * p + n < g.W && oct0 < Cin8) ? (unsigned)oct0 * HW8 + (unsigned)(16 * p + n) * 8u : DW_OOB;
     // (the other octets of this lane's reduction bytes: + 1, and + 8, + 9 in the second step; absent ones read zero)
     const bool ok1 = oct0 + 1 < Cin8, ok8 = oct0 + 8 < Cin8, ok9 = oct0 + 9 < Cin8;
-    const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, in_bytes);
-    const int oy0 = strip * rps;
-    const int nrows = min(rps, g.OH - oy0);
+    const int oy0 = strip * g.rps;
+    const int nrows = min(g.rps, g.OH - oy0);
     const int iy0 = oy0 * S - g.ph;
     const int nq = (nrows - 1) * S + 3;  // input rows this strip reads
     typedef v2i b_t[CK == 32 ? 1 : 2 * KST];
     auto issue = [&](int j, b_t (&dst)[NG]) {  // j: input row of the walk
         const int iy = iy0 + j;
         const bool ok = iy >= 0 && iy < g.H && j < nq;  // wave-uniform
-        const unsigned s_row = (unsigned)__builtin_amdgcn_readfirstlane((int)(ok ? s_in + (unsigned)(iy * g.W) * 8u : 0u));
+        // (an absent row through an empty descriptor: with its offset beyond the buffer instead the compiler branched around each load)
+        const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, ok ? g.in_bytes : 0u);
+        const unsigned s_row = (unsigned)__builtin_amdgcn_readfirstlane((int)(s_in + (unsigned)(iy * g.W) * 8u));
 #pragma unroll
         for (int p = 0; p < NG; ++p) {
-            const int vo = (int)(ok ? v_in[p] : DW_OOB);
+            const int vo = (int)v_in[p];
             dst[p][0] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, vo, (int)s_row, 0));
             if constexpr (CK != 32) {
                 dst[p][1] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, ok1 ? vo : (int)DW_OOB, (int)(s_row + HW8), 0));
@@ -158,6 +164,22 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
 #pragma unroll
     for (int j = 0; j < PF; ++j) issue(j, ld[j]);
 
+    // The padding slots of every line: pixels -2, -1 and 16 NG .. 64 NCH + 5 (the pixels from W to 16 NG - 1 are written as zeros
+    // with every row). Of narrow lines most are padding: all of it is cleared, 16 bytes a lane and store, without index arithmetic.
+    if constexpr (NG <= 2) {
+        static_assert(2 * OCT % 16 == 0, "whole 16-byte stores");
+#pragma unroll
+        for (int i = 0; i < 2 * OCT / 16; i += 64)
+            if (i + 64 <= 2 * OCT / 16 || i + lane < 2 * OCT / 16) *reinterpret_cast<v4i*>(lds + (i + lane) * 16) = v4i{0, 0, 0, 0};
+    } else {
+        constexpr int PADS = 64 * NCH + 8 - 16 * NG;
+        for (int i = lane; i < PADS * RL * 2; i += 64) {
+            const int line = i / PADS, k = i % PADS;
+            const int slot = k < 2 ? k : 16 * NG + k;
+            *reinterpret_cast<v2i*>(lds + (line / RL) * OCT + (line % RL) * LINE + slot * 8) = v2i{0, 0};
+        }
+    }
+
     v4i si[2][T], bi[2][T], so[2][T];
     unsigned qh[2][T][2] = {};
 #pragma unroll
@@ -186,7 +208,7 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
         v_out[c] = ox < g.OW ? (unsigned)ox * 8u + (S == 1 ? 0u : (unsigned)(q & 1) * 4u) : DW_OOB;
     }
     const unsigned s_out = (unsigned)(img * C8 + 2 * pr) * OHW * 8u, row_bytes = (unsigned)g.OW * 8u;
-    const __amdgpu_buffer_rsrc_t rout = dw_rsrc(out, out_bytes);
+    const __amdgpu_buffer_rsrc_t rout = dw_rsrc(out, g.out_bytes);
 
     v4i cur[2][NCH][T];
     auto epilogue_store = [&](int r) {  // output row r of the strip, from cur
@@ -320,10 +342,11 @@ hipError_t run_conv_xdw(const int8_t* x, const int8_t* wx, const int8_t* wa, voi
     const unsigned lds_bytes = (unsigned)wpb * 2u * (4u * (64u * nch + 8u) * 8u + 128u);
     const unsigned in_bytes = (unsigned)((size_t)gx.N * gx.C * gx.H * gx.W);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW);
+    const XdwArgs xa = {g.H, g.W, g.OH, g.OW, g.C, gx.C, g.ph, n_strips, rps, in_bytes, out_bytes, DwGrid::of(grid.x, grid.y, (unsigned)(g.C / 16), wpb)};
     const bool nn = epi_d == EPI_I8_P8_NONNEG;
 #define OHIP_XDW_L(S_, NN_, G_, CK_)                                                                                              \
     hipLaunchKernelGGL((conv_xdw_kernel<S_, NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8, NN_, G_, CK_>), grid, block, lds_bytes, stream, x, wx, wa, \
-                       out, g, gx.C, epx, ep, DwGrid::of(grid.x, grid.y, (unsigned)(g.C / 16), wpb), n_strips, rps, in_bytes, out_bytes)
+                       out, xa, EpiArgs<NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8>::of(epx), EpiArgs<NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8>::of(ep))
 #define OHIP_XDW_G(S_, NN_, CK_)                 \
     do {                                         \
         switch (NG) {                            \
