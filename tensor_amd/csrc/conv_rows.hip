@@ -16,9 +16,11 @@
 // byte offsets added to its pixel's address. The channel octets come in stages of at most 8; octet planes are 64 bytes off a
 // multiple of 128, which puts the pairs of neighbouring lane quarters into different halves of the banks.
 //
-// Measured, us per launch before / after: 256 -> 256 3x3 in 8 groups @28x28 b64 22.6 / 13.9; 384 -> 64 5x5 in 4 groups
+// Measured, us per launch before / after: 256 -> 256 3x3 in 8 groups @28x28 b64 22.6 / 13.2; 384 -> 64 5x5 in 4 groups
 // @67x67 b9 73 / 20; 272 -> 24 3x3 @157x157 b16 129 / 60; 24 -> 32 5x5 @162x162 b13 51.5 / 16.8; 16 -> 16 3x3 dilated
 // @204x204 b55 107 / 56; 8 -> 344 5x5 @113x113 b24 96 / 62; from fp32 128 -> 64 5x5 in 8 groups @75x89 b32 48.6 / 28.9.
+// The octets of a stage are requested together and the weights of a step ahead without a condition: with a branch on the parity of
+// the width at each load the compiler waited for every octet before the next. 256 -> 256 in 8 groups @28x28 b64 15.0 -> 14.2 per call.
 // What is left above the floor is the chain of a tile (rows in, barrier, steps, stores), which three or four workgroups per
 // compute unit hide in part; keeping eight octets or four weight steps in flight instead cost registers and was slower.
 #include "common.hpp"
@@ -72,10 +74,11 @@ static int rows_steps(int C, int taps) {
 
 template <int FM, int FN, int EPI, bool INF>
 __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
-                                                           void* __restrict__ out, RowsArgs ra, Epilogue ep) {
+                                                           void* __restrict__ out, RowsArgs ra, EpiArgs<EPI> ea) {
     constexpr int OOB = (int)0x80000000;  // beyond any buffer here (below 2 GiB)
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     const ConvGeom& g = ra.g;
+    Epilogue ep = ea.epilogue();
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, p = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int pt = blockIdx.x;
@@ -171,7 +174,10 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
         // 256 / pairs threads each
         const int pairs = rows * ra.VW2, sub = pairs > 128 ? 1 : 256 / pairs;
         const int oct0 = sub == 1 ? 0 : tid / pairs;
-        if (oct0 < sub) {
+        // (two walks, not a choice per load: behind loads on two branches the compiler waited for each octet before it requested the
+        // next, four memory latencies in a row)
+        auto stage_rows = [&](auto even_c) {
+            constexpr bool EVEN = decltype(even_c)::value;
             for (int pos = tid - oct0 * pairs; pos < pairs; pos += 256) {
                 const int row = (int)div_by((unsigned)pos, ra.vw), c0 = 2 * (pos - row * ra.VW2);
                 const v2i rt = row_tab[row];
@@ -192,7 +198,7 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
                             f[u][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0 + 16, 0, 0));
                             f[u][2] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1, 0, 0));
                             f[u][3] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1 + 16, 0, 0));
-                        } else if (even) {
+                        } else if constexpr (EVEN) {
                             v[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, 0, 0));
                         } else {
                             const v2i l = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a0, 0, 0));
@@ -200,6 +206,12 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
                             v[u] = v4i{l[0], l[1], h[0], h[1]};
                         }
                         so += sub * HW8 * INS;
+                    }
+                    // (all of them are requested here: the compiler would move the last one behind the condition of its write)
+#pragma unroll
+                    for (int u = 0; u < UN; ++u) {
+                        if constexpr (INF) asm volatile("" : "+v"(f[u][0]), "+v"(f[u][1]), "+v"(f[u][2]), "+v"(f[u][3]));
+                        else asm volatile("" : "+v"(v[u]));
                     }
 #pragma unroll
                     for (int u = 0; u < UN; ++u) {
@@ -211,6 +223,11 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
                     at += UN * sub * ra.plane;
                 }
             }
+        };
+        if (oct0 < sub) {
+            if constexpr (INF) stage_rows(std::true_type{});  // (reads values, not pixel pairs)
+            else if (even) stage_rows(std::true_type{});
+            else stage_rows(std::false_type{});
         }
         __syncthreads();
         // one block of output channels per pass over the stage; several only when there is one stage
@@ -235,13 +252,29 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
 #pragma unroll
                     for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(aa[i], b[j], acc[i][j], 0, 0, 0);
             };
-            for (int s = 0; s < steps; s += D) {
+            // No request is conditional where there are registers for it: behind one every load is waited for. The last step's weights
+            // are requested once more then. (Four row tiles: 0 to 3 % slower that way.)
+            if constexpr (FM == 2) {
+                int s = 0;
+                for (; s + D <= steps; s += D) {
 #pragma unroll
-                for (int d = 0; d < D; ++d)
-                    if (s + d < steps) {
-                        if (s + d + D - 1 < steps) load_a(a[(d + D - 1) % D], step0 + s + d + D - 1);
+                    for (int d = 0; d < D; ++d) {
+                        load_a(a[(d + D - 1) % D], step0 + min(s + d + D - 1, steps - 1));
                         multiply(s + d, a[d]);
                     }
+                }
+#pragma unroll
+                for (int d = 0; d + 1 < D; ++d)
+                    if (s + d < steps) multiply(s + d, a[d]);
+            } else {
+                for (int s = 0; s < steps; s += D) {
+#pragma unroll
+                    for (int d = 0; d < D; ++d)
+                        if (s + d < steps) {
+                            if (s + d + D - 1 < steps) load_a(a[(d + D - 1) % D], step0 + s + d + D - 1);
+                            multiply(s + d, a[d]);
+                        }
+                }
             }
             if (c + 1 < ra.stages) break;
             // ---- epilogue of the block -------------------------------------------------------------------------------------------
@@ -383,7 +416,9 @@ namespace {
 // runs as many of them one after the other as its workgroups do not fit side by side; per workgroup of the busiest compute unit
 // comes what they share: steps, staged places (pixel pairs of a thread) and row blocks; per launch the megabytes in and out. With
 // a stride the lanes of a pixel read lie on every other 8 bytes, and a step costs 1 + strided of what it does else. Fitted to 3000
-// drawn layers (k 3 and 5, 8..512 channels, 600..2.5 million pixels): median error 4 to 7 %, 9 in 10 below 12 to 18 %.
+// drawn layers (k 3 and 5, 8..512 channels, 600..2.5 million pixels): median error 4 to 7 %, 9 in 10 below 12 to 18 %. (What a tile
+// takes was scaled when the requests were put together: two row tiles 0.95 from int8 and 0.975 from fp32 of 67 and 23 layers, four row
+// tiles from fp32 1.035.)
 struct RowsCost {
     float start, step, stage, cu_step, cu_place, cu_block, strided, in_mb, out_mb;
 };
@@ -392,10 +427,10 @@ struct RowsConfig {
     RowsCost i8, f32;
 };
 constexpr RowsConfig kRowsConfigs[] = {
-    {2, 2, 5, {2.648f, 0.103f, 1.02f, 0.031f, 0.037f, 0.31f, 0.504f, 0.028f, 0.084f}, {2.228f, 0.126f, 1.373f, 0.027f, 0.133f, 0.252f, 0.858f, 0.053f, 0.097f}},
-    {2, 4, 4, {2.918f, 0.188f, 1.113f, 0.029f, 0.055f, 0.494f, 0.436f, 0.037f, 0.088f}, {2.53f, 0.26f, 1.306f, 0.f, 0.176f, 0.456f, 0.535f, 0.064f, 0.095f}},
-    {4, 2, 4, {2.723f, 0.12f, 1.003f, 0.072f, 0.043f, 0.458f, 0.366f, 0.f, 0.105f}, {2.446f, 0.181f, 1.174f, 0.056f, 0.147f, 0.355f, 0.627f, 0.045f, 0.112f}},
-    {4, 4, 3, {3.078f, 0.24f, 1.033f, 0.055f, 0.067f, 0.789f, 0.352f, 0.f, 0.115f}, {2.79f, 0.35f, 1.117f, 0.f, 0.21f, 0.701f, 0.375f, 0.049f, 0.121f}},
+    {2, 2, 5, {2.648f, 0.098f, 0.969f, 0.029f, 0.035f, 0.294f, 0.504f, 0.028f, 0.084f}, {2.228f, 0.123f, 1.339f, 0.026f, 0.13f, 0.246f, 0.858f, 0.053f, 0.097f}},
+    {2, 4, 4, {2.918f, 0.179f, 1.057f, 0.028f, 0.052f, 0.469f, 0.436f, 0.037f, 0.088f}, {2.53f, 0.254f, 1.273f, 0.f, 0.172f, 0.445f, 0.535f, 0.064f, 0.095f}},
+    {4, 2, 4, {2.723f, 0.12f, 1.003f, 0.072f, 0.043f, 0.458f, 0.366f, 0.f, 0.105f}, {2.446f, 0.187f, 1.215f, 0.058f, 0.152f, 0.367f, 0.627f, 0.045f, 0.112f}},
+    {4, 4, 3, {3.078f, 0.24f, 1.033f, 0.055f, 0.067f, 0.789f, 0.352f, 0.f, 0.115f}, {2.79f, 0.362f, 1.156f, 0.f, 0.217f, 0.726f, 0.375f, 0.049f, 0.121f}},
 };
 constexpr int kRowsConfigCount = (int)(sizeof(kRowsConfigs) / sizeof(kRowsConfigs[0]));
 }  // namespace
@@ -447,11 +482,11 @@ hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out
 #define OHIP_ROWS2(I_, FM_, FN_, E_)                                                                                         \
     if (config == I_ && epi == E_) {                                                                                         \
         if (!f32in) {                                                                                                        \
-            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, false>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, ep); \
+            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, false>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, EpiArgs<E_>::of(ep)); \
             return hipGetLastError();                                                                                        \
         }                                                                                                                    \
         if constexpr (E_ != EPI_GENERIC) {                                                                                   \
-            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, true>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, ep); \
+            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, true>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, EpiArgs<E_>::of(ep)); \
             return hipGetLastError();                                                                                        \
         }                                                                                                                    \
     }
