@@ -185,6 +185,8 @@ using JoinParam = typename JoinOf<EPI>::Type;
 
 // What a kernel instance reads of Epilogue, as its argument: 32 to 56 bytes instead of 112. A launch costs the host 0.1 us more for
 // every 32 bytes of arguments.
+// (A kernel's parameter type names an instance by its template argument, not by an expression of the EPI_ constants: their enum has no
+// name, and the host's and the device's symbols would number it differently.)
 struct EpiBase {
     const float *scale_in, *bias;
     float act_p0, act_lo, act_hi;
