@@ -1592,8 +1592,8 @@ int otter_hip_global_avgpool(const float* src, int src_layout, int n, int c, int
 
 // ---- a layer and the Concat -> ChannelShuffle(2), or the sum with a Concat, behind it ----------------------------------
 
-// The kernels that carry these epilogues, for an int8 Byte8 input: conv_tap_kernel and the implicit-GEMM kernel, as the
-// plain layer would choose between them. The other families' layers (depthwise, LDS-halo, streamed) stay two launches.
+// The kernels that carry these epilogues, for an int8 Byte8 input: the pointwise register kernels, conv_tap_kernel and the
+// implicit-GEMM kernel, as the plain layer would choose between them. The other families' layers (depthwise, LDS-halo, streamed) stay two launches.
 static AltKernel join_kernel(const otter_hip_conv* h, int in_layout, const ConvGeom& g, const Epilogue& ep, int* config, bool* ok) {
     *ok = false;
     if (in_layout != OTTER_HIP_I8_P8 || h->d.out_kind != OTTER_HIP_OUT_F32 || h->c_pad || g.groups != 1 || g.K % 8) return ALT_NONE;
@@ -1644,13 +1644,8 @@ int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* h, const void* in, in
     if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_shuffle: empty output");
     if ((size_t)n * g.C * in_h * in_w >= (1ull << 31) || (size_t)n * g.K * 2 * g.OH * g.OW >= (1ull << 31))
         return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: tensor exceeds 2^31 elements");
-    Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
-    int config;
-    bool ok;
-    const AltKernel alt = join_kernel(h, in_layout, g, ep, &config, &ok);
-    if (!ok) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: not a single launch (otter_hip_conv_join_launches)");
-    if (n == 0) return OTTER_HIP_OK;
     const size_t half = (size_t)g.K * g.OH * g.OW;  // elements of one half of one image
+    Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
     JoinArgs ja;
     ep.join = &ja;
     ja.other = other, ja.other_pack = layout_pack(other_layout), ja.other_odd = other_odd != 0;
@@ -1659,6 +1654,11 @@ int otter_hip_conv_forward_shuffle(const otter_hip_conv_t* h, const void* in, in
     ja.sh_out0 = first_half, ja.sh_q0 = first_half_q;
     ja.sh_out1 = joined ? (first_half ? first_half + half : nullptr) : second_half;
     ja.sh_q1 = joined ? (first_half_q ? first_half_q + half : nullptr) : second_half_q;
+    int config;
+    bool ok;
+    const AltKernel alt = join_kernel(h, in_layout, g, ep, &config, &ok);  // (with the join: its blobs count in a kernel's limits)
+    if (!ok) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_shuffle: not a single launch (otter_hip_conv_join_launches)");
+    if (n == 0) return OTTER_HIP_OK;
     return join_run(h, in, nullptr, g, ep, alt, config, (hipStream_t)stream_);
 }
 
@@ -1682,17 +1682,17 @@ int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* h, const void
     if ((size_t)n * g.C * in_h * in_w >= (1ull << 31) || (size_t)n * g.K * g.OH * g.OW >= (1ull << 31))
         return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_residual_concat: tensor exceeds 2^31 elements");
     Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
+    JoinArgs ja;
+    ep.join = &ja;
+    ep.residual = part0, ja.residual1 = part1, ja.res_split = part0_channels;
+    ja.res_pack0 = layout_pack(part0_layout), ja.res_pack1 = layout_pack(part1_layout);
+    ep.twin = out_q, ep.twin_scale = q_scale, ep.twin_half = q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     int config;
     bool ok;
     const AltKernel alt = join_kernel(h, in_layout, g, ep, &config, &ok);
     if (!ok)
         return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_residual_concat: not a single launch (otter_hip_conv_join_launches)");
     if (n == 0) return OTTER_HIP_OK;
-    JoinArgs ja;
-    ep.join = &ja;
-    ep.residual = part0, ja.residual1 = part1, ja.res_split = part0_channels;
-    ja.res_pack0 = layout_pack(part0_layout), ja.res_pack1 = layout_pack(part1_layout);
-    ep.twin = out_q, ep.twin_scale = q_scale, ep.twin_half = q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     return join_run(h, in, out, g, ep, alt, config, (hipStream_t)stream_);
 }
 

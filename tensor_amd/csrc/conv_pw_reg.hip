@@ -500,8 +500,9 @@ bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep) {
     const int epi = pw_reg_epilogue(ep, g.K);
     if (epi == EPI_GENERIC || ((ep.twin != nullptr || ep.join != nullptr) && g.K % 8)) return false;
     const size_t px = (size_t)g.N * g.H * g.W;
-    // 32-bit byte offsets into every blob
-    return px * g.C < ((size_t)1 << 31) && px * g.K * (epi == EPI_F32_SHUFFLE ? 8 : layout_elem_bytes(ep.out_layout)) < ((size_t)1 << 31);
+    // 32-bit byte offsets into every blob; a shuffled result that is one blob has twice the layer's channels
+    const size_t joined = epi == EPI_F32_SHUFFLE && ep.join->sh_image > (size_t)g.K * g.H * g.W ? 2 : 1;
+    return px * g.C < ((size_t)1 << 31) && px * g.K * joined * layout_elem_bytes(ep.out_layout) < ((size_t)1 << 31);
 }
 
 template <int FN, int CG, int EPI>

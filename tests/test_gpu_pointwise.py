@@ -96,3 +96,28 @@ def test_a_scale_per_output_channel_stays_with_the_other_kernels(hip):
                     out_scale=list(rng.uniform(5, 9, 16)), out_kind=capi.OUT_I8)
     assert conv.launch_choice(capi.I8_P8, 1, 7, 7, capi.I8_P8)[0] != 10
     conv.close()
+
+
+@pytest.mark.parametrize("C", [72, 264])
+@pytest.mark.parametrize("joined", [True, False])
+def test_shuffle_of_a_result_beyond_32_bit_offsets(hip, C, joined):
+    """2^28 values of the layer's own: the joined blob is 2 GiB, past the register kernel's offsets, each half by itself is not. What
+    otter_hip_conv_join_launches promises holds for both."""
+    torch = hip.torch
+    K, N, H, W = 64, 2, 1449, 1449
+    rng = np.random.default_rng(C)
+    conv = _layer(hip, rng, C, K, 1, False)
+    gen = torch.Generator(device=hip.device)
+    gen.manual_seed(C)
+    x = torch.randint(-127, 128, (N * C * H * W,), generator=gen, device=hip.device, dtype=torch.int8)
+    other = torch.randn(N * K * H * W, generator=gen, device=hip.device)
+    assert N * K * H * W * 8 >= 1 << 31 > N * K * H * W * 4
+    assert conv.join_launches(capi.I8_P8, N, H, W) == 1
+    got = conv.forward_shuffle(x, N, H, W, other, capi.F32_P8, False, joined, 9.0)
+    conv.set_tile(-4, 0)
+    want = conv.forward_shuffle(x, N, H, W, other, capi.F32_P8, False, joined, 9.0)
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    conv.close()
