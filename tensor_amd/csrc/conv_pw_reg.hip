@@ -500,6 +500,7 @@ bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep) {
     const int epi = pw_reg_epilogue(ep, g.K);
     if (epi == EPI_GENERIC || ((ep.twin != nullptr || ep.join != nullptr) && g.K % 8)) return false;
     const size_t px = (size_t)g.N * g.H * g.W;
+    if ((size_t)igemm_channel_groups(g.C) * igemm_padded_rows(g.K) * 64 >= ((size_t)1 << 31)) return false;  // (the packed weights)
     // 32-bit byte offsets into every blob; a shuffled result that is one blob has twice the layer's channels
     const size_t joined = epi == EPI_F32_SHUFFLE && ep.join->sh_image > (size_t)g.K * g.H * g.W ? 2 : 1;
     return px * g.C < ((size_t)1 << 31) && px * g.K * joined * layout_elem_bytes(ep.out_layout) < ((size_t)1 << 31);
@@ -577,6 +578,7 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
     const bool split = force ? (force & 64) != 0 : steps > PW_REG_STEPS;
     const bool wide = split || epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG;  // (registers)
     conv_pw_reg_plan(g, split, wide ? 4 : 2, layout_elem_bytes(ep.out_layout) == 4, &fn, &per);
+    per = std::max(per, (pairs + 65534) / 65535);  // (slices are grid.y)
     if (force) fn = force & 7, per = force >> 7;
     if ((fn != 1 && fn != 2 && !(fn == 4 && wide)) || per < 1 || (split ? steps < 2 : steps > PW_REG_STEPS)) return hipErrorInvalidValue;
     per = std::min(per, pairs);

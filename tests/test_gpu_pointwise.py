@@ -121,3 +121,14 @@ def test_shuffle_of_a_result_beyond_32_bit_offsets(hip, C, joined):
         if a is not None:
             assert torch.equal(a.view(torch.int32), b.view(torch.int32))
     conv.close()
+
+
+def test_more_channel_pairs_than_a_grid_dimension_holds(hip):
+    rng = np.random.default_rng(9)
+    C, K, N, H, W = 8, 32 * 65536 + 64, 1, 1, 3
+    conv = _layer(hip, rng, C, K, 1, True)
+    x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
+    got = conv.forward(x, capi.I8_P8, N, H, W)
+    conv.set_tile(-4, 0)
+    _same(hip, [got], [conv.forward(x, capi.I8_P8, N, H, W)])
+    conv.close()
