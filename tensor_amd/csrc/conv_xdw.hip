@@ -4,6 +4,7 @@
 #include "common.hpp"
 #include "conv_dw_common.hpp"
 #include "conv_igemm.hpp"
+#include "xdw_row.hpp"
 
 namespace ohip {
 
@@ -86,6 +87,7 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
     for (int p = 0; p < NG; ++p) v_in[p] = (16 * p + n < g.W && oct0 < Cin8) ? (unsigned)oct0 * HW8 + (unsigned)(16 * p + n) * 8u : DW_OOB;
     // (the other octets of this lane's reduction bytes: + 1, and + 8, + 9 in the second step; absent ones read zero)
     const bool ok1 = oct0 + 1 < Cin8, ok8 = oct0 + 8 < Cin8, ok9 = oct0 + 9 < Cin8;
+    const XdwOctets octets = xdw_octets(HW8, Cin8);
     const int oy0 = strip * g.rps;
     const int nrows = min(g.rps, g.OH - oy0);
     const int iy0 = oy0 * S - g.ph;
@@ -94,17 +96,17 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
     auto issue = [&](int j, b_t (&dst)[NG]) {  // j: input row of the walk
         const int iy = iy0 + j;
         const bool ok = iy >= 0 && iy < g.H && j < nq;  // wave-uniform
-        // (an absent row through an empty descriptor: with its offset beyond the buffer instead the compiler branched around each load)
-        const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, ok ? g.in_bytes : 0u);
-        const unsigned s_row = (unsigned)__builtin_amdgcn_readfirstlane((int)(s_in + (unsigned)(iy * g.W) * 8u));
+        // (an absent row through an empty descriptor: with a lane offset beyond the buffer instead the compiler branched around each load)
+        const XdwRow r = xdw_row(ok, g.in_bytes, (unsigned)__builtin_amdgcn_readfirstlane((int)(s_in + (unsigned)(iy * g.W) * 8u)), octets);
+        const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, r.bytes);
 #pragma unroll
         for (int p = 0; p < NG; ++p) {
             const int vo = (int)v_in[p];
-            dst[p][0] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, vo, (int)s_row, 0));
+            dst[p][0] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, vo, (int)r.at, 0));
             if constexpr (CK != 32) {
-                dst[p][1] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, ok1 ? vo : (int)DW_OOB, (int)(s_row + HW8), 0));
-                dst[p][2] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, ok8 ? vo : (int)DW_OOB, (int)(s_row + 8u * HW8), 0));
-                dst[p][3] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, ok9 ? vo : (int)DW_OOB, (int)(s_row + 9u * HW8), 0));
+                dst[p][1] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, ok1 ? vo : (int)DW_OOB, (int)r.at1, 0));
+                dst[p][2] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, ok8 ? vo : (int)DW_OOB, (int)r.at8, 0));
+                dst[p][3] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, ok9 ? vo : (int)DW_OOB, (int)r.at9, 0));
             }
         }
     };
