@@ -24,6 +24,7 @@
 #include "common.hpp"
 #include "conv_dw_common.hpp"
 #include "conv_igemm.hpp"
+#include "dw_strips.hpp"
 
 namespace ohip {
 
@@ -642,29 +643,6 @@ bool dw_mfma_applicable(const ConvGeom& g, const Epilogue& ep, int epi, bool sca
     return in_bytes < ((size_t)1 << 31) && out_bytes < ((size_t)1 << 31);  // 32-bit buffer offsets
 }
 
-// Output rows of a strip. Its wave takes `row` microseconds per row whatever else runs, and as much as `extra` rows more where the
-// strip is longer than the ring of input rows holds; a SIMD with several waves takes their instructions one after the other, and up
-// to six of them the fullest SIMD (ceil) counts. columns: waves side by side at one strip per image. Fitted to 260 drawn layers of
-// 16 .. 960 channels, 7x7 to 208x208, 1 .. 64 images: the chosen height is 0.5 % slower than the best on average, 9 % at worst.
-// With the rule and kernel before (the tallest strips that leave 2048 waves, 8 / stride rows at least; seven divisions per wave)
-// 128 channels 5x5 LeakyReLU @13x13 x16 took 4.4 us (now 3.1), 384 @14x14 x1 3.6 (2.8), 88 @52x52 x16 6.0 (5.1).
-static int dw_strip_rows(const ConvGeom& g, int epi, float columns) {
-    const float row = 0.139f * (g.sh == 2 ? 0.624f : 1.f) * (g.kh == 5 ? 0.763f : 1.f) *
-                      (epi == EPI_I8_P8_NONNEG ? 0.89f : epi == EPI_I8_P8 ? 1.f : 0.596f);
-    const int step = 8 / g.sh, ring = (8 - g.kh) / g.sh + 1;  // output rows of a step, and those that the first input rows make
-    float best = __builtin_inff();
-    int rows = g.OH;
-    for (int r = g.OH;;) {
-        const int strips = (g.OH + r - 1) / r;
-        const float extra = r <= ring ? 0.f : r % step ? 4.258f : 2.865f, walk = row * ((float)r + extra);
-        const float m = columns * (float)strips / 1024.f, full = m <= 6.f ? ceilf(m) : m + 0.311f;
-        const float t = 0.788f * walk + (0.88f * fmaxf(m, 1.f) + 0.443f * full) * (0.306f + 0.55f * walk);
-        if (t < best) best = t, rows = r;
-        if (r == 1) return rows;
-        r = std::min(r - 1, (g.OH + strips) / (strips + 1));  // the height of the next number of strips
-    }
-}
-
 // strip_blocks: 0 = automatic, > 0: steps of 8 / stride output rows of a strip, < 0: rows of it
 hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const ConvGeom& g, const Epilogue& ep, int epi,
                             int strip_blocks, hipStream_t stream) {
@@ -684,7 +662,8 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     const int U = 8 / g.sh;
     const int rps = strip_blocks > 0   ? std::min(strip_blocks, (g.OH + U - 1) / U) * U
                     : strip_blocks < 0 ? std::min(-strip_blocks, g.OH)
-                                       : dw_strip_rows(g, epi, (float)(col_chunks * groups));
+                                       : DwStrips(g.OH, g.sh, g.kh, epi == EPI_I8_P8_NONNEG ? 1 : epi == EPI_I8_P8 ? 0 : 2,
+                                                  (float)(col_chunks * groups)).choose();
     const int n_strips = (g.OH + rps - 1) / rps;
     // a workgroup is one strip: with two and four strips a workgroup, and shares of LDS reserved to even them out over the compute
     // units, 140 drawn layers were 2 % and 5 % slower at their best strip height
