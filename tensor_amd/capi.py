@@ -81,7 +81,8 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_chain_forward", "otter_hip_conv_chain_status", "otter_hip_conv_chain_launches",
            "otter_hip_conv_chain_last_launches", "otter_hip_conv_chain_clock_mhz",
            "otter_hip_conv_chain_set_min_tiles", "otter_hip_conv_block_launches", "otter_hip_conv_block_workspace_bytes",
-           "otter_hip_conv_block_layout_workspace_bytes",
+           "otter_hip_conv_block_layout_workspace_bytes", "otter_hip_conv_block_fastest", "otter_hip_conv_block_form_workspace_bytes",
+           "otter_hip_conv_block_forward_form", "otter_hip_conv_forward_making",
            "otter_hip_conv_block_forward", "otter_hip_conv_block_set_plan", "otter_hip_conv_block_set_always", "otter_hip_conv_block_set_pair",
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
            "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
@@ -121,6 +122,7 @@ class Library:
         L.otter_hip_conv_chain_workspace_bytes.restype = C.c_size_t
         L.otter_hip_conv_block_workspace_bytes.restype = C.c_size_t
         L.otter_hip_conv_block_layout_workspace_bytes.restype = C.c_size_t
+        L.otter_hip_conv_block_form_workspace_bytes.restype = C.c_size_t
         L.otter_hip_conv_avgpool_workspace_bytes.restype = C.c_size_t
         self.device = torch.device("cuda", device)
         self.native, self.device_index = load_binding(), device
@@ -294,6 +296,27 @@ class Library:
         out_layout = F32_P4 if project.out_kind == OUT_F32 else I8_P8
         return self.native.conv_block(expand._hp, dw._hp, project._hp, project.K, out_layout, x, n, h, w, residual, q_scale,
                                       q_round_mode, out, q, workspace, self.device_index)
+
+    def conv_block_fastest(self, expand, dw, project, n, h, w):
+        """otter_hip_conv_block_fastest: 1, 2 or 3 launches, the fastest form by the cost models."""
+        r = self.lib.otter_hip_conv_block_fastest(expand.h, dw.h, project.h, n, h, w)
+        self._check(min(r, 0))
+        return r
+
+    def conv_block_form(self, form, expand, dw, project, x, n, h, w, residual=None, q_scale=None, q_round_mode=ROUND_SSE, out_layout=None,
+                        workspace=None):
+        """conv_block in the form named: 1, 2 or 3 launches (otter_hip_conv_block_forward_form). Returns (out, q or None)."""
+        out_layout = (F32_P4 if project.out_kind == OUT_F32 else I8_P8) if out_layout is None else out_layout
+        oh, ow = project.out_hw(*dw.out_hw(*expand.out_hw(h, w)))
+        out = self.empty(n * project.K * oh * ow, layout_dtype(out_layout))
+        q = self.empty(n * project.K * oh * ow, np.int8) if q_scale is not None else None
+        if workspace is None:
+            workspace = self.empty(self.lib.otter_hip_conv_block_form_workspace_bytes(expand.h, dw.h, project.h, form, n, h, w), np.int8)
+        given = [self.ptr(t) if t is not None else None for t in (residual, out, q)]
+        self._check(self.lib.otter_hip_conv_block_forward_form(
+            expand.h, dw.h, project.h, form, self.ptr(x), n, h, w, given[0], given[1], out_layout, given[2], C.c_float(q_scale or 0.0),
+            q_round_mode, self.ptr(workspace) if workspace.numel() else None, C.c_size_t(workspace.numel()), self.stream()))
+        return out, q
 
     def conv_block_set_always(self, on):
         """otter_hip_conv_block_set_always: returns the previous setting."""
