@@ -693,7 +693,7 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 // set_tile(-8, tile), set_tile(-9, tile) and set_tile(-10, ...) force them.
 enum AltKernel { ALT_NONE, ALT_TAP, ALT_ROWS, ALT_PW_REG };
 static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, bool f32in, int family, bool fused, int* config) {
-    *config = h->force_tn;
+    *config = h->force_tm < 0 ? h->force_tn : 0;  // (tm == 0 forces nothing, whatever tn is)
     if (!f32in && (h->force_tm == 0 || h->force_tm == -10) && h->w_igemm && !h->c_pad && h->so_same && conv_pw_reg_applicable(g, ep))
         return ALT_PW_REG;
     const bool kxk = g.kh * g.kw > 1, tap = h->w_tap && conv_tap_supported(g, ep, f32in);

@@ -90,6 +90,23 @@ def test_sum_twin_and_joins(hip, C, K, N, H, W, act):
     conv.close()
 
 
+@pytest.mark.parametrize("C", [24, 264])
+def test_a_tile_of_no_launch_forces_nothing(hip, C):
+    """set_tile(0, tn) leaves every choice automatic, whatever tn is: below 128 it names no channel pairs, 321 a split reduction."""
+    rng = np.random.default_rng(C)
+    K, N, H, W = 40, 2, 9, 11
+    conv = _layer(hip, rng, C, K, 1, False)
+    x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
+    other = hip.to_device(rng.normal(0, 3, N * K * H * W).astype(np.float32))
+    want = conv.forward(x, capi.I8_P8, N, H, W), conv.forward_shuffle(x, N, H, W, other, capi.F32_P8, False, True, 9.0)
+    for tn in (1, 3, 1 | 64 | 2 << 7, 2 | 1 << 7):
+        conv.set_tile(0, tn)
+        assert conv.launch_choice(capi.I8_P8, N, H, W, conv.default_out_layout()) == (10, 0)
+        _same(hip, [conv.forward(x, capi.I8_P8, N, H, W)], [want[0]])
+        _same(hip, conv.forward_shuffle(x, N, H, W, other, capi.F32_P8, False, True, 9.0), want[1])
+    conv.close()
+
+
 def test_a_scale_per_output_channel_stays_with_the_other_kernels(hip):
     rng = np.random.default_rng(5)
     conv = hip.conv(wq=rng.integers(-127, 128, (16, 24, 1, 1)).astype(np.int8), scale_in=np.full(16, 1e-3, np.float32), in_scale=20.0,
