@@ -294,7 +294,7 @@ int otter_hip_conv_block_forward(const otter_hip_conv_t* expand, const otter_hip
 /* The same block in a form that the caller names: form = 1, 2 or 3 launches, refused where the block cannot run so.
  * otter_hip_conv_block_fastest names the fastest by cost models of the launches as they are (otter_hip_conv_block_launches goes on
  * giving the single launch to the blocks that it was the fastest form of before the layers by themselves became faster).
- * The result is the same, bit for bit. */
+ * The result is the same, bit for bit. otter_hip_conv_block_form_workspace_bytes is 0 for a form that is refused. */
 int otter_hip_conv_block_fastest(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise, const otter_hip_conv_t* project,
                                  int n, int in_h, int in_w);
 size_t otter_hip_conv_block_form_workspace_bytes(const otter_hip_conv_t* expand, const otter_hip_conv_t* depthwise,

@@ -1348,7 +1348,7 @@ size_t otter_hip_conv_block_form_workspace_bytes(const otter_hip_conv_t* e, cons
     if (!block_geoms(e, d, p, n, in_h, in_w, g)) return 0;
     int plan[6];
     if (form == 1) return block_single_takes(e, d, p, g, block_default_out_layout(p), plan) ? (size_t)plan[5] * sizeof(int) : 0;
-    return block_blob_bytes(g, nullptr);
+    return form == 3 || (form == 2 && block_pair_takes(e, d, g)) ? block_blob_bytes(g, nullptr) : 0;
 }
 
 size_t otter_hip_conv_block_workspace_bytes(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p,

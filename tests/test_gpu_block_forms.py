@@ -46,11 +46,16 @@ def test_every_form_from_its_reported_workspace(hip, cin, ce, cout, N, H, W, str
     q_scale = 19.0 if f32_out else None
     want, want_q = one_by_one(hip, layers, x, N, H, W, res, q_scale)
     assert hip.conv_block_fastest(*b, N, H, W) in forms
+
+    def reported(form):
+        return hip.lib.otter_hip_conv_block_form_workspace_bytes(*[c.h for c in b], form, N, H, W)
+
     for form in (1, 2, 3):
         if form not in forms:
+            assert reported(form) == 0, form
             refused(UNSUPPORTED, lambda: hip.conv_block_form(form, *b, x, N, H, W, residual=res, q_scale=q_scale))
             continue
-        need = hip.lib.otter_hip_conv_block_form_workspace_bytes(*[c.h for c in b], form, N, H, W)
+        need = reported(form)
         room = torch.full((need + 4096,), 85, dtype=torch.int8, device=hip.device)
         for _ in range(2):
             got, got_q = hip.conv_block_form(form, *b, x, N, H, W, residual=res, q_scale=q_scale, workspace=room[:need])
@@ -60,6 +65,7 @@ def test_every_form_from_its_reported_workspace(hip, cin, ce, cout, N, H, W, str
         if need:
             refused(INVALID, lambda: hip.conv_block_form(form, *b, x, N, H, W, residual=res, q_scale=q_scale, workspace=room[:need - 1]))
     for form in (0, 4):
+        assert reported(form) == 0, form
         refused(INVALID, lambda: hip.conv_block_form(form, *b, x, N, H, W, residual=res, q_scale=q_scale, workspace=room))
     for l in layers:
         l["conv"].close()
