@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
     typedef v2i b_t[CK == 32 ? 1 : 2 * KST];
     auto issue = [&](int j, b_t (&dst)[NG]) {  // j: input row of the walk
         const int iy = iy0 + j;
-        const bool ok = iy >= 0 && iy < g.H && j < nq;  // wave-uniform
+        const bool ok = (iy >= 0) & (iy < g.H) & (j < nq);  // wave-uniform (one selection of each value below, no branch around them)
         // (an absent row through an empty descriptor: with a lane offset beyond the buffer instead the compiler branched around each load)
         const XdwRow r = xdw_row(ok, g.in_bytes, (unsigned)__builtin_amdgcn_readfirstlane((int)(s_in + (unsigned)(iy * g.W) * 8u)), octets);
         const __amdgpu_buffer_rsrc_t rin = dw_rsrc(x, r.bytes);
