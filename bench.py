@@ -266,7 +266,8 @@ def build_c2(hip, capi, rng, int8_out=False):
               for i in range(n_dom)]
     ops = 2.0 * N * K * C * H * W
     tail = "requantize + ReLU -> int8" if int8_out else "dequantize + ReLU -> fp32"
-    i8_kernel = "conv_pw_stream_kernel" if conv.kernel_kind(capi.I8_P8, N, H, W, out_layout) == 5 else "conv_igemm_kernel"
+    i8_kernel = ("conv_pw_reg_kernel" if conv.launch_choice(capi.I8_P8, N, H, W, out_layout)[0] == 10 else
+                 "conv_pw_stream_kernel" if conv.kernel_kind(capi.I8_P8, N, H, W, out_layout) == 5 else "conv_igemm_kernel")
     return dict(name="c2i8" if int8_out else "c2", step=step, ops=ops, launches=1, dom_ops=ops, dom_fn_cold=dom_cold,
                 dom_bytes=dom_bytes, bound="hbm",
                 workload="int8 1x1 conv 256->512 @28x28 batch 32 (GEMM 512x25088x256), fp32 in -> quantize + conv + bias + "

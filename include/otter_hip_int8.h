@@ -352,8 +352,9 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * tm == -8: the launch of families 1 and 3 that reads both operands straight from memory and deals the reduction to the waves
  * of a workgroup, tn = 0..6 its tile. tm == -9 on a k x k layer: the launch of those families that stages input rows in LDS,
  * tn = 0..3 its tile. tm == -10 on a pointwise layer with an int8 blob: the launch that keeps its operands in registers wherever it
- * can run, tn = groups | 64 if the reduction is split among the waves of a workgroup | pairs << 7 forcing the 16-pixel groups a wave owns (1, 2, or 4 with at most 256 input channels and a result
- * without a sum, a twin or a shuffle) and the pairs of 16 output channels it walks (0 = automatic for both). */
+ * can run, tn = groups | split << 6 | pairs << 7 forcing the 16-pixel groups a wave owns (1, 2 or 4), whether the reduction is split
+ * among the waves of a workgroup (1: over 64 input channels; 0: at most 256, and four groups only for a result without a sum, a twin
+ * or a shuffle) and the pairs of 16 output channels a wave walks. tn = 0: all three automatic. */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 
 /* Test hook with no counterpart in the reference: which of the launches of its family a dense or grouped layer takes on a packed

@@ -1,4 +1,6 @@
-// Pointwise (1x1, stride 1) int8 convolution with every operand in registers: no LDS, no barrier, no loop over the reduction.
+// Pointwise (1x1, stride 1) int8 convolution with every operand in registers and no loop over the reduction. Up to 256 input channels
+// (conv_pw_reg_kernel) that is a wave's own work, without LDS or a barrier; up to 1024 (conv_pw_split_kernel) the four waves of a
+// workgroup share it, and their sums meet in LDS.
 //
 // The pointwise layers of a network are short: a wave's whole reduction is CG <= 4 matrix steps, and what their launches cost is
 // the instructions around those and the latency of the first loads. The implicit-GEMM kernel spends 750 to 1500 vector and 640 to
@@ -20,7 +22,6 @@
 #include <cmath>
 
 namespace ohip {
-
 
 namespace {
 
@@ -617,8 +618,8 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
 // Whole reductions (at most 256 channels): fitted to 150 drawn layers of 16 .. 384 channels, 49 to 800 000 pixels, 2.7 % above the
 // best measured split on average, 80 % of the time of the launches before (streamed, implicit GEMM, dealt reduction; the faster
 // by their cost models). Split reductions: 138 layers of 257 .. 960 channels, 2.3 % above the best, 85 % of the best of the
-// implicit-GEMM kernel and every tile of the dealt reduction. Where both can run: 257 .. 384 channels 5 % faster split, 193 .. 256 2 %
-// and up to 192 8 % slower.
+// implicit-GEMM kernel and every tile of the dealt reduction. The line between the two is at 256 channels (PW_REG_STEPS): 257 .. 384
+// channels, for which whole reductions were built then, are 5 % faster split, 193 .. 256 2 % and up to 192 8 % slower.
 void conv_pw_reg_plan(const ConvGeom& g, bool split, int max_groups, bool f32out, int* groups, int* per) {
     const int pairs = (g.K + 31) / 32, cg = igemm_channel_groups(g.C);
     const float px = (float)g.N * (float)g.H * (float)g.W;
