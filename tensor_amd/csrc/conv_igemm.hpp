@@ -49,6 +49,7 @@ hipError_t run_conv_pw_stream(const int8_t* x, const int8_t* wpk, const unsigned
 constexpr int PW_REG_STEPS = 4, PW_REG_STEPS_SPLIT = 16;
 bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep);
 void conv_pw_reg_plan(const ConvGeom& g, bool split, int max_groups, bool f32out, int* groups, int* per);
+void conv_pw_reg_plan_clamped(const ConvGeom& g, int* groups, int* per);
 hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* out, const ConvGeom& g, const Epilogue& ep, int force,
                            hipStream_t stream);
 

@@ -578,7 +578,8 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
     int fn = 1, per = 1;
     const bool split = force ? (force & 64) != 0 : steps > PW_REG_STEPS;
     const bool wide = split || epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG;  // (registers)
-    conv_pw_reg_plan(g, split, wide ? 4 : 2, layout_elem_bytes(ep.out_layout) == 4, &fn, &per);
+    if (epi == EPI_I8_P8_NONNEG && !split) conv_pw_reg_plan_clamped(g, &fn, &per);
+    else conv_pw_reg_plan(g, split, wide ? 4 : 2, layout_elem_bytes(ep.out_layout) == 4, &fn, &per);
     per = std::max(per, (pairs + 65534) / 65535);  // (slices are grid.y)
     if (force) fn = force & 7, per = force >> 7;
     if ((fn != 1 && fn != 2 && !(fn == 4 && wide)) || per < 1 || (split ? steps < 2 : steps > PW_REG_STEPS)) return hipErrorInvalidValue;
@@ -635,6 +636,34 @@ void conv_pw_reg_plan(const ConvGeom& g, bool split, int max_groups, bool f32out
         const float each = (split ? 0.017f * ta + 6.5f + 1.6f * f : 0.933f * ta + 0.404f * va) / 2300.f;
         const float t = (float)p * pair + (split ? 1.21f * f : 0.f) + waves * (float)slices * (once + (float)p * each);
         if (t < best) best = t, *groups = fn, *per = p;
+    }
+}
+
+// The same for a whole reduction with a clamped int8 result. Its requantization is two thirds of the others' instructions, so that a
+// wave should walk more pairs of more pixels: by the costs above such layers, which the streamed kernel used to take, were up to 1.26
+// times slower than there (16 -> 96 @112x112 x64 26.4 us, streamed 22.0; 256 -> 512 @28x28 x32 13.3, 11.9). Per pair a wave's latency,
+// per workgroup of a compute unit its share of the loads and instructions; of the last, incomplete round about half counts. Fitted to
+// 498 drawn layers of 8 .. 256 channels with all splits (median error 3 %): the split named is 1.2 % above the best one, 5.5 % before.
+// Against the streamed kernel over its own range, layers that were not fitted, of 2 million results or more, or of 200 .. 256 channels
+// and 20 000 pixels: 500 layers take 0.91 of its time, 9 % of them over 3 % more, 11 % at worst; 700 by the costs above 0.95, 22 % and
+// 22 %.
+void conv_pw_reg_plan_clamped(const ConvGeom& g, int* groups, int* per) {
+    const int pairs = (g.K + 31) / 32;
+    const float c = (float)igemm_channel_groups(g.C);
+    const long px = (long)g.N * g.H * g.W;
+    float best = __builtin_inff();
+    for (int fn = 1; fn <= 4; fn *= 2) {
+        const float f = (float)fn, pair = 0.066f + 0.083f * f + 0.02f * c, once = 0.017f + 0.065f * f * c, each = 0.1f + 0.059f * f + 0.049f * c;
+        const long tiles = (px + 64 * fn - 1) / (64 * fn);
+        // (slices of the pairs: the real optimum without rounds, and its neighbours)
+        const int near = std::clamp((int)(sqrtf(pair * (float)pairs * 256.f / ((float)tiles * once)) + 0.5f), 1, pairs);
+        for (int want = std::max(near - 1, 1); want <= std::min(near + 1, pairs); ++want) {
+            const int p = (pairs + want - 1) / want, slices = (pairs + p - 1) / p;
+            const long groups_all = tiles * slices;
+            const float share = (float)groups_all / 256.f, rounds = (float)((groups_all + 255) / 256);
+            const float t = (float)p * pair + 0.008f * f * c + (0.51f * share + 0.49f * rounds) * (once + (float)pairs / (float)slices * each);
+            if (t < best) best = t, *groups = fn, *per = p;
+        }
     }
 }
 
