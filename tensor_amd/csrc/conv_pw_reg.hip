@@ -578,7 +578,8 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
     int fn = 1, per = 1;
     const bool split = force ? (force & 64) != 0 : steps > PW_REG_STEPS;
     const bool wide = split || epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG;  // (registers)
-    if (epi == EPI_I8_P8_NONNEG && !split) conv_pw_reg_plan_clamped(g, &fn, &per);
+    constexpr long kClampedFrom = 4l << 20;  // results of a layer, see conv_pw_reg_plan_clamped
+    if (epi == EPI_I8_P8_NONNEG && !split && (long)pa.total_pix * g.K >= kClampedFrom) conv_pw_reg_plan_clamped(g, &fn, &per);
     else conv_pw_reg_plan(g, split, wide ? 4 : 2, layout_elem_bytes(ep.out_layout) == 4, &fn, &per);
     per = std::max(per, (pairs + 65534) / 65535);  // (slices are grid.y)
     if (force) fn = force & 7, per = force >> 7;
@@ -639,14 +640,15 @@ void conv_pw_reg_plan(const ConvGeom& g, bool split, int max_groups, bool f32out
     }
 }
 
-// The same for a whole reduction with a clamped int8 result. Its requantization is two thirds of the others' instructions, so that a
-// wave should walk more pairs of more pixels: by the costs above such layers, which the streamed kernel used to take, were up to 1.26
-// times slower than there (16 -> 96 @112x112 x64 26.4 us, streamed 22.0; 256 -> 512 @28x28 x32 13.3, 11.9). Per pair a wave's latency,
-// per workgroup of a compute unit its share of the loads and instructions; of the last, incomplete round about half counts. Fitted to
-// 498 drawn layers of 8 .. 256 channels with all splits (median error 3 %): the split named is 1.2 % above the best one, 5.5 % before.
-// Against the streamed kernel over its own range, layers that were not fitted, of 2 million results or more, or of 200 .. 256 channels
-// and 20 000 pixels: 500 layers take 0.91 of its time, 9 % of them over 3 % more, 11 % at worst; 700 by the costs above 0.95, 22 % and
-// 22 %.
+// The same for a whole reduction with a clamped int8 result and many of them. Its requantization is two thirds of the others'
+// instructions, so that a wave should walk more pairs of more pixels: by the costs above such layers, which the streamed kernel used to
+// take, were up to 1.26 times slower than there (16 -> 96 @112x112 x64 26.4 us, streamed 22.0, now 21.5; 256 -> 512 @28x28 x32 12.4 a
+// call, now 10.3). Per pair a wave's latency, per workgroup of a compute unit its share of the loads and instructions; of the last,
+// incomplete round about half counts. Fitted to 498 drawn layers of 8 .. 256 channels with all splits (median error 3 %): the split
+// named is 1.2 % above the best one, 5.5 % before. Against the streamed kernel over its own range, layers that were not fitted, of 2
+// million results or more, or of 200 .. 256 channels and 20 000 pixels: 500 layers take 0.91 of its time, 9 % of them over 3 % more, 11 %
+// at worst; 700 by the costs above 0.95, 22 % and 22 %. Below 4 million results the costs above lose to no launch of before; there these
+// are level (1.00 of the time over 200 drawn layers, 13 of them over 3 % slower), above 0.98, 0.95 and 0.95 at 4, 8 and 16 million.
 void conv_pw_reg_plan_clamped(const ConvGeom& g, int* groups, int* per) {
     const int pairs = (g.K + 31) / 32;
     const float c = (float)igemm_channel_groups(g.C);
