@@ -90,6 +90,27 @@ def test_sum_twin_and_joins(hip, C, K, N, H, W, act):
     conv.close()
 
 
+@pytest.mark.parametrize("C,K,N,H,W", [
+    (256, 512, 2, 64, 63),    # below 4 << 20 results
+    (256, 512, 2, 64, 64),    # that many
+    (136, 1048, 1, 61, 67),   # few pixels, more channel pairs than a wave walks, the last of one octet
+    (8, 8, 3, 421, 419),      # one channel pair, many pixels, the last group not full
+    (48, 72, 7, 97, 89),
+    (256, 4112, 1, 33, 31),
+])
+@pytest.mark.parametrize("act", [1, 3])
+def test_split_of_many_clamped_results(hip, C, K, N, H, W, act):
+    """The split that clamped int8 results have from 4 << 20 of them on."""
+    rng = np.random.default_rng(C + K + W)
+    x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
+    conv = _layer(hip, rng, C, K, act, True)
+    assert conv.launch_choice(capi.I8_P8, N, H, W, capi.I8_P8) == (10, 0)
+    got = conv.forward(x, capi.I8_P8, N, H, W)
+    conv.set_tile(-4, 0)
+    _same(hip, [got], [conv.forward(x, capi.I8_P8, N, H, W)])
+    conv.close()
+
+
 @pytest.mark.parametrize("C", [24, 264])
 def test_a_tile_of_no_launch_forces_nothing(hip, C):
     """set_tile(0, tn) leaves every choice automatic, whatever tn is: below 128 it names no channel pairs, 321 a split reduction."""
