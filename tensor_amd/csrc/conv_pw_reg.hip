@@ -3,9 +3,9 @@
 // workgroup share it, and their sums meet in LDS.
 //
 // The pointwise layers of a network are short: a wave's whole reduction is CG <= 4 matrix steps, and what their launches cost is
-// the instructions around those and the latency of the first loads. The implicit-GEMM kernel spends 750 to 1500 vector and 640 to
-// 1700 scalar instructions per wave on 16 results a lane (its tap and column arithmetic, divisions, the way through LDS, 64-bit
-// addresses), where the requantization itself is 110 to 140. Here
+// the instructions around those and the latency of the first loads. On 88 -> 88 @52x52 x16 with LeakyReLU the implicit-GEMM kernel issues
+// 1.6 million vector and 1.4 million scalar instructions for 43 000 matrix ones (its tap and column arithmetic, divisions, the way
+// through LDS, 64-bit addresses), this one 0.87 and 0.40 million, in 9300 cycles instead of 13700. Here
 //  * a wave owns FN groups of 16 consecutive pixels (of the whole batch) and requests all their channels at once: the octets of a
 //    reduction step differ by a uniform offset, so a load is one instruction with no address arithmetic;
 //  * it walks `per` pairs of 16-row tiles of the output channels. The weights of a pair are refilled in place behind its last
