@@ -5,7 +5,6 @@
 #include <stdint.h>
 
 #include <type_traits>
-#include <utility>
 
 #include "../../include/otter_hip_int8.h"
 
