@@ -5,10 +5,22 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 #include "../../include/otter_hip_int8.h"
 
 namespace ohip {
+
+// A launch without the call configuration that the <<<>>> form pushes and pops: 2.66 us of the host's time instead of 2.80 (a launch of
+// 112 bytes of arguments, 4000 in a row). The error, if any, is there for hipGetLastError.
+template <typename... P, typename... A>
+inline void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, A&&... args) {
+    static_assert(sizeof...(P) == sizeof...(A), "one argument for each parameter");
+    [&](P... p) {
+        void* ptrs[] = {const_cast<void*>(static_cast<const void*>(&p))...};
+        (void)hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, ptrs, lds, stream);
+    }(std::forward<A>(args)...);
+}
 
 // ---------------------------------------------------------------------------------------------------
 // layouts

@@ -416,7 +416,7 @@ hipError_t launch_halo_w(const int8_t* x, const int8_t* wpk, void* out, const Co
     int m_blocks, grid_x;
     halo_grid(mpad, WM * FM, total_tiles, &m_blocks, &grid_x);
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W);
-    hipLaunchKernelGGL(kern, dim3(grid_x, m_blocks), dim3(256), prm_ofs + 3 * WM * FM * 16 * sizeof(float), stream, x, wpk,
+    launch(kern, dim3(grid_x, m_blocks), dim3(256), prm_ofs + 3 * WM * FM * 16 * sizeof(float), stream, x, wpk,
                        out, g, ep, mpad / 16, igemm_channel_groups(g.C), pl.r_max, pl.cb, pl.tiles_per_img, prm_ofs,
                        total_tiles, in_bytes, halo_tile_invariant(WN * FN * 16, g.OW, g.OH * g.OW) ? 1 : 0);
     return hipGetLastError();

@@ -552,7 +552,7 @@ hipError_t run_conv3x3_chain(const ConvGeom& g, const Epilogue* eps, const int8_
             if (e2 != hipSuccess) return e2;                                                                           \
             attr_set[dev].store(true, std::memory_order_release);                                                      \
         }                                                                                                              \
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds_bytes, stream, g, eps[0], ca, igemm_padded_rows(g.K) / 16, \
+        launch(kern, dim3(grid), dim3(256), lds_bytes, stream, g, eps[0], ca, igemm_padded_rows(g.K) / 16, \
                            igemm_channel_groups(g.C), r_max, tpi, act_bytes);                                          \
     } while (0)
 #define OHIP_CHAIN(FN_, E_, P_)                                  \

@@ -655,7 +655,7 @@ static hipError_t block_counters(int words, hipStream_t stream, unsigned** out) 
         next += (unsigned)words;
     }
     if (half) {
-        hipLaunchKernelGGL(blk_zero_counters_kernel, dim3((words + 255) / 256), dim3(256), 0, stream, *out, words);
+        launch(blk_zero_counters_kernel, dim3((words + 255) / 256), dim3(256), 0, stream, *out, words);
         return hipGetLastError();
     }
     return hipSuccess;
@@ -677,7 +677,7 @@ static hipError_t launch_block(const BlockArgs& a, const dim3& grid, size_t lds,
             raised[dev].store(true, std::memory_order_release);
         }
     }
-    hipLaunchKernelGGL((conv_block_kernel<NN, E3, SL, NI, CGE, WV>), grid, dim3(64 * WV), lds, stream, a);
+    launch((conv_block_kernel<NN, E3, SL, NI, CGE, WV>), grid, dim3(64 * WV), lds, stream, a);
     return hipGetLastError();
 }
 

@@ -54,7 +54,7 @@ hipError_t run_conv_direct(const int8_t* x, int in_pack, const int8_t* wt, void*
     if (total == 0) return hipSuccess;
     size_t blocks = (total + 255) / 256;
     if (blocks > (1u << 20)) blocks = 1u << 20;
-    hipLaunchKernelGGL(conv_direct_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, in_pack, wt, out, g, ep);
+    launch(conv_direct_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, in_pack, wt, out, g, ep);
     return hipGetLastError();
 }
 

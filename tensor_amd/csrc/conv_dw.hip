@@ -272,7 +272,7 @@ hipError_t run_conv_dw(const int8_t* x, const int32_t* wmask, void* out, const C
         int epi = pick_epilogue(ep, g.K);
         if (g.pw > 1 || g.ph > 1) epi = EPI_GENERIC;  // the fast kernel assumes the window's middle column is inside
 #define OHIP_DW(S_, R_, E_) \
-    hipLaunchKernelGGL((conv_dw3x3_kernel<S_, R_, E_>), dim3(blocks, planes), dim3(256), 0, stream, x, wmask, out, g, ep, \
+    launch((conv_dw3x3_kernel<S_, R_, E_>), dim3(blocks, planes), dim3(256), 0, stream, x, wmask, out, g, ep, \
                        n_strips)
         // narrow images: several images of the same channel octet share a wave (lane offsets stay below 2^31)
         const int col_chunks = (g.OW + 63) / 64;
@@ -294,7 +294,7 @@ hipError_t run_conv_dw(const int8_t* x, const int32_t* wmask, void* out, const C
         const int wpb = strips8 % 4 == 0 ? 4 : (strips8 % 2 == 0 ? 2 : 1);
         const int blocks8 = col_chunks * (strips8 / wpb);
 #define OHIP_DW8(S_, R_, N_) \
-    hipLaunchKernelGGL((conv_dw3x3_i8_kernel<S_, R_, N_>), dim3(blocks8, groups8), dim3(64 * wpb), 0, stream, x, wmask, \
+    launch((conv_dw3x3_i8_kernel<S_, R_, N_>), dim3(blocks8, groups8), dim3(64 * wpb), 0, stream, x, wmask, \
                        (int8_t*)out, g, ep, strips8, col_chunks, ipw)
 #define OHIP_DW8_R(S_, RMAX_, N_)                  \
     do {                                           \
@@ -316,7 +316,7 @@ hipError_t run_conv_dw(const int8_t* x, const int32_t* wmask, void* out, const C
 #undef OHIP_DW8
     } else {
         const int blocks = (g.OH * g.OW + 255) / 256;
-        hipLaunchKernelGGL(conv_dw_generic_kernel, dim3(blocks, planes), dim3(256), 0, stream, x, wmask, out, g, ep);
+        launch(conv_dw_generic_kernel, dim3(blocks, planes), dim3(256), 0, stream, x, wmask, out, g, ep);
     }
     return hipGetLastError();
 }

@@ -597,7 +597,7 @@ hipError_t run_conv_dw_f32in(const float* x, const int8_t* wa, void* out, const 
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W * 4);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW * (epi == EPI_F32_P4 || epi == EPI_F32_P8 ? 4 : 1));
 #define OHIP_DWF_L(S_, E_, L_)                                                                                           \
-    hipLaunchKernelGGL((conv_dw3x3_f32in_kernel<S_, E_, L_>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
+    launch((conv_dw3x3_f32in_kernel<S_, E_, L_>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
                        DwGrid::of(grid.x, grid.y, (unsigned)C8, wpb), n_strips, rps, in_bytes, out_bytes)
 #define OHIP_DWF_N(S_, E_)                       \
     do {                                         \

@@ -494,7 +494,7 @@ static hipError_t launch_igemm_k(const int8_t* x, const int8_t* wpk, void* out, 
     const int mpad = igemm_padded_rows(g.K);
     const int m_tiles = (g.K + TM - 1) / TM;  // row blocks that hold at least one real channel (the rows are padded further)
     const int grid_z = g.Cs ? g.Cs / g.C : 1;  // groups of a grouped convolution
-    hipLaunchKernelGGL((conv_igemm_kernel<TM, TN, WM, WN, EPI, KC>), dim3(n_pix_tiles, m_tiles, grid_z), dim3(256), 0,
+    launch((conv_igemm_kernel<TM, TN, WM, WN, EPI, KC>), dim3(n_pix_tiles, m_tiles, grid_z), dim3(256), 0,
                        stream, x, wpk, out, g, ep, mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, (const float*)nullptr, 0.f, JoinParam<EPI>::of(ep));
     return hipGetLastError();
 }
@@ -508,7 +508,7 @@ static hipError_t launch_igemm_f32in(const float* x, const int8_t* wpk, void* ou
     const int mpad = igemm_padded_rows(g.K);
     const dim3 grid(n_pix_tiles, (g.K + TM - 1) / TM, 1);
 #define OHIP_IGF(E_)                                                                                                        \
-    hipLaunchKernelGGL((conv_igemm_kernel<TM, TN, WM, WN, E_, 1, true>), grid, dim3(256), 0, stream, (const int8_t*)x, wpk, out, g, ep, \
+    launch((conv_igemm_kernel<TM, TN, WM, WN, E_, 1, true>), grid, dim3(256), 0, stream, (const int8_t*)x, wpk, out, g, ep, \
                        mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, in_scale, in_half, NoJoin{})
     switch (pick_epilogue(ep, g.K)) {
     case EPI_I8_P8: OHIP_IGF(EPI_I8_P8); break;

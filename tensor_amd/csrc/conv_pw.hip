@@ -194,7 +194,7 @@ static hipError_t launch_pw(const int8_t* x, const int8_t* wpk, void* out, const
     const int HW = g.H * g.W, pairs = (g.K + 31) / 32;
     const int per = (pairs + slices - 1) / slices;
     const dim3 grid((HW + 64 * G - 1) / (64 * G), g.N, (pairs + per - 1) / per);
-    hipLaunchKernelGGL((conv_pw_stream_kernel<EPI, G, CG>), grid, dim3(256), (size_t)per * pw_pair_v4(CG) * 16, stream, x, wpk,
+    launch((conv_pw_stream_kernel<EPI, G, CG>), grid, dim3(256), (size_t)per * pw_pair_v4(CG) * 16, stream, x, wpk,
                        (int8_t*)out, ep, qh, g.C / 8, g.K, HW, per, igemm_padded_rows(g.K) / 16);
     return hipGetLastError();
 }
@@ -461,7 +461,7 @@ static hipError_t launch_pw_f32in(const float* x, const int8_t* wpk, void* out, 
     }
     const int HW = g.H * g.W;
     const dim3 grid((HW + 64 * G - 1) / (64 * G), g.N, 1);
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, x, wpk, out, ep, qh, g.C / 8, g.K, HW, per,
+    launch(kern, grid, dim3(256), lds, stream, x, wpk, out, ep, qh, g.C / 8, g.K, HW, per,
                        igemm_padded_rows(g.K) / 16, in_scale, in_half);
     return hipGetLastError();
 }
@@ -592,7 +592,7 @@ hipError_t run_conv_pw_avgpool(const int8_t* x, const int8_t* wpk, float* out, c
     const int mt16 = igemm_padded_rows(g.K) / 16, pairs = (mt16 + 1) / 2;
     const int cgs = igemm_channel_groups(g.C);
     const dim3 grid((unsigned)((pairs + 3) / 4), (unsigned)g.N);
-#define OHIP_PWA(N_) hipLaunchKernelGGL(conv_pw_avgpool_kernel<N_>, grid, dim3(256), 0, stream, x, wpk, out, g, ep, cgs, mt16)
+#define OHIP_PWA(N_) launch(conv_pw_avgpool_kernel<N_>, grid, dim3(256), 0, stream, x, wpk, out, g, ep, cgs, mt16)
     switch (cgs) {
     case 1: OHIP_PWA(1); break;
     case 2: OHIP_PWA(2); break;

@@ -510,7 +510,7 @@ bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep) {
 template <int FN, int CG, int EPI>
 static hipError_t launch_pw_reg(const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
                                 hipStream_t stream) {
-    hipLaunchKernelGGL((conv_pw_reg_kernel<FN, CG, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa,
+    launch((conv_pw_reg_kernel<FN, CG, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa,
                        PwAdd<EPI>::of(ep));
     return hipGetLastError();
 }
@@ -543,7 +543,7 @@ static hipError_t launch_pw_reg_wide(int epi, const int8_t* x, const int8_t* wpk
 template <int FN, int NS, int EPI>
 static hipError_t launch_pw_split(const int8_t* x, const int8_t* wpk, void* out, const PwRegArgs& pa, const Epilogue& ep, int slices,
                                   hipStream_t stream) {
-    hipLaunchKernelGGL((conv_pw_split_kernel<FN, NS, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa,
+    launch((conv_pw_split_kernel<FN, NS, EPI>), dim3((pa.tiles + 7) / 8 * 8, slices), dim3(256), 0, stream, x, wpk, out, pa,
                        PwAdd<EPI>::of(ep));
     return hipGetLastError();
 }

@@ -413,10 +413,10 @@ static hipError_t launch_stem_lds(const void* x, bool in_f32, const int8_t* wpk,
 #define OHIP_STEM_L(EPI_, FI_)                                                                                          \
     do {                                                                                                                \
         if (g.C == 3)                                                                                                   \
-            hipLaunchKernelGGL((conv_stem3x3_lds_kernel<MT, EPI_, FI_, 3>), grid, block, lds, stream, x, wpk, out, g, ep, \
+            launch((conv_stem3x3_lds_kernel<MT, EPI_, FI_, 3>), grid, block, lds, stream, x, wpk, out, g, ep, \
                                in_scale, in_round, p);                                                                  \
         else                                                                                                            \
-            hipLaunchKernelGGL((conv_stem3x3_lds_kernel<MT, EPI_, FI_, 0>), grid, block, lds, stream, x, wpk, out, g, ep, \
+            launch((conv_stem3x3_lds_kernel<MT, EPI_, FI_, 0>), grid, block, lds, stream, x, wpk, out, g, ep, \
                                in_scale, in_round, p);                                                                  \
     } while (0)
     if (in_f32) {
@@ -452,7 +452,7 @@ hipError_t run_conv_stem(const void* x, bool in_f32, const int8_t* wpk, void* ou
     const dim3 grid((unsigned)((total + 3) / 4)), block(256);
     const bool f32_out = ep.out_kind == OTTER_HIP_OUT_F32;
 #define OHIP_STEM(MT_, FO_, FI_)                                                                                   \
-    hipLaunchKernelGGL((conv_stem3x3_kernel<MT_, FO_, FI_>), grid, block, 0, stream, x, wpk, out, g, ep, in_scale,    \
+    launch((conv_stem3x3_kernel<MT_, FO_, FI_>), grid, block, 0, stream, x, wpk, out, g, ep, in_scale,    \
                        in_round, col_groups, strips, (int)total)
 #define OHIP_STEM_IO(MT_)                                  \
     do {                                                   \

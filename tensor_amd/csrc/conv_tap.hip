@@ -397,7 +397,7 @@ template <int FM, int FN, int WK, int WN, int DEPTH, int EPI, bool INF>
 hipError_t launch_tap(const void* x, const int8_t* wpk, void* out, const TapArgs& ta, const Epilogue& ep, int groups, hipStream_t stream) {
     const size_t lds = (size_t)ta.steps * 64 + (WK > 1 ? (size_t)WN * WK * (FM / 2) * FN * 2048 : 0);
     const dim3 grid((unsigned)ta.n_pix_tiles, (unsigned)((ta.K + 16 * FM - 1) / (16 * FM)), (unsigned)groups);
-    hipLaunchKernelGGL((conv_tap_kernel<FM, FN, WK, WN, DEPTH, EPI, INF>), grid, dim3(64 * WK * WN), lds, stream, (const int8_t*)x,
+    launch((conv_tap_kernel<FM, FN, WK, WN, DEPTH, EPI, INF>), grid, dim3(64 * WK * WN), lds, stream, (const int8_t*)x,
                        wpk, out, ta, EpiArgs<EPI>::of(ep), JoinParam<EPI>::of(ep));
     return hipGetLastError();
 }

@@ -347,7 +347,7 @@ hipError_t run_conv_xdw(const int8_t* x, const int8_t* wx, const int8_t* wa, voi
     const XdwArgs xa = {g.H, g.W, g.OH, g.OW, g.C, gx.C, g.ph, n_strips, rps, in_bytes, out_bytes, DwGrid::of(grid.x, grid.y, (unsigned)(g.C / 16), wpb)};
     const bool nn = epi_d == EPI_I8_P8_NONNEG;
 #define OHIP_XDW_L(S_, NN_, G_, CK_)                                                                                              \
-    hipLaunchKernelGGL((conv_xdw_kernel<S_, NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8, NN_, G_, CK_>), grid, block, lds_bytes, stream, x, wx, wa, \
+    launch((conv_xdw_kernel<S_, NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8, NN_, G_, CK_>), grid, block, lds_bytes, stream, x, wx, wa, \
                        out, xa, EpiArgs<NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8>::of(epx), EpiArgs<NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8>::of(ep))
 #define OHIP_XDW_G(S_, NN_, CK_)                 \
     do {                                         \

@@ -135,7 +135,7 @@ static hipError_t launch_ew(const TI* src, TO* dst, int N, int C, int HW, Op op,
     if (total == 0) return hipSuccess;
     size_t blocks = (total + 255) / 256;
     if (blocks > (1u << 20)) blocks = 1u << 20;
-    hipLaunchKernelGGL((ew_kernel<TI, TO, SP, DP, V, Op>), dim3((unsigned)blocks), dim3(256), 0, stream, src, dst, N, C,
+    launch((ew_kernel<TI, TO, SP, DP, V, Op>), dim3((unsigned)blocks), dim3(256), 0, stream, src, dst, N, C,
                        HW, (unsigned)blocks * 256u, op);
     return hipGetLastError();
 }
@@ -194,10 +194,10 @@ hipError_t run_pad_pack8(const void* src, bool src_is_float, int sp, int8_t* dst
     if (total == 0) return hipSuccess;
     const unsigned blocks = (unsigned)((total + 255) / 256);
     if (src_is_float)
-        hipLaunchKernelGGL(pad_pack8_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)src, sp, dst, N, C, Cp,
+        launch(pad_pack8_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)src, sp, dst, N, C, Cp,
                            HW, scale, round_mode);
     else
-        hipLaunchKernelGGL(pad_pack8_kernel<int8_t>, dim3(blocks), dim3(256), 0, stream, (const int8_t*)src, sp, dst, N, C,
+        launch(pad_pack8_kernel<int8_t>, dim3(blocks), dim3(256), 0, stream, (const int8_t*)src, sp, dst, N, C,
                            Cp, HW, scale, round_mode);
     return hipGetLastError();
 }

@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(256) copy_bytes_kernel(const uint4* __restrict
 hipError_t run_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream) {
     const size_t n16 = bytes / 16;
     const unsigned blocks = (unsigned)(n16 < 256 * 256 ? (n16 + 255) / 256 : 256);
-    hipLaunchKernelGGL(copy_bytes_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, stream, (const uint4*)src, (uint4*)dst, n16, bytes, blocks * 256);
+    launch(copy_bytes_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, stream, (const uint4*)src, (uint4*)dst, n16, bytes, blocks * 256);
     return hipGetLastError();
 }
 
@@ -127,7 +127,7 @@ hipError_t run_eltwise_add(const float* a, const float* b, float* out, size_t n,
     if (n == 0) return hipSuccess;
     const size_t n4 = n / 4;
     const size_t blocks = (n4 + 255) / 256 + (n4 == 0 ? 1 : 0);
-    hipLaunchKernelGGL(eltwise_add_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a, b, out, n4, n);
+    launch(eltwise_add_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, a, b, out, n4, n);
     return hipGetLastError();
 }
 
@@ -183,26 +183,26 @@ hipError_t run_eltwise_add_quantize(const float* a, const float* b, int pack, fl
     const float half = round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     const dim3 grid((unsigned)((total + 255) / 256)), block(256);
     if (pack == 8)
-        hipLaunchKernelGGL(eltwise_add_quantize_kernel<8>, grid, block, 0, stream, a, b, out, q, C / 8, HW, scale, half,
+        launch(eltwise_add_quantize_kernel<8>, grid, block, 0, stream, a, b, out, q, C / 8, HW, scale, half,
                            (unsigned)total);
     else
-        hipLaunchKernelGGL(eltwise_add_quantize_kernel<4>, grid, block, 0, stream, a, b, out, q, C / 8, HW, scale, half,
+        launch(eltwise_add_quantize_kernel<4>, grid, block, 0, stream, a, b, out, q, C / 8, HW, scale, half,
                            (unsigned)total);
     return hipGetLastError();
 }
 
 hipError_t run_activation(float* x, size_t n, int act, float p0, hipStream_t stream) {
     if (n == 0 || act == 0) return hipSuccess;
-    hipLaunchKernelGGL(activation_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x, n, act, p0);
+    launch(activation_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, x, n, act, p0);
     return hipGetLastError();
 }
 
 hipError_t run_global_avgpool(const float* x, int pack, int N, int C, int HW, float* out, hipStream_t stream) {
     if (N * C == 0) return hipSuccess;
     const unsigned blocks = (unsigned)((N * (C / pack) + 3) / 4);
-    if (pack == 8) hipLaunchKernelGGL(global_avgpool_kernel<8>, dim3(blocks), dim3(256), 0, stream, x, N, C, HW, out);
-    else if (pack == 4) hipLaunchKernelGGL(global_avgpool_kernel<4>, dim3(blocks), dim3(256), 0, stream, x, N, C, HW, out);
-    else if (pack == 1) hipLaunchKernelGGL(global_avgpool_kernel<1>, dim3(blocks), dim3(256), 0, stream, x, N, C, HW, out);
+    if (pack == 8) launch(global_avgpool_kernel<8>, dim3(blocks), dim3(256), 0, stream, x, N, C, HW, out);
+    else if (pack == 4) launch(global_avgpool_kernel<4>, dim3(blocks), dim3(256), 0, stream, x, N, C, HW, out);
+    else if (pack == 1) launch(global_avgpool_kernel<1>, dim3(blocks), dim3(256), 0, stream, x, N, C, HW, out);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -273,12 +273,12 @@ hipError_t run_inner_product(const float* x, const float* w, const float* b, flo
     if (IN % 16 == 0 && IN >= 64) {
         const dim3 grid((OUT + 15) / 16, (N + 15) / 16), block(64 * IPM_WAVES);
         if ((((uintptr_t)x | (uintptr_t)w) & 15) == 0)
-            hipLaunchKernelGGL(inner_product_mfma_kernel<true>, grid, block, 0, stream, x, w, b, y, N, IN, OUT);
+            launch(inner_product_mfma_kernel<true>, grid, block, 0, stream, x, w, b, y, N, IN, OUT);
         else
-            hipLaunchKernelGGL(inner_product_mfma_kernel<false>, grid, block, 0, stream, x, w, b, y, N, IN, OUT);
+            launch(inner_product_mfma_kernel<false>, grid, block, 0, stream, x, w, b, y, N, IN, OUT);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(inner_product_kernel, dim3((OUT + IP_OB - 1) / IP_OB, (N + IP_NB - 1) / IP_NB), dim3(256), 0, stream,
+    launch(inner_product_kernel, dim3((OUT + IP_OB - 1) / IP_OB, (N + IP_NB - 1) / IP_NB), dim3(256), 0, stream,
                        x, w, b, y, N, IN, OUT);
     return hipGetLastError();
 }
@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(256) shader_clock_kernel(int iters, unsigned l
 }
 
 hipError_t run_shader_clock(int blocks, int iters, unsigned long long* out, hipStream_t stream) {
-    hipLaunchKernelGGL(shader_clock_kernel, dim3(blocks), dim3(256), 0, stream, iters, out);
+    launch(shader_clock_kernel, dim3(blocks), dim3(256), 0, stream, iters, out);
     return hipGetLastError();
 }
 

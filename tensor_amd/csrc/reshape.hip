@@ -202,11 +202,11 @@ hipError_t run_concat_channels(const ConcatSources& srcs, float* dst, int Cd, in
         // small images: workgroups of one wave, or most lanes would have no pixel
         const unsigned t = HW >= 512 ? 256 : 64;
         const dim3 grid((HW + t * OCTET_PX - 1) / (t * OCTET_PX), (unsigned)(Cd / 8), (unsigned)N);
-        if (t == 256) hipLaunchKernelGGL((concat_octets_kernel<256>), grid, dim3(256), 0, stream, srcs, dst, Cd, pd, HW, q, scale, h);
-        else hipLaunchKernelGGL((concat_octets_kernel<64>), grid, dim3(64), 0, stream, srcs, dst, Cd, pd, HW, q, scale, h);
+        if (t == 256) launch((concat_octets_kernel<256>), grid, dim3(256), 0, stream, srcs, dst, Cd, pd, HW, q, scale, h);
+        else launch((concat_octets_kernel<64>), grid, dim3(64), 0, stream, srcs, dst, Cd, pd, HW, q, scale, h);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(concat_channels4_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, stream, srcs, dst, Cd, pd,
+    launch(concat_channels4_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, stream, srcs, dst, Cd, pd,
                        H, W, (unsigned)total4, q, scale, round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f);
     return hipGetLastError();
 }
@@ -223,14 +223,14 @@ hipError_t run_copy_channels(const float* src, int Cs, int ps, int cs0, float* d
     if (q != nullptr && !copy_channels_moves_quads(ps, cs0, pd, cd0, cnt)) return hipErrorInvalidValue;
     if (copy_channels_moves_quads(ps, cs0, pd, cd0, cnt)) {
         const size_t total4 = total / 4;
-        hipLaunchKernelGGL(copy_channels4_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, stream, src, Cs, ps,
+        launch(copy_channels4_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, stream, src, Cs, ps,
                            cs0, dst, Cd, pd, cd0, cnt, N, H, W, (unsigned)total4, q, scale,
                            round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f);
     } else if (whole) {
-        hipLaunchKernelGGL(copy_channels_kernel<true>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, Cs,
+        launch(copy_channels_kernel<true>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, Cs,
                            ps, cs0, dst, Cd, pd, cd0, cnt, N, H, W, (unsigned)total);
     } else {
-        hipLaunchKernelGGL(copy_channels_kernel<false>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, Cs,
+        launch(copy_channels_kernel<false>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, Cs,
                            ps, cs0, dst, Cd, pd, cd0, cnt, N, H, W, (unsigned)total);
     }
     return hipGetLastError();
@@ -330,7 +330,7 @@ hipError_t run_shuffle2_split(const float* a, int pa, const float* b, int pb, fl
     const size_t total = (size_t)N * (Ch / 4) * HW;
     if (total == 0) return hipSuccess;
     const float half = round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
-    hipLaunchKernelGGL(shuffle2_split_p8_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, a, b, c1, c2, q2,
+    launch(shuffle2_split_p8_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, a, b, c1, c2, q2,
                        scale, half, Ch, HW, pa, pb, (unsigned)total);
     return hipGetLastError();
 }
@@ -344,11 +344,11 @@ hipError_t run_channel_shuffle(const float* src, int ps, float* dst, int pd, int
     if (q != nullptr && !channel_shuffle_can_quantize(ps, pd, C, groups)) return hipErrorInvalidValue;
     if (channel_shuffle_can_quantize(ps, pd, C, groups)) {
         const size_t units = total / 8;
-        hipLaunchKernelGGL(channel_shuffle2_p8_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, src, dst, C,
+        launch(channel_shuffle2_p8_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, src, dst, C,
                            H * W, (unsigned)units, q, scale, round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(channel_shuffle_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, ps, dst, pd,
+    launch(channel_shuffle_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, ps, dst, pd,
                        N, C, H, W, groups, (unsigned)total);
     return hipGetLastError();
 }
@@ -472,7 +472,7 @@ hipError_t run_maxpool(const float* src, int ps, float* dst, int pd, int N, int 
         const Quads g = Quads::of(N, C, OH, OW, ps, pd, two ? 2 : 1);
         const dim3 grid((g.total + 255) / 256);
 #define OHIP_POOL(K_, P_)                                                                                                            \
-    hipLaunchKernelGGL((maxpool4_kernel<K_, P_>), grid, dim3(256), 0, stream, src, dst, g, H, W, (unsigned)OH * (unsigned)OW, kh, kw, sh, sw, \
+    launch((maxpool4_kernel<K_, P_>), grid, dim3(256), 0, stream, src, dst, g, H, W, (unsigned)OH * (unsigned)OW, kh, kw, sh, sw, \
                        ph, pw, dh, dw, pad_value)
         if (k3 && two) OHIP_POOL(3, 2);
         else if (k3) OHIP_POOL(3, 1);
@@ -481,7 +481,7 @@ hipError_t run_maxpool(const float* src, int ps, float* dst, int pd, int N, int 
 #undef OHIP_POOL
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(maxpool_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, ps, dst, pd, N, C, H,
+    launch(maxpool_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, ps, dst, pd, N, C, H,
                        W, OH, OW, kh, kw, sh, sw, ph, pw, dh, dw, pad_value, (unsigned)total);
     return hipGetLastError();
 }
@@ -590,7 +590,7 @@ hipError_t run_upsample(const float* src, int ps, float* dst, int pd, int N, int
         const double scale_y = linear_scale(H, OH, align_corner), scale_x = linear_scale(W, OW, align_corner);
         const float hs = (float)H / (float)OH, ws = (float)W / (float)OW;
 #define OHIP_UP(N_, P_)                                                                                                              \
-    hipLaunchKernelGGL((upsample4_kernel<N_, P_>), grid, dim3(256), 0, stream, src, dst, g, H, W, (unsigned)OH * (unsigned)OW, scale_y, scale_x, \
+    launch((upsample4_kernel<N_, P_>), grid, dim3(256), 0, stream, src, dst, g, H, W, (unsigned)OH * (unsigned)OW, scale_y, scale_x, \
                        hs, ws, align_corner)
         if (mode == 1 && four) OHIP_UP(true, 4);
         else if (mode == 1) OHIP_UP(true, 1);
@@ -599,7 +599,7 @@ hipError_t run_upsample(const float* src, int ps, float* dst, int pd, int N, int
 #undef OHIP_UP
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(upsample_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, ps, dst, pd, N, C, H,
+    launch(upsample_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, src, ps, dst, pd, N, C, H,
                        W, OH, OW, mode, align_corner, (unsigned)total);
     return hipGetLastError();
 }
