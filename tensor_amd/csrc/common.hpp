@@ -601,20 +601,18 @@ __device__ __forceinline__ void store_b128_row(ohip_v4i data, __amdgpu_buffer_rs
     asm volatile("s_nop 1" ::"v"(data) : "memory");
 }
 
-// n / d for 0 <= n < 2^31 as a multiplication: with 2^(l-1) < d <= 2^l and m = ceil(2^(31+l) / d) the error m d - 2^(31+l) is
-// below 2^l, so that n times it stays below 2^(31+l)
+// n / d for 0 <= n < 2^31 as a multiplication: with 2^(l-1) < d <= 2^l and m = ceil(2^(31+l) / d) < 2^32 the error m d - 2^(31+l) is
+// below 2^l, so that n times it stays below 2^(31+l). (n is doubled, for a product whose upper half begins at bit 31: with m a bit
+// longer d = 1 would need a branch, and a kernel's indices are a chain of such divisions.)
 struct FastDiv {
     unsigned m, s, d;
 };
 inline FastDiv fast_div(unsigned d) {
-    FastDiv f{0, 0, d};
-    if (d <= 1) return f;
-    unsigned l = 1;
+    if (d == 0) d = 1;
+    unsigned l = 0;
     while ((1ull << l) < d) ++l;
-    f.m = (unsigned)(((1ull << (31 + l)) + d - 1) / d);
-    f.s = l - 1;
-    return f;
+    return {(unsigned)(((1ull << (31 + l)) + d - 1) / d), l, d};
 }
-__device__ __forceinline__ unsigned div_by(unsigned n, const FastDiv& f) { return f.m ? __umulhi(n, f.m) >> f.s : n; }
+__device__ __forceinline__ unsigned div_by(unsigned n, const FastDiv& f) { return __umulhi(n << 1, f.m) >> f.s; }
 
 }  // namespace ohip
