@@ -415,50 +415,51 @@ __device__ __forceinline__ unsigned cvt_u32_floor0(float v) {
     return r;
 }
 
-// LRELU: 0 = no LeakyReLU, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time (a select per value)
+// LeakyReLU decided at run time: max(v, v * slope) with a slope of 1 where there is none, which is v itself. (A choice per value is two
+// instructions more, and it is made per value: the compiler turns a uniform branch around three instructions into a select.)
+__device__ __forceinline__ float lrelu_or_not(const Epilogue& ep, float v) { return fmaxf(v, __fmul_rn(v, ep.lrelu ? ep.act_p0 : 1.f)); }
+
+// requantize 4 channels: their bytes
+// LRELU: 0 = no LeakyReLU, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time
 template <bool NONNEG, int LRELU = -1>
-__device__ __forceinline__ ohip_v2i epi8_quant_i8p8(const Epilogue& ep, const Epi8& p, const int (&a8)[8]) {
-    int q[8];
+__device__ __forceinline__ int epi4_quant_i8(const Epilogue& ep, const float* si, const float* bi, const float* so, const unsigned* qh,
+                                             int a0, int a1, int a2, int a3) {
+    const int a[4] = {a0, a1, a2, a3};
+    int q[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        float v = __fmaf_rn((float)a8[e], p.si[e], p.bi[e]);
-        if constexpr (!NONNEG && LRELU != 0) {
-            if (LRELU == 1 || ep.lrelu) v = fmaxf(v, __fmul_rn(v, ep.act_p0));  // wave-uniform
-        }
-        v = __fmul_rn(v, p.so[e]);
+    for (int e = 0; e < 4; ++e) {
+        float v = __fmaf_rn((float)a[e], si[e], bi[e]);
+        if constexpr (!NONNEG && LRELU == 1) v = fmaxf(v, __fmul_rn(v, ep.act_p0));
+        if constexpr (!NONNEG && LRELU == -1) v = lrelu_or_not(ep, v);
+        v = __fmul_rn(v, so[e]);
         float adj = NONNEG ? __fadd_rn(v, ep.round_half) : __fadd_rn(v, __builtin_copysignf(ep.round_half, v));
         // toward zero, saturating. NONNEG: to UNSIGNED, which sends everything below zero to zero: the lower clamp of
         // the activation comes with the conversion, and only the upper one is left for the packed values
         if constexpr (NONNEG) q[e] = (int)cvt_u32_floor0(adj);
         else q[e] = (int)adj;
     }
-    ohip_v2i pk;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        // two int32 -> two saturated int16 in one dword, clamp both halves at once, then gather the low bytes
-        if constexpr (NONNEG) {
-            typedef unsigned short ohip_v2us __attribute__((ext_vector_type(2)));
-            ohip_v2us lo = __builtin_bit_cast(ohip_v2us, __builtin_amdgcn_cvt_pk_u16((unsigned)q[4 * h], (unsigned)q[4 * h + 1]));
-            ohip_v2us hi = __builtin_bit_cast(ohip_v2us, __builtin_amdgcn_cvt_pk_u16((unsigned)q[4 * h + 2], (unsigned)q[4 * h + 3]));
-            lo = __builtin_elementwise_min(lo, __builtin_bit_cast(ohip_v2us, p.qh[2 * h]));
-            hi = __builtin_elementwise_min(hi, __builtin_bit_cast(ohip_v2us, p.qh[2 * h + 1]));
-            pk[h] = (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
-            continue;
-        }
-        ohip_v2s lo = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(q[4 * h], q[4 * h + 1]));
-        ohip_v2s hi = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(q[4 * h + 2], q[4 * h + 3]));
-        if (NONNEG) {
-            const ohip_v2s zero = {0, 0};
-            lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, __builtin_bit_cast(ohip_v2s, p.qh[2 * h])), zero);
-            hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, __builtin_bit_cast(ohip_v2s, p.qh[2 * h + 1])), zero);
-        } else {
-            const ohip_v2s top = {127, 127}, bot = {-127, -127};
-            lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bot);
-            hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bot);
-        }
-        pk[h] = (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
+    // two int32 -> two saturated int16 in one dword, clamp both halves at once, then gather the low bytes
+    if constexpr (NONNEG) {
+        typedef unsigned short ohip_v2us __attribute__((ext_vector_type(2)));
+        ohip_v2us lo = __builtin_bit_cast(ohip_v2us, __builtin_amdgcn_cvt_pk_u16((unsigned)q[0], (unsigned)q[1]));
+        ohip_v2us hi = __builtin_bit_cast(ohip_v2us, __builtin_amdgcn_cvt_pk_u16((unsigned)q[2], (unsigned)q[3]));
+        lo = __builtin_elementwise_min(lo, __builtin_bit_cast(ohip_v2us, qh[0]));
+        hi = __builtin_elementwise_min(hi, __builtin_bit_cast(ohip_v2us, qh[1]));
+        return (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
+    } else {
+        ohip_v2s lo = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(q[0], q[1]));
+        ohip_v2s hi = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(q[2], q[3]));
+        const ohip_v2s top = {127, 127}, bot = {-127, -127};
+        lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bot);
+        hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bot);
+        return (int)__builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
     }
-    return pk;
+}
+
+template <bool NONNEG, int LRELU = -1>
+__device__ __forceinline__ ohip_v2i epi8_quant_i8p8(const Epilogue& ep, const Epi8& p, const int (&a8)[8]) {
+    return ohip_v2i{epi4_quant_i8<NONNEG, LRELU>(ep, p.si, p.bi, p.so, p.qh, a8[0], a8[1], a8[2], a8[3]),
+                    epi4_quant_i8<NONNEG, LRELU>(ep, p.si + 4, p.bi + 4, p.so + 4, p.qh + 2, a8[4], a8[5], a8[6], a8[7])};
 }
 
 template <bool NONNEG>
@@ -539,7 +540,7 @@ __device__ __forceinline__ const float* epi4_residual_at(const Epilogue& ep, con
 // dequantize (+clamp activation) 4 channels and store one Float4 element. FUSED: first add the residual blob's element
 // if the epilogue carries one, and return the four bytes of the blob's int8 twin (float2int8(v * twin_scale)) if it
 // carries one
-// LRELU: 0 = clamp activation only, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time (a select per value)
+// LRELU: 0 = clamp activation only, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time
 // res_at: where the residual's element is, if not at `elem` of one blob (epi4_residual_at)
 template <bool FUSED = false, int LRELU = -1>
 __device__ __forceinline__ unsigned epi4_store_f32p4(float* __restrict__ out, const Epilogue& ep, const float* si,
@@ -556,9 +557,8 @@ __device__ __forceinline__ unsigned epi4_store_f32p4(float* __restrict__ out, co
     for (int e = 0; e < 4; ++e) {
         float v = __fmaf_rn((float)a[e], si[e], bi[e]);
         if constexpr (LRELU != 1) v = fminf(fmaxf(v, ep.act_lo), ep.act_hi);  // (open for LeakyReLU)
-        if constexpr (LRELU != 0) {
-            if (LRELU == 1 || ep.lrelu) v = fmaxf(v, __fmul_rn(v, ep.act_p0));  // wave-uniform
-        }
+        if constexpr (LRELU == 1) v = fmaxf(v, __fmul_rn(v, ep.act_p0));
+        if constexpr (LRELU == -1) v = lrelu_or_not(ep, v);
         if constexpr (FUSED) {
             if (ep.residual != nullptr) v = __fadd_rn(v, __int_as_float(res[e]));
             if (ep.twin != nullptr) {  // wave-uniform

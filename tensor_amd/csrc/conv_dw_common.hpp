@@ -45,14 +45,16 @@ __device__ __forceinline__ unsigned dw_clamp_pair(const Epilogue& ep, int so0, i
     return (unsigned)(q0 & 0xffff) | ((unsigned)q1 << 16);
 }
 
-template <bool NONNEG>
+// LRELU: 0 = no LeakyReLU, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time
+template <bool NONNEG, int LRELU = -1>
 __device__ __forceinline__ unsigned dw_requant4(const Epilogue& ep, const v4i& acc, const v4i& si, const v4i& bi,
                                                 const v4i& so, unsigned qh01, unsigned qh23) {
     int qv[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         float v = __fmaf_rn((float)acc[e], __int_as_float(si[e]), __int_as_float(bi[e]));
-        if (!NONNEG && ep.lrelu) v = fmaxf(v, __fmul_rn(v, ep.act_p0));  // wave-uniform branch
+        if constexpr (!NONNEG && LRELU == 1) v = fmaxf(v, __fmul_rn(v, ep.act_p0));
+        if constexpr (!NONNEG && LRELU == -1) v = lrelu_or_not(ep, v);
         v = __fmul_rn(v, __int_as_float(so[e]));
         const float adj = NONNEG ? __fadd_rn(v, ep.round_half) : __fadd_rn(v, __builtin_copysignf(ep.round_half, v));
         // toward zero, saturating; NONNEG: to unsigned, which is also the activation's lower clamp

@@ -62,13 +62,16 @@ void dw_mfma_pack_weights(const int8_t* w, int C, int stride, int pad_w, int ks,
                 }
 }
 
+// LRELU as in dw_requant4 (its layers have an open clamp)
+template <int LRELU = -1>
 __device__ __forceinline__ v4i dw_dequant4(const Epilogue& ep, const v4i& acc, const v4i& si, const v4i& bi) {
     v4i res;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         float v = __fmaf_rn((float)acc[e], __int_as_float(si[e]), __int_as_float(bi[e]));
-        v = fminf(fmaxf(v, ep.act_lo), ep.act_hi);
-        if (ep.lrelu) v = fmaxf(v, __fmul_rn(v, ep.act_p0));  // wave-uniform branch; the clamp above is open then
+        if constexpr (LRELU != 1) v = fminf(fmaxf(v, ep.act_lo), ep.act_hi);
+        if constexpr (LRELU == 1) v = fmaxf(v, __fmul_rn(v, ep.act_p0));
+        if constexpr (LRELU == -1) v = lrelu_or_not(ep, v);
         res[e] = __float_as_int(v);
     }
     return res;
@@ -98,7 +101,8 @@ struct DwArgs {
 // down `rps` output rows. The input rows live in a ring of 8 register fragments: a step computes 8/S output rows
 // from the ring and refills every slot as soon as its last reader has issued, so the loads run 5 input rows ahead of
 // the matrix instructions for the whole walk. Narrow images sit side by side in the wave (`lpi` lane columns each).
-template <int S, int EPI, bool ODDW, int KS>
+// LR: the layer has LeakyReLU. Decided per value it made a signed result 12 vector instructions where it is 8 without.
+template <int S, int EPI, bool ODDW, int KS, bool LR>
 __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wa,
                                                               void* __restrict__ out, DwArgs g) {
     constexpr int RING = 8, U = RING / S;  // U output rows per step
@@ -226,7 +230,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
         if constexpr (EPI == EPI_F32_P4 || EPI == EPI_F32_P8) {
 #pragma unroll
             for (int t = 0; t < T; ++t) {
-                const v4i res = dw_dequant4(ep, cur[t], si[t], bi[t]);
+                const v4i res = dw_dequant4<LR ? 1 : 0>(ep, cur[t], si[t], bi[t]);
                 // the second set's channels 4..7: the next Float4 pack is one plane further, in Float8 they follow
                 const unsigned vo_t = (t == 0 || !row_ok) ? v_o : v_o + (EPI == EPI_F32_P4 ? OHW * 16u : 16u);
                 store_b128_row(res, rout, vo_t, s_row);
@@ -235,11 +239,11 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
             constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
             if constexpr (S == 1) {
                 v2i w2;
-                w2[0] = (int)dw_requant4<NONNEG>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
-                w2[1] = (int)dw_requant4<NONNEG>(ep, cur[T - 1], si[T - 1], bi[T - 1], so[T - 1], qh[T - 1][0], qh[T - 1][1]);
+                w2[0] = (int)dw_requant4<NONNEG, LR ? 1 : 0>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
+                w2[1] = (int)dw_requant4<NONNEG, LR ? 1 : 0>(ep, cur[T - 1], si[T - 1], bi[T - 1], so[T - 1], qh[T - 1][0], qh[T - 1][1]);
                 __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, w2), rout, (int)v_o, (int)s_row, 0);
             } else {
-                const unsigned w1 = dw_requant4<NONNEG>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
+                const unsigned w1 = dw_requant4<NONNEG, LR ? 1 : 0>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
                 __builtin_amdgcn_raw_buffer_store_b32(w1, rout, (int)v_o, (int)s_row, 0);
             }
         }
@@ -679,12 +683,17 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     pl.N = g.N, pl.H = g.H, pl.W = g.W, pl.OH = g.OH, pl.OW = g.OW, pl.ph = (unsigned char)g.ph, pl.rps = rps;
     pl.total = grid.x * grid.y, pl.in_bytes = in_bytes, pl.out_bytes = out_bytes;
     pl.p0 = ep.act_p0, pl.lo = ep.act_lo, pl.hi = ep.act_hi, pl.half = ep.round_half, pl.lrelu = ep.lrelu;
-#define OHIP_DWM_K(S_, E_, O_)                                                                                         \
-    do {                                                                                                               \
-        if (g.kh == 3)                                                                                                 \
-            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 3>), grid, block, 0, stream, x, wa, out, pl); \
-        else                                                                                                           \
-            hipLaunchKernelGGL((conv_dw3x3_mfma_kernel<S_, E_, O_, 5>), grid, block, 0, stream, x, wa, out, pl); \
+#define OHIP_DWM_L(S_, E_, O_, K_)                                                                                        \
+    do {                                                                                                                   \
+        if (E_ != EPI_I8_P8_NONNEG && ep.lrelu)                                                                            \
+            launch((conv_dw3x3_mfma_kernel<S_, E_, O_, K_, E_ != EPI_I8_P8_NONNEG>), grid, block, 0, stream, x, wa, out, pl); \
+        else                                                                                                               \
+            launch((conv_dw3x3_mfma_kernel<S_, E_, O_, K_, false>), grid, block, 0, stream, x, wa, out, pl);    \
+    } while (0)
+#define OHIP_DWM_K(S_, E_, O_)                  \
+    do {                                        \
+        if (g.kh == 3) OHIP_DWM_L(S_, E_, O_, 3); \
+        else OHIP_DWM_L(S_, E_, O_, 5);         \
     } while (0)
 #define OHIP_DWM(S_, E_) \
     do {                                                                                                               \
@@ -704,6 +713,7 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     else OHIP_DWM_E(2);
 #undef OHIP_DWM_E
 #undef OHIP_DWM_K
+#undef OHIP_DWM_L
 #undef OHIP_DWM
     return hipGetLastError();
 }

@@ -398,21 +398,21 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
         }
     };
     const __amdgpu_buffer_rsrc_t rout = rsrc(out, I8 ? pa.total_pix * K : f_bytes);
-    auto finish = [&](const Half& k, int pr, const v4i (&c)[OWN]) {
+    auto finish = [&](const Half& k, int pr, const v4i (&c)[OWN], auto lrelu_c) {
+        constexpr bool LRELU = decltype(lrelu_c)::value;
         const unsigned ch = 32u * pr + 8 * q + 4 * h;
 #pragma unroll
         for (int o = 0; o < OWN; ++o) {
             if constexpr (I8) {
                 const v4i so = v4i{1, 1, 1, 1} * __float_as_int(pa.scale);
-                const unsigned w = dw_requant4<NONNEG>(ep, c[o], k.si, k.bi, so, pa.qh, pa.qh);
+                const unsigned w = dw_requant4<NONNEG, LRELU ? 1 : 0>(ep, c[o], k.si, k.bi, so, pa.qh, pa.qh);
                 __builtin_amdgcn_raw_buffer_store_b32(w, rout, (int)(ch < K ? vo[o] : PR_OOB), (int)((unsigned)pr * 32u * HW), 0);
                 continue;
             }
             float si[4], bi[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) si[e] = __int_as_float(k.si[e]), bi[e] = __int_as_float(k.bi[e]);
-            v4i r = ep.lrelu ? epi4_dequant_f32p4<true>(ep, si, bi, c[o][0], c[o][1], c[o][2], c[o][3])  // (uniform)
-                             : epi4_dequant_f32p4<false>(ep, si, bi, c[o][0], c[o][1], c[o][2], c[o][3]);
+            v4i r = epi4_dequant_f32p4<LRELU>(ep, si, bi, c[o][0], c[o][1], c[o][2], c[o][3]);
             if constexpr (SHUF) {
                 // with the same channels of the other blob these are channels 2 ch .. 2 ch + 7 of the shuffled one: a pack of 8
                 const v4i even = ja.other_odd ? r : k.add[o], odd = ja.other_odd ? k.add[o] : r;  // (uniform)
@@ -479,7 +479,8 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
 #pragma unroll
                 for (int i = 0; i < 3; ++i) own[o] += red[pr & 1][u][i][lane];
             }
-            finish(k0, pr, own);
+            if (!NONNEG && ep.lrelu) finish(k0, pr, own, std::true_type{});  // (uniform)
+            else finish(k0, pr, own, std::false_type{});
             k0 = k1;
         }
     }
