@@ -21,8 +21,12 @@
 // @204x204 b55 107 / 56; 8 -> 344 5x5 @113x113 b24 96 / 62; from fp32 128 -> 64 5x5 in 8 groups @75x89 b32 48.6 / 28.9.
 // The octets of a stage are requested together and the weights of a step ahead without a condition: with a branch on the parity of
 // the width at each load the compiler waited for every octet before the next. 256 -> 256 in 8 groups @28x28 b64 15.0 -> 14.2 per call.
-// What is left above the floor is the chain of a tile (rows in, barrier, steps, stores), which three or four workgroups per
-// compute unit hide in part; keeping eight octets or four weight steps in flight instead cost registers and was slower.
+// What is left above the floor is the chain of a tile (rows in, barrier, steps, stores), which the workgroups of a compute unit hide
+// from each other: registers are held to what six (two row tiles, two pixel tiles), five (two, four), four and three of them leave, and the set-up
+// and the end of a tile to what they need. Pixels are walked, not divided out, the stage's dividers come with the arguments, the epilogue's
+// constants come through LDS and for four channels at a time (for eight from memory: 28 registers, and the wave waits for them at the end of its chain). us per
+// launch in a graph, over 26 layers 0.92 of the time: 256 -> 256 in 8 groups @28x28 b64 15.4 -> 13.6; 384 -> 352 in 4 groups
+// @147x147 b4 65.7 -> 53.7; 16 -> 48 @167x167 b47 60.3 -> 51.5; 40 -> 168 from fp32 @53x53 b14 14.5 -> 13.0.
 #include "common.hpp"
 #include "conv_igemm.hpp"
 
@@ -32,6 +36,7 @@
 namespace ohip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 
 namespace {
@@ -42,6 +47,8 @@ constexpr int ROWS_LDS = 64 * 1024;        // what a workgroup may use: two to a
 struct RowsArgs {
     ConvGeom g;                            // one group's channels; g.Cs / g.Ks the tensors'
     FastDiv img, tw, vh, vw, ntx, kw;      // dividers: pixels of a strip, its width, VH, VW2, strips per image, kernel width
+    FastDiv count, count1;                 // octets of a stage: the first `more` ones have one more
+    int base, more;
     int strips, strip_w, VH, VW2;          // column strips per image, output columns of one, padded height, pixel pairs of a row
     int rows_max, pitch, plane;            // LDS rows of an octet plane, bytes of a row and of a plane
     int stages, blocks_per_wg;             // stages of the channels; row blocks that a workgroup walks
@@ -50,10 +57,12 @@ struct RowsArgs {
     unsigned in_bytes, w_bytes;
     const float* in_scale;
     float in_half;
+    int warm_steps;                        // steps of a row block whose weights are requested ahead
+    int consts;                            // LDS bytes in front of the epilogue constants
 };
 
 // octets [first, first + count) of stage c: the C/8 octets dealt to the stages as evenly as whole octets allow
-__host__ __device__ inline void rows_stage(int C8, int stages, int c, int* first, int* count) {
+inline void rows_stage(int C8, int stages, int c, int* first, int* count) {
     const int base = C8 / stages, more = C8 % stages;
     *first = c * base + (c < more ? c : more);
     *count = base + (c < more ? 1 : 0);
@@ -73,8 +82,8 @@ static int rows_steps(int C, int taps) {
 }
 
 template <int FM, int FN, int EPI, bool INF>
-__global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
-                                                           void* __restrict__ out, RowsArgs ra, EpiArgs<EPI> ea) {
+__global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF ? (FN == 4 ? 5 : 6) : FM == 4 && FN == 2 ? 4 : 2)
+    conv_rows_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out, RowsArgs ra, EpiArgs<EPI> ea) {
     constexpr int OOB = (int)0x80000000;  // beyond any buffer here (below 2 GiB)
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     const ConvGeom& g = ra.g;
@@ -100,21 +109,60 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
     const int v0 = (int)r0 * g.sh;
     const int rows = (int)(m1 - m0) * ra.VH + (int)r1 * g.sh + (g.kh - 1) * g.dh + 1 - v0;  // at most rows_max
 
+    // The constants of the workgroup's channels come through LDS: a channel per thread, requested in front of everything else. (Where the
+    // lanes that finish eight channels each load them, every request brings 16 bytes to each lane, and the wave waits for them at the
+    // end of its chain.)
+    constexpr int CN = 16 * FM;
+    const int block0 = blockIdx.y * ra.blocks_per_wg, nc = ra.blocks_per_wg * CN;  // at most 256
+    float* const consts = reinterpret_cast<float*>(lds + ra.consts);
+    float c_si = 0.f, c_bi = 0.f, c_so = 0.f;
+    if (EPI != EPI_GENERIC && tid < nc && block0 * CN + tid < g.K) {
+        const int ch = grp * g.K + block0 * CN + tid;
+        c_si = ep.scale_in[ch], c_bi = ep.bias[ch];
+        if constexpr (EPI != EPI_F32_P4) c_so = ep.scale_out[ch];
+    }
+
     // ---- this lane's pixels: LDS address of tap (0, 0), place in the output -----------------------------------------------------------
     int px[FN];
     unsigned out_n[FN], out_pix[FN], out_at[FN];  // (the first two for the generic epilogue only)
     bool px_ok[FN];
+    constexpr unsigned OUT_E = EPI == EPI_F32_P4 ? 4u : 8u;
+    if (EPI != EPI_GENERIC && ra.strips == 1 && ra.tw.d >= 16) {
+        // One place by division, the next 16 pixels on from it: at most one row's end and one image's are passed on the way. (Three
+        // divisions are eight 32-bit multiplications, 16 cycles each; for four places they took as long as requantizing the wave's
+        // 2048 results.)
+        unsigned t = t0 + wave * FN * 16 + p;
+        const unsigned n = div_by(t, ra.img);
+        unsigned in = t - n * ra.img.d;
+        const unsigned oy = div_by(in, ra.tw);
+        unsigned ox = in - oy * ra.tw.d;
+        int at = ((int)(n - m0) * ra.VH + (int)oy * g.sh - v0) * ra.pitch + ((int)ox * g.sw + (g.pw & 1)) * 8;
+        unsigned o = n * (unsigned)(g.Ks * OHW) + in * OUT_E;
+        const int row_on = g.sh * ra.pitch - (int)ra.tw.d * g.sw * 8, image_on = (ra.VH - g.OH * g.sh) * ra.pitch;
+        const unsigned o_on = (unsigned)(g.Ks * OHW) - (unsigned)OHW * OUT_E;
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        const unsigned t = t0 + (wave * FN + j) * 16 + p;
-        const unsigned m = div_by(t, ra.img), in = t - m * ra.img.d, oy = div_by(in, ra.tw), oxs = in - oy * ra.tw.d;
-        const unsigned n = div_by(m, ra.ntx), ox = (m - n * ra.ntx.d) * (unsigned)ra.strip_w + oxs;
-        px_ok[j] = t < ra.total_pix && ox < (unsigned)g.OW;
-        px[j] = t < ra.total_pix ? ((int)(m - m0) * ra.VH + (int)oy * g.sh - v0) * ra.pitch +
-                                       ((int)oxs * g.sw + (((int)(m - n * ra.ntx.d) * ra.strip_w * g.sw - g.pw) & 1)) * 8
-                                 : 0;
-        out_n[j] = n, out_pix[j] = oy * (unsigned)g.OW + ox;
-        out_at[j] = n * (unsigned)(g.Ks * OHW) + out_pix[j] * (EPI == EPI_F32_P4 ? 4u : 8u);
+        for (int j = 0; j < FN; ++j) {
+            px_ok[j] = t < ra.total_pix;
+            px[j] = px_ok[j] ? at : 0;
+            out_at[j] = o;
+            t += 16, ox += 16, in += 16, at += 128 * g.sw, o += 16 * OUT_E;
+            const bool row = ox >= ra.tw.d, image = in >= ra.img.d;
+            ox -= row ? ra.tw.d : 0, in -= image ? ra.img.d : 0;
+            at += (row ? row_on : 0) + (image ? image_on : 0), o += image ? o_on : 0;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+            const unsigned t = t0 + (wave * FN + j) * 16 + p;
+            const unsigned m = div_by(t, ra.img), in = t - m * ra.img.d, oy = div_by(in, ra.tw), oxs = in - oy * ra.tw.d;
+            const unsigned n = div_by(m, ra.ntx), ox = (m - n * ra.ntx.d) * (unsigned)ra.strip_w + oxs;
+            px_ok[j] = t < ra.total_pix && ox < (unsigned)g.OW;
+            px[j] = t < ra.total_pix ? ((int)(m - m0) * ra.VH + (int)oy * g.sh - v0) * ra.pitch +
+                                           ((int)oxs * g.sw + (((int)(m - n * ra.ntx.d) * ra.strip_w * g.sw - g.pw) & 1)) * 8
+                                     : 0;
+            out_n[j] = n, out_pix[j] = oy * (unsigned)g.OW + ox;
+            out_at[j] = n * (unsigned)(g.Ks * OHW) + out_pix[j] * OUT_E;
+        }
     }
 
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
@@ -122,8 +170,21 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
     const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(x), 0, (int)ra.in_bytes, 0x00020000);
     float in_scale = 0.f;
     if constexpr (INF) in_scale = ra.in_scale[0];
-    ep.scale_in += grp * g.K, ep.bias += grp * g.K;
-    if (ep.scale_out) ep.scale_out += grp * g.K;
+
+    // Long reductions: the weights of the workgroup's first row block, lines of 128 bytes, into the L2 of this die. A launch finds it empty, and the loop
+    // below asks for one step at a time; the tiles that a die has of the block take a share each. (448 -> 168 k 5 on one 99x99 image, 175
+    // steps: 60 -> 54 us; 456 -> 256 k 3 @150x150, 66 steps: 39.3 -> 37.0. At 9 steps the requests cost 1 to 4 % and bring nothing.)
+    constexpr int LINES = FM * 8, WARM = 4;  // lines of a step; requests of a thread
+    int warm[WARM] = {};
+    if (ra.warm_steps) {
+        const unsigned per = max(ra.n_tiles / 8, 1), share = (unsigned)pt % per, total = (unsigned)ra.warm_steps * LINES;
+#pragma unroll
+        for (int u = 0; u < WARM; ++u) {
+            const unsigned l = (u * per + share) * 256 + tid;
+            warm[u] = __builtin_amdgcn_raw_buffer_load_b32(rw, l < total ? (int)(l / LINES * (unsigned)ra.m_tiles16 * 1024 + l % LINES * 128) : OOB,
+                                                           block0 * FM * 1024, 0);
+        }
+    }
 
     // the rows: a strip's columns start at an even one (the one before its first where that is odd), so that a pixel pair never
     // lies across the left edge of the image
@@ -137,6 +198,17 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
                          in && last > first ? first | last << 16 : 0};
     }
 
+    if (EPI != EPI_GENERIC && tid < nc) {
+        consts[tid] = c_si, consts[nc + tid] = c_bi;
+        if constexpr (EPI != EPI_F32_P4) consts[2 * nc + tid] = c_so;
+        if constexpr (EPI == EPI_I8_P8_NONNEG)
+            reinterpret_cast<unsigned short*>(consts + 3 * nc)[tid] =
+                (unsigned short)min((int)__fadd_rn(__fmul_rn(ep.act_hi, c_so), ep.round_half), 127);
+    }
+
+#pragma unroll
+    for (int u = 0; u < WARM; ++u) asm volatile("" ::"v"(warm[u]));
+
     const int HW8 = HW * 8;
     const bool even = (g.W & 1) == 0;    // then no pair lies across the right edge either
     constexpr int UN = INF ? 2 : 4;      // octets in flight per thread
@@ -144,7 +216,7 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
     constexpr int INS = INF ? 4 : 1;     // bytes of an input value
 
     v4i acc[FM][FN];
-    int block = blockIdx.y * ra.blocks_per_wg;
+    int block = block0;
     const int block_end = min(block + ra.blocks_per_wg, (g.K + 16 * FM - 1) / (16 * FM));
     auto load_a = [&](v4i (&a)[FM], int step) {
 #pragma unroll
@@ -154,8 +226,8 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
     };
 
     for (int c = 0, step0 = 0; c < ra.stages; ++c) {
-        int first, count;
-        rows_stage(C8, ra.stages, c, &first, &count);
+        const int first = c * ra.base + min(c, ra.more), count = ra.base + (c < ra.more ? 1 : 0);
+        const FastDiv by_count = c < ra.more ? ra.count1 : ra.count;
         const int steps = (taps * count + 7) / 8;
         v4i a[D][FM];
 #pragma unroll
@@ -164,21 +236,21 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
         __syncthreads();  // the row table stands / everyone has read the stage before
         // the table of this stage's pairs e = (tap e / count, octet e % count); pairs past the end meet zero weights
         for (int e = tid; e < steps * 8; e += 256) {
-            const unsigned tap = (unsigned)e / (unsigned)count, oct = (unsigned)e - tap * (unsigned)count;
+            const unsigned tap = div_by((unsigned)e, by_count), oct = (unsigned)e - tap * (unsigned)count;
             const unsigned dy = div_by(tap, ra.kw), dx = tap - dy * (unsigned)g.kw;
             reinterpret_cast<int*>(table)[e] =
                 e < taps * count ? (int)oct * ra.plane + (int)dy * g.dh * ra.pitch + (int)dx * g.dw * 8 : 0;
         }
         // the stage's rows, zeros outside the image, as pixel pairs. A thread keeps one place of the octet planes and walks the
         // octets, so that an octet costs it a load and a write and no address arithmetic; planes of at most 128 pairs are dealt to
-        // 256 / pairs threads each
-        const int pairs = rows * ra.VW2, sub = pairs > 128 ? 1 : 256 / pairs;
-        const int oct0 = sub == 1 ? 0 : tid / pairs;
+        // a half, a quarter or an eighth of the threads each
+        const int pairs = rows * ra.VW2, sub_shift = pairs > 128 ? 0 : pairs > 64 ? 1 : pairs > 32 ? 2 : 3, sub = 1 << sub_shift;
+        const int oct0 = tid >> (8 - sub_shift);
         // (two walks, not a choice per load: behind loads on two branches the compiler waited for each octet before it requested the
         // next, four memory latencies in a row)
         auto stage_rows = [&](auto even_c) {
             constexpr bool EVEN = decltype(even_c)::value;
-            for (int pos = tid - oct0 * pairs; pos < pairs; pos += 256) {
+            for (int pos = tid & ((256 >> sub_shift) - 1); pos < pairs; pos += 256) {
                 const int row = (int)div_by((unsigned)pos, ra.vw), c0 = 2 * (pos - row * ra.VW2);
                 const v2i rt = row_tab[row];
                 const int lo = rt[1] & 0xffff, hi = rt[1] >> 16;
@@ -192,17 +264,17 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
 #pragma unroll
                     for (int u = 0; u < UN; ++u) {
                         const bool there = u == 0 || oct + u * sub < count;
-                        const int a0 = there ? o0 + so : OOB, a1 = there ? o1 + so : OOB;  // (OOB + so stays beyond any buffer)
+                        const int a0 = there ? o0 : OOB, a1 = there ? o1 : OOB;
                         if constexpr (INF) {
-                            f[u][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, 0, 0));
-                            f[u][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0 + 16, 0, 0));
-                            f[u][2] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1, 0, 0));
-                            f[u][3] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1 + 16, 0, 0));
+                            f[u][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, so, 0));
+                            f[u][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0 + 16, so, 0));
+                            f[u][2] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1, so, 0));
+                            f[u][3] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a1 + 16, so, 0));
                         } else if constexpr (EVEN) {
-                            v[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, 0, 0));
+                            v[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, so, 0));
                         } else {
-                            const v2i l = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a0, 0, 0));
-                            const v2i h = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a1, 0, 0));
+                            const v2i l = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a0, so, 0));
+                            const v2i h = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a1, so, 0));
                             v[u] = v4i{l[0], l[1], h[0], h[1]};
                         }
                         so += sub * HW8 * INS;
@@ -224,11 +296,9 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
                 }
             }
         };
-        if (oct0 < sub) {
-            if constexpr (INF) stage_rows(std::true_type{});  // (reads values, not pixel pairs)
-            else if (even) stage_rows(std::true_type{});
-            else stage_rows(std::false_type{});
-        }
+        if constexpr (INF) stage_rows(std::true_type{});  // (reads values, not pixel pairs)
+        else if (even) stage_rows(std::true_type{});
+        else stage_rows(std::false_type{});
         __syncthreads();
         // one block of output channels per pass over the stage; several only when there is one stage
         for (;;) {
@@ -278,7 +348,7 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
             }
             if (c + 1 < ra.stages) break;
             // ---- epilogue of the block -------------------------------------------------------------------------------------------
-            const int mt0 = block * FM;
+            const int mt0 = block * FM, c0 = (block - block0) * CN;
             ++block;
             if (block < block_end)
 #pragma unroll
@@ -287,26 +357,46 @@ __global__ void __launch_bounds__(256, 2) conv_rows_kernel(const int8_t* __restr
 #pragma unroll
             for (int pair = 0; pair < FM / 2; ++pair) {
                 const int ch0 = 16 * mt0 + 32 * pair + 8 * q;  // this lane's 8 consecutive output channels of the group
-                if (ch0 < g.K) {
-                    Epi8 prm;
-                    if constexpr (EPI != EPI_GENERIC) epi8_load<EPI>(prm, ep, ch0);
-                    const unsigned ch = (unsigned)(grp * g.K + ch0);
+                if (ch0 >= g.K) continue;
+                if constexpr (EPI == EPI_GENERIC) {
 #pragma unroll
                     for (int j = 0; j < FN; ++j) {
                         const v4i lo = acc[2 * pair][j], hi = acc[2 * pair + 1][j];
-                        const int a8[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                        if (!px_ok[j]) continue;
-                        if constexpr (EPI == EPI_GENERIC) {
-                            epilogue_store8_generic(out, &ep, (int)out_n[j], ch0, (int)out_pix[j], g.K, OHW, a8[0], a8[1], a8[2], a8[3],
-                                                    a8[4], a8[5], a8[6], a8[7]);
-                        } else if constexpr (EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
-                            const size_t o = out_at[j] + ch * (unsigned)OHW;
-                            epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm, o, a8);
-                        } else {
-                            const size_t e = out_at[j] + ch * (unsigned)OHW;
-                            epi4_store_f32p4<false>((float*)out, ep, prm.si, prm.bi, e, a8[0], a8[1], a8[2], a8[3]);
-                            if (ch0 + 4 < g.K)
-                                epi4_store_f32p4<false>((float*)out, ep, prm.si + 4, prm.bi + 4, e + (size_t)OHW * 4, a8[4], a8[5], a8[6], a8[7]);
+                        if (px_ok[j])
+                            epilogue_store8_generic(out, &ep, (int)out_n[j], ch0, (int)out_pix[j], g.K, OHW, lo[0], lo[1], lo[2], lo[3], hi[0],
+                                                    hi[1], hi[2], hi[3]);
+                    }
+                } else {
+                    const unsigned ch_at = (unsigned)(grp * g.K + ch0) * (unsigned)OHW;
+                    int bytes[FN];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {  // (four channels at a time: the constants of eight are 28 registers)
+                        if (EPI == EPI_F32_P4 && ch0 + 4 * h >= g.K) continue;
+                        const float* const at = consts + c0 + 32 * pair + 8 * q + 4 * h;
+                        const v4f si4 = *reinterpret_cast<const v4f*>(at), bi4 = *reinterpret_cast<const v4f*>(at + nc);
+                        v4f so4 = {};
+                        if constexpr (EPI != EPI_F32_P4) so4 = *reinterpret_cast<const v4f*>(at + 2 * nc);
+                        const float si[4] = {si4[0], si4[1], si4[2], si4[3]}, bi[4] = {bi4[0], bi4[1], bi4[2], bi4[3]};
+                        const float so[4] = {so4[0], so4[1], so4[2], so4[3]};
+                        unsigned qh[2] = {};
+                        if constexpr (EPI == EPI_I8_P8_NONNEG) {
+                            const v2i t = *reinterpret_cast<const v2i*>(reinterpret_cast<const unsigned short*>(consts + 3 * nc) + (at - consts));
+                            qh[0] = (unsigned)t[0], qh[1] = (unsigned)t[1];
+                        }
+#pragma unroll
+                        for (int j = 0; j < FN; ++j) {
+                            const v4i v = acc[2 * pair + h][j];
+                            if constexpr (EPI == EPI_F32_P4) {
+                                if (px_ok[j])
+                                    epi4_store_f32p4<false>((float*)out, ep, si, bi, (size_t)(out_at[j] + ch_at + (unsigned)h * (unsigned)OHW * 4), v[0], v[1], v[2], v[3]);
+                            } else {
+                                const int b4 = epi4_quant_i8<EPI == EPI_I8_P8_NONNEG>(ep, si, bi, so, qh, v[0], v[1], v[2], v[3]);
+                                if (h == 0) {
+                                    bytes[j] = b4;
+                                    asm volatile("" : "+v"(bytes[j]));  // (packed here, not behind the condition of the store)
+                                }
+                                if (h == 1 && px_ok[j]) *reinterpret_cast<v2i*>((int8_t*)out + (out_at[j] + ch_at)) = v2i{bytes[j], b4};
+                            }
                         }
                     }
                 }
@@ -402,35 +492,43 @@ bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
     return (size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1) < ((size_t)1 << 31) && (size_t)g.N * g.K * g.OH * g.OW < ((size_t)1 << 31);
 }
 
-// one stage: a workgroup walks row blocks over its staged pixels, as many as leave two workgroups per compute unit
-static int rows_blocks_per_workgroup(const RowsArgs& ra, int blocks) {
+// one stage: a workgroup walks row blocks over its staged pixels, as many as leave two workgroups per compute unit, and at most 256
+// channels (a thread brings the constants of one)
+static int rows_blocks_per_workgroup(const RowsArgs& ra, int blocks, int fm) {
     if (ra.stages > 1) return 1;
     const long tiles = (long)ra.n_tiles * ra.g.groups;
     const int want = (int)((512 + tiles - 1) / tiles), slices = want > blocks ? blocks : want;
-    return (blocks + slices - 1) / slices;
+    const int each = (blocks + slices - 1) / slices;
+    return each < 16 / fm ? each : 16 / fm;
 }
+
+// LDS of a workgroup: what the plan takes, and the epilogue constants behind it
+static size_t rows_lds(size_t plan, int blocks_per_wg, int fm) { return (plan + 15) / 16 * 16 + (size_t)(blocks_per_wg * 16 * fm * 14); }
 
 namespace {
 // A tile, the workgroups of it that the register file holds per compute unit, and the coefficients of its duration in us (inside
 // a graph of launches, warm) for int8 and fp32 input. A workgroup's chain is step * steps + stage * stages, and a compute unit
 // runs as many of them one after the other as its workgroups do not fit side by side; per workgroup of the busiest compute unit
 // comes what they share: steps, staged places (pixel pairs of a thread) and row blocks; per launch the megabytes in and out. With
-// a stride the lanes of a pixel read lie on every other 8 bytes, and a step costs 1 + strided of what it does else. Fitted to 3000
-// drawn layers (k 3 and 5, 8..512 channels, 600..2.5 million pixels): median error 4 to 7 %, 9 in 10 below 12 to 18 %. (What a tile
-// takes was scaled when the requests were put together: two row tiles 0.95 from int8 and 0.975 from fp32 of 67 and 23 layers, four row
-// tiles from fp32 1.035.)
-struct RowsCost {
+// a stride the lanes of a pixel read lie on every other 8 bytes, and a step costs 1 + strided of what it does else. Fitted to 4700
+// drawn layers (k 3 and 5, 8..512 channels, up to 2.5 million pixels): median error 4 to 5 %, 9 in 10 below 11 to 13 % from int8 and
+// 15 to 17 % from fp32. The tile it chooses takes 0.7 % more than the fastest of the four on average, one in twenty 6 % or more.
+struct RowsCoef {
     float start, step, stage, cu_step, cu_place, cu_block, strided, in_mb, out_mb;
 };
+struct RowsCost {
+    int resident;
+    RowsCoef at;
+};
 struct RowsConfig {
-    int fm, fn, resident;
+    int fm, fn;
     RowsCost i8, f32;
 };
 constexpr RowsConfig kRowsConfigs[] = {
-    {2, 2, 5, {2.648f, 0.098f, 0.969f, 0.029f, 0.035f, 0.294f, 0.504f, 0.028f, 0.084f}, {2.228f, 0.123f, 1.339f, 0.026f, 0.13f, 0.246f, 0.858f, 0.053f, 0.097f}},
-    {2, 4, 4, {2.918f, 0.179f, 1.057f, 0.028f, 0.052f, 0.469f, 0.436f, 0.037f, 0.088f}, {2.53f, 0.254f, 1.273f, 0.f, 0.172f, 0.445f, 0.535f, 0.064f, 0.095f}},
-    {4, 2, 4, {2.723f, 0.12f, 1.003f, 0.072f, 0.043f, 0.458f, 0.366f, 0.f, 0.105f}, {2.446f, 0.187f, 1.215f, 0.058f, 0.152f, 0.367f, 0.627f, 0.045f, 0.112f}},
-    {4, 4, 3, {3.078f, 0.24f, 1.033f, 0.055f, 0.067f, 0.789f, 0.352f, 0.f, 0.115f}, {2.79f, 0.362f, 1.156f, 0.f, 0.217f, 0.726f, 0.375f, 0.049f, 0.121f}},
+    {2, 2, {6, {3.02f, 0.062f, 0.813f, 0.05f, 0.033f, 0.186f, 0.397f, 0.057f, 0.113f}}, {5, {2.65f, 0.1f, 1.21f, 0.035f, 0.143f, 0.143f, 0.897f, 0.067f, 0.124f}}},
+    {2, 4, {5, {3.21f, 0.106f, 0.818f, 0.055f, 0.045f, 0.38f, 0.504f, 0.057f, 0.12f}}, {4, {2.94f, 0.171f, 0.983f, 0.f, 0.212f, 0.439f, 0.613f, 0.066f, 0.125f}}},
+    {4, 2, {4, {3.09f, 0.067f, 0.811f, 0.094f, 0.034f, 0.271f, 0.279f, 0.032f, 0.138f}}, {4, {2.81f, 0.109f, 1.19f, 0.076f, 0.141f, 0.113f, 0.686f, 0.062f, 0.16f}}},
+    {4, 4, {3, {3.39f, 0.145f, 0.806f, 0.085f, 0.048f, 0.573f, 0.346f, 0.054f, 0.154f}}, {3, {3.06f, 0.249f, 1.14f, 0.f, 0.231f, 0.505f, 0.51f, 0.062f, 0.17f}}},
 };
 constexpr int kRowsConfigCount = (int)(sizeof(kRowsConfigs) / sizeof(kRowsConfigs[0]));
 }  // namespace
@@ -442,22 +540,27 @@ float conv_rows_cost(const ConvGeom& g_in, bool f32in, int out_bytes, int* confi
     size_t lds;
     bool fits = false;
     const int steps = rows_steps(g_in.C / g_in.groups, g_in.kh * g_in.kw);
+    // 2 % (four row tiles 4 %) per MB of weights beyond the first: every die fetches them all. (5 to 8 % is what layers of over 2 MB took
+    // more than the fit; 504 -> 264 k 5 on one 80x92 image 57 us with two row tiles, 65 with four.)
+    const float more_mb = std::max(0.f, (float)g_in.groups * rows_packed_weight_bytes(g_in.K / g_in.groups, g_in.C / g_in.groups, g_in.kh * g_in.kw) * 1e-6f - 1.f);
     const float in_mb = (float)g_in.N * g_in.C * g_in.H * g_in.W * (f32in ? 4e-6f : 1e-6f);
     const float out_mb = (float)g_in.N * g_in.K * g_in.OH * g_in.OW * 1e-6f * out_bytes;
     for (const int i : {0, 2, 1, 3}) {  // by pixels of a tile: one plan for two
         const RowsConfig& c = kRowsConfigs[i];
         if (i == 0 || i == 1) fits = rows_plan(g_in, c.fn, &ra, &lds);
         if (!fits) continue;
-        const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm), bpw = rows_blocks_per_workgroup(ra, blocks);
+        const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm), bpw = rows_blocks_per_workgroup(ra, blocks, c.fm);
         const int pairs = ra.rows_max * ra.VW2, oct = (ra.g.C / 8 + ra.stages - 1) / ra.stages;
         const float places = (float)(ra.stages * oct) * (pairs > 128 ? (float)((pairs + 255) / 256) : 1.f / (float)(256 / pairs));
         const int wgs = (int)std::min(((long)ra.n_tiles * ((blocks + bpw - 1) / bpw) * ra.g.groups + 255) / 256, 1l << 24);
-        const int side = std::min(c.resident, (int)(160 * 1024 / lds));
+        const RowsCost& cost = f32in ? c.f32 : c.i8;
+        const int side = std::min(cost.resident, (int)(160 * 1024 / rows_lds(lds, bpw, c.fm)));
         const float cu = (float)wgs, rounds = (float)((wgs + side - 1) / side);
-        const RowsCost& k = f32in ? c.f32 : c.i8;
+        const RowsCoef& k = cost.at;
         const float s = (float)(bpw * steps) * (g_in.sw > 1 ? 1.f + k.strided : 1.f);
-        const float t = k.start + rounds * (k.step * s + k.stage * (float)ra.stages) +
+        float t = k.start + rounds * (k.step * s + k.stage * (float)ra.stages) +
                         cu * (k.cu_step * s + k.cu_place * places + k.cu_block * (float)bpw) + k.in_mb * in_mb + k.out_mb * out_mb;
+        t *= 1.f + 0.01f * (float)c.fm * more_mb;
         if (t < best) best = t, *config = i;
     }
     return best;
@@ -473,22 +576,30 @@ hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out
     ra.img = fast_div((unsigned)(ra.g.OH * ra.strip_w)), ra.tw = fast_div((unsigned)ra.strip_w), ra.vh = fast_div((unsigned)ra.VH);
     ra.vw = fast_div((unsigned)ra.VW2), ra.ntx = fast_div((unsigned)ra.strips), ra.kw = fast_div((unsigned)ra.g.kw);
     ra.in_bytes = (unsigned)((size_t)ra.g.N * ra.g.Cs * ra.g.H * ra.g.W * (f32in ? 4 : 1));
+    ra.base = ra.g.C / 8 / ra.stages, ra.more = ra.g.C / 8 % ra.stages;
+    ra.count = fast_div((unsigned)ra.base), ra.count1 = fast_div((unsigned)ra.base + 1);
     ra.in_scale = in_scale;
     ra.in_half = in_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm);
-    ra.blocks_per_wg = rows_blocks_per_workgroup(ra, blocks);
+    ra.blocks_per_wg = rows_blocks_per_workgroup(ra, blocks, c.fm);
+    const int steps = rows_steps(ra.g.C, ra.g.kh * ra.g.kw);
+    ra.warm_steps = steps >= 24 ? steps : 0;
+    ra.consts = (int)((lds + 15) / 16 * 16);
+    lds = rows_lds(lds, ra.blocks_per_wg, c.fm);
     const dim3 grid((unsigned)ra.n_tiles, (unsigned)((blocks + ra.blocks_per_wg - 1) / ra.blocks_per_wg), (unsigned)g_in.groups);
     const int epi = pick_epilogue(ep, ra.g.K);
-#define OHIP_ROWS2(I_, FM_, FN_, E_)                                                                                         \
-    if (config == I_ && epi == E_) {                                                                                         \
-        if (!f32in) {                                                                                                        \
-            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, false>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, EpiArgs<E_>::of(ep)); \
-            return hipGetLastError();                                                                                        \
-        }                                                                                                                    \
-        if constexpr (E_ != EPI_GENERIC) {                                                                                   \
-            hipLaunchKernelGGL((conv_rows_kernel<FM_, FN_, E_, true>), grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, EpiArgs<E_>::of(ep)); \
-            return hipGetLastError();                                                                                        \
-        }                                                                                                                    \
+    auto go = [&](auto kernel, auto ea) {
+        if (lds > 64 * 1024) {  // (rows that fill the tile's share: the constants lie beyond it)
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024);
+            if (e != hipSuccess) return e;
+        }
+        launch(kernel, grid, dim3(256), lds, stream, (const int8_t*)x, wpk, out, ra, ea);
+        return hipGetLastError();
+    };
+#define OHIP_ROWS2(I_, FM_, FN_, E_)                                                                     \
+    if (config == I_ && epi == E_) {                                                                     \
+        if (!f32in) return go(conv_rows_kernel<FM_, FN_, E_, false>, EpiArgs<E_>::of(ep));               \
+        if constexpr (E_ != EPI_GENERIC) return go(conv_rows_kernel<FM_, FN_, E_, true>, EpiArgs<E_>::of(ep)); \
     }
 #define OHIP_ROWS(I_, FM_, FN_) \
     OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8) OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8_NONNEG) OHIP_ROWS2(I_, FM_, FN_, EPI_F32_P4) OHIP_ROWS2(I_, FM_, FN_, EPI_GENERIC)
