@@ -99,6 +99,18 @@ int otter_hip_stream_create(void** stream);
 int otter_hip_stream_destroy(void* stream);
 int otter_hip_stream_synchronize(void* stream);
 
+/* A sequence of launches made once and repeated as a whole, which spares the host 3 us a launch and the GPU 0.7. No counterpart in
+ * the reference. otter_hip_record_begin makes a stream of its own and records what this thread enqueues on it from then on (nothing
+ * runs); otter_hip_record_end ends that and gives the recording, or with recording == NULL drops it. Only kernel launches can be
+ * recorded: of this header, everything but the copies between host and device and otter_hip_conv_chain_forward's single launch. A
+ * recording reads and writes the buffers it was recorded with; otter_hip_record_launch enqueues it on any stream, one thread at a
+ * time. Wait for the last launch before otter_hip_record_destroy. */
+typedef struct otter_hip_recording otter_hip_recording_t;
+int otter_hip_record_begin(void** stream);
+int otter_hip_record_end(void* stream, otter_hip_recording_t** recording);
+int otter_hip_record_launch(otter_hip_recording_t* recording, void* stream);
+int otter_hip_record_destroy(otter_hip_recording_t* recording);
+
 /* ------------------------------------------------------------------------------------------------ */
 /* convolution layer                                                                                */
 /* ------------------------------------------------------------------------------------------------ */

@@ -86,7 +86,8 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_block_forward", "otter_hip_conv_block_set_plan", "otter_hip_conv_block_set_always", "otter_hip_conv_block_set_pair",
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
            "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
-           "otter_hip_conv_forward_residual_concat"]
+           "otter_hip_conv_forward_residual_concat",
+           "otter_hip_record_begin", "otter_hip_record_end", "otter_hip_record_launch", "otter_hip_record_destroy"]
 
 
 def load_cdll():

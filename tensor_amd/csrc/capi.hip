@@ -394,6 +394,71 @@ int otter_hip_stream_synchronize(void* stream) {
 }
 
 // -----------------------------------------------------------------------------------------------------
+// recorded launches
+// -----------------------------------------------------------------------------------------------------
+
+struct otter_hip_recording {
+    hipGraphExec_t exec = nullptr;
+};
+
+int otter_hip_record_begin(void** stream) {
+    if (!stream) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_record_begin: null");
+    hipStream_t s = nullptr;
+    // (non-blocking: other work on the null stream goes on meanwhile; relaxed: so do allocations)
+    OHIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    const hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed);
+    if (e != hipSuccess) {
+        (void)hipStreamDestroy(s);
+        return hip_fail(e, "hipStreamBeginCapture");
+    }
+    *stream = s;
+    return OTTER_HIP_OK;
+}
+
+int otter_hip_record_end(void* stream, otter_hip_recording_t** recording) {
+    if (recording) *recording = nullptr;
+    if (!stream) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_record_end: null");
+    hipGraph_t graph = nullptr;
+    hipError_t e = hipStreamEndCapture((hipStream_t)stream, &graph);
+    int rc = e == hipSuccess ? OTTER_HIP_OK : hip_fail(e, "hipStreamEndCapture");
+    if (rc == OTTER_HIP_OK && recording) {
+        // launches only: what the runtime makes of a recorded fill or copy is not what it makes of one that is issued
+        size_t n = 0;
+        std::vector<hipGraphNode_t> nodes;
+        e = hipGraphGetNodes(graph, nullptr, &n);
+        if (e == hipSuccess && n) nodes.resize(n), e = hipGraphGetNodes(graph, nodes.data(), &n);
+        bool launches = n > 0;
+        for (size_t i = 0; i < n && e == hipSuccess; ++i) {
+            hipGraphNodeType type;
+            if ((e = hipGraphNodeGetType(nodes[i], &type)) == hipSuccess) launches = launches && type == hipGraphNodeTypeKernel;
+        }
+        otter_hip_recording* r = nullptr;
+        if (e != hipSuccess) rc = hip_fail(e, "hipGraphGetNodes");
+        else if (!launches) rc = fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_record_end: kernel launches only, and at least one");
+        else if (!(r = new (std::nothrow) otter_hip_recording())) rc = fail(OTTER_HIP_ERR_ALLOC, "otter_hip_record_end: host allocation failed");
+        else if ((e = hipGraphInstantiate(&r->exec, graph, nullptr, nullptr, 0)) != hipSuccess) rc = hip_fail(e, "hipGraphInstantiate");
+        if (rc == OTTER_HIP_OK) *recording = r;
+        else delete r;
+    }
+    if (graph) (void)hipGraphDestroy(graph);
+    (void)hipStreamDestroy((hipStream_t)stream);
+    return rc;
+}
+
+int otter_hip_record_launch(otter_hip_recording_t* recording, void* stream) {
+    if (!recording) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_record_launch: null");
+    OHIP_CHECK(hipGraphLaunch(recording->exec, (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
+int otter_hip_record_destroy(otter_hip_recording_t* recording) {
+    if (!recording) return OTTER_HIP_OK;
+    (void)hipGraphExecDestroy(recording->exec);
+    delete recording;
+    return OTTER_HIP_OK;
+}
+
+// -----------------------------------------------------------------------------------------------------
 // convolution
 // -----------------------------------------------------------------------------------------------------
 
