@@ -196,6 +196,24 @@ PyObject* conv_chain(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 
 // (expand, depthwise, project, K, out_layout, x, n, h, w, residual or None, q_scale or None, q_round_mode, out or None,
 //  q or None, workspace or None, device) -> (out, q or None)
+// The form of a block that a single call runs in, or 0: as otter_hip_conv_block_launches says. The cost models of
+// otter_hip_conv_block_fastest are of the launches alone; of the host's time one launch takes 6.5 us a call, two 8.5 and three 11.
+// Their choice is taken where it is no more launches (128 -> 768 -> 128 on one 13x13 image 11.4 us a call in three, 8.3 in two;
+// 160 -> 960 -> 208 on 25 8x8 images 15.9 and 11.7). For more of them the two blobs between the layers have to be beyond 4 MB (two
+// launches) and 8 MB, which keep the GPU busy for longer than that: 48 -> 288 -> 32 on 16 27x27 images 12.6 us in one, 11.7 in two; but 24 ->
+// 144 -> 40 on 49 10x9 images 8.9 in one, 11 in three. A workspace that is given has to hold them. (workspace: its bytes, < 0:
+// none; *bytes: what the form needs)
+int block_form(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p, int n, int h, int w, int64_t workspace,
+               size_t* bytes) {
+    const int as_is = otter_hip_conv_block_launches(e, d, p, n, h, w);
+    int form = as_is < 1 ? 0 : otter_hip_conv_block_fastest(e, d, p, n, h, w);
+    if (form < 1) return 0;
+    *bytes = otter_hip_conv_block_form_workspace_bytes(e, d, p, form, n, h, w);
+    if (form > as_is && *bytes < ((size_t)(form == 2 ? 4 : 8) << 20))
+        *bytes = otter_hip_conv_block_form_workspace_bytes(e, d, p, form = as_is, n, h, w);
+    return workspace >= 0 && (size_t)workspace < *bytes ? 0 : form;
+}
+
 PyObject* conv_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     NEED(16)
     try {
@@ -219,17 +237,18 @@ PyObject* conv_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         at::Tensor made, made_q, made_ws;
         if (!out) out = &(made = device_empty(count, type_of_layout(out_layout), device));
         if (!q && with_q) q = &(made_q = device_empty(count, at::kChar, device));
-        if (!ws) {
-            const size_t need = otter_hip_conv_block_layout_workspace_bytes(e, d, p, out_layout, n, ih, iw);
-            if (need) ws = &(made_ws = device_empty((int64_t)need, at::kChar, device));
-        }
+        size_t need = 0;
+        const int form = block_form(e, d, p, n, ih, iw, ws ? (int64_t)bytes_of(*ws) : -1, &need);
+        if (!ws && !form) need = otter_hip_conv_block_layout_workspace_bytes(e, d, p, out_layout, n, ih, iw);
+        if (!ws && need) ws = &(made_ws = device_empty((int64_t)need, at::kChar, device));
         void* stream = stream_now();
         const void* px = x ? x->data_ptr() : nullptr;
         const float* pr = res ? (const float*)res->data_ptr() : nullptr;
         void *po = out->data_ptr(), *pq = q ? q->data_ptr() : nullptr, *pw = ws ? ws->data_ptr() : nullptr;
         const size_t wb = ws ? bytes_of(*ws) : 0;
         Py_BEGIN_ALLOW_THREADS
-        rc = otter_hip_conv_block_forward(e, d, p, px, n, ih, iw, pr, po, out_layout, pq, q_scale, q_round, pw, wb, stream);
+        rc = form ? otter_hip_conv_block_forward_form(e, d, p, form, px, n, ih, iw, pr, po, out_layout, pq, q_scale, q_round, pw, wb, stream)
+                      : otter_hip_conv_block_forward(e, d, p, px, n, ih, iw, pr, po, out_layout, pq, q_scale, q_round, pw, wb, stream);
         Py_END_ALLOW_THREADS
         if (rc) return raise_status(rc);
         PyObject* o = result(a[12], *out);
