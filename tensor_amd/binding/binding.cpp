@@ -194,8 +194,6 @@ PyObject* conv_chain(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     }
 }
 
-// (expand, depthwise, project, K, out_layout, x, n, h, w, residual or None, q_scale or None, q_round_mode, out or None,
-//  q or None, workspace or None, device) -> (out, q or None)
 // The form of a block that a single call runs in, or 0: as otter_hip_conv_block_launches says. The cost models of
 // otter_hip_conv_block_fastest are of the launches alone; of the host's time one launch takes 6.5 us a call, two 8.5 and three 11.
 // Their choice is taken where it is no more launches (128 -> 768 -> 128 on one 13x13 image 11.4 us a call in three, 8.3 in two;
@@ -214,6 +212,8 @@ int block_form(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter
     return workspace >= 0 && (size_t)workspace < *bytes ? 0 : form;
 }
 
+// (expand, depthwise, project, K, out_layout, x, n, h, w, residual or None, q_scale or None, q_round_mode, out or None,
+//  q or None, workspace or None, device) -> (out, q or None)
 PyObject* conv_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
     NEED(16)
     try {
@@ -238,7 +238,8 @@ PyObject* conv_block(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         if (!out) out = &(made = device_empty(count, type_of_layout(out_layout), device));
         if (!q && with_q) q = &(made_q = device_empty(count, at::kChar, device));
         size_t need = 0;
-        const int form = block_form(e, d, p, n, ih, iw, ws ? (int64_t)bytes_of(*ws) : -1, &need);
+        const bool usual = out_layout == OTTER_HIP_F32_P4 || out_layout == OTTER_HIP_I8_P8;  // (any other rules out a single launch)
+        const int form = usual ? block_form(e, d, p, n, ih, iw, ws ? (int64_t)bytes_of(*ws) : -1, &need) : 0;
         if (!ws && !form) need = otter_hip_conv_block_layout_workspace_bytes(e, d, p, out_layout, n, ih, iw);
         if (!ws && need) ws = &(made_ws = device_empty((int64_t)need, at::kChar, device));
         void* stream = stream_now();
