@@ -207,7 +207,7 @@ int block_form(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter
     int form = as_is < 1 ? 0 : otter_hip_conv_block_fastest(e, d, p, n, h, w);
     if (form < 1) return 0;
     *bytes = otter_hip_conv_block_form_workspace_bytes(e, d, p, form, n, h, w);
-    if (form > as_is && *bytes < ((size_t)(form == 2 ? 4 : 8) << 20))
+    if (form > as_is && *bytes < ((size_t)(form == 2 ? 4 : 12) << 20))
         *bytes = otter_hip_conv_block_form_workspace_bytes(e, d, p, form = as_is, n, h, w);
     return workspace >= 0 && (size_t)workspace < *bytes ? 0 : form;
 }
