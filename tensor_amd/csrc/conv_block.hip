@@ -52,6 +52,11 @@ struct BlockArgs {
     int GA, GD;           // 16-pixel groups: the band's input rows, the band's output rows
     int npairsP, itemsP;  // project: channel pairs (32 channels), pairs x GD
     unsigned inv_w;       // ceil(2^20 / W)
+    // dividers: bands, cgE, pixels of a band of H / bands and of one more row, cpr, rpi, npairsP. (Divisions were most of the set-up's
+    // vector instructions, and beside a workgroup of 16 waves nothing runs on a compute unit: 12.1 -> 11.5 us for 64 -> 384 -> 64 @14x14
+    // b64, 8.2 -> 7.4 with 128 expanded channels.)
+    FastDiv by_bands, by_cge, by_px0, by_px1, by_cpr, by_rpi, by_pairs;
+    int rows0;            // H / bands
     int lds_e, lds_d, lds_c1, lds_c2;  // byte offsets: expanded lines, depthwise results, constants of the two layers
     int lds_c3, lds_r;                 // constants of the project layer, the band's shortcut elements (fp32 result only)
     // The slices of a band dealt to `split` workgroups (grid.z), `spp` consecutive slices each: each adds its slices
@@ -83,7 +88,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
     const int band = blockIdx.x, n = blockIdx.y;
     const int s_begin = blockIdx.z * a.spp, s_end = min(s_begin + a.spp, a.slices);
     // bands of nearly equal height (at most RB rows): band b owns rows [b * H / bands, (b + 1) * H / bands)
-    const int r0 = band * a.H / a.bands, rows = (band + 1) * a.H / a.bands - r0;
+    const int r0 = (int)div_by((unsigned)(band * a.H), a.by_bands), rows = (int)div_by((unsigned)((band + 1) * a.H), a.by_bands) - r0;
     const int in_row0 = max(r0 - 1, 0), in_row1 = min(r0 + rows, a.H - 1);
     const int in_pix0 = in_row0 * a.W, in_pixN = (in_row1 + 1) * a.W - in_pix0;
     const int out_pixN = rows * a.W;
@@ -119,7 +124,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
         const int8_t* xi = a.x + (size_t)n * a.Cin8 * a.HW * 8;
         auto load_x = [&](int i, v2i& lo, v2i& hi) {
             const int l = i & 63, t = i >> 6;
-            const int ga = t / a.cgE, cg = t - ga * a.cgE;
+            const int ga = (int)div_by((unsigned)t, a.by_cge), cg = t - ga * a.cgE;
             const int pix = ga * 16 + (l & 15), oct = 8 * cg + 2 * (l >> 4);
             lo = hi = v2i{0, 0};
             if (i < nX && pix < in_pixN) {
@@ -148,7 +153,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
         const v4i* rg = reinterpret_cast<const v4i*>(a.e3.residual) + (size_t)n * (a.Cout / 4) * a.HW + r0 * a.W;
         const int n4 = with_res ? (a.Cout / 4) * out_pixN : 0;
         auto load_res = [&](int i) {
-            const int c4 = i / out_pixN, px = i - c4 * out_pixN;
+            const int c4 = (int)(rows == a.rows0 ? div_by((unsigned)i, a.by_px0) : div_by((unsigned)i, a.by_px1)), px = i - c4 * out_pixN;
             return rg[(size_t)c4 * a.HW + px];
         };
         // first round
@@ -185,7 +190,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
     // B: lane column -> (row within the item, column chunk); selectors that move a row's tap into the lane's byte of
     // the block-diagonal weight operand (dw_mfma_pack_weights: lane (r, g) holds, for pixel slot e, the tap
     // dx = 2g + e - 1 - r/4 of channel 4t + r%4 at byte 8e + 4t + r%4, zero when dx is outside the window)
-    const int row_sub = p / a.cpr, nx = p - row_sub * a.cpr;
+    const int row_sub = (int)div_by((unsigned)p, a.by_cpr), nx = p - row_sub * a.cpr;
     const bool laneB = row_sub < a.rpi;
     const int oxB = 4 * nx + q;
     unsigned selB[2];
@@ -212,7 +217,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
     auto load_wP = [&](int s) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-            const int prP = min(wave + WV * i, a.itemsP - 1) % a.npairsP;
+            const int it = min(wave + WV * i, a.itemsP - 1), prP = it - (int)div_by((unsigned)it, a.by_pairs) * a.npairsP;
 #pragma unroll
             for (int ks = 0; ks < KSS; ++ks) {
                 const int cgp = min(s * KSS + ks, a.cgP - 1);
@@ -262,10 +267,10 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
                     const int pix = ga * 16 + p;
                     if (pix < in_pixN) {
                         const unsigned ipix = (unsigned)(in_pix0 + pix);
-                        const unsigned iy = (ipix * a.inv_w) >> 20;
-                        const unsigned ix = ipix - iy * (unsigned)a.W;
+                        const unsigned iy = __umul24(ipix, a.inv_w) >> 20;  // (a full multiplication takes four times as long)
+                        const unsigned ix = ipix - __umul24(iy, (unsigned)a.W);
                         const int er = (int)iy - (r0 - 1);
-                        *reinterpret_cast<v2i*>(eo + er * a.pitch + (ix + 2) * 8) = r;
+                        *reinterpret_cast<v2i*>(eo + __mul24(er, a.pitch) + (ix + 2) * 8) = r;
                     }
                 }
             }
@@ -274,7 +279,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
         // ================= B: depthwise =================
         if (s + 1 < s_end) load_wA(s + 1);
         {
-            const int nrc = (rows + a.rpi - 1) / a.rpi;
+            const int nrc = (int)div_by((unsigned)(rows + a.rpi - 1), a.by_rpi);
 #pragma unroll
             for (int k = 0; k < OPW; ++k) {
             const int ol = wave % noct + WV * k;
@@ -307,15 +312,15 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
                     v4i c0 = zero4, c1 = zero4;
 #pragma unroll
                     for (int dy = 0; dy < 3; ++dy) {
-                        const v4i b = *reinterpret_cast<const v4i*>(ei + (orc + dy) * a.pitch);
+                        const v4i b = *reinterpret_cast<const v4i*>(ei + __mul24(orc + dy, a.pitch));
                         c0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(wB[dy][0], b, dy ? c0 : zero4, 0, 0, 0);
                         c1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(wB[dy][1], b, dy ? c1 : zero4, 0, 0, 0);
                     }
                     const int a8[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
                     const v2i r = epi8_quant_i8p8<NONNEG, 0>(a.e2, prm, a8);
                     if (laneB && orow < rows && oxB < a.W) {
-                        const int pix = orow * a.W + oxB;
-                        *reinterpret_cast<v2i*>(dout + (size_t)((pix >> 4) * kqs) * 256 + (pix & 15) * 16) = r;
+                        const int pix = __mul24(orow, a.W) + oxB;
+                        *reinterpret_cast<v2i*>(dout + (pix >> 4) * kqs * 256 + (pix & 15) * 16) = r;
                     }
                 }
             }
@@ -328,7 +333,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
         for (int i = 0; i < NI; ++i) {
             const int it = wave + WV * i;
             if (it < a.itemsP) {  // wave-uniform
-                const int gd = it / a.npairsP;
+                const int gd = (int)div_by((unsigned)it, a.by_pairs);
 #pragma unroll
                 for (int ks = 0; ks < KSS; ++ks) {
                     if (s * KSS + ks < a.cgP) {
@@ -392,7 +397,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
     for (int i = 0; i < NI; ++i) {
         const int it = wave + WV * i;
         if (it >= a.itemsP) break;  // wave-uniform
-        const int prP = it % a.npairsP, gd = it / a.npairsP;
+        const int gd = (int)div_by((unsigned)it, a.by_pairs), prP = it - gd * a.npairsP;
         const int ch0 = 32 * prP + 8 * q;
         const int pix = gd * 16 + p;
         if (ch0 >= a.Cout || pix >= out_pixN) continue;
@@ -546,6 +551,9 @@ bool conv_block_plan(const ConvGeom& ge, const ConvGeom& gp, int force_rb, int f
         a.GA = (std::min(RB + 2, H) * W + 15) / 16, a.GD = (RB * W + 15) / 16;
         a.npairsP = npairsP, a.itemsP = npairsP * a.GD;
         a.inv_w = ((1u << 20) + W - 1) / W;
+        a.rows0 = H / a.bands;
+        a.by_bands = fast_div((unsigned)a.bands), a.by_cge = fast_div((unsigned)cgE), a.by_cpr = fast_div((unsigned)cpr), a.by_rpi = fast_div((unsigned)rpi);
+        a.by_px0 = fast_div((unsigned)(a.rows0 * W)), a.by_px1 = fast_div((unsigned)((a.rows0 + 1) * W)), a.by_pairs = fast_div((unsigned)npairsP);
         a.lds_e = off[0], a.lds_d = off[1], a.lds_c1 = off[2], a.lds_c2 = off[3], a.lds_c3 = off[4], a.lds_r = off[5];
     }
     return true;
