@@ -39,7 +39,8 @@ template <int FM, int FN, int WM, int WN, int EPI, int LOGP, int S = 1, int D = 
 __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
                                                            void* __restrict__ out, ConvGeom g, Epilogue ep, int m_tiles16,
                                                            int c_groups, int r_max, int cb, int tiles_per_img, int prm_ofs,
-                                                           int total_tiles, unsigned in_bytes, int tile_inv) {
+                                                           int total_tiles, unsigned in_bytes, int tile_inv, FastDiv by_ow,
+                                                           FastDiv by_tiles) {
     static_assert(WM * WN == 4 && FM % 2 == 0, "four waves, row fragments in pairs");
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     constexpr int PT = WN * FN * 16;
@@ -83,14 +84,14 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
         int wg = wg0;
         const int per = total_tiles / 8;
         if (per > 0 && wg < per * 8) wg = (wg % 8) * per + wg / 8;
-        n = wg / tiles_per_img;
-        p0 = (wg % tiles_per_img) * PT;
+        n = (int)div_by((unsigned)wg, by_tiles);
+        p0 = (wg - n * tiles_per_img) * PT;
     };
     // Issue the LDS-DMA transfers of one (tile, channel block): this wave moves octets wave, wave+4, ...
     auto stage = [&](int n, int p0, int cb0) {
         const int p_last = min(p0 + PT, OHW) - 1;
-        const int r_lo = p0 / g.OW;
-        const int R = (p_last / g.OW - r_lo) * S + 2 * D + 1;
+        const int r_lo = (int)div_by((unsigned)p0, by_ow);
+        const int R = ((int)div_by((unsigned)p_last, by_ow) - r_lo) * S + 2 * D + 1;
         if constexpr (LOGP == 9) {
             // 512-byte lines: one instruction moves a row of BOTH octets of a pair (adjacent lines in LDS): lanes 0-31
             // the first octet, lanes 32-63 the second, 16 bytes = pixels 2*pp-2 and 2*pp-1 each
@@ -165,7 +166,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
     auto fix_odd = [&](int p0) {
         if constexpr (!ODDW) return;
         const int p_last = min(p0 + PT, OHW) - 1;
-        const int R = (p_last / g.OW - p0 / g.OW) * S + 2 * D + 1;
+        const int R = (int)(div_by((unsigned)p_last, by_ow) - div_by((unsigned)p0, by_ow)) * S + 2 * D + 1;
         // lane = octet of the stage (at most 64 octets = 512 channels per stage); the wave that staged octet oc: pairs go
         // round the four waves (512-byte lines, both octets of a pair in one transfer), or single octets do
         const int oc = lane;
@@ -186,7 +187,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
     int bcc[FN];
     for (int wg0 = blockIdx.x; wg0 < total_tiles; wg0 += gridDim.x) {
         tile_of(wg0, n, p0);
-        const int r_lo = p0 / g.OW;
+        const int r_lo = (int)div_by((unsigned)p0, by_ow);
 
         // LDS address of this lane's pixel (tap 0,0) per fragment, octet pair lane/16 of the current k-chunk; walks
         // forward by one chunk after the ninth tap and is wound back at the end of a stage
@@ -198,7 +199,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
 #pragma unroll
             for (int f = 0; f < FN; ++f) {
                 const int pix = min(p0 + (wn * FN + f) * 16 + (lane & 15), OHW - 1);
-                const int oy = pix / g.OW, ox = pix % g.OW;
+                const int oy = (int)div_by((unsigned)pix, by_ow), ox = pix - oy * g.OW;
                 bcc[f] = (oy - r_lo) * S * 2 * PITCH + (ox * S - g.pw + 2) * 8 + (lane >> 4) * pair_bytes;
             }
         }
@@ -418,7 +419,8 @@ hipError_t launch_halo_w(const int8_t* x, const int8_t* wpk, void* out, const Co
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W);
     launch(kern, dim3(grid_x, m_blocks), dim3(256), prm_ofs + 3 * WM * FM * 16 * sizeof(float), stream, x, wpk,
                        out, g, ep, mpad / 16, igemm_channel_groups(g.C), pl.r_max, pl.cb, pl.tiles_per_img, prm_ofs,
-                       total_tiles, in_bytes, halo_tile_invariant(WN * FN * 16, g.OW, g.OH * g.OW) ? 1 : 0);
+                       total_tiles, in_bytes, halo_tile_invariant(WN * FN * 16, g.OW, g.OH * g.OW) ? 1 : 0, fast_div((unsigned)g.OW),
+                       fast_div((unsigned)pl.tiles_per_img));
     return hipGetLastError();
 }
 

@@ -42,11 +42,20 @@ struct IgemmCfg {
 // INF: the input is the fp32 Float8 blob of a pointwise layer ([N][C/8][H*W][8 floats]); the loader reads the 32 bytes
 // of a pixel's octet and quantizes them with the layer's input scale and rounding primitive on the way into LDS
 // (quantize_to_int8, Tensor/ConvolutionLayer.cpp:770-775, without its own pass over the blob).
+// Dividers: pixels and columns of an image, reduction steps of a tap, the kernel's width. (Every division of the kernel was 20 to 30
+// instructions, two of them per reduction step.)
+struct IgemmDiv {
+    FastDiv ohw, ow, cg, kw;
+    static IgemmDiv of(const ConvGeom& g) {
+        return {fast_div((unsigned)(g.OH * g.OW)), fast_div((unsigned)g.OW), fast_div((unsigned)igemm_channel_groups(g.C)), fast_div((unsigned)g.kw)};
+    }
+};
+
 template <int TM, int TN, int WM, int WN, int EPI, int KC, bool INF = false>
 __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk,
                                                          void* __restrict__ out, ConvGeom g, Epilogue ep, int m_tiles16,
                                                          int c_groups, int n_pix_tiles, const float* __restrict__ in_scale_p,
-                                                         float in_half, JoinParam<EPI> ja) {
+                                                         float in_half, JoinParam<EPI> ja, IgemmDiv by) {
     using Cfg = IgemmCfg<TM, TN, WM, WN>;
     constexpr int FM = Cfg::FM, FN = Cfg::FN;
     constexpr int NBUF = KC == 1 ? 2 : KC;
@@ -90,14 +99,14 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
     // ---- per-thread constants of the activation loader -------------------------------------------
     // (image, pixel) of a global pixel index: the tile's first pixel is divided once for the whole workgroup (uniform
     // operands), a lane then only steps over at most one image boundary; images smaller than a tile take the division
-    const unsigned n_tile = tile_base / (unsigned)OHW;
+    const unsigned n_tile = div_by(tile_base, by.ohw);
     const unsigned rem_tile = tile_base - n_tile * (unsigned)OHW;
     auto locate = [&](unsigned ofs, unsigned& n, unsigned& pix) {  // pixel tile_base + ofs, ofs < TN
         n = n_tile, pix = rem_tile + ofs;
         if ((unsigned)OHW >= (unsigned)TN) {
             if (pix >= (unsigned)OHW) pix -= (unsigned)OHW, ++n;
         } else {
-            const unsigned k = pix / (unsigned)OHW;
+            const unsigned k = div_by(pix, by.ohw);
             n += k, pix -= k * (unsigned)OHW;
         }
     };
@@ -119,7 +128,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
         if (pointwise) {
             px_ofs = img + (int)pix * 8;
         } else {
-            const int oy = (int)(pix / (unsigned)g.OW), ox = (int)pix - oy * g.OW;
+            const int oy = (int)div_by(pix, by.ow), ox = (int)pix - oy * g.OW;
             iy0 = oy * g.sh - g.ph;
             ix0 = ox * g.sw - g.pw;
             px_ofs = img + (iy0 * g.W + ix0) * 8;
@@ -144,23 +153,23 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
 
     auto load_global = [&](int kc, int q) {
         if (tpk > 1) {  // (uniform)
-            const int per = 4 / tpk;
+            const int per = tpk == 2 ? 2 : 1, ps = per - 1;  // (two or four taps share a step)
 #pragma unroll
             for (int r = 0; r < Cfg::B_V; ++r) {
                 const int j = j0 + r * J_STEP;
-                const int tap = kc * tpk + j / per;
-                const int u = tap / g.kw, v = tap - u * g.kw;
+                const int tap = kc * tpk + (j >> ps);
+                const int u = (int)div_by((unsigned)tap, by.kw), v = tap - u * g.kw;
                 const int iy = iy0 + u * g.dh, ix = ix0 + v * g.dw;
                 const bool inb = pvalid && tap < g.kh * g.kw && iy >= 0 && iy < g.H && ix >= 0 && ix < g.W;
-                const int o0 = 2 * (j % per);
+                const int o0 = 2 * (j & ps);
                 const unsigned v_lo = (unsigned)(px_ofs + ((u * g.dh) * g.W + v * g.dw) * 8 + o0 * HW * 8);
                 breg[q][r][0] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, (int)(inb && o0 < C8 ? v_lo : IG_OOB), 0, 0));
                 breg[q][r][1] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(
                     rin, (int)(inb && o0 + 1 < C8 ? v_lo + (unsigned)(HW * 8) : IG_OOB), 0, 0));
             }
         } else {
-        const int tap = kc / c_groups, cgp = kc % c_groups;
-        const int u = tap / g.kw, v = tap % g.kw;
+        const int tap = (int)div_by((unsigned)kc, by.cg), cgp = kc - tap * c_groups;
+        const int u = (int)div_by((unsigned)tap, by.kw), v = tap - u * g.kw;
         bool inb = pvalid;
         if (!pointwise) {
             const int iy = iy0 + u * g.dh, ix = ix0 + v * g.dw;
@@ -322,7 +331,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
             if (wide) {
                 if (pp >= (unsigned)OHW) pp -= (unsigned)OHW, ++nn;
             } else {
-                nn = gpo / (unsigned)OHW;
+                nn = div_by(gpo, by.ohw);
                 pp = gpo - nn * (unsigned)OHW;
             }
             col_ok[j] = gpo < total_pix;
@@ -406,7 +415,7 @@ __global__ void __launch_bounds__(256) conv_igemm_kernel(const int8_t* __restric
                     if (wide) {
                         if (pp >= (unsigned)OHW) pp -= (unsigned)OHW, ++nn;
                     } else {
-                        nn = gpo / (unsigned)OHW;
+                        nn = div_by(gpo, by.ohw);
                         pp = gpo - nn * (unsigned)OHW;
                     }
                     const int n = (int)nn, pix = (int)pp;
@@ -495,7 +504,7 @@ static hipError_t launch_igemm_k(const int8_t* x, const int8_t* wpk, void* out, 
     const int m_tiles = (g.K + TM - 1) / TM;  // row blocks that hold at least one real channel (the rows are padded further)
     const int grid_z = g.Cs ? g.Cs / g.C : 1;  // groups of a grouped convolution
     launch((conv_igemm_kernel<TM, TN, WM, WN, EPI, KC>), dim3(n_pix_tiles, m_tiles, grid_z), dim3(256), 0,
-                       stream, x, wpk, out, g, ep, mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, (const float*)nullptr, 0.f, JoinParam<EPI>::of(ep));
+                       stream, x, wpk, out, g, ep, mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, (const float*)nullptr, 0.f, JoinParam<EPI>::of(ep), IgemmDiv::of(g));
     return hipGetLastError();
 }
 
@@ -509,7 +518,7 @@ static hipError_t launch_igemm_f32in(const float* x, const int8_t* wpk, void* ou
     const dim3 grid(n_pix_tiles, (g.K + TM - 1) / TM, 1);
 #define OHIP_IGF(E_)                                                                                                        \
     launch((conv_igemm_kernel<TM, TN, WM, WN, E_, 1, true>), grid, dim3(256), 0, stream, (const int8_t*)x, wpk, out, g, ep, \
-                       mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, in_scale, in_half, NoJoin{})
+                       mpad / 16, igemm_channel_groups(g.C), n_pix_tiles, in_scale, in_half, NoJoin{}, IgemmDiv::of(g))
     switch (pick_epilogue(ep, g.K)) {
     case EPI_I8_P8: OHIP_IGF(EPI_I8_P8); break;
     case EPI_I8_P8_NONNEG: OHIP_IGF(EPI_I8_P8_NONNEG); break;
