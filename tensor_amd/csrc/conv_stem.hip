@@ -179,6 +179,7 @@ __global__ void __launch_bounds__(256) conv_stem3x3_kernel(const void* __restric
 // padding columns), rows outside the image are zeros.
 struct StemPlan {
     int R, strips, cgs, RIN, pitch_dw, vec;
+    FastDiv by_strips, by_cgs;
     float inv_pitch, inv_c;
 };
 
@@ -194,7 +195,7 @@ __global__ void __launch_bounds__(256) conv_stem3x3_lds_kernel(const void* __res
     extern __shared__ unsigned stem_lds[];
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int img = (int)blockIdx.x / p.strips, strip = (int)blockIdx.x - img * p.strips;
+    const int img = (int)div_by(blockIdx.x, p.by_strips), strip = (int)blockIdx.x - img * p.strips;
     const int S = g.sh, C = CT ? CT : g.C;
     constexpr int NC = CT ? CT : STEM_LDS_MAX_C;
 
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(256) conv_stem3x3_lds_kernel(const void* __res
     const unsigned shift = 8u * (unsigned)(lc0 & 3);
     const int OHW = g.OH * g.OW;
     for (int it = wave; it < items; it += 4) {
-        const int orow = it / p.cgs, cg = it - orow * p.cgs;
+        const int orow = (int)div_by((unsigned)it, p.by_cgs), cg = it - orow * p.cgs;
         const int r = min(S * orow + kg, p.RIN - 1);  // (kernel row 3 does not exist: its bytes meet zero weights)
         const unsigned* line = stem_lds + r * C * p.pitch_dw + (lc0 >> 2) + 4 * S * cg;
         v4i b = {0, 0, 0, 0};
@@ -374,6 +375,7 @@ static bool stem_lds_plan(const ConvGeom& g, StemPlan* p, size_t* lds_bytes) {
         const size_t bytes = (size_t)RIN * g.C * pitch_dw * 4;
         if (bytes > 64 * 1024) continue;
         p->R = R, p->strips = (g.OH + R - 1) / R, p->cgs = cgs, p->RIN = RIN, p->pitch_dw = pitch_dw, p->vec = 0;
+        p->by_strips = fast_div((unsigned)p->strips), p->by_cgs = fast_div((unsigned)cgs);
         p->inv_pitch = 1.0f / (float)pitch_dw, p->inv_c = 1.0f / (float)g.C;
         *lds_bytes = bytes;
         return true;

@@ -110,15 +110,15 @@ struct CopyOp {
 
 template <typename TI, typename TO, int SP, int DP, int V, class Op>
 __global__ void __launch_bounds__(256) ew_kernel(const TI* __restrict__ src, TO* __restrict__ dst, int N, int C, int HW,
-                                                 unsigned stride, Op op) {
-    // 32-bit indices (the C ABI refuses tensors of 2^31 elements or more): 64-bit divisions would cost more vector
-    // instructions than the operation itself
+                                                 unsigned stride, FastDiv by_hw, FastDiv by_cv, Op op) {
+    // 32-bit indices (the C ABI refuses tensors of 2^31 elements or more), and dividers that come with the arguments: divisions were
+    // more vector instructions than the operation itself
     const unsigned cv_count = (unsigned)(C / V);
     const unsigned total = (unsigned)N * cv_count * (unsigned)HW;
     for (unsigned idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += stride) {  // (no gridDim: 256 bytes of hidden arguments)
-        const unsigned r = idx / (unsigned)HW;
+        const unsigned r = div_by(idx, by_hw);
         const int pix = (int)(idx - r * (unsigned)HW);
-        const int n = (int)(r / cv_count);
+        const int n = (int)div_by(r, by_cv);
         const int cv = (int)(r - (unsigned)n * cv_count);
         TI in[V];
         TO out[V];
@@ -136,7 +136,7 @@ static hipError_t launch_ew(const TI* src, TO* dst, int N, int C, int HW, Op op,
     size_t blocks = (total + 255) / 256;
     if (blocks > (1u << 20)) blocks = 1u << 20;
     launch((ew_kernel<TI, TO, SP, DP, V, Op>), dim3((unsigned)blocks), dim3(256), 0, stream, src, dst, N, C,
-                       HW, (unsigned)blocks * 256u, op);
+                       HW, (unsigned)blocks * 256u, fast_div((unsigned)HW), fast_div((unsigned)(C / V)), op);
     return hipGetLastError();
 }
 
@@ -163,13 +163,13 @@ hipError_t dispatch_ew(const TI* src, int sp, TO* dst, int dp, int N, int C, int
 template <typename T>
 __global__ void __launch_bounds__(256) pad_pack8_kernel(const T* __restrict__ src, int sp, int8_t* __restrict__ dst, int N,
                                                         int C, int Cp, int HW, const float* __restrict__ scale,
-                                                        int round_mode) {
+                                                        int round_mode, FastDiv by_hw, FastDiv by_c) {
     const unsigned total = (unsigned)N * (unsigned)(Cp / 8) * (unsigned)HW;
     const unsigned idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= total) return;
-    const unsigned r = idx / (unsigned)HW;
+    const unsigned r = div_by(idx, by_hw);
     const int pix = (int)(idx - r * (unsigned)HW);
-    const int n = (int)(r / (unsigned)(Cp / 8));
+    const int n = (int)div_by(r, by_c);
     const int o = (int)(r - (unsigned)n * (unsigned)(Cp / 8));
     int q[8];
 #pragma unroll
@@ -195,10 +195,10 @@ hipError_t run_pad_pack8(const void* src, bool src_is_float, int sp, int8_t* dst
     const unsigned blocks = (unsigned)((total + 255) / 256);
     if (src_is_float)
         launch(pad_pack8_kernel<float>, dim3(blocks), dim3(256), 0, stream, (const float*)src, sp, dst, N, C, Cp,
-                           HW, scale, round_mode);
+                           HW, scale, round_mode, fast_div((unsigned)HW), fast_div((unsigned)(Cp / 8)));
     else
         launch(pad_pack8_kernel<int8_t>, dim3(blocks), dim3(256), 0, stream, (const int8_t*)src, sp, dst, N, C,
-                           Cp, HW, scale, round_mode);
+                           Cp, HW, scale, round_mode, fast_div((unsigned)HW), fast_div((unsigned)(Cp / 8)));
     return hipGetLastError();
 }
 
