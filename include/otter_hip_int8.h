@@ -233,6 +233,28 @@ int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* handle, const
                                            int part1_layout, float* out, int8_t* out_q, float q_scale, int q_round_mode,
                                            void* stream);
 
+/* Two pointwise layers in one launch, the second reading the int8 form of the first's result, which the reference quantizes in front
+ * of the second layer (Tensor/ConvolutionLayer.cpp:770-775) and keeps in memory in between. What they give is what the layers give one
+ * by one. An int8 result of the first layer is read by the second alone; an fp32 one meets another blob's channels in a ChannelShuffle
+ * as in otter_hip_conv_forward_shuffle, and the second layer reads the second half of the shuffled channels. The tail, zero but
+ * for such a result:
+ *   other, other_layout, other_odd   the other blob
+ *   first_half                       the first half of the shuffled channels, Float8
+ *   q_scale, q_round_mode            the second layer's input scale and rounding primitive
+ * in: Byte8. out_layout: Byte8 or Float4. otter_hip_conv_pair_launches: 1 where the call runs, 2 where the layers are separate calls or faster so;
+ * of the tail's pointers it only asks which are null. */
+typedef struct otter_hip_conv_tail {
+    const float* other;
+    int other_layout, other_odd;
+    float* first_half;
+    float q_scale;
+    int q_round_mode;
+} otter_hip_conv_tail;
+int otter_hip_conv_pair_launches(const otter_hip_conv_t* first, const otter_hip_conv_t* second, int n, int in_h, int in_w,
+                                 const otter_hip_conv_tail* tail, int out_layout);
+int otter_hip_conv_pair_forward(const otter_hip_conv_t* first, const otter_hip_conv_t* second, const void* in, int n, int in_h, int in_w,
+                                const otter_hip_conv_tail* tail, void* out, int out_layout, void* stream);
+
 /* A chain of layers that each map an int8 Byte8 blob to an int8 Byte8 blob (consecutive Convolution layers of a
  * Net, Tensor/Net.cpp:413-505 runs them one after the other): out = layer[n-1](... layer[0](in)). The result is what
  * n calls of otter_hip_conv_forward give. The intermediate blobs live in `workspace`

@@ -86,7 +86,7 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_block_forward", "otter_hip_conv_block_set_plan", "otter_hip_conv_block_set_always", "otter_hip_conv_block_set_pair",
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
            "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
-           "otter_hip_conv_forward_residual_concat",
+           "otter_hip_conv_forward_residual_concat", "otter_hip_conv_pair_launches", "otter_hip_conv_pair_forward",
            "otter_hip_record_begin", "otter_hip_record_end", "otter_hip_record_launch", "otter_hip_record_destroy"]
 
 
@@ -107,6 +107,12 @@ def load_binding():
     loader.exec_module(mod)
     mod.set_error(HipError)
     return mod
+
+
+class Tail(C.Structure):
+    """otter_hip_conv_tail: what otter_hip_conv_pair_forward does with the first layer's result."""
+    _fields_ = [("other", C.c_void_p), ("other_layout", C.c_int), ("other_odd", C.c_int), ("first_half", C.c_void_p),
+                ("q_scale", C.c_float), ("q_round_mode", C.c_int)]
 
 
 class Library:
@@ -318,6 +324,32 @@ class Library:
             expand.h, dw.h, project.h, form, self.ptr(x), n, h, w, given[0], given[1], out_layout, given[2], C.c_float(q_scale or 0.0),
             q_round_mode, self.ptr(workspace) if workspace.numel() else None, C.c_size_t(workspace.numel()), self.stream()))
         return out, q
+
+    def conv_pair_launches(self, first, second, n, h, w, **tail):
+        """otter_hip_conv_pair_launches: 1 where conv_pair runs the two layers as one launch, else 2."""
+        r = self.lib.otter_hip_conv_pair_launches(first.h, second.h, n, h, w, C.byref(self._tail(tail)), self._packed_out(second))
+        self._check(min(r, 0))
+        return r
+
+    def conv_pair(self, first, second, x, n, h, w, **tail):
+        """otter_hip_conv_pair_forward: x (int8 Byte8) through two pointwise layers; `tail` holds the fields of Tail, tensors for its
+        pointers. Returns the second layer's result."""
+        layout = self._packed_out(second)
+        out = self.empty(n * second.K * h * w, layout_dtype(layout))
+        self._check(self.lib.otter_hip_conv_pair_forward(first.h, second.h, self.ptr(x), n, h, w, C.byref(self._tail(tail)), self.ptr(out),
+                                                         layout, self.stream()))
+        return out
+
+    @staticmethod
+    def _packed_out(conv):
+        return F32_P4 if conv.out_kind == OUT_F32 else I8_P8
+
+    @staticmethod
+    def _tail(fields):
+        t = Tail(q_round_mode=ROUND_SSE)
+        for k, v in fields.items():
+            setattr(t, k, v.data_ptr() if hasattr(v, "data_ptr") else v)
+        return t
 
     def conv_block_set_always(self, on):
         """otter_hip_conv_block_set_always: returns the previous setting."""

@@ -1767,6 +1767,74 @@ int otter_hip_conv_forward_residual_concat(const otter_hip_conv_t* h, const void
     return join_run(h, in, out, g, ep, alt, config, (hipStream_t)stream_);
 }
 
+// ---- two pointwise layers, the second reading the int8 form of the first's result --------------------------------------------
+
+struct PairArgs {
+    ConvGeom g[2];
+    Epilogue ep[2];
+    JoinArgs ja;
+};
+
+// the two layers and what becomes of the first's result as one launch has them; an error code for what no call may ask for
+static int pair_args(const char* who, const otter_hip_conv_t* first, const otter_hip_conv_t* second, int n, int in_h, int in_w,
+                     const otter_hip_conv_tail* t, int out_layout, PairArgs* a) {
+    auto bad = [&](const char* what) { return fail(OTTER_HIP_ERR_INVALID, std::string(who) + ": " + what); };
+    if (!first || !second || !t) return bad("null");
+    if (n < 0 || in_h < 1 || in_w < 1) return bad("bad shape");
+    const int K = first->d.out_channels;
+    const bool f32 = first->d.out_kind == OTTER_HIP_OUT_F32;
+    if (second->d.in_channels != K || K % 8) return bad("the second layer reads whole channel octets of the first's result");
+    if (first->d.out_kind == OTTER_HIP_OUT_I32 || second->d.out_kind == OTTER_HIP_OUT_I32) return bad("int8 or fp32 results expected");
+    const int want = second->d.out_kind == OTTER_HIP_OUT_F32 ? 0 : 1;
+    if (!valid_layout(out_layout) || layout_elem(out_layout) != want || second->d.out_channels % layout_pack(out_layout))
+        return bad("output layout does not match the second layer");
+    if (f32 != (t->other != nullptr)) return bad("a shuffle takes an fp32 result of the first layer, and it only takes one with a shuffle");
+    if (f32 && t->q_round_mode != OTTER_HIP_ROUND_SSE && t->q_round_mode != OTTER_HIP_ROUND_EXACT) return bad("unknown rounding mode");
+    if (t->other && t->other_layout != OTTER_HIP_F32_P4 && t->other_layout != OTTER_HIP_F32_P8) return bad("the other blob must be Float4 or Float8");
+    a->g[0] = make_geom(first->d, n, in_h, in_w);
+    if (a->g[0].OH < 1 || a->g[0].OW < 1) return bad("empty output");
+    a->g[1] = make_geom(second->d, n, a->g[0].OH, a->g[0].OW);
+    if (a->g[1].OH < 1 || a->g[1].OW < 1) return bad("empty output");
+    a->ep[0] = make_epilogue(first, f32 ? OTTER_HIP_F32_P4 : OTTER_HIP_I8_P8), a->ep[1] = make_epilogue(second, out_layout);
+    Epilogue& ep = a->ep[0];
+    ep.twin_scale = t->q_scale, ep.twin_half = t->q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+    if (t->other) {
+        a->ja.other = t->other, a->ja.other_pack = layout_pack(t->other_layout), a->ja.other_odd = t->other_odd != 0;
+        a->ja.sh_image = (size_t)K * a->g[0].OH * a->g[0].OW, a->ja.sh_out0 = t->first_half;
+        ep.join = &a->ja;
+    }
+    return OTTER_HIP_OK;
+}
+
+static bool pair_one_launch(const otter_hip_conv_t* first, const otter_hip_conv_t* second, const PairArgs& a) {
+    for (const otter_hip_conv_t* h : {first, second})
+        if (!h->w_igemm || h->c_pad || !h->so_same || (h->force_tm != 0 && h->force_tm != -11)) return false;
+    return conv_pwpw_applicable(a.g[0], a.ep[0], a.g[1], a.ep[1]) && (first->force_tm == -11 || conv_pwpw_faster(a.g[0], a.g[1]));
+}
+
+int otter_hip_conv_pair_launches(const otter_hip_conv_t* first, const otter_hip_conv_t* second, int n, int in_h, int in_w,
+                                 const otter_hip_conv_tail* tail, int out_layout) {
+    PairArgs a;
+    const int rc = pair_args("otter_hip_conv_pair_launches", first, second, n, in_h, in_w, tail, out_layout, &a);
+    return rc ? rc : pair_one_launch(first, second, a) ? 1 : 2;
+}
+
+int otter_hip_conv_pair_forward(const otter_hip_conv_t* first, const otter_hip_conv_t* second, const void* in, int n, int in_h, int in_w,
+                                const otter_hip_conv_tail* tail, void* out, int out_layout, void* stream) {
+    PairArgs a;
+    const int rc = pair_args("otter_hip_conv_pair_forward", first, second, n, in_h, in_w, tail, out_layout, &a);
+    if (rc) return rc;
+    if (!in || !out || (tail->other && !tail->first_half)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_pair_forward: null");
+    if (!pair_one_launch(first, second, a))
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_pair_forward: not a single launch (otter_hip_conv_pair_launches)");
+    if (n == 0) return OTTER_HIP_OK;
+    const int8_t* const w[2] = {first->w_igemm, second->w_igemm};
+    const float so[2] = {first->so_one, second->so_one};
+    OHIP_CHECK(run_conv_pwpw((const int8_t*)in, w, so, out, a.g[0], a.ep[0], a.g[1], a.ep[1],
+                             first->force_tm == -11 ? first->force_tn : 0, (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
 static bool conv_avgpool_one_launch(const otter_hip_conv_t* h, int in_layout, const ConvGeom& g) {
     if (in_layout != OTTER_HIP_I8_P8 || !h->w_igemm || h->c_pad || h->force_tm || h->d.out_kind != OTTER_HIP_OUT_F32) return false;
     return conv_pw_avgpool_applicable(g, make_epilogue(h, otter_hip_conv_default_out_layout(h)));

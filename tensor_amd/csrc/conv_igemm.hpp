@@ -53,6 +53,12 @@ void conv_pw_reg_plan_clamped(const ConvGeom& g, int* groups, int* per);
 hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* out, const ConvGeom& g, const Epilogue& ep, int force,
                            hipStream_t stream);
 
+// conv_pwpw.hip: two pointwise layers, the second reading the int8 form of the first's result, one launch
+bool conv_pwpw_applicable(const ConvGeom& g0, const Epilogue& e0, const ConvGeom& g1, const Epilogue& e1);
+bool conv_pwpw_faster(const ConvGeom& g0, const ConvGeom& g1);
+hipError_t run_conv_pwpw(const int8_t* x, const int8_t* const w[2], const float so[2], void* out, const ConvGeom& g0,
+                         const Epilogue& e0, const ConvGeom& g1, const Epilogue& e1, int force, hipStream_t stream);
+
 // conv_block.hip: 1x1 expand -> depthwise 3x3 -> 1x1 project (+ shortcut sum, + int8 twin) as one launch
 bool conv_block_applicable(const ConvGeom& ge, const Epilogue& e1, const ConvGeom& gd, const Epilogue& e2, const ConvGeom& gp,
                            const Epilogue& e3);

@@ -15,8 +15,8 @@
 // Epilogues: int8 Byte8 and fp32 Float4 results, the latter with the addend, the int8 twin and the shuffle of the implicit-GEMM
 // kernel (common.hpp).
 #include "common.hpp"
-#include "conv_dw_common.hpp"
 #include "conv_igemm.hpp"
+#include "conv_pw_common.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -24,8 +24,6 @@
 namespace ohip {
 
 namespace {
-
-constexpr unsigned PR_OOB = 0x80000000u;  // past any buffer here: a load returns zero, a store is dropped
 
 // What these kernels read of a layer. Launch arguments are written to device memory one by one: on the host a launch with 32 bytes
 // of them takes 3.1 us, with 96 3.35, with 180 (ConvGeom and Epilogue as they are) 3.85, and such a layer's kernel is done in less.
@@ -41,57 +39,6 @@ struct PwRegArgs {
 
     __device__ FastDiv hw() const { return {hw_m, hw_s, (unsigned)HW}; }
 };
-// the rest of an epilogue that needs more
-struct PwFused {
-    const float* residual;
-    int8_t* twin;
-    float twin_scale, twin_half;
-    static PwFused of(const Epilogue& ep) { return {ep.residual, ep.twin, ep.twin_scale, ep.twin_half}; }
-};
-struct PwParts : PwFused {  // JoinArgs::residual1 and the like
-    const float* residual1;
-    int split;
-    short pack0, pack1;
-    static PwParts of(const Epilogue& ep) {
-        return {PwFused::of(ep), ep.join->residual1, ep.join->res_split, (short)ep.join->res_pack0, (short)ep.join->res_pack1};
-    }
-    __device__ JoinArgs join() const {
-        JoinArgs ja{};
-        ja.residual1 = residual1, ja.res_split = split, ja.res_pack0 = pack0, ja.res_pack1 = pack1;
-        return ja;
-    }
-};
-struct PwShuffle {  // JoinArgs::other and the like
-    const float* other;
-    float *sh_out0, *sh_out1;
-    int8_t *sh_q0, *sh_q1;
-    float twin_scale, twin_half;
-    unsigned sh_image;
-    short other_pack, other_odd;
-    static PwShuffle of(const Epilogue& ep) {
-        const JoinArgs& j = *ep.join;
-        return {j.other, j.sh_out0, j.sh_out1, j.sh_q0, j.sh_q1, ep.twin_scale, ep.twin_half, (unsigned)j.sh_image, (short)j.other_pack, (short)j.other_odd};
-    }
-};
-template <int EPI>
-struct PwAddOf {
-    using Type = NoJoin;
-};
-template <>
-struct PwAddOf<EPI_F32_P4_FUSED> {
-    using Type = PwFused;
-};
-template <>
-struct PwAddOf<EPI_F32_SHUFFLE> {
-    using Type = PwShuffle;
-};
-template <>
-struct PwAddOf<EPI_F32_P4_PARTS> {
-    using Type = PwParts;
-};
-template <int EPI>
-using PwAdd = typename PwAddOf<EPI>::Type;
-
 template <int EPI>
 __device__ __forceinline__ Epilogue pw_epilogue(const PwRegArgs& pa, const PwAdd<EPI>& ja) {
     constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG;
@@ -102,20 +49,6 @@ __device__ __forceinline__ Epilogue pw_epilogue(const PwRegArgs& pa, const PwAdd
     if constexpr (!I8 && EPI != EPI_F32_P4) ep.twin_scale = ja.twin_scale, ep.twin_half = ja.twin_half;
     if constexpr (EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_P4_PARTS) ep.residual = ja.residual, ep.twin = ja.twin;
     return ep;
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, unsigned bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ v4i load16(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
-    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, (int)v, (int)s, 0));
-}
-__device__ __forceinline__ v2i load8(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s) {
-    return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, (int)s, 0));
-}
-__device__ __forceinline__ void store16(__amdgpu_buffer_rsrc_t r, v4i d, unsigned v, unsigned s) { store_b128_row(d, r, v, s); }
-__device__ __forceinline__ void store8(__amdgpu_buffer_rsrc_t r, v2i d, unsigned v, unsigned s) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, d), r, (int)v, (int)s, 0);
 }
 
 }  // namespace

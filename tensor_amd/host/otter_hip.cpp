@@ -942,6 +942,45 @@ int ConvolutionLayer::forward_shuffle(const Tensor& bottom_in, const Tensor& oth
     return 0;
 }
 
+int ConvolutionLayer::forward_pair(const ConvolutionLayer* a, const ConvolutionLayer* b, const Tensor& bottom_in, const Tensor* other,
+                                   bool other_odd, Tensor& first_half, Tensor& top, const NetOption& opt) {
+    if (!a->handle_ || !b->handle_ || a->force_out_layout >= 0 || b->force_out_layout >= 0 || !opt.use_packing_layout) return 1;
+    if ((a->int8_scale_term > 100) != (other == nullptr) || !a->int8_scale_term || !b->int8_scale_term) return 1;
+    Tensor bottom = bottom_in, twin;
+    if (!bottom.defined() || bottom.dim() != 4) return 1;
+    if (base_of(bottom.scalar_type()) == ScalarType::Float && a->in_channels % 8 == 0 &&
+        bottom.quantized_twin(a->bottom_blob_int8_scales.data_ptr<float>()[0], a->input_round_mode(opt), twin))
+        bottom = twin;
+    if (bottom.scalar_type() != ScalarType::Byte8 || bottom.channels() != a->in_channels) return 1;
+    const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3);
+    otter_hip_conv_tail tail{};
+    if (other) {
+        if (!other->defined() || other->dim() != 4 || base_of(other->scalar_type()) != ScalarType::Float || other->elempack() == 1 ||
+            other->channels() != a->out_channels || other->size(0) != N || other->size(2) != H || other->size(3) != W)
+            return 1;
+        tail.other = (const float*)other->device_ptr(), tail.other_layout = hip_layout_of(other->scalar_type()), tail.other_odd = other_odd;
+        tail.q_scale = b->bottom_blob_int8_scales.data_ptr<float>()[0], tail.q_round_mode = b->input_round_mode(opt);
+        tail.first_half = (float*)tail.other;  // (the question is only whether there is one)
+    }
+    const int layout = otter_hip_conv_default_out_layout(b->handle_);
+    if ((layout != OTTER_HIP_I8_P8 && layout != OTTER_HIP_F32_P4) || otter_hip_conv_pair_launches(a->handle_, b->handle_, N, H, W, &tail, layout) != 1) return 1;
+    try {
+        if (other) {
+            first_half = Tensor::empty_device({N, a->out_channels / 8, H, W}, ScalarType::Float8);
+            tail.first_half = (float*)first_half.device_ptr();
+        }
+        top = Tensor::empty_device({N, b->out_channels / (layout == OTTER_HIP_I8_P8 ? 8 : 4), H, W}, scalar_type_of_layout(layout));
+        const int rc = otter_hip_conv_pair_forward(a->handle_, b->handle_, bottom.device_ptr(), N, H, W, &tail, top.device_ptr(), layout,
+                                                   launch_stream());
+        if (rc) return rc;
+        if (other) first_half.mark_device_written();
+        top.mark_device_written();
+    } catch (const Error&) {
+        return -100;
+    }
+    return 0;
+}
+
 int ConvolutionLayer::block_launches(const ConvolutionLayer* e, const ConvolutionLayer* d, const ConvolutionLayer* p, int n, int h,
                                      int w) {
     return e->handle_ && d->handle_ && p->handle_ ? otter_hip_conv_block_fastest(e->handle_, d->handle_, p->handle_, n, h, w) : 3;
@@ -1995,10 +2034,19 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
             }
         }
     }
+    {
+        const auto unit = pair_units_.find(li);
+        // only when the blob between the two has not been computed (or set by the caller)
+        if (unit != pair_units_.end() && !blobs[layer->bottoms[0]].defined()) {
+            const int rc = forward_pair_unit(unit->second, li, nullptr, blobs, opt);
+            if (rc <= 0) return rc;
+        }
+    }
     for (int b : layer->bottoms)
         if (!blobs[b].defined()) {
             int rc = forward_layer(blobs_[b].producer, blobs, opt);
             if (rc) return rc;
+            if (!blobs[b].defined() && layer->tops.size() == 1 && blobs[layer->tops[0]].defined()) return 0;  // (forward_pair_unit)
         }
     if (layer->type() == "Input") return blobs[layer->tops[0]].defined() ? 0 : -1;
     if (layer->one_blob_only) {
@@ -2100,9 +2148,23 @@ void Net::plan_fused_quantize() const {
         if (blobs_[b].consumers.size() != 1) continue;
         pool_units_[(int)pi] = ci;
     }
+    // Pairs of pointwise layers, one reading the other's int8 result alone
+    auto sole_reader = [&](int blob) { return blobs_[blob].consumers.size() == 1 ? blobs_[blob].consumers[0] : -1; };
+    auto pair_layer = [&](int li) {
+        const auto* c = dynamic_cast<const ConvolutionLayer*>(layers_[li]);
+        return c && c->int8_scale_term && c->groups == 1 && c->kernel_height == 1 && c->kernel_width == 1 && c->stride_height == 1 &&
+               c->stride_width == 1 && c->padding_height == 0 && c->padding_width == 0 && c->bottoms.size() == 1 && c->tops.size() == 1 &&
+               c->force_out_layout < 0 && c->in_channels % 8 == 0;
+    };
+    auto int8_result = [&](int li) { return static_cast<const ConvolutionLayer*>(layers_[li])->int8_scale_term > 100; };
+    auto pair_reader = [&](int li) { return pair_layer(li) && (int8_result(li) || layers_[li]->fuse_scale == 0.f); };
+    pair_units_.clear();
+    for (size_t li = 0; li < layers_.size(); ++li) {
+        const int pi = pair_reader((int)li) ? blobs_[layers_[li]->bottoms[0]].producer : -1;
+        if (pi >= 0 && pair_layer(pi) && int8_result(pi) && sole_reader(layers_[pi]->tops[0]) == (int)li && !pair_units_.count(pi)) pair_units_[(int)li] = pi;
+    }
     // ShuffleNetV2 unit tails: Concat of two equal blobs -> ChannelShuffle(2) -> exactly the two half Crops
     shuffle_units_.clear();
-    auto sole_reader = [&](int blob) { return blobs_[blob].consumers.size() == 1 ? blobs_[blob].consumers[0] : -1; };
     for (size_t ci = 0; ci < layers_.size(); ++ci) {
         const Layer* cat = layers_[ci];
         if (cat->type() != "Concat" || cat->bottoms.size() != 2 || cat->bottom_shapes[0] != cat->bottom_shapes[1]) continue;
@@ -2119,7 +2181,7 @@ void Net::plan_fused_quantize() const {
             if (!pc || !pc->int8_scale_term || pc->int8_scale_term > 100 || pc->force_out_layout >= 0 || pc->bottoms.size() != 1) continue;
             if (blobs_[b].consumers.size() == 1 && pi > conv) conv = pi, conv_k = k;
         }
-        const ShuffleUnit whole{(int)ci, si, -1, -1, sh->fuse_scale, sh->fuse_round, sh->fuse_only, conv, conv_k};
+        const ShuffleUnit whole{(int)ci, si, -1, -1, sh->fuse_scale, sh->fuse_round, sh->fuse_only, conv, conv_k, -1};
         if (conv >= 0) shuffle_units_[si] = whole;
         int sp = sole_reader(sh->tops[0]);
         if (sp < 0 || layers_[sp]->type() != "Split" || layers_[sp]->tops.size() != 2) continue;
@@ -2147,7 +2209,9 @@ void Net::plan_fused_quantize() const {
             if (hs != 0.f && (sc != hs || r != hr)) agree = false;
             hs = sc, hr = r;
         }
-        const ShuffleUnit u{(int)ci, si, lo, hi, agree && hs > 0.f ? hs : 0.f, hr, agree && hs > 0.f, conv, conv_k};
+        const int reader = sole_reader(layers_[hi]->tops[0]);
+        const ShuffleUnit u{(int)ci, si, lo, hi, agree && hs > 0.f ? hs : 0.f, hr, agree && hs > 0.f, conv, conv_k,
+                            conv >= 0 && reader >= 0 && pair_reader(reader) && pair_layer(conv) ? reader : -1};
         shuffle_units_[lo] = u;
         shuffle_units_[hi] = u;
     }
@@ -2301,24 +2365,27 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
     return 0;
 }
 
+// 1 where the layer is the last of an inverted-residual block that has not been begun and that runs in fewer launches than its layers
+int Net::block_saves_launches(int conv, std::vector<Tensor>& blobs, const NetOption& opt) const {
+    const auto bu = block_units_.find(conv);
+    if (bu == block_units_.end() || blobs[layers_[bu->second.expand]->tops[0]].defined() || blobs[layers_[conv]->bottoms[0]].defined()) return 0;
+    const auto* ec = static_cast<const ConvolutionLayer*>(layers_[bu->second.expand]);
+    const int b = ec->bottoms[0];
+    if (!blobs[b].defined()) {
+        const int rc = forward_layer(blobs_[b].producer, blobs, opt);
+        if (rc) return rc;
+    }
+    return blobs[b].dim() == 4 && ConvolutionLayer::block_launches(ec, static_cast<const ConvolutionLayer*>(layers_[bu->second.depthwise]),
+                                                                   static_cast<const ConvolutionLayer*>(layers_[conv]), (int)blobs[b].size(0),
+                                                                   (int)blobs[b].size(2), (int)blobs[b].size(3)) < 3;
+}
+
 // The unit in the launch of the convolution in front of it. Returns 1 when the blobs at hand do not allow it.
 int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const {
     const auto* conv = static_cast<const ConvolutionLayer*>(layers_[u.conv]);
     const int other = layers_[u.concat]->bottoms[1 - u.conv_k], in_blob = conv->bottoms[0];
-    const auto bu = block_units_.find(u.conv);
-    if (bu != block_units_.end() && !blobs[layers_[bu->second.expand]->tops[0]].defined() && !blobs[in_blob].defined()) {
-        // the layer may be the last of an inverted-residual block: the block's shared launch saves more
-        const auto* ec = static_cast<const ConvolutionLayer*>(layers_[bu->second.expand]);
-        const int b = ec->bottoms[0];
-        if (!blobs[b].defined()) {
-            const int rc = forward_layer(blobs_[b].producer, blobs, opt);
-            if (rc) return rc;
-        }
-        if (blobs[b].dim() == 4 &&
-            ConvolutionLayer::block_launches(ec, static_cast<const ConvolutionLayer*>(layers_[bu->second.depthwise]), conv,
-                                             (int)blobs[b].size(0), (int)blobs[b].size(2), (int)blobs[b].size(3)) < 3)
-            return 1;
-    }
+    const int block = block_saves_launches(u.conv, blobs, opt);
+    if (block) return block;
     for (int b : {other, in_blob})
         if (!blobs[b].defined()) {
             const int rc = forward_layer(blobs_[b].producer, blobs, opt);
@@ -2328,6 +2395,10 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
     Tensor first, second;
     const int last = joined ? layers_[u.shuffle]->tops[0] : layers_[u.crop_hi]->tops[0];
     const bool int8_only = u.hi_only && opt.wanted && !(*opt.wanted)[last];
+    if (!joined && int8_only && u.next >= 0) {
+        const int rc = forward_pair_unit(u.conv, u.next, &u, blobs, opt);
+        if (rc <= 0) return rc;
+    }
     const int rc = conv->forward_shuffle(blobs[in_blob], blobs[other], u.conv_k == 0, joined, u.hi_scale, u.hi_round, first, second, opt,
                                          int8_only);
     if (rc) return rc;
@@ -2340,6 +2411,39 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
     if (opt.lightmode)
         for (int b : {other, in_blob})
             if (blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+    return 0;
+}
+
+// Two pointwise layers in one launch (ConvolutionLayer::forward_pair), with `u` across the end of that ShuffleNetV2 unit, whose inputs
+// are there. Returns 1 when the layers or the blobs at hand do not allow it, or when the second is the first of an inverted-residual
+// block that runs in fewer launches than its layers.
+int Net::forward_pair_unit(int first, int second, const ShuffleUnit* u, std::vector<Tensor>& blobs, const NetOption& opt) const {
+    const auto *a = static_cast<const ConvolutionLayer*>(layers_[first]), *b = static_cast<const ConvolutionLayer*>(layers_[second]);
+    const int in_blob = a->bottoms[0], top_blob = b->tops[0];
+    if (blobs[top_blob].defined() || (opt.wanted && (*opt.wanted)[a->tops[0]])) return 1;
+    const int block = block_saves_launches(first, blobs, opt);
+    if (block) return block;
+    if (!blobs[in_blob].defined()) {
+        const int rc = forward_layer(blobs_[in_blob].producer, blobs, opt);
+        if (rc) return rc;
+    }
+    const Tensor& x = blobs[in_blob];
+    if (x.dim() != 4) return 1;
+    for (const auto& bu : block_units_)
+        if (bu.second.expand == second &&
+            ConvolutionLayer::block_launches(b, static_cast<const ConvolutionLayer*>(layers_[bu.second.depthwise]),
+                                             static_cast<const ConvolutionLayer*>(layers_[bu.second.project]), (int)x.size(0), (int)x.size(2),
+                                             (int)x.size(3)) < 3)
+            return 1;
+    const int other = u ? layers_[u->concat]->bottoms[1 - u->conv_k] : -1;
+    Tensor lo, top;
+    const int rc = ConvolutionLayer::forward_pair(a, b, x, u ? &blobs[other] : nullptr, u && u->conv_k == 0, lo, top, opt);
+    if (rc) return rc;
+    blobs[top_blob] = top;
+    if (u) blobs[layers_[u->crop_lo]->tops[0]] = lo;
+    if (opt.lightmode)
+        for (int k : {in_blob, other})
+            if (k >= 0 && blobs_[k].consumers.size() == 1) blobs[k] = Tensor();
     return 0;
 }
 

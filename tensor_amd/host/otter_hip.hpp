@@ -254,6 +254,11 @@ public:
     // > 0 also quantizes the second half (joined: the blob). Returns 1, and does nothing, when that is not one launch here.
     int forward_shuffle(const Tensor& bottom_blob, const Tensor& other, bool other_odd, bool joined, float q_scale, int q_round,
                         Tensor& first, Tensor& second, const NetOption& opt, bool int8_only) const;
+    // Two pointwise layers, the second (no int8 form of an fp32 result wanted) the only reader of the first's int8 result (`other` null) or of the second half of
+    // what a ChannelShuffle(2) makes of its fp32 result and `other`, in one launch (otter_hip_conv_pair_forward): `first_half` is the
+    // other half, `top` the second layer's result. Returns 1, and does nothing, when that is not one launch here.
+    static int forward_pair(const ConvolutionLayer* first, const ConvolutionLayer* second, const Tensor& bottom_blob, const Tensor* other,
+                            bool other_odd, Tensor& first_half, Tensor& top, const NetOption& opt);
     // forward_residual where the shortcut is the concatenation of two blobs (otter_hip_conv_forward_residual_concat)
     int forward_residual_concat(const Tensor& bottom_blob, const Tensor& part0, const Tensor& part1, float q_scale, int q_round,
                                 Tensor& sum, const NetOption& opt, bool int8_only) const;
@@ -377,8 +382,13 @@ private:
         bool hi_only;    // ... and by nothing else
         int conv;        // the int8 convolution whose fp32 result is bottom conv_k of the Concat and read by nothing else, or -1
         int conv_k;
+        int next;        // the pointwise layer that alone reads the second half, or -1
     };
     mutable std::map<int, ShuffleUnit> shuffle_units_;
+    // pointwise layers that alone read another one's int8 result: the reader's index -> the other's
+    mutable std::map<int, int> pair_units_;
+    int forward_pair_unit(int first, int second, const ShuffleUnit* u, std::vector<Tensor>& blobs, const NetOption& opt) const;
+    int block_saves_launches(int conv, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_shuffle_unit(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const;
     // The tail of a residual block, found by the plan: an Eltwise sum of two blobs, one of them the fp32 result of an
