@@ -4,8 +4,8 @@
 //
 // What bounds the implicit-GEMM kernel on these layers is vector issue: addresses, bounds checks and 8-byte loads are paid per
 // tap (256 -> 256 3x3 in 8 groups @28x28 b64: 10.1 M vector instructions, 0.36 M of them memory reads, beside 0.25 M matrix
-// ones; issuing them takes 80 % of the 22.6 us). Here a tile pays them once per staged row and a step reads LDS: 3.8 M vector
-// instructions, 0.12 M memory reads, 48 % of the time in vector issue, 16 % in the LDS pipe, 13 % in the matrix cores.
+// ones; issuing them takes 80 % of the 22.6 us). Here a tile pays them once per staged row and a step reads LDS: 3.3 M vector
+// instructions, 0.09 M memory reads, 51 % of the time in vector issue, 22 % in the LDS pipe, 16 % in the matrix cores.
 //
 // A workgroup of four waves owns PT = 64 FN consecutive output pixels and FM 16-row tiles of output channels (all of them, one
 // block after the other, where the input channels fit one stage). Wide images are cut into column strips first, and a strip
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF 
     // lanes that finish eight channels each load them, every request brings 16 bytes to each lane, and the wave waits for them at the
     // end of its chain.)
     constexpr int CN = 16 * FM;
-    const int block0 = blockIdx.y * ra.blocks_per_wg, nc = ra.blocks_per_wg * CN;  // at most 256
+    const int block0 = blockIdx.y * ra.blocks_per_wg, nc = ra.blocks_per_wg * CN;  // at most 512
     float* const consts = reinterpret_cast<float*>(lds + ra.consts);
     float c_si = 0.f, c_bi = 0.f, c_so = 0.f;
     if (EPI != EPI_GENERIC && tid < nc && block0 * CN + tid < g.K) {
@@ -198,12 +198,23 @@ __global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF 
                          in && last > first ? first | last << 16 : 0};
     }
 
-    if (EPI != EPI_GENERIC && tid < nc) {
-        consts[tid] = c_si, consts[nc + tid] = c_bi;
-        if constexpr (EPI != EPI_F32_P4) consts[2 * nc + tid] = c_so;
+    auto put = [&](int c, float si, float bi, float so) {
+        consts[c] = si, consts[nc + c] = bi;
+        if constexpr (EPI != EPI_F32_P4) consts[2 * nc + c] = so;
         if constexpr (EPI == EPI_I8_P8_NONNEG)
-            reinterpret_cast<unsigned short*>(consts + 3 * nc)[tid] =
-                (unsigned short)min((int)__fadd_rn(__fmul_rn(ep.act_hi, c_so), ep.round_half), 127);
+            reinterpret_cast<unsigned short*>(consts + 3 * nc)[c] = (unsigned short)min((int)__fadd_rn(__fmul_rn(ep.act_hi, so), ep.round_half), 127);
+    };
+    if (EPI != EPI_GENERIC && tid < nc) {
+        put(tid, c_si, c_bi, c_so);
+        // (a workgroup of more channels than threads walks many row blocks: what it waits for here is little of its time)
+        if (const int c = tid + 256; c < nc) {
+            const bool ok = block0 * CN + c < g.K;
+            const int ch = grp * g.K + (ok ? block0 * CN + c : 0);
+            const float si = ep.scale_in[ch], bi = ep.bias[ch];
+            float so = 0.f;
+            if constexpr (EPI != EPI_F32_P4) so = ep.scale_out[ch];
+            put(c, ok ? si : 0.f, ok ? bi : 0.f, ok ? so : 0.f);
+        }
     }
 
 #pragma unroll
@@ -492,14 +503,16 @@ bool conv_rows_supported(const ConvGeom& g, const Epilogue& ep, bool f32in) {
     return (size_t)g.N * g.C * g.H * g.W * (f32in ? 4 : 1) < ((size_t)1 << 31) && (size_t)g.N * g.K * g.OH * g.OW < ((size_t)1 << 31);
 }
 
-// one stage: a workgroup walks row blocks over its staged pixels, as many as leave two workgroups per compute unit, and at most 256
-// channels (a thread brings the constants of one)
+// one stage: a workgroup walks row blocks over its staged pixels, as many as leave two workgroups per compute unit, and at most 512
+// channels (a thread brings the constants of two), dealt evenly: every further workgroup stages the rows again. With at most 256 channels,
+// the first workgroups filled: 64 -> 272 3x3 @216x216 b4 in four and one blocks 51.2 us, in one workgroup 47.4; 24 -> 344 @185x224 b7 48.3
+// (62.4 with the constants from memory, on the tile chosen then).
 static int rows_blocks_per_workgroup(const RowsArgs& ra, int blocks, int fm) {
     if (ra.stages > 1) return 1;
     const long tiles = (long)ra.n_tiles * ra.g.groups;
-    const int want = (int)((512 + tiles - 1) / tiles), slices = want > blocks ? blocks : want;
-    const int each = (blocks + slices - 1) / slices;
-    return each < 16 / fm ? each : 16 / fm;
+    const int want = (int)((512 + tiles - 1) / tiles), least = (blocks * fm + 31) / 32;
+    const int slices = want > blocks ? blocks : want > least ? want : least;
+    return (blocks + slices - 1) / slices;
 }
 
 // LDS of a workgroup: what the plan takes, and the epilogue constants behind it
@@ -552,14 +565,15 @@ float conv_rows_cost(const ConvGeom& g_in, bool f32in, int out_bytes, int* confi
         const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm), bpw = rows_blocks_per_workgroup(ra, blocks, c.fm);
         const int pairs = ra.rows_max * ra.VW2, oct = (ra.g.C / 8 + ra.stages - 1) / ra.stages;
         const float places = (float)(ra.stages * oct) * (pairs > 128 ? (float)((pairs + 255) / 256) : 1.f / (float)(256 / pairs));
-        const int wgs = (int)std::min(((long)ra.n_tiles * ((blocks + bpw - 1) / bpw) * ra.g.groups + 255) / 256, 1l << 24);
+        const int slices = (blocks + bpw - 1) / bpw;
+        const int wgs = (int)std::min(((long)ra.n_tiles * slices * ra.g.groups + 255) / 256, 1l << 24);
         const RowsCost& cost = f32in ? c.f32 : c.i8;
         const int side = std::min(cost.resident, (int)(160 * 1024 / rows_lds(lds, bpw, c.fm)));
         const float cu = (float)wgs, rounds = (float)((wgs + side - 1) / side);
         const RowsCoef& k = cost.at;
-        const float s = (float)(bpw * steps) * (g_in.sw > 1 ? 1.f + k.strided : 1.f);
-        float t = k.start + rounds * (k.step * s + k.stage * (float)ra.stages) +
-                        cu * (k.cu_step * s + k.cu_place * places + k.cu_block * (float)bpw) + k.in_mb * in_mb + k.out_mb * out_mb;
+        const float s = (float)steps * (g_in.sw > 1 ? 1.f + k.strided : 1.f), walked = (float)blocks / (float)slices;  // (of one workgroup, on average)
+        float t = k.start + rounds * (k.step * s * (float)bpw + k.stage * (float)ra.stages) +
+                        cu * (walked * (k.cu_step * s + k.cu_block) + k.cu_place * places) + k.in_mb * in_mb + k.out_mb * out_mb;
         t *= 1.f + 0.01f * (float)c.fm * more_mb;
         if (t < best) best = t, *config = i;
     }

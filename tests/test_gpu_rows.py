@@ -1,6 +1,6 @@
 """Every tile of the k x k launch on staged rows (set_tile(-9, tile)) against the implicit-GEMM kernel (set_tile(-4, 0)), bit for bit: rows
 shorter and longer than the 16 pixels from which a lane walks on instead of dividing, images that a tile runs over, column strips, output
-channels beyond the 256 whose constants a workgroup holds, and reductions of more than one stage whose weights are asked for ahead."""
+channels beyond the threads of a workgroup and those whose constants it holds, and reductions of more than one stage whose weights are asked for ahead."""
 import numpy as np
 import pytest
 
