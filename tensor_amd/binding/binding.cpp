@@ -198,9 +198,9 @@ PyObject* conv_chain(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
 // otter_hip_conv_block_fastest are of the launches alone; of the host's time one launch takes 6.5 us a call, two 8.5 and three 11.
 // Their choice is taken where it is no more launches (128 -> 768 -> 128 on one 13x13 image 11.4 us a call in three, 8.3 in two;
 // 160 -> 960 -> 208 on 25 8x8 images 15.9 and 11.7). For more of them the two blobs between the layers have to be beyond 4 MB (two
-// launches) and 8 MB, which keep the GPU busy for longer than that: 48 -> 288 -> 32 on 16 27x27 images 12.6 us in one, 11.7 in two; but 24 ->
-// 144 -> 40 on 49 10x9 images 8.9 in one, 11 in three. A workspace that is given has to hold them. (workspace: its bytes, < 0:
-// none; *bytes: what the form needs)
+// launches) and 12 MB (three), which keep the GPU busy for longer than that: 112 -> 672 -> 112 on 33 22x22 images 30.3 us in one, 24.7 in
+// three; but 64 -> 384 -> 64 on 58 14x14 images, with 8.7 MB, 11.4 in one and 14.2 in three, and 24 -> 144 -> 40 on 49 10x9 images 8.9
+// and 11. A workspace that is given has to hold them. (workspace: its bytes, < 0: none; *bytes: what the form needs)
 int block_form(const otter_hip_conv_t* e, const otter_hip_conv_t* d, const otter_hip_conv_t* p, int n, int h, int w, int64_t workspace,
                size_t* bytes) {
     const int as_is = otter_hip_conv_block_launches(e, d, p, n, h, w);
