@@ -1998,12 +1998,9 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
         if (unit != pool_units_.end() && !blobs[layers_[unit->second]->tops[0]].defined()) {
             const auto* conv = static_cast<const ConvolutionLayer*>(layers_[unit->second]);
             const int b = conv->bottoms[0];
-            if (!blobs[b].defined()) {
-                const int rc = forward_layer(blobs_[b].producer, blobs, opt);
-                if (rc) return rc;
-            }
             Tensor mean;
-            const int rc = conv->forward_avgpool(blobs[b], mean, opt);
+            int rc = forward_inputs(unit->second, {b}, blobs, opt);
+            if (rc == 0) rc = conv->forward_avgpool(blobs[b], mean, opt);
             if (rc < 0) return rc;
             if (rc == 0) {
                 blobs[layer->tops[0]] = mean;
@@ -2042,12 +2039,10 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
             if (rc <= 0) return rc;
         }
     }
-    for (int b : layer->bottoms)
-        if (!blobs[b].defined()) {
-            int rc = forward_layer(blobs_[b].producer, blobs, opt);
-            if (rc) return rc;
-            if (!blobs[b].defined() && layer->tops.size() == 1 && blobs[layer->tops[0]].defined()) return 0;  // (forward_pair_unit)
-        }
+    {
+        const int rc = forward_inputs(li, layer->bottoms, blobs, opt);
+        if (rc) return rc < 0 ? rc : 0;
+    }
     if (layer->type() == "Input") return blobs[layer->tops[0]].defined() ? 0 : -1;
     if (layer->one_blob_only) {
         Tensor bottom = blobs[layer->bottoms[0]];
@@ -2072,6 +2067,19 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
     if (opt.lightmode)  // Tensor/Net.cpp:449-451: the inputs are not needed any more
         for (int b : layer->bottoms)
             if (blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+    return 0;
+}
+
+// Makes those of the blobs `needed` that are not there, for a launch of layer li (or of several, li the first). Returns 1 when the
+// layer's own result came to be on the way, as the second layer of a pair does (forward_pair_unit): its input may then be missing for
+// good, and the caller goes on layer by layer.
+int Net::forward_inputs(int li, const std::vector<int>& needed, std::vector<Tensor>& blobs, const NetOption& opt) const {
+    for (int b : needed) {
+        if (b < 0 || blobs[b].defined()) continue;
+        const int rc = forward_layer(blobs_[b].producer, blobs, opt);
+        if (rc) return rc;
+        if (layers_[li]->tops.size() == 1 && blobs[layers_[li]->tops[0]].defined()) return 1;
+    }
     return 0;
 }
 
@@ -2215,6 +2223,14 @@ void Net::plan_fused_quantize() const {
         shuffle_units_[lo] = u;
         shuffle_units_[hi] = u;
     }
+    // (not where the layer that reads the second half runs in the launch of a sum, a pooling or the next unit's end)
+    std::vector<char> in_other_launch(layers_.size(), 0);
+    for (const auto& u : residual_units_) in_other_launch[u.second.conv] = 1;
+    for (const auto& u : pool_units_) in_other_launch[u.second] = 1;
+    for (const auto& u : shuffle_units_)
+        if (u.second.conv >= 0) in_other_launch[u.second.conv] = 1;
+    for (auto& u : shuffle_units_)
+        if (u.second.next >= 0 && in_other_launch[u.second.next]) u.second.next = -1;
     // Inverted-residual blocks: 1x1 (int8 result) -> depthwise (int8 result) -> 1x1, each blob with one reader
     block_units_.clear();
     for (size_t li = 0; li < layers_.size(); ++li) {
@@ -2294,11 +2310,8 @@ int Net::forward_block_unit(const BlockUnit& u, int out_layer, int shortcut, std
     const auto* dc = static_cast<const ConvolutionLayer*>(layers_[u.depthwise]);
     const auto* pc = static_cast<const ConvolutionLayer*>(layers_[u.project]);
     const int in_blob = ec->bottoms[0];
-    for (int b : {shortcut, in_blob})
-        if (b >= 0 && !blobs[b].defined()) {
-            const int rc = forward_layer(blobs_[b].producer, blobs, opt);
-            if (rc) return rc;
-        }
+    const int made = forward_inputs(u.expand, {shortcut, in_blob}, blobs, opt);
+    if (made) return made;
     // the block reads Byte8: the blob itself, or the int8 twin its producer made with the first layer's scale
     Tensor bottom = blobs[in_blob], twin;
     if (bottom.defined() && base_of(bottom.scalar_type()) == ScalarType::Float &&
@@ -2334,11 +2347,8 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
     if (u.concat >= 0 && !blobs[u.shortcut].defined()) {
         // the sum straight from the two blobs that the Concat would copy
         const int p0 = layers_[u.concat]->bottoms[0], p1 = layers_[u.concat]->bottoms[1];
-        for (int b : {p0, p1, conv->bottoms[0]})
-            if (!blobs[b].defined()) {
-                const int rc = forward_layer(blobs_[b].producer, blobs, opt);
-                if (rc) return rc;
-            }
+        const int made = forward_inputs(u.conv, {p0, p1, conv->bottoms[0]}, blobs, opt);
+        if (made) return made;
         const int rc = conv->forward_residual_concat(blobs[conv->bottoms[0]], blobs[p0], blobs[p1], e->fuse_scale, e->fuse_round, sum, opt,
                                                      e->int8_only(opt));
         if (rc < 0) return rc;
@@ -2350,11 +2360,8 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
             return 0;
         }
     }
-    for (int b : {u.shortcut, conv->bottoms[0]})
-        if (!blobs[b].defined()) {
-            const int rc = forward_layer(blobs_[b].producer, blobs, opt);
-            if (rc) return rc;
-        }
+    const int made = forward_inputs(u.conv, {u.shortcut, conv->bottoms[0]}, blobs, opt);
+    if (made) return made;
     const int rc = conv->forward_residual(blobs[conv->bottoms[0]], blobs[u.shortcut], e->fuse_scale, e->fuse_round, sum, opt,
                                           e->int8_only(opt));
     if (rc) return rc;
@@ -2370,11 +2377,8 @@ int Net::block_saves_launches(int conv, std::vector<Tensor>& blobs, const NetOpt
     const auto bu = block_units_.find(conv);
     if (bu == block_units_.end() || blobs[layers_[bu->second.expand]->tops[0]].defined() || blobs[layers_[conv]->bottoms[0]].defined()) return 0;
     const auto* ec = static_cast<const ConvolutionLayer*>(layers_[bu->second.expand]);
-    const int b = ec->bottoms[0];
-    if (!blobs[b].defined()) {
-        const int rc = forward_layer(blobs_[b].producer, blobs, opt);
-        if (rc) return rc;
-    }
+    const int b = ec->bottoms[0], made = forward_inputs(bu->second.expand, {b}, blobs, opt);
+    if (made) return made < 0 ? made : 0;  // (begun: its first layer ran in a pair)
     return blobs[b].dim() == 4 && ConvolutionLayer::block_launches(ec, static_cast<const ConvolutionLayer*>(layers_[bu->second.depthwise]),
                                                                    static_cast<const ConvolutionLayer*>(layers_[conv]), (int)blobs[b].size(0),
                                                                    (int)blobs[b].size(2), (int)blobs[b].size(3)) < 3;
@@ -2386,16 +2390,13 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
     const int other = layers_[u.concat]->bottoms[1 - u.conv_k], in_blob = conv->bottoms[0];
     const int block = block_saves_launches(u.conv, blobs, opt);
     if (block) return block;
-    for (int b : {other, in_blob})
-        if (!blobs[b].defined()) {
-            const int rc = forward_layer(blobs_[b].producer, blobs, opt);
-            if (rc) return rc;
-        }
+    const int made = forward_inputs(u.conv, {other, in_blob}, blobs, opt);
+    if (made) return made;
     const bool joined = u.crop_lo < 0;
     Tensor first, second;
     const int last = joined ? layers_[u.shuffle]->tops[0] : layers_[u.crop_hi]->tops[0];
     const bool int8_only = u.hi_only && opt.wanted && !(*opt.wanted)[last];
-    if (!joined && int8_only && u.next >= 0) {
+    if (!joined && int8_only && u.next >= 0 && opt.asked != last) {
         const int rc = forward_pair_unit(u.conv, u.next, &u, blobs, opt);
         if (rc <= 0) return rc;
     }
@@ -2423,10 +2424,8 @@ int Net::forward_pair_unit(int first, int second, const ShuffleUnit* u, std::vec
     if (blobs[top_blob].defined() || (opt.wanted && (*opt.wanted)[a->tops[0]])) return 1;
     const int block = block_saves_launches(first, blobs, opt);
     if (block) return block;
-    if (!blobs[in_blob].defined()) {
-        const int rc = forward_layer(blobs_[in_blob].producer, blobs, opt);
-        if (rc) return rc;
-    }
+    const int made = forward_inputs(first, {in_blob}, blobs, opt);
+    if (made) return made;
     const Tensor& x = blobs[in_blob];
     if (x.dim() != 4) return 1;
     for (const auto& bu : block_units_)
@@ -2523,6 +2522,7 @@ int Extractor::extract(const std::string& name, Tensor& feat, int type) {
     const int i = net_->find_blob_index_by_name(name);
     if (i < 0) return -1;
     int ret = 0;
+    option.asked = i;
     if (!blob_tensors_[i].defined()) ret = net_->forward_layer(net_->blobs_[i].producer, blob_tensors_, option);
     if (ret) return ret;
     feat = blob_tensors_[i];

@@ -120,6 +120,7 @@ public:
     // set by Extractor::only: by blob, whether it (or a Split of it) will be asked for. Null: any blob may be, so every fp32 blob
     // is made; else one that only int8 convolutions read may exist as their common int8 input alone.
     std::shared_ptr<const std::vector<char>> wanted;
+    int asked = -1;  // the blob that Extractor::extract was called for: made even where nothing in the net would read it
 };
 enum class CompileMode { Inference, Initial };
 
@@ -387,6 +388,7 @@ private:
     mutable std::map<int, ShuffleUnit> shuffle_units_;
     // pointwise layers that alone read another one's int8 result: the reader's index -> the other's
     mutable std::map<int, int> pair_units_;
+    int forward_inputs(int li, const std::vector<int>& needed, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_pair_unit(int first, int second, const ShuffleUnit* u, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int block_saves_launches(int conv, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const;

@@ -1,0 +1,179 @@
+"""CPU: the launches that a Net makes of several layers (pairs of pointwise layers, ShuffleNetV2 units, sums, blocks, pooled tails),
+over a stand-in for the C ABI whose blobs hold the expression that they were computed from (fake_capi.cpp): whatever the forms of the
+launches, in light mode or not, through a session or through eval, a pass gives the layers' own expression and runs every layer once."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+SCRIPT = r"""
+import ctypes as C, sys
+import numpy as np
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # (in front of the library that the host layer names)
+fake.fake_number.restype = fake.fake_count.restype = C.c_long
+fake.fake_expr.restype = C.c_char_p
+from tensor_amd import hostnet
+
+N, SIDE, CH = 1, 26, 88
+
+class Graph:
+    def __init__(self, light=True):
+        self.net = hostnet.Net(lightmode=light)
+        self.net.add_layer(type="Input", name="data", batchsize=N, channel=CH, height=SIDE, width=SIDE)
+        self.expr, self.convs = {"data": "x"}, []
+    def add(self, name, expr, **options):
+        self.net.add_layer(name=name, **options)
+        self.expr[name] = expr
+        return name
+    def conv(self, number, src, int8=False, dw=False):
+        name = "c%d" % number
+        opts = dict(kernel=3, padding=1, groups=CH, int8_scale_term=1) if dw else dict(kernel=1, int8_scale_term=2)
+        opts["int8_scale_term"] += 100 if int8 else 0
+        self.convs.append((number, dw))
+        return self.add(name, "%s(%s)" % (name, self.expr[src]), type="Convolution", input=src, out_channels=CH, **opts)
+    def sum(self, name, a, b):
+        return self.add(name, "sum(%s,%s)" % tuple(sorted([self.expr[a], self.expr[b]])), type="Eltwise", input=a + "," + b)
+    def shuffle(self, name, a, b):
+        self.add(name + "_cat", "cat(%s,%s)" % (self.expr[a], self.expr[b]), type="Concat", input=a + "," + b)
+        return self.add(name, "shuffle(%s)" % self.expr[name + "_cat"], type="ChannelShuffle", input=name + "_cat", groups=2)
+    def halves(self, name, src):
+        return [self.add(name + "_" + w, "half%d(%s)" % (k, self.expr[src]), type="Crop", input=src, start=k * CH, end=(k + 1) * CH)
+                for k, w in enumerate(("lo", "hi"))]
+    def mean(self, name, src):
+        return self.add(name, "mean(%s)" % self.expr[src], type="GlobalAvgPool", input=src)
+    def unit(self, name, other, branch):
+        return self.halves(name, self.shuffle(name + "_sh", other, branch))
+    def ready(self):
+        self.net.compile()
+        for number, dw in self.convs:
+            w = np.full((CH, 1, 3, 3) if dw else (CH, CH, 1, 1), number, np.int8)
+            self.net.set_conv("c%d" % number, w, None, np.full(CH, 50, np.float32), 20.0, 10.0)
+        return self
+
+def blob():
+    x = np.zeros((N, CH, SIDE, SIDE), np.float32)
+    x.reshape(-1)[:2].view(np.int64)[0] = fake.fake_number(b"x")
+    return x
+def expr_of(a):
+    return fake.fake_expr(C.c_long(int(np.frombuffer(a.tobytes()[:8], np.int64)[0]))).decode()
+def fetched(session):
+    return expr_of(session.fetch((2 * N * CH * SIDE * SIDE,), np.float32))
+
+def head(g):  # a unit's two halves
+    return g.unit("u", g.conv(1, "data"), g.conv(3, g.conv(2, "data", True)))
+
+# tails behind a unit: the blob that is asked for, and whether the unit's last layer and the next unit's first run as a pair
+def sum_with_first_half(g):
+    lo, hi = head(g)
+    return g.sum("out", lo, g.conv(4, hi)), False
+def sum_with_first_half_turned(g):
+    lo, hi = head(g)
+    return g.sum("out", g.conv(4, hi), lo), False
+def sum_from_elsewhere(g):
+    lo, hi = head(g)
+    return g.sum("out", g.conv(5, lo), g.conv(4, hi)), False
+def shuffle_again(g):
+    lo, hi = head(g)
+    return g.shuffle("out", lo, g.conv(4, hi)), False
+def shuffle_again_turned(g):
+    lo, hi = head(g)
+    return g.shuffle("out", g.conv(4, hi), lo), False
+def units_of_one_layer(g):
+    lo, hi = head(g)
+    lo, hi = g.unit("v", lo, g.conv(4, hi))
+    return g.shuffle("out", lo, g.conv(6, g.conv(5, hi, True))), True
+def pooled(g):
+    lo, hi = head(g)
+    g.conv(5, lo)
+    return g.mean("out", g.conv(4, hi)), False
+def next_unit(g):
+    lo, hi = head(g)
+    lo, hi = g.unit("v", lo, g.conv(6, g.conv(5, g.conv(4, hi, True), True, True)))
+    return g.shuffle("out", lo, g.conv(9, g.conv(8, g.conv(7, hi, True), True, True))), True
+def block_with_first_half(g):
+    lo, hi = head(g)
+    return g.sum("out", lo, g.conv(6, g.conv(5, g.conv(4, hi, True), True, True))), True
+def block_with_first_half_turned(g):
+    lo, hi = head(g)
+    return g.sum("out", g.conv(6, g.conv(5, g.conv(4, hi, True), True, True)), lo), True
+def another_pointwise(g):
+    lo, hi = head(g)
+    return g.sum("out", lo, g.conv(5, g.conv(4, hi, True))), True
+def three_pointwise(g):
+    lo, hi = head(g)
+    return g.sum("out", g.conv(6, g.conv(5, g.conv(4, hi, True), True)), g.conv(7, lo)), True
+TAILS = [sum_with_first_half, sum_with_first_half_turned, sum_from_elsewhere, shuffle_again, shuffle_again_turned, units_of_one_layer, pooled,
+         next_unit, block_with_first_half, block_with_first_half_turned, another_pointwise, three_pointwise]
+
+def ran(g):
+    return [int(fake.fake_count(b"c%d" % n)) for n, _ in g.convs]
+"""
+
+
+def run(tmp_path, script, program=False):
+    so, prog, lib = str(tmp_path / "libfake.so"), str(tmp_path / "libprogram.so"), os.path.join(os.path.dirname(HERE), "tensor_amd", "lib")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", os.path.join(HERE, "fake_capi.cpp"), "-o", so])
+    if program:
+        subprocess.check_call(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", os.path.join(HERE, "net_program.cpp"), "-L" + lib, "-lotter_hip_host",
+                               "-Wl,-rpath," + lib, "-o", prog])
+    r = subprocess.run([sys.executable, "-c", SCRIPT + script, so, prog], capture_output=True, text=True, timeout=120, cwd=os.path.dirname(HERE))
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("light", [True, False])
+def test_every_tail_of_a_unit(tmp_path, light):
+    run(tmp_path, r"""
+for form in (3, 2, 1):
+    for join in (1, 0):
+        for pair in (1, 0):
+            for what, v in ((b"form", form), (b"join", join), (b"pair", pair), (b"avgpool", join)): fake.fake_set(what, v)
+            for tail in TAILS:
+                g = Graph(%s)
+                out, pairs = tail(g)
+                where = (tail.__name__, form, join, pair)
+                g.ready()
+                s = g.net.session("data", blob(), out)
+                before, pairs0 = ran(g), fake.fake_count(b"pair")
+                s.run()
+                assert fetched(s) == g.expr[out], (where, fetched(s))
+                once = [b - a for a, b in zip(before, ran(g))]
+                if tail is pooled: del once[3]  # (nobody asks for that one)
+                assert max(once) == 1 and min(once) == 1, (where, once)
+                if pairs and pair and join and form == 3: assert fake.fake_count(b"pair") > pairs0, where
+                for _ in range(5):  # (recorded from the third on)
+                    s.run()
+                    assert fetched(s) == g.expr[out], where
+                    assert expr_of(g.net.eval({"data": blob()}, out)) == g.expr[out], where
+                s.close()
+                g.net.close()
+""" % light)
+
+
+def test_a_second_half_that_is_asked_for_is_there(tmp_path):
+    run(tmp_path, r"""
+for tail in (next_unit, sum_with_first_half, another_pointwise):
+    for ask in ("u_hi", "u_lo", "c4", "u_hi,out", "out,u_hi", "u_lo,c4,out"):
+        g = Graph(light=ask != "out,u_hi")  # (in light mode a pass lets go of what it has read)
+        tail(g)
+        g.ready()
+        s = g.net.session("data", blob(), ask)
+        for _ in range(5):
+            s.run()
+            assert fetched(s) == g.expr[ask.split(",")[-1]], (tail.__name__, ask, fetched(s))
+        if "," not in ask:
+            for _ in range(5): assert expr_of(g.net.eval({"data": blob()}, ask)) == g.expr[ask], (tail.__name__, ask)
+        s.close()
+        g.net.close()
+program = C.CDLL(sys.argv[2])
+program.program_extract.restype = C.c_long
+for tail in (next_unit, another_pointwise):  # not one of those that the program said it would ask for
+    g = Graph()
+    tail(g)
+    g.ready()
+    n = program.program_extract(g.net.h, b"data", blob().ctypes.data_as(C.c_void_p), CH, SIDE, SIDE, b"out", b"u_hi")
+    assert n >= 0 and fake.fake_expr(C.c_long(n)).decode() in (g.expr["u_hi"], "q(%s)" % g.expr["u_hi"]), n
+    g.net.close()
+""", program=True)
