@@ -99,6 +99,7 @@ int otter_host_net_set_conv(void* net, const char* layer_name, const int8_t* wei
         Net* n = static_cast<Net*>(net);
         auto* L = dynamic_cast<ConvolutionLayer*>(n->layer_by_name(layer_name));
         if (!L) return fail(std::string("no Convolution layer named ") + layer_name);
+        n->invalidate_plan();
         const int K = L->out_channels, C = L->in_channels, g = L->groups;
         L->weight_data = Tensor::from_blob(weight, {K, C / g, L->kernel_height, L->kernel_width}, ScalarType::Byte);
         if (L->bias_term && bias) L->bias_data = f32_vec(bias, K);
@@ -111,7 +112,6 @@ int otter_host_net_set_conv(void* net, const char* layer_name, const int8_t* wei
         if (L->int8_scale_term > 100) L->top_blob_int8_scales = f32_vec(ts.data(), (int)ts.size());
         const int rc = L->create_pipeline(n->option);
         if (rc) return fail(std::string("create_pipeline: ") + otter_hip_last_error());
-        n->invalidate_plan();
         return 0;
     } catch (const std::exception& e) {
         return fail(e.what());

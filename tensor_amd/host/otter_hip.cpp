@@ -746,6 +746,7 @@ int ConvolutionLayer::create_pipeline_int8(const NetOption& opt) {
     const bool dw8 = in_channels == groups && groups == out_channels && in_channels % 8 == 0;
     d.in_round_mode = input_round_mode(opt);
     d.out_round_mode = (pk && (dw8 || out_channels % 4 == 0)) ? OTTER_HIP_ROUND_SSE : OTTER_HIP_ROUND_EXACT;
+    ++replaced;
     if (handle_) {
         otter_hip_conv_destroy(handle_);
         handle_ = nullptr;
@@ -1717,6 +1718,7 @@ int InnerProductLayer::load_model(const Initializer& in) {
 // cost it 0.3 ms: one image through the classifier, 1090 us then, 780 now).
 int InnerProductLayer::create_pipeline(const NetOption&) {
     if (!weight_data.defined()) return -1;
+    ++replaced;
     try {
         weight_data.device_ptr();
         if (bias_term && bias_data.defined()) bias_data.device_ptr();
@@ -1925,6 +1927,12 @@ const std::vector<std::string> Net::blob_names() const {
     std::vector<std::string> v;
     for (const Blob& b : blobs_) v.push_back(b.name);
     return v;
+}
+
+unsigned long Net::changes() const {
+    unsigned long n = changes_.load();
+    for (const Layer* l : layers_) n += l->replaced;
+    return n;
 }
 
 std::string Net::describe() const {

@@ -193,6 +193,8 @@ public:
     float fuse_scale = 0.f;
     int fuse_round = 0;
     bool fuse_only = false;  // with fuse_scale > 0: nothing but those convolutions reads the blob
+    // how often create_pipeline has replaced what a pass reads: passes recorded before that are not replayed
+    unsigned long replaced = 0;
     bool int8_only(const NetOption& opt) const {
         return fuse_only && fuse_scale > 0.f && opt.use_packing_layout && opt.wanted && !(*opt.wanted)[tops[0]];
     }
@@ -350,7 +352,7 @@ public:
     // Says that a layer's weights, scales or parameters are no longer what they were (invalidate_plan does too): recorded passes of the
     // net are made again.
     void changed() { ++changes_; }
-    unsigned long changes() const { return changes_.load(); }
+    unsigned long changes() const;
     const std::vector<std::string> blob_names() const;
     std::string describe() const;  // one line per layer: type, name, bottoms, tops, top shape, convolution weights
     int find_blob_index_by_name(const std::string& name) const;

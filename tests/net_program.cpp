@@ -16,4 +16,9 @@ long program_extract(void* net, const char* in, const void* x, int c, int h, int
     if (rc) return rc;
     return t.defined() ? *static_cast<const long*>(t.data_ptr()) : -11;
 }
+// a layer's pipeline built anew by the program itself
+int program_rebuild(void* net, const char* layer) {
+    Net* n = static_cast<Net*>(net);
+    return n->layer_by_name(layer)->create_pipeline(n->option);
+}
 }

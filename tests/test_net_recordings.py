@@ -1,0 +1,74 @@
+"""CPU: the passes that a Net records, over a stand-in for the C ABI (fake_capi.cpp): replays are made where they should be, never of
+what a pass could not do again, and never over a convolution that has been destroyed."""
+from test_net_units import run
+
+NET = r"""
+def net(extra=None):
+    g = Graph()
+    g.conv(2, g.conv(1, "data", True))
+    if extra: extra(g)
+    return g.ready()
+def count(what): return fake.fake_count(what.encode())
+def passes(s, want, n, replays):
+    for _ in range(n):
+        before = count("replay")
+        s.run()
+        assert fetched(s) == want, (fetched(s), want)
+        assert count("replay") - before == replays
+W = lambda v: (np.full((CH, CH, 1, 1), v, np.int8), None, np.full(CH, 50, np.float32), 20.0, 10.0)
+"""
+
+
+def test_passes_are_replayed_from_the_third_on(tmp_path):
+    run(tmp_path, NET + r"""
+g = net()
+s = g.net.session("data", blob(), "c2")
+passes(s, "c2(c1(x))", 2, 0)
+passes(s, "c2(c1(x))", 4, 1)
+assert count("record") == 1
+for k in range(6):
+    x = blob()
+    x.reshape(-1)[:2].view(np.int64)[0] = fake.fake_number(b"y%d" % k)
+    before = count("replay")
+    assert expr_of(g.net.eval({"data": x}, "c2")) == "c2(c1(y%d))" % k
+    assert count("replay") - before == (k >= 3), k  # (the first asks for the size alone)
+""")
+
+
+def test_a_convolution_that_could_not_be_made_again_is_not_replayed(tmp_path):
+    run(tmp_path, NET + r"""
+g = net()
+s = g.net.session("data", blob(), "c2")
+for _ in range(4): s.run()
+fake.fake_set(b"no_conv", 1)
+try:
+    g.net.set_conv("c1", *W(7))
+    raise SystemExit("no error")
+except hostnet.HostError:
+    pass
+for f in (s.run, lambda: g.net.eval({"data": blob()}, "c2")):
+    for _ in range(4):
+        try:
+            f()
+            raise SystemExit("a pass without its layer")
+        except hostnet.HostError:
+            pass
+fake.fake_set(b"no_conv", 0)
+g.net.set_conv("c1", *W(8))
+passes(s, "c2(c8(x))", 2, 0)
+passes(s, "c2(c8(x))", 3, 1)
+assert count("dead") == 0
+""")
+
+
+def test_a_pipeline_that_the_program_builds_anew_is_recorded_anew(tmp_path):
+    run(tmp_path, NET + r"""
+g = net()
+s = g.net.session("data", blob(), "c2")
+for _ in range(4): s.run()
+program = C.CDLL(sys.argv[2])
+assert program.program_rebuild(g.net.h, b"c1") == 0
+passes(s, "c2(c1(x))", 2, 0)
+passes(s, "c2(c1(x))", 3, 1)
+assert count("dead") == 0 and count("record") == 2
+""", program=True)
