@@ -533,14 +533,24 @@ int Layer::forward(const std::vector<Tensor>& bottoms, std::vector<Tensor>& tops
 }
 int Layer::forward_inplace(Tensor&, const NetOption&) const { return -1; }
 
-static std::map<std::string, LayerRegistry::Creator>& registry() {
-    static auto* r = new std::map<std::string, LayerRegistry::Creator>();
+namespace {
+struct Registered {
+    LayerRegistry::Creator creator = nullptr;
+    bool own = false;  // one of this library
+};
+std::map<std::string, Registered>& registry() {
+    static auto* r = new std::map<std::string, Registered>();
     return *r;
 }
-void LayerRegistry::AddCreator(const std::string& type, Creator creator) { registry()[type] = creator; }
+void add_own(const std::string& type, LayerRegistry::Creator creator) { registry()[type] = {creator, true}; }
+}  // namespace
+void LayerRegistry::AddCreator(const std::string& type, Creator creator) { registry()[type] = {creator, false}; }
 Layer* LayerRegistry::CreateLayer(const std::string& type) {
     auto it = registry().find(type);
-    return it == registry().end() ? nullptr : it->second();
+    if (it == registry().end()) return nullptr;
+    Layer* layer = it->second.creator();
+    if (layer) layer->of_library = it->second.own;
+    return layer;
 }
 std::vector<std::string> LayerRegistry::TypeList() {
     std::vector<std::string> v;
@@ -1741,23 +1751,22 @@ int InnerProductLayer::forward(const Tensor& b, Tensor& top, const NetOption&) c
 }
 
 void register_hip_layers() {
-    LayerRegistry::AddCreator("Input", []() -> Layer* { return new InputLayer(); });
-    LayerRegistry::AddCreator("Convolution", []() -> Layer* { return new ConvolutionLayer(); });
-    LayerRegistry::AddCreator("Relu", []() -> Layer* { return new ActivationLayer(1, "Relu"); });
-    LayerRegistry::AddCreator("LRelu", []() -> Layer* { return new ActivationLayer(2, "LRelu"); });
-    LayerRegistry::AddCreator("Relu6", []() -> Layer* { return new ActivationLayer(3, "Relu6"); });
-    LayerRegistry::AddCreator("Eltwise", []() -> Layer* { return new EltwiseLayer(); });
-    LayerRegistry::AddCreator("Split", []() -> Layer* { return new SplitLayer(); });
-    LayerRegistry::AddCreator("InnerProduct", []() -> Layer* { return new InnerProductLayer(); });
-    LayerRegistry::AddCreator("GlobalAvgPool", []() -> Layer* { return new GlobalAvgPoolLayer(); });
-    LayerRegistry::AddCreator("MaxPool", []() -> Layer* { return new MaxPoolLayer(); });
-    LayerRegistry::AddCreator("Concat", []() -> Layer* { return new ConcatLayer(); });
-    LayerRegistry::AddCreator("Crop", []() -> Layer* { return new CropLayer(); });
-    LayerRegistry::AddCreator("ChannelShuffle", []() -> Layer* { return new ChannelShuffleLayer(); });
-    LayerRegistry::AddCreator("ShortCut", []() -> Layer* { return new ShortCutLayer(); });
-    LayerRegistry::AddCreator("Upsample", []() -> Layer* { return new UpsampleLayer(); });
-    LayerRegistry::AddCreator("NanodetPlusDetectionOutput",
-                              []() -> Layer* { return new OffPathLayer("NanodetPlusDetectionOutput"); });
+    add_own("Input", []() -> Layer* { return new InputLayer(); });
+    add_own("Convolution", []() -> Layer* { return new ConvolutionLayer(); });
+    add_own("Relu", []() -> Layer* { return new ActivationLayer(1, "Relu"); });
+    add_own("LRelu", []() -> Layer* { return new ActivationLayer(2, "LRelu"); });
+    add_own("Relu6", []() -> Layer* { return new ActivationLayer(3, "Relu6"); });
+    add_own("Eltwise", []() -> Layer* { return new EltwiseLayer(); });
+    add_own("Split", []() -> Layer* { return new SplitLayer(); });
+    add_own("InnerProduct", []() -> Layer* { return new InnerProductLayer(); });
+    add_own("GlobalAvgPool", []() -> Layer* { return new GlobalAvgPoolLayer(); });
+    add_own("MaxPool", []() -> Layer* { return new MaxPoolLayer(); });
+    add_own("Concat", []() -> Layer* { return new ConcatLayer(); });
+    add_own("Crop", []() -> Layer* { return new CropLayer(); });
+    add_own("ChannelShuffle", []() -> Layer* { return new ChannelShuffleLayer(); });
+    add_own("ShortCut", []() -> Layer* { return new ShortCutLayer(); });
+    add_own("Upsample", []() -> Layer* { return new UpsampleLayer(); });
+    add_own("NanodetPlusDetectionOutput", []() -> Layer* { return new OffPathLayer("NanodetPlusDetectionOutput"); });
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -1933,6 +1942,10 @@ unsigned long Net::changes() const {
     unsigned long n = changes_.load();
     for (const Layer* l : layers_) n += l->replaced;
     return n;
+}
+
+bool Net::recordable() const {
+    return std::all_of(layers_.begin(), layers_.end(), [](const Layer* l) { return l->of_library; });
 }
 
 std::string Net::describe() const {
@@ -2657,7 +2670,8 @@ RecordedPasses::Lease RecordedPasses::lease(const Net& net, const std::string& k
         p->drop();
         p->settings = now;
     }
-    if (p->recording || p->refused || ++p->seen < kRecordFrom || !worth_recording(p->blobs, p->bytes, waited_for)) return l;
+    if (p->recording || p->refused || ++p->seen < kRecordFrom || !worth_recording(p->blobs, p->bytes, waited_for) || !net.recordable())
+        return l;
     struct Scope {  // what this thread launches and allocates until the end belongs to the recording
         bool on = false;
         ~Scope() {

@@ -193,6 +193,9 @@ public:
     float fuse_scale = 0.f;
     int fuse_round = 0;
     bool fuse_only = false;  // with fuse_scale > 0: nothing but those convolutions reads the blob
+    // made by a creator of this library: its launches go where a recording finds them. (A program's own layer launches on the null stream,
+    // at once, and would be missing from the replays.)
+    bool of_library = false;
     // how often create_pipeline has replaced what a pass reads: passes recorded before that are not replayed
     unsigned long replaced = 0;
     bool int8_only(const NetOption& opt) const {
@@ -353,6 +356,7 @@ public:
     // net are made again.
     void changed() { ++changes_; }
     unsigned long changes() const;
+    bool recordable() const;  // every layer is one of this library's
     const std::vector<std::string> blob_names() const;
     std::string describe() const;  // one line per layer: type, name, bottoms, tops, top shape, convolution weights
     int find_blob_index_by_name(const std::string& name) const;

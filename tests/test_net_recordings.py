@@ -1,5 +1,7 @@
 """CPU: the passes that a Net records, over a stand-in for the C ABI (fake_capi.cpp): replays are made where they should be, never of
 what a pass could not do again, and never over a convolution that has been destroyed."""
+import pytest
+
 from test_net_units import run
 
 NET = r"""
@@ -72,3 +74,28 @@ passes(s, "c2(c1(x))", 2, 0)
 passes(s, "c2(c1(x))", 3, 1)
 assert count("dead") == 0 and count("record") == 2
 """, program=True)
+
+
+@pytest.mark.parametrize("own_convolution", [0, 1])
+def test_a_net_with_a_layer_of_the_program_is_not_recorded(tmp_path, own_convolution):
+    run(tmp_path, NET + r"""
+own = %d
+program = C.CDLL(sys.argv[2])
+Graph().net.close()  # (the library's layers are there)
+program.program_register(own)
+g = Graph()
+g.conv(2, g.conv(1, "data", True))
+out = "c2"
+if not own: out = g.add("twice", "", type="Doubled", input="c2")
+g.ready()
+s = g.net.session("data", blob(), out)
+s.run()
+want = fetched(s)
+assert want == (own and "sum(c2(sum(c1(x),c1(x))),c2(sum(c1(x),c1(x))))" or "sum(c2(c1(x)),c2(c1(x)))")
+passes(s, want, 6, 0)
+for k in range(6):
+    x = blob()
+    x.reshape(-1)[:2].view(np.int64)[0] = fake.fake_number(b"y%%d" %% k)
+    assert expr_of(g.net.eval({"data": x}, out)) == want.replace("(x)", "(y%%d)" %% k), k
+assert count("record") == 0
+""" % own_convolution, program=True)
