@@ -29,6 +29,7 @@
 // @147x147 b4 65.7 -> 53.7; 16 -> 48 @167x167 b47 60.3 -> 51.5; 40 -> 168 from fp32 @53x53 b14 14.5 -> 13.0.
 #include "common.hpp"
 #include "conv_igemm.hpp"
+#include "rows_stage.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -269,13 +270,14 @@ __global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF 
                 const int o = rt[0] + c0 * 8 + oct0 * HW8;
                 const int o0 = in0 ? o * INS : OOB, o1 = in1 ? (o + 8) * INS : OOB;
                 int8_t* at = data + oct0 * ra.plane + pos * 16;  // (rows are VW2 pairs long)
-                for (int oct = oct0, so = first * HW8 * INS; oct < count; oct += UN * sub) {
+                RowsWalk walk = rows_walk((unsigned)(HW8 * INS), first, count, sub);
+                for (int oct = oct0; oct < count; oct += UN * sub) {
                     v4i v[UN];
                     v4i f[INF ? UN : 1][4];
 #pragma unroll
                     for (int u = 0; u < UN; ++u) {
                         const bool there = u == 0 || oct + u * sub < count;
-                        const int a0 = there ? o0 : OOB, a1 = there ? o1 : OOB;
+                        const int a0 = there ? o0 : OOB, a1 = there ? o1 : OOB, so = (int)walk.next();
                         if constexpr (INF) {
                             f[u][0] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0, so, 0));
                             f[u][1] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rin, a0 + 16, so, 0));
@@ -288,7 +290,6 @@ __global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF 
                             const v2i h = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rin, a1, so, 0));
                             v[u] = v4i{l[0], l[1], h[0], h[1]};
                         }
-                        so += sub * HW8 * INS;
                     }
                     // (all of them are requested here: the compiler would move the last one behind the condition of its write)
 #pragma unroll
