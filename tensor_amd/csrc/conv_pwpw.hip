@@ -304,16 +304,19 @@ bool conv_pwpw_applicable(const ConvGeom& g0, const Epilogue& e0, const ConvGeom
     return px * g0.C < limit && px * g0.K * (k0 == PP_F32 ? 4 : 1) < limit && px * g1.K * layout_elem_bytes(e1.out_layout) < limit;
 }
 
-// Whether the launch is faster than the two, which deal a layer's channels to workgroups as well: here a workgroup walks through all of
-// both. us as two / one, a layer as wide as its input, int8 between them: 88 channels @26x26 b16 6.6 / 4.7, @52x52 b16 9.8 / 8.3; 176
-// @26x26 b16 8.7 / 7.2, @13x13 b16 6.3 / 5.2, on one 13x13 image 5.0 / 5.1; 232 @52x52 b16 25 / 17.9; 352 @52x52 b16 40 / 30, @26x26
-// b16 14.6 / 13.2, @13x13 b16 8.1 / 8.6, on one 13x13 image 5.2 / 8.3; 48 @26x26 b16 5.4 / 4.4, @52x52 b16 6.6 / 7.0 (with a shuffle
-// 9.4 / 11.4). With a shuffle the others are as far apart.
+// Whether the launch is faster than the two. It saves a launch and the blob in between, but a workgroup walks through all the channels of
+// both layers, a pair of row tiles a wave, where the two launches deal them to workgroups as well: the more pairs, the more workgroups it
+// takes before that is made up for. us as two / one: 88 channels @26x26 b16 (6 pairs, 676 tiles) 6.6 / 4.7; 64 -> 128 -> 1280 on one 7x7
+// image (44 pairs, 4 tiles) 4.8 / 8.4, on 16 of them 5.9 / 8.1; 176 @26x26 b16 (12 pairs) 8.2 / 6.4, on one 13x13 image 5.0 / 5.1; 352 @26x26
+// b16 (22 pairs, 676 tiles) 14.6 / 13.2, @13x13 b16 (169) 8.1 / 8.6. Where the first layer has at most two pairs, two of the four waves
+// idle through it: small launches gain all the same, large ones do not (48 channels @26x26 b16 5.4 / 4.4, @52x52 b16 6.6 / 7.0; with a
+// shuffle 9.4 / 11.4). Over 11600 drawn pairs of 8 to 512 and 8 to 1280 channels, half of them with a shuffle, the faster of the two is missed
+// by 0.5 % on average, by over 5 % for 270 of the 7200 taken and for 210 of the others.
 bool conv_pwpw_faster(const ConvGeom& g0, const ConvGeom& g1) {
     const long tiles = ((long)g0.N * g0.H * g0.W + 15) / 16;
-    const int steps = std::max(igemm_channel_groups(g0.C), igemm_channel_groups(g1.C));
-    if (steps == 1) return tiles < 1024;
-    return tiles >= (steps <= 2 ? 1 : steps <= 4 ? 128 : 512);
+    const int first = (g0.K + 31) / 32, pairs = first + (g1.K + 31) / 32;
+    if (first <= 2) return pairs <= 10 && tiles < 1536;
+    return tiles >= (pairs > 17 ? 640 : pairs > 10 ? 128 : first > 4 ? 8 : 1);
 }
 
 template <int FN, int SC, int EPI>

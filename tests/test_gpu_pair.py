@@ -53,6 +53,11 @@ def test_which_are_one_launch(hip):
                          (48, 16, 52, 2)):
         a, b = layer(hip, rng, C, C, 2, False), layer(hip, rng, C, C, 2, False)
         assert hip.conv_pair_launches(a, b, n, h, h) == one, (C, n, h)
+    # channels that one workgroup would walk for all the others, first layers of two pairs on large batches
+    for C, K, K2, n, h, one in ((64, 128, 1280, 1, 7, 2), (64, 128, 1280, 16, 7, 2), (128, 512, 128, 1, 14, 2), (88, 88, 88, 64, 56, 1),
+                                (128, 64, 128, 64, 56, 2), (128, 16, 64, 1, 14, 1), (136, 24, 40, 1, 7, 1)):
+        a, b = layer(hip, rng, C, K, 2, False), layer(hip, rng, K, K2, 2, False)
+        assert hip.conv_pair_launches(a, b, n, h, h) == one, (C, K, K2, n, h)
 
 
 @pytest.mark.parametrize("C,K,K2,n,h,w,act0,act1", CASES)
