@@ -23,6 +23,9 @@
 #include "common.hpp"
 #include "conv_igemm.hpp"
 
+#include <algorithm>
+#include <numeric>
+
 namespace ohip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -376,15 +379,17 @@ struct HaloPlan {
     double cost;
 };
 
-// input rows a run of pt output pixels starting at a multiple of pt can touch (stride s, dilation d), halo included
+// input rows a run of pt output pixels starting at a multiple of pt can touch (stride s, dilation d), halo included. (Tiles start at
+// multiples of gcd(pt, OW) in a row; the first one that starts at the last of them, or a like one, ends the search: on a 216x216 image a plan
+// took 4 us of host time without that.)
 int halo_rows(int pt, int OW, int OHW, int s, int d) {
+    const int most = (OW - std::gcd(pt, OW) + pt - 1) / OW;
     int worst = 0;
-    for (int p0 = 0; p0 < OHW; p0 += pt) {
+    for (int p0 = 0; p0 < OHW && worst < most; p0 += pt) {
         const int last = (p0 + pt < OHW ? p0 + pt : OHW) - 1;
-        const int rows = (last / OW - p0 / OW) * s + 2 * d + 1;
-        if (rows > worst) worst = rows;
+        worst = std::max(worst, last / OW - p0 / OW);
     }
-    return worst;
+    return worst * s + 2 * d + 1;
 }
 
 // The per-lane LDS offsets of a tile may be reused for the workgroup's next tile only if every tile covers the same
@@ -544,6 +549,23 @@ bool conv3x3_halo_plan(const ConvGeom& g, int force_fn, int plan[8]) {
     plan[0] = p.fn, plan[1] = pt, plan[2] = p.tiles_per_img, plan[3] = grid_x, plan[4] = m_blocks;
     plan[5] = halo_tile_invariant(pt, g.OW, g.OH * g.OW) ? 1 : 0, plan[6] = p.r_max, plan[7] = p.cb;
     return true;
+}
+
+// A launch's time in us (in a row of launches, warm): per tile that a workgroup walks the matrix work and the epilogue of its fragments and
+// the rows that a wave stages, which two workgroups of a compute unit share, and a latency per stage of the channels; bytes out.
+// Fitted to 2200 drawn layers of 3 to 130 us (an early form of pixels, rows and chunks alone was off by over 28 % for one in ten of them and took
+// launches of over 30 us for 14 % shorter than they are, so that they kept layers which the staged rows run in half the time); over 1150
+// others the median error is 6 %, 9 in 10 below 13 %.
+float conv3x3_halo_cost(const ConvGeom& g, float out_mb) {
+    HaloPlan p;
+    if (!plan_halo(g, 0, &p)) return __builtin_inff();
+    const int mpad = igemm_padded_rows(g.K), cpad = igemm_channel_groups(g.C) * 64, total = g.N * p.tiles_per_img, oct = (g.C + 7) / 8;
+    int m_blocks, grid_x;
+    halo_grid(mpad, mpad > 64 ? 8 : mpad / 16, total, &m_blocks, &grid_x);
+    const float walk = (float)((total + grid_x - 1) / grid_x), share = grid_x * m_blocks > 256 ? 1.64f : 1.f;
+    const float frags = (float)((mpad >= 64 ? 4 : 2) * p.fn), stages = (float)(cpad / p.cb);
+    const float moves = 0.25f * (float)p.r_max * (float)(p.logp == 9 ? (oct + 1) / 2 : p.logp == 10 ? oct : 2 * oct);
+    return 2.44f + walk * (share * (frags * (0.008f * (float)(9 * (cpad / 64)) + 0.0727f) + 0.0775f * moves) + 0.888f * stages) + 0.111f * out_mb;
 }
 
 hipError_t run_conv3x3_halo(const int8_t* x, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep,

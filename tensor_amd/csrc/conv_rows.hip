@@ -254,9 +254,8 @@ __global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF 
                 e < taps * count ? (int)oct * ra.plane + (int)dy * g.dh * ra.pitch + (int)dx * g.dw * 8 : 0;
         }
         // the stage's rows, zeros outside the image, as pixel pairs. A thread keeps one place of the octet planes and walks the
-        // octets, so that an octet costs it a load and a write and no address arithmetic; planes of at most 128 pairs are dealt to
-        // a half, a quarter or an eighth of the threads each
-        const int pairs = rows * ra.VW2, sub_shift = pairs > 128 ? 0 : pairs > 64 ? 1 : pairs > 32 ? 2 : 3, sub = 1 << sub_shift;
+        // octets, so that an octet costs it a load and a write and no address arithmetic
+        const int pairs = rows * ra.VW2, sub_shift = rows_parts_shift(pairs), sub = 1 << sub_shift;
         const int oct0 = tid >> (8 - sub_shift);
         // (two walks, not a choice per load: behind loads on two branches the compiler waited for each octet before it requested the
         // next, four memory latencies in a row)
@@ -565,7 +564,8 @@ float conv_rows_cost(const ConvGeom& g_in, bool f32in, int out_bytes, int* confi
         if (!fits) continue;
         const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm), bpw = rows_blocks_per_workgroup(ra, blocks, c.fm);
         const int pairs = ra.rows_max * ra.VW2, oct = (ra.g.C / 8 + ra.stages - 1) / ra.stages;
-        const float places = (float)(ra.stages * oct) * (pairs > 128 ? (float)((pairs + 255) / 256) : 1.f / (float)(256 / pairs));
+        const int parts = 1 << rows_parts_shift(pairs), part = 256 / parts;
+        const float places = (float)(ra.stages * oct * ((pairs + part - 1) / part)) / (float)parts;
         const int slices = (blocks + bpw - 1) / bpw;
         const int wgs = (int)std::min(((long)ra.n_tiles * slices * ra.g.groups + 255) / 256, 1l << 24);
         const RowsCost& cost = f32in ? c.f32 : c.i8;

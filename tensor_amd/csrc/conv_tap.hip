@@ -455,7 +455,8 @@ float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config) {
 
 // The same for the launches that the kernel above competes with (families of otter_hip_conv_kernel_kind): the
 // implicit-GEMM kernel (1; with fp32 input for pointwise layers), the LDS-halo kernel (3), the fp32 pointwise kernel (6).
-// Start + chain * chunks + matrix work + epilogue + bytes in + bytes out, fitted to drawn layers; median error 4 to 11 %. The fp32
+// Start + chain * chunks + matrix work + epilogue + bytes in + bytes out, fitted to drawn layers; median error 4 to 11 % (k x k layers of
+// the implicit-GEMM kernel 6 %, 13 % on the slow side before its index divisions became multiplications). The fp32
 // pointwise kernel walks all output channels per workgroup of 64 pixels, so that its chain grows with them (128 -> 1280 on one
 // 29x29 image: 15.6 us, where the kernel above takes 5.8).
 float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes) {
@@ -468,8 +469,8 @@ float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes)
         const float cu = ceilf((float)g.N * (float)((g.H * g.W + 63) / 64) / 256), k = 0.01f * (float)K;
         return 2.18f + 0.5f * cu + 0.2f * chunks + k * (0.336f + 0.333f * cu + chunks * (0.063f + 0.096f * cu)) + 0.39f * in_mb + 0.048f * out_mb;
     }
-    if (family == 3) return 2.97f + 0.27f * chunks + 25.2f * mac + 39.6f * epi + 0.055f * out_mb;
-    if (taps > 1) return 3.08f + 0.327f * chunks + 62.1f * mac + 44.2f * epi + px * (6.5e-6f + 1.71e-6f * chunks) + 0.061f * in_mb + 0.052f * out_mb;
+    if (family == 3) return conv3x3_halo_cost(g, out_mb);
+    if (taps > 1) return 2.93f + 0.308f * chunks + 59.7f * mac + 30.2f * epi + px * (3.43e-6f + 1.121e-6f * chunks) + 0.095f * in_mb + 0.065f * out_mb;
     if (f32in) return 2.37f + 0.50f * chunks + 201.f * mac + 18.f * epi + 0.33f * in_mb + 0.09f * out_mb;
     return 2.46f + 0.34f * chunks + 94.f * mac + 26.f * epi + 0.03f * in_mb + 0.07f * out_mb;
 }

@@ -1,6 +1,7 @@
 """CPU: the scalar offsets with which the launch on staged rows requests the octets of a stage (rows_stage.hpp). None is beyond the blob's bytes,
 where the difference that the hardware compares a lane's offset with would wrap, and every octet that the stage has is asked for at
-its place: layers of few octets on one image, of several stages, of blobs of up to 2 GB."""
+its place: layers of few octets on one image, of several stages, of blobs of up to 2 GB. The parts that the threads are dealt in hold
+the places of a plane."""
 import os
 import subprocess
 
@@ -27,6 +28,14 @@ static const char* check(u64 plane, int octets, int first, int count, int sub, i
     return nullptr;
 }
 int main() {
+    for (int places = 1; places <= 4096; ++places) {
+        const int shift = rows_parts_shift(places), part = 256 >> shift;
+        // a part holds the plane where there are several, and is no larger than it has to be
+        if (shift < 0 || shift > 3 || (shift > 0 && places > part) || (shift < 3 && places <= part / 2)) {
+            std::printf("%d places in parts of %d threads\n", places, part);
+            return 1;
+        }
+    }
     for (int octets = 1; octets <= 40; ++octets)
         for (u64 plane : {8ull, 32ull, 392ull, 40000ull, 1ull << 26, (1ull << 31) / (u64)octets / 8 * 8})
             if (plane * (u64)octets < (1ull << 31))
