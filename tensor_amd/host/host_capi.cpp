@@ -319,6 +319,11 @@ int otter_host_net_load_weight(void* net, const char* path, int ncnn) {
 // how many runs of convolution layers went through the chain entry point as one launch, in this process
 long otter_host_chain_forward_count(void) { return ConvolutionLayer::chain_forward_count(); }
 long otter_host_block_forward_count(void) { return ConvolutionLayer::block_forward_count(); }
+// of this process so far: passes recorded, replays, passes that turned out not to be recordable
+void otter_host_recording_counts(long counts[3]) {
+    const RecordedPasses::Counts c = RecordedPasses::counts();
+    counts[0] = c.recorded, counts[1] = c.replayed, counts[2] = c.refused;
+}
 
 long otter_host_net_describe(void* net, char* buf, size_t capacity) {
     try {

@@ -2568,6 +2568,9 @@ RecordedPasses::Settings settings_of(const Net& net) {
 }
 }  // namespace
 
+static std::atomic<long> g_recorded{0}, g_replayed{0}, g_refused{0};
+RecordedPasses::Counts RecordedPasses::counts() { return {g_recorded.load(), g_replayed.load(), g_refused.load()}; }
+
 struct RecordedPasses::Pass {
     std::string key;
     Settings settings;
@@ -2616,6 +2619,7 @@ void RecordedPasses::drop_idle() {
 void RecordedPasses::Lease::replay() const {
     hip_check(otter_hip_record_launch(pass_->recording, nullptr), "replay");
     g_block_forwards += pass_->blocks;
+    ++g_replayed;
 }
 
 const std::vector<Tensor>& RecordedPasses::Lease::inputs() const { return pass_->inputs; }
@@ -2697,10 +2701,12 @@ RecordedPasses::Lease RecordedPasses::lease(const Net& net, const std::string& k
         scope.on = false;
         hip_check(otter_hip_record_end(stream, &p->recording), "recording");
         p->arena = arena, p->blocks = t_made.blocks - blocks;
+        ++g_recorded;
     } catch (const std::exception&) {
         t_recording.arena.reset();
         p->drop();
         p->refused = true;
+        ++g_refused;
     }
     return l;
 }

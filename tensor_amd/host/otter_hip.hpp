@@ -493,6 +493,11 @@ public:
     Lease lease(const Net& net, const std::string& key, bool waited_for, const std::function<std::vector<Tensor>()>& make_inputs,
                 const std::function<Tensor(const std::vector<Tensor>&)>& pass);
     static void drop_idle();  // gives back what no thread is using
+    // of this process so far (for tests): passes recorded, replays, passes that turned out not to be recordable
+    struct Counts {
+        long recorded, replayed, refused;
+    };
+    static Counts counts();
 
 private:
     std::mutex mu_;

@@ -15,7 +15,7 @@ EXPORTS = ["otter_host_last_error", "otter_host_net_create", "otter_host_net_des
            "otter_host_functional_chain", "otter_host_net_load_otter", "otter_host_net_load_weight",
            "otter_host_net_describe", "otter_host_net_conv_fp32_probe", "otter_host_net_eval", "otter_host_net_eval_fetch",
            "otter_host_otter_dump", "otter_host_ncnn_read",
-           "otter_host_chain_forward_count", "otter_host_block_forward_count"]
+           "otter_host_chain_forward_count", "otter_host_block_forward_count", "otter_host_recording_counts"]
 
 
 def load_cdll():
@@ -42,6 +42,13 @@ def block_forward_count():
 def chain_forward_count():
     """Runs of convolution layers that went through the C ABI's chain entry point as one launch, in this process."""
     return load_cdll().otter_host_chain_forward_count()
+
+
+def recording_counts():
+    """(passes recorded, replays, passes that turned out not to be recordable) of this process so far."""
+    c = (C.c_long * 3)()
+    load_cdll().otter_host_recording_counts(c)
+    return tuple(c)
 
 
 def _opts(d):

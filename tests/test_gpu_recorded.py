@@ -1,11 +1,12 @@
 """Passes that a Net records and replays (Session.run and Net.eval from the third pass on): every replay gives what a pass made launch
 by launch gives, with other work in between, and a net whose weights have changed is recorded anew."""
+import os
 import threading
 
 import numpy as np
 import pytest
 
-from tensor_amd import capi, hostnet, mobilenet
+from tensor_amd import hostnet, mobilenet, modelfile
 
 pytestmark = pytest.mark.gpu
 
@@ -21,8 +22,18 @@ def classifier(rng, n, side=SIDE):
     return mobilenet.build_net(hostnet, layers, params, n, side), layers, params
 
 
-def unrecorded(net, x, out="fc"):
-    return net.run("data", x, out)  # (never recorded)
+class Counted:
+    """What has been recorded, replayed and refused since it was made."""
+
+    def __init__(self):
+        self.start = hostnet.recording_counts()
+
+    def __call__(self):
+        return tuple(b - a for a, b in zip(self.start, hostnet.recording_counts()))
+
+
+def unrecorded(net, x, out="fc", into="data"):
+    return net.run(into, x, out)  # (never recorded)
 
 
 @pytest.mark.parametrize("n", [1, 3])
@@ -34,8 +45,10 @@ def test_session_replays_equal_passes_by_launches(hip, n):
     s = net.session("data", x, "fc")
     other = rng.random((n, 3, SIDE, SIDE), dtype=np.float32)
     busy = hip.empty(1 << 20, np.float32)
+    counted = Counted()
     for i in range(8):
         s.run()
+        assert counted() == ((1, i - 1, 0) if i > 1 else (0, 0, 0)), i
         if i % 2:
             unrecorded(net, other)  # takes and gives back blobs of the same sizes
             busy.zero_()
@@ -47,15 +60,19 @@ def test_session_replays_equal_passes_by_launches(hip, n):
 def test_eval_replays_on_new_inputs_and_shapes(hip):
     rng = np.random.default_rng(5)
     net, _, _ = classifier(rng, 2)
+    counted = Counted()
     for i in range(10):
         n, side = ((2, SIDE), (1, SIDE), (2, 96))[i % 3 if i < 6 else 0]
         x = rng.random((n, 3, side, side), dtype=np.float32)
         np.testing.assert_array_equal(net.eval({"data": x}, "fc").reshape(n, 1000), unrecorded(net, x).reshape(n, 1000))
+    # (a first pass of a shape asks for the size alone; of the others the third is recorded)
+    assert counted() == (1, 3, 0)
     # a blob inside the net, a packed one
     name = next(l["name"] for l in mobilenet.describe() if l["kind"] == "add")
     for i in range(5):
         x = rng.random((1, 3, SIDE, SIDE), dtype=np.float32)
         np.testing.assert_array_equal(net.eval({"data": x}, name), unrecorded(net, x, name))
+    assert counted() == (2, 5, 0)
     net.close()
 
 
@@ -78,10 +95,12 @@ def test_new_weights_and_settings_are_recorded_anew(hip):
             if rnd == 3:
                 hip.conv_block_set_always(2)
             want = unrecorded(net, x).reshape(-1)
+            counted = Counted()
             for _ in range(5):
                 s.run()
                 np.testing.assert_array_equal(s.fetch((1, 1000), np.float32).reshape(-1), want)
                 np.testing.assert_array_equal(net.eval({"data": x}, "fc").reshape(-1), want)
+            assert counted() == (2, 5 if rnd == 0 else 6, 0), rnd  # (the first eval asks for the size alone)
     finally:
         hip.conv_block_set_always(always)
     s.close()
@@ -94,6 +113,7 @@ def test_threads_share_a_recorded_net(hip):
     xs = [rng.random((1, 3, SIDE, SIDE), dtype=np.float32) for _ in range(3)]
     want = [unrecorded(net, x).reshape(-1) for x in xs]
     errors = []
+    counted = Counted()
 
     def work(i):
         try:
@@ -109,7 +129,88 @@ def test_threads_share_a_recorded_net(hip):
         t.join(timeout=60)
         assert not t.is_alive()
     assert not errors, errors[0]
+    recorded, replayed, refused = counted()
+    assert recorded == 1 and 1 <= replayed <= 36 and refused == 0  # (a thread whose turn it is not launches for itself)
     net.close()
+
+
+HEADS = ["conv_95", "conv_100", "conv_105", "conv_110"]
+
+
+@pytest.mark.parametrize("last", HEADS)
+def test_detector_with_several_results(hip, tmp_path, last):
+    net = hostnet.Net()
+    net.load_otter(os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "nanodet-plus-m-1.5x_416_int8_fused.otter"))
+    weights, _ = modelfile.synthetic_int8_weights(net.describe(), np.random.default_rng(3))
+    path = tmp_path / "weights.bin"
+    path.write_bytes(weights)
+    net.load_weight(str(path), ncnn=True)
+    x = np.random.default_rng(4).random((1, 3, 416, 416), dtype=np.float32)
+    want = unrecorded(net, x, last, into="data_1")
+    s = net.session("data_1", x, ",".join([h for h in HEADS if h != last] + [last]))
+    counted = Counted()
+    for i in range(6):
+        s.run()
+        np.testing.assert_array_equal(s.fetch(want.shape, want.dtype), want)
+    assert counted() == (1, 4, 0)
+    s.close()
+    net.close()
+
+
+def stack(rng, layers, C, side, kernel, n=2, int8_in=False):
+    net = hostnet.Net()
+    net.add_layer(type="Input", name="data", batchsize=n, channel=C, height=side, width=side)
+    for i in range(layers):
+        net.add_layer(type="Convolution", name="s%d" % i, out_channels=C, kernel=kernel, padding=kernel // 2,
+                      int8_scale_term=102 if i < layers - 1 else 2, activation="Relu")
+    net.compile()
+    for i in range(layers):
+        net.set_conv("s%d" % i, rng.integers(-127, 128, (C, C, kernel, kernel)).astype(np.int8), rng.normal(0, 0.1, C).astype(np.float32),
+                     rng.uniform(300, 900, C).astype(np.float32), 25.0, 25.0)
+    return net, "s%d" % (layers - 1)
+
+
+def test_an_int8_input(hip):
+    rng = np.random.default_rng(8)
+    net, out = stack(rng, 13, 24, 9, 5)
+    counted = Counted()
+    x = rng.integers(-127, 128, (2, 24, 9, 9)).astype(np.int8)
+    want = unrecorded(net, x, out)
+    assert len(np.unique(want)) > 100
+    s = net.session("data", x, out)
+    for i in range(6):
+        s.run()
+        y = rng.integers(-127, 128, x.shape).astype(np.int8)
+        np.testing.assert_array_equal(net.eval({"data": y}, out), unrecorded(net, y, out))
+        s.run()
+    assert s.fetch((want.size,), np.float32).size == want.size and counted()[0] == 2 and counted()[1] >= 10
+    np.testing.assert_array_equal(net.eval({"data": x}, out), want)
+    s.close()
+    net.close()
+
+
+def test_a_net_with_a_chain_goes_on_without_a_recording(hip):
+    rng = np.random.default_rng(9)
+    tiles = hip.conv_chain_set_min_tiles(0)
+    try:
+        net, out = stack(rng, 14, 64, 14, 3)
+        chains = hostnet.chain_forward_count()
+        counted = Counted()
+        x = rng.random((2, 64, 14, 14), dtype=np.float32)
+        want = unrecorded(net, x, out)
+        assert hostnet.chain_forward_count() > chains and len(np.unique(want)) > 100
+        s = net.session("data", x, out)
+        for i in range(6):
+            s.run()
+            y = rng.random(x.shape, dtype=np.float32)
+            np.testing.assert_array_equal(net.eval({"data": y}, out), unrecorded(net, y, out))
+            np.testing.assert_array_equal(net.eval({"data": x}, out), want)
+        recorded, replayed, refused = counted()
+        assert (recorded, replayed) == (0, 0) and refused >= 1
+        s.close()
+        net.close()
+    finally:
+        hip.conv_chain_set_min_tiles(tiles)
 
 
 def test_recordings_take_launches_only(hip):

@@ -99,3 +99,24 @@ for k in range(6):
     assert expr_of(g.net.eval({"data": x}, out)) == want.replace("(x)", "(y%%d)" %% k), k
 assert count("record") == 0
 """ % own_convolution, program=True)
+
+
+def test_passes_go_on_after_memory_ran_out_while_one_was_recorded(tmp_path):
+    run(tmp_path, NET + r"""
+g = net()
+s = g.net.session("data", blob(), "c2")
+passes(s, "c2(c1(x))", 2, 0)
+other = g.net.session("data", blob(), "c2")  # (its input takes the blob that the first pass has given back)
+fake.fake_set(b"no_memory", 1)
+try:
+    s.run()
+    raise SystemExit("a pass without its blobs")
+except hostnet.HostError:
+    pass
+fake.fake_set(b"no_memory", 0)
+assert hostnet.recording_counts() == (0, 0, 1)
+passes(s, "c2(c1(x))", 4, 0)
+g.net.set_conv("c1", *W(5))  # (recorded again once the net has changed)
+passes(s, "c2(c5(x))", 2, 0)
+passes(s, "c2(c5(x))", 2, 1)
+""")
