@@ -118,12 +118,15 @@ static thread_local struct {
     void* stream = nullptr;
     std::shared_ptr<BlobArena> arena;
 } t_recording;
-// what this thread's passes have made so far
+// what this thread's passes have made so far: calls that launch, blocks that ran as one of them, bytes of device blobs
 static thread_local struct {
-    long blocks = 0, blobs = 0;
+    long launches = 0, blocks = 0;
     size_t bytes = 0;
 } t_made;
-static void* launch_stream() { return t_recording.stream; }
+static void* launch_stream() {
+    ++t_made.launches;
+    return t_recording.stream;
+}
 static void not_while_recording(const char* what) {
     if (t_recording.stream) throw Error(std::string("a recorded pass cannot ") + what);
 }
@@ -297,7 +300,7 @@ struct Tensor::Storage {
         else pool().put(bytes, dev);
     }
     void take_device() {
-        ++t_made.blobs, t_made.bytes += bytes;
+        t_made.bytes += bytes;
         arena = t_recording.arena;
         dev = arena ? arena->get(bytes) : pool().get(bytes);
     }
@@ -2575,7 +2578,7 @@ struct RecordedPasses::Pass {
     std::string key;
     Settings settings;
     int seen = 0;          // passes that ran one launch at a time
-    long blobs = 0;        // of the last one of them
+    long launches = 0;     // of the last one of them
     size_t bytes = 0;
     bool refused = false;  // cannot be recorded
     bool busy = false;     // leased by a thread
@@ -2625,23 +2628,32 @@ void RecordedPasses::Lease::replay() const {
 const std::vector<Tensor>& RecordedPasses::Lease::inputs() const { return pass_->inputs; }
 const Tensor* RecordedPasses::Lease::result() const { return pass_ && pass_->recording ? &pass_->out : nullptr; }
 
-RecordedPasses::Lease::Lease(RecordedPasses* owner, Pass* pass) : owner_(owner), pass_(pass), blobs_(t_made.blobs), bytes_(t_made.bytes) {}
+RecordedPasses::Lease::Lease(RecordedPasses* owner, Pass* pass) : owner_(owner), pass_(pass), launches_(t_made.launches), bytes_(t_made.bytes) {}
 
 RecordedPasses::Lease::~Lease() {
     if (!pass_) return;
-    if (!pass_->recording) pass_->blobs = t_made.blobs - blobs_, pass_->bytes = t_made.bytes - bytes_;
+    if (!pass_->recording) pass_->launches = t_made.launches - launches_, pass_->bytes = t_made.bytes - bytes_;
     std::lock_guard<std::mutex> lock(owner_->mu_);
     pass_->busy = false;
 }
 
-// Whether a pass is made faster by its recording: a replay costs 5 us of its own, and where the launches' work is longer than the
-// host's 3.7 us for each nothing is gained. Passes one after the other / each waited for, recorded against launched, by the bytes
-// of a blob on average: classifier (41 launches, 55 blobs) 28 KB 0.82 / 0.67, 113 KB 0.95 / 0.83, 153 KB 0.93 / 0.82, 226 KB 1.02 /
-// 0.89, 310 KB 1.02 / 0.91, 620 KB 1.02 / 0.95, 1.2 MB 1.02 / 1.00; detection model (124 launches, 146 blobs) 0.27 MB 0.80 / 0.76,
-// 1.1 MB 0.95 / 0.87, 1.6 MB 1.00 / 0.93, 2.2 MB 1.00 / 1.00, 4.4 MB 1.01 / 1.03.
-static bool worth_recording(long blobs, size_t bytes, bool waited_for) {
-    const size_t most = waited_for ? 900u << 10 : blobs < 80 ? 160u << 10 : 1100u << 10;
-    return bytes <= most * (size_t)blobs;
+// Whether a pass is made faster by its recording. Launch by launch the host spends 3.3 to 3.8 us on each; of a recording a launch takes the
+// GPU 1.8 us and its own time, and the replay 5 us. So it has to be many launches, which share those, and short ones: what a launch
+// takes goes by its blobs' bytes, if loosely. Recorded against launched, passes one after the other, by KB of blobs made per launching call:
+//   7 calls   3x3 48 <-> 72              5 1.13, 83 1.17, 333 1.20
+//   13        5x5 depthwise, 1x1, sum    61 0.86, 486 0.93, 973 1.03
+//   21        3x3                        59 0.89, 237 0.99, 473 1.03
+//   27        classifier                 62 0.79, 171 0.93, 334 0.95, 668 1.00, 1000 1.02
+//   41        3x3                        53 0.89, 213 0.95, 426 0.99, 852 1.00
+//   63        5x5 depthwise, 1x1, sum    57 0.65, 459 0.68, 918 0.72, 1835 0.91
+//   103       detection model            368 1.02, 737 1.02, 1546 1.00
+//   123       5x5 depthwise, 1x1, sum    57 0.80, 455 0.83, 911 0.91, 1821 0.99
+//   141       3x3                        3 0.96, 49 1.02, 195 1.03, 391 1.06
+// A host that waits for every pass also waits for its first launches: 7 calls 5 0.71, 333 0.93, 667 1.03; 9 502 1.06; 13 486 0.80, 973 0.91;
+// 27 334 0.79, 668 0.93, 1336 0.97, 2308 0.99; 43 1848 0.97; 103 368 1.01, 737 0.99, 1546 1.00.
+static bool worth_recording(long launches, size_t bytes, bool waited_for) {
+    if (waited_for) return bytes <= (size_t)launches * std::min<size_t>((size_t)launches * 50 << 10, 1536 << 10);
+    return launches > 10 && bytes <= (size_t)(launches - 10) << 20;
 }
 
 RecordedPasses::Lease RecordedPasses::lease(const Net& net, const std::string& key, bool waited_for, const std::function<std::vector<Tensor>()>& make_inputs,
@@ -2674,7 +2686,7 @@ RecordedPasses::Lease RecordedPasses::lease(const Net& net, const std::string& k
         p->drop();
         p->settings = now;
     }
-    if (p->recording || p->refused || ++p->seen < kRecordFrom || !worth_recording(p->blobs, p->bytes, waited_for) || !net.recordable())
+    if (p->recording || p->refused || ++p->seen < kRecordFrom || !worth_recording(p->launches, p->bytes, waited_for) || !net.recordable())
         return l;
     struct Scope {  // what this thread launches and allocates until the end belongs to the recording
         bool on = false;

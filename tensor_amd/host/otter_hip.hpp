@@ -475,7 +475,7 @@ public:
     public:
         Lease() = default;
         Lease(RecordedPasses* owner, Pass* pass);
-        Lease(Lease&& o) : owner_(o.owner_), pass_(o.pass_), blobs_(o.blobs_), bytes_(o.bytes_) { o.pass_ = nullptr; }
+        Lease(Lease&& o) : owner_(o.owner_), pass_(o.pass_), launches_(o.launches_), bytes_(o.bytes_) { o.pass_ = nullptr; }
         Lease& operator=(Lease&&) = delete;
         ~Lease();
         const Tensor* result() const;               // the blob that a replay leaves its result in, until the next one; or null
@@ -485,7 +485,7 @@ public:
     private:
         RecordedPasses* owner_ = nullptr;
         Pass* pass_ = nullptr;
-        long blobs_ = 0;  // what the thread had made when the lease began
+        long launches_ = 0;  // what the thread had made when the lease began
         size_t bytes_ = 0;
     };
     // key: what the pass is, its inputs' shapes included; waited_for: whether the host waits for every pass; make_inputs: the blobs
