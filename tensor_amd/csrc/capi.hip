@@ -753,11 +753,11 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 //
 // Otherwise, of families 1 and 3 (with an fp32 blob also 6), by the cost models: the kernel
 // whose workgroups deal the reduction to their waves (conv_tap.hip) and, for k x k layers without a sum or a twin, the one on
-// staged rows (conv_rows.hip). A k x k layer on an int8 blob takes the fastest of the three by their models, the
-// last one's less 5 % where there is no stride, which is what it says too much. Drawn layers of over 4 us that the fits had not seen then take
-// longer than the fastest of the three by 1.0 % on average (2358 without a stride; 68 by over 10 %) and 2.2 % (614 with one; 38); where either
-// has to be faster by 5 % 1.4 % (112) and 2.9 % (50). Else the first has to be faster by 5 % (pointwise layers on an fp32 blob with a
-// launch of their own there: 10 %), and on an fp32 blob the second as well where there is a stride (in between it is 6 % slower). An fp32 blob is otherwise quantized by a pass of its own, 2 us and
+// staged rows (conv_rows.hip). A k x k layer on an int8 blob takes the fastest of the three by their models: drawn
+// layers of over 4 us that the fits had not seen then take longer than the fastest by 0.9 % on average (2084 without a stride; 44 by over 10 %)
+// and 1.6 % (589 with one; 32); with the halo and implicit-GEMM kernels' models of before, and 5 % to be won by with a stride, 1.4 % (85)
+// and 1.8 % (40). Else the first has to be faster by 5 % (pointwise layers on an fp32 blob with a launch of their own there: 10 %), and
+// on an fp32 blob the second as well where there is a stride (in between it is 6 % slower). An fp32 blob is otherwise quantized by a pass of its own, 2 us and
 // 0.65 us per million values (0.85 beyond 50 million), in front of whichever int8 kernel is faster (strided pointwise layers, 32 -> 56
 // on three 24x24 images: 5.9 us with that pass, 3.7 without). Over 2000 drawn layers that the fits had not seen,
 // each on an int8 and on an fp32 blob, the choice takes 53 % of the time of the families' launches alone (k x k; pointwise 88 and
@@ -789,8 +789,7 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
         other = pass + (tap_t < 0.95f * (pass + fminf(other, least)) ? other : fminf(other, rows_cost(false, other, &unused)));
     }
     const float best = tap_t < (own ? 0.9f : f32in || !kxk ? 0.95f : 1.f) * other ? tap_t : other;
-    const float most = f32in ? (g.sw > 1 ? 0.95f : 1.f) : g.sw > 1 ? 1.f : 1.05f;
-    if (rows_cost(f32in, best, &rows_tile) < most * best) return *config = rows_tile, ALT_ROWS;
+    if (rows_cost(f32in, best, &rows_tile) < (f32in && g.sw > 1 ? 0.95f : 1.f) * best) return *config = rows_tile, ALT_ROWS;
     return *config = tap_tile, best < other ? ALT_TAP : ALT_NONE;
 }
 

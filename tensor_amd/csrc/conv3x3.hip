@@ -552,20 +552,24 @@ bool conv3x3_halo_plan(const ConvGeom& g, int force_fn, int plan[8]) {
 }
 
 // A launch's time in us (in a row of launches, warm): per tile that a workgroup walks the matrix work and the epilogue of its fragments and
-// the rows that a wave stages, which two workgroups of a compute unit share, and a latency per stage of the channels; bytes out.
-// Fitted to 2200 drawn layers of 3 to 130 us (an early form of pixels, rows and chunks alone was off by over 28 % for one in ten of them and took
-// launches of over 30 us for 14 % shorter than they are, so that they kept layers which the staged rows run in half the time); over 1150
-// others the median error is 6 %, 9 in 10 below 13 %.
+// the rows that a wave stages, which two workgroups of a compute unit share (in the last round only where there are as many), and a
+// latency per stage of the channels; bytes out. Fitted to 2200 drawn layers of 3 to 130 us (a form of pixels, rows and chunks alone was off by
+// over 28 % for one in ten of them and took launches of over 30 us for 14 % shorter than they are, so that they kept layers which the staged
+// rows run in half the time); over 6200 others the median error is 5 %, 9 in 10 below 12 %. (Lines of 2048 bytes take two transfers, the
+// second one short; at 0.9 the layers that the models leave here are those that run well: 64 -> 64 @224x224 b8 24 us, 27 on staged rows.)
 float conv3x3_halo_cost(const ConvGeom& g, float out_mb) {
     HaloPlan p;
     if (!plan_halo(g, 0, &p)) return __builtin_inff();
-    const int mpad = igemm_padded_rows(g.K), cpad = igemm_channel_groups(g.C) * 64, total = g.N * p.tiles_per_img, oct = (g.C + 7) / 8;
+    const int mpad = igemm_padded_rows(g.K), cpad = igemm_channel_groups(g.C) * 64, total = g.N * p.tiles_per_img, oct = g.C / 8;
     int m_blocks, grid_x;
     halo_grid(mpad, mpad > 64 ? 8 : mpad / 16, total, &m_blocks, &grid_x);
-    const float walk = (float)((total + grid_x - 1) / grid_x), share = grid_x * m_blocks > 256 ? 1.64f : 1.f;
-    const float frags = (float)((mpad >= 64 ? 4 : 2) * p.fn), stages = (float)(cpad / p.cb);
-    const float moves = 0.25f * (float)p.r_max * (float)(p.logp == 9 ? (oct + 1) / 2 : p.logp == 10 ? oct : 2 * oct);
-    return 2.44f + walk * (share * (frags * (0.008f * (float)(9 * (cpad / 64)) + 0.0727f) + 0.0775f * moves) + 0.888f * stages) + 0.111f * out_mb;
+    const int full = total / grid_x, rest = total - full * grid_x;
+    const float moves = 0.25f * (float)p.r_max * (p.logp == 9 ? (float)((oct + 1) / 2) : (float)oct * (p.logp == 10 ? 1.f : 0.9f));
+    const float tile = (float)((mpad >= 64 ? 4 : 2) * p.fn) * (0.008f * (float)(9 * (cpad / 64)) + 0.0732f) + 0.0794f * moves;
+    const float stages = 0.892f * (float)(cpad / p.cb), both = 1.73f;
+    float t = 2.42f + (float)full * ((grid_x * m_blocks > 256 ? both : 1.f) * tile + stages) + 0.1084f * out_mb;
+    if (rest > 0) t += (rest * m_blocks > 256 ? both : 1.f) * tile + stages;
+    return t;
 }
 
 hipError_t run_conv3x3_halo(const int8_t* x, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep,

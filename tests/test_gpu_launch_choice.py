@@ -21,6 +21,7 @@ CASES = [
     (336, 184, 3, 1, 1, 1, 13, 13, False, False, (TAP,)),            # 22.7 / 4.5
     (24, 32, 3, 1, 1, 42, 205, 224, True, False, (ROWS,)),           # 107 / 180 / 71
     (56, 40, 3, 1, 1, 7, 123, 123, False, False, (FAMILY,)),         # 8.0 / 11.9 / 8.6
+    (64, 64, 3, 1, 1, 8, 224, 224, False, False, (FAMILY,)),         # 22.4 / 38.7 / 23.4, with the tile that its model names 25.3
     (504, 144, 3, 1, 1, 2, 141, 141, False, False, (ROWS,)),         # 72 / 73 / 45
     (88, 32, 3, 1, 1, 38, 81, 65, False, False, (ROWS,)),            # 17.0 / 24.9 / 12.1
     (232, 224, 3, 1, 1, 2, 132, 132, False, True, (ROWS,)),          # 41 / 43 / 28
