@@ -757,7 +757,7 @@ static bool use_pw_f32in(const otter_hip_conv* h, int in_layout, const ConvGeom&
 // layers of over 4 us that the fits had not seen then take longer than the fastest by 0.9 % on average (2084 without a stride; 44 by over 10 %)
 // and 1.6 % (589 with one; 32); with the halo and implicit-GEMM kernels' models of before, and 5 % to be won by with a stride, 1.4 % (85)
 // and 1.8 % (40). Else the first has to be faster by 5 % (pointwise layers on an fp32 blob with a launch of their own there: 10 %), and
-// on an fp32 blob the second as well where there is a stride (in between it is 6 % slower). An fp32 blob is otherwise quantized by a pass of its own, 2 us and
+// on an fp32 blob the second by 10 % where there is a stride and it is the first that it would replace (in between it is 4 % slower). An fp32 blob is otherwise quantized by a pass of its own, 2 us and
 // 0.65 us per million values (0.85 beyond 50 million), in front of whichever int8 kernel is faster (strided pointwise layers, 32 -> 56
 // on three 24x24 images: 5.9 us with that pass, 3.7 without). Over 2000 drawn layers that the fits had not seen,
 // each on an int8 and on an fp32 blob, the choice takes 53 % of the time of the families' launches alone (k x k; pointwise 88 and
@@ -789,7 +789,8 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
         other = pass + (tap_t < 0.95f * (pass + fminf(other, least)) ? other : fminf(other, rows_cost(false, other, &unused)));
     }
     const float best = tap_t < (own ? 0.9f : f32in || !kxk ? 0.95f : 1.f) * other ? tap_t : other;
-    if (rows_cost(f32in, best, &rows_tile) < (f32in && g.sw > 1 ? 0.95f : 1.f) * best) return *config = rows_tile, ALT_ROWS;
+    const float most = f32in && g.sw > 1 && best < other ? 0.9f : 1.f;
+    if (rows_cost(f32in, best, &rows_tile) < most * best) return *config = rows_tile, ALT_ROWS;
     return *config = tap_tile, best < other ? ALT_TAP : ALT_NONE;
 }
 

@@ -523,9 +523,10 @@ namespace {
 // a graph of launches, warm) for int8 and fp32 input. A workgroup's chain is step * steps + stage * stages, and a compute unit
 // runs as many of them one after the other as its workgroups do not fit side by side; per workgroup of the busiest compute unit
 // comes what they share: steps, staged places (pixel pairs of a thread) and row blocks; per launch the megabytes in and out. With
-// a stride the lanes of a pixel read lie on every other 8 bytes, and a step costs 1 + strided of what it does else. Fitted to 4700
-// drawn layers (k 3 and 5, 8..512 channels, up to 2.5 million pixels): median error 4 to 5 %, 9 in 10 below 11 to 13 % from int8 and
-// 15 to 17 % from fp32. The tile it chooses takes 0.7 % more than the fastest of the four on average, one in twenty 6 % or more.
+// a stride the lanes of a pixel read lie on every other 8 bytes, and a step costs 1 + strided of what it does else. Fitted to drawn layers (k 3
+// and 5, 8..512 channels, up to 2.5 million pixels), from int8 4700 of them: median error 4 to 5 %, 9 in 10 below 11 to 13 %; from fp32 2600:
+// 6 %, 9 in 10 below 18 to 24 % without a stride, 8 % and 34 to 40 % with one. The tile it chooses takes 0.6 % (0.5 %) more than the
+// fastest of the four on average, one in seventy 10 % or more.
 struct RowsCoef {
     float start, step, stage, cu_step, cu_place, cu_block, strided, in_mb, out_mb;
 };
@@ -538,10 +539,10 @@ struct RowsConfig {
     RowsCost i8, f32;
 };
 constexpr RowsConfig kRowsConfigs[] = {
-    {2, 2, {6, {3.02f, 0.062f, 0.813f, 0.05f, 0.033f, 0.186f, 0.397f, 0.057f, 0.113f}}, {5, {2.65f, 0.1f, 1.21f, 0.035f, 0.143f, 0.143f, 0.897f, 0.067f, 0.124f}}},
-    {2, 4, {5, {3.21f, 0.106f, 0.818f, 0.055f, 0.045f, 0.38f, 0.504f, 0.057f, 0.12f}}, {4, {2.94f, 0.171f, 0.983f, 0.f, 0.212f, 0.439f, 0.613f, 0.066f, 0.125f}}},
-    {4, 2, {4, {3.09f, 0.067f, 0.811f, 0.094f, 0.034f, 0.271f, 0.279f, 0.032f, 0.138f}}, {4, {2.81f, 0.109f, 1.19f, 0.076f, 0.141f, 0.113f, 0.686f, 0.062f, 0.16f}}},
-    {4, 4, {3, {3.39f, 0.145f, 0.806f, 0.085f, 0.048f, 0.573f, 0.346f, 0.054f, 0.154f}}, {3, {3.06f, 0.249f, 1.14f, 0.f, 0.231f, 0.505f, 0.51f, 0.062f, 0.17f}}},
+    {2, 2, {6, {3.02f, 0.062f, 0.813f, 0.05f, 0.033f, 0.186f, 0.397f, 0.057f, 0.113f}}, {5, {2.42f, 0.099f, 1.33f, 0.041f, 0.108f, 0.123f, 0.964f, 0.067f, 0.102f}}},
+    {2, 4, {5, {3.21f, 0.106f, 0.818f, 0.055f, 0.045f, 0.38f, 0.504f, 0.057f, 0.12f}}, {4, {2.75f, 0.176f, 1.19f, 0.038f, 0.141f, 0.287f, 0.708f, 0.073f, 0.111f}}},
+    {4, 2, {4, {3.09f, 0.067f, 0.811f, 0.094f, 0.034f, 0.271f, 0.279f, 0.032f, 0.138f}}, {4, {2.61f, 0.114f, 1.28f, 0.079f, 0.106f, 0.124f, 0.768f, 0.058f, 0.143f}}},
+    {4, 4, {3, {3.39f, 0.145f, 0.806f, 0.085f, 0.048f, 0.573f, 0.346f, 0.054f, 0.154f}}, {3, {2.85f, 0.246f, 1.39f, 0.056f, 0.145f, 0.335f, 0.637f, 0.065f, 0.154f}}},
 };
 constexpr int kRowsConfigCount = (int)(sizeof(kRowsConfigs) / sizeof(kRowsConfigs[0]));
 }  // namespace
