@@ -2180,11 +2180,11 @@ void Net::plan_fused_quantize() const {
         if (blobs_[b].consumers.size() != 1) continue;
         pool_units_[(int)pi] = ci;
     }
-    // Pairs of pointwise layers, one reading the other's int8 result alone
+    // Pairs of pointwise layers, one reading the other's int8 result alone. (Not a program's own kind of convolution: its forward may do more.)
     auto sole_reader = [&](int blob) { return blobs_[blob].consumers.size() == 1 ? blobs_[blob].consumers[0] : -1; };
     auto pair_layer = [&](int li) {
         const auto* c = dynamic_cast<const ConvolutionLayer*>(layers_[li]);
-        return c && c->int8_scale_term && c->groups == 1 && c->kernel_height == 1 && c->kernel_width == 1 && c->stride_height == 1 &&
+        return c && c->of_library && c->int8_scale_term && c->groups == 1 && c->kernel_height == 1 && c->kernel_width == 1 && c->stride_height == 1 &&
                c->stride_width == 1 && c->padding_height == 0 && c->padding_width == 0 && c->bottoms.size() == 1 && c->tops.size() == 1 &&
                c->force_out_layout < 0 && c->in_channels % 8 == 0;
     };

@@ -177,3 +177,24 @@ for tail in (next_unit, another_pointwise):  # not one of those that the program
     assert n >= 0 and fake.fake_expr(C.c_long(n)).decode() in (g.expr["u_hi"], "q(%s)" % g.expr["u_hi"]), n
     g.net.close()
 """, program=True)
+
+
+def test_a_convolution_of_the_program_runs_its_own_forward(tmp_path):
+    """Two pointwise layers that would be a pair, of a class that the program has put in the place of the library's."""
+    run(tmp_path, r"""
+program = C.CDLL(sys.argv[2])
+for own in (0, 1):
+    if own:
+        program.program_register(1)
+    g = Graph()
+    out = g.conv(3, g.conv(2, g.conv(1, "data", True, dw=True), True))
+    g.ready()
+    s = g.net.session("data", blob(), out)
+    pairs = fake.fake_count(b"pair")
+    s.run()
+    twice = lambda e: "sum(%s,%s)" % (e, e) if own else e
+    assert fetched(s) == twice("c3(%s)" % twice("c2(%s)" % twice("c1(x)"))), fetched(s)
+    assert fake.fake_count(b"pair") - pairs == (not own)
+    s.close()
+    g.net.close()
+""", program=True)
