@@ -450,9 +450,9 @@ private:
     std::vector<Tensor> blob_tensors_;
 };
 
-// Passes of a net that are asked for again and again on inputs of the same shapes: from the third on their launches are recorded
-// once and replayed as a whole. A launch by itself costs the host 3 to 4 us and the GPU 2.5 us of its own, one of a recording 0.2
-// and 1.8. A recording has blobs and inputs of its own, keeps no data from one pass to the next, and is made again when the net or
+// Passes of a net that are asked for again and again on inputs of the same shapes, as the C facade's sessions and evals do (an Extractor
+// does not: its blobs are the caller's): the launches of the third are recorded, and replayed as a whole from then on. A launch by itself
+// costs the host 3 to 4 us and the GPU 2.5 us of its own, one of a recording 0.2 and 1.8. A recording has blobs and inputs of its own, keeps no data from one pass to the next, and is made again when the net or
 // a setting that chooses launches has changed. Everything runs on the null stream, as other passes do.
 class RecordedPasses {
 public:
