@@ -781,7 +781,7 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
     const float tap_t = tap ? conv_tap_cost(g, f32in, ob, &tap_tile) : __builtin_inff();
     // (without a launch of its own on fp32: k x k, strided or padded)
     const bool own = f32in && (family == 6 || use_igemm_f32in(h, OTTER_HIP_F32_P8, g, ep));
-    float other = conv_family_cost(g, family, own, ob);
+    float other = conv_family_cost(g, family, own, ob, tap_t);
     if (f32in && !own) {
         const float millions = (float)g.N * g.C * g.H * g.W * 1e-6f, pass = 2.f + 0.65f * millions + 0.2f * fmaxf(0.f, millions - 50.f);
         // (the launches behind the pass are only looked at where they could still be faster than the one without it; 2.2: none costs less)

@@ -557,15 +557,19 @@ bool conv3x3_halo_plan(const ConvGeom& g, int force_fn, int plan[8]) {
 // over 28 % for one in ten of them and took launches of over 30 us for 14 % shorter than they are, so that they kept layers which the staged
 // rows run in half the time); over 6200 others the median error is 5 %, 9 in 10 below 12 %. (Lines of 2048 bytes take two transfers, the
 // second one short; at 0.9 the layers that the models leave here are those that run well: 64 -> 64 @224x224 b8 24 us, 27 on staged rows.)
-float conv3x3_halo_cost(const ConvGeom& g, float out_mb) {
+// A launch that takes longer than `other` may be given a shorter time, which is longer than `other` still.
+float conv3x3_halo_cost(const ConvGeom& g, float out_mb, float other) {
+    // one tile of the smallest size, nothing staged: where that is longer than `other`, the plan (0.1 us of host time) is not asked for
+    const float step = 0.008f * (float)(9 * igemm_channel_groups(g.C)) + 0.0732f, least = 3.31f + (g.K > 32 ? 16.f : 8.f) * step;
     HaloPlan p;
+    if (least > other) return least;
     if (!plan_halo(g, 0, &p)) return __builtin_inff();
     const int mpad = igemm_padded_rows(g.K), cpad = igemm_channel_groups(g.C) * 64, total = g.N * p.tiles_per_img, oct = g.C / 8;
     int m_blocks, grid_x;
     halo_grid(mpad, mpad > 64 ? 8 : mpad / 16, total, &m_blocks, &grid_x);
     const int full = total / grid_x, rest = total - full * grid_x;
     const float moves = 0.25f * (float)p.r_max * (p.logp == 9 ? (float)((oct + 1) / 2) : (float)oct * (p.logp == 10 ? 1.f : 0.9f));
-    const float tile = (float)((mpad >= 64 ? 4 : 2) * p.fn) * (0.008f * (float)(9 * (cpad / 64)) + 0.0732f) + 0.0794f * moves;
+    const float tile = (float)((mpad >= 64 ? 4 : 2) * p.fn) * step + 0.0794f * moves;
     const float stages = 0.892f * (float)(cpad / p.cb), both = 1.73f;
     float t = 2.42f + (float)full * ((grid_x * m_blocks > 256 ? both : 1.f) * tile + stages) + 0.1084f * out_mb;
     if (rest > 0) t += (rest * m_blocks > 256 ? both : 1.f) * tile + stages;

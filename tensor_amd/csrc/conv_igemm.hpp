@@ -25,7 +25,7 @@ size_t tap_grouped_weight_bytes(int K, int C, int groups, int kh, int kw);
 void tap_pack_weights_grouped(const int8_t* w, int K, int C, int groups, int kh, int kw, int8_t* dst);
 bool conv_tap_supported(const ConvGeom& g, const Epilogue& ep, bool f32in);
 float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config);
-float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes);
+float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes, float other);
 hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep, int config,
                         const float* in_scale, int in_round_mode, hipStream_t stream);
 
@@ -77,7 +77,7 @@ hipError_t run_conv_block(const int8_t* x, const int8_t* w_exp, const int32_t* k
 
 // conv3x3.hip
 bool conv3x3_halo_supported(const ConvGeom& g, const Epilogue& ep);
-float conv3x3_halo_cost(const ConvGeom& g, float out_mb);
+float conv3x3_halo_cost(const ConvGeom& g, float out_mb, float other);
 bool conv3x3_halo_plan(const ConvGeom& g, int force_fn, int plan[8]);
 hipError_t run_conv3x3_halo(const int8_t* x, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep,
                             int force_fn, hipStream_t stream);

@@ -565,8 +565,8 @@ float conv_rows_cost(const ConvGeom& g_in, bool f32in, int out_bytes, int* confi
         if (!fits) continue;
         const int blocks = (ra.g.K + 16 * c.fm - 1) / (16 * c.fm), bpw = rows_blocks_per_workgroup(ra, blocks, c.fm);
         const int pairs = ra.rows_max * ra.VW2, oct = (ra.g.C / 8 + ra.stages - 1) / ra.stages;
-        const int parts = 1 << rows_parts_shift(pairs), part = 256 / parts;
-        const float places = (float)(ra.stages * oct * ((pairs + part - 1) / part)) / (float)parts;
+        const int shift = rows_parts_shift(pairs);
+        const float places = (float)(ra.stages * oct * ((pairs + (256 >> shift) - 1) >> (8 - shift))) * (shift == 0 ? 1.f : shift == 1 ? 0.5f : shift == 2 ? 0.25f : 0.125f);
         const int slices = (blocks + bpw - 1) / bpw;
         const int wgs = (int)std::min(((long)ra.n_tiles * slices * ra.g.groups + 255) / 256, 1l << 24);
         const RowsCost& cost = f32in ? c.f32 : c.i8;

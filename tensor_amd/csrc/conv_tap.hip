@@ -458,8 +458,8 @@ float conv_tap_cost(const ConvGeom& g, bool f32in, int out_bytes, int* config) {
 // Start + chain * chunks + matrix work + epilogue + bytes in + bytes out, fitted to drawn layers; median error 4 to 11 % (k x k layers of
 // the implicit-GEMM kernel 6 %, 13 % on the slow side before its index divisions became multiplications). The fp32
 // pointwise kernel walks all output channels per workgroup of 64 pixels, so that its chain grows with them (128 -> 1280 on one
-// 29x29 image: 15.6 us, where the kernel above takes 5.8).
-float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes) {
+// 29x29 image: 15.6 us, where the kernel above takes 5.8). other: what it is compared with (conv3x3_halo_cost).
+float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes, float other) {
     const int C = g.C / g.groups, K = g.K / g.groups, taps = g.kh * g.kw, tp = g.groups > 1 ? igemm_tap_pack(C, g.kh, g.kw) : 1;
     const float chunks = tp > 1 ? (float)((taps + tp - 1) / tp) : (float)(taps * igemm_channel_groups(C));
     const float px = (float)g.N * g.OH * g.OW * g.groups, rows = K <= 32 ? 32.f : (float)((K + 63) / 64 * 64);
@@ -469,7 +469,7 @@ float conv_family_cost(const ConvGeom& g, int family, bool f32in, int out_bytes)
         const float cu = ceilf((float)g.N * (float)((g.H * g.W + 63) / 64) / 256), k = 0.01f * (float)K;
         return 2.18f + 0.5f * cu + 0.2f * chunks + k * (0.336f + 0.333f * cu + chunks * (0.063f + 0.096f * cu)) + 0.39f * in_mb + 0.048f * out_mb;
     }
-    if (family == 3) return conv3x3_halo_cost(g, out_mb);
+    if (family == 3) return conv3x3_halo_cost(g, out_mb, other);
     if (taps > 1) return 2.93f + 0.308f * chunks + 59.7f * mac + 30.2f * epi + px * (3.43e-6f + 1.121e-6f * chunks) + 0.095f * in_mb + 0.065f * out_mb;
     if (f32in) return 2.37f + 0.50f * chunks + 201.f * mac + 18.f * epi + 0.33f * in_mb + 0.09f * out_mb;
     return 2.46f + 0.34f * chunks + 94.f * mac + 26.f * epi + 0.03f * in_mb + 0.07f * out_mb;
