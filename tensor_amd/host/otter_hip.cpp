@@ -2064,7 +2064,8 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
         }
     }
     {
-        const int rc = forward_inputs(li, layer->bottoms, blobs, opt);
+        const int* const b = layer->bottoms.data();
+        const int rc = forward_inputs(li, b, b + layer->bottoms.size(), blobs, opt);
         if (rc) return rc < 0 ? rc : 0;
     }
     if (layer->type() == "Input") return blobs[layer->tops[0]].defined() ? 0 : -1;
@@ -2094,11 +2095,12 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
     return 0;
 }
 
-// Makes those of the blobs `needed` that are not there, for a launch of layer li (or of several, li the first). Returns 1 when the
+// Makes those of the blobs first .. last that are not there, for a launch of layer li (or of several, li the first). Returns 1 when the
 // layer's own result came to be on the way, as the second layer of a pair does (forward_pair_unit): its input may then be missing for
 // good, and the caller goes on layer by layer.
-int Net::forward_inputs(int li, const std::vector<int>& needed, std::vector<Tensor>& blobs, const NetOption& opt) const {
-    for (int b : needed) {
+int Net::forward_inputs(int li, const int* first, const int* last, std::vector<Tensor>& blobs, const NetOption& opt) const {
+    for (; first != last; ++first) {
+        const int b = *first;
         if (b < 0 || blobs[b].defined()) continue;
         const int rc = forward_layer(blobs_[b].producer, blobs, opt);
         if (rc) return rc;
@@ -2651,9 +2653,10 @@ RecordedPasses::Lease::~Lease() {
 //   141       3x3                        3 0.96, 49 1.02, 195 1.03, 391 1.06
 // A host that waits for every pass also waits for its first launches: 7 calls 5 0.71, 333 0.93, 667 1.03; 9 502 1.06; 13 486 0.80, 973 0.91;
 // 27 334 0.79, 668 0.93, 1336 0.97, 2308 0.99; 43 1848 0.97; 103 368 1.01, 737 0.99, 1546 1.00.
+// On a slower host (4.6 us a launch) 96 calls of 1546 KB 0.92 to 0.93: long passes, which lose least, are given the benefit.
 static bool worth_recording(long launches, size_t bytes, bool waited_for) {
     if (waited_for) return bytes <= (size_t)launches * std::min<size_t>((size_t)launches * 50 << 10, 1536 << 10);
-    return launches > 10 && bytes <= (size_t)(launches - 10) << 20;
+    return launches > 10 && bytes <= (size_t)(launches - 10 + 2 * std::max(0l, launches - 60)) << 20;
 }
 
 RecordedPasses::Lease RecordedPasses::lease(const Net& net, const std::string& key, bool waited_for, const std::function<std::vector<Tensor>()>& make_inputs,

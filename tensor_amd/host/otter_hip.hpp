@@ -13,6 +13,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <functional>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -394,7 +395,10 @@ private:
     mutable std::map<int, ShuffleUnit> shuffle_units_;
     // pointwise layers that alone read another one's int8 result: the reader's index -> the other's
     mutable std::map<int, int> pair_units_;
-    int forward_inputs(int li, const std::vector<int>& needed, std::vector<Tensor>& blobs, const NetOption& opt) const;
+    int forward_inputs(int li, const int* first, const int* last, std::vector<Tensor>& blobs, const NetOption& opt) const;
+    int forward_inputs(int li, std::initializer_list<int> needed, std::vector<Tensor>& blobs, const NetOption& opt) const {
+        return forward_inputs(li, needed.begin(), needed.end(), blobs, opt);
+    }
     int forward_pair_unit(int first, int second, const ShuffleUnit* u, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int block_saves_launches(int conv, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, const NetOption& opt) const;
