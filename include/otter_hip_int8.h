@@ -255,6 +255,35 @@ int otter_hip_conv_pair_launches(const otter_hip_conv_t* first, const otter_hip_
 int otter_hip_conv_pair_forward(const otter_hip_conv_t* first, const otter_hip_conv_t* second, const void* in, int n, int in_h, int in_w,
                                 const otter_hip_conv_tail* tail, void* out, int out_layout, void* stream);
 
+/* A depthwise int8 -> int8 layer and the pointwise layer that alone reads its result in one launch, and with `next` the pointwise layer
+ * behind that as well. The results are those of the layers (and of the calls above for what their ends carry) one by one. What becomes of
+ * the first pointwise layer's result; all zero: it goes to out (Byte8 or Float4, out_layout; K % 4 == 0):
+ *   next                 reads its int8 result, or the quantize_to_int8 (q_scale, q_round_mode) of its fp32 one after what follows here;
+ *                        out and out_layout are then next's, and the fp32 result goes to sum (Float4) unless that is NULL
+ *   residual             Float4 addend of an fp32 result (otter_hip_conv_forward_residual); with residual1 the addend's first
+ *                        part0_channels channels, residual1 the rest, each Float4 or Float8 (otter_hip_conv_forward_residual_concat; no next)
+ *   out_q                the Byte8 quantization of the fp32 result beside it (no next); out may then be NULL
+ *   other, ...           the shuffle of otter_hip_conv_forward_shuffle; out is not used without next, which reads the second half
+ * in: Byte8. otter_hip_conv_dwpw_launches: 1 where the call runs and is the faster way, 2 where the layers are separate calls or
+ * faster so; of the pointers, next apart, it only asks which are null. The call itself runs wherever it can. */
+typedef struct otter_hip_conv_end {
+    const otter_hip_conv_t* next;
+    const float *residual, *residual1;
+    int part0_channels, part0_layout, part1_layout;
+    const float* other;
+    int other_layout, other_odd, joined;
+    float *first_half, *second_half;
+    int8_t *first_half_q, *second_half_q;
+    float* sum;
+    int8_t* out_q;
+    float q_scale;
+    int q_round_mode;
+} otter_hip_conv_end;
+int otter_hip_conv_dwpw_launches(const otter_hip_conv_t* depthwise, const otter_hip_conv_t* pointwise, int n, int in_h, int in_w,
+                                 const otter_hip_conv_end* end, int out_layout);
+int otter_hip_conv_dwpw_forward(const otter_hip_conv_t* depthwise, const otter_hip_conv_t* pointwise, const void* in, int n, int in_h,
+                                int in_w, const otter_hip_conv_end* end, void* out, int out_layout, void* stream);
+
 /* A chain of layers that each map an int8 Byte8 blob to an int8 Byte8 blob (consecutive Convolution layers of a
  * Net, Tensor/Net.cpp:413-505 runs them one after the other): out = layer[n-1](... layer[0](in)). The result is what
  * n calls of otter_hip_conv_forward give. The intermediate blobs live in `workspace`
@@ -388,7 +417,8 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * tn = 0..3 its tile. tm == -10 on a pointwise layer with an int8 blob: the launch that keeps its operands in registers wherever it
  * can run, tn = groups | split << 6 | pairs << 7 forcing the 16-pixel groups a wave owns (1, 2 or 4), whether the reduction is split
  * among the waves of a workgroup (1: over 64 input channels; 0: at most 256, and four groups only for a result without a sum, a twin
- * or a shuffle) and the pairs of 16 output channels a wave walks. tn = 0: all three automatic. */
+ * or a shuffle) and the pairs of 16 output channels a wave walks. tn = 0: all three automatic. tm == -12 on a depthwise layer:
+ * otter_hip_conv_dwpw_launches says 1 wherever that launch can run, tn = 1, 2, 4 or 8 its groups of 16 pixels (0 = automatic). */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 
 /* Test hook with no counterpart in the reference: which of the launches of its family a dense or grouped layer takes on a packed

@@ -87,6 +87,7 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
            "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
            "otter_hip_conv_forward_residual_concat", "otter_hip_conv_pair_launches", "otter_hip_conv_pair_forward",
+           "otter_hip_conv_dwpw_launches", "otter_hip_conv_dwpw_forward",
            "otter_hip_record_begin", "otter_hip_record_end", "otter_hip_record_launch", "otter_hip_record_destroy"]
 
 
@@ -112,6 +113,15 @@ def load_binding():
 class Tail(C.Structure):
     """otter_hip_conv_tail: what otter_hip_conv_pair_forward does with the first layer's result."""
     _fields_ = [("other", C.c_void_p), ("other_layout", C.c_int), ("other_odd", C.c_int), ("first_half", C.c_void_p),
+                ("q_scale", C.c_float), ("q_round_mode", C.c_int)]
+
+
+class End(C.Structure):
+    """otter_hip_conv_end: what otter_hip_conv_dwpw_forward does with the pointwise layer's result."""
+    _fields_ = [("next", C.c_void_p), ("residual", C.c_void_p), ("residual1", C.c_void_p), ("part0_channels", C.c_int),
+                ("part0_layout", C.c_int), ("part1_layout", C.c_int), ("other", C.c_void_p), ("other_layout", C.c_int),
+                ("other_odd", C.c_int), ("joined", C.c_int), ("first_half", C.c_void_p), ("second_half", C.c_void_p),
+                ("first_half_q", C.c_void_p), ("second_half_q", C.c_void_p), ("sum", C.c_void_p), ("out_q", C.c_void_p),
                 ("q_scale", C.c_float), ("q_round_mode", C.c_int)]
 
 
@@ -338,6 +348,27 @@ class Library:
         out = self.empty(n * second.K * h * w, layout_dtype(layout))
         self._check(self.lib.otter_hip_conv_pair_forward(first.h, second.h, self.ptr(x), n, h, w, C.byref(self._tail(tail)), self.ptr(out),
                                                          layout, self.stream()))
+        return out
+
+    def _end(self, end):
+        return End(**{k: v.h if k == "next" else self.ptr(v) if hasattr(v, "data_ptr") else v for k, v in end.items() if v is not None})
+
+    def conv_dwpw_launches(self, dw, pw, n, h, w, **end):
+        """otter_hip_conv_dwpw_launches: 1 where conv_dwpw runs the layers as one launch, else 2."""
+        last = end.get("next") or pw
+        r = self.lib.otter_hip_conv_dwpw_launches(dw.h, pw.h, n, h, w, C.byref(self._end(end)), self._packed_out(last))
+        self._check(min(r, 0))
+        return r
+
+    def conv_dwpw(self, dw, pw, x, n, h, w, wants_out=True, **end):
+        """otter_hip_conv_dwpw_forward: x (int8 Byte8) through a depthwise layer, the pointwise layer behind it and end["next"]; `end` holds
+        the fields of End, tensors for its pointers. Returns the last layer's result (None without wants_out)."""
+        last = end.get("next") or pw
+        layout = self._packed_out(last)
+        oh, ow = dw.out_hw(h, w)
+        out = self.empty(n * last.K * oh * ow, layout_dtype(layout)) if wants_out else None
+        self._check(self.lib.otter_hip_conv_dwpw_forward(dw.h, pw.h, self.ptr(x), n, h, w, C.byref(self._end(end)),
+                                                         self.ptr(out) if wants_out else None, layout, self.stream()))
         return out
 
     @staticmethod

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "conv_dwpw.hpp"
 #include "conv_igemm.hpp"
 
 using namespace ohip;
@@ -99,6 +100,7 @@ struct otter_hip_conv {
     int8_t* w_stem = nullptr;    // MFMA lane order of the few-channel 3x3 kernel (C <= 5, K <= 64)
     int32_t* w_dw = nullptr;     // dot4 weight words          (depthwise, C % 8 == 0)
     int8_t* w_dw_mfma = nullptr; // block-diagonal MFMA operands (depthwise 3x3, C % 8 == 0)
+    int8_t* w_dwpw = nullptr;    // a byte per lane and tap of a depthwise 3x3 / 5x5 layer for the launch it shares with its pointwise reader
     int8_t* w_xdw = nullptr;     // MFMA operands of a pointwise int8 -> int8 layer for the launch it shares with its depthwise reader
     int32_t* blk_consts = nullptr; // the layer's constants (and depthwise 3x3 weights) as the fused block launch keeps them in LDS
     bool so_positive = true;     // every output scale is finite and > 0
@@ -471,6 +473,7 @@ int otter_hip_conv_destroy(otter_hip_conv_t* h) {
     (void)hipFree(h->w_stem);
     (void)hipFree(h->w_dw);
     (void)hipFree(h->w_dw_mfma);
+    (void)hipFree(h->w_dwpw);
     (void)hipFree(h->w_xdw);
     (void)hipFree(h->blk_consts);
     (void)hipFree(h->scale_in);
@@ -569,7 +572,11 @@ int otter_hip_conv_create(const otter_hip_conv_desc* desc, const int8_t* weight,
                 dw_mfma_pack_weights(weight, C, d.stride_w, d.pad_w, d.kernel_w, wa.data());
                 if ((rc = upload<int8_t>(&h->w_dw_mfma, wa.data(), wa.size(), wa.size(), 0))) break;
             }
-
+            if (d.out_kind == OTTER_HIP_OUT_I8 && d.kernel_h == d.kernel_w && (d.kernel_h == 3 || d.kernel_h == 5)) {
+                std::vector<int8_t> wd(dwpw_weight_bytes(C, d.kernel_w));
+                dwpw_pack_weights(weight, C, d.kernel_w, wd.data());
+                if ((rc = upload<int8_t>(&h->w_dwpw, wd.data(), wd.size(), wd.size(), 0))) break;
+            }
         } else if (g == 1 && C % 8 == 0) {
             std::vector<int8_t> wp(igemm_packed_weight_bytes(K, C, d.kernel_h, d.kernel_w));
             igemm_pack_weights(weight, K, C, d.kernel_h, d.kernel_w, wp.data());
@@ -1834,6 +1841,112 @@ int otter_hip_conv_pair_forward(const otter_hip_conv_t* first, const otter_hip_c
     const float so[2] = {first->so_one, second->so_one};
     OHIP_CHECK(run_conv_pwpw((const int8_t*)in, w, so, out, a.g[0], a.ep[0], a.g[1], a.ep[1],
                              first->force_tm == -11 ? first->force_tn : 0, (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
+// ---- a depthwise layer and the pointwise layers behind it -----------------------------------------------------------------------
+
+struct DwPwCall {
+    ConvGeom g[3];  // depthwise, pointwise, next
+    Epilogue ep[3];
+    JoinArgs ja;
+    bool next = false;
+};
+
+// the layers and what becomes of their results as one launch has them; an error code for what no call may ask for
+static int dwpw_args(const char* who, const otter_hip_conv_t* d, const otter_hip_conv_t* p, int n, int in_h, int in_w,
+                     const otter_hip_conv_end* t, int out_layout, DwPwCall* a) {
+    auto bad = [&](const char* what) { return fail(OTTER_HIP_ERR_INVALID, std::string(who) + ": " + what); };
+    if (!d || !p || !t) return bad("null");
+    if (n < 0 || in_h < 1 || in_w < 1) return bad("bad shape");
+    if (!d->depthwise || d->d.out_kind != OTTER_HIP_OUT_I8 || p->d.in_channels != d->d.out_channels) return bad("a depthwise layer with an int8 result that the other reads expected");
+    const otter_hip_conv_t *const nx = t->next, *const last = nx ? nx : p;
+    if (p->d.out_kind == OTTER_HIP_OUT_I32 || last->d.out_kind == OTTER_HIP_OUT_I32) return bad("int8 or fp32 results expected");
+    const bool f32 = p->d.out_kind == OTTER_HIP_OUT_F32, quantizes = f32 && (nx || t->out_q || t->first_half_q || t->second_half_q);
+    const int K = p->d.out_channels;
+    if (nx && (nx->d.in_channels != K || K % 8)) return bad("the last layer reads whole channel octets of the pointwise one's result");
+    if (!valid_layout(out_layout) || layout_elem(out_layout) != (last->d.out_kind == OTTER_HIP_OUT_F32 ? 0 : 1) || last->d.out_channels % layout_pack(out_layout))
+        return bad("output layout does not match the last layer");
+    if (!f32 && (t->residual || t->other || t->out_q || t->sum)) return bad("sums, shuffles and twins are of fp32 results");
+    if (quantizes && t->q_round_mode != OTTER_HIP_ROUND_SSE && t->q_round_mode != OTTER_HIP_ROUND_EXACT) return bad("unknown rounding mode");
+    if ((t->out_q || t->other) && K % 8) return bad("whole channel octets expected");
+    if (t->residual1) {
+        if (!t->residual || nx) return bad("an addend in two parts has both, and no layer behind it");
+        for (int l : {t->part0_layout, t->part1_layout})
+            if (l != OTTER_HIP_F32_P4 && l != OTTER_HIP_F32_P8) return bad("the parts must be Float4 or Float8");
+        if (K % 8 || t->part0_channels < 8 || t->part0_channels % 8 || t->part0_channels >= K) return bad("parts of whole channel octets expected");
+    }
+    if (t->other) {
+        if (t->residual || t->out_q || t->sum) return bad("a shuffle has no sum");
+        if (t->other_layout != OTTER_HIP_F32_P4 && t->other_layout != OTTER_HIP_F32_P8) return bad("the other blob must be Float4 or Float8");
+        if ((t->joined || nx) && (t->second_half || t->second_half_q)) return bad("the second half is not a blob here");
+        if (nx && (t->joined || !t->first_half || t->first_half_q)) return bad("in front of a layer the shuffle leaves its first half");
+    }
+    if (nx && t->out_q) return bad("the quantized result is the next layer's");
+    if (!nx && t->sum) return bad("the result goes to out");
+    a->next = nx != nullptr;
+    a->g[0] = make_geom(d->d, n, in_h, in_w);
+    if (a->g[0].OH < 1 || a->g[0].OW < 1) return bad("empty output");
+    a->g[1] = make_geom(p->d, n, a->g[0].OH, a->g[0].OW);
+    if (a->g[1].OH < 1 || a->g[1].OW < 1) return bad("empty output");
+    if (nx) {
+        a->g[2] = make_geom(nx->d, n, a->g[1].OH, a->g[1].OW);
+        if (a->g[2].OH < 1 || a->g[2].OW < 1) return bad("empty output");
+    }
+    a->ep[0] = make_epilogue(d, OTTER_HIP_I8_P8);
+    a->ep[1] = make_epilogue(p, !nx ? out_layout : f32 ? OTTER_HIP_F32_P4 : OTTER_HIP_I8_P8);
+    if (nx) a->ep[2] = make_epilogue(nx, out_layout);
+    Epilogue& ep = a->ep[1];
+    ep.twin_scale = t->q_scale, ep.twin_half = t->q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+    ep.residual = t->residual, ep.twin = t->out_q;
+    if (t->residual1) {
+        ep.join = &a->ja;
+        a->ja.residual1 = t->residual1, a->ja.res_split = t->part0_channels;
+        a->ja.res_pack0 = layout_pack(t->part0_layout), a->ja.res_pack1 = layout_pack(t->part1_layout);
+    }
+    if (t->other) {
+        const size_t half = (size_t)K * a->g[1].OH * a->g[1].OW;  // elements of one half of one image
+        ep.join = &a->ja;
+        a->ja.other = t->other, a->ja.other_pack = layout_pack(t->other_layout), a->ja.other_odd = t->other_odd != 0;
+        a->ja.sh_image = t->joined ? 2 * half : half;
+        a->ja.sh_out0 = t->first_half, a->ja.sh_q0 = t->first_half_q;
+        a->ja.sh_out1 = t->joined ? (t->first_half ? t->first_half + half : nullptr) : t->second_half;
+        a->ja.sh_q1 = t->joined ? (t->first_half_q ? t->first_half_q + half : nullptr) : t->second_half_q;
+    }
+    return OTTER_HIP_OK;
+}
+
+// whether the launch takes the layers
+static bool dwpw_one_launch(const otter_hip_conv_t* d, const otter_hip_conv_t* p, const otter_hip_conv_t* nx, const DwPwCall& a) {
+    if (!d->w_dwpw || !d->so_same || (d->force_tm != 0 && d->force_tm != -12)) return false;
+    for (const otter_hip_conv_t* h : {p, nx})
+        if (h && (!h->w_igemm || h->c_pad || !h->so_same || h->force_tm != 0)) return false;
+    return conv_dwpw_applicable(a.g[0], a.ep[0], a.g[1], a.ep[1], nx ? &a.g[2] : nullptr, nx ? &a.ep[2] : nullptr);
+}
+
+int otter_hip_conv_dwpw_launches(const otter_hip_conv_t* d, const otter_hip_conv_t* p, int n, int in_h, int in_w,
+                                 const otter_hip_conv_end* end, int out_layout) {
+    DwPwCall a;
+    const int rc = dwpw_args("otter_hip_conv_dwpw_launches", d, p, n, in_h, in_w, end, out_layout, &a);
+    if (rc) return rc;
+    const bool one = dwpw_one_launch(d, p, end->next, a);
+    return one && (d->force_tm == -12 || conv_dwpw_faster(a.g[0], a.g[1], a.ep[1], end->next ? &a.g[2] : nullptr)) ? 1 : 2;
+}
+
+int otter_hip_conv_dwpw_forward(const otter_hip_conv_t* d, const otter_hip_conv_t* p, const void* in, int n, int in_h, int in_w,
+                                const otter_hip_conv_end* end, void* out, int out_layout, void* stream) {
+    DwPwCall a;
+    const int rc = dwpw_args("otter_hip_conv_dwpw_forward", d, p, n, in_h, in_w, end, out_layout, &a);
+    if (rc) return rc;
+    const otter_hip_conv_t* const nx = end->next;
+    if (!in || (!out && (nx || (!end->other && !end->out_q)))) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_dwpw_forward: null");
+    if (!dwpw_one_launch(d, p, nx, a))
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_dwpw_forward: not a single launch (otter_hip_conv_dwpw_launches)");
+    if (n == 0) return OTTER_HIP_OK;
+    const int8_t* const w[2] = {p->w_igemm, nx ? nx->w_igemm : nullptr};
+    const float so[2] = {p->so_one, nx ? nx->so_one : 1.f};
+    OHIP_CHECK(run_conv_dwpw((const int8_t*)in, d->w_dwpw, d->so_one, a.g[0], a.ep[0], w, so, out, end->sum, a.g[1], a.ep[1],
+                             nx ? &a.g[2] : nullptr, nx ? &a.ep[2] : nullptr, d->force_tm == -12 ? d->force_tn : 0, (hipStream_t)stream));
     return OTTER_HIP_OK;
 }
 

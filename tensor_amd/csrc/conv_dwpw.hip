@@ -1,0 +1,541 @@
+// A depthwise k x k layer and the pointwise layer that alone reads its int8 result in one launch, and with them the pointwise layer that
+// reads the int8 form of what the first leaves behind, where there is one (conv_pwpw.hip's pair, across a residual sum as well).
+//
+// What bounds these layers one by one is not bytes and not operations: a launch takes 2 us behind the one in front of it, then a chain of
+// memory latencies, and the blob between the layers is written and read back for nothing. Here a workgroup of eight waves owns 16 G
+// pixels (G = 1, 2, 4, 8 groups of 16, a wave belongs to one) with all their channels:
+//  * The depthwise layer goes through the matrix cores, 16 channels x 16 pixels at a time: a B column is one output pixel, its 64
+//    reduction bytes are four taps of two channel octets, and the A operand holds each channel's weights at that channel's bytes and
+//    zeros elsewhere: 3 instructions for a 3x3 window, 7 for 5x5. (conv_dw_mfma.hip puts eight neighbouring pixels of one octet into a
+//    column: half the loads, but runs of four output pixels of a row. Here the pixels are any: no lane idles at the end of a row, and
+//    strides, padding and dilation are in the lanes' addresses.) A tap of a pixel is an 8-byte load; one outside the image is out of
+//    range and zero. The weights come as one byte per lane and tap and are spread out by v_perm_b32: as whole operands they would be as
+//    many bytes as the pixels.
+//  * The bytes go to LDS, a row per pixel, and the pointwise layer's waves take its pairs of 16-row tiles in turn, weights straight
+//    from memory in a ring of four reduction steps that is refilled across pairs and layers: the first ones are requested before the
+//    depthwise layer begins, as are the elements of a residual or of a shuffle's other blob.
+//  * Behind a barrier they do the same for the second pointwise layer.
+#include "conv_dwpw.hpp"
+
+#include "conv_pwpw_common.hpp"
+
+#include <algorithm>
+
+namespace ohip {
+
+namespace {
+
+constexpr int DP_WAVES = 8;
+enum { DP_NONE = 3 };  // no second pointwise layer (KIND1, beside PP_I8, PP_NONNEG and PP_F32)
+
+struct DwPwArgs {
+    PwPwLayer l[2];
+    // the depthwise layer
+    const int8_t* dw_w;
+    const float *dw_scale_in, *dw_bias;
+    float dw_p0, dw_scale, dw_half;
+    unsigned dw_qh, in_bytes;
+    unsigned hw_m, ow_m, total_pix;  // divisions (FastDiv) by the pixels and the columns of an output image
+    int HW, OW, H, W, tiles;         // H, W: of the input
+    int sh, sw, ph, pw, dh, dw, C8;
+    unsigned hw_s, ow_s;
+    int lg, dw_lrelu, dw_nonneg;     // lg: log2 of the pixel groups
+};
+
+// the fp32 blob whose elements an epilogue reads
+template <class A>
+__device__ __forceinline__ const float* add_blob(const A& ja) {
+    if constexpr (std::is_same_v<A, PwShuffle>) return ja.other;
+    else if constexpr (std::is_same_v<A, NoJoin>) return nullptr;
+    else return ja.residual;
+}
+template <class A>
+__device__ __forceinline__ int ja_pack(const A& ja) {
+    if constexpr (std::is_same_v<A, PwShuffle>) return ja.other_pack;
+    else return 4;
+}
+
+}  // namespace
+
+// A operands of the depthwise layer: [pair of octets][lane 64][4 PK bytes], PK = 2 (3x3) or 4 (5x5) dwords; byte 2 m + e of lane
+// (r = lane % 16, g = lane / 16) is channel r's weight of tap 4 m + 2 (g % 2) + e if r is of octet g / 2 of the pair, else zero.
+static int dwpw_dwords(int ks) { return ks == 3 ? 2 : 4; }
+size_t dwpw_weight_bytes(int C, int ks) { return (size_t)((C / 8 + 1) / 2) * 256 * dwpw_dwords(ks); }
+void dwpw_pack_weights(const int8_t* w, int C, int ks, int8_t* dst) {
+    const int taps = ks * ks, row = 4 * dwpw_dwords(ks);
+    std::fill(dst, dst + dwpw_weight_bytes(C, ks), (int8_t)0);
+    for (int op = 0; op < (C / 8 + 1) / 2; ++op)
+        for (int lane = 0; lane < 64; ++lane) {
+            const int r = lane % 16, g = lane / 16, c = 16 * op + r;
+            if (r / 8 != g / 2 || c >= C) continue;
+            for (int k = 0; k < (taps + 3) / 4 * 2; ++k) {
+                const int tap = 4 * (k / 2) + 2 * (g % 2) + k % 2;
+                if (tap < taps) dst[((size_t)op * 64 + lane) * row + k] = w[(size_t)c * taps + tap];
+            }
+        }
+}
+
+// TAPS: 9 or 25. EPI: the first pointwise layer's epilogue: EPI_I8_P8; EPI_F32_P4_FUSED (with or without a residual and a twin; without
+// a second layer this is the plain fp32 result as well), EPI_F32_P4_PARTS, EPI_F32_SHUFFLE. KIND1: the second layer's result or DP_NONE.
+// out: the last layer's result; sum: with a second layer, the first one's fp32 result (null: not wanted).
+template <int TAPS, int EPI, int KIND1>
+__global__ void __launch_bounds__(64 * DP_WAVES) conv_dwpw_kernel(const int8_t* __restrict__ x, void* __restrict__ out, float* __restrict__ sum,
+                                                                  DwPwArgs pa, PwAdd<EPI> ja) {
+    constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, I8 = EPI == EPI_I8_P8, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
+    constexpr bool NEXT = KIND1 != DP_NONE;
+    constexpr int KS = TAPS == 9 ? 3 : 5, M = (TAPS + 3) / 4, PK = TAPS == 9 ? 2 : 4;
+    constexpr int NW = DP_WAVES, SC = 4;
+    extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+    const unsigned tid = threadIdx.x, lane = tid & 63, q = lane >> 4, p = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane((int)tid >> 6);
+    const int xcd = blockIdx.x & 7, tile = (xcd * pa.tiles >> 3) + (int)(blockIdx.x >> 3);  // (grid.x is a multiple of 8)
+    if (tile >= (xcd + 1) * pa.tiles >> 3) return;  // (uniform)
+    const PwPwLayer &l0 = pa.l[0], &l1 = pa.l[1];
+    const unsigned HW = pa.HW, C8 = pa.C8, K0 = l0.K, rb0 = 64u * l0.steps + 16u, rb1 = NEXT ? 64u * l1.steps + 16u : 0u;  // bytes of a pixel's row
+    const int pairs0 = (l0.K + 31) / 32, pairs1 = NEXT ? (l1.K + 31) / 32 : 0;
+    const int PIX = 16 << pa.lg, group = wave & ((1 << pa.lg) - 1), first = wave >> pa.lg, stride = NW >> pa.lg;
+    int8_t *const px0 = lds, *const px1 = lds + PIX * rb0;
+    const unsigned Cd = 16u * ((C8 + 1) / 2);  // channels of the depthwise layer, whole pairs of octets
+    float *const constsd = reinterpret_cast<float*>(px1 + PIX * rb1), *const consts0 = constsd + 2 * Cd, *const consts1 = consts0 + 64 * pairs0;
+
+    // ---- the wave's pixels -----------------------------------------------------------------------------------------------------
+    const unsigned gp = (unsigned)(tile * PIX + 16 * group) + p;
+    const bool ok = gp < pa.total_pix;
+    const unsigned n = div_by(gp, FastDiv{pa.hw_m, pa.hw_s, (unsigned)pa.HW}), pix = gp - n * HW;
+    const unsigned row0 = (16u * group + p) * rb0, row1 = (16u * group + p) * rb1;
+    // byte offset of (image, this lane's channels of a pair, pixel) in a blob of K channels: Byte8, Float4, Float8; a pair is 32 HW
+    // (Byte8) or 128 HW (fp32) bytes further
+    const unsigned outside = ok ? 0u : PR_OOB;
+    auto at_b8 = [&](unsigned K) { return ((n * (K / 8) + q) * HW + pix) * 8u | outside; };
+    auto at_f4 = [&](unsigned K) { return ((n * (K / 4) + 2 * q) * HW + pix) * 16u | outside; };
+    auto at_f8 = [&](unsigned K) { return ((n * (K / 8) + q) * HW + pix) * 32u | outside; };
+
+    // ---- the pointwise weights: four reduction steps of a pair ----------------------------------------------------------------------
+    v4i a[SC][2];
+    // (second: of the second layer. Chosen by values and not by branches: behind a branch a wave waits for the loads in front of it)
+    auto load_a = [&](bool second, int pr, int step0) {  // (steps that do not exist: past the weights, zero)
+        const int steps = second ? l1.steps : l0.steps, mt = second ? l1.mt : l0.mt;
+        const __amdgpu_buffer_rsrc_t rw = rsrc(second ? l1.w : l0.w, (unsigned)steps * (unsigned)mt * 1024u);
+        auto one = [&](int s) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                a[s][h] = load16(rw, (lane * 16 | (step0 + s < steps ? 0u : PR_OOB)) + h * 1024, ((unsigned)(step0 + s) * (unsigned)mt + 2u * pr) * 1024u);
+        };
+        one(0), one(1);
+#pragma unroll
+        for (int s = 2; s < SC; s += 2) {
+            if (step0 + s < steps) one(s), one(s + 1);  // (uniform)
+            else a[s][0] = a[s][1] = a[s + 1][0] = a[s + 1][1] = v4i{0, 0, 0, 0};
+        }
+    };
+
+    // ---- elements of other blobs ---------------------------------------------------------------------------------------------------
+    struct {
+        v4i v[2];
+    } add;
+    const unsigned f_bytes = pa.total_pix * K0 * 4u;
+    Epilogue ep0 = pp_epilogue(l0);
+    if constexpr (FUSED) ep0.residual = ja.residual, ep0.twin = ja.twin;
+    if constexpr (FUSED || SHUF) ep0.twin_scale = ja.twin_scale, ep0.twin_half = ja.twin_half;
+    const unsigned add_at = SHUF ? ja_pack(ja) == 8 ? at_f8(K0) : at_f4(K0) : at_f4(K0), add_half = SHUF && ja_pack(ja) == 8 ? 16u : HW * 16u;
+    auto load_add = [&](int pr) {
+        const unsigned s = pr < pairs0 ? (unsigned)pr * 128u : 0u;
+        if constexpr (PARTS) {
+            if (pr < pairs0 && 32u * pr + 8 * q < K0 && ok)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    add.v[h] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep0, ja.join(), n, pix, (int)(32u * pr + 8 * q + 4 * h), (int)K0, (int)HW));
+        } else if constexpr (FUSED || SHUF) {
+            const __amdgpu_buffer_rsrc_t r = rsrc(add_blob(ja), pr < pairs0 && add_blob(ja) != nullptr ? f_bytes : 0u);  // (none: zero, and not used)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) add.v[h] = load16(r, add_at | (32u * pr + 8 * q + 4 * h < K0 ? 0u : PR_OOB), s * HW + h * add_half);
+        }
+    };
+
+    // ---- the depthwise layer -----------------------------------------------------------------------------------------------------------
+    {
+        const unsigned HWi = (unsigned)(pa.H * pa.W), second = q & 1;  // second: of the two pairs of taps in a reduction step
+        const unsigned oy = div_by(pix, FastDiv{pa.ow_m, pa.ow_s, (unsigned)pa.OW}), ox = pix - oy * pa.OW;
+        const int y0 = (int)oy * pa.sh - pa.ph, x0 = (int)ox * pa.sw - pa.pw;
+        const int base = (int)((n * C8 + (q >> 1)) * HWi) + y0 * pa.W + x0;
+        // the taps inside the image as bits, shifted to the lane's own
+        unsigned columns = 0, taps = 0;
+#pragma unroll
+        for (int d = 0; d < KS; ++d) columns |= (unsigned)(x0 + d * pa.dw) < (unsigned)pa.W ? 1u << d : 0u;
+#pragma unroll
+        for (int d = 0; d < KS; ++d) taps |= (unsigned)(y0 + d * pa.dh) < (unsigned)pa.H ? columns << KS * d : 0u;
+        taps = ok ? second ? taps >> 2 : taps : 0u;
+        unsigned v[M][2];
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int t0 = 4 * m + e, t1 = t0 + 2;
+                const int at0 = t0 / KS * pa.dh * pa.W + t0 % KS * pa.dw, at1 = t1 / KS * pa.dh * pa.W + t1 % KS * pa.dw;
+                v[m][e] = taps >> t0 & 1 ? (unsigned)(base + (second ? at1 : at0)) * 8u : PR_OOB;
+            }
+        // channel r = p's bytes in the operand: dword p / 4 of its octet's two pixels, if the lane's bytes are of that octet
+        unsigned sel[2][4];
+        {
+            const bool mine = (p >> 3) == (q >> 1);
+            const unsigned zero = 0x0c0c0c0cu, at = 8u * (p & 3);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (unsigned b = 0; b < 4; ++b) sel[h][b] = mine && ((p >> 2) & 1) == (unsigned)h ? (zero & ~(0xffu << at)) | b << at : zero;
+        }
+        const int pairs = ((int)C8 + 1) / 2;  // of octets
+        const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.in_bytes), rw = rsrc(pa.dw_w, (unsigned)pairs * 256u * PK);
+        v4i b[M];
+        int w[PK];
+        auto load = [&](int op) {
+            const unsigned s = (unsigned)op * 16u * HWi;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const v2i lo = load8(rin, v[m][0], s), hi = 4 * m + 1 < TAPS ? load8(rin, v[m][1], s) : v2i{0, 0};
+                b[m] = v4i{lo[0], lo[1], hi[0], hi[1]};
+            }
+            if constexpr (PK == 2) {
+                const v2i t = load8(rw, lane * 8, (unsigned)op * 512u);
+                w[0] = t[0], w[1] = t[1];
+            } else {
+                const v4i t = load16(rw, lane * 16, (unsigned)op * 1024u);
+#pragma unroll
+                for (int i = 0; i < PK; ++i) w[i] = t[i];
+            }
+        };
+        load(min(first, pairs - 1));
+        asm volatile("" ::: "memory");  // (in front of the others: the compiler would move them to the loop)
+
+        // ---- constants into LDS: scale_in and bias of each layer (they are padded to whole pairs of tiles and more) ---------------------
+        // (an array a wave: six of them, the waves behind have none)
+        {
+            const unsigned d = wave >> 1;  // 0: the depthwise layer, 1, 2: the others
+            const float* const si = d == 0 ? pa.dw_scale_in : d == 1 ? l0.scale_in : l1.scale_in;
+            const float* const bi = d == 0 ? pa.dw_bias : d == 1 ? l0.bias : l1.bias;
+            const unsigned quads = d == 0 ? Cd / 4 : d == 1 ? 8u * pairs0 : d == 2 ? 8u * pairs1 : 0u;
+            const __amdgpu_buffer_rsrc_t r = rsrc(wave & 1 ? bi : si, quads * 16u);
+            v4i* const to = reinterpret_cast<v4i*>(d == 0 ? constsd : d == 1 ? consts0 : consts1) + (wave & 1 ? quads : 0u);
+            for (unsigned i0 = 0; i0 < quads; i0 += 256) {
+                v4i c[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (k == 0 || i0 + 64 * k < quads) c[k] = load16(r, lane * 16 + k * 1024, i0 * 16);  // (uniform)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (i0 + 64 * k + lane < quads) to[i0 + 64 * k + lane] = c[k];
+            }
+        }
+        __syncthreads();
+
+        // ---- what comes behind the depthwise layer, requested now: weights, elements of another blob --------------------------------------
+        const bool begins1 = NEXT && first >= pairs0;  // a wave without a pair of the first layer
+        load_a(begins1, min(first, (begins1 ? pairs1 : pairs0) - 1), 0);
+        load_add(first);
+
+        // LeakyReLU or none, and the clamp of the rounded result: [0, dw_qh] behind ReLU / clip, else the int8 range
+        Epilogue epd{};
+        epd.act_p0 = pa.dw_p0, epd.lrelu = pa.dw_lrelu != 0;
+        const ohip_v2s top = __builtin_bit_cast(ohip_v2s, pa.dw_qh), bottom = __builtin_bit_cast(ohip_v2s, pa.dw_nonneg ? 0u : 0xff81ff81u);
+        for (int op = first; op < pairs;) {
+            v4i acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                constexpr unsigned Z = 0;
+                const int e = 2 * (m & 1);
+                const v4i A = {(int)__builtin_amdgcn_perm(Z, (unsigned)w[m >> 1], sel[0][e]), (int)__builtin_amdgcn_perm(Z, (unsigned)w[m >> 1], sel[1][e]),
+                               (int)__builtin_amdgcn_perm(Z, (unsigned)w[m >> 1], sel[0][e + 1]), (int)__builtin_amdgcn_perm(Z, (unsigned)w[m >> 1], sel[1][e + 1])};
+                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, b[m], acc, 0, 0, 0);
+            }
+            const int now = op;
+            op += stride;
+            if (op < pairs) load(op);  // (refilled in place: the next pair's bytes arrive under this one's requantization)
+            const v4i si = *reinterpret_cast<const v4i*>(constsd + 16 * now + 4 * q), bi = *reinterpret_cast<const v4i*>(constsd + Cd + 16 * now + 4 * q);
+            int k[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float t = __fmul_rn(lrelu_or_not(epd, __fmaf_rn((float)acc[e], __int_as_float(si[e]), __int_as_float(bi[e]))), pa.dw_scale);
+                k[e] = (int)__fadd_rn(t, __builtin_copysignf(pa.dw_half, t));
+            }
+            ohip_v2s lo = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[0], k[1])), hi = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[2], k[3]));
+            lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bottom);
+            hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bottom);
+            if (2u * now + (q >> 1) < C8)
+                *reinterpret_cast<unsigned*>(px0 + row0 + 16 * now + 4 * q) =
+                    __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
+        }
+    }
+    __syncthreads();
+
+    // One pointwise layer: the wave's pairs; finish(pair, sums). Behind the last one the next layer's first weights are requested.
+    auto layer = [&](auto second_c, const PwPwLayer& l, int pairs, const int8_t* px, auto finish) {
+        constexpr bool SECOND = decltype(second_c)::value;
+        for (int pr = first; pr < pairs; pr += stride) {
+            v4i c0 = {0, 0, 0, 0}, c1 = {0, 0, 0, 0};
+            for (int s0 = 0; s0 < l.steps; s0 += SC) {
+                auto step = [&](int s) {  // (one that does not exist: zero weights, and bytes of this workgroup's LDS)
+                    const v4i b = *reinterpret_cast<const v4i*>(px + 64 * (s0 + s));
+                    c0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[s][0], b, c0, 0, 0, 0);
+                    c1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[s][1], b, c1, 0, 0, 0);
+                };
+                step(0), step(1);
+#pragma unroll
+                for (int s = 2; s < SC; s += 2)
+                    if (s0 + s < l.steps) step(s), step(s + 1);  // (uniform)
+                const bool same = s0 + SC < l.steps, more = same || pr + stride < pairs;
+                const bool then = NEXT && !SECOND && !more;
+                load_a(SECOND || then, same ? pr : more ? pr + stride : then ? min(first, pairs1 - 1) : pr, same ? s0 + SC : 0);
+            }
+            finish(pr, c0, c1);
+        }
+    };
+    auto constants = [&](const float* c, int pairs, unsigned ch0, float (&si)[8], float (&bi)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) si[e] = c[ch0 + e], bi[e] = c[32 * pairs + ch0 + e];
+    };
+
+    // ---- the first pointwise layer --------------------------------------------------------------------------------------------------
+    int8_t* const to1 = px1 + row1;  // this lane's pixel of the second layer's input
+    const __amdgpu_buffer_rsrc_t rout0 = NEXT ? rsrc(sum, sum != nullptr ? f_bytes : 0u) : rsrc(out, out == nullptr ? 0u : I8 ? f_bytes / 4u : f_bytes);
+    auto finish0 = [&](int pr, const v4i& c0, const v4i& c1) {
+        const unsigned ch0 = 32u * pr + 8 * q;
+        float si[8], bi[8];
+        constants(consts0, pairs0, ch0, si, bi);
+        if constexpr (I8) {
+            const v2i b = pp_bytes<false>(ep0, l0, si, bi, c0, c1);
+            if constexpr (NEXT) {
+                if (ch0 < K0) *reinterpret_cast<v2i*>(to1 + ch0) = b;
+            } else {
+                store8(rout0, b, ch0 < K0 ? at_b8(K0) : PR_OOB, (unsigned)pr * 32u * HW);
+            }
+        } else {
+            v4i r[2] = {pp_values(ep0, si, bi, c0), pp_values(ep0, si + 4, bi + 4, c1)};
+            if constexpr (SHUF) {
+                // with the same channels of the other blob these are channels 2 ch0 .. 2 ch0 + 15 of the shuffled one: two packs of 8
+                const unsigned half = K0 / 8;  // packs of 8 in each half
+#pragma unroll
+                for (int w = 0; w < 2; ++w) {
+                    float* const f = w ? ja.sh_out1 : ja.sh_out0;
+                    int8_t* const b8 = w ? ja.sh_q1 : ja.sh_q0;
+                    if (w ? 8u * pr + 8 <= half : 8u * pr >= half) continue;  // (uniform: none of the pair's packs is in this half)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const v4i o = add.v[h];
+                        const v4i even = ja.other_odd ? r[h] : o, odd = ja.other_odd ? o : r[h];  // (uniform)
+                        const v4i lo = {even[0], odd[0], even[1], odd[1]}, hi = {even[2], odd[2], even[3], odd[3]};
+                        const unsigned pack = ch0 / 4 + h - (w ? half : 0u);  // in this half; beyond it on either side: the other half's
+                        const unsigned e = n * ja.sh_image + (pack * HW + pix) * 8u;
+                        const bool live = ok && pack < half;  // (a channel past the last one is a pack past the second half)
+                        if (NEXT && w) {
+                            const v2i b = {quantize4(lo, ja.twin_scale, ja.twin_half), quantize4(hi, ja.twin_scale, ja.twin_half)};
+                            if (pack < half) *reinterpret_cast<v2i*>(to1 + 8 * pack) = b;
+                            continue;
+                        }
+                        if (f != nullptr) {
+                            const __amdgpu_buffer_rsrc_t rf = rsrc(f, PR_OOB);
+                            store16(rf, lo, live ? e * 4u : PR_OOB, 0), store16(rf, hi, (live ? e * 4u : PR_OOB) + 16u, 0);
+                        }
+                        if (b8 != nullptr)
+                            store8(rsrc(b8, PR_OOB), v2i{quantize4(lo, ja.twin_scale, ja.twin_half), quantize4(hi, ja.twin_scale, ja.twin_half)},
+                                   live ? e : PR_OOB, 0);
+                    }
+                }
+            } else {
+                v2i tw;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (PARTS || ep0.residual != nullptr)  // (uniform)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) r[h][e] = __float_as_int(__fadd_rn(__int_as_float(r[h][e]), __int_as_float(add.v[h][e])));
+                    if (NEXT || ep0.twin != nullptr) tw[h] = quantize4(r[h], ep0.twin_scale, ep0.twin_half);
+                    // (no blob: a descriptor of no bytes, the store is dropped)
+                    store16(rout0, r[h], ch0 + 4 * h < K0 ? at_f4(K0) : PR_OOB, (unsigned)pr * 128u * HW + h * HW * 16u);
+                }
+                if constexpr (NEXT) {
+                    if (ch0 < K0) *reinterpret_cast<v2i*>(to1 + ch0) = tw;
+                } else if (ep0.twin != nullptr) {  // K % 8 == 0 then: the lane's 8 channels are one Byte8 element
+                    store8(rsrc(ep0.twin, f_bytes / 4u), tw, ch0 < K0 ? at_b8(K0) : PR_OOB, (unsigned)pr * 32u * HW);
+                }
+            }
+        }
+    };
+    auto finish_then_add = [&](int pr, const v4i& c0, const v4i& c1) {
+        finish0(pr, c0, c1);
+        if ((SHUF || FUSED) && pr + stride < pairs0) load_add(pr + stride);
+    };
+    if constexpr (!NEXT) {
+        layer(std::false_type{}, l0, pairs0, px0 + row0 + 16 * q, finish_then_add);
+    } else {
+        layer(std::false_type{}, l0, pairs0, px0 + row0 + 16 * q, finish_then_add);
+        __syncthreads();
+
+        // ---- the second ------------------------------------------------------------------------------------------------------------
+        const unsigned K1 = l1.K;
+        const Epilogue ep1 = pp_epilogue(l1);
+        const __amdgpu_buffer_rsrc_t rout = rsrc(out, pa.total_pix * K1 * (KIND1 == PP_F32 ? 4u : 1u));
+        auto finish1 = [&](int pr, const v4i& c0, const v4i& c1) {
+            const unsigned ch0 = 32u * pr + 8 * q;
+            float si[8], bi[8];
+            constants(consts1, pairs1, ch0, si, bi);
+            if constexpr (KIND1 == PP_F32) {
+                const v4i r0 = pp_values(ep1, si, bi, c0), r1 = pp_values(ep1, si + 4, bi + 4, c1);
+                const unsigned v = at_f4(K1), s = (unsigned)pr * 128u * HW;
+                store16(rout, r0, ch0 < K1 ? v : PR_OOB, s), store16(rout, r1, ch0 + 4 < K1 ? v : PR_OOB, s + HW * 16u);
+            } else {
+                store8(rout, pp_bytes<KIND1 == PP_NONNEG>(ep1, l1, si, bi, c0, c1), ch0 < K1 ? at_b8(K1) : PR_OOB, (unsigned)pr * 32u * HW);
+            }
+        };
+        layer(std::true_type{}, l1, pairs1, px1 + row1 + 16 * q, finish1);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------------------------------------------------------------
+
+static size_t dwpw_lds_bytes(const ConvGeom& g0, const ConvGeom* g1, int groups) {
+    const size_t rows = 64 * (size_t)igemm_channel_groups(g0.C) + 16 + (g1 ? 64 * (size_t)igemm_channel_groups(g1->C) + 16 : 0);
+    return 16 * (size_t)groups * rows + 256 * (size_t)((g0.K + 31) / 32 + (g1 ? (g1->K + 31) / 32 : 0)) +
+           128 * (size_t)((g0.C / 8 + 1) / 2);
+}
+
+bool dwpw_front_applicable(const ConvGeom& gd, const Epilogue& ed) {
+    if (gd.groups != gd.C || gd.K != gd.C || gd.C % 8 || gd.kh != gd.kw || (gd.kh != 3 && gd.kh != 5)) return false;
+    for (int v : {gd.sh, gd.sw, gd.ph, gd.pw, gd.dh, gd.dw})
+        if (v > 255) return false;
+    const int epi = dw_mfma_epilogue(ed, gd.K);
+    if (epi != EPI_I8_P8 && epi != EPI_I8_P8_NONNEG) return false;
+    const size_t limit = (size_t)1 << 31;
+    return (size_t)gd.N * gd.C * gd.H * gd.W < limit && (size_t)gd.C * 64 < limit;
+}
+
+bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, const Epilogue* e1) {
+    if (!dwpw_front_applicable(gd, ed) || !pwpw_pointwise(g0) || g0.C != gd.K || g0.N != gd.N || g0.H != gd.OH || g0.W != gd.OW || g0.N < 1) return false;
+    if (dwpw_lds_bytes(g0, g1, 1) > 65536) return false;
+    const int k0 = pwpw_kind(e0, g0.K);
+    const bool shuffle = e0.join && e0.join->other, parts = e0.join && !shuffle;
+    if (k0 != PP_I8 && k0 != PP_F32) return false;
+    if (k0 == PP_I8 && e0.fused()) return false;
+    if ((e0.twin || shuffle || parts || g1) && g0.K % 8) return false;
+    if (g1) {
+        if (!pwpw_pointwise(*g1) || g1->C != g0.K || g1->N != g0.N || g1->H != g0.H || g1->W != g0.W) return false;
+        if (parts || e0.twin || pwpw_kind(*e1, g1->K) < 0) return false;
+        if (shuffle && (e0.join->sh_image != (size_t)g0.K * g0.H * g0.W || !e0.join->sh_out0)) return false;  // (two halves)
+        if (gd.kh == 5 && k0 != PP_I8) return false;
+    } else if (gd.kh == 5 && shuffle) {
+        return false;
+    }
+    const size_t px = (size_t)g0.N * g0.H * g0.W, limit = (size_t)1 << 31;
+    if (px * g0.C >= limit || px * g0.K * (k0 == PP_F32 ? 4 : 1) >= limit) return false;
+    if (shuffle && px * g0.K * 4 * (g1 ? 1 : 2) >= limit) return false;
+    if (g1 && px * g1->K * layout_elem_bytes(e1->out_layout) >= limit) return false;
+    for (const ConvGeom* g : {&g0, g1})
+        if (g && (size_t)igemm_channel_groups(g->C) * igemm_padded_rows(g->K) * 64 >= limit) return false;  // (the packed weights)
+    return true;
+}
+
+// Cost models in us, fitted to launches replayed from captured graphs over drawn layers (8 to 960 channels, 4x4 to 112x112 pixels, batches
+// of 1 to 64, every end). The launch: a wave walks `nd` pairs of octets and n0 and n1 pairs of row tiles one behind the other, once if
+// every workgroup is resident, and the more often the more workgroups there are for a compute unit.
+struct DwPwShape {
+    double px;  // output pixels
+    int pairs_d, pairs[2], steps[2];
+    bool k5, f32, adds;
+    DwPwShape(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1)
+        : px((double)g0.N * g0.H * g0.W), pairs_d((gd.C / 8 + 1) / 2),
+          pairs{(g0.K + 31) / 32, g1 ? (g1->K + 31) / 32 : 0}, steps{igemm_channel_groups(g0.C), g1 ? igemm_channel_groups(g1->C) : 0},
+          k5(gd.kh == 5), f32(e0.out_kind == OTTER_HIP_OUT_F32), adds(e0.residual || e0.join) {}
+};
+static double dwpw_cost(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1, int groups) {
+    static const double once[8] = {3.13, 0.450, 0.831, 0.528, 0.100, 0.461, 0.113, 0.308}, more[8] = {0.833, 0.258, 0.709, 0.087, 0.107, 0.281, 0.018, 0};
+    const int stride = DP_WAVES / groups, nd = (s.pairs_d + stride - 1) / stride;
+    const int n0 = (s.pairs[0] + stride - 1) / stride, n1 = (s.pairs[1] + stride - 1) / stride;
+    const double f[8] = {1, s.k5 ? 0. : nd, s.k5 ? (double)nd : 0, (double)n0, (double)n0 * s.steps[0], (double)n1, (double)n1 * s.steps[1], s.f32 ? (double)n0 : 0};
+    const double rounds = std::max(0., s.px / (16 * groups) / 256 - 1);
+    double t = 0;
+    for (int i = 0; i < 8; ++i) t += f[i] * (once[i] + rounds * more[i]);
+    const double bytes = s.px * ((double)gd.C * gd.sh * gd.sw + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (g1 ? g1->K : 0));
+    return t + 0.163e-6 * bytes;
+}
+static double dwpw_cost_apart(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1) {
+    const double mbd = 1e-6 * s.px * gd.C * (gd.sh * gd.sw + 1.);
+    const double mb0 = 1e-6 * s.px * (gd.C + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (s.f32 ? g0.K : 0));
+    double t = 4.86 + (0.254 + (s.k5 ? 0.025 : 0)) * mbd + 0.210 * mb0 + 1.395e-9 * s.px * g0.C * g0.K + 0.976e-3 * gd.C + 1.006e-3 * g0.K +
+               (gd.C > 256 ? 0.068 + 0.035e-6 * s.px * gd.C : 0);
+    if (g1) t += 1.80 + 0.323e-6 * s.px * ((double)g0.K + g1->K) + 1.065e-9 * s.px * g0.K * g1->K + 2.19e-3 * g1->K;
+    return t;
+}
+
+// Groups of 16 pixels for a workgroup.
+static int dwpw_groups(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
+    const DwPwShape s(gd, g0, e0, g1);
+    int best = 1;
+    for (int g = 2; g <= 8; g *= 2)
+        if (dwpw_lds_bytes(g0, g1, g) <= 65536 && dwpw_cost(s, gd, g0, g1, g) < dwpw_cost(s, gd, g0, g1, best)) best = g;
+    return best;
+}
+bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
+    const DwPwShape s(gd, g0, e0, g1);
+    return dwpw_cost(s, gd, g0, g1, dwpw_groups(gd, g0, e0, g1)) < 0.95 * dwpw_cost_apart(s, gd, g0, g1);
+}
+
+template <int TAPS, int EPI, int KIND1>
+static hipError_t launch_dwpw(const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
+    launch((conv_dwpw_kernel<TAPS, EPI, KIND1>), dim3((pa.tiles + 7) / 8 * 8), dim3(64 * DP_WAVES), lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0));
+    return hipGetLastError();
+}
+
+hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const ConvGeom& gd, const Epilogue& ed, const int8_t* const w[2],
+                         const float so[2], void* out, float* sum, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, const Epilogue* e1,
+                         int force, hipStream_t stream) {
+    if (!conv_dwpw_applicable(gd, ed, g0, e0, g1, e1)) return hipErrorInvalidValue;
+    DwPwArgs pa{};
+    pa.l[0] = pwpw_layer(g0, e0, w[0], so[0]);
+    if (g1) pa.l[1] = pwpw_layer(*g1, *e1, w[1], so[1]);
+    pa.dw_w = dw_w, pa.dw_scale_in = ed.scale_in, pa.dw_bias = ed.bias, pa.dw_p0 = ed.act_p0, pa.dw_lrelu = ed.lrelu;
+    pa.dw_scale = dw_so, pa.dw_half = ed.round_half, pa.dw_nonneg = dw_mfma_epilogue(ed, gd.K) == EPI_I8_P8_NONNEG;
+    const float both[2] = {dw_so, dw_so};
+    pa.dw_qh = 0x007f007fu;
+    if (pa.dw_nonneg) conv_pw_stream_clamps(ed.act_hi, ed.round_half, both, 2, &pa.dw_qh);
+    const FastDiv hw = fast_div((unsigned)(g0.H * g0.W)), ow = fast_div((unsigned)g0.W);
+    pa.hw_m = hw.m, pa.hw_s = hw.s, pa.ow_m = ow.m, pa.ow_s = ow.s;
+    pa.HW = g0.H * g0.W, pa.OW = g0.W, pa.H = gd.H, pa.W = gd.W, pa.total_pix = (unsigned)g0.N * (unsigned)pa.HW;
+    pa.in_bytes = (unsigned)((size_t)gd.N * gd.C * gd.H * gd.W);
+    pa.sh = gd.sh, pa.sw = gd.sw, pa.ph = gd.ph, pa.pw = gd.pw, pa.dh = gd.dh, pa.dw = gd.dw, pa.C8 = gd.C / 8;
+    const int groups = force ? force : dwpw_groups(gd, g0, e0, g1);
+    if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return hipErrorInvalidValue;
+    const size_t lds = dwpw_lds_bytes(g0, g1, groups);
+    if (lds > 65536) return hipErrorInvalidValue;
+    pa.lg = groups == 1 ? 0 : groups == 2 ? 1 : groups == 4 ? 2 : 3;
+    pa.tiles = (int)((pa.total_pix + 16 * groups - 1) / (16 * groups));
+    const int next = g1 ? pa.l[1].kind : (int)DP_NONE;
+    const bool shuffle = e0.join && e0.join->other;
+#define OHIP_DP(T_, E_, N_) return launch_dwpw<T_, E_, N_>(x, out, sum, pa, e0, lds, stream)
+#define OHIP_DPN(T_, E_)                             \
+    do {                                             \
+        if (next == PP_I8) OHIP_DP(T_, E_, PP_I8);   \
+        if (next == PP_NONNEG) OHIP_DP(T_, E_, PP_NONNEG); \
+        if (next == PP_F32) OHIP_DP(T_, E_, PP_F32); \
+    } while (0)
+    if (gd.kh == 3) {
+        if (shuffle) {
+            OHIP_DPN(9, EPI_F32_SHUFFLE);
+            OHIP_DP(9, EPI_F32_SHUFFLE, DP_NONE);
+        }
+        if (e0.join) OHIP_DP(9, EPI_F32_P4_PARTS, DP_NONE);
+        if (pa.l[0].kind == PP_F32) {
+            OHIP_DPN(9, EPI_F32_P4_FUSED);
+            OHIP_DP(9, EPI_F32_P4_FUSED, DP_NONE);
+        }
+        OHIP_DPN(9, EPI_I8_P8);
+        OHIP_DP(9, EPI_I8_P8, DP_NONE);
+    }
+    if (e0.join) OHIP_DP(25, EPI_F32_P4_PARTS, DP_NONE);
+    if (pa.l[0].kind == PP_F32) OHIP_DP(25, EPI_F32_P4_FUSED, DP_NONE);
+    OHIP_DPN(25, EPI_I8_P8);
+    OHIP_DP(25, EPI_I8_P8, DP_NONE);
+#undef OHIP_DPN
+#undef OHIP_DP
+}
+
+}  // namespace ohip

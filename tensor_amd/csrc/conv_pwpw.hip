@@ -11,8 +11,7 @@
 //    conv_pw_reg.hip, with that kernel's epilogues; the bytes that the second layer reads go to LDS;
 //  * behind a barrier they do the same for the second layer.
 #include "common.hpp"
-#include "conv_igemm.hpp"
-#include "conv_pw_common.hpp"
+#include "conv_pwpw_common.hpp"
 
 #include <algorithm>
 
@@ -21,18 +20,7 @@ namespace ohip {
 namespace {
 
 constexpr int PP_WAVES = 4;  // of a workgroup (eight: faster only at 13x13 and below, by 0.1 us)
-enum { PP_I8, PP_NONNEG, PP_F32 };  // an int8 result, one behind ReLU / clip, an fp32 one
 
-// one of the two layers, as PwRegArgs has it
-struct PwPwLayer {
-    const int8_t* w;
-    const float *scale_in, *bias;
-    float p0, scale, half;
-    unsigned qh;
-    int K, mt;
-    unsigned short steps;
-    unsigned char kind, lrelu;
-};
 struct PwPwArgs {
     PwPwLayer l[2];
     unsigned hw_m, total_pix;
@@ -40,32 +28,6 @@ struct PwPwArgs {
     unsigned short C8;
     unsigned char hw_s;
 };
-
-// Eight channels of a pixel as bytes (PP_I8, PP_NONNEG); four as values (PP_F32). (The clamp is open for LeakyReLU.)
-template <bool NONNEG>
-__device__ __forceinline__ v2i pp_bytes(const Epilogue& ep, const PwPwLayer& l, const float (&si)[8], const float (&bi)[8], const v4i& c0, const v4i& c1) {
-    Epi8 prm;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) prm.si[e] = si[e], prm.bi[e] = bi[e], prm.so[e] = l.scale;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) prm.qh[e] = l.qh;
-    const int a8[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
-    return epi8_quant_i8p8<NONNEG>(ep, prm, a8);
-}
-__device__ __forceinline__ v4i pp_values(const Epilogue& ep, const float* si, const float* bi, const v4i& c) {
-    v4i r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        r[e] = __float_as_int(lrelu_or_not(ep, fminf(fmaxf(__fmaf_rn((float)c[e], si[e], bi[e]), ep.act_lo), ep.act_hi)));
-    return r;
-}
-__device__ __forceinline__ Epilogue pp_epilogue(const PwPwLayer& l) {
-    Epilogue ep{};
-    ep.act_p0 = l.p0, ep.lrelu = l.lrelu;
-    if (l.kind == PP_F32) ep.act_lo = l.scale, ep.act_hi = l.half;
-    else ep.round_half = l.half;
-    return ep;
-}
 
 }  // namespace
 
@@ -274,17 +236,6 @@ __global__ void __launch_bounds__(64 * PP_WAVES) conv_pwpw_kernel(const int8_t* 
 // host side
 // ---------------------------------------------------------------------------------------------------------------------------------
 
-static bool pwpw_pointwise(const ConvGeom& g) {
-    return g.groups == 1 && g.kh == 1 && g.kw == 1 && g.sh == 1 && g.sw == 1 && g.ph == 0 && g.pw == 0 && g.C % 8 == 0;
-}
-static int pwpw_kind(const Epilogue& ep, int K) {
-    switch (pick_epilogue(ep, K)) {
-    case EPI_I8_P8: return PP_I8;
-    case EPI_I8_P8_NONNEG: return PP_NONNEG;
-    case EPI_F32_P4: return PP_F32;
-    }
-    return -1;
-}
 static size_t pwpw_lds_bytes(const ConvGeom& g0, const ConvGeom& g1, int fn) {
     const size_t rows = 64 * (size_t)(igemm_channel_groups(g0.C) + igemm_channel_groups(g1.C)) + 32;
     return 16 * (size_t)fn * rows + 256 * (size_t)((g0.K + 31) / 32 + (g1.K + 31) / 32);
@@ -333,16 +284,7 @@ hipError_t run_conv_pwpw(const int8_t* x, const int8_t* const w[2], const float 
                          const Epilogue& e0, const ConvGeom& g1, const Epilogue& e1, int force, hipStream_t stream) {
     if (!conv_pwpw_applicable(g0, e0, g1, e1)) return hipErrorInvalidValue;
     PwPwArgs pa{};
-    for (int i = 0; i < 2; ++i) {
-        const ConvGeom& g = i ? g1 : g0;
-        const Epilogue& ep = i ? e1 : e0;
-        PwPwLayer& l = pa.l[i];
-        l.w = w[i], l.scale_in = ep.scale_in, l.bias = ep.bias, l.p0 = ep.act_p0, l.lrelu = ep.lrelu, l.K = g.K;
-        l.mt = igemm_padded_rows(g.K) / 16, l.steps = (unsigned short)igemm_channel_groups(g.C), l.kind = (unsigned char)pwpw_kind(ep, g.K);
-        l.scale = l.kind == PP_F32 ? ep.act_lo : so[i], l.half = l.kind == PP_F32 ? ep.act_hi : ep.round_half;
-        const float both[2] = {so[i], so[i]};
-        if (l.kind == PP_NONNEG) conv_pw_stream_clamps(ep.act_hi, ep.round_half, both, 2, &l.qh);
-    }
+    for (int i = 0; i < 2; ++i) pa.l[i] = pwpw_layer(i ? g1 : g0, i ? e1 : e0, w[i], so[i]);
     const FastDiv hw = fast_div((unsigned)(g0.H * g0.W));
     pa.hw_m = hw.m, pa.hw_s = (unsigned char)hw.s, pa.HW = g0.H * g0.W, pa.total_pix = (unsigned)g0.N * (unsigned)pa.HW, pa.C8 = (unsigned short)(g0.C / 8);
     int fn = force ? force : pa.total_pix >= 16384 ? 2 : 1;  // (88 channels @52x52 b16 9.6 us with one group of pixels, 8.3 with two; @26x26 4.8 and 4.7)

@@ -995,6 +995,91 @@ int ConvolutionLayer::forward_pair(const ConvolutionLayer* a, const ConvolutionL
     return 0;
 }
 
+int ConvolutionLayer::forward_dwpw(const ConvolutionLayer* d, const ConvolutionLayer* p, const Tensor& bottom_in, DwPw& u, const NetOption& opt) {
+    for (const ConvolutionLayer* c : {d, p, u.next})
+        if (c && (!c->handle_ || c->force_out_layout >= 0 || !c->int8_scale_term)) return 1;
+    if (!opt.use_packing_layout || !bottom_in.defined() || bottom_in.dim() != 4) return 1;
+    Tensor bottom = bottom_in, twin;
+    if (base_of(bottom.scalar_type()) == ScalarType::Float &&
+        bottom.quantized_twin(d->bottom_blob_int8_scales.data_ptr<float>()[0], d->input_round_mode(opt), twin))
+        bottom = twin;
+    if (bottom.scalar_type() != ScalarType::Byte8 || bottom.channels() != d->in_channels) return 1;
+    const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3), K = p->out_channels;
+    int oh = 0, ow = 0;
+    if (otter_hip_conv_output_shape(d->handle_, H, W, &oh, &ow)) return 1;
+    const ConvolutionLayer* const last = u.next ? u.next : p;
+    const int layout = otter_hip_conv_default_out_layout(last->handle_);
+    const bool f32 = p->int8_scale_term <= 100, with_q = f32 && u.q_scale > 0.f && K % 8 == 0;
+    if (layout != OTTER_HIP_I8_P8 && layout != OTTER_HIP_F32_P4) return 1;
+    if (u.next && f32 && !with_q) return 1;
+    auto addend = [&](const Tensor* t, int channels) {
+        return t->defined() && t->dim() == 4 && base_of(t->scalar_type()) == ScalarType::Float && t->elempack() != 1 && t->size(0) == N &&
+               t->size(2) == oh && t->size(3) == ow && (channels < 0 || t->channels() == channels);
+    };
+    otter_hip_conv_end end{};
+    float some;  // (a place for pointers of which only whether they are null is asked)
+    end.next = u.next ? u.next->handle_ : nullptr, end.q_scale = u.q_scale, end.q_round_mode = u.q_round;
+    if (u.shortcut) {
+        if (!f32 || !addend(u.shortcut, u.part1 ? -1 : K)) return 1;
+        end.residual = (const float*)u.shortcut->device_ptr();
+        if (u.part1) {
+            if (!addend(u.part1, K - (int)u.shortcut->channels()) || u.shortcut->channels() % 8) return 1;
+            end.residual1 = (const float*)u.part1->device_ptr(), end.part0_channels = (int)u.shortcut->channels();
+            end.part0_layout = hip_layout_of(u.shortcut->scalar_type()), end.part1_layout = hip_layout_of(u.part1->scalar_type());
+        } else if (u.shortcut->elempack() != 4) {
+            return 1;
+        }
+    }
+    const bool no_f32 = u.int8_only && with_q;
+    if (u.other) {
+        if (!f32 || !addend(u.other, K)) return 1;
+        end.other = (const float*)u.other->device_ptr(), end.other_layout = hip_layout_of(u.other->scalar_type()), end.other_odd = u.other_odd;
+        end.joined = u.joined, end.first_half = &some;
+    } else if (with_q && !u.next) {
+        end.out_q = (int8_t*)&some;
+    }
+    if (otter_hip_conv_dwpw_launches(d->handle_, p->handle_, N, H, W, &end, layout) != 1) return 1;
+    try {
+        const ScalarType odt = scalar_type_of_layout(layout);
+        Tensor q, &whole = !u.other ? u.out : u.joined ? u.first : u.second;  // whole: the blob that is quantized
+        void* out = nullptr;
+        if (u.other) {
+            const std::vector<int64_t> sizes = {N, (u.joined ? 2 : 1) * K / 8, oh, ow};
+            if (!u.next) {
+                if (with_q) q = Tensor::empty_device(sizes, ScalarType::Byte8);
+                if (!no_f32) whole = Tensor::empty_device(sizes, ScalarType::Float8);
+            }
+            if (!u.joined) u.first = Tensor::empty_device(sizes, ScalarType::Float8);
+            end.first_half = u.first.defined() ? (float*)u.first.device_ptr() : nullptr;
+            if (!u.joined && u.second.defined()) end.second_half = (float*)u.second.device_ptr();
+            (u.joined ? end.first_half_q : end.second_half_q) = q.defined() ? (int8_t*)q.device_ptr() : nullptr;
+        } else {
+            if (with_q && !u.next) q = Tensor::empty_device({N, K / 8, oh, ow}, ScalarType::Byte8);
+            if (f32 ? !no_f32 : !u.next)
+                u.out = Tensor::empty_device({N, K / (f32 ? 4 : 8), oh, ow}, f32 ? ScalarType::Float4 : ScalarType::Byte8);
+            void* const result = u.out.defined() ? u.out.device_ptr() : nullptr;
+            if (u.next) end.sum = (float*)result;
+            else out = result;
+            end.out_q = q.defined() ? (int8_t*)q.device_ptr() : nullptr;
+        }
+        if (u.next) {
+            u.behind = Tensor::empty_device({N, u.next->out_channels / elempack_of(odt), oh, ow}, odt);
+            out = u.behind.device_ptr();
+        }
+        const int rc = otter_hip_conv_dwpw_forward(d->handle_, p->handle_, bottom.device_ptr(), N, H, W, &end, out, layout, launch_stream());
+        if (rc) return rc;
+        for (Tensor* t : {&u.out, &u.first, &u.second, &u.behind, &q})
+            if (t->defined()) t->mark_device_written();
+        if (q.defined()) {
+            if (whole.defined()) whole.attach_quantized(q, u.q_scale, u.q_round);
+            else whole = q;
+        }
+    } catch (const Error&) {
+        return -100;
+    }
+    return 0;
+}
+
 int ConvolutionLayer::block_launches(const ConvolutionLayer* e, const ConvolutionLayer* d, const ConvolutionLayer* p, int n, int h,
                                      int w) {
     return e->handle_ && d->handle_ && p->handle_ ? otter_hip_conv_block_fastest(e->handle_, d->handle_, p->handle_, n, h, w) : 3;
@@ -2056,6 +2141,10 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
         }
     }
     {
+        const int rc = forward_dwpw_unit(li, li, -1, -1, blobs, opt);
+        if (rc <= 0) return rc;
+    }
+    {
         const auto unit = pair_units_.find(li);
         // only when the blob between the two has not been computed (or set by the caller)
         if (unit != pair_units_.end() && !blobs[layer->bottoms[0]].defined()) {
@@ -2197,6 +2286,31 @@ void Net::plan_fused_quantize() const {
         const int pi = pair_reader((int)li) ? blobs_[layers_[li]->bottoms[0]].producer : -1;
         if (pi >= 0 && pair_layer(pi) && int8_result(pi) && sole_reader(layers_[pi]->tops[0]) == (int)li && !pair_units_.count(pi)) pair_units_[(int)li] = pi;
     }
+    // Pointwise layers behind a depthwise one that nothing else reads, and the pointwise layer that reads a blob's quantization
+    front_units_.clear();
+    next_units_.clear();
+    for (size_t li = 0; li < layers_.size(); ++li) {
+        if (pair_layer((int)li)) {
+            const int di = blobs_[layers_[li]->bottoms[0]].producer;
+            const auto* d = di < 0 ? nullptr : dynamic_cast<const ConvolutionLayer*>(layers_[di]);
+            if (d && d->of_library && d->int8_scale_term > 100 && d->groups == d->in_channels && d->groups == d->out_channels && d->in_channels % 8 == 0 &&
+                d->bottoms.size() == 1 && d->tops.size() == 1 && d->force_out_layout < 0 && sole_reader(d->tops[0]) == (int)li)
+                front_units_[(int)li] = di;
+        }
+        const Layer* l = layers_[li];
+        if (l->fuse_scale <= 0.f || (l->type() != "Eltwise" && l->type() != "ShortCut" && !pair_layer((int)li))) continue;
+        int next = -1, readers = 0;
+        std::vector<int> pending(l->tops.begin(), l->tops.end());
+        while (!pending.empty()) {
+            const int b = pending.back();
+            pending.pop_back();
+            for (int ci : blobs_[b].consumers) {
+                if (layers_[ci]->type() == "Split") pending.insert(pending.end(), layers_[ci]->tops.begin(), layers_[ci]->tops.end());
+                else if (dynamic_cast<const ConvolutionLayer*>(layers_[ci])) next = ci, ++readers;
+            }
+        }
+        if (readers == 1 && pair_reader(next)) next_units_[(int)li] = next;
+    }
     // ShuffleNetV2 unit tails: Concat of two equal blobs -> ChannelShuffle(2) -> exactly the two half Crops
     shuffle_units_.clear();
     for (size_t ci = 0; ci < layers_.size(); ++ci) {
@@ -2257,6 +2371,7 @@ void Net::plan_fused_quantize() const {
         if (u.second.conv >= 0) in_other_launch[u.second.conv] = 1;
     for (auto& u : shuffle_units_)
         if (u.second.next >= 0 && in_other_launch[u.second.next]) u.second.next = -1;
+    for (auto it = next_units_.begin(); it != next_units_.end();) it = in_other_launch[it->second] ? next_units_.erase(it) : std::next(it);
     // Inverted-residual blocks: 1x1 (int8 result) -> depthwise (int8 result) -> 1x1, each blob with one reader
     block_units_.clear();
     for (size_t li = 0; li < layers_.size(); ++li) {
@@ -2373,6 +2488,8 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
     if (u.concat >= 0 && !blobs[u.shortcut].defined()) {
         // the sum straight from the two blobs that the Concat would copy
         const int p0 = layers_[u.concat]->bottoms[0], p1 = layers_[u.concat]->bottoms[1];
+        const int behind = forward_dwpw_unit(u.conv, u.eltwise, p0, p1, blobs, opt);
+        if (behind <= 0) return behind;
         const int made = forward_inputs(u.conv, {p0, p1, conv->bottoms[0]}, blobs, opt);
         if (made) return made;
         const int rc = conv->forward_residual_concat(blobs[conv->bottoms[0]], blobs[p0], blobs[p1], e->fuse_scale, e->fuse_round, sum, opt,
@@ -2385,6 +2502,10 @@ int Net::forward_residual_unit(const ResidualUnit& u, std::vector<Tensor>& blobs
                     if (blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
             return 0;
         }
+    }
+    if (u.concat < 0 || blobs[u.shortcut].defined()) {
+        const int behind = forward_dwpw_unit(u.conv, u.eltwise, u.shortcut, -1, blobs, opt);
+        if (behind <= 0) return behind;
     }
     const int made = forward_inputs(u.conv, {u.shortcut, conv->bottoms[0]}, blobs, opt);
     if (made) return made;
@@ -2416,13 +2537,37 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
     const int other = layers_[u.concat]->bottoms[1 - u.conv_k], in_blob = conv->bottoms[0];
     const int block = block_saves_launches(u.conv, blobs, opt);
     if (block) return block;
-    const int made = forward_inputs(u.conv, {other, in_blob}, blobs, opt);
-    if (made) return made;
     const bool joined = u.crop_lo < 0;
     Tensor first, second;
     const int last = joined ? layers_[u.shuffle]->tops[0] : layers_[u.crop_hi]->tops[0];
-    const bool int8_only = u.hi_only && opt.wanted && !(*opt.wanted)[last];
-    if (!joined && int8_only && u.next >= 0 && opt.asked != last) {
+    const bool int8_only = u.hi_only && opt.wanted && !(*opt.wanted)[last], with_next = !joined && int8_only && u.next >= 0 && opt.asked != last;
+    if (const ConvolutionLayer* d = front_of(u.conv, blobs, opt)) {
+        // with the depthwise layer in front, and with the layer behind where that is a launch or that pair is none
+        const int x = d->bottoms[0], made = forward_inputs(u.conv, {other, x}, blobs, opt);
+        if (made) return made;
+        int rc = 1;
+        for (int k = with_next && !blobs[layers_[u.next]->tops[0]].defined() && !begins_block(u.next, blobs[x], d) ? 0 : 1; k < 2 && rc > 0; ++k) {
+            ConvolutionLayer::DwPw e;
+            e.next = k ? nullptr : static_cast<const ConvolutionLayer*>(layers_[u.next]);
+            e.other = &blobs[other], e.other_odd = u.conv_k == 0, e.joined = joined, e.int8_only = int8_only, e.q_scale = u.hi_scale, e.q_round = u.hi_round;
+            rc = ConvolutionLayer::forward_dwpw(d, conv, blobs[x], e, opt);
+            if (rc < 0) return rc;
+            if (rc == 0 && joined) blobs[layers_[u.shuffle]->tops[0]] = e.first;
+            if (rc == 0 && !joined) blobs[layers_[u.crop_lo]->tops[0]] = e.first;
+            if (rc == 0 && !joined && !e.next) blobs[layers_[u.crop_hi]->tops[0]] = e.second;
+            if (rc == 0 && e.next) blobs[e.next->tops[0]] = e.behind;
+            if (rc > 0 && !k) break;
+        }
+        if (rc == 0) {
+            if (opt.lightmode)
+                for (int b : {other, x})
+                    if (blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+            return 0;
+        }
+    }
+    const int made = forward_inputs(u.conv, {other, in_blob}, blobs, opt);
+    if (made) return made;
+    if (with_next) {
         const int rc = forward_pair_unit(u.conv, u.next, &u, blobs, opt);
         if (rc <= 0) return rc;
     }
@@ -2441,6 +2586,61 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
     return 0;
 }
 
+// The depthwise layer whose result the pointwise layer alone reads, if that may be left out: nobody has computed it or asked for it.
+const ConvolutionLayer* Net::front_of(int pointwise, const std::vector<Tensor>& blobs, const NetOption& opt) const {
+    const auto f = front_units_.find(pointwise);
+    if (f == front_units_.end()) return nullptr;
+    const int b = layers_[pointwise]->bottoms[0];
+    return blobs[b].defined() || opt.asked == b || (opt.wanted && (*opt.wanted)[b]) ? nullptr : static_cast<const ConvolutionLayer*>(layers_[f->second]);
+}
+
+// Whether the layer is the first of an inverted-residual block that runs in fewer launches than its layers on the blob x, or (d) on what
+// that depthwise layer makes of x.
+bool Net::begins_block(int li, const Tensor& x, const ConvolutionLayer* d) const {
+    if (x.dim() != 4) return false;
+    int h = (int)x.size(2), w = (int)x.size(3);
+    if (d) {
+        h = (h + 2 * d->padding_height - d->dilation_height * (d->kernel_height - 1) - 1) / d->stride_height + 1;
+        w = (w + 2 * d->padding_width - d->dilation_width * (d->kernel_width - 1) - 1) / d->stride_width + 1;
+    }
+    for (const auto& bu : block_units_)
+        if (bu.second.expand == li &&
+            ConvolutionLayer::block_launches(static_cast<const ConvolutionLayer*>(layers_[li]), static_cast<const ConvolutionLayer*>(layers_[bu.second.depthwise]),
+                                             static_cast<const ConvolutionLayer*>(layers_[bu.second.project]), (int)x.size(0), h, w) < 3)
+            return true;
+    return false;
+}
+
+// A pointwise layer and the depthwise one in front of it in one launch (ConvolutionLayer::forward_dwpw), with the sum behind it where
+// out_layer is that (shortcut, part1: its addend, or the parts of it; -1: none) and with the pointwise layer that reads the quantized
+// result. Returns 1 when the layers or the blobs at hand do not allow it.
+int Net::forward_dwpw_unit(int pointwise, int out_layer, int shortcut, int part1, std::vector<Tensor>& blobs, const NetOption& opt) const {
+    const ConvolutionLayer* const d = front_of(pointwise, blobs, opt);
+    if (!d) return 1;
+    const auto* const p = static_cast<const ConvolutionLayer*>(layers_[pointwise]);  // (as the end of a block, the callers have tried it)
+    const Layer* const e = layers_[out_layer];
+    const int x = d->bottoms[0], made = forward_inputs(pointwise, {shortcut, part1, x}, blobs, opt);
+    if (made) return made;
+    const auto next = part1 < 0 ? next_units_.find(out_layer) : next_units_.end();
+    const bool with_next = next != next_units_.end() && !blobs[layers_[next->second]->tops[0]].defined() && !begins_block(next->second, blobs[x], d);
+    for (int k = with_next ? 0 : 1; k < 2; ++k) {
+        ConvolutionLayer::DwPw u;
+        u.next = k ? nullptr : static_cast<const ConvolutionLayer*>(layers_[next->second]);
+        u.shortcut = shortcut >= 0 ? &blobs[shortcut] : nullptr, u.part1 = part1 >= 0 ? &blobs[part1] : nullptr;
+        u.q_scale = e->fuse_scale, u.q_round = e->fuse_round, u.int8_only = e->int8_only(opt);
+        const int rc = ConvolutionLayer::forward_dwpw(d, p, blobs[x], u, opt);
+        if (rc < 0) return rc;
+        if (rc > 0) continue;
+        if (u.out.defined()) blobs[e->tops[0]] = u.out;
+        if (u.next) blobs[u.next->tops[0]] = u.behind;
+        if (opt.lightmode)
+            for (int b : {shortcut, part1, x})
+                if (b >= 0 && blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+        return 0;
+    }
+    return 1;
+}
+
 // Two pointwise layers in one launch (ConvolutionLayer::forward_pair), with `u` across the end of that ShuffleNetV2 unit, whose inputs
 // are there. Returns 1 when the layers or the blobs at hand do not allow it, or when the second is the first of an inverted-residual
 // block that runs in fewer launches than its layers.
@@ -2450,16 +2650,25 @@ int Net::forward_pair_unit(int first, int second, const ShuffleUnit* u, std::vec
     if (blobs[top_blob].defined() || (opt.wanted && (*opt.wanted)[a->tops[0]])) return 1;
     const int block = block_saves_launches(first, blobs, opt);
     if (block) return block;
+    if (const ConvolutionLayer* d = u ? nullptr : front_of(first, blobs, opt)) {
+        const int in = d->bottoms[0], made = forward_inputs(first, {in}, blobs, opt);
+        if (made) return made;
+        if (!begins_block(second, blobs[in], d)) {
+            ConvolutionLayer::DwPw e;
+            e.next = b;
+            const int rc = ConvolutionLayer::forward_dwpw(d, a, blobs[in], e, opt);
+            if (rc < 0) return rc;
+            if (rc == 0) {
+                blobs[top_blob] = e.behind;
+                if (opt.lightmode && blobs_[in].consumers.size() == 1) blobs[in] = Tensor();
+                return 0;
+            }
+        }
+    }
     const int made = forward_inputs(first, {in_blob}, blobs, opt);
     if (made) return made;
     const Tensor& x = blobs[in_blob];
-    if (x.dim() != 4) return 1;
-    for (const auto& bu : block_units_)
-        if (bu.second.expand == second &&
-            ConvolutionLayer::block_launches(b, static_cast<const ConvolutionLayer*>(layers_[bu.second.depthwise]),
-                                             static_cast<const ConvolutionLayer*>(layers_[bu.second.project]), (int)x.size(0), (int)x.size(2),
-                                             (int)x.size(3)) < 3)
-            return 1;
+    if (x.dim() != 4 || begins_block(second, x, nullptr)) return 1;
     const int other = u ? layers_[u->concat]->bottoms[1 - u->conv_k] : -1;
     Tensor lo, top;
     const int rc = ConvolutionLayer::forward_pair(a, b, x, u ? &blobs[other] : nullptr, u && u->conv_k == 0, lo, top, opt);

@@ -266,6 +266,18 @@ public:
     // other half, `top` the second layer's result. Returns 1, and does nothing, when that is not one launch here.
     static int forward_pair(const ConvolutionLayer* first, const ConvolutionLayer* second, const Tensor& bottom_blob, const Tensor* other,
                             bool other_odd, Tensor& first_half, Tensor& top, const NetOption& opt);
+    // A depthwise layer, the pointwise layer that alone reads its int8 result and, where there is one, the pointwise layer `next` behind
+    // that in one launch (otter_hip_conv_dwpw_forward). What the pointwise layer's result meets: a shortcut, the two parts of one, or
+    // `other` in a ChannelShuffle(2); q_scale, q_round: the quantization that its readers agree on (next's, where there is a next).
+    struct DwPw {
+        const ConvolutionLayer* next = nullptr;
+        const Tensor *shortcut = nullptr, *part1 = nullptr, *other = nullptr;
+        bool other_odd = false, joined = false, int8_only = false;
+        float q_scale = 0.f;
+        int q_round = 0;
+        Tensor out, first, second, behind;  // the result (a sum), a shuffle's halves, next's result
+    };
+    static int forward_dwpw(const ConvolutionLayer* depthwise, const ConvolutionLayer* pointwise, const Tensor& bottom_blob, DwPw& u, const NetOption& opt);
     // forward_residual where the shortcut is the concatenation of two blobs (otter_hip_conv_forward_residual_concat)
     int forward_residual_concat(const Tensor& bottom_blob, const Tensor& part0, const Tensor& part1, float q_scale, int q_round,
                                 Tensor& sum, const NetOption& opt, bool int8_only) const;
@@ -395,6 +407,13 @@ private:
     mutable std::map<int, ShuffleUnit> shuffle_units_;
     // pointwise layers that alone read another one's int8 result: the reader's index -> the other's
     mutable std::map<int, int> pair_units_;
+    // pointwise layers that alone read a depthwise layer's int8 result: the reader's index -> the other's
+    mutable std::map<int, int> front_units_;
+    // layers with an fp32 blob that one pointwise int8 convolution reads quantized: the layer's index -> the convolution's
+    mutable std::map<int, int> next_units_;
+    const ConvolutionLayer* front_of(int pointwise, const std::vector<Tensor>& blobs, const NetOption& opt) const;
+    bool begins_block(int li, const Tensor& x, const ConvolutionLayer* d) const;
+    int forward_dwpw_unit(int pointwise, int out_layer, int shortcut, int part1, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_inputs(int li, const int* first, const int* last, std::vector<Tensor>& blobs, const NetOption& opt) const;
     int forward_inputs(int li, std::initializer_list<int> needed, std::vector<Tensor>& blobs, const NetOption& opt) const {
         return forward_inputs(li, needed.begin(), needed.end(), blobs, opt);

@@ -160,6 +160,28 @@ int otter_hip_conv_pair_forward(const otter_hip_conv_t* a, const otter_hip_conv_
         put(out, conv(b, r));
     });
 }
+int otter_hip_conv_dwpw_launches(const otter_hip_conv_t*, const otter_hip_conv_t*, int, int, int, const otter_hip_conv_end* e, int) {
+    return on(e->next ? "dwpw_next" : "dwpw") ? 1 : 2;
+}
+int otter_hip_conv_dwpw_forward(const otter_hip_conv_t* d, const otter_hip_conv_t* p, const void* in, int, int, int, const otter_hip_conv_end* e, void* out,
+                                int, void* s) {
+    const otter_hip_conv_end end = *e;
+    return launched(end.next ? "dwpw_next" : "dwpw", s, [=] {
+        std::string r = conv(p, conv(d, at(in)));
+        if (end.residual) r = sum(r, end.residual1 ? cat2(at(end.residual), at(end.residual1)) : at(end.residual));
+        if (end.other) {
+            const std::string o = at(end.other), sh = shuffle(end.other_odd ? cat2(r, o) : cat2(o, r));
+            if (end.joined) put(end.first_half, sh), put(end.first_half_q, q(sh));
+            else put(end.first_half, half(sh, 0)), put(end.second_half, half(sh, 1)), put(end.second_half_q, q(half(sh, 1)));
+            r = half(sh, 1);
+        } else if (end.next) {
+            put(end.sum, r);
+        } else {
+            put(out, r), put(end.out_q, q(r));
+        }
+        if (end.next) put(out, conv(end.next, r));
+    });
+}
 int otter_hip_conv_avgpool_launches(const otter_hip_conv_t*, int, int, int, int) { return on("avgpool") ? 1 : 2; }
 int otter_hip_conv_forward_avgpool(const otter_hip_conv_t* h, const void* in, int, int, int, int, float* out, void*, size_t, void* s) {
     return launched("avgpool", s, [=] { put(out, "mean(" + conv(h, at(in)) + ")"); });

@@ -1,0 +1,148 @@
+"""otter_hip_conv_dwpw_forward: a depthwise layer, the pointwise layer behind it and the one behind that in one launch. The results must be,
+bit for bit, what the layers give one by one through the calls for what their ends carry."""
+import numpy as np
+import pytest
+
+from gpu_util import host_scale_in
+from tensor_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # C, kernel, stride, pad, dilation, act of the depthwise layer, K, K2, N, H, W
+    (88, 3, 1, 1, 1, 0, 88, 88, 2, 13, 13),       # an odd count of octets, pairs that are no multiple of the waves
+    (176, 3, 2, 1, 1, 0, 176, 40, 2, 26, 26),
+    (384, 3, 1, 1, 1, 3, 64, 384, 1, 14, 14),     # six reduction steps: two rounds of weights; more pairs behind than in front
+    (960, 3, 1, 1, 1, 1, 160, 960, 1, 7, 7),      # the longest reduction; 49 pixels an image
+    (32, 3, 1, 1, 1, 3, 16, 96, 1, 20, 31),       # half a pair: seven of eight waves begin with the second layer
+    (8, 3, 1, 0, 1, 2, 8, 8, 3, 3, 3),            # one pixel an image, no padding
+    (24, 3, 2, 0, 2, 2, 40, 24, 2, 9, 12),        # dilation, the window off the image's end; channels past the last ones
+    (64, 3, 3, 2, 1, 2, 264, 72, 1, 11, 10),      # more padding than the window needs, a stride of three
+    (128, 5, 1, 2, 1, 2, 128, 112, 2, 13, 13),
+    (128, 5, 2, 2, 1, 2, 128, 128, 1, 26, 27),
+    (40, 5, 1, 1, 2, 0, 24, 8, 1, 12, 9),
+]
+
+
+def weights(rng, K, C, k):
+    return rng.integers(-127, 128, (K, C, k, k)).astype(np.int8), rng.uniform(40, 400, K).astype(np.float32) * np.float32(np.sqrt(C * k * k))
+
+
+def layer(hip, rng, C, K, act, f32, half=capi.ROUND_SSE):
+    w, ws = weights(rng, K, C, 1)
+    return hip.conv(wq=w, scale_in=host_scale_in(ws, 31.0), bias=rng.normal(0, 0.4, K).astype(np.float32), in_scale=31.0,
+                    out_scale=None if f32 else [23.0], act=act, act_p0=0.1, out_kind=capi.OUT_F32 if f32 else capi.OUT_I8, out_round=half)
+
+
+def depthwise(hip, rng, C, k, stride, pad, dil, act, half=capi.ROUND_SSE):
+    w, ws = weights(rng, C, 1, k)
+    return hip.conv(wq=w, scale_in=host_scale_in(ws, 29.0), bias=rng.normal(0, 0.4, C).astype(np.float32), in_scale=29.0, out_scale=[37.0], act=act,
+                    act_p0=0.2, groups=C, stride=(stride, stride), pad=(pad, pad), dil=(dil, dil), out_kind=capi.OUT_I8, out_round=half)
+
+
+def forms(k, last):
+    """(name, fields of the end beside the blobs) that run with this window, without and with a layer behind the pointwise one"""
+    shuffles = [("shuffle", dict(odd=odd, layout=layout)) for odd, layout in ((0, capi.F32_P8), (1, capi.F32_P4))]
+    if last:
+        return [("i8", {})] + ([("sum", {}), ("f32", {}), ("wanted", {})] + shuffles if k == 3 else [])
+    return [("i8", {}), ("f32", {}), ("twin", {}), ("sum", {}), ("parts", {})] + (shuffles + [("joined", dict(odd=1, layout=capi.F32_P8))] if k == 3 else [])
+
+
+def one_and_two(hip, rng, form, how, dw, pw, nx, x, n, h, w):
+    """(the launch's results, those of the layers one by one)"""
+    K, (oh, ow) = pw.K, dw.out_hw(h, w)
+    count = n * K * oh * ow
+    blob = lambda c=K: hip.to_device(rng.normal(0, 2, n * c * oh * ow).astype(np.float32))
+    new = lambda dtype, k=1: hip.empty(k * count, dtype).fill_(77)
+    q = dict(q_scale=19.0, q_round_mode=capi.ROUND_EXACT if K % 16 else capi.ROUND_SSE)
+    run = lambda **end: hip.conv_dwpw(dw, pw, x, n, h, w, next=nx, **end)
+    force = dw.force
+    dw.set_tile(0, 0)
+    mid = dw.forward(x, capi.I8_P8, n, h, w, capi.I8_P8)
+    dw.set_tile(*force)
+    then = lambda t: [nx.forward(t, capi.I8_P8, n, oh, ow, hip._packed_out(nx))] if nx else []
+    if form == "i8":
+        t = pw.forward(mid, capi.I8_P8, n, oh, ow, capi.I8_P8)
+        return [run()], then(t) if nx else [t]
+    if form in ("f32", "twin", "wanted"):
+        f, t = pw.forward_twin(mid, capi.I8_P8, n, oh, ow, q["q_scale"], q["q_round_mode"])
+        if nx:
+            s = new(np.float32) if form == "wanted" else None
+            return [run(sum=s, **q)] + [s] * (form == "wanted"), then(t) + [f] * (form == "wanted")
+        if form == "f32":
+            return [run()], [f]
+        o, only = new(np.int8), new(np.int8)
+        got = run(out_q=o, **q)
+        hip.conv_dwpw(dw, pw, x, n, h, w, wants_out=False, out_q=only, **q)
+        return [got, o, only], [f, t, t]
+    if form == "sum":
+        r = blob()
+        f, t = pw.forward_residual(mid, capi.I8_P8, n, oh, ow, r, q["q_scale"], q["q_round_mode"])
+        if nx:
+            s = new(np.float32)
+            return [run(residual=r, sum=s, **q), s], then(t) + [f]
+        o = new(np.int8)
+        return [run(residual=r, out_q=o, **q), o, run(residual=r)], [f, t, f]
+    if form == "parts":
+        c0 = max(8, K // 16 * 8) if K > 8 else 0
+        if not c0:
+            return [], []
+        a, b, o = blob(c0), blob(K - c0), new(np.int8)
+        f, t = pw.forward_residual_concat(mid, n, oh, ow, a, capi.F32_P4, c0, b, capi.F32_P8, **q)
+        return [run(residual=a, residual1=b, part0_channels=c0, part0_layout=capi.F32_P4, part1_layout=capi.F32_P8, out_q=o, **q), o], [f, t]
+    other = blob()
+    end = dict(other=other, other_layout=how["layout"], other_odd=how["odd"], **q)
+    t = pw.forward_shuffle(mid, n, oh, ow, other, how["layout"], bool(how["odd"]), form == "joined", q["q_scale"], q["q_round_mode"])
+    if form == "joined":
+        f, o = new(np.float32, 2), new(np.int8, 2)
+        hip.conv_dwpw(dw, pw, x, n, h, w, wants_out=False, joined=1, first_half=f, first_half_q=o, **end)
+        return [f, o], [t[0], t[2]]
+    lo = new(np.float32)
+    if nx:
+        return [run(first_half=lo, **end), lo], then(t[3]) + [t[0]]
+    hi, lq, hq = new(np.float32), new(np.int8), new(np.int8)
+    hip.conv_dwpw(dw, pw, x, n, h, w, wants_out=False, first_half=lo, second_half=hi, first_half_q=lq, second_half_q=hq, **end)
+    return [lo, hi, lq, hq], list(t)
+
+
+@pytest.mark.parametrize("C,k,stride,pad,dil,act,K,K2,n,h,w", CASES)
+def test_one_launch_equals_the_layers(hip, C, k, stride, pad, dil, act, K, K2, n, h, w):
+    rng = np.random.default_rng(C * 7 + K + w)
+    x = hip.to_device(rng.integers(-127, 128, n * C * h * w).astype(np.int8))
+    dw = depthwise(hip, rng, C, k, stride, pad, dil, act, capi.ROUND_EXACT if K % 16 else capi.ROUND_SSE)
+    for last in (None, "i8", "nonneg", "f32"):
+        nx = layer(hip, rng, K, K2, {"nonneg": 3, "i8": 2, "f32": 1, None: 0}[last], last == "f32") if last else None
+        for form, how in forms(k, last):
+            pw = layer(hip, rng, C, K, 2 if form != "sum" else 0, form != "i8")
+            for groups in (1, 2, 4, 8):  # of 16 pixels
+                if 16 * groups * (C + 160 + (K + 160 if nx else 0)) > 60000:
+                    continue
+                dw.force = (-12, groups)
+                dw.set_tile(-12, groups)
+                got, want = one_and_two(hip, rng, form, how, dw, pw, nx, x, n, h, w)
+                hip.torch.cuda.synchronize()
+                assert len(got) == len(want)
+                for i, (g, v) in enumerate(zip(got, want)):
+                    assert hip.torch.equal(g, v), (last, form, how, groups, i)
+            pw.close()
+
+
+def test_what_is_refused(hip):
+    rng = np.random.default_rng(3)
+    n, h, w = 2, 6, 6
+    x = hip.empty(n * 64 * h * w, np.int8)
+    dw = depthwise(hip, rng, 64, 3, 1, 1, 1, 0)
+    dw.set_tile(-12, 0)
+    i8, f32, odd, clipped = (layer(hip, rng, 64, K, act, f) for K, act, f in ((64, 0, False), (64, 0, True), (60, 0, True), (64, 1, False)))
+    r, b = hip.empty(n * 64 * h * w, np.float32), hip.empty(n * 64 * h * w, np.int8)
+    other = dict(other=r, other_layout=capi.F32_P8, first_half=r.clone(), q_scale=1.0)
+    assert hip.conv_dwpw_launches(dw, i8, n, h, w) == 1 and hip.conv_dwpw_launches(dw, f32, n, h, w, next=i8, **other) == 1
+    assert hip.conv_dwpw_launches(dw, clipped, n, h, w) == 2  # (its clamp is not among this launch's ends)
+    assert hip.conv_dwpw_launches(dw, odd, n, h, w) == 1      # (Float4 alone)
+    for first, second, end in ((i8, i8, {}), (dw, dw, {}), (dw, i8, dict(residual=r)), (dw, i8, other), (dw, i8, dict(out_q=b)), (dw, odd, dict(out_q=b, q_scale=1.0)),
+                               (dw, odd, dict(next=i8)), (dw, f32, dict(next=i8, out_q=b)), (dw, f32, dict(sum=r)), (dw, f32, dict(residual1=r)),
+                               (dw, f32, dict(next=i8, q_round_mode=9)), (dw, f32, dict(other, residual=r)), (dw, f32, dict(other, first_half=None, next=i8)),
+                               (dw, f32, dict(other, joined=1, second_half=r)), (dw, f32, dict(other, other_layout=capi.F32)), (dw, clipped, {}),
+                               (dw, f32, dict(residual=r, residual1=r, part0_channels=60, part0_layout=capi.F32_P8, part1_layout=capi.F32_P8))):
+        with pytest.raises(capi.HipError):
+            hip.conv_dwpw(first, second, x, n, h, w, **end)

@@ -198,3 +198,79 @@ for own in (0, 1):
     s.close()
     g.net.close()
 """, program=True)
+
+
+BEHIND = r"""
+def residual_blocks(g):  # the sum of one block is read by the next one's first layer and by its sum
+    s = g.conv(1, "data")
+    for k in (2, 5):
+        s = g.sum("s%d" % k, s, g.conv(k + 2, g.conv(k + 1, g.conv(k, s, True), True, True)))
+    return g.mean("out", g.conv(8, s))
+def without_a_sum(g):  # an fp32 result that the next block's first layer and its sum read
+    s = g.conv(3, g.conv(2, g.conv(1, "data", True), True, True))
+    return g.sum("out", s, g.conv(6, g.conv(5, g.conv(4, s, True), True, True)))
+def head_of_three(g):
+    return g.conv(4, g.conv(3, g.conv(2, g.conv(1, "data", True), True, True), True))
+def two_readers(g):  # the depthwise result has another reader
+    d = g.conv(2, g.conv(1, "data", True), True, True)
+    return g.sum("out", g.conv(3, d), g.conv(4, d))
+MORE = [residual_blocks, without_a_sum, head_of_three, two_readers]
+def set_all(**kw):
+    for k, v in kw.items(): fake.fake_set(k.encode(), v)
+"""
+
+
+@pytest.mark.parametrize("light", [True, False])
+def test_depthwise_layers_in_the_launch_of_their_reader(tmp_path, light):
+    run(tmp_path, BEHIND + r"""
+seen = {}
+for form in (3, 1):
+    for join, pair, alone, behind in ((1, 1, 1, 1), (1, 1, 1, 0), (1, 1, 0, 1), (0, 1, 1, 1), (1, 0, 1, 0), (1, 1, 0, 0)):
+        set_all(form=form, join=join, pair=pair, dwpw=alone, dwpw_next=behind)
+        for tail in TAILS + MORE:
+            g = Graph(%s)
+            made = tail(g)
+            out = made[0] if isinstance(made, tuple) else made
+            where = (tail.__name__, form, join, pair, alone, behind)
+            g.ready()
+            s = g.net.session("data", blob(), out)
+            before, launches = ran(g), [fake.fake_count(k) for k in (b"dwpw", b"dwpw_next")]
+            s.run()
+            assert fetched(s) == g.expr[out], (where, fetched(s))
+            once = [b - a for a, b in zip(before, ran(g))]
+            if tail is pooled: del once[3]  # (nobody asks for that one)
+            assert max(once) == 1 and min(once) == 1, (where, once)
+            took = [fake.fake_count(k) - n for k, n in zip((b"dwpw", b"dwpw_next"), launches)]
+            assert (alone or not took[0]) and (behind or not took[1]), where
+            if form == 3 and join: seen[(tail.__name__, alone, behind)] = took
+            for _ in range(5):  # (recorded from the third on)
+                s.run()
+                assert fetched(s) == g.expr[out], where
+                assert expr_of(g.net.eval({"data": blob()}, out)) == g.expr[out], where
+            s.close()
+            g.net.close()
+assert seen["residual_blocks", 1, 1] == [1, 1] and seen["residual_blocks", 1, 0] == [2, 0], seen  # (the second block's sum has no such reader)
+assert seen["without_a_sum", 1, 1] == [1, 1] and seen["head_of_three", 1, 1] == [0, 1] and seen["next_unit", 1, 1][1] == 1, seen
+assert seen["two_readers", 1, 1] == [0, 0], seen
+""" % light)
+
+
+def test_what_is_inside_such_a_launch_is_there_when_asked_for(tmp_path):
+    run(tmp_path, BEHIND + r"""
+for form in (3, 1):
+    set_all(form=form)
+    for tail, asks in ((residual_blocks, ("c3", "c4", "s2", "c5", "c6", "s2,out", "c3,out", "out,c3", "c5,out", "out,s2")),
+                       (without_a_sum, ("c2", "c3", "c4", "c5", "c3,out", "c4,out", "c5,out", "out,c3")), (head_of_three, ("c2", "c3", "c2,c4", "c4,c3"))):
+        for ask in asks:
+            for light in (True, False) if ask.split(",")[0] not in ("out", asks[-1].split(",")[0]) else (False,):  # (light: a pass lets go of what it has read)
+                g = Graph(light)
+                tail(g)
+                g.ready()
+                s = g.net.session("data", blob(), ask)
+                for _ in range(5):
+                    s.run()
+                    got, want = fetched(s), g.expr[ask.split(",")[-1]]
+                    assert got in (want, "q(%s)" % want), (tail.__name__, ask, light, got)
+                s.close()
+                g.net.close()
+""")
