@@ -255,6 +255,15 @@ int otter_hip_conv_pair_launches(const otter_hip_conv_t* first, const otter_hip_
 int otter_hip_conv_pair_forward(const otter_hip_conv_t* first, const otter_hip_conv_t* second, const void* in, int n, int in_h, int in_w,
                                 const otter_hip_conv_tail* tail, void* out, int out_layout, void* stream);
 
+/* An image stem (3x3, stride 2, at most 4 channels straight from the unpacked blob) with an fp32 result and the max pooling (3x3, stride 2,
+ * padding 1, dilation 1, no ceil mode: Tensor/Pool.cpp) that alone reads it, one launch: the layer's own result is not made. pad_value:
+ * what a pooling tap outside the layer's result counts as (otter_hip_maxpool2d). out: Float8, out_q: the quantize_to_int8 of it (q_scale,
+ * q_round_mode), Byte8; either may be NULL. Needs scale_in >= 0 and finite constants, K % 8 == 0 and
+ * otter_hip_conv_maxpool_launches(...) == 1 (2: the layer and the pooling are separate calls). */
+int otter_hip_conv_maxpool_launches(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w);
+int otter_hip_conv_forward_maxpool(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w, float pad_value,
+                                   float* out, int8_t* out_q, float q_scale, int q_round_mode, void* stream);
+
 /* A depthwise int8 -> int8 layer and the pointwise layer that alone reads its result in one launch, and with `next` the pointwise layer
  * behind that as well. The results are those of the layers (and of the calls above for what their ends carry) one by one. What becomes of
  * the first pointwise layer's result; all zero: it goes to out (Byte8 or Float4, out_layout; K % 4 == 0):
@@ -418,7 +427,8 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * can run, tn = groups | split << 6 | pairs << 7 forcing the 16-pixel groups a wave owns (1, 2 or 4), whether the reduction is split
  * among the waves of a workgroup (1: over 64 input channels; 0: at most 256, and four groups only for a result without a sum, a twin
  * or a shuffle) and the pairs of 16 output channels a wave walks. tn = 0: all three automatic. tm == -12 on a depthwise layer:
- * otter_hip_conv_dwpw_launches says 1 wherever that launch can run, tn = 1, 2, 4 or 8 its groups of 16 pixels (0 = automatic). */
+ * otter_hip_conv_dwpw_launches says 1 wherever that launch can run, tn = 1, 2, 4 or 8 its groups of 16 pixels (0 = automatic). tm == -13
+ * on an image stem: tn pooled rows a workgroup in the launch with its max pooling (1, 2, 4; 0 = automatic). */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 
 /* Test hook with no counterpart in the reference: which of the launches of its family a dense or grouped layer takes on a packed

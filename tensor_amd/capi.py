@@ -87,7 +87,8 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_avgpool_launches", "otter_hip_conv_avgpool_workspace_bytes", "otter_hip_conv_forward_avgpool",
            "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
            "otter_hip_conv_forward_residual_concat", "otter_hip_conv_pair_launches", "otter_hip_conv_pair_forward",
-           "otter_hip_conv_dwpw_launches", "otter_hip_conv_dwpw_forward",
+           "otter_hip_conv_dwpw_launches", "otter_hip_conv_dwpw_forward", "otter_hip_conv_maxpool_launches",
+           "otter_hip_conv_forward_maxpool",
            "otter_hip_record_begin", "otter_hip_record_end", "otter_hip_record_launch", "otter_hip_record_destroy"]
 
 
@@ -488,6 +489,23 @@ class Conv:
             self.h, self.L.ptr(x), in_layout, n, h, w, self.L.ptr(out),
             self.L.ptr(workspace) if workspace is not None else None, C.c_size_t(ws_bytes), self.L.stream()))
         return out
+
+    def maxpool_launches(self, in_layout, n, h, w):
+        r = self.L.lib.otter_hip_conv_maxpool_launches(self.h, in_layout, n, h, w)
+        self.L._check(min(r, 0))
+        return r
+
+    def forward_maxpool(self, x, in_layout, n, h, w, pad_value=0.0, q_scale=None, q_round_mode=ROUND_SSE, whole=True):
+        """The layer and a 3x3 stride-2 max pooling behind it (otter_hip_conv_forward_maxpool). Returns (Float8 blob or None, its Byte8
+        quantization or None)."""
+        oh, ow = self.out_hw(h, w)
+        count = n * self.K * ((oh - 1) // 2 + 1) * ((ow - 1) // 2 + 1)
+        out = self.L.empty(count, np.float32) if whole else None
+        q = self.L.empty(count, np.int8) if q_scale is not None else None
+        self.L._check(self.L.lib.otter_hip_conv_forward_maxpool(
+            self.h, self.L.ptr(x), in_layout, n, h, w, C.c_float(pad_value), self.L.ptr(out) if whole else None,
+            self.L.ptr(q) if q is not None else None, C.c_float(q_scale or 0.0), q_round_mode, self.L.stream()))
+        return out, q
 
     def forward_static(self, x, in_layout, n, h, w, out_layout=None, out=None):
         """otter_hip_conv_forward_static: the workspace is the library's static device array (no allocation inside)."""

@@ -103,6 +103,7 @@ struct otter_hip_conv {
     int8_t* w_dwpw = nullptr;    // a byte per lane and tap of a depthwise 3x3 / 5x5 layer for the launch it shares with its pointwise reader
     int8_t* w_xdw = nullptr;     // MFMA operands of a pointwise int8 -> int8 layer for the launch it shares with its depthwise reader
     int32_t* blk_consts = nullptr; // the layer's constants (and depthwise 3x3 weights) as the fused block launch keeps them in LDS
+    bool monotone = true;        // scale_in >= 0, and scale_in and bias are finite: larger sums give no smaller results
     bool so_positive = true;     // every output scale is finite and > 0
     bool so_same = true;         // the output scales are all so_one
     float so_one = 1.f;
@@ -509,6 +510,7 @@ int otter_hip_conv_create(const otter_hip_conv_desc* desc, const int8_t* weight,
     h->depthwise = (C == g && g == K);
     // the kernels read the per-channel arrays up to the padded row count (of the last group, for a grouped layer)
     const int kpad = g > 1 ? K + 128 : igemm_padded_rows(K);
+    for (int i = 0; i < K; ++i) h->monotone = h->monotone && scale_in[i] >= 0.f && std::isfinite(scale_in[i]) && (!bias || std::isfinite(bias[i]));
     int rc = OTTER_HIP_OK;
     do {
         const size_t wcount = (size_t)K * (C / g) * maxk;
@@ -1841,6 +1843,39 @@ int otter_hip_conv_pair_forward(const otter_hip_conv_t* first, const otter_hip_c
     const float so[2] = {first->so_one, second->so_one};
     OHIP_CHECK(run_conv_pwpw((const int8_t*)in, w, so, out, a.g[0], a.ep[0], a.g[1], a.ep[1],
                              first->force_tm == -11 ? first->force_tn : 0, (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
+// ---- an image stem and the max pooling that alone reads it --------------------------------------------------------------------------
+
+static bool conv_maxpool_one_launch(const otter_hip_conv_t* h, int in_layout, const ConvGeom& g) {
+    return h->w_stem && (h->force_tm == 0 || h->force_tm == -13) && h->monotone && h->d.out_kind == OTTER_HIP_OUT_F32 &&
+           conv_stem_pool_applicable(g, make_epilogue(h, OTTER_HIP_F32_P4), in_layout);
+}
+
+int otter_hip_conv_maxpool_launches(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w) {
+    if (!h || !valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_maxpool_launches: bad argument");
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_maxpool_launches: empty output");
+    return conv_maxpool_one_launch(h, in_layout, g) ? 1 : 2;
+}
+
+int otter_hip_conv_forward_maxpool(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w, float pad_value,
+                                   float* out, int8_t* out_q, float q_scale, int q_round_mode, void* stream) {
+    if (!h || !in || (!out && !out_q)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_maxpool: null");
+    if (!valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1 || std::isnan(pad_value))
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_maxpool: bad argument");
+    if (out_q && q_round_mode != OTTER_HIP_ROUND_EXACT && q_round_mode != OTTER_HIP_ROUND_SSE)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_maxpool: unknown rounding mode");
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_maxpool: empty output");
+    if (!conv_maxpool_one_launch(h, in_layout, g))
+        return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_maxpool: not a single launch (otter_hip_conv_maxpool_launches)");
+    Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
+    ep.twin_scale = q_scale, ep.twin_half = q_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+    OHIP_CHECK(run_conv_stem_pool(in, layout_elem(in_layout) == 0, h->w_stem, out, out_q, g, ep, h->in_scale, h->d.in_round_mode, pad_value,
+                                  h->force_tm == -13 ? h->force_tn : 0, (hipStream_t)stream));
     return OTTER_HIP_OK;
 }
 

@@ -163,6 +163,10 @@ hipError_t run_inner_product(const float* x, const float* w, const float* b, flo
 size_t stem_packed_weight_bytes(int K);
 void stem_pack_weights(const int8_t* w, int K, int C, int8_t* dst);
 bool conv_stem_applicable(const ConvGeom& g, const Epilogue& ep, int in_layout);
+// a stride-2 stem with an fp32 result and the 3x3 stride-2 max pooling (padding 1) that alone reads it, one launch
+bool conv_stem_pool_applicable(const ConvGeom& g, const Epilogue& ep, int in_layout);
+hipError_t run_conv_stem_pool(const void* x, bool in_f32, const int8_t* wpk, float* out, int8_t* out_q, const ConvGeom& g, const Epilogue& ep,
+                              const float* in_scale, int in_round, float pad_value, int force, hipStream_t stream);
 hipError_t run_conv_stem(const void* x, bool in_f32, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep,
                          const float* in_scale, int in_round, hipStream_t stream);
 

@@ -184,7 +184,85 @@ struct StemPlan {
 };
 
 constexpr int STEM_UN = 8;        // 4-pixel units a thread has in flight while the strip is loaded
+constexpr int STEM_POOL_ROWS = 4;  // pooled rows per workgroup with the pooling behind it (2, 4 level from 16 images on, 8 slower below 64)
 constexpr int STEM_LDS_ROWS = 4;  // output rows per workgroup (measured: 2, 4, 8 within 5 % of each other at 224 x 224, 16 slower)
+
+// Input rows iy0 .. iy0 + RIN - 1 of an image, quantized, into the LDS lines of a strip, a load per unit of four pixels: fp32 rows of four
+// pixels and more (16-byte loads need 4-byte alignment; the last unit of a row of no whole units is loaded where it ends with the row and
+// moved down), int8 rows of whole, aligned units. A wave takes lines, 64 units of one at a time: row and channel of a line are scalar, what is outside the image lies
+// outside a descriptor and is zero, and a unit costs its quantization and little else (a thread per unit that works out its own row,
+// channel and column: 28 vector instructions more, as many as the quantization, and the loads behind conditions; the stem of 224x224 images on
+// one of them 6.6 us so, 5.6 now).
+template <bool IN_F32, int CT>
+__device__ __forceinline__ void stem_fill(unsigned* stem_lds, const void* __restrict__ x_, const ConvGeom& g, const StemPlan& p, size_t img_in, int iy0,
+                                          float qs, float half) {
+    constexpr unsigned E = IN_F32 ? 4 : 1, OUT = 0x80000000u;
+    const unsigned lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int C = CT ? CT : g.C, lines = p.RIN * C;
+    const unsigned plane = (unsigned)(g.H * g.W), bytes = (unsigned)C * plane * E;
+    const char* const image = static_cast<const char*>(x_) + img_in * E;
+    for (int d0 = 0; d0 < p.pitch_dw; d0 += 64) {
+        const int d = d0 + (int)lane, ix = 4 * (d - 1);
+        const int over = max(ix + 4 - g.W, 0);  // pixels of the unit past the row's end
+        const unsigned v = ix >= 0 && ix < g.W ? (unsigned)(ix - over) * E : OUT, down = 8u * (unsigned)(over & 3);
+        for (int l0 = wave; l0 < lines; l0 += 4 * STEM_UN) {
+            v4i raw[STEM_UN];
+#pragma unroll
+            for (int j = 0; j < STEM_UN; ++j) {
+                const int line = l0 + 4 * j, r = line / C, c = line - r * C, iy = iy0 + r;
+                const bool in = line < lines && iy >= 0 && iy < g.H;  // (uniform; a line that does not exist: a descriptor of no bytes)
+                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(image), 0, in ? (int)bytes : 0, 0x00020000);
+                const unsigned at = in ? ((unsigned)c * plane + (unsigned)iy * (unsigned)g.W) * E : 0u;
+                if constexpr (IN_F32) raw[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)v, (int)at, 0));
+                else raw[j][0] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)v, (int)at, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < STEM_UN; ++j) {
+                const int line = l0 + 4 * j;
+                if (line >= lines) break;  // (uniform)
+                const unsigned pk = IN_F32 ? (unsigned)quantize4(raw[j], qs, half) >> down : (unsigned)raw[j][0];
+                if (d < p.pitch_dw) stem_lds[line * p.pitch_dw + d] = pk;
+            }
+        }
+    }
+}
+
+// the same for any rows, a value at a time
+template <bool IN_F32>
+__device__ __forceinline__ void stem_fill_any(unsigned* stem_lds, const void* __restrict__ x_, const ConvGeom& g, const StemPlan& p, int C, size_t img_in,
+                                              int iy0, float qs, float half) {
+    const int tid = threadIdx.x;
+    const int total = p.RIN * C * p.pitch_dw;
+    const unsigned plane = (unsigned)(g.H * g.W);
+    for (int idx = tid; idx < total; idx += 256) {
+        // dword idx of the LDS image: line = idx / pitch, row = line / C (exact: the quotients' fractional
+        // parts stay 0.5 / divisor away from an integer, far more than the rounding of these products)
+        const int line = (int)(((float)idx + 0.5f) * p.inv_pitch);
+        const int d = idx - line * p.pitch_dw;
+        const int r = (int)(((float)line + 0.5f) * p.inv_c);
+        const int c = line - r * C;
+        const int iy = iy0 + r, ix = 4 * (d - 1);
+        const bool row_ok = iy >= 0 && iy < g.H;
+        const unsigned off0 = (unsigned)c * plane + (unsigned)min(max(iy, 0), g.H - 1) * (unsigned)g.W;
+        // every load from a clamped (always valid) address, so that all are in flight together; what lies outside
+        // the image is zeroed afterwards
+        v4i raw;
+        unsigned keep = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int ixe = ix + e;
+            const unsigned off = off0 + (unsigned)min(max(ixe, 0), g.W - 1);
+            if constexpr (IN_F32) raw[e] = __float_as_int(static_cast<const float*>(x_)[img_in + off]);
+            else raw[e] = static_cast<const int8_t*>(x_)[img_in + off];
+            if (row_ok && ixe >= 0 && ixe < g.W) keep |= 0xffu << (8 * e);
+        }
+        unsigned pk;
+        if constexpr (IN_F32) pk = (unsigned)quantize4(raw, qs, half);
+        else pk = (unsigned)(raw[0] & 0xff) | (unsigned)(raw[1] & 0xff) << 8 | (unsigned)(raw[2] & 0xff) << 16 | (unsigned)raw[3] << 24;
+        stem_lds[idx] = pk & keep;
+    }
+}
 
 // EPI: 0 = fp32 Float4 result, 1 = int8 Byte8, 2 = int8 Byte8 of a layer that clamps at zero with positive output
 // scales (the clamp applied to the rounded values, see epi8_quant_i8p8)
@@ -201,79 +279,11 @@ __global__ void __launch_bounds__(256) conv_stem3x3_lds_kernel(const void* __res
 
     // ---- the strip's input rows -> int8 lines in LDS
     const int oy0 = strip * p.R, iy0 = oy0 * S - g.ph;
-    const int total = p.RIN * C * p.pitch_dw;
-    const unsigned plane = (unsigned)(g.H * g.W);
-    const size_t img_in = (size_t)img * g.C * plane;
+    const size_t img_in = (size_t)img * g.C * (unsigned)(g.H * g.W);
     const float qs = IN_F32 ? in_scale[0] : 0.f;
     const float half = in_round == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
-    auto fill = [&](auto vec_tag) {
-        constexpr bool VEC = decltype(vec_tag)::value;  // rows of whole, aligned 4-pixel units: one load per unit
-        for (int base = 0; base < total; base += 256 * STEM_UN) {
-            v4i raw[STEM_UN];
-            unsigned keep[STEM_UN];
-#pragma unroll
-            for (int j = 0; j < STEM_UN; ++j) {
-                if (base + 256 * j + 64 * wave >= total) continue;  // (none of this wave's units exists)
-                // unit idx = dword idx of the LDS image: line = idx / pitch, row = line / C (exact: the quotients' fractional
-                // parts stay 0.5 / divisor away from an integer, far more than the rounding of these products)
-                const int idx = min(base + 256 * j + tid, total - 1);
-                const int line = (int)(((float)idx + 0.5f) * p.inv_pitch);
-                const int d = idx - line * p.pitch_dw;
-                const int r = (int)(((float)line + 0.5f) * p.inv_c);
-                const int c = line - r * C;
-                const int iy = iy0 + r, ix = 4 * (d - 1);
-                const bool row_ok = iy >= 0 && iy < g.H;
-                const unsigned off0 = (unsigned)c * plane + (unsigned)min(max(iy, 0), g.H - 1) * (unsigned)g.W;
-                // every load from a clamped (always valid) address, so that all are in flight together; what lies outside
-                // the image is zeroed afterwards
-                if constexpr (VEC) {
-                    const unsigned off = off0 + (unsigned)min(max(ix, 0), g.W - 4);
-                    if constexpr (IN_F32) raw[j] = *reinterpret_cast<const v4i*>(static_cast<const float*>(x_) + img_in + off);
-                    else raw[j][0] = *reinterpret_cast<const int*>(static_cast<const int8_t*>(x_) + img_in + off);
-                    keep[j] = row_ok && ix >= 0 && ix < g.W ? 0xffffffffu : 0u;
-                } else {
-                    unsigned k = 0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int ixe = ix + e;
-                        const unsigned off = off0 + (unsigned)min(max(ixe, 0), g.W - 1);
-                        if constexpr (IN_F32) raw[j][e] = __float_as_int(static_cast<const float*>(x_)[img_in + off]);
-                        else raw[j][e] = static_cast<const int8_t*>(x_)[img_in + off];
-                        if (row_ok && ixe >= 0 && ixe < g.W) k |= 0xffu << (8 * e);
-                    }
-                    keep[j] = k;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < STEM_UN; ++j) {
-                if (base + 256 * j + 64 * wave >= total) continue;
-                unsigned pk;
-                if constexpr (IN_F32) {
-                    int q[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float t = __fmul_rn(__int_as_float(raw[j][e]), qs);
-                        q[e] = (int)__fadd_rn(t, __builtin_copysignf(half, t));
-                    }
-                    const ohip_v2s top = {127, 127}, bot = {-127, -127};
-                    ohip_v2s lo = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(q[0], q[1]));
-                    ohip_v2s hi = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(q[2], q[3]));
-                    lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bot);
-                    hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bot);
-                    pk = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
-                } else if constexpr (VEC) {
-                    pk = (unsigned)raw[j][0];
-                } else {
-                    pk = (unsigned)(raw[j][0] & 0xff) | (unsigned)(raw[j][1] & 0xff) << 8 | (unsigned)(raw[j][2] & 0xff) << 16 |
-                         (unsigned)raw[j][3] << 24;
-                }
-                const int idx = base + 256 * j + tid;
-                if (idx < total) stem_lds[idx] = pk & keep[j];
-            }
-        }
-    };
-    if (p.vec) fill(std::true_type{});
-    else fill(std::false_type{});
+    if (p.vec) stem_fill<IN_F32, CT>(stem_lds, x_, g, p, img_in, iy0, qs, half);
+    else stem_fill_any<IN_F32>(stem_lds, x_, g, p, C, img_in, iy0, qs, half);
 
     // ---- this lane's weights and the constants of its channels 16*m + 4*kg + i (requested once the strip's loads have
     // been consumed, so that their registers are not held across them; they arrive while the workgroup meets at the barrier)
@@ -366,6 +376,122 @@ __global__ void __launch_bounds__(256) conv_stem3x3_lds_kernel(const void* __res
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------------
+// A stride-2 layer and the 3x3 stride-2 max pooling that alone reads its fp32 result
+// ---------------------------------------------------------------------------------------------------------------------
+
+// What the two cost as launches is the blob between them: the layer's result is four times the pooled one and fp32 (24 channels, 416x416
+// -> 208x208 -> 104x104, 16 images: 66 MB written and read, 24.4 + 19.4 us; its quantization for the layers behind 5.4 us more). As one launch
+// 17.0 us, for one image 5.9 (14.7 as three); the bytes it cannot do without take 8, the rest is the chain of a strip: rows in, barrier, windows. Dequantization, clamp and LeakyReLU are monotone where scale_in >= 0, rounding included: the largest of nine
+// results is the result of the largest sum, and a pooled value costs nine integer comparisons and one epilogue.
+//
+// A workgroup owns R pooled rows. A lane's pixel is a pooled one, and its three columns of the layer come from the same three LDS dwords
+// of a line (windows 2 pixels apart); a column or row outside the layer's result repeats the one beside it, and the window then also
+// counts pad_value. What is computed twice, the rows and columns that neighbouring windows share, is matrix work: 9 instructions of 16
+// cycles for 16 pixels x 16 channels.
+template <int MT, bool IN_F32, int CT>
+__global__ void __launch_bounds__(256) conv_stem_pool_kernel(const void* __restrict__ x_, const int8_t* __restrict__ wpk, float* __restrict__ out,
+                                                             int8_t* __restrict__ out_q, ConvGeom g, Epilogue ep, const float* __restrict__ in_scale,
+                                                             int in_round, StemPlan p, int POH, int POW, float pad_value) {
+    extern __shared__ unsigned stem_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, kg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int img = (int)div_by(blockIdx.x, p.by_strips), strip = (int)blockIdx.x - img * p.strips;
+    const int C = CT ? CT : g.C;
+    constexpr int NC = CT ? CT : STEM_LDS_MAX_C;
+    const int py0 = strip * p.R, r0 = 2 * py0 - 1;  // first pooled row; first row of the layer
+    {
+        const size_t img_in = (size_t)img * g.C * (unsigned)(g.H * g.W);
+        const float qs = IN_F32 ? in_scale[0] : 0.f;
+        const float half = in_round == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
+        if (p.vec) stem_fill<IN_F32, CT>(stem_lds, x_, g, p, img_in, 2 * r0 - g.ph, qs, half);
+        else stem_fill_any<IN_F32>(stem_lds, x_, g, p, C, img_in, 2 * r0 - g.ph, qs, half);
+    }
+    v4i a[MT];
+    float si[MT][4], bi[MT][4];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        a[m] = reinterpret_cast<const v4i*>(wpk)[m * 64 + lane];
+        const int ch = 16 * m + 4 * kg;
+        const v4i s4 = *reinterpret_cast<const v4i*>(ep.scale_in + ch), b4 = *reinterpret_cast<const v4i*>(ep.bias + ch);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) si[m][i] = __int_as_float(s4[i]), bi[m][i] = __int_as_float(b4[i]);
+    }
+    __syncthreads();
+
+    // a wave walks down a group of 16 columns, or a part of it where the groups are fewer than the waves: the layer's row that two windows
+    // share is computed once
+    const int rows = min(p.R, POH - py0);
+    const int parts = p.cgs >= 4 ? 1 : p.cgs >= 2 ? 2 : 4, per = (rows + parts - 1) / parts;
+    // the window of the layer's column 2 x - 1 + j starts at byte 4 x + 2 + 2 j - pw of a line
+    const unsigned shift[3] = {8u * ((2u - g.pw) & 3u), 8u * ((4u - g.pw) & 3u), 8u * ((6u - g.pw) & 3u)};
+    const bool first_aligned = g.pw == 0;  // the middle window: at dword x + 1, else at the end of dword x
+    const int POHW = POH * POW;
+    for (int it = wave; it < p.cgs * parts; it += 4) {
+        const int cg = it >> (parts >> 1), part = it - cg * parts, x = 16 * cg + n;  // (parts: 1, 2, 4)
+        const bool left = x == 0, right = 2 * x + 1 >= g.OW;
+        // the largest sums of the three columns of the layer's row r0 + row
+        auto across = [&](int row, v4i (&most)[MT]) {
+            const int r = min(2 * row + kg, p.RIN - 1);  // (kernel row 3 does not exist: its bytes meet zero weights)
+            const unsigned* line = stem_lds + r * C * p.pitch_dw + x;
+            v4i b[3] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const unsigned* l = line + (CT ? c : min(c, C - 1)) * p.pitch_dw;  // (absent channels meet zero weights too)
+                const unsigned d0 = l[0], d1 = l[1], d2 = l[2];
+                const int mid = (int)(first_aligned ? d1 : __builtin_amdgcn_alignbit(d1, d0, shift[1]));
+                b[1][c] = mid;
+                b[0][c] = left ? mid : (int)__builtin_amdgcn_alignbit(d1, d0, shift[0]);
+                b[2][c] = right ? mid : (int)__builtin_amdgcn_alignbit(d2, d1, shift[2]);
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                v4i acc[3];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[m], b[j], v4i{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) most[m][e] = max(max(acc[0][e], acc[1][e]), acc[2][e]);
+            }
+        };
+        v4i above[MT];
+        const int first = part * per, last = min(first + per, rows);
+        for (int orow = first; orow < last; ++orow) {
+            const int py = py0 + orow;
+            const bool top = py == 0, bottom = 2 * py + 1 >= g.OH;  // (uniform)
+            v4i middle[MT], below[MT], best[MT];
+            across(2 * orow + 1, middle);
+            across(bottom ? 2 * orow + 1 : 2 * orow + 2, below);
+            if (orow == first) across(top ? 2 * orow + 1 : 2 * orow, above);  // (uniform)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) best[m][e] = max(max(above[m][e], middle[m][e]), below[m][e]), above[m][e] = below[m][e];
+            const float pad = left || right || top || bottom ? pad_value : -__builtin_inff();
+            const unsigned pix = (unsigned)(py * POW + x);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const int ch0 = 16 * m + 4 * kg;  // D rows 4*kg .. 4*kg+3 of column n
+                v4i v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float t = __fmaf_rn((float)best[m][e], si[m][e], bi[m][e]);
+                    t = lrelu_or_not(ep, fminf(fmaxf(t, ep.act_lo), ep.act_hi));
+                    v[e] = __float_as_int(fmaxf(t, pad));
+                }
+                if (x >= POW || ch0 >= g.K) continue;
+                const size_t at = (((size_t)img * (g.K / 8) + ch0 / 8) * (size_t)POHW + pix) * 8 + (ch0 & 4);
+                if (out != nullptr) *reinterpret_cast<v4i*>(out + at) = v;
+                if (out_q != nullptr) *reinterpret_cast<int*>(out_q + at) = quantize4(v, ep.twin_scale, ep.twin_half);
+            }
+        }
+    }
+}
+
+// whether stem_fill takes the rows (its offsets inside an image are of 32 bits)
+static bool stem_vec(const void* x, bool in_f32, const ConvGeom& g) {
+    if ((size_t)g.C * g.H * g.W * (in_f32 ? 4 : 1) >= ((size_t)1 << 31)) return false;
+    return in_f32 ? g.W >= 4 && ((uintptr_t)x & 3) == 0 : g.W % 4 == 0 && ((uintptr_t)x & 3) == 0;
+}
 // rows per workgroup and the LDS image of a strip; false where even one output row's input does not fit 64 KB
 static bool stem_lds_plan(const ConvGeom& g, StemPlan* p, size_t* lds_bytes) {
     const int S = g.sh, cgs = (g.OW + 15) / 16;
@@ -400,6 +526,63 @@ bool conv_stem_applicable(const ConvGeom& g, const Epilogue& ep, int in_layout) 
     return false;
 }
 
+// the strip of R pooled rows; false where it does not fit 64 KB
+static bool stem_pool_plan(const ConvGeom& g, int R, int POH, int POW, StemPlan* p, size_t* lds_bytes) {
+    p->R = R, p->strips = (POH + R - 1) / R, p->cgs = (POW + 15) / 16, p->RIN = 4 * R + 3, p->vec = 0;
+    p->pitch_dw = std::max(16 * p->cgs + 2, (g.W + 3) / 4 + 1);
+    p->by_strips = fast_div((unsigned)p->strips), p->by_cgs = fast_div((unsigned)p->cgs);
+    p->inv_pitch = 1.0f / (float)p->pitch_dw, p->inv_c = 1.0f / (float)g.C;
+    *lds_bytes = (size_t)p->RIN * g.C * p->pitch_dw * 4;
+    return *lds_bytes <= 64 * 1024;
+}
+static int stem_pooled(int size) { return (size - 1) / 2 + 1; }  // (3x3, stride 2, padding 1)
+
+// (scale_in >= 0 and finite constants are the caller's to check: they are on the device)
+bool conv_stem_pool_applicable(const ConvGeom& g, const Epilogue& ep, int in_layout) {
+    if (!conv_stem_applicable(g, ep, in_layout) || g.C > STEM_LDS_MAX_C || g.sh != 2 || g.K % 8 || ep.out_kind != OTTER_HIP_OUT_F32) return false;
+    if (g.OH < 1 || g.OW < 1 || (size_t)g.N * g.K * g.OH * g.OW >= ((size_t)1 << 31)) return false;
+    StemPlan p;
+    size_t lds;
+    return stem_pool_plan(g, 1, stem_pooled(g.OH), stem_pooled(g.OW), &p, &lds);
+}
+
+template <int MT>
+static hipError_t launch_stem_pool(const void* x, bool in_f32, const int8_t* wpk, float* out, int8_t* out_q, const ConvGeom& g, const Epilogue& ep,
+                                   const float* in_scale, int in_round, float pad_value, const StemPlan& p, size_t lds, hipStream_t stream) {
+    const int POH = stem_pooled(g.OH), POW = stem_pooled(g.OW);
+    const dim3 grid((unsigned)((long)g.N * p.strips)), block(256);
+#define OHIP_STEM_P(FI_, CT_) \
+    launch((conv_stem_pool_kernel<MT, FI_, CT_>), grid, block, lds, stream, x, wpk, out, out_q, g, ep, in_scale, in_round, p, POH, POW, pad_value)
+    if (in_f32 && g.C == 3) OHIP_STEM_P(true, 3);
+    else if (in_f32) OHIP_STEM_P(true, 0);
+    else if (g.C == 3) OHIP_STEM_P(false, 3);
+    else OHIP_STEM_P(false, 0);
+#undef OHIP_STEM_P
+    return hipGetLastError();
+}
+
+// out (Float8), out_q (Byte8, quantized with ep.twin_scale): either may be null. force: pooled rows of a workgroup, 0 = automatic
+hipError_t run_conv_stem_pool(const void* x, bool in_f32, const int8_t* wpk, float* out, int8_t* out_q, const ConvGeom& g, const Epilogue& ep,
+                              const float* in_scale, int in_round, float pad_value, int force, hipStream_t stream) {
+    if (g.N == 0) return hipSuccess;
+    StemPlan p;
+    size_t lds = 0;
+    const int POH = stem_pooled(g.OH), POW = stem_pooled(g.OW);
+    int R = force ? force : STEM_POOL_ROWS;
+    // fewer rows where the workgroups would not fill the compute units: a row more is read for every strip
+    while (!force && R > 1 && (long)g.N * ((POH + R - 1) / R) < 512) R /= 2;
+    while (R > 1 && !stem_pool_plan(g, R, POH, POW, &p, &lds)) R /= 2;
+    if (!stem_pool_plan(g, R, POH, POW, &p, &lds) || (long)g.N * p.strips >= (1l << 31)) return hipErrorInvalidValue;
+    p.vec = stem_vec(x, in_f32, g);
+    switch ((g.K + 15) / 16) {
+    case 1: return launch_stem_pool<1>(x, in_f32, wpk, out, out_q, g, ep, in_scale, in_round, pad_value, p, lds, stream);
+    case 2: return launch_stem_pool<2>(x, in_f32, wpk, out, out_q, g, ep, in_scale, in_round, pad_value, p, lds, stream);
+    case 3: return launch_stem_pool<3>(x, in_f32, wpk, out, out_q, g, ep, in_scale, in_round, pad_value, p, lds, stream);
+    case 4: return launch_stem_pool<4>(x, in_f32, wpk, out, out_q, g, ep, in_scale, in_round, pad_value, p, lds, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 template <int MT>
 static hipError_t launch_stem_lds(const void* x, bool in_f32, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep,
                                   const float* in_scale, int in_round, hipStream_t stream) {
@@ -408,8 +591,7 @@ static hipError_t launch_stem_lds(const void* x, bool in_f32, const int8_t* wpk,
     if (!stem_lds_plan(g, &p, &lds)) return hipErrorInvalidValue;
     const long wgs = (long)g.N * p.strips;
     if (wgs >= (1l << 31)) return hipErrorInvalidValue;
-    // whole 4-pixel units at aligned addresses: one 16-byte (fp32) or 4-byte (int8) load per unit
-    p.vec = g.W % 4 == 0 && ((uintptr_t)x & (in_f32 ? 15 : 3)) == 0;
+    p.vec = stem_vec(x, in_f32, g);
     const int epi = ep.out_kind == OTTER_HIP_OUT_F32 ? 0 : pick_epilogue(ep, g.K) == EPI_I8_P8_NONNEG ? 2 : 1;
     const dim3 grid((unsigned)wgs), block(256);
 #define OHIP_STEM_L(EPI_, FI_)                                                                                          \

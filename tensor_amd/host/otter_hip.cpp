@@ -995,6 +995,37 @@ int ConvolutionLayer::forward_pair(const ConvolutionLayer* a, const ConvolutionL
     return 0;
 }
 
+int ConvolutionLayer::forward_maxpool(const Tensor& bottom, float pad_value, float q_scale, int q_round, Tensor& pooled, const NetOption& opt,
+                                      bool int8_only) const {
+    if (!handle_ || !int8_scale_term || int8_scale_term > 100 || force_out_layout >= 0 || !opt.use_packing_layout || out_channels % 8) return 1;
+    if (!bottom.defined() || bottom.dim() != 4 || bottom.channels() != in_channels) return 1;
+    const int layout = hip_layout_of(bottom.scalar_type());
+    const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3);
+    int oh = 0, ow = 0;
+    if (layout < 0 || otter_hip_conv_output_shape(handle_, H, W, &oh, &ow) || otter_hip_conv_maxpool_launches(handle_, layout, N, H, W) != 1) return 1;
+    try {
+        const std::vector<int64_t> sizes = {N, out_channels / 8, (oh - 1) / 2 + 1, (ow - 1) / 2 + 1};
+        Tensor q;
+        if (q_scale > 0.f) q = Tensor::empty_device(sizes, ScalarType::Byte8);
+        const bool no_f32 = int8_only && q.defined();
+        if (!no_f32) pooled = Tensor::empty_device(sizes, ScalarType::Float8);
+        const int rc = otter_hip_conv_forward_maxpool(handle_, bottom.device_ptr(), layout, N, H, W, pad_value,
+                                                      no_f32 ? nullptr : (float*)pooled.device_ptr(), q.defined() ? (int8_t*)q.device_ptr() : nullptr,
+                                                      q_scale, q_round, launch_stream());
+        if (rc) return rc;
+        if (q.defined()) q.mark_device_written();
+        if (no_f32) {
+            pooled = q;
+        } else {
+            pooled.mark_device_written();
+            if (q.defined()) pooled.attach_quantized(q, q_scale, q_round);
+        }
+    } catch (const Error&) {
+        return -100;
+    }
+    return 0;
+}
+
 int ConvolutionLayer::forward_dwpw(const ConvolutionLayer* d, const ConvolutionLayer* p, const Tensor& bottom_in, DwPw& u, const NetOption& opt) {
     for (const ConvolutionLayer* c : {d, p, u.next})
         if (c && (!c->handle_ || c->force_out_layout >= 0 || !c->int8_scale_term)) return 1;
@@ -1506,6 +1537,7 @@ public:
         return 0;
     }
     std::string type() const override { return "MaxPool"; }
+    bool halves() const { return kh_ == 3 && kw_ == 3 && sh_ == 2 && sw_ == 2 && ph_ == 1 && pw_ == 1 && dh_ == 1 && dw_ == 1 && !ceil_; }
 
 private:
     int kh_ = 1, kw_ = 1, sh_ = 1, sw_ = 1, ph_ = 0, pw_ = 0, dh_ = 1, dw_ = 1;
@@ -2094,6 +2126,25 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
         }
     }
     {
+        const auto unit = maxpool_units_.find(li);
+        // only when the convolution's own result has not been computed (or set by the caller) and nobody wants it
+        if (unit != maxpool_units_.end() && !blobs[layer->bottoms[0]].defined() && !(opt.wanted && (*opt.wanted)[layer->bottoms[0]])) {
+            const auto* conv = static_cast<const ConvolutionLayer*>(layers_[unit->second]);
+            const int b = conv->bottoms[0];
+            Tensor pooled;
+            int rc = forward_inputs(unit->second, {b}, blobs, opt);
+            if (rc == 0)
+                rc = conv->forward_maxpool(blobs[b], static_cast<const MaxPoolLayer*>(layer)->pad_value(conv->out_channels, opt), layer->fuse_scale,
+                                           layer->fuse_round, pooled, opt, layer->int8_only(opt));
+            if (rc < 0) return rc;
+            if (rc == 0) {
+                blobs[layer->tops[0]] = pooled;
+                if (opt.lightmode && blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+                return 0;
+            }
+        }
+    }
+    {
         const auto unit = residual_units_.find(li);
         // only when the convolution's own result has not been computed (or set by the caller)
         if (unit != residual_units_.end() && !blobs[layers_[unit->second.conv]->tops[0]].defined()) {
@@ -2270,6 +2321,16 @@ void Net::plan_fused_quantize() const {
         if (!pc || !pc->int8_scale_term || pc->int8_scale_term > 100 || pc->force_out_layout >= 0 || pc->bottoms.size() != 1) continue;
         if (blobs_[b].consumers.size() != 1) continue;
         pool_units_[(int)pi] = ci;
+    }
+    // Max poolings that alone read the fp32 result of an int8 convolution over an image
+    maxpool_units_.clear();
+    for (size_t pi = 0; pi < layers_.size(); ++pi) {
+        const auto* p = dynamic_cast<const MaxPoolLayer*>(layers_[pi]);
+        if (!p || !p->halves() || p->bottoms.size() != 1 || p->tops.size() != 1) continue;
+        const int b = p->bottoms[0], ci = blobs_[b].producer;
+        const auto* c = ci < 0 ? nullptr : dynamic_cast<const ConvolutionLayer*>(layers_[ci]);
+        if (!c || !c->of_library || !c->int8_scale_term || c->int8_scale_term > 100 || c->force_out_layout >= 0 || c->bottoms.size() != 1) continue;
+        if (blobs_[b].consumers.size() == 1 && c->in_channels <= 4) maxpool_units_[(int)pi] = ci;
     }
     // Pairs of pointwise layers, one reading the other's int8 result alone. (Not a program's own kind of convolution: its forward may do more.)
     auto sole_reader = [&](int blob) { return blobs_[blob].consumers.size() == 1 ? blobs_[blob].consumers[0] : -1; };

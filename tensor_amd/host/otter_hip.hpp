@@ -266,6 +266,8 @@ public:
     // other half, `top` the second layer's result. Returns 1, and does nothing, when that is not one launch here.
     static int forward_pair(const ConvolutionLayer* first, const ConvolutionLayer* second, const Tensor& bottom_blob, const Tensor* other,
                             bool other_odd, Tensor& first_half, Tensor& top, const NetOption& opt);
+    // An image stem and the 3x3 stride-2 max pooling behind it in one launch (otter_hip_conv_forward_maxpool)
+    int forward_maxpool(const Tensor& bottom_blob, float pad_value, float q_scale, int q_round, Tensor& pooled, const NetOption& opt, bool int8_only) const;
     // A depthwise layer, the pointwise layer that alone reads its int8 result and, where there is one, the pointwise layer `next` behind
     // that in one launch (otter_hip_conv_dwpw_forward). What the pointwise layer's result meets: a shortcut, the two parts of one, or
     // `other` in a ChannelShuffle(2); q_scale, q_round: the quantization that its readers agree on (next's, where there is a next).
@@ -407,6 +409,8 @@ private:
     mutable std::map<int, ShuffleUnit> shuffle_units_;
     // pointwise layers that alone read another one's int8 result: the reader's index -> the other's
     mutable std::map<int, int> pair_units_;
+    // max poolings (3x3, stride 2, padding 1) that alone read an int8 convolution's fp32 result: the pooling's index -> the convolution's
+    mutable std::map<int, int> maxpool_units_;
     // pointwise layers that alone read a depthwise layer's int8 result: the reader's index -> the other's
     mutable std::map<int, int> front_units_;
     // layers with an fp32 blob that one pointwise int8 convolution reads quantized: the layer's index -> the convolution's

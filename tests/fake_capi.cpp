@@ -182,6 +182,10 @@ int otter_hip_conv_dwpw_forward(const otter_hip_conv_t* d, const otter_hip_conv_
         if (end.next) put(out, conv(end.next, r));
     });
 }
+int otter_hip_conv_maxpool_launches(const otter_hip_conv_t*, int, int, int, int) { return on("stem_pool") ? 1 : 2; }
+int otter_hip_conv_forward_maxpool(const otter_hip_conv_t* h, const void* in, int, int, int, int, float, float* out, int8_t* oq, float, int, void* s) {
+    return launched("stem_pool", s, [=] { const std::string r = "maxpool(" + conv(h, at(in)) + ")"; put(out, r), put(oq, q(r)); });
+}
 int otter_hip_conv_avgpool_launches(const otter_hip_conv_t*, int, int, int, int) { return on("avgpool") ? 1 : 2; }
 int otter_hip_conv_forward_avgpool(const otter_hip_conv_t* h, const void* in, int, int, int, int, float* out, void*, size_t, void* s) {
     return launched("avgpool", s, [=] { put(out, "mean(" + conv(h, at(in)) + ")"); });
@@ -249,6 +253,9 @@ int otter_hip_shuffle2_split(const float* a, int, const float* b, int, int, int,
         const std::string sh = shuffle(cat2(at(a), at(b)));
         put(lo, half(sh, 0)), put(hi, half(sh, 1)), put(oq, q(half(sh, 1)));
     });
+}
+int otter_hip_maxpool2d(const float* src, int, int, int, int, int, int, int, int, int, int, int, int, int, int, int, float, float* dst, int, void* s) {
+    return launched("maxpool", s, [=] { put(dst, "maxpool(" + at(src) + ")"); });
 }
 // (the Crop layers of the tests take one half of their input)
 int otter_hip_copy_channels(const float* src, int, int, int c0, float* dst, int, int, int, int, int, int, int, void* s) {

@@ -274,3 +274,37 @@ for form in (3, 1):
                 s.close()
                 g.net.close()
 """)
+
+
+@pytest.mark.parametrize("light", [True, False])
+def test_a_max_pooling_in_the_launch_of_an_image_stem(tmp_path, light):
+    run(tmp_path, r"""
+CH3 = 3
+for on in (1, 0):
+    for ask in ("out", "pool", "c1", "pool,out", "c1,out", "out,c1"):
+        if %s and ask == "out,c1": continue  # (in light mode a pass lets go of what it has read)
+        fake.fake_set(b"stem_pool", on)
+        net = hostnet.Net(lightmode=%s)
+        net.add_layer(type="Input", name="data", batchsize=1, channel=3, height=16, width=16)
+        net.add_layer(type="Convolution", name="c1", input="data", out_channels=8, kernel=3, stride=2, padding=1, int8_scale_term=2)
+        net.add_layer(type="MaxPool", name="pool", input="c1", kernel=3, stride=2, padding=1)
+        net.add_layer(type="Convolution", name="c2", input="pool", out_channels=8, kernel=1, int8_scale_term=2)
+        net.add_layer(type="Convolution", name="c3", input="pool", out_channels=8, kernel=1, int8_scale_term=2)
+        net.add_layer(type="Eltwise", name="out", input="c2,c3")
+        net.compile()
+        net.set_conv("c1", np.full((8, 3, 3, 3), 1, np.int8), None, np.full(8, 50, np.float32), 20.0, 10.0)
+        for n in (2, 3): net.set_conv("c%%d" %% n, np.full((8, 8, 1, 1), n, np.int8), None, np.full(8, 50, np.float32), 20.0, 10.0)
+        x = np.zeros((1, 3, 16, 16), np.float32)
+        x.reshape(-1)[:2].view(np.int64)[0] = fake.fake_number(b"x")
+        expr = dict(c1="c1(x)", pool="maxpool(c1(x))")
+        expr["out"] = "sum(c2(%%s),c3(%%s))" %% (expr["pool"], expr["pool"])
+        s = net.session("data", x, ask)
+        launches = fake.fake_count(b"stem_pool")
+        for _ in range(5):
+            s.run()
+            got, want = expr_of(s.fetch((2 * 8 * 64,), np.float32)), expr[ask.split(",")[-1]]
+            assert got in (want, "q(%%s)" %% want), (on, ask, got)
+        assert (fake.fake_count(b"stem_pool") > launches) == (on and "c1" not in ask), (on, ask)
+        s.close()
+        net.close()
+""" % (light, light))
