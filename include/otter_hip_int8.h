@@ -272,7 +272,8 @@ int otter_hip_conv_forward_maxpool(const otter_hip_conv_t* handle, const void* i
  *   residual             Float4 addend of an fp32 result (otter_hip_conv_forward_residual); with residual1 the addend's first
  *                        part0_channels channels, residual1 the rest, each Float4 or Float8 (otter_hip_conv_forward_residual_concat; no next)
  *   out_q                the Byte8 quantization of the fp32 result beside it (no next); out may then be NULL
- *   other, ...           the shuffle of otter_hip_conv_forward_shuffle; out is not used without next, which reads the second half
+ *   other, ...           the shuffle of otter_hip_conv_forward_shuffle; out is not used without next, which reads the second half.
+ *                        first_float4: first_half is Float4 (not joined), which this launch writes and reads as `other` faster
  * in: Byte8. otter_hip_conv_dwpw_launches: 1 where the call runs and is the faster way, 2 where the layers are separate calls or
  * faster so; of the pointers, next apart, it only asks which are null. The call itself runs wherever it can. */
 typedef struct otter_hip_conv_end {
@@ -280,7 +281,7 @@ typedef struct otter_hip_conv_end {
     const float *residual, *residual1;
     int part0_channels, part0_layout, part1_layout;
     const float* other;
-    int other_layout, other_odd, joined;
+    int other_layout, other_odd, joined, first_float4;
     float *first_half, *second_half;
     int8_t *first_half_q, *second_half_q;
     float* sum;
@@ -427,7 +428,8 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * can run, tn = groups | split << 6 | pairs << 7 forcing the 16-pixel groups a wave owns (1, 2 or 4), whether the reduction is split
  * among the waves of a workgroup (1: over 64 input channels; 0: at most 256, and four groups only for a result without a sum, a twin
  * or a shuffle) and the pairs of 16 output channels a wave walks. tn = 0: all three automatic. tm == -12 on a depthwise layer:
- * otter_hip_conv_dwpw_launches says 1 wherever that launch can run, tn = 1, 2, 4 or 8 its groups of 16 pixels (0 = automatic). tm == -13
+ * otter_hip_conv_dwpw_launches says 1 wherever that launch can run, tn = 1, 2, 4 or 8 its groups of 16 pixels,
+ * + 16 with four waves to a workgroup (0 = automatic). tm == -13
  * on an image stem: tn pooled rows a workgroup in the launch with its max pooling (1, 2, 4; 0 = automatic). */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 

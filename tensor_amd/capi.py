@@ -121,7 +121,7 @@ class End(C.Structure):
     """otter_hip_conv_end: what otter_hip_conv_dwpw_forward does with the pointwise layer's result."""
     _fields_ = [("next", C.c_void_p), ("residual", C.c_void_p), ("residual1", C.c_void_p), ("part0_channels", C.c_int),
                 ("part0_layout", C.c_int), ("part1_layout", C.c_int), ("other", C.c_void_p), ("other_layout", C.c_int),
-                ("other_odd", C.c_int), ("joined", C.c_int), ("first_half", C.c_void_p), ("second_half", C.c_void_p),
+                ("other_odd", C.c_int), ("joined", C.c_int), ("first_float4", C.c_int), ("first_half", C.c_void_p), ("second_half", C.c_void_p),
                 ("first_half_q", C.c_void_p), ("second_half_q", C.c_void_p), ("sum", C.c_void_p), ("out_q", C.c_void_p),
                 ("q_scale", C.c_float), ("q_round_mode", C.c_int)]
 

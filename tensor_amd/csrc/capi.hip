@@ -1915,6 +1915,7 @@ static int dwpw_args(const char* who, const otter_hip_conv_t* d, const otter_hip
         if (t->residual || t->out_q || t->sum) return bad("a shuffle has no sum");
         if (t->other_layout != OTTER_HIP_F32_P4 && t->other_layout != OTTER_HIP_F32_P8) return bad("the other blob must be Float4 or Float8");
         if ((t->joined || nx) && (t->second_half || t->second_half_q)) return bad("the second half is not a blob here");
+        if (t->first_float4 && t->joined) return bad("a joined result is Float8");
         if (nx && (t->joined || !t->first_half || t->first_half_q)) return bad("in front of a layer the shuffle leaves its first half");
     }
     if (nx && t->out_q) return bad("the quantized result is the next layer's");
@@ -1943,7 +1944,7 @@ static int dwpw_args(const char* who, const otter_hip_conv_t* d, const otter_hip
         const size_t half = (size_t)K * a->g[1].OH * a->g[1].OW;  // elements of one half of one image
         ep.join = &a->ja;
         a->ja.other = t->other, a->ja.other_pack = layout_pack(t->other_layout), a->ja.other_odd = t->other_odd != 0;
-        a->ja.sh_image = t->joined ? 2 * half : half;
+        a->ja.sh_image = t->joined ? 2 * half : half, a->ja.sh_pack0 = t->first_float4 ? 4 : 8;
         a->ja.sh_out0 = t->first_half, a->ja.sh_q0 = t->first_half_q;
         a->ja.sh_out1 = t->joined ? (t->first_half ? t->first_half + half : nullptr) : t->second_half;
         a->ja.sh_q1 = t->joined ? (t->first_half_q ? t->first_half_q + half : nullptr) : t->second_half_q;

@@ -159,6 +159,7 @@ struct JoinArgs {
     float *sh_out0 = nullptr, *sh_out1 = nullptr;
     int8_t *sh_q0 = nullptr, *sh_q1 = nullptr;
     size_t sh_image = 0;
+    int sh_pack0 = 8;  // channels of an element of sh_out0: 8, or 4 (the launch behind a depthwise layer only)
 };
 
 // which epilogue code a kernel instance carries

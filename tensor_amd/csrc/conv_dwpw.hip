@@ -2,7 +2,7 @@
 // reads the int8 form of what the first leaves behind, where there is one (conv_pwpw.hip's pair, across a residual sum as well).
 //
 // What bounds these layers one by one is not bytes and not operations: a launch takes 2 us behind the one in front of it, then a chain of
-// memory latencies, and the blob between the layers is written and read back for nothing. Here a workgroup of eight waves owns 16 G
+// memory latencies, and the blob between the layers is written and read back for nothing. Here a workgroup of eight or four waves owns 16 G
 // pixels (G = 1, 2, 4, 8 groups of 16, a wave belongs to one) with all their channels:
 //  * The depthwise layer goes through the matrix cores, 16 channels x 16 pixels at a time: a B column is one output pixel, its 64
 //    reduction bytes are four taps of two channel octets, and the A operand holds each channel's weights at that channel's bytes and
@@ -25,7 +25,6 @@ namespace ohip {
 
 namespace {
 
-constexpr int DP_WAVES = 8;
 enum { DP_NONE = 3 };  // no second pointwise layer (KIND1, beside PP_I8, PP_NONNEG and PP_F32)
 
 struct DwPwArgs {
@@ -40,6 +39,7 @@ struct DwPwArgs {
     int sh, sw, ph, pw, dh, dw, C8;
     unsigned hw_s, ow_s;
     int lg, dw_lrelu, dw_nonneg;     // lg: log2 of the pixel groups
+    unsigned first_pack;             // channels of an element of a shuffle's first half
 };
 
 // the fp32 blob whose elements an epilogue reads
@@ -48,6 +48,11 @@ __device__ __forceinline__ const float* add_blob(const A& ja) {
     if constexpr (std::is_same_v<A, PwShuffle>) return ja.other;
     else if constexpr (std::is_same_v<A, NoJoin>) return nullptr;
     else return ja.residual;
+}
+template <class A>
+__device__ __forceinline__ unsigned sh_image(const A& ja) {
+    if constexpr (std::is_same_v<A, PwShuffle>) return ja.sh_image;
+    else return 0;
 }
 template <class A>
 __device__ __forceinline__ int ja_pack(const A& ja) {
@@ -78,13 +83,13 @@ void dwpw_pack_weights(const int8_t* w, int C, int ks, int8_t* dst) {
 // TAPS: 9 or 25. EPI: the first pointwise layer's epilogue: EPI_I8_P8; EPI_F32_P4_FUSED (with or without a residual and a twin; without
 // a second layer this is the plain fp32 result as well), EPI_F32_P4_PARTS, EPI_F32_SHUFFLE. KIND1: the second layer's result or DP_NONE.
 // out: the last layer's result; sum: with a second layer, the first one's fp32 result (null: not wanted).
-template <int TAPS, int EPI, int KIND1>
-__global__ void __launch_bounds__(64 * DP_WAVES) conv_dwpw_kernel(const int8_t* __restrict__ x, void* __restrict__ out, float* __restrict__ sum,
+template <int NW, int TAPS, int EPI, int KIND1>
+__global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __restrict__ x, void* __restrict__ out, float* __restrict__ sum,
                                                                   DwPwArgs pa, PwAdd<EPI> ja) {
     constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, I8 = EPI == EPI_I8_P8, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
     constexpr bool NEXT = KIND1 != DP_NONE;
     constexpr int KS = TAPS == 9 ? 3 : 5, M = (TAPS + 3) / 4, PK = TAPS == 9 ? 2 : 4;
-    constexpr int NW = DP_WAVES, SC = 4;
+    constexpr int SC = 4;
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     const unsigned tid = threadIdx.x, lane = tid & 63, q = lane >> 4, p = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane((int)tid >> 6);
@@ -177,12 +182,12 @@ __global__ void __launch_bounds__(64 * DP_WAVES) conv_dwpw_kernel(const int8_t* 
         // channel r = p's bytes in the operand: dword p / 4 of its octet's two pixels, if the lane's bytes are of that octet
         unsigned sel[2][4];
         {
-            const bool mine = (p >> 3) == (q >> 1);
-            const unsigned zero = 0x0c0c0c0cu, at = 8u * (p & 3);
+            // (byte 0x0c of a selector is zero; one byte more of the source is 1 << at further)
+            const bool mine = (p >> 3) == (q >> 1), upper = (p >> 2) & 1;
+            const unsigned zero = 0x0c0c0c0cu, at = 8u * (p & 3), one = 1u << at;
+            const unsigned low = mine && !upper ? one : 0u, high = mine && upper ? one : 0u;
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (unsigned b = 0; b < 4; ++b) sel[h][b] = mine && ((p >> 2) & 1) == (unsigned)h ? (zero & ~(0xffu << at)) | b << at : zero;
+            for (unsigned b = 0; b < 4; ++b) sel[0][b] = zero - 12u * low + b * low, sel[1][b] = zero - 12u * high + b * high;
         }
         const int pairs = ((int)C8 + 1) / 2;  // of octets
         const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.in_bytes), rw = rsrc(pa.dw_w, (unsigned)pairs * 256u * PK);
@@ -208,14 +213,14 @@ __global__ void __launch_bounds__(64 * DP_WAVES) conv_dwpw_kernel(const int8_t* 
         asm volatile("" ::: "memory");  // (in front of the others: the compiler would move them to the loop)
 
         // ---- constants into LDS: scale_in and bias of each layer (they are padded to whole pairs of tiles and more) ---------------------
-        // (an array a wave: six of them, the waves behind have none)
-        {
-            const unsigned d = wave >> 1;  // 0: the depthwise layer, 1, 2: the others
+        // (an array a wave: six of them)
+        for (int w = wave; w < (NEXT ? 6 : 4); w += NW) {
+            const unsigned d = w >> 1;  // 0: the depthwise layer, 1, 2: the others
             const float* const si = d == 0 ? pa.dw_scale_in : d == 1 ? l0.scale_in : l1.scale_in;
             const float* const bi = d == 0 ? pa.dw_bias : d == 1 ? l0.bias : l1.bias;
-            const unsigned quads = d == 0 ? Cd / 4 : d == 1 ? 8u * pairs0 : d == 2 ? 8u * pairs1 : 0u;
-            const __amdgpu_buffer_rsrc_t r = rsrc(wave & 1 ? bi : si, quads * 16u);
-            v4i* const to = reinterpret_cast<v4i*>(d == 0 ? constsd : d == 1 ? consts0 : consts1) + (wave & 1 ? quads : 0u);
+            const unsigned quads = d == 0 ? Cd / 4 : 8u * (d == 1 ? pairs0 : pairs1);
+            const __amdgpu_buffer_rsrc_t r = rsrc(w & 1 ? bi : si, quads * 16u);
+            v4i* const to = reinterpret_cast<v4i*>(d == 0 ? constsd : d == 1 ? consts0 : consts1) + (w & 1 ? quads : 0u);
             for (unsigned i0 = 0; i0 < quads; i0 += 256) {
                 v4i c[4];
 #pragma unroll
@@ -297,6 +302,11 @@ __global__ void __launch_bounds__(64 * DP_WAVES) conv_dwpw_kernel(const int8_t* 
     // ---- the first pointwise layer --------------------------------------------------------------------------------------------------
     int8_t* const to1 = px1 + row1;  // this lane's pixel of the second layer's input
     const __amdgpu_buffer_rsrc_t rout0 = NEXT ? rsrc(sum, sum != nullptr ? f_bytes : 0u) : rsrc(out, out == nullptr ? 0u : I8 ? f_bytes / 4u : f_bytes);
+    // elements of a shuffle's blobs. The first half is Float4 or Float8: a store to Float4 touches 8 lines of 128 bytes where it touches 16
+    // of Float8's, and the address unit works line by line (88 channels @52x52 b16 16.8 us
+    // with Float8 on both sides, 16.4 with Float4; 176 channels on one 26x26 image 6.9 and 6.5)
+    const unsigned sh_lane = SHUF ? n * sh_image(ja) + (2u * q * HW + pix) * 8u : 0u;
+    const unsigned sh_first = SHUF ? n * sh_image(ja) + 2u * q * HW * 8u + pix * pa.first_pack : 0u, sh_next = pa.first_pack == 4 ? HW * 16u : 16u;
     auto finish0 = [&](int pr, const v4i& c0, const v4i& c1) {
         const unsigned ch0 = 32u * pr + 8 * q;
         float si[8], bi[8];
@@ -324,7 +334,7 @@ __global__ void __launch_bounds__(64 * DP_WAVES) conv_dwpw_kernel(const int8_t* 
                         const v4i even = ja.other_odd ? r[h] : o, odd = ja.other_odd ? o : r[h];  // (uniform)
                         const v4i lo = {even[0], odd[0], even[1], odd[1]}, hi = {even[2], odd[2], even[3], odd[3]};
                         const unsigned pack = ch0 / 4 + h - (w ? half : 0u);  // in this half; beyond it on either side: the other half's
-                        const unsigned e = n * ja.sh_image + (pack * HW + pix) * 8u;
+                        const unsigned e = sh_lane + (8u * pr + h - (w ? half : 0u)) * HW * 8u;
                         const bool live = ok && pack < half;  // (a channel past the last one is a pack past the second half)
                         if (NEXT && w) {
                             const v2i b = {quantize4(lo, ja.twin_scale, ja.twin_half), quantize4(hi, ja.twin_scale, ja.twin_half)};
@@ -333,7 +343,8 @@ __global__ void __launch_bounds__(64 * DP_WAVES) conv_dwpw_kernel(const int8_t* 
                         }
                         if (f != nullptr) {
                             const __amdgpu_buffer_rsrc_t rf = rsrc(f, PR_OOB);
-                            store16(rf, lo, live ? e * 4u : PR_OOB, 0), store16(rf, hi, (live ? e * 4u : PR_OOB) + 16u, 0);
+                            const unsigned v = live ? (w ? e : sh_first + (8u * pr + h) * HW * 8u) * 4u : PR_OOB;
+                            store16(rf, lo, v, 0), store16(rf, hi, v + (w ? 16u : sh_next), 0);
                         }
                         if (b8 != nullptr)
                             store8(rsrc(b8, PR_OOB), v2i{quantize4(lo, ja.twin_scale, ja.twin_half), quantize4(hi, ja.twin_scale, ja.twin_half)},
@@ -434,9 +445,10 @@ bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom
     return true;
 }
 
-// Cost models in us, fitted to launches replayed from captured graphs over drawn layers (8 to 960 channels, 4x4 to 112x112 pixels, batches
-// of 1 to 64, every end). The launch: a wave walks `nd` pairs of octets and n0 and n1 pairs of row tiles one behind the other, once if
-// every workgroup is resident, and the more often the more workgroups there are for a compute unit.
+// Cost models in us, fitted to launches replayed from captured graphs behind a copy that leaves the L2 caches cold, over 2500 drawn layers
+// (16 to 960 channels, 4x4 to 112x112 pixels, batches of 1 to 64, every end): half of them within 5 %, nine in ten within 13 %. The launch:
+// a wave walks nd pairs of octets and n0 and n1 pairs of row tiles one behind the other, once if every workgroup is resident, and the more
+// often the more of eight waves there are for a compute unit.
 struct DwPwShape {
     double px;  // output pixels
     int pairs_d, pairs[2], steps[2];
@@ -446,43 +458,58 @@ struct DwPwShape {
           pairs{(g0.K + 31) / 32, g1 ? (g1->K + 31) / 32 : 0}, steps{igemm_channel_groups(g0.C), g1 ? igemm_channel_groups(g1->C) : 0},
           k5(gd.kh == 5), f32(e0.out_kind == OTTER_HIP_OUT_F32), adds(e0.residual || e0.join) {}
 };
-static double dwpw_cost(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1, int groups) {
-    static const double once[8] = {3.13, 0.450, 0.831, 0.528, 0.100, 0.461, 0.113, 0.308}, more[8] = {0.833, 0.258, 0.709, 0.087, 0.107, 0.281, 0.018, 0};
-    const int stride = DP_WAVES / groups, nd = (s.pairs_d + stride - 1) / stride;
-    const int n0 = (s.pairs[0] + stride - 1) / stride, n1 = (s.pairs[1] + stride - 1) / stride;
-    const double f[8] = {1, s.k5 ? 0. : nd, s.k5 ? (double)nd : 0, (double)n0, (double)n0 * s.steps[0], (double)n1, (double)n1 * s.steps[1], s.f32 ? (double)n0 : 0};
-    const double rounds = std::max(0., s.px / (16 * groups) / 256 - 1);
+static double dwpw_cost(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1, int waves, int groups) {
+    static const double once[2][9] = {{3.20, 0.391, 0.720, 0.351, 0.100, 0.497, 0.070, 0.173, 0.140}, {3.08, 0.432, 0.859, 0.421, 0.114, 0.563, 0.098, 0.244, 0.157}};
+    static const double more[2][9] = {{0.736, 0.222, 0.732, 0, 0.132, 0.279, 0.068, 0, 0}, {0.874, 0.266, 0.719, 0, 0.115, 0.315, 0.061, 0, 0}};
+    const int w = waves == 8, stride = waves / groups, nd = (s.pairs_d + stride - 1) / stride;
+    const double n0 = (s.pairs[0] + stride - 1) / stride, n1 = (s.pairs[1] + stride - 1) / stride;
+    const double f[9] = {1, s.k5 ? 0. : nd, s.k5 ? (double)nd : 0, n0, n0 * s.steps[0], n1, n1 * s.steps[1], s.f32 ? n0 : 0, s.adds ? n0 : 0};
+    const double rounds = std::max(0., s.px / (16 * groups) * waves / 2048 - 1);
     double t = 0;
-    for (int i = 0; i < 8; ++i) t += f[i] * (once[i] + rounds * more[i]);
+    for (int i = 0; i < 9; ++i) t += f[i] * (once[w][i] + rounds * more[w][i]);
     const double bytes = s.px * ((double)gd.C * gd.sh * gd.sw + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (g1 ? g1->K : 0));
-    return t + 0.163e-6 * bytes;
+    return t + 0.134e-6 * bytes;
 }
+// the layers by themselves, the pointwise ones as a pair where that is a launch
 static double dwpw_cost_apart(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1) {
     const double mbd = 1e-6 * s.px * gd.C * (gd.sh * gd.sw + 1.);
     const double mb0 = 1e-6 * s.px * (gd.C + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (s.f32 ? g0.K : 0));
-    double t = 4.86 + (0.254 + (s.k5 ? 0.025 : 0)) * mbd + 0.210 * mb0 + 1.395e-9 * s.px * g0.C * g0.K + 0.976e-3 * gd.C + 1.006e-3 * g0.K +
-               (gd.C > 256 ? 0.068 + 0.035e-6 * s.px * gd.C : 0);
-    if (g1) t += 1.80 + 0.323e-6 * s.px * ((double)g0.K + g1->K) + 1.065e-9 * s.px * g0.K * g1->K + 2.19e-3 * g1->K;
+    double t = 4.94 + (0.255 + (s.k5 ? 0.025 : 0)) * mbd + 0.178 * mb0 + 1.745e-9 * s.px * g0.C * g0.K + 0.879e-3 * gd.C + 0.671e-3 * g0.K +
+               (gd.C > 256 ? 0.059e-6 * s.px * gd.C : 0);
+    if (g1) t += 1.92 + 0.346e-6 * s.px * ((double)g0.K + g1->K) + 1.206e-9 * s.px * g0.K * g1->K + 1.054e-3 * g1->K + (g0.K > 256 ? 0.76 : 0);
     return t;
 }
 
-// Groups of 16 pixels for a workgroup.
-static int dwpw_groups(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
+// Groups of 16 pixels for a workgroup, + 16 for one of four waves: those have fewer idle waves where there are many pixels and few
+// channels (88 -> 88 -> 88 @52x52 b16 with a shuffle: eight waves and four groups 17.9 us, four and four 16.4), eight a shorter chain.
+static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, double* cost) {
     const DwPwShape s(gd, g0, e0, g1);
-    int best = 1;
-    for (int g = 2; g <= 8; g *= 2)
-        if (dwpw_lds_bytes(g0, g1, g) <= 65536 && dwpw_cost(s, gd, g0, g1, g) < dwpw_cost(s, gd, g0, g1, best)) best = g;
+    int best = 0;
+    for (int waves = 8; waves >= 4; waves -= 4)
+        for (int g = 1; g <= waves; g *= 2) {
+            if (dwpw_lds_bytes(g0, g1, g) > 65536) break;
+            const double c = dwpw_cost(s, gd, g0, g1, waves, g);
+            if (!best || c < *cost) best = g + (waves == 4 ? 16 : 0), *cost = c;
+        }
     return best;
 }
+// Over the drawn layers the rule takes two thirds and gives 0.88 of the time; 36 of the 2500 are over 5 % slower. (Five taps a row are where
+// the launch's loads cost most: nearer to the line it loses.)
 bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
-    const DwPwShape s(gd, g0, e0, g1);
-    return dwpw_cost(s, gd, g0, g1, dwpw_groups(gd, g0, e0, g1)) < 0.95 * dwpw_cost_apart(s, gd, g0, g1);
+    double cost = 0;
+    dwpw_plan(gd, g0, e0, g1, &cost);
+    return cost < (gd.kh == 5 ? 0.90 : 0.92) * dwpw_cost_apart(DwPwShape(gd, g0, e0, g1), gd, g0, g1);
 }
 
-template <int TAPS, int EPI, int KIND1>
-static hipError_t launch_dwpw(const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
-    launch((conv_dwpw_kernel<TAPS, EPI, KIND1>), dim3((pa.tiles + 7) / 8 * 8), dim3(64 * DP_WAVES), lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0));
+template <int NW, int TAPS, int EPI, int KIND1>
+static hipError_t launch_dwpw_waves(const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
+    launch((conv_dwpw_kernel<NW, TAPS, EPI, KIND1>), dim3((pa.tiles + 7) / 8 * 8), dim3(64 * NW), lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0));
     return hipGetLastError();
+}
+template <int TAPS, int EPI, int KIND1>
+static hipError_t launch_dwpw(int waves, const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
+    return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1>(x, out, sum, pa, e0, lds, stream)
+                      : launch_dwpw_waves<8, TAPS, EPI, KIND1>(x, out, sum, pa, e0, lds, stream);
 }
 
 hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const ConvGeom& gd, const Epilogue& ed, const int8_t* const w[2],
@@ -502,15 +529,18 @@ hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const
     pa.HW = g0.H * g0.W, pa.OW = g0.W, pa.H = gd.H, pa.W = gd.W, pa.total_pix = (unsigned)g0.N * (unsigned)pa.HW;
     pa.in_bytes = (unsigned)((size_t)gd.N * gd.C * gd.H * gd.W);
     pa.sh = gd.sh, pa.sw = gd.sw, pa.ph = gd.ph, pa.pw = gd.pw, pa.dh = gd.dh, pa.dw = gd.dw, pa.C8 = gd.C / 8;
-    const int groups = force ? force : dwpw_groups(gd, g0, e0, g1);
+    double cost = 0;
+    const int plan = force ? force : dwpw_plan(gd, g0, e0, g1, &cost), groups = plan & 15, waves = plan & 16 ? 4 : 8;
+    if (groups > waves) return hipErrorInvalidValue;
     if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return hipErrorInvalidValue;
     const size_t lds = dwpw_lds_bytes(g0, g1, groups);
     if (lds > 65536) return hipErrorInvalidValue;
+    pa.first_pack = e0.join ? (unsigned)e0.join->sh_pack0 : 8u;
     pa.lg = groups == 1 ? 0 : groups == 2 ? 1 : groups == 4 ? 2 : 3;
     pa.tiles = (int)((pa.total_pix + 16 * groups - 1) / (16 * groups));
     const int next = g1 ? pa.l[1].kind : (int)DP_NONE;
     const bool shuffle = e0.join && e0.join->other;
-#define OHIP_DP(T_, E_, N_) return launch_dwpw<T_, E_, N_>(x, out, sum, pa, e0, lds, stream)
+#define OHIP_DP(T_, E_, N_) return launch_dwpw<T_, E_, N_>(waves, x, out, sum, pa, e0, lds, stream)
 #define OHIP_DPN(T_, E_)                             \
     do {                                             \
         if (next == PP_I8) OHIP_DP(T_, E_, PP_I8);   \

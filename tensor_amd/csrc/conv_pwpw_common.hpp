@@ -35,7 +35,7 @@ __device__ __forceinline__ v4i pp_values(const Epilogue& ep, const float* si, co
     v4i r;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        r[e] = __float_as_int(lrelu_or_not(ep, fminf(fmaxf(__fmaf_rn((float)c[e], si[e], bi[e]), ep.act_lo), ep.act_hi)));
+        r[e] = __float_as_int(lrelu_or_not(ep, __builtin_amdgcn_fmed3f(__fmaf_rn((float)c[e], si[e], bi[e]), ep.act_lo, ep.act_hi)));
     return r;
 }
 __device__ __forceinline__ Epilogue pp_epilogue(const PwPwLayer& l) {

@@ -1080,7 +1080,7 @@ int ConvolutionLayer::forward_dwpw(const ConvolutionLayer* d, const ConvolutionL
                 if (with_q) q = Tensor::empty_device(sizes, ScalarType::Byte8);
                 if (!no_f32) whole = Tensor::empty_device(sizes, ScalarType::Float8);
             }
-            if (!u.joined) u.first = Tensor::empty_device(sizes, ScalarType::Float8);
+            if (!u.joined) u.first = Tensor::empty_device({N, K / 4, oh, ow}, ScalarType::Float4), end.first_float4 = 1;
             end.first_half = u.first.defined() ? (float*)u.first.device_ptr() : nullptr;
             if (!u.joined && u.second.defined()) end.second_half = (float*)u.second.device_ptr();
             (u.joined ? end.first_half_q : end.second_half_q) = q.defined() ? (int8_t*)q.device_ptr() : nullptr;

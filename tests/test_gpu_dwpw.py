@@ -97,12 +97,16 @@ def one_and_two(hip, rng, form, how, dw, pw, nx, x, n, h, w):
         f, o = new(np.float32, 2), new(np.int8, 2)
         hip.conv_dwpw(dw, pw, x, n, h, w, wants_out=False, joined=1, first_half=f, first_half_q=o, **end)
         return [f, o], [t[0], t[2]]
-    lo = new(np.float32)
+    lo, p4 = new(np.float32), new(np.float32)
+
+    def float8(t):  # what is Float4, as Float8
+        return t.view(n, K // 8, 2, oh * ow, 4).permute(0, 1, 3, 2, 4).reshape(-1)
     if nx:
-        return [run(first_half=lo, **end), lo], then(t[3]) + [t[0]]
+        return [run(first_half=lo, **end), lo, run(first_half=p4, first_float4=1, **end), float8(p4)], (then(t[3]) + [t[0]]) * 2
     hi, lq, hq = new(np.float32), new(np.int8), new(np.int8)
     hip.conv_dwpw(dw, pw, x, n, h, w, wants_out=False, first_half=lo, second_half=hi, first_half_q=lq, second_half_q=hq, **end)
-    return [lo, hi, lq, hq], list(t)
+    hip.conv_dwpw(dw, pw, x, n, h, w, wants_out=False, first_half=p4, first_float4=1, second_half_q=hq, **end)
+    return [lo, hi, lq, hq, float8(p4)], list(t) + [t[0]]
 
 
 @pytest.mark.parametrize("C,k,stride,pad,dil,act,K,K2,n,h,w", CASES)
@@ -114,8 +118,8 @@ def test_one_launch_equals_the_layers(hip, C, k, stride, pad, dil, act, K, K2, n
         nx = layer(hip, rng, K, K2, {"nonneg": 3, "i8": 2, "f32": 1, None: 0}[last], last == "f32") if last else None
         for form, how in forms(k, last):
             pw = layer(hip, rng, C, K, 2 if form != "sum" else 0, form != "i8")
-            for groups in (1, 2, 4, 8):  # of 16 pixels
-                if 16 * groups * (C + 160 + (K + 160 if nx else 0)) > 60000:
+            for groups in (1, 2, 4, 8, 17, 18, 20):  # of 16 pixels, + 16 with four waves
+                if 16 * (groups & 15) * (C + 160 + (K + 160 if nx else 0)) > 60000:
                     continue
                 dw.force = (-12, groups)
                 dw.set_tile(-12, groups)
@@ -142,7 +146,7 @@ def test_what_is_refused(hip):
     for first, second, end in ((i8, i8, {}), (dw, dw, {}), (dw, i8, dict(residual=r)), (dw, i8, other), (dw, i8, dict(out_q=b)), (dw, odd, dict(out_q=b, q_scale=1.0)),
                                (dw, odd, dict(next=i8)), (dw, f32, dict(next=i8, out_q=b)), (dw, f32, dict(sum=r)), (dw, f32, dict(residual1=r)),
                                (dw, f32, dict(next=i8, q_round_mode=9)), (dw, f32, dict(other, residual=r)), (dw, f32, dict(other, first_half=None, next=i8)),
-                               (dw, f32, dict(other, joined=1, second_half=r)), (dw, f32, dict(other, other_layout=capi.F32)), (dw, clipped, {}),
+                               (dw, f32, dict(other, joined=1, second_half=r)), (dw, f32, dict(other, joined=1, first_float4=1)), (dw, f32, dict(other, other_layout=capi.F32)), (dw, clipped, {}),
                                (dw, f32, dict(residual=r, residual1=r, part0_channels=60, part0_layout=capi.F32_P8, part1_layout=capi.F32_P8))):
         with pytest.raises(capi.HipError):
             hip.conv_dwpw(first, second, x, n, h, w, **end)
