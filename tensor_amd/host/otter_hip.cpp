@@ -1070,6 +1070,7 @@ int ConvolutionLayer::forward_dwpw(const ConvolutionLayer* d, const ConvolutionL
         end.out_q = (int8_t*)&some;
     }
     if (otter_hip_conv_dwpw_launches(d->handle_, p->handle_, N, H, W, &end, layout) != 1) return 1;
+    if (u.ask) return 0;
     try {
         const ScalarType odt = scalar_type_of_layout(layout);
         Tensor q, &whole = !u.other ? u.out : u.joined ? u.first : u.second;  // whole: the blob that is quantized
@@ -2607,17 +2608,26 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
         const int x = d->bottoms[0], made = forward_inputs(u.conv, {other, x}, blobs, opt);
         if (made) return made;
         int rc = 1;
-        for (int k = with_next && !blobs[layers_[u.next]->tops[0]].defined() && !begins_block(u.next, blobs[x], d) ? 0 : 1; k < 2 && rc > 0; ++k) {
+        for (int k = with_next && !blobs[layers_[u.next]->tops[0]].defined() ? 0 : 1; k < 2 && rc > 0; ++k) {
             ConvolutionLayer::DwPw e;
             e.next = k ? nullptr : static_cast<const ConvolutionLayer*>(layers_[u.next]);
             e.other = &blobs[other], e.other_odd = u.conv_k == 0, e.joined = joined, e.int8_only = int8_only, e.q_scale = u.hi_scale, e.q_round = u.hi_round;
+            e.ask = k == 0;  // (the question about the next block is the dearer one)
             rc = ConvolutionLayer::forward_dwpw(d, conv, blobs[x], e, opt);
+            if (e.ask && rc == 0) {
+                if (begins_block(u.next, blobs[x], d)) {
+                    rc = 1;
+                    continue;
+                }
+                e.ask = false;
+                rc = ConvolutionLayer::forward_dwpw(d, conv, blobs[x], e, opt);
+            }
             if (rc < 0) return rc;
             if (rc == 0 && joined) blobs[layers_[u.shuffle]->tops[0]] = e.first;
             if (rc == 0 && !joined) blobs[layers_[u.crop_lo]->tops[0]] = e.first;
             if (rc == 0 && !joined && !e.next) blobs[layers_[u.crop_hi]->tops[0]] = e.second;
             if (rc == 0 && e.next) blobs[e.next->tops[0]] = e.behind;
-            if (rc > 0 && !k) break;
+            if (rc > 0 && !k) break;  // (then the pointwise layers as a pair, behind a launch of the depthwise one)
         }
         if (rc == 0) {
             if (opt.lightmode)
@@ -2683,12 +2693,17 @@ int Net::forward_dwpw_unit(int pointwise, int out_layer, int shortcut, int part1
     const int x = d->bottoms[0], made = forward_inputs(pointwise, {shortcut, part1, x}, blobs, opt);
     if (made) return made;
     const auto next = part1 < 0 ? next_units_.find(out_layer) : next_units_.end();
-    const bool with_next = next != next_units_.end() && !blobs[layers_[next->second]->tops[0]].defined() && !begins_block(next->second, blobs[x], d);
+    const bool with_next = next != next_units_.end() && !blobs[layers_[next->second]->tops[0]].defined();
     for (int k = with_next ? 0 : 1; k < 2; ++k) {
         ConvolutionLayer::DwPw u;
         u.next = k ? nullptr : static_cast<const ConvolutionLayer*>(layers_[next->second]);
         u.shortcut = shortcut >= 0 ? &blobs[shortcut] : nullptr, u.part1 = part1 >= 0 ? &blobs[part1] : nullptr;
         u.q_scale = e->fuse_scale, u.q_round = e->fuse_round, u.int8_only = e->int8_only(opt);
+        if (!k) {  // (the question about the next block is the dearer one)
+            u.ask = true;
+            if (ConvolutionLayer::forward_dwpw(d, p, blobs[x], u, opt) || begins_block(next->second, blobs[x], d)) continue;
+            u.ask = false;
+        }
         const int rc = ConvolutionLayer::forward_dwpw(d, p, blobs[x], u, opt);
         if (rc < 0) return rc;
         if (rc > 0) continue;
@@ -2714,9 +2729,10 @@ int Net::forward_pair_unit(int first, int second, const ShuffleUnit* u, std::vec
     if (const ConvolutionLayer* d = u ? nullptr : front_of(first, blobs, opt)) {
         const int in = d->bottoms[0], made = forward_inputs(first, {in}, blobs, opt);
         if (made) return made;
-        if (!begins_block(second, blobs[in], d)) {
-            ConvolutionLayer::DwPw e;
-            e.next = b;
+        ConvolutionLayer::DwPw e;
+        e.next = b, e.ask = true;
+        if (ConvolutionLayer::forward_dwpw(d, a, blobs[in], e, opt) == 0 && !begins_block(second, blobs[in], d)) {
+            e.ask = false;
             const int rc = ConvolutionLayer::forward_dwpw(d, a, blobs[in], e, opt);
             if (rc < 0) return rc;
             if (rc == 0) {

@@ -275,6 +275,7 @@ public:
         const ConvolutionLayer* next = nullptr;
         const Tensor *shortcut = nullptr, *part1 = nullptr, *other = nullptr;
         bool other_odd = false, joined = false, int8_only = false;
+        bool ask = false;  // only whether it would run
         float q_scale = 0.f;
         int q_round = 0;
         Tensor out, first, second, behind;  // the result (a sum), a shuffle's halves, next's result
