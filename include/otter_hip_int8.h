@@ -586,6 +586,20 @@ int otter_hip_maxpool2d(const float* src, int src_layout, int n, int c, int h, i
 int otter_hip_upsample2d(const float* src, int src_layout, int n, int c, int h, int w, int out_h, int out_w, int mode,
                          int align_corner, float* dst, int dst_layout, void* stream);
 
+/* Layers whose fp32 result is part of a channel concatenation that only int8 convolutions read, each writing its channels of the
+ * concatenation's Byte8 blob (total_channels of them, this layer's from first_channel on; both multiples of 8), quantized as
+ * quantize_to_int8 does with q_scale, q_round_mode: neither the fp32 result nor the concatenation is ever in memory. A convolution may
+ * leave a second quantization of its result (twin, twin_scale, twin_round_mode; null: none), a Byte8 blob of its own, for int8 layers that
+ * read it directly. The _launches calls say 1 where the layer's own launch does it (the others are refused): pointwise convolutions on a
+ * Byte8 blob, depthwise ones of stride 1 without a twin, upsamplings of packed blobs. mode as in otter_hip_upsample2d. */
+int otter_hip_conv_slice_launches(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w, int total_channels, int with_twin);
+int otter_hip_conv_forward_slice(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w, int8_t* twin,
+                                 float twin_scale, int twin_round_mode, int8_t* blob, int total_channels, int first_channel, float q_scale,
+                                 int q_round_mode, void* stream);
+int otter_hip_upsample2d_slice_launches(int src_layout, int n, int c, int h, int w, int out_h, int out_w, int mode, int total_channels);
+int otter_hip_upsample2d_slice(const float* src, int src_layout, int n, int c, int h, int w, int out_h, int out_w, int mode, int align_corner,
+                               int8_t* blob, int total_channels, int first_channel, float q_scale, int q_round_mode, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -88,7 +88,8 @@ EXPORTS = ["otter_hip_init", "otter_hip_shutdown", "otter_hip_last_error", "otte
            "otter_hip_conv_block_plan", "otter_hip_conv_join_launches", "otter_hip_conv_forward_shuffle",
            "otter_hip_conv_forward_residual_concat", "otter_hip_conv_pair_launches", "otter_hip_conv_pair_forward",
            "otter_hip_conv_dwpw_launches", "otter_hip_conv_dwpw_forward", "otter_hip_conv_maxpool_launches",
-           "otter_hip_conv_forward_maxpool",
+           "otter_hip_conv_forward_maxpool", "otter_hip_conv_slice_launches", "otter_hip_conv_forward_slice",
+           "otter_hip_upsample2d_slice_launches", "otter_hip_upsample2d_slice",
            "otter_hip_record_begin", "otter_hip_record_end", "otter_hip_record_launch", "otter_hip_record_destroy"]
 
 
@@ -277,6 +278,13 @@ class Library:
         self._check(self.lib.otter_hip_upsample2d(self.ptr(src), src_layout, n, c, h, w, out_hw[0], out_hw[1], mode,
                                                   int(align_corner), self.ptr(dst), dst_layout, self.stream()))
         return dst
+
+    def upsample2d_slice(self, src, src_layout, shape, out_hw, mode, align_corner, blob, total_channels, first_channel, scale, round_mode):
+        """The upsampled blob quantized into channels first_channel .. of a Byte8 blob (otter_hip_upsample2d_slice)."""
+        n, c, h, w = shape
+        self._check(self.lib.otter_hip_upsample2d_slice(self.ptr(src), src_layout, n, c, h, w, out_hw[0], out_hw[1], mode,
+                                                        int(align_corner), self.ptr(blob), total_channels, first_channel,
+                                                        C.c_float(scale), round_mode, self.stream()))
 
     def inner_product(self, x, n, in_features, weight, bias, out_features):
         """otter_hip_inner_product: y[n][o] = sum_i x[n][i] * weight[o][i] + bias[o] (device tensors; bias may be None)."""
@@ -506,6 +514,22 @@ class Conv:
             self.h, self.L.ptr(x), in_layout, n, h, w, C.c_float(pad_value), self.L.ptr(out) if whole else None,
             self.L.ptr(q) if q is not None else None, C.c_float(q_scale or 0.0), q_round_mode, self.L.stream()))
         return out, q
+
+    def slice_launches(self, in_layout, n, h, w, total_channels, with_twin=False):
+        r = self.L.lib.otter_hip_conv_slice_launches(self.h, in_layout, n, h, w, total_channels, int(with_twin))
+        self.L._check(min(r, 0))
+        return r
+
+    def forward_slice(self, x, in_layout, n, h, w, blob, total_channels, first_channel, scale, round_mode=ROUND_SSE, twin_scale=None,
+                      twin_round_mode=ROUND_SSE):
+        """The layer's result quantized into channels first_channel .. of a Byte8 blob (otter_hip_conv_forward_slice). Returns the Byte8
+        blob quantized with twin_scale, or None."""
+        oh, ow = self.out_hw(h, w)
+        twin = self.L.empty(n * self.K * oh * ow, np.int8) if twin_scale is not None else None
+        self.L._check(self.L.lib.otter_hip_conv_forward_slice(
+            self.h, self.L.ptr(x), in_layout, n, h, w, self.L.ptr(twin) if twin is not None else None, C.c_float(twin_scale or 0.0),
+            twin_round_mode, self.L.ptr(blob), total_channels, first_channel, C.c_float(scale), round_mode, self.L.stream()))
+        return twin
 
     def forward_static(self, x, in_layout, n, h, w, out_layout=None, out=None):
         """otter_hip_conv_forward_static: the workspace is the library's static device array (no allocation inside)."""

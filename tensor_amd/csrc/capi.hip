@@ -2193,4 +2193,79 @@ int otter_hip_upsample2d(const float* src, int src_layout, int n, int c, int h, 
     return OTTER_HIP_OK;
 }
 
+// ---- layers whose result is a slice of a concatenation's Byte8 blob ------------------------------------------------------------------
+
+static int slice_args(const char* who, int channels, int total_channels, int first_channel, int round_mode) {
+    if (channels % 8 || total_channels % 8 || first_channel % 8 || first_channel < 0 || channels < 1 || total_channels - first_channel < channels)
+        return fail(OTTER_HIP_ERR_INVALID, std::string(who) + ": a slice is whole channel octets of the blob");
+    if (round_mode != OTTER_HIP_ROUND_EXACT && round_mode != OTTER_HIP_ROUND_SSE) return fail(OTTER_HIP_ERR_INVALID, std::string(who) + ": unknown rounding mode");
+    return OTTER_HIP_OK;
+}
+static float round_half(int mode) { return mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f; }
+
+// 1: the pointwise kernels with their operands in registers, 2: the depthwise matrix-core kernel, 0: neither
+static int conv_slice_kernel(const otter_hip_conv_t* h, int in_layout, const ConvGeom& g, const Epilogue& ep, bool twin) {
+    if (in_layout != OTTER_HIP_I8_P8 || h->d.out_kind != OTTER_HIP_OUT_F32 || h->c_pad || g.N < 1 || g.K % 8) return 0;
+    if ((h->force_tm == 0 || h->force_tm == -10) && h->w_igemm && h->so_same && conv_pw_reg_applicable(g, ep)) return 1;
+    const size_t octets = (size_t)ep.join->slice_octets;
+    return !twin && h->w_dw_mfma && (h->force_tm == 0 || h->force_tm == -2) && g.sh == 1 && dw_mfma_applicable(g, ep, dw_mfma_epilogue(ep, g.K), h->so_positive) &&
+                   (size_t)g.N * (g.C / 8) <= 32768 && (size_t)g.N * octets * 8 * g.OH * g.OW < ((size_t)1 << 31)
+               ? 2
+               : 0;
+}
+
+int otter_hip_conv_slice_launches(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w, int total_channels, int with_twin) {
+    if (!h || !valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_slice_launches: bad argument");
+    if (h->d.out_channels % 8) return 2;
+    if (const int rc = slice_args("otter_hip_conv_slice_launches", h->d.out_channels, total_channels, 0, OTTER_HIP_ROUND_SSE)) return rc;
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_slice_launches: empty output");
+    Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
+    JoinArgs ja;
+    int8_t some;
+    ja.slice = &some, ja.slice_octets = total_channels / 8, ep.join = &ja;
+    return conv_slice_kernel(h, in_layout, g, ep, with_twin != 0) ? 1 : 2;
+}
+
+int otter_hip_conv_forward_slice(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w, int8_t* twin, float twin_scale,
+                                 int twin_round_mode, int8_t* blob, int total_channels, int first_channel, float q_scale, int q_round_mode, void* stream) {
+    if (!h || !in || !blob) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_slice: null");
+    if (!valid_layout(in_layout) || n < 0 || in_h < 1 || in_w < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_slice: bad argument");
+    if (const int rc = slice_args("otter_hip_conv_forward_slice", h->d.out_channels, total_channels, first_channel, q_round_mode)) return rc;
+    if (twin && twin_round_mode != OTTER_HIP_ROUND_EXACT && twin_round_mode != OTTER_HIP_ROUND_SSE)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_slice: unknown rounding mode");
+    const ConvGeom g = make_geom(h->d, n, in_h, in_w);
+    if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_slice: empty output");
+    Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
+    JoinArgs ja;
+    ja.slice = blob + (size_t)first_channel * g.OH * g.OW, ja.slice_octets = total_channels / 8;
+    ja.slice_scale = q_scale, ja.slice_half = round_half(q_round_mode);
+    ep.twin = twin, ep.twin_scale = twin_scale, ep.twin_half = round_half(twin_round_mode), ep.join = &ja;
+    const int kernel = conv_slice_kernel(h, in_layout, g, ep, twin != nullptr);
+    if (!kernel) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_forward_slice: not a single launch (otter_hip_conv_slice_launches)");
+    if (kernel == 1)
+        OHIP_CHECK(run_conv_pw_reg((const int8_t*)in, h->w_igemm, h->so_one, nullptr, g, ep, h->force_tm < 0 ? h->force_tn : 0, (hipStream_t)stream));
+    else
+        OHIP_CHECK(run_conv_dw_mfma((const int8_t*)in, h->w_dw_mfma, ja.slice, g, ep, EPI_F32_SLICE, h->force_tm == -2 ? h->force_tn : 0, (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
+int otter_hip_upsample2d_slice_launches(int src_layout, int n, int c, int h, int w, int out_h, int out_w, int mode, int total_channels) {
+    if (!valid_layout(src_layout) || n < 0 || c < 1 || h < 1 || w < 1 || out_h < 1 || out_w < 1 || (mode != 1 && mode != 2) || total_channels % 8 || total_channels < c)
+        return fail(OTTER_HIP_ERR_INVALID, "otter_hip_upsample2d_slice_launches: bad argument");
+    return layout_elem(src_layout) == 0 && upsample_slice_applicable(layout_pack(src_layout), n, c, h, w, total_channels / 8, out_h, out_w) ? 1 : 2;
+}
+
+int otter_hip_upsample2d_slice(const float* src, int src_layout, int n, int c, int h, int w, int out_h, int out_w, int mode, int align_corner, int8_t* blob,
+                               int total_channels, int first_channel, float q_scale, int q_round_mode, void* stream) {
+    const int launches = otter_hip_upsample2d_slice_launches(src_layout, n, c, h, w, out_h, out_w, mode, total_channels);
+    if (launches < 0) return launches;
+    if (!src || !blob) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_upsample2d_slice: null");
+    if (const int rc = slice_args("otter_hip_upsample2d_slice", c, total_channels, first_channel, q_round_mode)) return rc;
+    if (launches != 1) return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_upsample2d_slice: not a single launch (otter_hip_upsample2d_slice_launches)");
+    OHIP_CHECK(run_upsample_slice(src, layout_pack(src_layout), blob + (size_t)first_channel * out_h * out_w, total_channels / 8, n, c, h, w, out_h, out_w, mode,
+                                  align_corner ? 1 : 0, q_scale, round_half(q_round_mode), (hipStream_t)stream));
+    return OTTER_HIP_OK;
+}
+
 }  // extern "C"

@@ -159,6 +159,11 @@ struct JoinArgs {
     float *sh_out0 = nullptr, *sh_out1 = nullptr;
     int8_t *sh_q0 = nullptr, *sh_q1 = nullptr;
     size_t sh_image = 0;
+    // The result is a slice of a Byte8 blob of slice_octets octets, quantized with slice_scale (null: none); Epilogue::twin then is a blob of
+    // its own with the same result quantized with twin_scale, or null, and there is no fp32 blob
+    int8_t* slice = nullptr;
+    int slice_octets = 0;
+    float slice_scale = 0.f, slice_half = 0.f;
     int sh_pack0 = 8;  // channels of an element of sh_out0: 8, or 4 (the launch behind a depthwise layer only)
 };
 
@@ -171,7 +176,8 @@ enum {
     EPI_F32_P8 = 4,       // depthwise only
     EPI_F32_P4_FUSED = 5,  // implicit GEMM only: EPI_F32_P4 plus the residual addend and / or the int8 twin
     EPI_F32_SHUFFLE = 6,   // the same kernels: the channels interleaved with another blob's (JoinArgs::other)
-    EPI_F32_P4_PARTS = 7   // EPI_F32_P4_FUSED with the addend in two parts (JoinArgs::residual1)
+    EPI_F32_P4_PARTS = 7,  // EPI_F32_P4_FUSED with the addend in two parts (JoinArgs::residual1)
+    EPI_F32_SLICE = 8      // the pointwise register kernels: the quantized result in a slice of a blob (JoinArgs::slice)
 };
 
 // the argument that an instance takes for them

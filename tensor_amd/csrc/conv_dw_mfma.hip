@@ -85,6 +85,8 @@ struct DwArgs {
     unsigned gx_m, gx, c8_m, chunks_m, chunks;  // divisions (FastDiv) by the workgroups along x, the octets, the column chunks of a row
     int N, H, W, OH, OW, rps;           // rps: output rows of a strip
     unsigned total, in_bytes, out_bytes;
+    unsigned octets;                    // EPI_F32_SLICE: octets of an image of the blob that the result is a slice of,
+    float q_scale, q_half;              // and what it is quantized with
     float p0, lo, hi, half;             // LeakyReLU slope, clamp of an fp32 result, rounding constant
     unsigned short c8, lpi_m;           // octets; 1 / lane columns of an image, for lanes below 16 (16.8 fixed point)
     unsigned char gx_s, c8_s, chunks_s, lpi, ipw, ph, lrelu;  // ipw: images of a wave
@@ -173,7 +175,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
         si[t] = *reinterpret_cast<const v4i*>(ep.scale_in + ch + 4 * t);
         bi[t] = *reinterpret_cast<const v4i*>(ep.bias + ch + 4 * t);
         so[t] = v4i{0, 0, 0, 0};
-        if constexpr (EPI != EPI_F32_P4 && EPI != EPI_F32_P8) so[t] = *reinterpret_cast<const v4i*>(ep.scale_out + ch + 4 * t);
+        if constexpr (EPI != EPI_F32_P4 && EPI != EPI_F32_P8 && EPI != EPI_F32_SLICE) so[t] = *reinterpret_cast<const v4i*>(ep.scale_out + ch + 4 * t);
         // the bias is the fma's vector operand in every row: keep it resident (the compiler would otherwise re-copy
         // it from scalar registers row after row)
 #pragma unroll
@@ -204,9 +206,10 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
         s_out = (unsigned)(n0 * C8 + o) * OHW * 32u;
         row_bytes = (unsigned)g.OW * 32u;
     } else {  // Byte8: [N][C/8][OH*OW][8 bytes]
-        v_out = st_ok ? (unsigned)di * (unsigned)C8 * OHW * 8u + (unsigned)ox * 8u + (S == 1 ? 0u : (unsigned)(q & 1) * 4u)
+        const unsigned octets = EPI == EPI_F32_SLICE ? g.octets : (unsigned)C8;
+        v_out = st_ok ? (unsigned)di * octets * OHW * 8u + (unsigned)ox * 8u + (S == 1 ? 0u : (unsigned)(q & 1) * 4u)
                       : DW_OOB;
-        s_out = (unsigned)(n0 * C8 + o) * OHW * 8u;
+        s_out = ((unsigned)n0 * octets + (unsigned)o) * OHW * 8u;
         row_bytes = (unsigned)g.OW * 8u;
     }
     const __amdgpu_buffer_rsrc_t rout = dw_rsrc(out, g.out_bytes);
@@ -235,6 +238,11 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
                 const unsigned vo_t = (t == 0 || !row_ok) ? v_o : v_o + (EPI == EPI_F32_P4 ? OHW * 16u : 16u);
                 store_b128_row(res, rout, vo_t, s_row);
             }
+        } else if constexpr (EPI == EPI_F32_SLICE) {  // (stride 1)
+            v2i w2;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) w2[t] = quantize4(dw_dequant4<LR ? 1 : 0>(ep, cur[t % T], si[t % T], bi[t % T]), g.q_scale, g.q_half);
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, w2), rout, (int)v_o, (int)s_row, 0);
         } else {
             constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
             if constexpr (S == 1) {
@@ -650,6 +658,8 @@ bool dw_mfma_applicable(const ConvGeom& g, const Epilogue& ep, int epi, bool sca
 // strip_blocks: 0 = automatic, > 0: steps of 8 / stride output rows of a strip, < 0: rows of it
 hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const ConvGeom& g, const Epilogue& ep, int epi,
                             int strip_blocks, hipStream_t stream) {
+    const JoinArgs* const slice = epi == EPI_F32_SLICE ? ep.join : nullptr;
+    if (slice != nullptr && g.sh != 1) return hipErrorInvalidValue;
     if (g.N == 0 || g.OH * g.OW == 0) return hipSuccess;
     const int C8 = g.C / 8;
     const int PH = 4 / g.sh;  // output pixels per lane column
@@ -666,7 +676,7 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     const int U = 8 / g.sh;
     const int rps = strip_blocks > 0   ? std::min(strip_blocks, (g.OH + U - 1) / U) * U
                     : strip_blocks < 0 ? std::min(-strip_blocks, g.OH)
-                                       : DwStrips(g.OH, g.sh, g.kh, epi == EPI_I8_P8_NONNEG ? 1 : epi == EPI_I8_P8 ? 0 : 2,
+                                       : DwStrips(g.OH, g.sh, g.kh, epi == EPI_I8_P8_NONNEG ? 1 : epi == EPI_I8_P8 || slice ? 0 : 2,
                                                   (float)(col_chunks * groups)).choose();
     const int n_strips = (g.OH + rps - 1) / rps;
     // a workgroup is one strip: with two and four strips a workgroup, and shares of LDS reserved to even them out over the compute
@@ -674,6 +684,7 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     const dim3 grid((unsigned)(col_chunks * n_strips), (unsigned)groups), block(64);
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW * (epi == EPI_F32_P4 || epi == EPI_F32_P8 ? 4 : 1));
+    const size_t slice_bytes = slice ? ((size_t)(g.N - 1) * slice->slice_octets + C8) * g.OH * g.OW * 8 : 0;
     const FastDiv gx = fast_div(grid.x), c8 = fast_div((unsigned)C8), ch = fast_div((unsigned)col_chunks);
     DwArgs pl{};
     pl.scale_in = ep.scale_in, pl.bias = ep.bias, pl.scale_out = ep.scale_out;
@@ -681,7 +692,8 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     pl.chunks_m = ch.m, pl.chunks_s = (unsigned char)ch.s, pl.chunks = (unsigned)col_chunks;
     pl.lpi = (unsigned char)lpi, pl.lpi_m = (unsigned short)(256 / lpi + 1), pl.ipw = (unsigned char)ipw;
     pl.N = g.N, pl.H = g.H, pl.W = g.W, pl.OH = g.OH, pl.OW = g.OW, pl.ph = (unsigned char)g.ph, pl.rps = rps;
-    pl.total = grid.x * grid.y, pl.in_bytes = in_bytes, pl.out_bytes = out_bytes;
+    pl.total = grid.x * grid.y, pl.in_bytes = in_bytes, pl.out_bytes = slice ? (unsigned)slice_bytes : out_bytes;
+    if (slice) pl.octets = (unsigned)slice->slice_octets, pl.q_scale = slice->slice_scale, pl.q_half = slice->slice_half;
     pl.p0 = ep.act_p0, pl.lo = ep.act_lo, pl.hi = ep.act_hi, pl.half = ep.round_half, pl.lrelu = ep.lrelu;
 #define OHIP_DWM_L(S_, E_, O_, K_)                                                                                        \
     do {                                                                                                                   \
@@ -709,7 +721,8 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
         else if (epi == EPI_F32_P8) OHIP_DWM(S_, EPI_F32_P8);         \
         else OHIP_DWM(S_, EPI_F32_P4);                                \
     } while (0)
-    if (g.sh == 1) OHIP_DWM_E(1);
+    if (slice != nullptr) OHIP_DWM(1, EPI_F32_SLICE);
+    else if (g.sh == 1) OHIP_DWM_E(1);
     else OHIP_DWM_E(2);
 #undef OHIP_DWM_E
 #undef OHIP_DWM_K

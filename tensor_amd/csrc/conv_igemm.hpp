@@ -193,6 +193,9 @@ hipError_t run_shuffle2_split(const float* a, int pa, const float* b, int pb, fl
                               int round_mode, int N, int Ch, int HW, hipStream_t stream);
 hipError_t run_maxpool(const float* src, int ps, float* dst, int pd, int N, int C, int H, int W, int OH, int OW, int kh,
                        int kw, int sh, int sw, int ph, int pw, int dh, int dw, float pad_value, hipStream_t stream);
+bool upsample_slice_applicable(int ps, int N, int C, int H, int W, int octets, int OH, int OW);
+hipError_t run_upsample_slice(const float* src, int ps, int8_t* dst, int octets, int N, int C, int H, int W, int OH, int OW, int mode, int align_corner,
+                              float qs, float half, hipStream_t stream);
 hipError_t run_upsample(const float* src, int ps, float* dst, int pd, int N, int C, int H, int W, int OH, int OW, int mode,
                         int align_corner, hipStream_t stream);
 

@@ -42,6 +42,15 @@ struct PwShuffle {  // JoinArgs::other and the like
         return {j.other, j.sh_out0, j.sh_out1, j.sh_q0, j.sh_q1, ep.twin_scale, ep.twin_half, (unsigned)j.sh_image, (short)j.other_pack, (short)j.other_odd};
     }
 };
+struct PwSlice {  // JoinArgs::slice and the like
+    int8_t *twin, *slice;
+    float twin_scale, twin_half, slice_scale, slice_half;
+    unsigned octets;
+    static PwSlice of(const Epilogue& ep) {
+        const JoinArgs& j = *ep.join;
+        return {ep.twin, j.slice, ep.twin_scale, ep.twin_half, j.slice_scale, j.slice_half, (unsigned)j.slice_octets};
+    }
+};
 template <int EPI>
 struct PwAddOf {
     using Type = NoJoin;
@@ -53,6 +62,10 @@ struct PwAddOf<EPI_F32_P4_FUSED> {
 template <>
 struct PwAddOf<EPI_F32_SHUFFLE> {
     using Type = PwShuffle;
+};
+template <>
+struct PwAddOf<EPI_F32_SLICE> {
+    using Type = PwSlice;
 };
 template <>
 struct PwAddOf<EPI_F32_P4_PARTS> {

@@ -57,7 +57,7 @@ template <int FN, int CG, int EPI>
 __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
                                                           PwRegArgs pa, PwAdd<EPI> ja) {
     constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
-    constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
+    constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS, SLICE = EPI == EPI_F32_SLICE;
     constexpr bool ADD = SHUF || FUSED;  // reads elements of another fp32 blob
     const Epilogue ep = pw_epilogue<EPI>(pa, ja);
     const unsigned lane = threadIdx.x & 63, q = lane >> 4, p = lane & 15;
@@ -197,6 +197,12 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
                                        live ? e : PR_OOB, 0);
                         }
                     }
+                } else if constexpr (SLICE) {
+                    if (ja.twin != nullptr)  // (uniform)
+                        store8(rsrc(ja.twin, pa.total_pix * K), v2i{quantize4(r[0], ja.twin_scale, ja.twin_half), quantize4(r[1], ja.twin_scale, ja.twin_half)},
+                               ok[j] && ch0 < K ? at_b8(j) : PR_OOB, (unsigned)pr * 32u * HW);
+                    store8(rsrc(ja.slice, PR_OOB), v2i{quantize4(r[0], ja.slice_scale, ja.slice_half), quantize4(r[1], ja.slice_scale, ja.slice_half)},
+                           ok[j] && ch0 < K ? ((n[j] * ja.octets + q) * HW + pix[j]) * 8u : PR_OOB, (unsigned)pr * 32u * HW);
                 } else {
                     v2i tw;
 #pragma unroll
@@ -248,7 +254,7 @@ template <int FN, int NS, int EPI>
 __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
                                                             PwRegArgs pa, PwAdd<EPI> ja) {
     constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
-    constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
+    constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS, SLICE = EPI == EPI_F32_SLICE;
     constexpr int OWN = FN < 2 ? 1 : FN / 2;  // half pairs that a wave finishes (of 2 FN; with FN == 1 waves 0 and 1 have one each)
     __shared__ v4i red[2][2 * FN][3][64];     // [buffer][half pair][the other waves][lane]
     const Epilogue ep = pw_epilogue<EPI>(pa, ja);
@@ -367,6 +373,13 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
                         store8(rsrc(b8, PR_OOB), v2i{quantize4(lo, ep.twin_scale, ep.twin_half), quantize4(hi, ep.twin_scale, ep.twin_half)},
                                live ? e : PR_OOB, 0);
                 }
+            } else if constexpr (SLICE) {
+                const bool live = oko[o] && ch < K;
+                if (ja.twin != nullptr)  // (uniform)
+                    __builtin_amdgcn_raw_buffer_store_b32((unsigned)quantize4(r, ja.twin_scale, ja.twin_half), rsrc(ja.twin, pa.total_pix * K),
+                                                          (int)(live ? ((no[o] * (K / 8) + q) * HW + po[o]) * 8u + 4 * h : PR_OOB), (int)((unsigned)pr * 32u * HW), 0);
+                __builtin_amdgcn_raw_buffer_store_b32((unsigned)quantize4(r, ja.slice_scale, ja.slice_half), rsrc(ja.slice, PR_OOB),
+                                                      (int)(live ? ((no[o] * ja.octets + q) * HW + po[o]) * 8u + 4 * h : PR_OOB), (int)((unsigned)pr * 32u * HW), 0);
             } else {
                 if constexpr (FUSED)
                     if (PARTS || ep.residual != nullptr)
@@ -429,6 +442,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
 static int pw_reg_epilogue(const Epilogue& ep, int K) {
     const int epi = pick_epilogue(ep, K);
     if (epi != EPI_F32_P4 || !ep.fused()) return epi;
+    if (ep.join != nullptr && ep.join->slice != nullptr) return EPI_F32_SLICE;
     return ep.join == nullptr ? EPI_F32_P4_FUSED : ep.join->other != nullptr ? EPI_F32_SHUFFLE : EPI_F32_P4_PARTS;
 }
 
@@ -441,6 +455,7 @@ bool conv_pw_reg_applicable(const ConvGeom& g, const Epilogue& ep) {
     if ((size_t)igemm_channel_groups(g.C) * igemm_padded_rows(g.K) * 64 >= ((size_t)1 << 31)) return false;  // (the packed weights)
     // 32-bit byte offsets into every blob; a shuffled result that is one blob has twice the layer's channels
     const size_t joined = epi == EPI_F32_SHUFFLE && ep.join->sh_image > (size_t)g.K * g.H * g.W ? 2 : 1;
+    if (epi == EPI_F32_SLICE && (ep.residual || px * ep.join->slice_octets * 8 >= ((size_t)1 << 31))) return false;
     return px * g.C < ((size_t)1 << 31) && px * g.K * joined * layout_elem_bytes(ep.out_layout) < ((size_t)1 << 31);
 }
 
@@ -462,6 +477,7 @@ static hipError_t launch_pw_reg_e(int epi, const int8_t* x, const int8_t* wpk, v
     case EPI_F32_P4_FUSED: return launch_pw_reg<FN, CG, EPI_F32_P4_FUSED>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_SHUFFLE: return launch_pw_reg<FN, CG, EPI_F32_SHUFFLE>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_P4_PARTS: return launch_pw_reg<FN, CG, EPI_F32_P4_PARTS>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_SLICE: return launch_pw_reg<FN, CG, EPI_F32_SLICE>(x, wpk, out, pa, ep, slices, stream);
     }
     return hipErrorInvalidValue;
 }
@@ -495,6 +511,7 @@ static hipError_t launch_pw_split_e(int epi, const int8_t* x, const int8_t* wpk,
     case EPI_F32_P4_FUSED: return launch_pw_split<FN, NS, EPI_F32_P4_FUSED>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_SHUFFLE: return launch_pw_split<FN, NS, EPI_F32_SHUFFLE>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_P4_PARTS: return launch_pw_split<FN, NS, EPI_F32_P4_PARTS>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_F32_SLICE: return launch_pw_split<FN, NS, EPI_F32_SLICE>(x, wpk, out, pa, ep, slices, stream);
     }
     return hipErrorInvalidValue;
 }

@@ -2,6 +2,7 @@
 #include "otter_hip.hpp"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -809,10 +810,7 @@ int ConvolutionLayer::forward_int8(const Tensor& bottom_in, const Tensor* shortc
                                    const NetOption& opt, bool int8_only) const {
     if (!handle_ || !bottom_in.defined() || bottom_in.dim() != 4) return -1;
     // the producer may already have quantized this blob with this layer's scale (see Net::plan_fused_quantize)
-    Tensor bottom = bottom_in, twin;
-    if (base_of(bottom_in.scalar_type()) == ScalarType::Float && in_channels % 8 == 0 &&
-        bottom_in.quantized_twin(bottom_blob_int8_scales.data_ptr<float>()[0], input_round_mode(opt), twin))
-        bottom = twin;
+    const Tensor bottom = int8_input(bottom_in, opt);
     const int in_layout = hip_layout_of(bottom.scalar_type());
     if (in_layout < 0 || base_of(bottom.scalar_type()) == ScalarType::Int) return -1;
     const int N = (int)bottom.size(0), H = (int)bottom.size(2), W = (int)bottom.size(3);
@@ -989,6 +987,35 @@ int ConvolutionLayer::forward_pair(const ConvolutionLayer* a, const ConvolutionL
         if (rc) return rc;
         if (other) first_half.mark_device_written();
         top.mark_device_written();
+    } catch (const Error&) {
+        return -100;
+    }
+    return 0;
+}
+
+Tensor ConvolutionLayer::int8_input(const Tensor& bottom, const NetOption& opt) const {
+    Tensor twin;
+    return base_of(bottom.scalar_type()) == ScalarType::Float && in_channels % 8 == 0 &&
+                   bottom.quantized_twin(bottom_blob_int8_scales.data_ptr<float>()[0], input_round_mode(opt), twin)
+               ? twin
+               : bottom;
+}
+
+bool ConvolutionLayer::can_slice(ScalarType dtype, int n, int h, int w, int total_channels, bool with_twin, const NetOption& opt, int* oh, int* ow) const {
+    const int layout = hip_layout_of(dtype);
+    return handle_ && int8_scale_term && int8_scale_term <= 100 && force_out_layout < 0 && opt.use_packing_layout && layout >= 0 &&
+           otter_hip_conv_output_shape(handle_, h, w, oh, ow) == 0 &&
+           otter_hip_conv_slice_launches(handle_, layout, n, h, w, total_channels, with_twin ? 1 : 0) == 1;
+}
+
+int ConvolutionLayer::forward_slice(const Tensor& bottom, Tensor& whole, int at, float q_scale, int q_round, float twin_scale, int twin_round, Tensor& twin) const {
+    try {
+        if (twin_scale > 0.f) twin = Tensor::empty_device({whole.size(0), out_channels / 8, whole.size(2), whole.size(3)}, ScalarType::Byte8);
+        const int rc = otter_hip_conv_forward_slice(handle_, bottom.device_ptr(), hip_layout_of(bottom.scalar_type()), (int)bottom.size(0), (int)bottom.size(2),
+                                                    (int)bottom.size(3), twin_scale > 0.f ? (int8_t*)twin.device_ptr() : nullptr, twin_scale, twin_round,
+                                                    (int8_t*)whole.device_ptr(), (int)whole.channels(), at, q_scale, q_round, launch_stream());
+        if (rc) return rc;
+        if (twin.defined()) twin.mark_device_written();
     } catch (const Error&) {
         return -100;
     }
@@ -1798,6 +1825,19 @@ public:
         top.mark_device_written();
         return 0;
     }
+    // The result quantized into channels `at` .. of the Byte8 blob `whole` (otter_hip_upsample2d_slice); whether that can be, and its size
+    bool can_slice(const Tensor& b, int total_channels, int* oh, int* ow) const {
+        if (!f32_4d(b) || b.channels() % 8) return false;
+        *oh = (int)(b.size(2) * scale_h_), *ow = (int)(b.size(3) * scale_w_);
+        return *oh >= 1 && *ow >= 1 &&
+               otter_hip_upsample2d_slice_launches(hip_layout_of(b.scalar_type()), (int)b.size(0), (int)b.channels(), (int)b.size(2), (int)b.size(3), *oh, *ow, mode_,
+                                                   total_channels) == 1;
+    }
+    int forward_slice(const Tensor& b, Tensor& whole, int at, float q_scale, int q_round) const {
+        return otter_hip_upsample2d_slice((const float*)b.device_ptr(), hip_layout_of(b.scalar_type()), (int)b.size(0), (int)b.channels(), (int)b.size(2),
+                                          (int)b.size(3), (int)whole.size(2), (int)whole.size(3), mode_, 0, (int8_t*)whole.device_ptr(), (int)whole.channels(), at,
+                                          q_scale, q_round, launch_stream());
+    }
     std::string type() const override { return "Upsample"; }
 
 private:
@@ -2146,6 +2186,13 @@ int Net::forward_layer(int li, std::vector<Tensor>& blobs, const NetOption& opt)
         }
     }
     {
+        const auto unit = slice_units_.find(li);
+        if (unit != slice_units_.end() && layer->int8_only(opt)) {
+            const int rc = forward_slices(li, unit->second, blobs, opt);
+            if (rc <= 0) return rc;
+        }
+    }
+    {
         const auto unit = residual_units_.find(li);
         // only when the convolution's own result has not been computed (or set by the caller)
         if (unit != residual_units_.end() && !blobs[layers_[unit->second.conv]->tops[0]].defined()) {
@@ -2425,6 +2472,57 @@ void Net::plan_fused_quantize() const {
         shuffle_units_[lo] = u;
         shuffle_units_[hi] = u;
     }
+    // Concats that only int8 convolutions read, of blobs whose layers can write their channels of the quantized result
+    slice_units_.clear();
+    auto reads_int8 = [&](int li) {
+        const auto* c = dynamic_cast<const ConvolutionLayer*>(layers_[li]);
+        return c && c->int8_scale_term && c->bottom_blob_int8_scales.defined() && c->in_channels % 8 == 0;
+    };
+    for (size_t ci = 0; ci < layers_.size(); ++ci) {
+        const Layer* cat = layers_[ci];
+        if (cat->type() != "Concat" || !cat->of_library || !cat->fuse_only || cat->fuse_scale <= 0.f || cat->tops.size() != 1) continue;
+        std::vector<SlicePart> parts;
+        for (size_t k = 0; k < cat->bottoms.size(); ++k) {
+            const int b = cat->bottoms[k], r = root_[b], pi = blobs_[r].producer;
+            const Layer* const l = pi < 0 ? nullptr : layers_[pi];
+            if (!l || !l->of_library || l->bottoms.size() != 1 || l->tops.size() != 1 || sole_reader(b) != (int)ci) break;
+            SlicePart p{pi, (int)k, l->type() == "Upsample", false, -1};
+            const auto* c = dynamic_cast<const ConvolutionLayer*>(l);
+            if (p.upsample) {
+                if (r != b || !dynamic_cast<const UpsampleLayer*>(l)) break;
+            } else {
+                if (!c || !c->int8_scale_term || c->int8_scale_term > 100 || c->force_out_layout >= 0 || c->out_channels % 8 || c->in_channels % 8) break;
+                const bool depthwise = c->groups == c->in_channels && c->groups == c->out_channels;
+                // (a pointwise layer behind a depthwise or another pointwise one runs in that one's launch)
+                if (r == b ? !depthwise && !pair_layer(pi) : !pair_layer(pi)) break;
+                if (pair_units_.count(pi) || front_units_.count(pi)) break;
+                const int split = sole_reader(r);  // (or the Concat itself)
+                if (r != b) {  // beside the Concat only int8 convolutions that agree on the scale
+                    p.twin = true;
+                    bool only = l->fuse_scale > 0.f && split >= 0 && layers_[split]->type() == "Split";
+                    for (size_t t = 0; only && t < layers_[split]->tops.size(); ++t)
+                        for (int reader : blobs_[layers_[split]->tops[t]].consumers)
+                            only = only && ((reader == (int)ci && layers_[split]->tops[t] == b) || reads_int8(reader));
+                    if (!only) break;
+                }
+            }
+            parts.push_back(p);
+        }
+        if (parts.size() != cat->bottoms.size()) continue;
+        std::sort(parts.begin(), parts.end(), [](const SlicePart& a, const SlicePart& b) { return a.layer < b.layer; });
+        bool ok = true;
+        for (size_t k = 0; k < parts.size(); ++k) {
+            if (k && parts[k].layer == parts[k - 1].layer) ok = false;
+            for (size_t j = 0; j < parts.size(); ++j) {
+                const int x = layers_[parts[k].layer]->bottoms[0];
+                if (root_[x] != layers_[parts[j].layer]->tops[0]) continue;
+                // (its input is another part's: the quantization that one leaves, or nothing)
+                ok = ok && j < k && parts[j].twin && !parts[k].upsample;
+                parts[k].source = (int)j;
+            }
+        }
+        if (ok) slice_units_[(int)ci] = parts;
+    }
     // (not where the layer that reads the second half runs in the launch of a sum, a pooling or the next unit's end)
     std::vector<char> in_other_launch(layers_.size(), 0);
     for (const auto& u : residual_units_) in_other_launch[u.second.conv] = 1;
@@ -2654,6 +2752,89 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
     if (opt.lightmode)
         for (int b : {other, in_blob})
             if (blobs_[b].consumers.size() == 1) blobs[b] = Tensor();
+    return 0;
+}
+
+// The layers in front of a Concat that only int8 convolutions read, each writing its channels of the quantized result. Returns 1 when one
+// of their blobs is there or asked for, or the layers or the blobs at hand do not allow it.
+int Net::forward_slices(int concat, const std::vector<SlicePart>& parts, std::vector<Tensor>& blobs, const NetOption& opt) const {
+    const Layer* const cat = layers_[concat];
+    auto fresh = [&] {
+        for (const SlicePart& p : parts)
+            for (int b : {cat->bottoms[p.at], layers_[p.layer]->tops[0]})
+                if (blobs[b].defined() || opt.asked == b || (*opt.wanted)[b]) return false;
+        return true;
+    };
+    if (!fresh()) return 1;
+    for (const SlicePart& p : parts) {
+        if (p.source >= 0) continue;
+        const int made = forward_inputs(p.layer, {layers_[p.layer]->bottoms[0]}, blobs, opt);
+        if (made) return made;
+    }
+    if (!fresh()) return 1;
+    int total = 0, N = 0, H = 0, W = 0;
+    std::vector<int> first(cat->bottoms.size()), channels(cat->bottoms.size());
+    std::vector<Tensor> in(parts.size());
+    for (const SlicePart& p : parts) {
+        const auto* conv = p.upsample ? nullptr : static_cast<const ConvolutionLayer*>(layers_[p.layer]);
+        channels[p.at] = conv ? conv->out_channels : (int)blobs[layers_[p.layer]->bottoms[0]].channels();
+    }
+    for (size_t k = 0; k < channels.size(); ++k) first[k] = total, total += channels[k];
+    if (total % 8) return 1;
+    std::vector<std::array<int, 3>> made(parts.size());  // the shapes of the results
+    for (size_t k = 0; k < parts.size(); ++k) {
+        const SlicePart& p = parts[k];
+        int oh = 0, ow = 0, n;
+        if (p.source >= 0) {
+            n = made[p.source][0];
+            if (!static_cast<const ConvolutionLayer*>(layers_[p.layer])->can_slice(ScalarType::Byte8, n, made[p.source][1], made[p.source][2], total, p.twin, opt, &oh, &ow)) return 1;
+        } else {
+            const Tensor& b = blobs[layers_[p.layer]->bottoms[0]];
+            if (!b.defined() || b.dim() != 4) return 1;
+            n = (int)b.size(0);
+            if (p.upsample) {
+                in[k] = b;
+                if (!static_cast<const UpsampleLayer*>(layers_[p.layer])->can_slice(b, total, &oh, &ow)) return 1;
+            } else {
+                const auto* conv = static_cast<const ConvolutionLayer*>(layers_[p.layer]);
+                in[k] = conv->int8_input(b, opt);
+                if (b.channels() != conv->in_channels || !conv->can_slice(in[k].scalar_type(), n, (int)b.size(2), (int)b.size(3), total, p.twin, opt, &oh, &ow)) return 1;
+            }
+        }
+        made[k] = {n, oh, ow};
+        if (k && made[k] != made[0]) return 1;
+    }
+    N = made[0][0], H = made[0][1], W = made[0][2];
+    Tensor whole;
+    try {
+        whole = Tensor::empty_device({N, total / 8, H, W}, ScalarType::Byte8);
+    } catch (const Error&) {
+        return -100;
+    }
+    for (size_t k = 0; k < parts.size(); ++k) {
+        const SlicePart& p = parts[k];
+        const Layer* const l = layers_[p.layer];
+        Tensor twin;
+        const int rc = p.upsample ? static_cast<const UpsampleLayer*>(l)->forward_slice(in[k], whole, first[p.at], cat->fuse_scale, cat->fuse_round)
+                                  : static_cast<const ConvolutionLayer*>(l)->forward_slice(p.source >= 0 ? blobs[layers_[parts[p.source].layer]->tops[0]] : in[k], whole, first[p.at],
+                                                                                           cat->fuse_scale, cat->fuse_round, p.twin ? l->fuse_scale : 0.f, l->fuse_round, twin);
+        if (rc) return rc;
+        if (p.twin) blobs[l->tops[0]] = twin;
+    }
+    whole.mark_device_written();
+    blobs[cat->tops[0]] = whole;
+    if (opt.lightmode)
+        for (const SlicePart& p : parts) {
+            const int b = p.source >= 0 ? layers_[parts[p.source].layer]->tops[0] : layers_[p.layer]->bottoms[0];
+            // (a source's blob may have a Split's other readers still to come)
+            bool done = blobs_[b].consumers.size() == 1;
+            if (p.source >= 0)
+                for (int ci : blobs_[b].consumers)
+                    if (layers_[ci]->type() == "Split")
+                        for (int t : layers_[ci]->tops)
+                            for (int r : blobs_[t].consumers) done = done && (r == concat || r == p.layer);
+            if (done) blobs[b] = Tensor();
+        }
     return 0;
 }
 

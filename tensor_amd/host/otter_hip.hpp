@@ -266,6 +266,12 @@ public:
     // other half, `top` the second layer's result. Returns 1, and does nothing, when that is not one launch here.
     static int forward_pair(const ConvolutionLayer* first, const ConvolutionLayer* second, const Tensor& bottom_blob, const Tensor* other,
                             bool other_odd, Tensor& first_half, Tensor& top, const NetOption& opt);
+    // This layer's fp32 result quantized into channels `at` .. of the Byte8 blob `whole` (otter_hip_conv_forward_slice), and with twin_scale
+    // > 0 into a blob of its own. can_slice: whether it can, on a blob of that type and shape; (*oh, *ow): the result's size.
+    bool can_slice(ScalarType dtype, int n, int h, int w, int total_channels, bool with_twin, const NetOption& opt, int* oh, int* ow) const;
+    int forward_slice(const Tensor& bottom_blob, Tensor& whole, int at, float q_scale, int q_round, float twin_scale, int twin_round, Tensor& twin) const;
+    // `bottom_blob`, or the quantization of it for this layer that came with it
+    Tensor int8_input(const Tensor& bottom_blob, const NetOption& opt) const;
     // An image stem and the 3x3 stride-2 max pooling behind it in one launch (otter_hip_conv_forward_maxpool)
     int forward_maxpool(const Tensor& bottom_blob, float pad_value, float q_scale, int q_round, Tensor& pooled, const NetOption& opt, bool int8_only) const;
     // A depthwise layer, the pointwise layer that alone reads its int8 result and, where there is one, the pointwise layer `next` behind
@@ -416,6 +422,17 @@ private:
     mutable std::map<int, int> front_units_;
     // layers with an fp32 blob that one pointwise int8 convolution reads quantized: the layer's index -> the convolution's
     mutable std::map<int, int> next_units_;
+    // Concat layers whose result only int8 convolutions read, every blob of it made by a layer that can write its channels of the quantized
+    // result itself: the Concat's index -> those layers, in the order in which they run
+    struct SlicePart {
+        int layer;       // an int8 convolution with an fp32 result, or an Upsample layer
+        int at;          // its place among the Concat's bottom blobs
+        bool upsample;
+        bool twin;       // a convolution whose blob int8 convolutions read as well
+        int source;      // the part that makes its input's quantization, or -1
+    };
+    mutable std::map<int, std::vector<SlicePart>> slice_units_;
+    int forward_slices(int concat, const std::vector<SlicePart>& parts, std::vector<Tensor>& blobs, const NetOption& opt) const;
     const ConvolutionLayer* front_of(int pointwise, const std::vector<Tensor>& blobs, const NetOption& opt) const;
     bool begins_block(int li, const Tensor& x, const ConvolutionLayer* d) const;
     int forward_dwpw_unit(int pointwise, int out_layer, int shortcut, int part1, std::vector<Tensor>& blobs, const NetOption& opt) const;

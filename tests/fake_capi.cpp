@@ -65,6 +65,19 @@ std::string sum(std::string a, std::string b) {
 std::string half(const std::string& e, int k) { return "half" + std::to_string(k) + "(" + e + ")"; }
 std::string shuffle(const std::string& cat) { return "shuffle(" + cat + ")"; }
 std::string cat2(const std::string& a, const std::string& b) { return "cat(" + a + "," + b + ")"; }
+// a blob that is written slice by slice: it holds the concatenation once every channel is there
+void slice(void* blob, int total, int first, int channels, const std::string& e) {
+    static std::map<void*, std::map<int, std::pair<int, std::string>>> open;
+    auto& parts = open[blob];
+    parts[first] = {channels, e};
+    int at = 0;
+    std::string all;
+    for (const auto& p : parts) {
+        if (p.first != at) return;
+        at += p.second.first, all += (all.empty() ? "cat(" : ",") + p.second.second;
+    }
+    if (at == total) put(blob, q(all + ")")), open.erase(blob);
+}
 int form() { return g_set.count("form") ? g_set["form"] : 3; }
 bool on(const char* what) { return !g_set.count(what) || g_set[what]; }
 void out_hw(const otter_hip_conv_desc& d, int h, int w, int* oh, int* ow) {
@@ -185,6 +198,18 @@ int otter_hip_conv_dwpw_forward(const otter_hip_conv_t* d, const otter_hip_conv_
 int otter_hip_conv_maxpool_launches(const otter_hip_conv_t*, int, int, int, int) { return on("stem_pool") ? 1 : 2; }
 int otter_hip_conv_forward_maxpool(const otter_hip_conv_t* h, const void* in, int, int, int, int, float, float* out, int8_t* oq, float, int, void* s) {
     return launched("stem_pool", s, [=] { const std::string r = "maxpool(" + conv(h, at(in)) + ")"; put(out, r), put(oq, q(r)); });
+}
+int otter_hip_conv_slice_launches(const otter_hip_conv_t*, int, int, int, int, int, int) { return on("slice") ? 1 : 2; }
+int otter_hip_conv_forward_slice(const otter_hip_conv_t* h, const void* in, int, int, int, int, int8_t* twin, float, int, int8_t* blob, int total, int first,
+                                 float, int, void* s) {
+    return launched("slice", s, [=] { const std::string r = conv(h, at(in)); put(twin, q(r)), slice(blob, total, first, h->d.out_channels, r); });
+}
+int otter_hip_upsample2d(const float* src, int, int, int, int, int, int, int, int, int, float* dst, int, void* s) {
+    return launched("upsample", s, [=] { put(dst, "up(" + at(src) + ")"); });
+}
+int otter_hip_upsample2d_slice_launches(int, int, int, int, int, int, int, int, int) { return on("slice") ? 1 : 2; }
+int otter_hip_upsample2d_slice(const float* src, int, int, int c, int, int, int, int, int, int, int8_t* blob, int total, int first, float, int, void* s) {
+    return launched("slice", s, [=] { slice(blob, total, first, c, "up(" + at(src) + ")"); });
 }
 int otter_hip_conv_avgpool_launches(const otter_hip_conv_t*, int, int, int, int) { return on("avgpool") ? 1 : 2; }
 int otter_hip_conv_forward_avgpool(const otter_hip_conv_t* h, const void* in, int, int, int, int, float* out, void*, size_t, void* s) {

@@ -179,6 +179,78 @@ for tail in (next_unit, another_pointwise):  # not one of those that the program
 """, program=True)
 
 
+def test_layers_in_front_of_a_concat_write_their_slices(tmp_path):
+    """A Concat that an int8 convolution reads, of a pointwise layer and the depthwise one behind it (a ghost module), of an upsampling and
+    a pointwise layer, and of what has to stay as it is."""
+    run(tmp_path, r"""
+def up(g, name, src):
+    return g.add(name, "up(%s)" % g.expr[src], type="Upsample", input=src, stride=1)
+def cat(g, name, *src):
+    return g.add(name, "cat(%s)" % ",".join(g.expr[s] for s in src), type="Concat", input=",".join(src))
+def wide(g, number, src):  # a pointwise layer over a concatenation
+    name = "c%d" % number
+    g.wide = getattr(g, "wide", []) + [(number, 0)]
+    return g.add(name, "%s(%s)" % (name, g.expr[src]), type="Convolution", input=src, out_channels=CH, kernel=1, int8_scale_term=2)
+def ghost(g, a=3, b=2):  # 3: the pointwise layer's channels come first
+    first = g.conv(2, g.conv(1, "data"))
+    second = g.conv(3, first, dw=True)
+    return wide(g, 4, cat(g, "cat", *((first, second) if a > b else (second, first))))
+def ghost_turned(g):
+    return ghost(g, 2, 3)
+def lateral(g):
+    x = g.conv(1, "data")
+    return wide(g, 4, cat(g, "cat", up(g, "up", x), g.conv(2, x)))
+def three(g):
+    x = g.conv(1, "data")
+    p = g.conv(2, x)
+    return wide(g, 4, cat(g, "cat", p, up(g, "up", x), g.conv(3, p, dw=True)))
+def two_readers(g):  # (beside the Concat a depthwise and a pointwise layer)
+    p = g.conv(2, g.conv(1, "data"))
+    out = wide(g, 4, cat(g, "cat", p, g.conv(3, p, dw=True)))
+    return g.sum("out", out, g.conv(5, p))
+def read_by_a_sum(g):
+    p = g.conv(2, g.conv(1, "data"))
+    return g.sum("out", wide(g, 4, cat(g, "cat", p, g.conv(3, p, dw=True))), p)
+def read_twice(g):
+    p = g.conv(2, g.conv(1, "data"))
+    c = cat(g, "cat", p, g.conv(3, p, dw=True))
+    return g.sum("out", wide(g, 4, c), wide(g, 5, c))
+def read_in_fp32(g):
+    x = g.conv(1, "data")
+    return up(g, "out", cat(g, "cat", up(g, "up", x), g.conv(2, x)))
+def the_same_twice(g):
+    p = g.conv(2, g.conv(1, "data"))
+    return wide(g, 4, cat(g, "cat", p, p))
+for light in (True, False):
+  for on in (1, 0):
+    fake.fake_set(b"slice", on)
+    for tail, slices in ((ghost, 2), (ghost_turned, 2), (lateral, 2), (three, 3), (two_readers, 2), (read_by_a_sum, 0), (read_twice, 2), (read_in_fp32, 0), (the_same_twice, 0)):
+        for ask in (None, "c2", "cat", "c3"):
+            if ask == "c3" and tail in (lateral, read_in_fp32, the_same_twice): continue
+            g = Graph(light)
+            out = tail(g)
+            g.ready()
+            for number, _ in getattr(g, "wide", []):
+                g.net.set_conv("c%d" % number, np.full((CH, (3 if tail is three else 2) * CH, 1, 1), number, np.int8), None, np.full(CH, 50, np.float32), 20.0, 10.0)
+            names = out if ask is None else ask + "," + out
+            s = g.net.session("data", blob(), names)
+            g.convs += getattr(g, "wide", [])
+            for k in range(5):
+                before, made = ran(g), fake.fake_count(b"slice")
+                s.run()
+                where = (tail.__name__, light, on, ask, k)
+                assert fetched(s) == g.expr[out], (where, fetched(s))
+                assert all(b - a == 1 for a, b in zip(before, ran(g))) or (light and ask), where
+                if not light or ask is None:
+                    assert (fake.fake_count(b"slice") - made == slices) or ask or not on, where
+                if not on or ask in ("cat", "c2"): assert fake.fake_count(b"slice") == made, where
+            if ask is None or not light:
+                assert expr_of(g.net.eval({"data": blob()}, out)) == g.expr[out], where
+            s.close()
+            g.net.close()
+""")
+
+
 def test_a_convolution_of_the_program_runs_its_own_forward(tmp_path):
     """Two pointwise layers that would be a pair, of a class that the program has put in the place of the library's."""
     run(tmp_path, r"""
