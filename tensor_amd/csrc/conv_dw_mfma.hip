@@ -205,7 +205,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
                       : DW_OOB;
         s_out = (unsigned)(n0 * C8 + o) * OHW * 32u;
         row_bytes = (unsigned)g.OW * 32u;
-    } else {  // Byte8: [N][C/8][OH*OW][8 bytes]
+    } else {  // Byte8: [N][C/8][OH*OW][8 bytes], or (EPI_F32_SLICE) a slice of such a blob: the quantized result where a Concat would put it
         const unsigned octets = EPI == EPI_F32_SLICE ? g.octets : (unsigned)C8;
         v_out = st_ok ? (unsigned)di * octets * OHW * 8u + (unsigned)ox * 8u + (S == 1 ? 0u : (unsigned)(q & 1) * 4u)
                       : DW_OOB;

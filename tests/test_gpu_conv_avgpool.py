@@ -52,6 +52,27 @@ def test_conv_avgpool_equals_layer_then_pooling(hip, oracle, C, K, N, H, W, k, p
     conv.close()
 
 
+@pytest.mark.parametrize("C,K,N,H,W,act,p0", [
+    (320, 1280, 26, 7, 7, 3, 0.0),   # workgroups of four waves: the fewest images that make 256 of them
+    (320, 1280, 25, 7, 7, 3, 0.0),   # and of one
+    (64, 40, 256, 8, 8, 4, 0.0),     # four waves, two of them without channels, and a sigmoid
+    (24, 8, 3, 4, 4, 2, 1.5),        # a LeakyReLU that is no maximum
+    (520, 96, 2, 5, 5, 2, 0.25),     # the looped form, an odd octet count
+])
+def test_conv_avgpool_equals_the_two_launches(hip, C, K, N, H, W, act, p0):
+    rng = np.random.default_rng(C + N)
+    conv = hip.conv(wq=rng.integers(-127, 128, (K, C, 1, 1)).astype(np.int8), scale_in=rng.uniform(2e-4, 1e-3, K).astype(np.float32) / np.float32(np.sqrt(C)),
+                    bias=rng.normal(0, 0.5, K).astype(np.float32), in_scale=25.0, act=act, act_p0=p0, out_kind=capi.OUT_F32)
+    assert conv.avgpool_launches(capi.I8_P8, N, H, W) == 1
+    x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
+    got = conv.forward_avgpool(x, capi.I8_P8, N, H, W).cpu().numpy().reshape(N, K)
+    blob = conv.forward(x, capi.I8_P8, N, H, W, capi.F32_P4).cpu().numpy().reshape(N, K // 4, H * W, 4).transpose(0, 1, 3, 2).reshape(N, K, H * W)
+    # a sum of H * W terms in fp32 is off by at most that many half units of the sum of their magnitudes
+    bound = H * W * 2.0 ** -24 * np.abs(blob).astype(np.float64).mean(axis=2) + 1e-30
+    assert (np.abs(got - blob.astype(np.float64).mean(axis=2)) <= bound).all()
+    conv.close()
+
+
 def test_conv_avgpool_refuses_an_int8_layer(hip):
     rng = np.random.default_rng(1)
     wq = rng.integers(-127, 128, (16, 16, 1, 1)).astype(np.int8)
