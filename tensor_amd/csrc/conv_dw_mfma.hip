@@ -81,21 +81,19 @@ __device__ __forceinline__ v4i dw_dequant4(const Epilogue& ep, const v4i& acc, c
 // argument is some 40 scalar instructions, and a short strip's wave issues few others). 152 bytes, where ConvGeom and Epilogue
 // made 268: the host writes launch arguments to device memory one by one (3.85 us a launch with 180 bytes, 3.35 with 96).
 struct DwArgs {
-    const float *scale_in, *bias;
-    union {
-        const float* scale_out;
-        float q[2];                     // EPI_F32_SLICE: the scale and the rounding constant of the quantized result
-    };
+    const float *scale_in, *bias, *scale_out;
     unsigned gx_m, gx, c8_m, chunks_m, chunks;  // divisions (FastDiv) by the workgroups along x, the octets, the column chunks of a row
     int N, H, W, OH, OW, rps;           // rps: output rows of a strip
     unsigned total, in_bytes, out_bytes;
-    float p0, lo, hi;                   // LeakyReLU slope, clamp of an fp32 result
-    union {                             // (with 12 bytes of its own for a slice every launch was 0.03 us longer)
-        float half;                     // rounding constant
-        unsigned octets;                // EPI_F32_SLICE: octets of an image of the blob that the result is a slice of
-    };
+    float p0, lo, hi, half;             // LeakyReLU slope, clamp of an fp32 result, rounding constant (EPI_F32_SLICE: of its quantization)
     unsigned short c8, lpi_m;           // octets; 1 / lane columns of an image, for lanes below 16 (16.8 fixed point)
     unsigned char gx_s, c8_s, chunks_s, lpi, ipw, ph, lrelu;  // ipw: images of a wave
+    // EPI_F32_SLICE: octets of an image of the blob that the result is a slice of. (In what was padding: with 12 bytes more every launch was
+    // 0.03 us longer. In a union with the words above they became an array in LDS and the launch three times as long.)
+    unsigned octets;
+    // and the scale of its quantization, in the clamp's or the slope's place, whichever the instance does not read
+    template <bool LR>
+    __device__ float q_scale() const { return LR ? lo : p0; }
 
     __device__ Epilogue epilogue() const {
         Epilogue ep{};
@@ -247,7 +245,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
         } else if constexpr (EPI == EPI_F32_SLICE) {  // (stride 1)
             v2i w2;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) w2[t] = quantize4(dw_dequant4<LR ? 1 : 0>(ep, cur[t % T], si[t % T], bi[t % T]), g.q[0], g.q[1]);
+            for (int t = 0; t < 2; ++t) w2[t] = quantize4(dw_dequant4<LR ? 1 : 0>(ep, cur[t % T], si[t % T], bi[t % T]), g.q_scale<LR>(), g.half);
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, w2), rout, (int)v_o, (int)s_row, 0);
         } else {
             constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
@@ -700,7 +698,8 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     pl.N = g.N, pl.H = g.H, pl.W = g.W, pl.OH = g.OH, pl.OW = g.OW, pl.ph = (unsigned char)g.ph, pl.rps = rps;
     pl.total = grid.x * grid.y, pl.in_bytes = in_bytes, pl.out_bytes = slice ? (unsigned)slice_bytes : out_bytes;
     pl.p0 = ep.act_p0, pl.lo = ep.act_lo, pl.hi = ep.act_hi, pl.half = ep.round_half, pl.lrelu = ep.lrelu;
-    if (slice) pl.octets = (unsigned)slice->slice_octets, pl.q[0] = slice->slice_scale, pl.q[1] = slice->slice_half;
+    if (slice) pl.octets = (unsigned)slice->slice_octets, pl.half = slice->slice_half, (ep.lrelu ? pl.lo : pl.p0) = slice->slice_scale;
+    static_assert(sizeof(DwArgs) == 112);
 #define OHIP_DWM_L(S_, E_, O_, K_)                                                                                        \
     do {                                                                                                                   \
         if (E_ != EPI_I8_P8_NONNEG && ep.lrelu)                                                                            \
