@@ -15,6 +15,9 @@
 //    from memory in a ring of four reduction steps that is refilled across pairs and layers: the first ones are requested before the
 //    depthwise layer begins, as are the elements of a residual or of a shuffle's other blob.
 //  * Behind a barrier they do the same for the second pointwise layer.
+// Vector issue is 40 % of the kernel's time, waits are half of it, at two to three waves a SIMD. In the detection model, 16 images, us as two
+// or three launches / as one, with the unit's shuffle and the next unit's first layer: 88 channels @52x52 5.1 + 14.3 / 15.8, 176 @26x26
+// 4.1 + 10.0 / 12.5, 352 @13x13 3.7 + 6.1 + 4.9 / 11.7; 5x5 with two pointwise layers, 64 @13x13 3.4 + 4.7 / 6.5.
 #include "conv_dwpw.hpp"
 
 #include "conv_pwpw_common.hpp"
