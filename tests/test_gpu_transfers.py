@@ -47,3 +47,30 @@ def test_copy_from_pinned_memory(hip, count):
     got = dev.cpu().numpy()
     assert (got[:count] == src).all() and not got[count:].any()
     hip._check(lib.otter_hip_host_free(pin))
+
+
+@pytest.mark.parametrize("count,offset", [(1, 0), (15, 0), (16, 0), (4000, 0), (4000, 4), (256 * 16 + 7, 0), (MIB - 1, 16), (MIB, 0), (MIB + 1, 0)])
+def test_download_behind_a_launch(hip, count, offset):
+    """One piece behind a launch of this thread goes through the copy kernel, from aligned memory of the GPU; from anywhere else and
+    on an idle stream through the runtime. On the null stream and on one of the program's."""
+    torch, lib = hip.torch, hip.lib
+    src = torch.from_numpy(np.random.default_rng(count).integers(0, 256, count + 64, dtype=np.uint8)).cuda()
+    pinned = torch.zeros(count + 64, dtype=torch.uint8, pin_memory=True)
+    torch.cuda.synchronize()
+
+    def check(at):
+        dev = torch.zeros(count + 64 + offset, dtype=torch.uint8, device="cuda")
+        hip._check(lib.otter_hip_copy(hip.ptr(dev), hip.ptr(src), C.c_size_t(count + 64), at))  # the launch in front
+        for _ in range(2):  # behind it, and on an idle stream
+            back = np.full(count + 1, 7, np.uint8)
+            hip._check(lib.otter_hip_download(C.c_void_p(back.ctypes.data), C.c_void_p(dev.data_ptr() + offset), C.c_size_t(count), at))
+            assert (back[:count] == src.cpu().numpy()[offset:offset + count]).all() and back[count] == 7
+
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            check(hip.stream())
+            # pinned host memory is not the GPU's: the runtime's copy, as ever
+            hip._check(lib.otter_hip_copy(hip.ptr(src), hip.ptr(src), C.c_size_t(16), hip.stream()))
+            back = np.full(count, 7, np.uint8)
+            hip._check(lib.otter_hip_download(C.c_void_p(back.ctypes.data), C.c_void_p(pinned.data_ptr()), C.c_size_t(count), hip.stream()))
+            assert not back.any()
