@@ -331,7 +331,7 @@ bool download_by_kernel(const void* src, size_t bytes, hipStream_t stream, const
     hipPointerAttribute_t at{};
     const bool ours = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices && pool == &g_staging[dev] &&
                       hipPointerGetAttributes(&at, src) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == dev;
-    if (!ours) (void)hipGetLastError();
+    (void)hipGetLastError();  // (the launch asks for it: an error that a caller's query has left there is none of the copy's)
     return ours;
 }
 
