@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
     struct {
         v4i v[2];
     } add;
-    const unsigned f_bytes = pa.total_pix * K0 * 4u;
+    const unsigned f_bytes = pa.total_pix * K0 * 4u;  // of an fp32 result or addend; an int8 result may be as many elements as this has bytes
     Epilogue ep0 = pp_epilogue(l0);
     if constexpr (FUSED) ep0.residual = ja.residual, ep0.twin = ja.twin;
     if constexpr (FUSED || SHUF) ep0.twin_scale = ja.twin_scale, ep0.twin_half = ja.twin_half;
@@ -304,7 +304,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
 
     // ---- the first pointwise layer --------------------------------------------------------------------------------------------------
     int8_t* const to1 = px1 + row1;  // this lane's pixel of the second layer's input
-    const __amdgpu_buffer_rsrc_t rout0 = NEXT ? rsrc(sum, sum != nullptr ? f_bytes : 0u) : rsrc(out, out == nullptr ? 0u : I8 ? f_bytes / 4u : f_bytes);
+    const __amdgpu_buffer_rsrc_t rout0 = NEXT ? rsrc(sum, sum != nullptr ? f_bytes : 0u) : rsrc(out, out == nullptr ? 0u : I8 ? pa.total_pix * K0 : f_bytes);
     // elements of a shuffle's blobs. The first half is Float4 or Float8: a store to Float4 touches 8 lines of 128 bytes where it touches 16
     // of Float8's, and the address unit works line by line (88 channels @52x52 b16 16.8 us
     // with Float8 on both sides, 16.4 with Float4; 176 channels on one 26x26 image 6.9 and 6.5)
@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
                 if constexpr (NEXT) {
                     if (ch0 < K0) *reinterpret_cast<v2i*>(to1 + ch0) = tw;
                 } else if (ep0.twin != nullptr) {  // K % 8 == 0 then: the lane's 8 channels are one Byte8 element
-                    store8(rsrc(ep0.twin, f_bytes / 4u), tw, ch0 < K0 ? at_b8(K0) : PR_OOB, (unsigned)pr * 32u * HW);
+                    store8(rsrc(ep0.twin, pa.total_pix * K0), tw, ch0 < K0 ? at_b8(K0) : PR_OOB, (unsigned)pr * 32u * HW);
                 }
             }
         }

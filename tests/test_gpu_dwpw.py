@@ -131,6 +131,19 @@ def test_one_launch_equals_the_layers(hip, C, k, stride, pad, dil, act, K, K2, n
             pw.close()
 
 
+@pytest.mark.parametrize("n", [16, 17])  # 2^30 bytes of int8 result, and 64 MiB more
+def test_an_int8_result_of_a_gigabyte(hip, n):
+    C, K, h, w = 64, 1024, 256, 256
+    rng = np.random.default_rng(n)
+    x = hip.to_device(rng.integers(-127, 128, n * C * h * w, dtype=np.int8))
+    dw, pw = depthwise(hip, rng, C, 3, 1, 1, 1, 0), layer(hip, rng, C, K, 2, False)
+    want = pw.forward(dw.forward(x, capi.I8_P8, n, h, w, capi.I8_P8), capi.I8_P8, n, h, w, capi.I8_P8)
+    dw.set_tile(-12, 0)
+    unwritten = hip.empty(n * K * h * w, np.int8).fill_(77)  # (the memory that the result is given next)
+    del unwritten
+    assert hip.torch.equal(hip.conv_dwpw(dw, pw, x, n, h, w), want)
+
+
 def test_what_is_refused(hip):
     rng = np.random.default_rng(3)
     n, h, w = 2, 6, 6
