@@ -21,6 +21,7 @@
 #include "conv_dwpw.hpp"
 
 #include "conv_pwpw_common.hpp"
+#include "dwpw_requests.hpp"
 
 #include <algorithm>
 
@@ -125,9 +126,9 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
         const int steps = second ? l1.steps : l0.steps, mt = second ? l1.mt : l0.mt;
         const __amdgpu_buffer_rsrc_t rw = rsrc(second ? l1.w : l0.w, (unsigned)steps * (unsigned)mt * 1024u);
         auto one = [&](int s) {
+            const unsigned at = dwpw_weights_at(step0 + s, steps, mt, pr);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-                a[s][h] = load16(rw, (lane * 16 | (step0 + s < steps ? 0u : PR_OOB)) + h * 1024, ((unsigned)(step0 + s) * (unsigned)mt + 2u * pr) * 1024u);
+            for (int h = 0; h < 2; ++h) a[s][h] = load16(rw, (lane * 16 | (step0 + s < steps ? 0u : PR_OOB)) + h * 1024, at);
         };
         one(0), one(1);
 #pragma unroll
@@ -147,16 +148,16 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
     if constexpr (FUSED || SHUF) ep0.twin_scale = ja.twin_scale, ep0.twin_half = ja.twin_half;
     const unsigned add_at = SHUF ? ja_pack(ja) == 8 ? at_f8(K0) : at_f4(K0) : at_f4(K0), add_half = SHUF && ja_pack(ja) == 8 ? 16u : HW * 16u;
     auto load_add = [&](int pr) {
-        const unsigned s = pr < pairs0 ? (unsigned)pr * 128u : 0u;
         if constexpr (PARTS) {
             if (pr < pairs0 && 32u * pr + 8 * q < K0 && ok)
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
                     add.v[h] = *reinterpret_cast<const v4i*>(epi4_residual_at(ep0, ja.join(), n, pix, (int)(32u * pr + 8 * q + 4 * h), (int)K0, (int)HW));
         } else if constexpr (FUSED || SHUF) {
-            const __amdgpu_buffer_rsrc_t r = rsrc(add_blob(ja), pr < pairs0 && add_blob(ja) != nullptr ? f_bytes : 0u);  // (none: zero, and not used)
+            const DwPwFloats f = dwpw_floats(pr < pairs0 && add_blob(ja) != nullptr, f_bytes, HW, add_half);  // (none: zero, and not used)
+            const __amdgpu_buffer_rsrc_t r = rsrc(add_blob(ja), f.bytes);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) add.v[h] = load16(r, add_at | (32u * pr + 8 * q + 4 * h < K0 ? 0u : PR_OOB), s * HW + h * add_half);
+            for (int h = 0; h < 2; ++h) add.v[h] = load16(r, add_at | (32u * pr + 8 * q + 4 * h < K0 ? 0u : PR_OOB), f.at(pr, h));
         }
     };
 
@@ -304,7 +305,9 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
 
     // ---- the first pointwise layer --------------------------------------------------------------------------------------------------
     int8_t* const to1 = px1 + row1;  // this lane's pixel of the second layer's input
-    const __amdgpu_buffer_rsrc_t rout0 = NEXT ? rsrc(sum, sum != nullptr ? f_bytes : 0u) : rsrc(out, out == nullptr ? 0u : I8 ? pa.total_pix * K0 : f_bytes);
+    float* const f_out = NEXT ? sum : static_cast<float*>(out);
+    const DwPwFloats f0 = dwpw_floats(f_out != nullptr, f_bytes, HW, HW * 16u);
+    const __amdgpu_buffer_rsrc_t rout0 = I8 ? rsrc(out, NEXT ? 0u : pa.total_pix * K0) : rsrc(f_out, f0.bytes);
     // elements of a shuffle's blobs. The first half is Float4 or Float8: a store to Float4 touches 8 lines of 128 bytes where it touches 16
     // of Float8's, and the address unit works line by line (88 channels @52x52 b16 16.8 us
     // with Float8 on both sides, 16.4 with Float4; 176 channels on one 26x26 image 6.9 and 6.5)
@@ -362,8 +365,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
 #pragma unroll
                         for (int e = 0; e < 4; ++e) r[h][e] = __float_as_int(__fadd_rn(__int_as_float(r[h][e]), __int_as_float(add.v[h][e])));
                     if (NEXT || ep0.twin != nullptr) tw[h] = quantize4(r[h], ep0.twin_scale, ep0.twin_half);
-                    // (no blob: a descriptor of no bytes, the store is dropped)
-                    store16(rout0, r[h], ch0 + 4 * h < K0 ? at_f4(K0) : PR_OOB, (unsigned)pr * 128u * HW + h * HW * 16u);
+                    store16(rout0, r[h], ch0 + 4 * h < K0 ? at_f4(K0) : PR_OOB, f0.at(pr, h));
                 }
                 if constexpr (NEXT) {
                     if (ch0 < K0) *reinterpret_cast<v2i*>(to1 + ch0) = tw;
