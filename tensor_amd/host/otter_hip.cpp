@@ -2874,7 +2874,8 @@ int Net::forward_dwpw_unit(int pointwise, int out_layer, int shortcut, int part1
     const int x = d->bottoms[0], made = forward_inputs(pointwise, {shortcut, part1, x}, blobs, opt);
     if (made) return made;
     const auto next = part1 < 0 ? next_units_.find(out_layer) : next_units_.end();
-    const bool with_next = next != next_units_.end() && !blobs[layers_[next->second]->tops[0]].defined();
+    // (not where this blob is what is asked for: with the next layer it may be left out, if it was not announced)
+    const bool with_next = next != next_units_.end() && !blobs[layers_[next->second]->tops[0]].defined() && opt.asked != e->tops[0];
     for (int k = with_next ? 0 : 1; k < 2; ++k) {
         ConvolutionLayer::DwPw u;
         u.next = k ? nullptr : static_cast<const ConvolutionLayer*>(layers_[next->second]);

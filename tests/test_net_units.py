@@ -348,6 +348,27 @@ for form in (3, 1):
 """)
 
 
+def test_a_blob_in_front_of_such_a_launch_is_there_unannounced(tmp_path):
+    """A program says that it will ask for the last blob, and asks for one whose only reader would run in the launch that makes it."""
+    run(tmp_path, BEHIND + r"""
+program = C.CDLL(sys.argv[2])
+program.program_extract.restype = C.c_long
+def read_by_one(g):
+    s = g.sum("s", g.conv(1, "data"), g.conv(4, g.conv(3, g.conv(2, "data", True), True, True)))
+    return g.conv(5, s)
+def without_a_sum(g):
+    return g.conv(4, g.conv(3, g.conv(2, g.conv(1, "data", True), True, True)))
+for light in (True, False):
+    for tail, asked in ((read_by_one, "s"), (without_a_sum, "c3")):
+        g = Graph(light)
+        out = tail(g)
+        g.ready()
+        n = program.program_extract(g.net.h, b"data", blob().ctypes.data_as(C.c_void_p), CH, SIDE, SIDE, out.encode(), asked.encode())
+        assert n >= 0 and fake.fake_expr(C.c_long(n)).decode() in (g.expr[asked], "q(%s)" % g.expr[asked]), (tail.__name__, light, n)
+        g.net.close()
+""", program=True)
+
+
 @pytest.mark.parametrize("light", [True, False])
 def test_a_max_pooling_in_the_launch_of_an_image_stem(tmp_path, light):
     run(tmp_path, r"""
