@@ -2532,6 +2532,24 @@ void Net::plan_fused_quantize() const {
     for (auto& u : shuffle_units_)
         if (u.second.next >= 0 && in_other_launch[u.second.next]) u.second.next = -1;
     for (auto it = next_units_.begin(); it != next_units_.end();) it = in_other_launch[it->second] ? next_units_.erase(it) : std::next(it);
+    // what is made of the result of a layer that could run in the launch in front of it
+    made_of_.clear();
+    auto follow = [&](int li) {
+        std::vector<char>& made = made_of_[li];
+        if (!made.empty()) return;
+        made.resize(blobs_.size());
+        std::vector<int> pending(layers_[li]->tops.begin(), layers_[li]->tops.end());
+        while (!pending.empty()) {
+            const int b = pending.back();
+            pending.pop_back();
+            if (made[b]) continue;
+            made[b] = 1;
+            for (int ci : blobs_[b].consumers) pending.insert(pending.end(), layers_[ci]->tops.begin(), layers_[ci]->tops.end());
+        }
+    };
+    for (const auto& u : next_units_) follow(u.second);
+    for (const auto& u : shuffle_units_)
+        if (u.second.next >= 0) follow(u.second.next);
     // Inverted-residual blocks: 1x1 (int8 result) -> depthwise (int8 result) -> 1x1, each blob with one reader
     block_units_.clear();
     for (size_t li = 0; li < layers_.size(); ++li) {
@@ -2700,7 +2718,7 @@ int Net::forward_conv_shuffle(const ShuffleUnit& u, std::vector<Tensor>& blobs, 
     const bool joined = u.crop_lo < 0;
     Tensor first, second;
     const int last = joined ? layers_[u.shuffle]->tops[0] : layers_[u.crop_hi]->tops[0];
-    const bool int8_only = u.hi_only && opt.wanted && !(*opt.wanted)[last], with_next = !joined && int8_only && u.next >= 0 && opt.asked != last;
+    const bool int8_only = u.hi_only && opt.wanted && !(*opt.wanted)[last], with_next = !joined && int8_only && u.next >= 0 && asked_for(u.next, last, opt);
     if (const ConvolutionLayer* d = front_of(u.conv, blobs, opt)) {
         // with the depthwise layer in front, and with the layer behind where that is a launch or that pair is none
         const int x = d->bottoms[0], made = forward_inputs(u.conv, {other, x}, blobs, opt);
@@ -2846,6 +2864,18 @@ const ConvolutionLayer* Net::front_of(int pointwise, const std::vector<Tensor>& 
     return blobs[b].defined() || opt.asked == b || (opt.wanted && (*opt.wanted)[b]) ? nullptr : static_cast<const ConvolutionLayer*>(layers_[f->second]);
 }
 
+// Whether a layer of made_of_ has to run for the blob that is being extracted, or for one that will be. (Not with the blob that it reads, if
+// that is being extracted: this may then be left out, and was not among those that were announced.)
+bool Net::asked_for(int layer, int reads, const NetOption& opt) const {
+    if (opt.asked == reads) return false;
+    const std::vector<char>& made = made_of_.at(layer);
+    if (opt.asked >= 0 && made[opt.asked]) return true;
+    if (opt.wanted)
+        for (size_t b = 0; b < made.size(); ++b)
+            if (made[b] && (*opt.wanted)[b]) return true;
+    return false;
+}
+
 // Whether the layer is the first of an inverted-residual block that runs in fewer launches than its layers on the blob x, or (d) on what
 // that depthwise layer makes of x.
 bool Net::begins_block(int li, const Tensor& x, const ConvolutionLayer* d) const {
@@ -2874,8 +2904,7 @@ int Net::forward_dwpw_unit(int pointwise, int out_layer, int shortcut, int part1
     const int x = d->bottoms[0], made = forward_inputs(pointwise, {shortcut, part1, x}, blobs, opt);
     if (made) return made;
     const auto next = part1 < 0 ? next_units_.find(out_layer) : next_units_.end();
-    // (not where this blob is what is asked for: with the next layer it may be left out, if it was not announced)
-    const bool with_next = next != next_units_.end() && !blobs[layers_[next->second]->tops[0]].defined() && opt.asked != e->tops[0];
+    const bool with_next = next != next_units_.end() && !blobs[layers_[next->second]->tops[0]].defined() && asked_for(next->second, e->tops[0], opt);
     for (int k = with_next ? 0 : 1; k < 2; ++k) {
         ConvolutionLayer::DwPw u;
         u.next = k ? nullptr : static_cast<const ConvolutionLayer*>(layers_[next->second]);

@@ -422,6 +422,9 @@ private:
     mutable std::map<int, int> front_units_;
     // layers with an fp32 blob that one pointwise int8 convolution reads quantized: the layer's index -> the convolution's
     mutable std::map<int, int> next_units_;
+    // of those and of the layers behind a unit's second half: by blob, whether it is made of the layer's result
+    mutable std::map<int, std::vector<char>> made_of_;
+    bool asked_for(int layer, int reads, const NetOption& opt) const;
     // Concat layers whose result only int8 convolutions read, every blob of it made by a layer that can write its channels of the quantized
     // result itself: the Concat's index -> those layers, in the order in which they run
     struct SlicePart {

@@ -370,6 +370,53 @@ for light in (True, False):
 
 
 @pytest.mark.parametrize("light", [True, False])
+def test_no_layer_runs_that_nobody_asked_for(tmp_path, light):
+    """A blob in front of a layer that could run in the same launch, and one on another way through the net."""
+    run(tmp_path, BEHIND + r"""
+import re
+def two_heads(g):  # c5 reads the sum of a block, and so does a mean
+    s = g.sum("s", g.conv(1, "data"), g.conv(4, g.conv(3, g.conv(2, "data", True), True, True)))
+    g.mean("m", s)
+    return g.conv(5, s)
+for form in (3, 1):
+    for join, pair, behind in ((1, 1, 1), (1, 1, 0), (0, 1, 1), (1, 0, 1)):
+        set_all(form=form, join=join, pair=pair, dwpw_next=behind)
+        for tail in TAILS + MORE + [two_heads]:
+            probe = Graph(%s)
+            tail(probe)
+            asks = sorted(n for n in probe.expr if n != "data" and "_" not in n or n in ("u_lo", "u_hi", "v_lo", "v_hi"))
+            probe.ready().net.close()
+            for ask in asks:
+                g = Graph(%s)
+                tail(g)
+                g.ready()
+                s = g.net.session("data", blob(), ask)
+                before = ran(g)
+                s.run()
+                got, want = fetched(s), g.expr[ask]
+                assert got in (want, "q(%%s)" %% want), (tail.__name__, ask, got)
+                used = set(re.findall(r"c(\d+)\(", want))
+                once = {n: b - a for (n, _), a, b in zip(g.convs, before, ran(g))}
+                assert once == {n: int(str(n) in used) for n, _ in g.convs}, (tail.__name__, form, join, pair, behind, ask, once)
+                s.close()
+                g.net.close()
+set_all(form=3, join=1, pair=1, dwpw_next=1)
+for asks, launches in (("m", 0), ("m,c5", 1), ("c5", 1)):  # (wanted later in the pass: run now)
+    g = Graph(%s)
+    two_heads(g)
+    g.ready()
+    s = g.net.session("data", blob(), asks)
+    before, made = ran(g), fake.fake_count(b"dwpw_next")
+    s.run()
+    assert fetched(s) == g.expr[asks.split(",")[-1]]
+    assert fake.fake_count(b"dwpw_next") - made == launches, asks
+    assert [b - a for a, b in zip(before, ran(g))] == [1, 1, 1, 1, launches], asks
+    s.close()
+    g.net.close()
+""" % (light, light, light))
+
+
+@pytest.mark.parametrize("light", [True, False])
 def test_a_max_pooling_in_the_launch_of_an_image_stem(tmp_path, light):
     run(tmp_path, r"""
 CH3 = 3
