@@ -1995,9 +1995,9 @@ int otter_hip_conv_dwpw_forward(const otter_hip_conv_t* d, const otter_hip_conv_
     if (rc) return rc;
     const otter_hip_conv_t* const nx = end->next;
     if (!in || (!out && (nx || (!end->other && !end->out_q)))) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_dwpw_forward: null");
+    if (n == 0) return OTTER_HIP_OK;
     if (!dwpw_one_launch(d, p, nx, a))
         return fail(OTTER_HIP_ERR_UNSUPPORTED, "otter_hip_conv_dwpw_forward: not a single launch (otter_hip_conv_dwpw_launches)");
-    if (n == 0) return OTTER_HIP_OK;
     const int8_t* const w[2] = {p->w_igemm, nx ? nx->w_igemm : nullptr};
     const float so[2] = {p->so_one, nx ? nx->so_one : 1.f};
     OHIP_CHECK(run_conv_dwpw((const int8_t*)in, d->w_dwpw, d->so_one, a.g[0], a.ep[0], w, so, out, end->sum, a.g[1], a.ep[1],
@@ -2255,6 +2255,7 @@ int otter_hip_conv_forward_slice(const otter_hip_conv_t* h, const void* in, int 
         return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_slice: unknown rounding mode");
     const ConvGeom g = make_geom(h->d, n, in_h, in_w);
     if (g.OH < 1 || g.OW < 1) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_forward_slice: empty output");
+    if (n == 0) return OTTER_HIP_OK;
     Epilogue ep = make_epilogue(h, OTTER_HIP_F32_P4);
     JoinArgs ja;
     ja.slice = blob + (size_t)first_channel * g.OH * g.OW, ja.slice_octets = total_channels / 8;

@@ -1,5 +1,7 @@
 """otter_hip_conv_dwpw_forward: a depthwise layer, the pointwise layer behind it and the one behind that in one launch. The results must be,
 bit for bit, what the layers give one by one through the calls for what their ends carry."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -142,6 +144,14 @@ def test_an_int8_result_of_a_gigabyte(hip, n):
     unwritten = hip.empty(n * K * h * w, np.int8).fill_(77)  # (the memory that the result is given next)
     del unwritten
     assert hip.torch.equal(hip.conv_dwpw(dw, pw, x, n, h, w), want)
+
+
+def test_an_empty_batch(hip):
+    rng = np.random.default_rng(1)
+    dw, pw, buf, end = depthwise(hip, rng, 64, 3, 1, 1, 1, 0), layer(hip, rng, 64, 64, 0, False), hip.empty(64, np.int8).fill_(5), hip._end({})
+    call = lambda n, h: hip.lib.otter_hip_conv_dwpw_forward(dw.h, pw.h, hip.ptr(buf), n, h, 6, ctypes.byref(end), hip.ptr(buf), capi.I8_P8, hip.stream())
+    assert call(0, 6) == 0 and (buf == 5).all()
+    assert call(0, 0) < 0 and call(-1, 6) < 0
 
 
 def test_what_is_refused(hip):

@@ -78,6 +78,16 @@ def test_upsample(hip, c, n, h, w, oh, ow, layout):
             check_slice(hip, blob, quantized(hip, y, capi.F32_P8, n, c, oh, ow, scale, rounding), n, c, oh, ow)
 
 
+def test_an_empty_batch(hip):
+    conv = hip.conv(wq=np.ones((16, 16, 1, 1), np.int8), scale_in=np.full(16, 0.01, np.float32), in_scale=31.0, out_kind=capi.OUT_F32)
+    x, blob = hip.to_device(np.zeros(16, np.int8)), hip.to_device(np.full(32, FILL, np.int8))
+    conv.forward_slice(x, capi.I8_P8, 0, 5, 5, blob, 32, 16, 10.0)
+    hip.upsample2d_slice(x, capi.F32_P8, (0, 16, 5, 5), (10, 10), 1, False, blob, 32, 16, 10.0, capi.ROUND_SSE)
+    assert (blob == FILL).all()
+    with pytest.raises(capi.HipError):
+        conv.forward_slice(x, capi.I8_P8, 0, 5, 5, blob, 32, 24, 10.0)
+
+
 def test_what_is_refused(hip):
     rng = np.random.default_rng(5)
     conv = hip.conv(wq=rng.integers(-127, 128, (16, 16, 1, 1)).astype(np.int8), scale_in=np.full(16, 0.01, np.float32), in_scale=31.0, out_kind=capi.OUT_F32)
