@@ -323,10 +323,11 @@ void staging_put(StagingPool& pool, Staging& s) {
 
 // Whether a download of one piece goes through a copy kernel. Behind work that is still running the runtime's copy starts some 10 us after it
 // (the result of the classifier at batch 64, 256 KB: 391 us a pass, 378 with the kernel; of the detection model at batch 16, 352 KB: 564 and
-// 550); on an idle stream its copy is the faster one (32 KB 11 and 15 us, 256 KB 20 and 24). To ask the stream which it is costs 5 us of
-// them, so the thread's own launches say it. Only for memory of the current GPU, which is the stream's: the runtime copies from anywhere.
+// 550); on an idle stream its copy is the faster one (up to 4 KB level, 32 KB 10.4 and 14.3 us, 256 KB 20.2 and 23.1). To ask the stream which
+// it is costs 5 us of them where it is running, so the thread's own launches say it; a thread that has waited for its launches by other means
+// than the library's pays those 3 to 4 us. Only for memory of the current GPU, which is the stream's: the runtime copies from anywhere.
 bool download_by_kernel(const void* src, size_t bytes, hipStream_t stream, const StagingPool* pool) {
-    if (!t_launched || bytes > kStagingBytes || ((uintptr_t)src & 15)) return false;
+    if (!t_launched.is(stream) || bytes > kStagingBytes || ((uintptr_t)src & 15)) return false;
     int dev = -1;
     hipPointerAttribute_t at{};
     const bool ours = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices && pool == &g_staging[dev] &&
@@ -388,7 +389,7 @@ int otter_hip_download(void* dst, const void* src, size_t bytes, void* stream_) 
             if (e == hipSuccess) std::memcpy((char*)dst + (c - 1) * kStagingBytes, b.host, length(c - 1));
         }
     }
-    t_launched = false;  // (the copy is one, and waited for)
+    t_launched.waited_for(stream);
     if (e != hipSuccess) (void)hipStreamSynchronize(stream);  // nothing may still write into a buffer that goes back
     if (pool)
         for (Staging& b : s) staging_put(*pool, b);
@@ -409,7 +410,7 @@ int otter_hip_stream_destroy(void* stream) {
 }
 
 int otter_hip_stream_synchronize(void* stream) {
-    t_launched = false;
+    t_launched.waited_for((hipStream_t)stream);
     OHIP_CHECK(hipStreamSynchronize((hipStream_t)stream));
     return OTTER_HIP_OK;
 }
@@ -469,7 +470,7 @@ int otter_hip_record_end(void* stream, otter_hip_recording_t** recording) {
 int otter_hip_record_launch(otter_hip_recording_t* recording, void* stream) {
     if (!recording) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_record_launch: null");
     OHIP_CHECK(hipGraphLaunch(recording->exec, (hipStream_t)stream));
-    t_launched = true;
+    t_launched.set((hipStream_t)stream);
     return OTTER_HIP_OK;
 }
 

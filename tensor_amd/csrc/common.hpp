@@ -11,8 +11,16 @@
 
 namespace ohip {
 
-// This thread has launched since it last waited for a stream in a call of the library (otter_hip_download chooses by it how it copies).
-inline thread_local bool t_launched = false;
+// The stream of this thread's last launch, unless it has waited for that stream in a call of the library since (otter_hip_download chooses by
+// it how it copies).
+struct LaunchedOn {
+    bool any = false;
+    hipStream_t stream = nullptr;
+    void set(hipStream_t s) { any = true, stream = s; }
+    void waited_for(hipStream_t s) { any = any && stream != s; }
+    bool is(hipStream_t s) const { return any && stream == s; }
+};
+inline thread_local LaunchedOn t_launched;
 
 // A launch without the call configuration that the <<<>>> form pushes and pops: 0.05 to 0.2 us of the host's time less (112 bytes of arguments,
 // 4000 in a row: 2.48 -> 2.43 us in one process, 3.90 -> 3.73 in another). The error, if any, is there for hipGetLastError.
@@ -22,7 +30,7 @@ inline void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipS
     [&](P... p) {
         void* ptrs[] = {const_cast<void*>(static_cast<const void*>(&p))...};
         (void)hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, ptrs, lds, stream);
-        t_launched = true;
+        t_launched.set(stream);
     }(std::forward<A>(args)...);
 }
 

@@ -51,8 +51,8 @@ def test_copy_from_pinned_memory(hip, count):
 
 @pytest.mark.parametrize("count,offset", [(1, 0), (15, 0), (16, 0), (4000, 0), (4000, 4), (256 * 16 + 7, 0), (MIB - 1, 16), (MIB, 0), (MIB + 1, 0)])
 def test_download_behind_a_launch(hip, count, offset):
-    """One piece behind a launch of this thread goes through the copy kernel, from aligned memory of the GPU; from anywhere else and
-    on an idle stream through the runtime. On the null stream and on one of the program's."""
+    """The bytes of a download behind a launch of this thread, by the copy kernel where its conditions hold (one piece of aligned memory of
+    the GPU; test_staging.py sees which way each goes), and of one on an idle stream. On the null stream and on one of the program's."""
     torch, lib = hip.torch, hip.lib
     src = torch.from_numpy(np.random.default_rng(count).integers(0, 256, count + 64, dtype=np.uint8)).cuda()
     pinned = torch.zeros(count + 64, dtype=torch.uint8, pin_memory=True)

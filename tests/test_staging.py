@@ -71,6 +71,48 @@ good(*upload(100))
 fake.fake_capture(0)
 good(*upload(100, s), s)
 """,
+    # behind a launch of this thread on its stream one piece of the GPU's aligned memory goes by a kernel, everything else by the runtime
+    "which way a download goes": """
+import threading
+MIB = 1 << 20
+memory = np.zeros(2 * MIB, np.uint8)
+memory[:] = rng.integers(0, 256, memory.size)
+base = (-memory.ctypes.data) % 16
+def launch(stream=None):
+    a = np.zeros(64, np.uint8)
+    assert lib.otter_hip_copy(C.c_void_p(memory.ctypes.data), C.c_void_p(memory.ctypes.data), C.c_size_t(16), C.c_void_p(stream)) == 0
+def way(stream=None, count=4000, offset=0, of=0):
+    fake.fake_memory_of(of)
+    before, back = (fake.fake_copies(), fake.fake_launches()), np.zeros(count, np.uint8)
+    assert lib.otter_hip_download(C.c_void_p(back.ctypes.data), C.c_void_p(memory.ctypes.data + base + offset), C.c_size_t(count), C.c_void_p(stream)) == 0
+    assert (back == memory[base + offset:base + offset + count]).all()
+    fake.fake_memory_of(0)
+    copies, launches = fake.fake_copies() - before[0], fake.fake_launches() - before[1]
+    assert copies + launches == (count + MIB - 1) // MIB and (not copies or not launches)
+    return "kernel" if launches else "runtime"
+a, b, other_gpu = fake.fake_stream(0), fake.fake_stream(0), fake.fake_stream(1)
+for s in (None, a):
+    assert way(s) == "runtime"
+    launch(s)
+    assert way(s) == "kernel" and way(s) == "runtime"  # (the first one has waited)
+    for kw, how in ((dict(offset=4), "runtime"), (dict(offset=16), "kernel"), (dict(count=1), "kernel"), (dict(count=MIB), "kernel"), (dict(count=MIB + 1), "runtime"),
+                    (dict(of=-1), "runtime"), (dict(of=1), "runtime")):
+        launch(s)
+        assert way(s, **kw) == how, kw
+    launch(s)
+    assert lib.otter_hip_stream_synchronize(C.c_void_p(s)) == 0 and way(s) == "runtime"
+# a launch on one stream says nothing of another one
+launch(a)
+assert way(b) == "runtime" and way(None) == "runtime" and way(a) == "kernel"
+launch(None)
+assert lib.otter_hip_stream_synchronize(C.c_void_p(a)) == 0 and way(a) == "runtime" and way(None) == "kernel"
+launch(other_gpu)
+assert way(other_gpu) == "runtime"  # (memory of the current GPU alone)
+# nor does another thread's
+t = threading.Thread(target=launch, args=(a,))
+t.start(), t.join()
+assert way(a) == "runtime"
+""",
     # buffers are kept up to 16 per GPU
     "what is kept": """
 for device in (0, 1):
