@@ -330,10 +330,12 @@ bool download_by_kernel(const void* src, size_t bytes, hipStream_t stream, const
     if (!t_launched.is(stream) || bytes > kStagingBytes || ((uintptr_t)src & 15)) return false;
     int dev = -1;
     hipPointerAttribute_t at{};
-    const bool ours = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices && pool == &g_staging[dev] &&
-                      hipPointerGetAttributes(&at, src) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == dev;
-    (void)hipGetLastError();  // (the launch asks for it: an error that a caller's query has left there is none of the copy's)
-    return ours;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices || pool != &g_staging[dev]) return false;
+    if (hipPointerGetAttributes(&at, src) != hipSuccess) {
+        (void)hipGetLastError();  // (the query's: the runtime's copy may still know the memory)
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == dev;
 }
 
 }  // namespace
@@ -379,7 +381,7 @@ int otter_hip_download(void* dst, const void* src, size_t bytes, void* stream_) 
     for (size_t c = 0; c <= chunks && e == hipSuccess; ++c) {
         if (c < chunks) {
             Staging& b = s[c & 1];
-            e = kernel ? run_copy_bytes(src, b.host, bytes, stream)
+            e = kernel ? launch_copy_bytes(src, b.host, bytes, stream)
                        : hipMemcpyAsync(b.host, (const char*)src + c * kStagingBytes, length(c), hipMemcpyDeviceToHost, stream);
             if (e == hipSuccess && chunks > 1) e = staging_record(b, stream);
         }

@@ -23,15 +23,20 @@ struct LaunchedOn {
 inline thread_local LaunchedOn t_launched;
 
 // A launch without the call configuration that the <<<>>> form pushes and pops: 0.05 to 0.2 us of the host's time less (112 bytes of arguments,
-// 4000 in a row: 2.48 -> 2.43 us in one process, 3.90 -> 3.73 in another). The error, if any, is there for hipGetLastError.
+// 4000 in a row: 2.48 -> 2.43 us in one process, 3.90 -> 3.73 in another). The error, if any, is there for hipGetLastError; launched
+// returns it.
+template <typename... P, typename... A>
+inline hipError_t launched(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, A&&... args) {
+    static_assert(sizeof...(P) == sizeof...(A), "one argument for each parameter");
+    return [&](P... p) {
+        void* ptrs[] = {const_cast<void*>(static_cast<const void*>(&p))...};
+        t_launched.set(stream);
+        return hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, ptrs, lds, stream);
+    }(std::forward<A>(args)...);
+}
 template <typename... P, typename... A>
 inline void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, A&&... args) {
-    static_assert(sizeof...(P) == sizeof...(A), "one argument for each parameter");
-    [&](P... p) {
-        void* ptrs[] = {const_cast<void*>(static_cast<const void*>(&p))...};
-        (void)hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, ptrs, lds, stream);
-        t_launched.set(stream);
-    }(std::forward<A>(args)...);
+    (void)launched(kernel, grid, block, lds, stream, std::forward<A>(args)...);
 }
 
 // ---------------------------------------------------------------------------------------------------

@@ -149,6 +149,7 @@ hipError_t run_repack(const void* src, int sp, void* dst, int dp, int elem_bytes
 
 
 // glue.hip
+hipError_t launch_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream);  // (without a look at hipGetLastError)
 hipError_t run_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream);
 hipError_t run_eltwise_add(const float* a, const float* b, float* out, size_t n, hipStream_t stream);
 hipError_t run_activation(float* x, size_t n, int act, float p0, hipStream_t stream);

@@ -116,10 +116,15 @@ __global__ void __launch_bounds__(256) copy_bytes_kernel(const uint4* __restrict
         reinterpret_cast<char*>(dst)[n16 * 16 + threadIdx.x] = reinterpret_cast<const char*>(src)[n16 * 16 + threadIdx.x];
 }
 
-hipError_t run_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream) {
+// (the launch's own error: what an earlier call of the program's has left for hipGetLastError stays there)
+hipError_t launch_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream) {
     const size_t n16 = bytes / 16;
     const unsigned blocks = (unsigned)(n16 < 256 * 256 ? (n16 + 255) / 256 : 256);
-    launch(copy_bytes_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, stream, (const uint4*)src, (uint4*)dst, n16, bytes, blocks * 256);
+    return launched(copy_bytes_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, stream, (const uint4*)src, (uint4*)dst, n16, bytes, blocks * 256);
+}
+
+hipError_t run_copy_bytes(const void* src, void* dst, size_t bytes, hipStream_t stream) {
+    (void)launch_copy_bytes(src, dst, bytes, stream);
     return hipGetLastError();
 }
 

@@ -113,6 +113,22 @@ t = threading.Thread(target=launch, args=(a,))
 t.start(), t.join()
 assert way(a) == "runtime"
 """,
+    # an error that a call of the program's own has left is none of the copy's, and is still there for the program to see
+    "an error of the program's own": """
+data, back = rng.integers(0, 256, 4000, dtype=np.uint8), np.zeros(4000, np.uint8)
+memory = np.zeros(4016, np.uint8)
+memory = memory[(-memory.ctypes.data) % 16:][:4000]
+memory[:] = data
+args = [C.c_void_p(back.ctypes.data), C.c_void_p(memory.ctypes.data), C.c_size_t(4000), None]
+assert lib.otter_hip_download(*args) == 0
+for launched in (0, 1):
+    if launched: assert lib.otter_hip_copy(C.c_void_p(memory.ctypes.data), C.c_void_p(memory.ctypes.data), C.c_size_t(4000), None) == 0
+    fake.fake_error(9)
+    back[:] = 0
+    launches = fake.fake_launches()
+    assert lib.otter_hip_download(*args) == 0 and (back == data).all() and fake.fake_launches() - launches == launched
+    assert fake.hipGetLastError() == 9 and fake.hipGetLastError() == 0
+""",
     # buffers are kept up to 16 per GPU
     "what is kept": """
 for device in (0, 1):
