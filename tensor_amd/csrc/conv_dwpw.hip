@@ -451,7 +451,8 @@ bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom
 }
 
 // Cost models in us, fitted to launches replayed from captured graphs behind a copy that leaves the L2 caches cold, over 2500 drawn layers
-// (16 to 960 channels, 4x4 to 112x112 pixels, batches of 1 to 64, every end): half of them within 5 %, nine in ten within 13 %. The launch:
+// (16 to 960 channels, 4x4 to 112x112 pixels, batches of 1 to 64, every end): half of them within 6 %, nine in ten within 15 %, and so are
+// both models over 2500 others. The launch:
 // a wave walks nd pairs of octets and n0 and n1 pairs of row tiles one behind the other, once if every workgroup is resident, and the more
 // often the more of eight waves there are for a compute unit.
 struct DwPwShape {
@@ -498,12 +499,16 @@ static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0,
         }
     return best;
 }
-// Over the drawn layers the rule takes two thirds and gives 0.88 of the time; 36 of the 2500 are over 5 % slower. (Five taps a row are where
-// the launch's loads cost most: nearer to the line it loses.)
+// Over 2500 layers drawn anew the rule takes 61 % and gives 0.89 of the time; 20 of them are over 5 % slower than apart, the worst 1.27. Five
+// taps a row are where the launch's loads cost most: nearer to the line it loses. So it does with 640 channels and more on many pixels,
+// where every workgroup of 32 pixels streams 0.4 MB of weights and up and its LDS leaves few of them on a compute unit: between 0.84 and 0.92 of
+// the models' time apart it took 0.98 of the real one, up to 1.50 (664 -> 664 -> 32 @49x49, 7 images: 41.9 us apart, 62.7).
 bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
     double cost = 0;
     dwpw_plan(gd, g0, e0, g1, &cost);
-    return cost < (gd.kh == 5 ? 0.90 : 0.92) * dwpw_cost_apart(DwPwShape(gd, g0, e0, g1), gd, g0, g1);
+    const DwPwShape s(gd, g0, e0, g1);
+    const double line = s.k5 ? 0.90 : gd.C >= 640 && s.px >= 4096 ? 0.84 : 0.92;
+    return cost < line * dwpw_cost_apart(s, gd, g0, g1);
 }
 
 template <int NW, int TAPS, int EPI, int KIND1>

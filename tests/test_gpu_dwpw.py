@@ -133,6 +133,31 @@ def test_one_launch_equals_the_layers(hip, C, k, stride, pad, dil, act, K, K2, n
             pw.close()
 
 
+@pytest.mark.parametrize("C,k,stride,K,K2,n,side,form,ratio", [
+    # drawn layers, the launch's time over that of the layers one by one where the rule was measured
+    (32, 3, 1, 32, 32, 6, 88, "shuffle", 0.60), (72, 3, 1, 72, 24, 9, 13, "sum", 0.61), (48, 3, 1, 16, 96, 7, 19, "f32", 0.62),
+    (120, 3, 1, 32, 0, 6, 24, "i8", 0.71), (128, 5, 1, 128, 112, 16, 13, "i8", 0.75),
+    (952, 3, 2, 952, 0, 2, 8, "f32", 3.47), (600, 5, 2, 600, 0, 1, 10, "i8", 2.99), (848, 3, 1, 848, 848, 3, 10, "i8", 2.56),
+    # many channels and many pixels, where the models are too kind to the launch
+    (664, 3, 1, 664, 32, 7, 49, "f32", 1.50), (696, 3, 1, 696, 120, 4, 75, "i8", 1.47), (904, 3, 2, 904, 904, 3, 78, "f32", 1.19),
+])
+def test_the_launch_is_taken_where_it_is_faster(hip, C, k, stride, K, K2, n, side, form, ratio):
+    """Which way the rule decides by itself, and the result of the plan that it chooses."""
+    rng = np.random.default_rng(C + side)
+    dw, pw = depthwise(hip, rng, C, k, stride, k // 2, 1, 0), layer(hip, rng, C, K, 0, form != "i8")
+    nx = layer(hip, rng, K, K2, 2, False) if K2 else None
+    x = hip.to_device(rng.integers(-127, 128, n * C * side * side, dtype=np.int8))
+    some = hip.empty(4, np.float32)  # (of the pointers it is only asked which are null)
+    end = dict(dict(q_scale=19.0, q_round_mode=1) if nx and form != "i8" else {}, **{"shuffle": dict(other=some, other_layout=capi.F32_P8, first_half=some),
+                                                                                     "sum": dict(residual=some)}.get(form, {}))
+    assert hip.conv_dwpw_launches(dw, pw, n, side, side, next=nx, **end) == (1 if ratio < 1 else 2)
+    if ratio < 1:
+        dw.force = (0, 0)
+        got, want = one_and_two(hip, rng, form, dict(odd=0, layout=capi.F32_P8), dw, pw, nx, x, n, side, side)
+        for g, v in zip(got, want):
+            assert hip.torch.equal(g, v)
+
+
 @pytest.mark.parametrize("n", [16, 17])  # 2^30 bytes of int8 result, and 64 MiB more
 def test_an_int8_result_of_a_gigabyte(hip, n):
     C, K, h, w = 64, 1024, 256, 256
