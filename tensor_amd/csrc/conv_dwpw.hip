@@ -122,13 +122,13 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
     // ---- the pointwise weights: four reduction steps of a pair ----------------------------------------------------------------------
     v4i a[SC][2];
     // (second: of the second layer. Chosen by values and not by branches: behind a branch a wave waits for the loads in front of it)
-    auto load_a = [&](bool second, int pr, int step0) {  // (steps that do not exist: past the weights, zero)
+    auto load_a = [&](bool second, int pr, int step0) {  // (steps that do not exist: at the weights' end, zero)
         const int steps = second ? l1.steps : l0.steps, mt = second ? l1.mt : l0.mt;
         const __amdgpu_buffer_rsrc_t rw = rsrc(second ? l1.w : l0.w, (unsigned)steps * (unsigned)mt * 1024u);
         auto one = [&](int s) {
             const unsigned at = dwpw_weights_at(step0 + s, steps, mt, pr);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) a[s][h] = load16(rw, (lane * 16 | (step0 + s < steps ? 0u : PR_OOB)) + h * 1024, at);
+            for (int h = 0; h < 2; ++h) a[s][h] = load16(rw, lane * 16 + h * 1024, at);
         };
         one(0), one(1);
 #pragma unroll

@@ -14,9 +14,9 @@ namespace ohip {
 // not wrap: no scalar offset here is beyond the bytes.
 
 // Step `step` of the `steps` reduction steps of row tiles 2 pair, 2 pair + 1 (mt tiles a step, 1024 bytes each). A step that does not exist is
-// asked for at the weights' begin, by lanes whose own offsets are beyond them.
+// asked for at the weights' very end, where every lane is out of range.
 OHIP_DWPW_FN unsigned dwpw_weights_at(int step, int steps, int mt, int pair) {
-    return step < steps ? ((unsigned)step * (unsigned)mt + 2u * (unsigned)pair) * 1024u : 0u;
+    return step < steps ? ((unsigned)step * (unsigned)mt + 2u * (unsigned)pair) * 1024u : (unsigned)steps * (unsigned)mt * 1024u;
 }
 
 // An fp32 blob of `bytes` bytes of which a lane reads or writes two elements of four channels for a pair of row tiles, `half` bytes apart, and

@@ -23,6 +23,7 @@ int main() {
                 for (int pair = 0; pair < pairs; ++pair) {
                     const u64 at = dwpw_weights_at(step, steps, mt, pair);
                     if (at > bytes) return fail("weights: beyond them", step, steps, K, pair);
+                    if (step >= steps && at != bytes) return fail("weights: a step that does not exist", step, steps, K, pair);  // (every lane is out of range there)
                     if (step < steps && at != ((u64)step * mt + 2 * pair) * 1024) return fail("weights: another step", step, steps, K, pair);
                 }
         }
