@@ -342,7 +342,7 @@ for form in (3, 1):
                 for _ in range(5):
                     s.run()
                     got, want = fetched(s), g.expr[ask.split(",")[-1]]
-                    assert got in (want, "q(%s)" % want), (tail.__name__, ask, light, got)
+                    assert got == want, (tail.__name__, ask, light, got)
                 s.close()
                 g.net.close()
 """)
@@ -394,7 +394,7 @@ for form in (3, 1):
                 before = ran(g)
                 s.run()
                 got, want = fetched(s), g.expr[ask]
-                assert got in (want, "q(%%s)" %% want), (tail.__name__, ask, got)
+                assert got == want, (tail.__name__, ask, got)
                 used = set(re.findall(r"c(\d+)\(", want))
                 once = {n: b - a for (n, _), a, b in zip(g.convs, before, ran(g))}
                 assert once == {n: int(str(n) in used) for n, _ in g.convs}, (tail.__name__, form, join, pair, behind, ask, once)
@@ -443,7 +443,7 @@ for on in (1, 0):
         for _ in range(5):
             s.run()
             got, want = expr_of(s.fetch((2 * 8 * 64,), np.float32)), expr[ask.split(",")[-1]]
-            assert got in (want, "q(%%s)" %% want), (on, ask, got)
+            assert got == want, (on, ask, got)
         assert (fake.fake_count(b"stem_pool") > launches) == (on and "c1" not in ask), (on, ask)
         s.close()
         net.close()
