@@ -177,8 +177,9 @@ __global__ void __launch_bounds__(256) conv_stem3x3_kernel(const void* __restric
 // A workgroup (4 waves) owns R output rows of one image. LDS: [input row r < RIN][channel][pitch_dw dwords] of int8;
 // dword d of a line holds pixels 4*(d-1) .. 4*(d-1)+3 (dword 0 and everything past the row's end are zeros: the
 // padding columns), rows outside the image are zeros.
+enum { STEM_VALUES, STEM_UNITS, STEM_LINES };  // how the strip is loaded
 struct StemPlan {
-    int R, strips, cgs, RIN, pitch_dw, vec;
+    int R, strips, cgs, RIN, pitch_dw, fill;
     FastDiv by_strips, by_cgs;
     float inv_pitch, inv_c;
 };
@@ -187,50 +188,99 @@ constexpr int STEM_UN = 8;        // 4-pixel units a thread has in flight while 
 constexpr int STEM_POOL_ROWS = 4;  // pooled rows per workgroup with the pooling behind it (2, 4 level from 16 images on, 8 slower below 64)
 constexpr int STEM_LDS_ROWS = 4;  // output rows per workgroup (measured: 2, 4, 8 within 5 % of each other at 224 x 224, 16 slower)
 
-// Input rows iy0 .. iy0 + RIN - 1 of an image, quantized, into the LDS lines of a strip, a load per unit of four pixels: fp32 rows of four
-// pixels and more (16-byte loads need 4-byte alignment; the last unit of a row of no whole units is loaded where it ends with the row and
-// moved down), int8 rows of whole, aligned units. A wave takes lines, 64 units of one at a time: row and channel of a line are scalar, what is outside the image lies
-// outside a descriptor and is zero, and a unit costs its quantization and little else (a thread per unit that works out its own row,
-// channel and column: 28 vector instructions more, as many as the quantization, and the loads behind conditions; the stem of 224x224 images on
-// one of them 6.6 us so, 5.6 now).
+// Input rows iy0 .. iy0 + RIN - 1 of an image, quantized, into the LDS lines of a strip, in one of three ways (stem_fill_rule). Those that load
+// units of four pixels take fp32 rows of four pixels and more (a 16-byte load at any pixel; the last unit of a row of no whole units is loaded
+// where it ends with the row and moved down) and int8 rows of whole, aligned units.
+
+// STEM_LINES: a wave takes lines, 64 units of one at a time. Row and channel of a line are scalar and go on by additions (worked out anew for each
+// they were 25 scalar instructions and a branch in front of every load), what is outside the image lies outside a descriptor and is zero, and a unit
+// costs its quantization and little else.
 template <bool IN_F32, int CT>
-__device__ __forceinline__ void stem_fill(unsigned* stem_lds, const void* __restrict__ x_, const ConvGeom& g, const StemPlan& p, size_t img_in, int iy0,
-                                          float qs, float half) {
+__device__ __forceinline__ void stem_fill_lines(unsigned* stem_lds, const void* __restrict__ x_, const ConvGeom& g, const StemPlan& p, size_t img_in, int iy0,
+                                                float qs, float half) {
     constexpr unsigned E = IN_F32 ? 4 : 1, OUT = 0x80000000u;
     const unsigned lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int C = CT ? CT : g.C, lines = p.RIN * C;
-    const unsigned plane = (unsigned)(g.H * g.W), bytes = (unsigned)C * plane * E;
+    const unsigned row = (unsigned)g.W * E, plane = (unsigned)g.H * row, bytes = (unsigned)C * plane;
     const char* const image = static_cast<const char*>(x_) + img_in * E;
+    // the wave's first line, and four lines further
+    const int r0 = C == 1 ? wave : C == 2 ? wave >> 1 : C == 3 && wave == 3 ? 1 : 0, c0 = wave - r0 * C;
+    const int dr = C == 1 ? 4 : C == 2 ? 2 : 1, dc = C == 3 ? 1 : 0;
     for (int d0 = 0; d0 < p.pitch_dw; d0 += 64) {
         const int d = d0 + (int)lane, ix = 4 * (d - 1);
         const int over = max(ix + 4 - g.W, 0);  // pixels of the unit past the row's end
         const unsigned v = ix >= 0 && ix < g.W ? (unsigned)(ix - over) * E : OUT, down = 8u * (unsigned)(over & 3);
-        for (int l0 = wave; l0 < lines; l0 += 4 * STEM_UN) {
+        int iy = iy0 + r0, c = c0;
+        unsigned at = (unsigned)iy * row + (unsigned)c * plane;
+        unsigned* to = stem_lds + wave * p.pitch_dw + d;
+        for (int left = lines - wave; left > 0; left -= 4 * STEM_UN) {
             v4i raw[STEM_UN];
 #pragma unroll
             for (int j = 0; j < STEM_UN; ++j) {
-                const int line = l0 + 4 * j, r = line / C, c = line - r * C, iy = iy0 + r;
-                const bool in = line < lines && iy >= 0 && iy < g.H;  // (uniform; a line that does not exist: a descriptor of no bytes)
+                const bool in = left > 4 * j && (unsigned)iy < (unsigned)g.H;  // (uniform; a line that does not exist: a descriptor of no bytes)
                 const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(image), 0, in ? (int)bytes : 0, 0x00020000);
-                const unsigned at = in ? ((unsigned)c * plane + (unsigned)iy * (unsigned)g.W) * E : 0u;
-                if constexpr (IN_F32) raw[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)v, (int)at, 0));
-                else raw[j][0] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)v, (int)at, 0);
+                if constexpr (IN_F32) raw[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)v, in ? (int)at : 0, 0));
+                else raw[j][0] = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)v, in ? (int)at : 0, 0);
+                iy += dr, c += dc, at += (unsigned)dr * row + (unsigned)dc * plane;
+                const bool next = dc != 0 && c >= C;
+                iy += next ? 1 : 0, c -= next ? C : 0, at += next ? row - bytes : 0u;
             }
 #pragma unroll
             for (int j = 0; j < STEM_UN; ++j) {
-                const int line = l0 + 4 * j;
-                if (line >= lines) break;  // (uniform)
+                if (left <= 4 * j) break;  // (uniform)
                 const unsigned pk = IN_F32 ? (unsigned)quantize4(raw[j], qs, half) >> down : (unsigned)raw[j][0];
-                if (d < p.pitch_dw) stem_lds[line * p.pitch_dw + d] = pk;
+                if (d < p.pitch_dw) to[4 * j * p.pitch_dw] = pk;
             }
+            to += 4 * STEM_UN * p.pitch_dw;
         }
     }
 }
 
-// the same for any rows, a value at a time
+// STEM_UNITS: the units of all lines dealt to the threads. Row, channel and column of a unit are worked out by each (28 vector instructions, as many
+// as its quantization), but nothing else stands in front of its load.
+typedef v4i v4i_any __attribute__((aligned(4)));  // (four floats of rows of any width)
+template <bool IN_F32, int CT>
+__device__ __forceinline__ void stem_fill_units(unsigned* stem_lds, const void* __restrict__ x_, const ConvGeom& g, const StemPlan& p, size_t img_in, int iy0,
+                                                float qs, float half) {
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int C = CT ? CT : g.C, total = p.RIN * C * p.pitch_dw;
+    const unsigned plane = (unsigned)(g.H * g.W);
+    for (int base = 0; base < total; base += 256 * STEM_UN) {
+        v4i raw[STEM_UN];
+        unsigned keep[STEM_UN], down[STEM_UN];
+#pragma unroll
+        for (int j = 0; j < STEM_UN; ++j) {
+            if (base + 256 * j + 64 * wave >= total) continue;  // (none of this wave's units exists)
+            // unit idx = dword idx of the LDS image: line = idx / pitch, row = line / C (exact: the quotients' fractional
+            // parts stay 0.5 / divisor away from an integer, far more than the rounding of these products)
+            const int idx = min(base + 256 * j + tid, total - 1);
+            const int line = (int)(((float)idx + 0.5f) * p.inv_pitch);
+            const int d = idx - line * p.pitch_dw;
+            const int r = (int)(((float)line + 0.5f) * p.inv_c);
+            const int c = line - r * C;
+            const int iy = iy0 + r, ix = 4 * (d - 1);
+            // every load from a clamped (always valid) address, so that all are in flight together; what lies outside
+            // the image is zeroed afterwards
+            const unsigned off = (unsigned)c * plane + (unsigned)min(max(iy, 0), g.H - 1) * (unsigned)g.W + (unsigned)min(max(ix, 0), g.W - 4);
+            if constexpr (IN_F32) raw[j] = *reinterpret_cast<const v4i_any*>(static_cast<const float*>(x_) + img_in + off);
+            else raw[j][0] = *reinterpret_cast<const int*>(static_cast<const int8_t*>(x_) + img_in + off);
+            keep[j] = iy >= 0 && iy < g.H && ix >= 0 && ix < g.W ? 0xffffffffu : 0u;
+            if constexpr (IN_F32) down[j] = 8u * (unsigned)(max(ix + 4 - g.W, 0) & 3);
+        }
+#pragma unroll
+        for (int j = 0; j < STEM_UN; ++j) {
+            if (base + 256 * j + 64 * wave >= total) continue;
+            const unsigned pk = IN_F32 ? (unsigned)quantize4(raw[j], qs, half) >> down[j] : (unsigned)raw[j][0];
+            const int idx = base + 256 * j + tid;
+            if (idx < total) stem_lds[idx] = pk & keep[j];
+        }
+    }
+}
+
+// STEM_VALUES: any rows, a value at a time
 template <bool IN_F32>
-__device__ __forceinline__ void stem_fill_any(unsigned* stem_lds, const void* __restrict__ x_, const ConvGeom& g, const StemPlan& p, int C, size_t img_in,
+__device__ __forceinline__ void stem_fill_values(unsigned* stem_lds, const void* __restrict__ x_, const ConvGeom& g, const StemPlan& p, int C, size_t img_in,
                                               int iy0, float qs, float half) {
     const int tid = threadIdx.x;
     const int total = p.RIN * C * p.pitch_dw;
@@ -282,8 +332,9 @@ __global__ void __launch_bounds__(256) conv_stem3x3_lds_kernel(const void* __res
     const size_t img_in = (size_t)img * g.C * (unsigned)(g.H * g.W);
     const float qs = IN_F32 ? in_scale[0] : 0.f;
     const float half = in_round == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
-    if (p.vec) stem_fill<IN_F32, CT>(stem_lds, x_, g, p, img_in, iy0, qs, half);
-    else stem_fill_any<IN_F32>(stem_lds, x_, g, p, C, img_in, iy0, qs, half);
+    if (p.fill == STEM_LINES) stem_fill_lines<IN_F32, CT>(stem_lds, x_, g, p, img_in, iy0, qs, half);
+    else if (p.fill == STEM_UNITS) stem_fill_units<IN_F32, CT>(stem_lds, x_, g, p, img_in, iy0, qs, half);
+    else stem_fill_values<IN_F32>(stem_lds, x_, g, p, C, img_in, iy0, qs, half);
 
     // ---- this lane's weights and the constants of its channels 16*m + 4*kg + i (requested once the strip's loads have
     // been consumed, so that their registers are not held across them; they arrive while the workgroup meets at the barrier)
@@ -404,8 +455,8 @@ __global__ void __launch_bounds__(256) conv_stem_pool_kernel(const void* __restr
         const size_t img_in = (size_t)img * g.C * (unsigned)(g.H * g.W);
         const float qs = IN_F32 ? in_scale[0] : 0.f;
         const float half = in_round == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
-        if (p.vec) stem_fill<IN_F32, CT>(stem_lds, x_, g, p, img_in, 2 * r0 - g.ph, qs, half);
-        else stem_fill_any<IN_F32>(stem_lds, x_, g, p, C, img_in, 2 * r0 - g.ph, qs, half);
+        if (p.fill == STEM_LINES) stem_fill_lines<IN_F32, CT>(stem_lds, x_, g, p, img_in, 2 * r0 - g.ph, qs, half);
+        else stem_fill_values<IN_F32>(stem_lds, x_, g, p, C, img_in, 2 * r0 - g.ph, qs, half);
     }
     v4i a[MT];
     float si[MT][4], bi[MT][4];
@@ -487,10 +538,20 @@ __global__ void __launch_bounds__(256) conv_stem_pool_kernel(const void* __restr
     }
 }
 
-// whether stem_fill takes the rows (its offsets inside an image are of 32 bits)
-static bool stem_vec(const void* x, bool in_f32, const ConvGeom& g) {
+// whether the rows can be loaded in units (offsets inside an image are of 32 bits)
+static bool stem_units(const void* x, bool in_f32, const ConvGeom& g) {
     if ((size_t)g.C * g.H * g.W * (in_f32 ? 4 : 1) >= ((size_t)1 << 31)) return false;
     return in_f32 ? g.W >= 4 && ((uintptr_t)x & 3) == 0 : g.W % 4 == 0 && ((uintptr_t)x & 3) == 0;
+}
+// How a strip of the layer alone is loaded. Lines where they keep three quarters of a wave's lanes busy and every wave has three of them: 3 -> 32
+// stride 2 @224x224 on one image 5.4 us (units 5.9), 64 images 16.6 (18.5), 3 -> 24 @416x416, 16 images, 19.7 (20.8); with lanes idle or fewer lines
+// they lose: 2 -> 48 @199x244, two images, 7.3 (6.5). Rows below 64 pixels value by value, the least code in front of the loads: 3 -> 16
+// stride 2 @32x32, 64 images, 3.3 (units 3.4, lines 3.9), 1 -> 8 @28x28, 64 images, 3.4 (3.6, 4.2). Between them units: 3 -> 32 @96x96, one image,
+// 4.1 (lines 4.4). Over 1067 drawn layers 0.976 of the time with units of whole rows and values for the others, with lines alone 1.08.
+static int stem_fill_rule(const void* x, bool in_f32, const ConvGeom& g, const StemPlan& p) {
+    if (!stem_units(x, in_f32, g)) return STEM_VALUES;
+    if (4 * p.pitch_dw >= 3 * 64 * ((p.pitch_dw + 63) / 64) && p.RIN * g.C >= 12) return STEM_LINES;
+    return g.W < 64 ? STEM_VALUES : STEM_UNITS;
 }
 // rows per workgroup and the LDS image of a strip; false where even one output row's input does not fit 64 KB
 static bool stem_lds_plan(const ConvGeom& g, StemPlan* p, size_t* lds_bytes) {
@@ -500,7 +561,7 @@ static bool stem_lds_plan(const ConvGeom& g, StemPlan* p, size_t* lds_bytes) {
         const int RIN = S * (R - 1) + 3;
         const size_t bytes = (size_t)RIN * g.C * pitch_dw * 4;
         if (bytes > 64 * 1024) continue;
-        p->R = R, p->strips = (g.OH + R - 1) / R, p->cgs = cgs, p->RIN = RIN, p->pitch_dw = pitch_dw, p->vec = 0;
+        p->R = R, p->strips = (g.OH + R - 1) / R, p->cgs = cgs, p->RIN = RIN, p->pitch_dw = pitch_dw, p->fill = STEM_VALUES;
         p->by_strips = fast_div((unsigned)p->strips), p->by_cgs = fast_div((unsigned)cgs);
         p->inv_pitch = 1.0f / (float)pitch_dw, p->inv_c = 1.0f / (float)g.C;
         *lds_bytes = bytes;
@@ -528,7 +589,7 @@ bool conv_stem_applicable(const ConvGeom& g, const Epilogue& ep, int in_layout) 
 
 // the strip of R pooled rows; false where it does not fit 64 KB
 static bool stem_pool_plan(const ConvGeom& g, int R, int POH, int POW, StemPlan* p, size_t* lds_bytes) {
-    p->R = R, p->strips = (POH + R - 1) / R, p->cgs = (POW + 15) / 16, p->RIN = 4 * R + 3, p->vec = 0;
+    p->R = R, p->strips = (POH + R - 1) / R, p->cgs = (POW + 15) / 16, p->RIN = 4 * R + 3, p->fill = STEM_VALUES;
     p->pitch_dw = std::max(16 * p->cgs + 2, (g.W + 3) / 4 + 1);
     p->by_strips = fast_div((unsigned)p->strips), p->by_cgs = fast_div((unsigned)p->cgs);
     p->inv_pitch = 1.0f / (float)p->pitch_dw, p->inv_c = 1.0f / (float)g.C;
@@ -573,7 +634,7 @@ hipError_t run_conv_stem_pool(const void* x, bool in_f32, const int8_t* wpk, flo
     while (!force && R > 1 && (long)g.N * ((POH + R - 1) / R) < 512) R /= 2;
     while (R > 1 && !stem_pool_plan(g, R, POH, POW, &p, &lds)) R /= 2;
     if (!stem_pool_plan(g, R, POH, POW, &p, &lds) || (long)g.N * p.strips >= (1l << 31)) return hipErrorInvalidValue;
-    p.vec = stem_vec(x, in_f32, g);
+    p.fill = stem_units(x, in_f32, g) ? STEM_LINES : STEM_VALUES;
     switch ((g.K + 15) / 16) {
     case 1: return launch_stem_pool<1>(x, in_f32, wpk, out, out_q, g, ep, in_scale, in_round, pad_value, p, lds, stream);
     case 2: return launch_stem_pool<2>(x, in_f32, wpk, out, out_q, g, ep, in_scale, in_round, pad_value, p, lds, stream);
@@ -591,7 +652,7 @@ static hipError_t launch_stem_lds(const void* x, bool in_f32, const int8_t* wpk,
     if (!stem_lds_plan(g, &p, &lds)) return hipErrorInvalidValue;
     const long wgs = (long)g.N * p.strips;
     if (wgs >= (1l << 31)) return hipErrorInvalidValue;
-    p.vec = stem_vec(x, in_f32, g);
+    p.fill = stem_fill_rule(x, in_f32, g, p);
     const int epi = ep.out_kind == OTTER_HIP_OUT_F32 ? 0 : pick_epilogue(ep, g.K) == EPI_I8_P8_NONNEG ? 2 : 1;
     const dim3 grid((unsigned)wgs), block(256);
 #define OHIP_STEM_L(EPI_, FI_)                                                                                          \

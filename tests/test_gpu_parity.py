@@ -551,6 +551,20 @@ def test_grouped_and_odd_depthwise_routes(hip, oracle, C, K, k, s, p, g, N, H, W
     (3, 16, 1, 1, 2, 9, 16, True, 0, True),      # int8 planar rows of whole 4-byte units, signed result
     (2, 8, 2, 0, 1, 11, 23, False, 3, True),     # two channels, no padding, odd width: scalar loads, clip at six
     (4, 32, 2, 1, 2, 3, 4, True, 2, True),       # fewer output rows than a strip, one 4-pixel unit per row
+    # the three ways in which a strip is loaded: value by value below 64 pixels, units of four dealt to the threads, a wave per line
+    (3, 16, 1, 1, 2, 7, 63, False, 1, True),
+    (3, 16, 1, 1, 2, 7, 64, False, 1, True),     # units, whole ones
+    (3, 16, 2, 0, 1, 9, 65, False, 0, False),    # the last unit holds one pixel
+    (2, 24, 2, 1, 1, 12, 131, False, 2, True),
+    (2, 8, 1, 0, 3, 8, 66, False, 3, True),
+    (4, 16, 1, 1, 2, 6, 72, True, 0, True),
+    (3, 32, 2, 1, 1, 13, 183, False, 3, True),   # 50 of 64 lanes hold a unit: lines
+    (3, 32, 2, 1, 1, 13, 159, False, 3, True),   # 42: units
+    (3, 16, 1, 1, 1, 5, 254, False, 1, True),    # 66 in two rounds: units
+    (3, 16, 1, 1, 1, 5, 382, False, 1, True),    # 98: lines, the last unit of two pixels
+    (1, 8, 2, 1, 2, 21, 389, False, 2, True),    # nine lines of one channel are units, twelve of two are lines
+    (2, 8, 1, 0, 1, 21, 389, False, 2, False),
+    (2, 8, 2, 1, 1, 6, 384, True, 0, True),
 ])
 def test_few_channel_3x3_stem_kernel(hip, oracle, C, K, s, p, N, H, W, in_i8, act, int8_out):
     """3x3 on a blob with at most 5 channels goes straight from the unpacked blob (quantized on the way) to the
