@@ -194,7 +194,7 @@ enum {
     EPI_F32_P4_FUSED = 5,  // implicit GEMM only: EPI_F32_P4 plus the residual addend and / or the int8 twin
     EPI_F32_SHUFFLE = 6,   // the same kernels: the channels interleaved with another blob's (JoinArgs::other)
     EPI_F32_P4_PARTS = 7,  // EPI_F32_P4_FUSED with the addend in two parts (JoinArgs::residual1)
-    EPI_F32_SLICE = 8      // the pointwise register kernels: the quantized result in a slice of a blob (JoinArgs::slice)
+    EPI_F32_SLICE = 8      // the pointwise register kernels and the depthwise matrix-core kernel: the quantized result in a slice of a blob (JoinArgs::slice)
 };
 
 // the argument that an instance takes for them

@@ -432,9 +432,11 @@ __global__ void __launch_bounds__(256) conv_stem3x3_lds_kernel(const void* __res
 // ---------------------------------------------------------------------------------------------------------------------
 
 // What the two cost as launches is the blob between them: the layer's result is four times the pooled one and fp32 (24 channels, 416x416
-// -> 208x208 -> 104x104, 16 images: 66 MB written and read, 24.4 + 19.4 us; its quantization for the layers behind 5.4 us more). As one launch
-// 17.0 us, for one image 5.9 (14.7 as three); the bytes it cannot do without take 8, the rest is the chain of a strip: rows in, barrier, windows. Dequantization, clamp and LeakyReLU are monotone where scale_in >= 0, rounding included: the largest of nine
-// results is the result of the largest sum, and a pooled value costs nine integer comparisons and one epilogue.
+// -> 208x208 -> 104x104, 16 images: 66 MB written and read, 19.8 + 20.0 us, 25 + 19.5 in the detection model; its quantization for the layers behind
+// 4.2 us more). As one launch 19.4 us with both results, 17.1 with the int8 one alone, 18.0 in the model; for one image 6.0 (14.5 as three). The bytes it
+// cannot do without take 8, the rest is the chain of a strip: rows in, barrier, windows. Dequantization, clamp and LeakyReLU are monotone where
+// scale_in >= 0, rounding included: the largest of nine results is the result of the largest sum, and a pooled value costs nine integer comparisons
+// and one epilogue.
 //
 // A workgroup owns R pooled rows. A lane's pixel is a pooled one, and its three columns of the layer come from the same three LDS dwords
 // of a line (windows 2 pixels apart); a column or row outside the layer's result repeats the one beside it, and the window then also

@@ -3142,14 +3142,17 @@ RecordedPasses::Lease::~Lease() {
 //   7 calls   3x3 48 <-> 72              5 1.13, 83 1.17, 333 1.20
 //   13        5x5 depthwise, 1x1, sum    61 0.86, 486 0.93, 973 1.03
 //   21        3x3                        59 0.89, 237 0.99, 473 1.03
-//   27        classifier                 62 0.79, 171 0.93, 334 0.95, 668 1.00, 1000 1.02
+//   26-35     classifier                 301 0.85, 2102 0.95, 6944 1.01, 15182 0.99, 27158 1.01 (1, 8, 32, 64, 128 images)
 //   41        3x3                        53 0.89, 213 0.95, 426 0.99, 852 1.00
 //   63        5x5 depthwise, 1x1, sum    57 0.65, 459 0.68, 918 0.72, 1835 0.91
-//   103       detection model            368 1.02, 737 1.02, 1546 1.00
+//   76-83     detection model            271 0.83, 1103 0.99, 4744 0.97 (1, 4, 16 images)
+//   12        5x5 depthwise, 1x1, sum    128 0.65, 1029 0.71, 4116 1.06, 8232 1.05, 32928 1.00
+//   40        the same                   128 0.62, 1029 0.66, 4116 1.10, 8232 1.14, 32928 0.97
+//   80        the same                   128 0.60, 1029 0.66, 4116 1.06, 8232 1.14, 32928 0.95
 //   123       5x5 depthwise, 1x1, sum    57 0.80, 455 0.83, 911 0.91, 1821 0.99
 //   141       3x3                        3 0.96, 49 1.02, 195 1.03, 391 1.06
 // A host that waits for every pass also waits for its first launches: 7 calls 5 0.71, 333 0.93, 667 1.03; 9 502 1.06; 13 486 0.80, 973 0.91;
-// 27 334 0.79, 668 0.93, 1336 0.97, 2308 0.99; 43 1848 0.97; 103 368 1.01, 737 0.99, 1546 1.00.
+// 43 1848 0.97; the classifier with its image from the host 323 0.81, 2254 1.04, 7514 0.94, 16526 0.95; the detection model 295 0.89, 1202 1.03, 5208 0.94.
 // On a slower host (4.6 us a launch) 96 calls of 1546 KB 0.92 to 0.93: long passes, which lose least, are given the benefit.
 static bool worth_recording(long launches, size_t bytes, bool waited_for) {
     if (waited_for) return bytes <= (size_t)launches * std::min<size_t>((size_t)launches * 50 << 10, 1536 << 10);
