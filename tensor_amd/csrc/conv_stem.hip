@@ -545,14 +545,16 @@ static bool stem_units(const void* x, bool in_f32, const ConvGeom& g) {
     if ((size_t)g.C * g.H * g.W * (in_f32 ? 4 : 1) >= ((size_t)1 << 31)) return false;
     return in_f32 ? g.W >= 4 && ((uintptr_t)x & 3) == 0 : g.W % 4 == 0 && ((uintptr_t)x & 3) == 0;
 }
-// How a strip of the layer alone is loaded. Lines where they keep three quarters of a wave's lanes busy and every wave has three of them: 3 -> 32
-// stride 2 @224x224 on one image 5.4 us (units 5.9), 64 images 16.6 (18.5), 3 -> 24 @416x416, 16 images, 19.7 (20.8); with lanes idle or fewer lines
-// they lose: 2 -> 48 @199x244, two images, 7.3 (6.5). Rows below 64 pixels value by value, the least code in front of the loads: 3 -> 16
-// stride 2 @32x32, 64 images, 3.3 (units 3.4, lines 3.9), 1 -> 8 @28x28, 64 images, 3.4 (3.6, 4.2). Between them units: 3 -> 32 @96x96, one image,
-// 4.1 (lines 4.4). Over 1067 drawn layers 0.976 of the time with units of whole rows and values for the others, with lines alone 1.08.
+// How a strip of the layer alone is loaded. Lines where they keep five lanes of eight busy (six where the channels are not the three that the line's
+// figures are compiled for) and every wave has three of them: 3 -> 32 stride 2 @224x224 on one image 5.4 us (units 5.9), 64 images 16.6 (18.5),
+// 3 -> 24 @416x416, 16 images, 19.7 (20.8), 3 -> 40 @334x334, 14 images, 14.8 (16.0); with more lanes idle or fewer lines they lose: 2 -> 48
+// @199x244, two images, 7.3 (6.5). Rows below 64 pixels value by value, the least code in front of the loads: 3 -> 16 stride 2 @32x32, 64 images, 3.3
+// (units 3.4, lines 3.9), 1 -> 8 @28x28, 64 images, 3.4 (3.6, 4.2). Between them units: 3 -> 32 @96x96, one image, 4.1 (lines 4.4). Over drawn
+// layers 0.97 of the time with units of whole rows and values for the others, with lines alone 1.08.
 static int stem_fill_rule(const void* x, bool in_f32, const ConvGeom& g, const StemPlan& p) {
     if (!stem_units(x, in_f32, g)) return STEM_VALUES;
-    if (4 * p.pitch_dw >= 3 * 64 * ((p.pitch_dw + 63) / 64) && p.RIN * g.C >= 12) return STEM_LINES;
+    const int busy = g.C == 3 ? 5 : 6;  // lanes of eight
+    if (8 * p.pitch_dw >= busy * 64 * ((p.pitch_dw + 63) / 64) && p.RIN * g.C >= 12) return STEM_LINES;
     return g.W < 64 ? STEM_VALUES : STEM_UNITS;
 }
 // rows per workgroup and the LDS image of a strip; false where even one output row's input does not fit 64 KB

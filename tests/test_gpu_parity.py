@@ -558,8 +558,8 @@ def test_grouped_and_odd_depthwise_routes(hip, oracle, C, K, k, s, p, g, N, H, W
     (2, 24, 2, 1, 1, 12, 131, False, 2, True),
     (2, 8, 1, 0, 3, 8, 66, False, 3, True),
     (4, 16, 1, 1, 2, 6, 72, True, 0, True),
-    (3, 32, 2, 1, 1, 13, 183, False, 3, True),   # 50 of 64 lanes hold a unit: lines
-    (3, 32, 2, 1, 1, 13, 159, False, 3, True),   # 42: units
+    (3, 32, 2, 1, 1, 13, 159, False, 3, True),   # 42 of 64 lanes hold a unit: lines
+    (3, 32, 2, 1, 1, 13, 127, False, 3, True),   # 34: units
     (3, 16, 1, 1, 1, 5, 254, False, 1, True),    # 66 in two rounds: units
     (3, 16, 1, 1, 1, 5, 382, False, 1, True),    # 98: lines, the last unit of two pixels
     (1, 8, 2, 1, 2, 21, 389, False, 2, True),    # nine lines of one channel are units, twelve of two are lines
