@@ -105,6 +105,7 @@ struct otter_hip_conv {
     int32_t* blk_consts = nullptr; // the layer's constants (and depthwise 3x3 weights) as the fused block launch keeps them in LDS
     bool monotone = true;        // scale_in >= 0, and scale_in and bias are finite: larger sums give no smaller results
     bool so_positive = true;     // every output scale is finite and > 0
+    bool so_full = true;         // and every upper clamp of a rounded result is int8's own (Epilogue::so_full)
     bool so_same = true;         // the output scales are all so_one
     float so_one = 1.f;
     float* scale_in = nullptr;   // [Kpad]
@@ -546,6 +547,9 @@ int otter_hip_conv_create(const otter_hip_conv_desc* desc, const int8_t* weight,
                 so[i] = n_out_scale == 1 ? out_scale[0] : out_scale[i];
                 if (!(so[i] > 0.f) || std::isinf(so[i])) h->so_positive = false;
                 if (so[i] != so[0]) h->so_same = false;
+                // (the doubled scale is finite as well)
+                const float top = d.activation_type == 3 ? 6.f * so[i] : 127.f;
+                if (!(so[i] > 0.f) || !std::isfinite(2.f * so[i]) || !(top + (d.out_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f) >= 127.f)) h->so_full = false;
             }
             h->so_one = so[0];
             if ((rc = upload<float>(&h->scale_out, so.data(), K, kpad, 1.f))) break;
@@ -715,6 +719,8 @@ static Epilogue make_epilogue(const otter_hip_conv* h, int out_layout) {
     ep.act_hi = d.activation_type == 3 ? 6.f : __builtin_inff();
     ep.round_half = d.out_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     ep.so_positive = h->so_positive;
+    ep.so_full = h->so_full;
+    ep.so_one = h->so_same ? h->so_one : 0.f;
     ep.lrelu = d.activation_type == 2 && d.activation_param0 >= 0.f && d.activation_param0 <= 1.f;
     return ep;
 }

@@ -147,6 +147,8 @@ struct Epilogue {
     float round_half;      // 0.5f (ROUND_SSE) or 0.49999997f (ROUND_EXACT)
     bool so_positive;      // every output scale is finite and > 0 (lets the int8 epilogue clamp after rounding)
     bool lrelu;            // LeakyReLU with a slope in [0, 1]: v = max(v, v * act_p0), applied by the fast epilogues
+    bool so_full = false;  // so_positive, and the activation's upper end is no tighter than int8's: every upper clamp is 127
+    float so_one = 0.f;    // the output scale of every channel, 0 where they differ (host side; with so_full in what was padding)
     // fp32 output only: also write the Byte8 quantization of the result, q = float2int8(v * twin_scale), for an int8
     // convolution that reads this blob next (null: no twin). Honoured by the implicit-GEMM Float4 epilogue.
     int8_t* twin = nullptr;
@@ -194,8 +196,12 @@ enum {
     EPI_F32_P4_FUSED = 5,  // implicit GEMM only: EPI_F32_P4 plus the residual addend and / or the int8 twin
     EPI_F32_SHUFFLE = 6,   // the same kernels: the channels interleaved with another blob's (JoinArgs::other)
     EPI_F32_P4_PARTS = 7,  // EPI_F32_P4_FUSED with the addend in two parts (JoinArgs::residual1)
-    EPI_F32_SLICE = 8      // the pointwise register kernels and the depthwise matrix-core kernel: the quantized result in a slice of a blob (JoinArgs::slice)
+    EPI_F32_SLICE = 8,     // the pointwise register kernels and the depthwise matrix-core kernel: the quantized result in a slice of a blob (JoinArgs::slice)
+    EPI_I8_P8_FULL = 9     // EPI_I8_P8_NONNEG with every upper clamp at 127 (Epilogue::so_full), see quant4_full; its instances take doubled output scales
 };
+constexpr bool epi_is_i8(int epi) { return epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG || epi == EPI_I8_P8_FULL; }
+// how an int8 epilogue ends: 0 = the int8 range alone, 1 = clamped to [0, its channel's upper clamp], 2 = to [0, 127]
+constexpr int epi_clamp(int epi) { return epi == EPI_I8_P8_FULL ? 2 : epi == EPI_I8_P8_NONNEG ? 1 : 0; }
 
 // the argument that an instance takes for them
 struct NoJoin {
@@ -241,7 +247,7 @@ struct EpiFused : EpiTwin {
 };
 template <int EPI>
 struct EpiArgs {
-    static constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, FUSED = EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_P4_PARTS;
+    static constexpr bool I8 = epi_is_i8(EPI), FUSED = EPI == EPI_F32_P4_FUSED || EPI == EPI_F32_P4_PARTS;
     std::conditional_t<I8, EpiI8, std::conditional_t<FUSED, EpiFused, std::conditional_t<EPI == EPI_F32_SHUFFLE, EpiTwin, EpiBase>>> a;
     static EpiArgs of(const Epilogue& ep) {
         EpiArgs r{};
@@ -282,6 +288,9 @@ __host__ inline int pick_epilogue(const Epilogue& ep, int K) {
     if (clamp_act && ep.out_kind == OTTER_HIP_OUT_F32 && ep.out_layout == OTTER_HIP_F32_P4 && K % 4 == 0) return EPI_F32_P4;
     return EPI_GENERIC;
 }
+
+// the instance to launch for an epilogue code of pick_epilogue, in kernels that have one for EPI_I8_P8_FULL
+__host__ inline int full_epilogue(int epi, const Epilogue& ep) { return epi == EPI_I8_P8_NONNEG && ep.so_full ? (int)EPI_I8_P8_FULL : epi; }
 
 struct ConvGeom {
     int N, C, H, W;        // input
@@ -395,7 +404,7 @@ __device__ __forceinline__ void epi8_load(Epi8& p, const Epilogue& ep, int ch0) 
         p.bi[e] = __int_as_float(b0[e]);
         p.bi[4 + e] = __int_as_float(b1[e]);
     }
-    if constexpr (EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
+    if constexpr (epi_is_i8(EPI)) {
         const ohip_v4i* o = reinterpret_cast<const ohip_v4i*>(ep.scale_out + ch0);
         ohip_v4i o0 = o[0], o1 = o[1];
 #pragma unroll
@@ -404,6 +413,9 @@ __device__ __forceinline__ void epi8_load(Epi8& p, const Epilogue& ep, int ch0) 
             p.so[4 + e] = __int_as_float(o1[e]);
         }
         if constexpr (EPI == EPI_I8_P8_NONNEG) epi8_clamp_init(ep, p);
+        if constexpr (EPI == EPI_I8_P8_FULL)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) p.so[e] += p.so[e];
     }
 }
 
@@ -443,12 +455,33 @@ __device__ __forceinline__ unsigned cvt_u32_floor0(float v) {
 // instructions more, and it is made per value: the compiler turns a uniform branch around three instructions into a select.)
 __device__ __forceinline__ float lrelu_or_not(const Epilogue& ep, float v) { return fmaxf(v, __fmul_rn(v, ep.lrelu ? ep.act_p0 : 1.f)); }
 
+// Four values behind ReLU / clip as the bytes min(max((int)fl(t + half), 0), 127), from t2 = 2 t (exact). v_cvt_pk_u8_f32 converts, saturates to
+// [0, 255] and packs in one instruction, but rounds to nearest even; with t doubled that is no matter: fl(2 t + half) rounds to 2 q or 2 q + 1
+// wherever fl(t + half) truncates to q (a value that lies between two of them is even below, and there the tie goes), and 255 is 127 with a
+// bit behind it. For every float t and both rounding constants: tests/test_requant_full.py goes over them. It takes the place of the
+// conversion, two packings with saturation, two minima and a permutation: of four requantized values' 96 cycles of vector issue 17.
+// Launches that this bounds take 0.92 of the time (16 -> 96 pointwise + depthwise stride 2 @112x112 b64 26.5 -> 24.5 us).
+__device__ __forceinline__ unsigned quant4_full(const float (&t2)[4], float half) {
+    unsigned w = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w = __builtin_amdgcn_cvt_pk_u8_f32(__fadd_rn(t2[e], half), e, w);
+    return w >> 1 & 0x7f7f7f7fu;
+}
+
 // requantize 4 channels: their bytes
+// CLAMP: as epi_clamp says (2: `so` are the doubled output scales)
 // LRELU: 0 = no LeakyReLU, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time
-template <bool NONNEG, int LRELU = -1>
+template <int CLAMP, int LRELU = -1>
 __device__ __forceinline__ int epi4_quant_i8(const Epilogue& ep, const float* si, const float* bi, const float* so, const unsigned* qh,
                                              int a0, int a1, int a2, int a3) {
+    constexpr bool NONNEG = CLAMP != 0;
     const int a[4] = {a0, a1, a2, a3};
+    if constexpr (CLAMP == 2) {
+        float t2[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t2[e] = __fmul_rn(__fmaf_rn((float)a[e], si[e], bi[e]), so[e]);
+        return (int)quant4_full(t2, ep.round_half);
+    }
     int q[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -480,16 +513,16 @@ __device__ __forceinline__ int epi4_quant_i8(const Epilogue& ep, const float* si
     }
 }
 
-template <bool NONNEG, int LRELU = -1>
+template <int CLAMP, int LRELU = -1>
 __device__ __forceinline__ ohip_v2i epi8_quant_i8p8(const Epilogue& ep, const Epi8& p, const int (&a8)[8]) {
-    return ohip_v2i{epi4_quant_i8<NONNEG, LRELU>(ep, p.si, p.bi, p.so, p.qh, a8[0], a8[1], a8[2], a8[3]),
-                    epi4_quant_i8<NONNEG, LRELU>(ep, p.si + 4, p.bi + 4, p.so + 4, p.qh + 2, a8[4], a8[5], a8[6], a8[7])};
+    return ohip_v2i{epi4_quant_i8<CLAMP, LRELU>(ep, p.si, p.bi, p.so, p.qh, a8[0], a8[1], a8[2], a8[3]),
+                    epi4_quant_i8<CLAMP, LRELU>(ep, p.si + 4, p.bi + 4, p.so + 4, p.qh + 2, a8[4], a8[5], a8[6], a8[7])};
 }
 
-template <bool NONNEG>
+template <int CLAMP>
 __device__ __forceinline__ void epi8_store_i8p8(int8_t* __restrict__ out, const Epilogue& ep, const Epi8& p, size_t elem,
                                                 const int (&a8)[8]) {
-    *reinterpret_cast<ohip_v2i*>(out + elem) = epi8_quant_i8p8<NONNEG>(ep, p, a8);
+    *reinterpret_cast<ohip_v2i*>(out + elem) = epi8_quant_i8p8<CLAMP>(ep, p, a8);
 }
 
 // dequantize 4 channels with the clamp activation (LRELU false) or LeakyReLU (true): the bits of one Float4 element

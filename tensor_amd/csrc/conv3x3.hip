@@ -68,7 +68,8 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
     for (int i = tid; i < 3 * ROWS; i += 256) {
         const int which = i / ROWS, c = blockIdx.y * ROWS + (i - which * ROWS);
         const float* src = which == 0 ? ep.scale_in : (which == 1 ? ep.bias : ep.scale_out);
-        lds_prm[i] = src ? src[c] : 1.f;
+        const float v = src ? src[c] : 1.f;
+        lds_prm[i] = EPI == EPI_I8_P8_FULL && which == 2 ? v + v : v;
     }
     // (int8 result behind ReLU / clip: the upper clamp of the rounded value per channel, once per workgroup instead of
     // once per tile and wave)
@@ -345,9 +346,9 @@ __global__ void __launch_bounds__(256, 2) conv3x3_halo_kernel(const int8_t* __re
                     a8[4 + e] = acc[2 * ip + 1][f][e];
                 }
                 if (ch_ok && pix < OHW) {
-                    if constexpr (EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
-                        epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm,
-                                                                 elem_offset(8, n, ch0, pix, g.K, OHW), a8);
+                    if constexpr (epi_is_i8(EPI)) {
+                        epi8_store_i8p8<epi_clamp(EPI)>((int8_t*)out, ep, prm,
+                                                        elem_offset(8, n, ch0, pix, g.K, OHW), a8);
                     } else if constexpr (EPI == EPI_F32_P4) {
                         epi4_store_f32p4((float*)out, ep, prm.si, prm.bi, elem_offset(4, n, ch0, pix, g.K, OHW), a8[0],
                                          a8[1], a8[2], a8[3]);
@@ -465,11 +466,13 @@ hipError_t launch_halo_e(const int8_t* x, const int8_t* wpk, void* out, const Co
 template <int FM, int FN, int WM, int WN>
 hipError_t launch_halo(const int8_t* x, const int8_t* wpk, void* out, const ConvGeom& g, const Epilogue& ep,
                        const HaloPlan& pl, hipStream_t stream) {
-    switch (pick_epilogue(ep, g.K)) {
+    switch (full_epilogue(pick_epilogue(ep, g.K), ep)) {
     case EPI_I8_P8:
         return launch_halo_e<FM, FN, WM, WN, EPI_I8_P8>(x, wpk, out, g, ep, pl, stream);
     case EPI_I8_P8_NONNEG:
         return launch_halo_e<FM, FN, WM, WN, EPI_I8_P8_NONNEG>(x, wpk, out, g, ep, pl, stream);
+    case EPI_I8_P8_FULL:
+        return launch_halo_e<FM, FN, WM, WN, EPI_I8_P8_FULL>(x, wpk, out, g, ep, pl, stream);
     case EPI_F32_P4:
         return launch_halo_e<FM, FN, WM, WN, EPI_F32_P4>(x, wpk, out, g, ep, pl, stream);
     default:

@@ -86,7 +86,6 @@ __global__ void __launch_bounds__(256, 2) conv3x3_chain_kernel(ConvGeom g, Epilo
                                                             int c_groups, int r_max, int tiles_per_img,
                                                             unsigned act_bytes) {
     constexpr int FM = 4, WN = 4 / WM;
-    constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     constexpr int PT = WN * FN * 16;
     constexpr int PITCH = 1 << LOGP;
@@ -376,7 +375,10 @@ __global__ void __launch_bounds__(256, 2) conv3x3_chain_kernel(ConvGeom g, Epilo
                 prm.so[e] = __int_as_float(r4[e]);
                 prm.so[4 + e] = __int_as_float(r5[e]);
             }
-            if constexpr (NONNEG) epi8_clamp_init(ep, prm);
+            if constexpr (EPI == EPI_I8_P8_NONNEG) epi8_clamp_init(ep, prm);
+            if constexpr (EPI == EPI_I8_P8_FULL)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) prm.so[e] += prm.so[e];
 #pragma unroll
             for (int f = 0; f < FN; ++f) {
                 const int pix = p0 + (wn * FN + f) * 16 + (lane & 15);
@@ -386,7 +388,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_chain_kernel(ConvGeom g, Epilo
                     a8[e] = acc[2 * ip][f][e];
                     a8[4 + e] = acc[2 * ip + 1][f][e];
                 }
-                if (ch_ok && pix < OHW) epi8_store_i8p8<NONNEG>(out, ep, prm, elem_offset(8, n, ch0, pix, g.K, OHW), a8);
+                if (ch_ok && pix < OHW) epi8_store_i8p8<epi_clamp(EPI)>(out, ep, prm, elem_offset(8, n, ch0, pix, g.K, OHW), a8);
             }
         }
         done_i = cur_i;
@@ -542,7 +544,9 @@ hipError_t run_conv3x3_chain(const ConvGeom& g, const Epilogue* eps, const int8_
     ca.inv_ow20 = ((1u << 20) + (unsigned)g.OW - 1u) / (unsigned)g.OW;
     ca.flags = cd.flags + (size_t)slot * CHAIN_MAX_FLAGS, ca.ctl = cd.ctl + slot * 16;
     const int fn = plan[0], r_max = plan[1], tpi = plan[2], logp = plan[3];
-    const int epi = pick_epilogue(eps[0], g.K);
+    bool full = true;  // (of every layer)
+    for (int l = 0; l < layers; ++l) full = full && eps[l].so_full;
+    const int epi = full ? full_epilogue(pick_epilogue(eps[0], g.K), eps[0]) : pick_epilogue(eps[0], g.K);
     const unsigned act_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W);
     const size_t lds_bytes = (size_t)(igemm_channel_groups(g.C) * 8) * r_max << logp;
     const long total = (long)layers * g.N * tpi;
@@ -572,7 +576,8 @@ hipError_t run_conv3x3_chain(const ConvGeom& g, const Epilogue* eps, const int8_
     } while (0)
 #define OHIP_CHAIN_E(FN_)                                                 \
     do {                                                                  \
-        if (epi == EPI_I8_P8_NONNEG) OHIP_CHAIN_P(FN_, EPI_I8_P8_NONNEG); \
+        if (epi == EPI_I8_P8_FULL) OHIP_CHAIN_P(FN_, EPI_I8_P8_FULL);     \
+        else if (epi == EPI_I8_P8_NONNEG) OHIP_CHAIN_P(FN_, EPI_I8_P8_NONNEG); \
         else OHIP_CHAIN_P(FN_, EPI_I8_P8);                                \
     } while (0)
     switch (fn) {

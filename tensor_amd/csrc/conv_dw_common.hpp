@@ -44,11 +44,26 @@ __device__ __forceinline__ unsigned dw_clamp_pair(const Epilogue& ep, int so0, i
     const int q1 = min((int)__fadd_rn(__fmul_rn(ep.act_hi, __int_as_float(so1)), ep.round_half), 127);
     return (unsigned)(q0 & 0xffff) | ((unsigned)q1 << 16);
 }
+// the output scales as quant4_full takes them
+__device__ __forceinline__ v4i dw_doubled(const v4i& so) {
+    v4i r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = __float_as_int(__int_as_float(so[e]) + __int_as_float(so[e]));
+    return r;
+}
 
-// LRELU: 0 = no LeakyReLU, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time
-template <bool NONNEG, int LRELU = -1>
+// CLAMP: as epi_clamp says (2: `so` are the doubled output scales). LRELU: 0 = no LeakyReLU, 1 = LeakyReLU, -1 = decided by ep.lrelu at run time
+template <int CLAMP, int LRELU = -1>
 __device__ __forceinline__ unsigned dw_requant4(const Epilogue& ep, const v4i& acc, const v4i& si, const v4i& bi,
                                                 const v4i& so, unsigned qh01, unsigned qh23) {
+    constexpr bool NONNEG = CLAMP != 0;
+    if constexpr (CLAMP == 2) {
+        float t2[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            t2[e] = __fmul_rn(__fmaf_rn((float)acc[e], __int_as_float(si[e]), __int_as_float(bi[e])), __int_as_float(so[e]));
+        return quant4_full(t2, ep.round_half);
+    }
     int qv[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -71,15 +86,9 @@ __device__ __forceinline__ unsigned dw_requant4(const Epilogue& ep, const v4i& a
     }
     ohip_v2s lo = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(qv[0], qv[1]));
     ohip_v2s hi = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(qv[2], qv[3]));
-    if (NONNEG) {
-        const ohip_v2s zero = {0, 0};
-        lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, __builtin_bit_cast(ohip_v2s, qh01)), zero);
-        hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, __builtin_bit_cast(ohip_v2s, qh23)), zero);
-    } else {
-        const ohip_v2s top = {127, 127}, bot = {-127, -127};
-        lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bot);
-        hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bot);
-    }
+    const ohip_v2s top = {127, 127}, bot = {-127, -127};
+    lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bot);
+    hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bot);
     return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
 }
 

@@ -185,6 +185,9 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
 #pragma unroll
         for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(bi[t][e]));
     }
+    if constexpr (EPI == EPI_I8_P8_FULL)
+#pragma unroll
+        for (int t = 0; t < T; ++t) so[t] = dw_doubled(so[t]);
     unsigned qh[T][2] = {};
     if constexpr (EPI == EPI_I8_P8_NONNEG) {
 #pragma unroll
@@ -248,14 +251,14 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
             for (int t = 0; t < 2; ++t) w2[t] = quantize4(dw_dequant4<LR ? 1 : 0>(ep, cur[t % T], si[t % T], bi[t % T]), g.q_scale<LR>(), g.half);
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, w2), rout, (int)v_o, (int)s_row, 0);
         } else {
-            constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
+            constexpr int CLAMP = epi_clamp(EPI);
             if constexpr (S == 1) {
                 v2i w2;
-                w2[0] = (int)dw_requant4<NONNEG, LR ? 1 : 0>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
-                w2[1] = (int)dw_requant4<NONNEG, LR ? 1 : 0>(ep, cur[T - 1], si[T - 1], bi[T - 1], so[T - 1], qh[T - 1][0], qh[T - 1][1]);
+                w2[0] = (int)dw_requant4<CLAMP, LR ? 1 : 0>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
+                w2[1] = (int)dw_requant4<CLAMP, LR ? 1 : 0>(ep, cur[T - 1], si[T - 1], bi[T - 1], so[T - 1], qh[T - 1][0], qh[T - 1][1]);
                 __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, w2), rout, (int)v_o, (int)s_row, 0);
             } else {
-                const unsigned w1 = dw_requant4<NONNEG, LR ? 1 : 0>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
+                const unsigned w1 = dw_requant4<CLAMP, LR ? 1 : 0>(ep, cur[0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
                 __builtin_amdgcn_raw_buffer_store_b32(w1, rout, (int)v_o, (int)s_row, 0);
             }
         }
@@ -455,6 +458,9 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
         so[t] = v4i{0, 0, 0, 0};
         if constexpr (EPI != EPI_F32_P4 && EPI != EPI_F32_P8) so[t] = *reinterpret_cast<const v4i*>(ep.scale_out + ch + 4 * t);
     }
+    if constexpr (EPI == EPI_I8_P8_FULL)
+#pragma unroll
+        for (int t = 0; t < T; ++t) so[t] = dw_doubled(so[t]);
     unsigned qh[T][2] = {};
     if constexpr (EPI == EPI_I8_P8_NONNEG) {
 #pragma unroll
@@ -496,14 +502,14 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
                     store_b128_row(res, rout, vo_t, s_row);
                 }
             } else {
-                constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
+                constexpr int CLAMP = epi_clamp(EPI);
                 if constexpr (S == 1) {
                     v2i w2;
-                    w2[0] = (int)dw_requant4<NONNEG>(ep, cur[c][0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
-                    w2[1] = (int)dw_requant4<NONNEG>(ep, cur[c][T - 1], si[T - 1], bi[T - 1], so[T - 1], qh[T - 1][0], qh[T - 1][1]);
+                    w2[0] = (int)dw_requant4<CLAMP>(ep, cur[c][0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
+                    w2[1] = (int)dw_requant4<CLAMP>(ep, cur[c][T - 1], si[T - 1], bi[T - 1], so[T - 1], qh[T - 1][0], qh[T - 1][1]);
                     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, w2), rout, (int)v_out[c], (int)s_row, 0);
                 } else {
-                    const unsigned w1 = dw_requant4<NONNEG>(ep, cur[c][0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
+                    const unsigned w1 = dw_requant4<CLAMP>(ep, cur[c][0], si[0], bi[0], so[0], qh[0][0], qh[0][1]);
                     __builtin_amdgcn_raw_buffer_store_b32(w1, rout, (int)v_out[c], (int)s_row, 0);
                 }
             }
@@ -626,7 +632,9 @@ hipError_t run_conv_dw_f32in(const float* x, const int8_t* wa, void* out, const 
     } while (0)
 #define OHIP_DWF_E(S_)                                                  \
     do {                                                                \
-        if (epi == EPI_I8_P8_NONNEG) OHIP_DWF_N(S_, EPI_I8_P8_NONNEG);  \
+        const int e = full_epilogue(epi, ep);                           \
+        if (e == EPI_I8_P8_FULL) OHIP_DWF_N(S_, EPI_I8_P8_FULL);        \
+        else if (epi == EPI_I8_P8_NONNEG) OHIP_DWF_N(S_, EPI_I8_P8_NONNEG); \
         else if (epi == EPI_I8_P8) OHIP_DWF_N(S_, EPI_I8_P8);           \
         else if (epi == EPI_F32_P8) OHIP_DWF_N(S_, EPI_F32_P8);         \
         else OHIP_DWF_N(S_, EPI_F32_P4);                                \
@@ -702,8 +710,8 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     static_assert(sizeof(DwArgs) == 112);
 #define OHIP_DWM_L(S_, E_, O_, K_)                                                                                        \
     do {                                                                                                                   \
-        if (E_ != EPI_I8_P8_NONNEG && ep.lrelu)                                                                            \
-            launch((conv_dw3x3_mfma_kernel<S_, E_, O_, K_, E_ != EPI_I8_P8_NONNEG>), grid, block, 0, stream, x, wa, out, pl); \
+        if (epi_clamp(E_) == 0 && ep.lrelu)                                                                                \
+            launch((conv_dw3x3_mfma_kernel<S_, E_, O_, K_, epi_clamp(E_) == 0>), grid, block, 0, stream, x, wa, out, pl);  \
         else                                                                                                               \
             launch((conv_dw3x3_mfma_kernel<S_, E_, O_, K_, false>), grid, block, 0, stream, x, wa, out, pl);    \
     } while (0)
@@ -721,7 +729,9 @@ hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const 
     } while (0)
 #define OHIP_DWM_E(S_)                                                \
     do {                                                              \
-        if (epi == EPI_I8_P8_NONNEG) OHIP_DWM(S_, EPI_I8_P8_NONNEG);  \
+        const int e = full_epilogue(epi, ep);                         \
+        if (e == EPI_I8_P8_FULL) OHIP_DWM(S_, EPI_I8_P8_FULL);        \
+        else if (epi == EPI_I8_P8_NONNEG) OHIP_DWM(S_, EPI_I8_P8_NONNEG); \
         else if (epi == EPI_I8_P8) OHIP_DWM(S_, EPI_I8_P8);           \
         else if (epi == EPI_F32_P8) OHIP_DWM(S_, EPI_F32_P8);         \
         else OHIP_DWM(S_, EPI_F32_P4);                                \

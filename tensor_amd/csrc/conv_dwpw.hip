@@ -30,7 +30,7 @@ namespace ohip {
 
 namespace {
 
-enum { DP_NONE = 3 };  // no second pointwise layer (KIND1, beside PP_I8, PP_NONNEG and PP_F32)
+enum { DP_NONE = 3, DP_FULL = 4 };  // no second pointwise layer, PP_NONNEG with Epilogue::so_full (KIND1, beside PP_I8, PP_NONNEG and PP_F32)
 
 struct DwPwArgs {
     PwPwLayer l[2];
@@ -87,8 +87,9 @@ void dwpw_pack_weights(const int8_t* w, int C, int ks, int8_t* dst) {
 
 // TAPS: 9 or 25. EPI: the first pointwise layer's epilogue: EPI_I8_P8; EPI_F32_P4_FUSED (with or without a residual and a twin; without
 // a second layer this is the plain fp32 result as well), EPI_F32_P4_PARTS, EPI_F32_SHUFFLE. KIND1: the second layer's result or DP_NONE.
+// DFULL: the depthwise layer ends as EPI_I8_P8_FULL says (else any int8 end).
 // out: the last layer's result; sum: with a second layer, the first one's fp32 result (null: not wanted).
-template <int NW, int TAPS, int EPI, int KIND1>
+template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>
 __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __restrict__ x, void* __restrict__ out, float* __restrict__ sum,
                                                                   DwPwArgs pa, PwAdd<EPI> ja) {
     constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, I8 = EPI == EPI_I8_P8, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
@@ -261,18 +262,25 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
             op += stride;
             if (op < pairs) load(op);  // (refilled in place: the next pair's bytes arrive under this one's requantization)
             const v4i si = *reinterpret_cast<const v4i*>(constsd + 16 * now + 4 * q), bi = *reinterpret_cast<const v4i*>(constsd + Cd + 16 * now + 4 * q);
-            int k[4];
+            unsigned bytes;
+            if constexpr (DFULL) {  // (dw_scale is doubled)
+                float t2[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float t = __fmul_rn(lrelu_or_not(epd, __fmaf_rn((float)acc[e], __int_as_float(si[e]), __int_as_float(bi[e]))), pa.dw_scale);
-                k[e] = (int)__fadd_rn(t, __builtin_copysignf(pa.dw_half, t));
+                for (int e = 0; e < 4; ++e) t2[e] = __fmul_rn(__fmaf_rn((float)acc[e], __int_as_float(si[e]), __int_as_float(bi[e])), pa.dw_scale);
+                bytes = quant4_full(t2, pa.dw_half);
+            } else {
+                int k[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float t = __fmul_rn(lrelu_or_not(epd, __fmaf_rn((float)acc[e], __int_as_float(si[e]), __int_as_float(bi[e]))), pa.dw_scale);
+                    k[e] = (int)__fadd_rn(t, __builtin_copysignf(pa.dw_half, t));
+                }
+                ohip_v2s lo = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[0], k[1])), hi = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[2], k[3]));
+                lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bottom);
+                hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bottom);
+                bytes = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
             }
-            ohip_v2s lo = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[0], k[1])), hi = __builtin_bit_cast(ohip_v2s, __builtin_amdgcn_cvt_pk_i16(k[2], k[3]));
-            lo = __builtin_elementwise_max(__builtin_elementwise_min(lo, top), bottom);
-            hi = __builtin_elementwise_max(__builtin_elementwise_min(hi, top), bottom);
-            if (2u * now + (q >> 1) < C8)
-                *reinterpret_cast<unsigned*>(px0 + row0 + 16 * now + 4 * q) =
-                    __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
+            if (2u * now + (q >> 1) < C8) *reinterpret_cast<unsigned*>(px0 + row0 + 16 * now + 4 * q) = bytes;
         }
     }
     __syncthreads();
@@ -319,7 +327,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
         float si[8], bi[8];
         constants(consts0, pairs0, ch0, si, bi);
         if constexpr (I8) {
-            const v2i b = pp_bytes<false>(ep0, l0, si, bi, c0, c1);
+            const v2i b = pp_bytes<0>(ep0, l0, si, bi, c0, c1);
             if constexpr (NEXT) {
                 if (ch0 < K0) *reinterpret_cast<v2i*>(to1 + ch0) = b;
             } else {
@@ -399,7 +407,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
                 const unsigned v = at_f4(K1), s = (unsigned)pr * 128u * HW;
                 store16(rout, r0, ch0 < K1 ? v : PR_OOB, s), store16(rout, r1, ch0 + 4 < K1 ? v : PR_OOB, s + HW * 16u);
             } else {
-                store8(rout, pp_bytes<KIND1 == PP_NONNEG>(ep1, l1, si, bi, c0, c1), ch0 < K1 ? at_b8(K1) : PR_OOB, (unsigned)pr * 32u * HW);
+                store8(rout, pp_bytes<KIND1 == DP_FULL ? 2 : KIND1 == PP_NONNEG ? 1 : 0>(ep1, l1, si, bi, c0, c1), ch0 < K1 ? at_b8(K1) : PR_OOB, (unsigned)pr * 32u * HW);
             }
         };
         layer(std::true_type{}, l1, pairs1, px1 + row1 + 16 * q, finish1);
@@ -512,15 +520,18 @@ bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0
     return cost < line * dwpw_cost_apart(s, gd, g0, g1);
 }
 
-template <int NW, int TAPS, int EPI, int KIND1>
+template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>
 static hipError_t launch_dwpw_waves(const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
-    launch((conv_dwpw_kernel<NW, TAPS, EPI, KIND1>), dim3((pa.tiles + 7) / 8 * 8), dim3(64 * NW), lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0));
+    launch((conv_dwpw_kernel<NW, TAPS, EPI, KIND1, DFULL>), dim3((pa.tiles + 7) / 8 * 8), dim3(64 * NW), lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0));
     return hipGetLastError();
 }
 template <int TAPS, int EPI, int KIND1>
-static hipError_t launch_dwpw(int waves, const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
-    return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1>(x, out, sum, pa, e0, lds, stream)
-                      : launch_dwpw_waves<8, TAPS, EPI, KIND1>(x, out, sum, pa, e0, lds, stream);
+static hipError_t launch_dwpw(int waves, bool dfull, const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
+    if (dfull)
+        return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1, true>(x, out, sum, pa, e0, lds, stream)
+                          : launch_dwpw_waves<8, TAPS, EPI, KIND1, true>(x, out, sum, pa, e0, lds, stream);
+    return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1, false>(x, out, sum, pa, e0, lds, stream)
+                      : launch_dwpw_waves<8, TAPS, EPI, KIND1, false>(x, out, sum, pa, e0, lds, stream);
 }
 
 hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const ConvGeom& gd, const Epilogue& ed, const int8_t* const w[2],
@@ -549,13 +560,17 @@ hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const
     pa.first_pack = e0.join ? (unsigned)e0.join->sh_pack0 : 8u;
     pa.lg = groups == 1 ? 0 : groups == 2 ? 1 : groups == 4 ? 2 : 3;
     pa.tiles = (int)((pa.total_pix + 16 * groups - 1) / (16 * groups));
-    const int next = g1 ? pa.l[1].kind : (int)DP_NONE;
+    const int next = !g1 ? (int)DP_NONE : pa.l[1].kind == PP_NONNEG && e1->so_full ? (int)DP_FULL : pa.l[1].kind;
+    if (next == DP_FULL) pa.l[1].scale += pa.l[1].scale;
+    const bool dfull = pa.dw_nonneg && ed.so_full;
+    if (dfull) pa.dw_scale += pa.dw_scale;
     const bool shuffle = e0.join && e0.join->other;
-#define OHIP_DP(T_, E_, N_) return launch_dwpw<T_, E_, N_>(waves, x, out, sum, pa, e0, lds, stream)
+#define OHIP_DP(T_, E_, N_) return launch_dwpw<T_, E_, N_>(waves, dfull, x, out, sum, pa, e0, lds, stream)
 #define OHIP_DPN(T_, E_)                             \
     do {                                             \
         if (next == PP_I8) OHIP_DP(T_, E_, PP_I8);   \
         if (next == PP_NONNEG) OHIP_DP(T_, E_, PP_NONNEG); \
+        if (next == DP_FULL) OHIP_DP(T_, E_, DP_FULL); \
         if (next == PP_F32) OHIP_DP(T_, E_, PP_F32); \
     } while (0)
     if (gd.kh == 3) {

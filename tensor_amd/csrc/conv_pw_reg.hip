@@ -34,14 +34,14 @@ struct PwRegArgs {
     unsigned short C8;
     unsigned char hw_s, lrelu;
     float p0;                    // slope of LeakyReLU
-    float scale, half;           // int8 result: the output scale of every channel, the rounding constant; fp32: act_lo, act_hi
+    float scale, half;           // int8 result: the output scale of every channel (EPI_I8_P8_FULL: doubled), the rounding constant; fp32: act_lo, act_hi
     unsigned qh;                 // upper clamp of the rounded result, in both halves (EPI_I8_P8_NONNEG)
 
     __device__ FastDiv hw() const { return {hw_m, hw_s, (unsigned)HW}; }
 };
 template <int EPI>
 __device__ __forceinline__ Epilogue pw_epilogue(const PwRegArgs& pa, const PwAdd<EPI>& ja) {
-    constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG;
+    constexpr bool I8 = epi_is_i8(EPI);
     Epilogue ep{};
     ep.lrelu = pa.lrelu != 0, ep.act_p0 = pa.p0;
     if (I8) ep.round_half = pa.half;
@@ -56,7 +56,7 @@ __device__ __forceinline__ Epilogue pw_epilogue(const PwRegArgs& pa, const PwAdd
 template <int FN, int CG, int EPI>
 __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
                                                           PwRegArgs pa, PwAdd<EPI> ja) {
-    constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
+    constexpr bool I8 = epi_is_i8(EPI), NONNEG = epi_clamp(EPI) != 0;
     constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS, SLICE = EPI == EPI_F32_SLICE;
     constexpr bool ADD = SHUF || FUSED;  // reads elements of another fp32 blob
     const Epilogue ep = pw_epilogue<EPI>(pa, ja);
@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
                 const int a8[8] = {c0[j][0], c0[j][1], c0[j][2], c0[j][3], c1[j][0], c1[j][1], c1[j][2], c1[j][3]};
-                store8(rout, epi8_quant_i8p8<NONNEG, LRELU ? 1 : 0>(ep, prm, a8), ch0 < K ? vo[j] : PR_OOB, (unsigned)pr * 32u * HW);
+                store8(rout, epi8_quant_i8p8<epi_clamp(EPI), LRELU ? 1 : 0>(ep, prm, a8), ch0 < K ? vo[j] : PR_OOB, (unsigned)pr * 32u * HW);
             }
         } else {
 #pragma unroll
@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(256) conv_pw_reg_kernel(const int8_t* __restri
 template <int FN, int NS, int EPI>
 __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wpk, void* __restrict__ out,
                                                             PwRegArgs pa, PwAdd<EPI> ja) {
-    constexpr bool I8 = EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG, NONNEG = EPI == EPI_I8_P8_NONNEG;
+    constexpr bool I8 = epi_is_i8(EPI), NONNEG = epi_clamp(EPI) != 0;
     constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS, SLICE = EPI == EPI_F32_SLICE;
     constexpr int OWN = FN < 2 ? 1 : FN / 2;  // half pairs that a wave finishes (of 2 FN; with FN == 1 waves 0 and 1 have one each)
     __shared__ v4i red[2][2 * FN][3][64];     // [buffer][half pair][the other waves][lane]
@@ -344,7 +344,7 @@ __global__ void __launch_bounds__(256) conv_pw_split_kernel(const int8_t* __rest
         for (int o = 0; o < OWN; ++o) {
             if constexpr (I8) {
                 const v4i so = v4i{1, 1, 1, 1} * __float_as_int(pa.scale);
-                const unsigned w = dw_requant4<NONNEG, LRELU ? 1 : 0>(ep, c[o], k.si, k.bi, so, pa.qh, pa.qh);
+                const unsigned w = dw_requant4<epi_clamp(EPI), LRELU ? 1 : 0>(ep, c[o], k.si, k.bi, so, pa.qh, pa.qh);
                 __builtin_amdgcn_raw_buffer_store_b32(w, rout, (int)(ch < K ? vo[o] : PR_OOB), (int)((unsigned)pr * 32u * HW), 0);
                 continue;
             }
@@ -473,6 +473,7 @@ static hipError_t launch_pw_reg_e(int epi, const int8_t* x, const int8_t* wpk, v
     switch (epi) {
     case EPI_I8_P8: return launch_pw_reg<FN, CG, EPI_I8_P8>(x, wpk, out, pa, ep, slices, stream);
     case EPI_I8_P8_NONNEG: return launch_pw_reg<FN, CG, EPI_I8_P8_NONNEG>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_I8_P8_FULL: return launch_pw_reg<FN, CG, EPI_I8_P8_FULL>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_P4: return launch_pw_reg<FN, CG, EPI_F32_P4>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_P4_FUSED: return launch_pw_reg<FN, CG, EPI_F32_P4_FUSED>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_SHUFFLE: return launch_pw_reg<FN, CG, EPI_F32_SHUFFLE>(x, wpk, out, pa, ep, slices, stream);
@@ -488,6 +489,7 @@ static hipError_t launch_pw_reg_wide(int epi, const int8_t* x, const int8_t* wpk
     switch (epi) {
     case EPI_I8_P8: return launch_pw_reg<4, CG, EPI_I8_P8>(x, wpk, out, pa, ep, slices, stream);
     case EPI_I8_P8_NONNEG: return launch_pw_reg<4, CG, EPI_I8_P8_NONNEG>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_I8_P8_FULL: return launch_pw_reg<4, CG, EPI_I8_P8_FULL>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_P4: return launch_pw_reg<4, CG, EPI_F32_P4>(x, wpk, out, pa, ep, slices, stream);
     }
     return hipErrorInvalidValue;
@@ -507,6 +509,7 @@ static hipError_t launch_pw_split_e(int epi, const int8_t* x, const int8_t* wpk,
     switch (epi) {
     case EPI_I8_P8: return launch_pw_split<FN, NS, EPI_I8_P8>(x, wpk, out, pa, ep, slices, stream);
     case EPI_I8_P8_NONNEG: return launch_pw_split<FN, NS, EPI_I8_P8_NONNEG>(x, wpk, out, pa, ep, slices, stream);
+    case EPI_I8_P8_FULL: return launch_pw_split<FN, NS, EPI_I8_P8_FULL>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_P4: return launch_pw_split<FN, NS, EPI_F32_P4>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_P4_FUSED: return launch_pw_split<FN, NS, EPI_F32_P4_FUSED>(x, wpk, out, pa, ep, slices, stream);
     case EPI_F32_SHUFFLE: return launch_pw_split<FN, NS, EPI_F32_SHUFFLE>(x, wpk, out, pa, ep, slices, stream);
@@ -529,6 +532,8 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
     pa.lrelu = ep.lrelu, pa.p0 = ep.act_p0, pa.scale = i8 ? so : ep.act_lo, pa.half = i8 ? ep.round_half : ep.act_hi;
     const float both[2] = {so, so};
     if (epi == EPI_I8_P8_NONNEG) conv_pw_stream_clamps(ep.act_hi, ep.round_half, both, 2, &pa.qh);
+    const int instance = full_epilogue(epi, ep);
+    if (instance == EPI_I8_P8_FULL) pa.scale = so + so;
     int fn = 1, per = 1;
     const bool split = force ? (force & 64) != 0 : steps > PW_REG_STEPS;
     const bool wide = split || epi == EPI_F32_P4 || epi == EPI_I8_P8 || epi == EPI_I8_P8_NONNEG;  // (registers)
@@ -545,9 +550,9 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
     if (slices > 65535) return hipErrorInvalidValue;
     if (split) {
 #define OHIP_PWS(NS_)                                                                                             \
-    if ((steps + 3) / 4 == NS_) return fn == 1   ? launch_pw_split_e<1, NS_>(epi, x, wpk, out, pa, ep, slices, stream) \
-                                       : fn == 2 ? launch_pw_split_e<2, NS_>(epi, x, wpk, out, pa, ep, slices, stream) \
-                                                 : launch_pw_split_e<4, NS_>(epi, x, wpk, out, pa, ep, slices, stream);
+    if ((steps + 3) / 4 == NS_) return fn == 1   ? launch_pw_split_e<1, NS_>(instance, x, wpk, out, pa, ep, slices, stream) \
+                                       : fn == 2 ? launch_pw_split_e<2, NS_>(instance, x, wpk, out, pa, ep, slices, stream) \
+                                                 : launch_pw_split_e<4, NS_>(instance, x, wpk, out, pa, ep, slices, stream);
         OHIP_PWS(1)
         OHIP_PWS(2)
         OHIP_PWS(3)
@@ -556,9 +561,9 @@ hipError_t run_conv_pw_reg(const int8_t* x, const int8_t* wpk, float so, void* o
         return hipErrorInvalidValue;
     }
 #define OHIP_PWR(CG_)                                                                                      \
-    if (steps == CG_ && fn == 4) return launch_pw_reg_wide<CG_>(epi, x, wpk, out, pa, ep, slices, stream); \
-    if (steps == CG_) return fn == 1 ? launch_pw_reg_e<1, CG_>(epi, x, wpk, out, pa, ep, slices, stream)    \
-                                     : launch_pw_reg_e<2, CG_>(epi, x, wpk, out, pa, ep, slices, stream);
+    if (steps == CG_ && fn == 4) return launch_pw_reg_wide<CG_>(instance, x, wpk, out, pa, ep, slices, stream); \
+    if (steps == CG_) return fn == 1 ? launch_pw_reg_e<1, CG_>(instance, x, wpk, out, pa, ep, slices, stream)    \
+                                     : launch_pw_reg_e<2, CG_>(instance, x, wpk, out, pa, ep, slices, stream);
     OHIP_PWR(1)
     OHIP_PWR(2)
     OHIP_PWR(3)

@@ -21,7 +21,8 @@ struct PwPwLayer {
 };
 
 // Eight channels of a pixel as bytes (PP_I8, PP_NONNEG); four as values (PP_F32). (The clamp is open for LeakyReLU.)
-template <bool NONNEG>
+// CLAMP: as epi_clamp says (2: PwPwLayer::scale is doubled)
+template <int CLAMP>
 __device__ __forceinline__ v2i pp_bytes(const Epilogue& ep, const PwPwLayer& l, const float (&si)[8], const float (&bi)[8], const v4i& c0, const v4i& c1) {
     Epi8 prm;
 #pragma unroll
@@ -29,7 +30,7 @@ __device__ __forceinline__ v2i pp_bytes(const Epilogue& ep, const PwPwLayer& l, 
 #pragma unroll
     for (int e = 0; e < 4; ++e) prm.qh[e] = l.qh;
     const int a8[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
-    return epi8_quant_i8p8<NONNEG>(ep, prm, a8);
+    return epi8_quant_i8p8<CLAMP>(ep, prm, a8);
 }
 __device__ __forceinline__ v4i pp_values(const Epilogue& ep, const float* si, const float* bi, const v4i& c) {
     v4i r;

@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF 
 
     auto put = [&](int c, float si, float bi, float so) {
         consts[c] = si, consts[nc + c] = bi;
-        if constexpr (EPI != EPI_F32_P4) consts[2 * nc + c] = so;
+        if constexpr (EPI != EPI_F32_P4) consts[2 * nc + c] = EPI == EPI_I8_P8_FULL ? so + so : so;
         if constexpr (EPI == EPI_I8_P8_NONNEG)
             reinterpret_cast<unsigned short*>(consts + 3 * nc)[c] = (unsigned short)min((int)__fadd_rn(__fmul_rn(ep.act_hi, so), ep.round_half), 127);
     };
@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(256, EPI == EPI_GENERIC ? 2 : FM == 2 && !INF 
                                 if (px_ok[j])
                                     epi4_store_f32p4<false>((float*)out, ep, si, bi, (size_t)(out_at[j] + ch_at + (unsigned)h * (unsigned)OHW * 4), v[0], v[1], v[2], v[3]);
                             } else {
-                                const int b4 = epi4_quant_i8<EPI == EPI_I8_P8_NONNEG>(ep, si, bi, so, qh, v[0], v[1], v[2], v[3]);
+                                const int b4 = epi4_quant_i8<epi_clamp(EPI)>(ep, si, bi, so, qh, v[0], v[1], v[2], v[3]);
                                 if (h == 0) {
                                     bytes[j] = b4;
                                     asm volatile("" : "+v"(bytes[j]));  // (packed here, not behind the condition of the store)
@@ -603,7 +603,7 @@ hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out
     ra.consts = (int)((lds + 15) / 16 * 16);
     lds = rows_lds(lds, ra.blocks_per_wg, c.fm);
     const dim3 grid((unsigned)ra.n_tiles, (unsigned)((blocks + ra.blocks_per_wg - 1) / ra.blocks_per_wg), (unsigned)g_in.groups);
-    const int epi = pick_epilogue(ep, ra.g.K);
+    const int epi = full_epilogue(pick_epilogue(ep, ra.g.K), ep);
     auto go = [&](auto kernel, auto ea) {
         if (lds > 64 * 1024) {  // (rows that fill the tile's share: the constants lie beyond it)
             const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024);
@@ -618,7 +618,7 @@ hipError_t run_conv_rows(const void* x, bool f32in, const int8_t* wpk, void* out
         if constexpr (E_ != EPI_GENERIC) return go(conv_rows_kernel<FM_, FN_, E_, true>, EpiArgs<E_>::of(ep)); \
     }
 #define OHIP_ROWS(I_, FM_, FN_) \
-    OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8) OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8_NONNEG) OHIP_ROWS2(I_, FM_, FN_, EPI_F32_P4) OHIP_ROWS2(I_, FM_, FN_, EPI_GENERIC)
+    OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8) OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8_NONNEG) OHIP_ROWS2(I_, FM_, FN_, EPI_I8_P8_FULL) OHIP_ROWS2(I_, FM_, FN_, EPI_F32_P4) OHIP_ROWS2(I_, FM_, FN_, EPI_GENERIC)
     OHIP_ROWS(0, 2, 2)
     OHIP_ROWS(1, 2, 4)
     OHIP_ROWS(2, 4, 2)

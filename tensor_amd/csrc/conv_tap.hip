@@ -274,9 +274,9 @@ __global__ void __launch_bounds__(64 * WK * WN) conv_tap_kernel(const int8_t* __
             Epi8 prm;
             epi8_load<EPI>(prm, ep, ch0);
             const unsigned ch = (unsigned)ch_base + (unsigned)ch0;  // in the tensor
-            if constexpr (EPI == EPI_I8_P8 || EPI == EPI_I8_P8_NONNEG) {
+            if constexpr (epi_is_i8(EPI)) {
                 const size_t o = ((size_t)(n * (unsigned)(Ks / 8) + ch / 8) * (unsigned)OHW + pix) * 8;
-                epi8_store_i8p8<EPI == EPI_I8_P8_NONNEG>((int8_t*)out, ep, prm, o, a8);
+                epi8_store_i8p8<epi_clamp(EPI)>((int8_t*)out, ep, prm, o, a8);
             } else if constexpr (EPI == EPI_F32_SHUFFLE) {
                 if (ep.lrelu) epi8_store_shuffle<1>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, K, OHW);
                 else epi8_store_shuffle<0>(ep, ja, prm.si, prm.bi, a8, n, pix, ch0, K, OHW);
@@ -499,16 +499,17 @@ hipError_t run_conv_tap(const void* x, bool f32in, const int8_t* wpk, void* out,
     const TapConfig c = kTapConfigs[config];
     const long px = (long)g.N * g.OH * g.OW, per = 16l * c.fn * c.wn;
     ta.n_pix_tiles = (int)((px + per - 1) / per);
-    int epi = pick_epilogue(ep, K);
+    int epi = full_epilogue(pick_epilogue(ep, K), ep);
     if (epi == EPI_F32_P4 && ep.fused()) epi = ep.join == nullptr ? EPI_F32_P4_FUSED : ep.join->other != nullptr ? EPI_F32_SHUFFLE : EPI_F32_P4_PARTS;
 #define OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, E_)                                                                           \
     if (config == I_ && epi == E_) {                                                                                        \
         if (!f32in) return launch_tap<FM_, FN_, WK_, WN_, D_, E_, false>(x, wpk, out, ta, ep, g.groups, stream);         \
-        if constexpr (E_ != EPI_GENERIC && E_ < EPI_F32_SHUFFLE && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g.groups, stream); \
+        if constexpr (E_ != EPI_GENERIC && (E_ < EPI_F32_SHUFFLE || E_ == EPI_I8_P8_FULL) && FN_ < 4) return launch_tap<FM_, FN_, WK_, WN_, D_ < 4 ? D_ : 2, E_, true>(x, wpk, out, ta, ep, g.groups, stream); \
     }
 #define OHIP_TAP(I_, FM_, FN_, WK_, WN_, D_)                 \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8)         \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8_NONNEG)  \
+    OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_I8_P8_FULL)    \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4)        \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_P4_FUSED)  \
     OHIP_TAP2(I_, FM_, FN_, WK_, WN_, D_, EPI_F32_SHUFFLE)   \

@@ -52,7 +52,8 @@ struct XdwArgs {  // (a launch costs the host 0.1 us more for every 32 bytes of 
     DwGrid dg;
 };
 
-template <int S, int EPI, bool XNN, int NG, int CK>
+// EPI: the depthwise layer's epilogue, and the pointwise one's
+template <int S, int EPI, int NG, int CK>
 __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S == 2 && NG <= 2)) ? 3 : 2) conv_xdw_kernel(const int8_t* __restrict__ x, const int8_t* __restrict__ wx,
                                                        const int8_t* __restrict__ wa, void* __restrict__ out, XdwArgs g,
                                                        EpiArgs<EPI> eax, EpiArgs<EPI> ea) {
@@ -121,9 +122,10 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
     const int chx = 16 * pr + 4 * q;
     const v4i six = *reinterpret_cast<const v4i*>(epx.scale_in + chx);
     const v4i bix = *reinterpret_cast<const v4i*>(epx.bias + chx);
-    const v4i sox = *reinterpret_cast<const v4i*>(epx.scale_out + chx);
+    v4i sox = *reinterpret_cast<const v4i*>(epx.scale_out + chx);
+    if constexpr (EPI == EPI_I8_P8_FULL) sox = dw_doubled(sox);
     unsigned qx01 = 0, qx23 = 0;
-    if constexpr (XNN) qx01 = dw_clamp_pair(epx, sox[0], sox[1]), qx23 = dw_clamp_pair(epx, sox[2], sox[3]);
+    if constexpr (EPI == EPI_I8_P8_NONNEG) qx01 = dw_clamp_pair(epx, sox[0], sox[1]), qx23 = dw_clamp_pair(epx, sox[2], sox[3]);
     int8_t* const lds_w = lds + (q >> 1) * OCT + (n + 2) * 8 + 4 * (q & 1);  // this lane's dword of pixel group 0, line 0
     // the pointwise layer on input row j of the walk (in src) into LDS line `line` of both octets
     auto expand_write = [&](int j, int line, const b_t (&src)[NG]) {
@@ -144,7 +146,7 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
         }
 #pragma unroll
         for (int p = 0; p < NG; ++p) {
-            unsigned w = dw_requant4<XNN>(epx, d[p], six, bix, sox, qx01, qx23) & rowm;
+            unsigned w = dw_requant4<epi_clamp(EPI)>(epx, d[p], six, bix, sox, qx01, qx23) & rowm;
             if (16 * p + n >= g.W) w = 0;
             *reinterpret_cast<unsigned*>(lds_w + line * LINE + p * 128) = w;
         }
@@ -196,6 +198,7 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
             // it from scalar registers value after value)
 #pragma unroll
             for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(bi[oo][t][e]));
+            if constexpr (EPI == EPI_I8_P8_FULL) so[oo][t] = dw_doubled(so[oo][t]);
             if constexpr (EPI == EPI_I8_P8_NONNEG) {
                 qh[oo][t][0] = dw_clamp_pair(ep, so[oo][t][0], so[oo][t][1]);
                 qh[oo][t][1] = dw_clamp_pair(ep, so[oo][t][2], so[oo][t][3]);
@@ -214,7 +217,7 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
 
     v4i cur[2][NCH][T];
     auto epilogue_store = [&](int r) {  // output row r of the strip, from cur
-        constexpr bool NONNEG = EPI == EPI_I8_P8_NONNEG;
+        constexpr int CLAMP = epi_clamp(EPI);
 #pragma unroll
         for (int oo = 0; oo < 2; ++oo) {
             const unsigned s_row =
@@ -223,12 +226,12 @@ __global__ void __launch_bounds__(256, ((CK == 32 && (NG <= 4 || S == 2)) || (S 
             for (int c = 0; c < NCH; ++c) {
                 if constexpr (S == 1) {
                     v2i w2;
-                    w2[0] = (int)dw_requant4<NONNEG>(ep, cur[oo][c][0], si[oo][0], bi[oo][0], so[oo][0], qh[oo][0][0], qh[oo][0][1]);
-                    w2[1] = (int)dw_requant4<NONNEG>(ep, cur[oo][c][T - 1], si[oo][T - 1], bi[oo][T - 1], so[oo][T - 1], qh[oo][T - 1][0],
+                    w2[0] = (int)dw_requant4<CLAMP>(ep, cur[oo][c][0], si[oo][0], bi[oo][0], so[oo][0], qh[oo][0][0], qh[oo][0][1]);
+                    w2[1] = (int)dw_requant4<CLAMP>(ep, cur[oo][c][T - 1], si[oo][T - 1], bi[oo][T - 1], so[oo][T - 1], qh[oo][T - 1][0],
                                                      qh[oo][T - 1][1]);
                     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u_store, w2), rout, (int)v_out[c], (int)s_row, 0);
                 } else {
-                    const unsigned w1 = dw_requant4<NONNEG>(ep, cur[oo][c][0], si[oo][0], bi[oo][0], so[oo][0], qh[oo][0][0], qh[oo][0][1]);
+                    const unsigned w1 = dw_requant4<CLAMP>(ep, cur[oo][c][0], si[oo][0], bi[oo][0], so[oo][0], qh[oo][0][0], qh[oo][0][1]);
                     __builtin_amdgcn_raw_buffer_store_b32(w1, rout, (int)v_out[c], (int)s_row, 0);
                 }
             }
@@ -345,32 +348,33 @@ hipError_t run_conv_xdw(const int8_t* x, const int8_t* wx, const int8_t* wa, voi
     const unsigned in_bytes = (unsigned)((size_t)gx.N * gx.C * gx.H * gx.W);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW);
     const XdwArgs xa = {g.H, g.W, g.OH, g.OW, g.C, gx.C, g.ph, n_strips, rps, in_bytes, out_bytes, DwGrid::of(grid.x, grid.y, (unsigned)(g.C / 16), wpb)};
-    const bool nn = epi_d == EPI_I8_P8_NONNEG;
-#define OHIP_XDW_L(S_, NN_, G_, CK_)                                                                                              \
-    launch((conv_xdw_kernel<S_, NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8, NN_, G_, CK_>), grid, block, lds_bytes, stream, x, wx, wa, \
-                       out, xa, EpiArgs<NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8>::of(epx), EpiArgs<NN_ ? EPI_I8_P8_NONNEG : EPI_I8_P8>::of(ep))
-#define OHIP_XDW_G(S_, NN_, CK_)                 \
+    const int epi = epx.so_full ? full_epilogue(epi_d, ep) : epi_d;
+#define OHIP_XDW_L(S_, E_, G_, CK_)                                                                                   \
+    launch((conv_xdw_kernel<S_, E_, G_, CK_>), grid, block, lds_bytes, stream, x, wx, wa, out, xa, EpiArgs<E_>::of(epx), EpiArgs<E_>::of(ep))
+#define OHIP_XDW_G(S_, E_, CK_)                  \
     do {                                         \
         switch (NG) {                            \
-        case 1: OHIP_XDW_L(S_, NN_, 1, CK_); break; \
-        case 2: OHIP_XDW_L(S_, NN_, 2, CK_); break; \
-        case 4: OHIP_XDW_L(S_, NN_, 4, CK_); break; \
-        case 7: OHIP_XDW_L(S_, NN_, 7, CK_); break; \
-        default: OHIP_XDW_L(S_, NN_, 8, CK_); break; \
+        case 1: OHIP_XDW_L(S_, E_, 1, CK_); break; \
+        case 2: OHIP_XDW_L(S_, E_, 2, CK_); break; \
+        case 4: OHIP_XDW_L(S_, E_, 4, CK_); break; \
+        case 7: OHIP_XDW_L(S_, E_, 7, CK_); break; \
+        default: OHIP_XDW_L(S_, E_, 8, CK_); break; \
         }                                        \
     } while (0)
-#define OHIP_XDW_C(S_, NN_)                      \
+#define OHIP_XDW_C(S_, E_)                       \
     do {                                         \
-        if (gx.C <= 32) OHIP_XDW_G(S_, NN_, 32); \
-        else OHIP_XDW_G(S_, NN_, 128);           \
+        if (gx.C <= 32) OHIP_XDW_G(S_, E_, 32);  \
+        else OHIP_XDW_G(S_, E_, 128);            \
     } while (0)
-    if (g.sh == 1) {
-        if (nn) OHIP_XDW_C(1, true);
-        else OHIP_XDW_C(1, false);
-    } else {
-        if (nn) OHIP_XDW_C(2, true);
-        else OHIP_XDW_C(2, false);
-    }
+#define OHIP_XDW_E(S_)                                                        \
+    do {                                                                      \
+        if (epi == EPI_I8_P8_FULL) OHIP_XDW_C(S_, EPI_I8_P8_FULL);            \
+        else if (epi == EPI_I8_P8_NONNEG) OHIP_XDW_C(S_, EPI_I8_P8_NONNEG);   \
+        else OHIP_XDW_C(S_, EPI_I8_P8);                                       \
+    } while (0)
+    if (g.sh == 1) OHIP_XDW_E(1);
+    else OHIP_XDW_E(2);
+#undef OHIP_XDW_E
 #undef OHIP_XDW_C
 #undef OHIP_XDW_G
 #undef OHIP_XDW_L
