@@ -229,6 +229,53 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
             }
         }
     };
+    // A: where this lane's pixel of a group goes in the expanded lines, -1 beyond the band. It is the same for every slice: a wave's first two
+    // groups keep it, as a wave's first item of B keeps its places. (What the address arithmetic of every item took, and the operands of B
+    // behind the barrier: 64 -> 384 -> 64 @14x14 b64 10.55 -> 9.80 us; two groups of A interleaved in a wave's code: 9.97.)
+    const int GA = (in_pixN + 15) / 16;  // (of this band: at most a.GA)
+    auto line_at = [&](int ga) {
+        const int pix = ga * 16 + p;
+        const unsigned ipix = (unsigned)(in_pix0 + pix);
+        const unsigned iy = __umul24(ipix, a.inv_w) >> 20;  // (a full multiplication takes four times as long)
+        const unsigned ix = ipix - __umul24(iy, (unsigned)a.W);
+        const int er = (int)iy - (r0 - 1);
+        return pix < in_pixN ? __mul24((4 * prE + q) * a.ER + er, a.pitch) + ((int)ix + 2) * 8 : -1;
+    };
+    const int line_at0 = line_at(gaE0), line_at1 = line_at(gaE0 + gaEs);
+    // B: where this lane reads an item's rows (line of the expanded octet) and puts its pixel's eight results, -1 for none; the first item's kept
+    constexpr int rcs = WV > noct ? WV / noct : 1;
+    const int rc0 = WV > noct ? wave / noct : 0, nrc = (int)div_by((unsigned)(rows + a.rpi - 1), a.by_rpi);
+    auto from_line = [&](int rc) { return __mul24(min(rc * a.rpi + row_sub, a.RB - 1), a.pitch) + (4 * nx + 2 * q) * 8; };
+    auto to_group = [&](int rc) {
+        const int orow = rc * a.rpi + row_sub, pix = __mul24(orow, a.W) + oxB;
+        return laneB && orow < rows && oxB < a.W ? (pix >> 4) * kqs * 256 + (pix & 15) * 16 : -1;
+    };
+    constexpr bool KEEP = CLAMP == 2 || WV == 8;  // (the others have no registers left for it)
+    const int from0 = KEEP ? from_line(rc0) : 0, to0 = KEEP ? to_group(rc0) : 0;
+    // B: the weight operands and the constants of an octet. Where a wave has one per slice they are made in front of the barrier behind A,
+    // by the waves that have fewer groups there while the others are at their last
+    Epi8 prmB;
+    auto depthwise_operands = [&](int oct_abs) {
+        oct_abs = min(oct_abs, a.Ce8 - 1);
+        const int* const c = ldsC2 + oct_abs * BLK_OCT_DW;
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy) {
+            const unsigned w0 = (unsigned)c[dy * 8 + (p & 3)], w1 = (unsigned)c[dy * 8 + 4 + (p & 3)];
+            wB[dy][0][0] = (int)__builtin_amdgcn_perm(0u, w0, selB[0]), wB[dy][0][2] = (int)__builtin_amdgcn_perm(0u, w0, selB[1]);
+            wB[dy][1][1] = (int)__builtin_amdgcn_perm(0u, w1, selB[0]), wB[dy][1][3] = (int)__builtin_amdgcn_perm(0u, w1, selB[1]);
+        }
+        const v4i* cv = reinterpret_cast<const v4i*>(c + 24);
+        const v4i s0 = cv[0], s1 = cv[1], b0 = cv[2], b1 = cv[3];
+        v4i o0 = {}, o1 = {}, ch = {};
+        if constexpr (CLAMP != 2) o0 = cv[4], o1 = cv[5], ch = cv[6];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            prmB.si[e] = __int_as_float(s0[e]), prmB.si[4 + e] = __int_as_float(s1[e]);
+            prmB.bi[e] = __int_as_float(b0[e]), prmB.bi[4 + e] = __int_as_float(b1[e]);
+            prmB.so[e] = CLAMP == 2 ? a.so2 : __int_as_float(o0[e]), prmB.so[4 + e] = CLAMP == 2 ? a.so2 : __int_as_float(o1[e]);
+            prmB.qh[e] = (unsigned)ch[e];
+        }
+    };
     blk_barrier();
 
     for (int s = s_begin; s < s_end; ++s) {
@@ -236,7 +283,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
         if constexpr (PFP) load_wP(s);
         {
             const int pair_abs = s * npairsE + prE;
-            if (32 * pair_abs < a.Ce) {  // wave-uniform
+            if (32 * pair_abs < a.Ce && gaE0 < GA) {  // wave-uniform
                 Epi8 prm;
                 {
                     const v4i* c = reinterpret_cast<const v4i*>(ldsC1 + pair_abs * BLK_PAIR_DW);
@@ -251,8 +298,7 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
                         prm.qh[e] = (unsigned)ch[e];
                     }
                 }
-                char* const eo = ldsE + (size_t)((4 * prE + q) * a.ER) * a.pitch;
-                for (int ga = gaE0; ga < a.GA; ga += gaEs) {
+                auto item = [&](int ga, int at) {
                     v4i c0, c1;
                     {
                         const v4i b = blk_lds[(ga * a.cgE) * 64 + lane];
@@ -268,67 +314,46 @@ __global__ void __launch_bounds__(64 * WV) conv_block_kernel(const BlockArgs a) 
                         }
                     const int a8[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
                     const v2i r = epi8_quant_i8p8<CLAMP, 0>(a.e1, prm, a8);
-                    const int pix = ga * 16 + p;
-                    if (pix < in_pixN) {
-                        const unsigned ipix = (unsigned)(in_pix0 + pix);
-                        const unsigned iy = __umul24(ipix, a.inv_w) >> 20;  // (a full multiplication takes four times as long)
-                        const unsigned ix = ipix - __umul24(iy, (unsigned)a.W);
-                        const int er = (int)iy - (r0 - 1);
-                        *reinterpret_cast<v2i*>(eo + __mul24(er, a.pitch) + (ix + 2) * 8) = r;
-                    }
-                }
+                    if (at >= 0) *reinterpret_cast<v2i*>(ldsE + at) = r;
+                };
+                item(gaE0, line_at0);
+                if (gaE0 + gaEs < GA) item(gaE0 + gaEs, line_at1);
+                for (int ga = gaE0 + 2 * gaEs; ga < GA; ga += gaEs) item(ga, line_at(ga));
             }
         }
+        if constexpr (OPW == 1) depthwise_operands(s * noct + wave % noct);
         blk_barrier();
         // ================= B: depthwise =================
         if (s + 1 < s_end) load_wA(s + 1);
         {
-            const int nrc = (int)div_by((unsigned)(rows + a.rpi - 1), a.by_rpi);
 #pragma unroll
             for (int k = 0; k < OPW; ++k) {
             const int ol = wave % noct + WV * k;
             const int oct_abs = s * noct + ol;
             if (oct_abs < a.Ce8) {  // wave-uniform
-                const int* const c = ldsC2 + oct_abs * BLK_OCT_DW;
-#pragma unroll
-                for (int dy = 0; dy < 3; ++dy) {
-                    const unsigned w0 = (unsigned)c[dy * 8 + (p & 3)], w1 = (unsigned)c[dy * 8 + 4 + (p & 3)];
-                    wB[dy][0][0] = (int)__builtin_amdgcn_perm(0u, w0, selB[0]), wB[dy][0][2] = (int)__builtin_amdgcn_perm(0u, w0, selB[1]);
-                    wB[dy][1][1] = (int)__builtin_amdgcn_perm(0u, w1, selB[0]), wB[dy][1][3] = (int)__builtin_amdgcn_perm(0u, w1, selB[1]);
-                }
-                Epi8 prm;
-                {
-                    const v4i* cv = reinterpret_cast<const v4i*>(c + 24);
-                    const v4i s0 = cv[0], s1 = cv[1], b0 = cv[2], b1 = cv[3];
-                    v4i o0 = {}, o1 = {}, ch = {};
-                    if constexpr (CLAMP != 2) o0 = cv[4], o1 = cv[5], ch = cv[6];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        prm.si[e] = __int_as_float(s0[e]), prm.si[4 + e] = __int_as_float(s1[e]);
-                        prm.bi[e] = __int_as_float(b0[e]), prm.bi[4 + e] = __int_as_float(b1[e]);
-                        prm.so[e] = CLAMP == 2 ? a.so2 : __int_as_float(o0[e]), prm.so[4 + e] = CLAMP == 2 ? a.so2 : __int_as_float(o1[e]);
-                        prm.qh[e] = (unsigned)ch[e];
-                    }
-                }
-                const char* const ei = ldsE + (size_t)(ol * a.ER) * a.pitch + (4 * nx + 2 * q) * 8;
-                char* const dout = ldsD + (size_t)(ol >> 1) * 256 + (ol & 1) * 8;
-                for (int rc = WV > noct ? wave / noct : 0; rc < nrc; rc += WV > noct ? WV / noct : 1) {
-                    const int orow = rc * a.rpi + row_sub;
-                    const int orc = min(orow, a.RB - 1);
+                if constexpr (OPW > 1) depthwise_operands(oct_abs);
+                const int at_e = __mul24(ol * a.ER, a.pitch), at_d = (ol >> 1) * 256 + (ol & 1) * 8;
+                auto item = [&](int from, int to) {
+                    const char* const row = ldsE + at_e + from;
                     v4i c0 = zero4, c1 = zero4;
 #pragma unroll
                     for (int dy = 0; dy < 3; ++dy) {
-                        const v4i b = *reinterpret_cast<const v4i*>(ei + __mul24(orc + dy, a.pitch));
+                        const v4i b = *reinterpret_cast<const v4i*>(row + dy * a.pitch);
                         c0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(wB[dy][0], b, dy ? c0 : zero4, 0, 0, 0);
                         c1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(wB[dy][1], b, dy ? c1 : zero4, 0, 0, 0);
                     }
                     const int a8[8] = {c0[0], c0[1], c0[2], c0[3], c1[0], c1[1], c1[2], c1[3]};
-                    const v2i r = epi8_quant_i8p8<CLAMP, 0>(a.e2, prm, a8);
-                    if (laneB && orow < rows && oxB < a.W) {
-                        const int pix = __mul24(orow, a.W) + oxB;
-                        *reinterpret_cast<v2i*>(dout + (pix >> 4) * kqs * 256 + (pix & 15) * 16) = r;
-                    }
+                    const v2i r = epi8_quant_i8p8<CLAMP, 0>(a.e2, prmB, a8);
+                    if (to >= 0) *reinterpret_cast<v2i*>(ldsD + at_d + to) = r;
+                };
+                int rc = rc0;
+                if constexpr (KEEP) {
+                    if (rc < nrc) item(from0, to0);
+                    rc += rcs;
+                } else {
+                    asm volatile("" : "+s"(rc));  // (worked out here, for each slice)
                 }
+                for (; rc < nrc; rc += rcs) item(from_line(rc), to_group(rc));
             }
             }
         }
