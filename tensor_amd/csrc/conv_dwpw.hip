@@ -11,6 +11,11 @@
 //    strides, padding and dilation are in the lanes' addresses.) A tap of a pixel is an 8-byte load; one outside the image is out of
 //    range and zero. The weights come as one byte per lane and tap and are spread out by v_perm_b32: as whole operands they would be as
 //    many bytes as the pixels.
+//  * Where the depthwise layer keeps the image's sides, a workgroup may copy the run of pixels that its windows touch into LDS first (plan + 32,
+//    DwPwStage), with the weights: a tap is then an LDS read, and the address unit, which takes some 28 cycles for every 8-byte load of
+//    scattered pixels, sees a 16-byte copy for two pixels once. What that gives grows with the taps (5x5 128 -> 128 -> 128 @52x52 b16 21.0 -> 18.9
+//    us, 88 -> 88 -> 88 @52x52 with a shuffle 15.6 -> 15.3); with wide rows and small tiles the run is several times the tile, and the plan without it stays
+//    (32 -> 16 @112x112 b64 52.8, 56.9). The copies go straight to LDS: through registers, with an exposed latency for each batch of them, it was slower.
 //  * The bytes go to LDS, a row per pixel, and the pointwise layer's waves take its pairs of 16-row tiles in turn, weights straight
 //    from memory in a ring of four reduction steps that is refilled across pairs and layers: the first ones are requested before the
 //    depthwise layer begins, as are the elements of a residual or of a shuffle's other blob.
@@ -45,6 +50,8 @@ struct DwPwArgs {
     unsigned hw_s, ow_s;
     int lg, dw_lrelu, dw_nonneg;     // lg: log2 of the pixel groups
     unsigned first_pack;             // channels of an element of a shuffle's first half
+    DwPwStage st;                    // the pixels that a workgroup stages, st.pitch 0: none
+    unsigned between;                // bytes of LDS between the first layer's pixels and the constants
 };
 
 // the fp32 blob whose elements an epilogue reads
@@ -53,6 +60,10 @@ __device__ __forceinline__ const float* add_blob(const A& ja) {
     if constexpr (std::is_same_v<A, PwShuffle>) return ja.other;
     else if constexpr (std::is_same_v<A, NoJoin>) return nullptr;
     else return ja.residual;
+}
+// 16 bytes a lane from a buffer to `to` (the same for the wave) and on in LDS, in the lanes' order; out of range: zeros
+__device__ __forceinline__ void copy16(__amdgpu_buffer_rsrc_t r, int8_t* to, unsigned v, unsigned s) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)to, 16, (int)v, (int)s, 0, 0);
 }
 template <class A>
 __device__ __forceinline__ unsigned sh_image(const A& ja) {
@@ -105,9 +116,9 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
     const unsigned HW = pa.HW, C8 = pa.C8, K0 = l0.K, rb0 = 64u * l0.steps + 16u, rb1 = NEXT ? 64u * l1.steps + 16u : 0u;  // bytes of a pixel's row
     const int pairs0 = (l0.K + 31) / 32, pairs1 = NEXT ? (l1.K + 31) / 32 : 0;
     const int PIX = 16 << pa.lg, group = wave & ((1 << pa.lg) - 1), first = wave >> pa.lg, stride = NW >> pa.lg;
-    int8_t *const px0 = lds, *const px1 = lds + PIX * rb0;
+    int8_t *const px0 = lds, *const px1 = lds + PIX * rb0, *const staged = px1;  // (staged: until the depthwise layer ends)
     const unsigned Cd = 16u * ((C8 + 1) / 2);  // channels of the depthwise layer, whole pairs of octets
-    float *const constsd = reinterpret_cast<float*>(px1 + PIX * rb1), *const consts0 = constsd + 2 * Cd, *const consts1 = consts0 + 64 * pairs0;
+    float *const constsd = reinterpret_cast<float*>(px1 + pa.between), *const consts0 = constsd + 2 * Cd, *const consts1 = consts0 + 64 * pairs0;
 
     // ---- the wave's pixels -----------------------------------------------------------------------------------------------------
     const unsigned gp = (unsigned)(tile * PIX + 16 * group) + p;
@@ -168,7 +179,12 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
         const unsigned HWi = (unsigned)(pa.H * pa.W), second = q & 1;  // second: of the two pairs of taps in a reduction step
         const unsigned oy = div_by(pix, FastDiv{pa.ow_m, pa.ow_s, (unsigned)pa.OW}), ox = pix - oy * pa.OW;
         const int y0 = (int)oy * pa.sh - pa.ph, x0 = (int)ox * pa.sw - pa.pw;
-        const int base = (int)((n * C8 + (q >> 1)) * HWi) + y0 * pa.W + x0;
+        // a tap's place in units of 8 bytes: in the blob, or among the staged pixels (one outside the image: the zeros behind them)
+        const bool st = pa.st.pitch != 0;  // (uniform)
+        const unsigned t_first = (unsigned)(tile * PIX), n_first = div_by(t_first, FastDiv{pa.hw_m, pa.hw_s, HW});
+        const int s_first = dwpw_run(pa.st, HW, t_first, n_first);
+        const int base = st ? (int)((q >> 1) * pa.st.pitch) + dwpw_window(pa.st, n, pix) - s_first : (int)((n * C8 + (q >> 1)) * HWi) + y0 * pa.W + x0;
+        const unsigned none = st ? ((q >> 1) * pa.st.pitch + pa.st.slots) * 8u : PR_OOB;
         // the taps inside the image as bits, shifted to the lane's own
         unsigned columns = 0, taps = 0;
 #pragma unroll
@@ -183,7 +199,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
             for (int e = 0; e < 2; ++e) {
                 const int t0 = 4 * m + e, t1 = t0 + 2;
                 const int at0 = t0 / KS * pa.dh * pa.W + t0 % KS * pa.dw, at1 = t1 / KS * pa.dh * pa.W + t1 % KS * pa.dw;
-                v[m][e] = taps >> t0 & 1 ? (unsigned)(base + (second ? at1 : at0)) * 8u : PR_OOB;
+                v[m][e] = taps >> t0 & 1 ? (unsigned)(base + (second ? at1 : at0)) * 8u : none;
             }
         // channel r = p's bytes in the operand: dword p / 4 of its octet's two pixels, if the lane's bytes are of that octet
         unsigned sel[2][4];
@@ -199,6 +215,11 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
         const __amdgpu_buffer_rsrc_t rin = rsrc(x, pa.in_bytes), rw = rsrc(pa.dw_w, (unsigned)pairs * 256u * PK);
         v4i b[M];
         int w[PK];
+        using Weights = std::conditional_t<PK == 2, v2i, v4i>;
+        auto weights = [&](const Weights& t) {
+#pragma unroll
+            for (int i = 0; i < PK; ++i) w[i] = t[i];
+        };
         auto load = [&](int op) {
             const unsigned s = (unsigned)op * 16u * HWi;
 #pragma unroll
@@ -206,37 +227,51 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
                 const v2i lo = load8(rin, v[m][0], s), hi = 4 * m + 1 < TAPS ? load8(rin, v[m][1], s) : v2i{0, 0};
                 b[m] = v4i{lo[0], lo[1], hi[0], hi[1]};
             }
-            if constexpr (PK == 2) {
-                const v2i t = load8(rw, lane * 8, (unsigned)op * 512u);
-                w[0] = t[0], w[1] = t[1];
-            } else {
-                const v4i t = load16(rw, lane * 16, (unsigned)op * 1024u);
-#pragma unroll
-                for (int i = 0; i < PK; ++i) w[i] = t[i];
-            }
+            if constexpr (PK == 2) weights(load8(rw, lane * 8, (unsigned)op * 512u));
+            else weights(load16(rw, lane * 16, (unsigned)op * 1024u));
         };
-        load(min(first, pairs - 1));
+        int8_t* const staged_w = staged + pa.st.octets * pa.st.pitch * 8u;
+        auto load_staged = [&](int op) {
+            const int8_t* const from = staged + (unsigned)op * 16u * pa.st.pitch;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const v2i lo = *reinterpret_cast<const v2i*>(from + v[m][0]), hi = 4 * m + 1 < TAPS ? *reinterpret_cast<const v2i*>(from + v[m][1]) : v2i{0, 0};
+                b[m] = v4i{lo[0], lo[1], hi[0], hi[1]};
+            }
+            weights(*reinterpret_cast<const Weights*>(staged_w + (op * 64 + (int)lane) * 4 * PK));
+        };
+
+        if (st) {
+            // ---- the pixels that the tile's windows touch, octet by octet, and the weights into LDS: two pixels a lane -------------------------
+            const unsigned lg = pa.st.lg_lanes, unit = lane & ((1u << lg) - 1), sub = lane >> lg, sets = 64u >> lg;  // sets: octets of a copy
+            for (unsigned c = 0; c < pa.st.units; c += 64) {
+                const int at = s_first + 2 * (int)(c + unit);
+                const unsigned im = div_by((unsigned)at, FastDiv{pa.st.image_m, pa.st.image_s, pa.st.image});
+                const bool in = at >= 0 && 2 * (c + unit) < pa.st.slots && im * HW < pa.total_pix;
+                const unsigned from = in ? dwpw_copied(pa.st, HW, C8, im, sub, (unsigned)at) : PR_OOB;
+                if (c + unit < pa.st.units)
+                    for (unsigned o = wave * sets; o < C8; o += NW * sets) copy16(rin, staged + (o * pa.st.pitch + 2 * c) * 8, from, o * HW * 8u);
+            }
+            for (unsigned i = wave; i < ((unsigned)pairs * PK + 3) / 4; i += NW) copy16(rw, staged_w + i * 1024, lane * 16, i * 1024);
+        } else {
+            load(min(first, pairs - 1));
+        }
         asm volatile("" ::: "memory");  // (in front of the others: the compiler would move them to the loop)
 
         // ---- constants into LDS: scale_in and bias of each layer (they are padded to whole pairs of tiles and more) ---------------------
-        // (an array a wave: six of them)
+        // (an array a wave: six of them. Copied without registers, so that one wait covers them and what was requested before: 88 @52x52 16.6 ->
+        // 15.6 us, 5x5 128 @26x26 8.8 -> 8.6)
         for (int w = wave; w < (NEXT ? 6 : 4); w += NW) {
             const unsigned d = w >> 1;  // 0: the depthwise layer, 1, 2: the others
             const float* const si = d == 0 ? pa.dw_scale_in : d == 1 ? l0.scale_in : l1.scale_in;
             const float* const bi = d == 0 ? pa.dw_bias : d == 1 ? l0.bias : l1.bias;
             const unsigned quads = d == 0 ? Cd / 4 : 8u * (d == 1 ? pairs0 : pairs1);
             const __amdgpu_buffer_rsrc_t r = rsrc(w & 1 ? bi : si, quads * 16u);
-            v4i* const to = reinterpret_cast<v4i*>(d == 0 ? constsd : d == 1 ? consts0 : consts1) + (w & 1 ? quads : 0u);
-            for (unsigned i0 = 0; i0 < quads; i0 += 256) {
-                v4i c[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k == 0 || i0 + 64 * k < quads) c[k] = load16(r, lane * 16 + k * 1024, i0 * 16);  // (uniform)
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (i0 + 64 * k + lane < quads) to[i0 + 64 * k + lane] = c[k];
-            }
+            int8_t* const to = reinterpret_cast<int8_t*>(d == 0 ? constsd : d == 1 ? consts0 : consts1) + (w & 1 ? quads * 16u : 0u);
+            for (unsigned i = 0; i < quads; i += 64)
+                if (i + lane < quads) copy16(r, to + i * 16, lane * 16, i * 16);
         }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's copies have arrived
         __syncthreads();
 
         // ---- what comes behind the depthwise layer, requested now: weights, elements of another blob --------------------------------------
@@ -248,6 +283,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
         Epilogue epd{};
         epd.act_p0 = pa.dw_p0, epd.lrelu = pa.dw_lrelu != 0;
         const ohip_v2s top = __builtin_bit_cast(ohip_v2s, pa.dw_qh), bottom = __builtin_bit_cast(ohip_v2s, pa.dw_nonneg ? 0u : 0xff81ff81u);
+        auto walk = [&](auto load) {
         for (int op = first; op < pairs;) {
             v4i acc = {0, 0, 0, 0};
 #pragma unroll
@@ -281,6 +317,13 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
                 bytes = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
             }
             if (2u * now + (q >> 1) < C8) *reinterpret_cast<unsigned*>(px0 + row0 + 16 * now + 4 * q) = bytes;
+        }
+        };
+        if (st) {
+            load_staged(min(first, pairs - 1));
+            walk(load_staged);
+        } else {
+            walk(load);
         }
     }
     __syncthreads();
@@ -418,10 +461,21 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
 // host side
 // ---------------------------------------------------------------------------------------------------------------------------------
 
-static size_t dwpw_lds_bytes(const ConvGeom& g0, const ConvGeom* g1, int groups) {
-    const size_t rows = 64 * (size_t)igemm_channel_groups(g0.C) + 16 + (g1 ? 64 * (size_t)igemm_channel_groups(g1->C) + 16 : 0);
-    return 16 * (size_t)groups * rows + 256 * (size_t)((g0.K + 31) / 32 + (g1 ? (g1->K + 31) / 32 : 0)) +
-           128 * (size_t)((g0.C / 8 + 1) / 2);
+// the staged pixels and weights make room for the second layer's pixels
+static size_t dwpw_between(const ConvGeom& gd, const ConvGeom* g1, int groups, const DwPwStage& st) {
+    const size_t weights = (dwpw_weight_bytes(gd.C, gd.kh) + 1023) / 1024 * 1024;
+    return std::max(g1 ? 16 * (size_t)groups * (64 * (size_t)igemm_channel_groups(g1->C) + 16) : 0, st.pitch ? 8 * (size_t)st.octets * st.pitch + weights : 0);
+}
+static size_t dwpw_lds_bytes(const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1, int groups, const DwPwStage& st) {
+    return 16 * (size_t)groups * (64 * (size_t)igemm_channel_groups(g0.C) + 16) + dwpw_between(gd, g1, groups, st) +
+           256 * (size_t)((g0.K + 31) / 32 + (g1 ? (g1->K + 31) / 32 : 0)) + 128 * (size_t)((g0.C / 8 + 1) / 2);
+}
+static DwPwStage dwpw_staged(const ConvGeom& gd, int groups) {
+    if (gd.sh != 1 || gd.sw != 1 || gd.OH != gd.H || gd.OW != gd.W) return {};
+    DwPwStage st = dwpw_stage(gd.C, gd.H, gd.W, gd.kh, gd.ph, gd.pw, gd.dh, gd.dw, 16 * groups);
+    const FastDiv f = fast_div(st.image);
+    st.image_m = f.m, st.image_s = f.s;
+    return st;
 }
 
 bool dwpw_front_applicable(const ConvGeom& gd, const Epilogue& ed) {
@@ -436,7 +490,7 @@ bool dwpw_front_applicable(const ConvGeom& gd, const Epilogue& ed) {
 
 bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, const Epilogue* e1) {
     if (!dwpw_front_applicable(gd, ed) || !pwpw_pointwise(g0) || g0.C != gd.K || g0.N != gd.N || g0.H != gd.OH || g0.W != gd.OW || g0.N < 1) return false;
-    if (dwpw_lds_bytes(g0, g1, 1) > 65536) return false;
+    if (dwpw_lds_bytes(gd, g0, g1, 1, DwPwStage{}) > 65536) return false;
     const int k0 = pwpw_kind(e0, g0.K);
     const bool shuffle = e0.join && e0.join->other, parts = e0.join && !shuffle;
     if (k0 != PP_I8 && k0 != PP_F32) return false;
@@ -459,11 +513,11 @@ bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom
     return true;
 }
 
-// Cost models in us, fitted to launches replayed from captured graphs behind a copy that leaves the L2 caches cold, over 2500 drawn layers
-// (16 to 960 channels, 4x4 to 112x112 pixels, batches of 1 to 64, every end): half of them within 6 %, nine in ten within 15 %, and so are
-// both models over 2500 others. The launch:
+// Cost models in us, fitted to launches replayed from captured graphs behind a copy that leaves the L2 caches cold, over 7000 drawn layers
+// (16 to 720 channels, 5x5 to 112x112 pixels, batches of 1 to 64, every end) and every plan of them: half of the times within 4 %, nine in ten within
+// 12 %, and so over 2300 other layers; the plan that they choose takes 1.017 of the fastest one's time there. The launch:
 // a wave walks nd pairs of octets and n0 and n1 pairs of row tiles one behind the other, once if every workgroup is resident, and the more
-// often the more of eight waves there are for a compute unit.
+// often the more waves there are for a compute unit than it holds; with staged pixels it issues its share of the copies in front of that.
 struct DwPwShape {
     double px;  // output pixels
     int pairs_d, pairs[2], steps[2];
@@ -473,51 +527,60 @@ struct DwPwShape {
           pairs{(g0.K + 31) / 32, g1 ? (g1->K + 31) / 32 : 0}, steps{igemm_channel_groups(g0.C), g1 ? igemm_channel_groups(g1->C) : 0},
           k5(gd.kh == 5), f32(e0.out_kind == OTTER_HIP_OUT_F32), adds(e0.residual || e0.join) {}
 };
-static double dwpw_cost(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1, int waves, int groups) {
-    static const double once[2][9] = {{3.20, 0.391, 0.720, 0.351, 0.100, 0.497, 0.070, 0.173, 0.140}, {3.08, 0.432, 0.859, 0.421, 0.114, 0.563, 0.098, 0.244, 0.157}};
-    static const double more[2][9] = {{0.736, 0.222, 0.732, 0, 0.132, 0.279, 0.068, 0, 0}, {0.874, 0.266, 0.719, 0, 0.115, 0.315, 0.061, 0, 0}};
-    const int w = waves == 8, stride = waves / groups, nd = (s.pairs_d + stride - 1) / stride;
+static double dwpw_cost(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1, int waves, int groups, const DwPwStage& st, size_t lds) {
+    static const struct {
+        double once[10], more[10], byte, mac, wide;  // for 10^6 bytes, 10^9 multiply-adds of the pointwise layers, 10^6 values past the 256th channel
+    } table[4] = {  // four and eight waves, without and with staged pixels
+        {{3.11, 0.394, 0.726, 0.319, 0.082, 0.438, 0.0434, 0.166, 0.26}, {0.637, 0.334, 1.12, 0.408, 0.00861, 0.347, 0, 0, 0}, 0.11, 0.878, 0.081},
+        {{3.12, 0.416, 0.885, 0.46, 0.104, 0.563, 0.0802, 0.177, 0.24}, {0.702, 0.283, 1.5, 0.309, 0.0625, 0.344, 0, 0.0807, 0.00366}, 0.105, 0.69, 0},
+        {{3.38, 0.161, 0.305, 0.359, 0.0646, 0.445, 0.0341, 0.16, 0.218, 0.1}, {1.02, 0.226, 0.92, 0.186, 0.0325, 0.328, 0, 0, 0, 0.00464}, 0.12, 1.14, 1.44},
+        {{3.12, 0.267, 0.474, 0.552, 0.0722, 0.597, 0.0785, 0.154, 0.192, 0.139}, {0.945, 0.174, 1.37, 0.283, 0.0383, 0.365, 0, 0.00306, 0, 0.03}, 0.114, 0.558, 0.558}};
+    const int stride = waves / groups, nd = (s.pairs_d + stride - 1) / stride;
+    const auto& k = table[(st.pitch ? 2 : 0) + (waves == 8)];
     const double n0 = (s.pairs[0] + stride - 1) / stride, n1 = (s.pairs[1] + stride - 1) / stride;
-    const double f[9] = {1, s.k5 ? 0. : nd, s.k5 ? (double)nd : 0, n0, n0 * s.steps[0], n1, n1 * s.steps[1], s.f32 ? n0 : 0, s.adds ? n0 : 0};
-    const double rounds = std::max(0., s.px / (16 * groups) * waves / 2048 - 1);
+    const double copies = st.pitch ? (double)((st.units + 63) / 64) * ((gd.C / 8 + (64 >> st.lg_lanes) - 1) >> (6 - st.lg_lanes)) / waves : 0.;
+    const double f[10] = {1, s.k5 ? 0. : nd, s.k5 ? (double)nd : 0, n0, n0 * s.steps[0], n1, n1 * s.steps[1], s.f32 ? n0 : 0, s.adds ? n0 : 0, copies};
+    const double held = st.pitch ? std::min(8., (double)waves * (163840 / lds)) : 8.;
+    const double rounds = std::max(0., s.px / (16 * groups) * waves / (256 * held) - 1);
     double t = 0;
-    for (int i = 0; i < 9; ++i) t += f[i] * (once[w][i] + rounds * more[w][i]);
-    const double bytes = s.px * ((double)gd.C * gd.sh * gd.sw + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (g1 ? g1->K : 0));
-    return t + 0.134e-6 * bytes;
+    for (int i = 0; i < 10; ++i) t += f[i] * (k.once[i] + rounds * k.more[i]);
+    const double mb = 1e-6 * s.px * ((double)gd.C * gd.sh * gd.sw + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (g1 ? g1->K : 0));
+    return t + k.byte * mb + 1e-9 * s.px * g0.K * (gd.C + (g1 ? g1->K : 0.)) * k.mac + 1e-6 * s.px * std::max(0, gd.C - 256) * k.wide;
 }
 // the layers by themselves, the pointwise ones as a pair where that is a launch
 static double dwpw_cost_apart(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1) {
     const double mbd = 1e-6 * s.px * gd.C * (gd.sh * gd.sw + 1.);
     const double mb0 = 1e-6 * s.px * (gd.C + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (s.f32 ? g0.K : 0));
-    double t = 4.94 + (0.255 + (s.k5 ? 0.025 : 0)) * mbd + 0.178 * mb0 + 1.745e-9 * s.px * g0.C * g0.K + 0.879e-3 * gd.C + 0.671e-3 * g0.K +
-               (gd.C > 256 ? 0.059e-6 * s.px * gd.C : 0);
-    if (g1) t += 1.92 + 0.346e-6 * s.px * ((double)g0.K + g1->K) + 1.206e-9 * s.px * g0.K * g1->K + 1.054e-3 * g1->K + (g0.K > 256 ? 0.76 : 0);
+    double t = 4.86 + (0.299 + (s.k5 ? 0.051 : 0)) * mbd + 0.173 * mb0 + 2.396e-9 * s.px * g0.C * g0.K + 1.193e-3 * gd.C + 0.213e-3 * g0.K;
+    if (g1) t += 1.91 + 0.379e-6 * s.px * ((double)g0.K + g1->K) + 1.007e-9 * s.px * g0.K * g1->K + 1.519e-3 * g1->K + (g0.K > 256 ? 0.54 : 0);
     return t;
 }
 
 // Groups of 16 pixels for a workgroup, + 16 for one of four waves: those have fewer idle waves where there are many pixels and few
-// channels (88 -> 88 -> 88 @52x52 b16 with a shuffle: eight waves and four groups 17.9 us, four and four 16.4), eight a shorter chain.
-static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, double* cost) {
+// channels (88 -> 88 -> 88 @52x52 b16 with a shuffle: eight waves and four groups 17.6 us, four and four 15.6), eight a shorter chain;
+// + 32 with staged pixels (15.3): not where the input's address is no multiple of their eight bytes.
+static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, bool aligned, double* cost) {
     const DwPwShape s(gd, g0, e0, g1);
     int best = 0;
     for (int waves = 8; waves >= 4; waves -= 4)
-        for (int g = 1; g <= waves; g *= 2) {
-            if (dwpw_lds_bytes(g0, g1, g) > 65536) break;
-            const double c = dwpw_cost(s, gd, g0, g1, waves, g);
-            if (!best || c < *cost) best = g + (waves == 4 ? 16 : 0), *cost = c;
-        }
+        for (int g = 1; g <= waves; g *= 2)
+            for (int staged = 0; staged <= (aligned ? 1 : 0); ++staged) {
+                const DwPwStage st = staged ? dwpw_staged(gd, g) : DwPwStage{};
+                const size_t lds = dwpw_lds_bytes(gd, g0, g1, g, st);
+                if (lds > 65536 || (staged && !st.pitch)) continue;
+                const double c = dwpw_cost(s, gd, g0, g1, waves, g, st, lds);
+                if (!best || c < *cost) best = g + (waves == 4 ? 16 : 0) + 32 * staged, *cost = c;
+            }
     return best;
 }
-// Over 2500 layers drawn anew the rule takes 61 % and gives 0.89 of the time; 20 of them are over 5 % slower than apart, the worst 1.27. Five
-// taps a row are where the launch's loads cost most: nearer to the line it loses. So it does with 640 channels and more on many pixels,
-// where every workgroup of 32 pixels streams 0.4 MB of weights and up and its LDS leaves few of them on a compute unit: between 0.84 and 0.92 of
-// the models' time apart it took 0.98 of the real one, up to 1.50 (664 -> 664 -> 32 @49x49, 7 images: 41.9 us apart, 62.7).
+// Over 2330 layers beside the fit the rule takes 67 % and gives 0.88 of the time (the faster of both each time: 0.868); 42 of them are over 5 %
+// slower than apart, the worst 1.38. Of 88 with 640 channels and more on 4096 pixels and more, where both models are further off, those
+// under 0.75 take 0.80 of the time and none is slower; 664 -> 664 -> 40 on 17340 pixels, 0.78 by the models, is level.
 bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
     double cost = 0;
-    dwpw_plan(gd, g0, e0, g1, &cost);
+    dwpw_plan(gd, g0, e0, g1, true, &cost);
     const DwPwShape s(gd, g0, e0, g1);
-    const double line = s.k5 ? 0.90 : gd.C >= 640 && s.px >= 4096 ? 0.84 : 0.92;
-    return cost < line * dwpw_cost_apart(s, gd, g0, g1);
+    return cost < (gd.C >= 640 && s.px >= 4096 ? 0.75 : 0.92) * dwpw_cost_apart(s, gd, g0, g1);
 }
 
 template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>
@@ -552,10 +615,13 @@ hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const
     pa.in_bytes = (unsigned)((size_t)gd.N * gd.C * gd.H * gd.W);
     pa.sh = gd.sh, pa.sw = gd.sw, pa.ph = gd.ph, pa.pw = gd.pw, pa.dh = gd.dh, pa.dw = gd.dw, pa.C8 = gd.C / 8;
     double cost = 0;
-    const int plan = force ? force : dwpw_plan(gd, g0, e0, g1, &cost), groups = plan & 15, waves = plan & 16 ? 4 : 8;
+    const int plan = force ? force : dwpw_plan(gd, g0, e0, g1, (uintptr_t)x % 8 == 0, &cost), groups = plan & 15, waves = plan & 16 ? 4 : 8;
     if (groups > waves) return hipErrorInvalidValue;
     if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return hipErrorInvalidValue;
-    const size_t lds = dwpw_lds_bytes(g0, g1, groups);
+    if (plan & 32) pa.st = dwpw_staged(gd, groups);
+    if ((plan & 32) && (!pa.st.pitch || (uintptr_t)x % 8)) return hipErrorInvalidValue;
+    pa.between = (unsigned)dwpw_between(gd, g1, groups, pa.st);
+    const size_t lds = dwpw_lds_bytes(gd, g0, g1, groups, pa.st);
     if (lds > 65536) return hipErrorInvalidValue;
     pa.first_pack = e0.join ? (unsigned)e0.join->sh_pack0 : 8u;
     pa.lg = groups == 1 ? 0 : groups == 2 ? 1 : groups == 4 ? 2 : 3;

@@ -61,3 +61,71 @@ def test_requests_stay_inside_what_they_name(tmp_path):
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", CSRC, str(src), "-o", exe])
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+STAGED = r"""
+#include <cstdio>
+#include <initializer_list>
+#include <vector>
+#include "dwpw_requests.hpp"
+using namespace ohip;
+// N images of C channels (octets of 8 bytes), copied into places as the launch copies them; a place holds the number of the blob's element plus one
+int main() {
+    struct Case { int ks, pad, dil, C, N, H, W; };
+    for (const Case& c : {Case{3, 1, 1, 88, 3, 13, 13}, {3, 1, 1, 16, 5, 7, 7}, {5, 2, 1, 24, 2, 9, 26}, {3, 1, 1, 8, 9, 1, 1}, {3, 2, 2, 40, 2, 12, 9}, {5, 2, 1, 128, 2, 52, 52},
+                          {3, 1, 1, 72, 4, 3, 5}, {3, 1, 1, 32, 2, 4, 112}, {5, 4, 2, 8, 3, 6, 3}, {3, 1, 1, 136, 1, 14, 14}})
+        for (int pixels : {16, 32, 64, 128}) {
+            const DwPwStage st = dwpw_stage(c.C, c.H, c.W, c.ks, c.pad, c.pad, c.dil, c.dil, pixels);
+            const unsigned HW = c.H * c.W, C8 = c.C / 8, total = c.N * HW, sets = 64u >> st.lg_lanes;
+            const size_t elements = (size_t)total * C8, places = (size_t)st.octets * st.pitch;
+            if (st.octets < (C8 + 1) / 2 * 2 || st.slots + 2 > st.pitch) return std::printf("room\n"), 1;
+            for (unsigned first = 0; first < total; first += pixels) {
+                const unsigned n_first = first / HW;
+                const int begin = dwpw_run(st, HW, first, n_first);
+                std::vector<size_t> lds(places, ~(size_t)0);
+                for (unsigned from = 0; from < st.units; from += 64)
+                    for (unsigned o = 0; o < C8; o += sets)
+                        for (unsigned lane = 0; lane < 64; ++lane) {
+                            const unsigned unit = lane & ((1u << st.lg_lanes) - 1), sub = lane >> st.lg_lanes;
+                            if (from + unit >= st.units) continue;
+                            const int at = begin + 2 * (int)(from + unit);
+                            const unsigned im = (unsigned)at / st.image;
+                            const bool in = at >= 0 && 2 * (from + unit) < st.slots && im * HW < total;
+                            const size_t place = (size_t)o * st.pitch + 2 * from + 2 * lane;
+                            if (place + 2 > places) return std::printf("a copy beyond its room\n"), 1;
+                            for (int e = 0; e < 2; ++e) {
+                                const size_t element = in ? ((size_t)dwpw_copied(st, HW, C8, im, sub, (unsigned)at) + (size_t)o * HW * 8) / 8 + e : elements;
+                                lds[place + e] = element < elements ? element + 1 : 0;
+                            }
+                        }
+                for (unsigned p = 0; p < (unsigned)pixels && first + p < total; ++p) {
+                    const unsigned n = (first + p) / HW, pix = first + p - n * HW;
+                    const int y = pix / c.W, x = pix % c.W, window = dwpw_window(st, n, pix) - begin;
+                    for (unsigned o = 0; o < C8; ++o) {
+                        if (lds[(size_t)o * st.pitch + st.slots] != 0) return std::printf("no zeros behind the pixels\n"), 1;
+                        for (int dy = 0; dy < c.ks; ++dy)
+                            for (int dx = 0; dx < c.ks; ++dx) {
+                                const int iy = y - c.pad + dy * c.dil, ix = x - c.pad + dx * c.dil;
+                                if (iy < 0 || iy >= c.H || ix < 0 || ix >= c.W) continue;
+                                const int slot = window + dy * c.dil * c.W + dx * c.dil;
+                                if (slot < 0 || slot >= (int)st.slots) return std::printf("a tap beyond the run\n"), 1;
+                                if (lds[(size_t)o * st.pitch + slot] != ((size_t)n * C8 + o) * HW + iy * c.W + ix + 1)
+                                    return std::printf("another pixel: %dx%d k%d, %d pixels, octet %u\n", c.H, c.W, c.ks, pixels, o), 1;
+                            }
+                    }
+                }
+            }
+        }
+    return 0;
+}
+"""
+
+
+def test_staged_pixels_are_those_of_the_windows(tmp_path):
+    """Every tap inside the image finds its pixel among the places that a tile's copies fill (image sides whose product is odd and even, images of
+    one pixel, tiles over several images, dilation), one outside it zeros, and no copy leaves its room."""
+    src, exe = tmp_path / "dwpw_stage.cpp", str(tmp_path / "dwpw_stage")
+    src.write_text(STAGED)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", CSRC, str(src), "-o", exe])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout

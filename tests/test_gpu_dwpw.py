@@ -133,6 +133,57 @@ def test_one_launch_equals_the_layers(hip, C, k, stride, pad, dil, act, K, K2, n
             pw.close()
 
 
+@pytest.mark.parametrize("C,k,pad,dil,act,K,K2,N,H,W", [
+    (88, 3, 1, 1, 0, 88, 88, 3, 13, 13),     # an odd count of octets, images of an odd count of pixels that begin inside a tile
+    (16, 3, 1, 1, 3, 24, 16, 9, 3, 3),       # several images in a tile, octets that share a copy
+    (8, 3, 1, 1, 2, 8, 8, 21, 1, 1),         # one pixel an image
+    (72, 3, 2, 2, 2, 40, 24, 2, 12, 9),      # dilation
+    (32, 3, 1, 1, 3, 16, 96, 1, 7, 112),     # an octet takes several copies
+    (256, 3, 1, 1, 1, 64, 128, 1, 14, 14),
+    (128, 5, 2, 1, 2, 128, 112, 2, 13, 13),
+    (40, 5, 2, 1, 0, 24, 8, 1, 26, 40),
+    (24, 5, 4, 2, 3, 24, 8, 3, 5, 7),
+])
+def test_staged_pixels(hip, C, k, pad, dil, act, K, K2, N, H, W):
+    """The plans (+ 32) that copy the windows' pixels into LDS first."""
+    rng = np.random.default_rng(C + K + W)
+    x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
+    dw = depthwise(hip, rng, C, k, 1, pad, dil, act)
+    ran = 0
+    for last in (None, "nonneg"):
+        nx = layer(hip, rng, K, K2, 3, False) if last else None
+        for form, how in forms(k, last):
+            pw = layer(hip, rng, C, K, 2 if form != "sum" else 0, form != "i8")
+            for plan in (33, 34, 36, 40, 49, 50, 52):
+                dw.force = (-12, plan)
+                dw.set_tile(-12, plan)
+                try:
+                    got, want = one_and_two(hip, rng, form, how, dw, pw, nx, x, N, H, W)
+                except capi.HipError:  # (more LDS than a launch has)
+                    assert plan > 34
+                    continue
+                ran += 1
+                for i, (g, v) in enumerate(zip(got, want)):
+                    assert hip.torch.equal(g, v), (last, form, how, plan, i)
+    assert ran
+
+
+def test_a_blob_at_an_odd_address(hip):
+    """An input that is not on eight bytes is not copied in pairs of pixels: refused where that is forced, another plan otherwise."""
+    rng = np.random.default_rng(9)
+    n, C, side = 2, 88, 13
+    values = rng.integers(-127, 128, n * C * side * side).astype(np.int8)
+    dw, pw = depthwise(hip, rng, C, 3, 1, 1, 1, 0), layer(hip, rng, C, 88, 2, False)
+    base = hip.empty(values.size + 16, np.int8)
+    base[4:4 + values.size] = hip.to_device(values)
+    dw.set_tile(-12, 0)
+    want = hip.conv_dwpw(dw, pw, hip.to_device(values), n, side, side)
+    assert hip.torch.equal(hip.conv_dwpw(dw, pw, base[4:4 + values.size], n, side, side), want)
+    dw.set_tile(-12, 34)
+    with pytest.raises(capi.HipError):
+        hip.conv_dwpw(dw, pw, base[4:4 + values.size], n, side, side)
+
+
 @pytest.mark.parametrize("C,k,stride,K,K2,n,side,form,ratio", [
     # drawn layers, the launch's time over that of the layers one by one where the rule was measured
     (32, 3, 1, 32, 32, 6, 88, "shuffle", 0.60), (72, 3, 1, 72, 24, 9, 13, "sum", 0.61), (48, 3, 1, 16, 96, 7, 19, "f32", 0.62),
