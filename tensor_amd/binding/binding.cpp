@@ -144,7 +144,7 @@ PyObject* conv_forward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         rc = ws ? otter_hip_conv_forward(h, px, in_layout, n, ih, iw, po, out_layout, pw, wb, stream)
                 : otter_hip_conv_forward_making(h, px, in_layout, n, ih, iw, po, out_layout, Workspace::make, &made_ws, stream);
         Py_END_ALLOW_THREADS
-        if (!made_ws.error.empty()) throw std::runtime_error(made_ws.error);
+        if (rc && !made_ws.error.empty()) throw std::runtime_error(made_ws.error);
         if (rc) return raise_status(rc);
         return result(a[8], *out);
     } catch (const std::exception& e) {

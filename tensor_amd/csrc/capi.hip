@@ -831,6 +831,23 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
     return *config = tap_tile, best < other ? ALT_TAP : ALT_NONE;
 }
 
+// A pointwise layer on an fp32 blob that one of the two launches above would take, as a quantize pass in front of the launch with its operands
+// in registers (conv_pw_reg.hip): those quantize a value once for every row tile or hold all of a pixel's values, which many channels on many
+// pixels make dear. us as one launch / as two: 752 -> 352 @40x40 b22 97 / 43, 616 -> 328 @109x112 b2 63 / 30, 360 -> 344 @31x31 b43 63 / 37; but
+// 256 -> 512 @28x28 b32 17.0 / 18.3 and 96 -> 576 @14x14 b4 5.1 / 7.4. The two launches' model is fitted to 4700 drawn layers replayed from graphs (half within
+// 3 %, nine in ten within 8 %), against the family's own, which is a third too kind to the implicit-GEMM launch. Over 1060 others of that family
+// the rule takes 16 % and gives 0.964 of all layers' time (the faster of both each time: 0.954), 15 over 3 % slower, the worst 1.30; over 200 of the
+// other 0.98 (0.966) and none. Without room for the int8 blob it is one launch.
+static bool pw_quantized_apart(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, int family) {
+    if (h->force_tm != 0 || !h->so_same || !conv_pw_reg_applicable(g, ep)) return false;
+    const float px = (float)g.N * g.H * g.W * 1e-6f, C = (float)g.C, K = (float)g.K;
+    if (px * C < 2.f) return false;  // (of fewer values one launch is the host's time already)
+    const int ob = layout_elem_bytes(ep.out_layout);
+    const float apart = 5.80f + 0.785f * px * C + 0.142f * px * K * ob + 0.0967f * px * igemm_channel_groups(g.C) * (float)((g.K + 31) / 32 * 32) +
+                        1.95e-3f * C + 0.45e-3f * K + 0.1f * px * K;
+    return apart < (family == 1 ? 1.05f : 1.f) * conv_family_cost(g, family, true, ob, __builtin_inff());
+}
+
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* h, int in_layout, int n, int in_h, int in_w, int out_layout) {
     if (!h || !valid_layout(in_layout)) return fail(OTTER_HIP_ERR_INVALID, "otter_hip_conv_kernel_kind: bad argument");
     int l = in_layout;
@@ -891,7 +908,7 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
                         otter_hip_workspace_fn make_workspace = nullptr, void* make_ctx = nullptr) {
     // the caller's workspace, or one that it makes now: most launches on an fp32 blob quantize for themselves and need none
     auto workspace_of = [&](size_t need) {
-        if (make_workspace && need) workspace = make_workspace(make_ctx, need), workspace_bytes = workspace ? need : 0;
+        if (make_workspace && need && (!workspace || workspace_bytes < need)) workspace = make_workspace(make_ctx, need), workspace_bytes = workspace ? need : 0;
         return workspace && workspace_bytes >= need;
     };
 
@@ -978,12 +995,14 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
     // A pointwise layer on an fp32 Float8 blob: quantize_to_int8 inside the convolution's launch.
     {
         Epilogue ep = make_epilogue(h, out_layout);
-        if (!twin && !residual && use_pw_f32in(h, in_layout, g, ep)) {
+        const bool alone = !twin && !residual, own6 = alone && use_pw_f32in(h, in_layout, g, ep), own1 = !own6 && use_igemm_f32in(h, in_layout, g, ep);
+        if (alone && (own6 || own1) && pw_quantized_apart(h, g, ep, own6 ? 6 : 1) && workspace_of((size_t)n * g.C * in_h * in_w)) {
+            // as two launches, below
+        } else if (own6) {
             OHIP_CHECK(run_conv_pw_f32in((const float*)in, h->w_igemm, h->clamp_hi, out, g, ep, h->in_scale, d.in_round_mode,
                                          h->force_tm == -7 ? (h->force_tn & 7) : 0, h->force_tm == -7 ? (h->force_tn >> 3) : 0, stream));
             return OTTER_HIP_OK;
-        }
-        if (use_igemm_f32in(h, in_layout, g, ep)) {
+        } else if (own1) {
             if ((twin || residual) && (!twin || g.K % 8 == 0) && pick_epilogue(ep, g.K) == EPI_F32_P4) {
                 ep.twin = twin, ep.twin_scale = twin_scale;
                 ep.twin_half = twin_round == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;

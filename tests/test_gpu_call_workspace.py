@@ -34,3 +34,29 @@ def test_workspace_only_where_used(hip, C, K, k, hw, tile, made):
     assert hip.torch.equal(got.view(hip.torch.int32), want.view(hip.torch.int32))
     assert count == made
     conv.close()
+
+
+@pytest.mark.parametrize("C,K,n,h,w,kind,act,made", [
+    (520, 264, 3, 37, 53, capi.OUT_I8, 3, 2),    # an odd count of pixels, channels that fill neither tile
+    (1016, 520, 2, 40, 41, capi.OUT_F32, 2, 2),
+    (264, 960, 5, 81, 77, capi.OUT_I8, 0, 2),
+    (256, 1280, 10, 27, 31, capi.OUT_I8, 1, 2),   # from the kernel that reads the blob once
+    (520, 264, 1, 13, 13, capi.OUT_I8, 0, 1),    # few values: one launch
+])
+def test_a_pointwise_layer_on_many_fp32_values(hip, C, K, n, h, w, kind, act, made):
+    """A quantize pass and the launch with its operands in registers, where those are faster and there is room for the int8 blob: the bits of the
+    single launch, which a caller without a workspace still gets."""
+    rng = np.random.default_rng(C + K)
+    conv = hip.conv(wq=rng.integers(-127, 128, (K, C, 1, 1)).astype(np.int8), scale_in=host_scale_in(np.full(K, 60.0, np.float32), 20.0),
+                    bias=rng.normal(0, 1, K).astype(np.float32), in_scale=20.0, act=act, act_p0=0.1, out_kind=kind,
+                    out_scale=[0.07] if kind == capi.OUT_I8 else None)
+    x = hip.to_device((rng.integers(-260, 260, n * C * h * w) / np.float32(40)).astype(np.float32))  # ties and saturated values among them
+    out_layout = capi.I8_P8 if kind == capi.OUT_I8 else capi.F32_P4
+    got, count = _allocations(hip.torch, lambda: conv.forward(x, capi.F32_P8, n, h, w))
+    assert count == made
+    one = hip.torch.empty_like(got)
+    assert hip.lib.otter_hip_conv_forward(conv.h, hip.ptr(x), capi.F32_P8, n, h, w, hip.ptr(one), out_layout, None, 0, hip.stream()) == 0
+    assert hip.torch.equal(got, one)
+    conv.set_tile(-6, 0)
+    assert hip.torch.equal(got, conv.forward(x, capi.F32_P8, n, h, w))
+    conv.close()
