@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
-// The same layer straight from an fp32 blob: quantize_to_int8 (Tensor/ConvolutionLayer.cpp:770-775,
+// The same layer (3x3 or 5x5) straight from an fp32 blob: quantize_to_int8 (Tensor/ConvolutionLayer.cpp:770-775,
 // Tensor/QuantizeX86.cpp:402-490) and the depthwise convolution in ONE launch, for a Float8 input ([N][C/8][H*W][8
 // floats]) of at most 128 columns. As two launches the int8 copy of the blob is written and read back (c1: 103 MB in +
 // 26 MB out + 26 MB back in + 26 MB out); here every fp32 value is read once and nothing but the result is written.
@@ -348,18 +348,18 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
 // columns). Loading a whole pixel per lane instead (two 16-byte loads 32 bytes apart) touches every cache line twice,
 // and the texture addresser, which works per cache line touched, then bounds the kernel: measured 30 us against 24 us.
 // The lane quantizes its four values with the layer's input scale and rounding primitive -- every value once -- and
-// writes the four bytes into the wave's own ring of four LDS lines [pixel + 2][8 B] (pixels -2, -1 and the ones past
+// writes the four bytes into the wave's own ring of four (5x5: eight) LDS lines [pixel + 2][8 B] (pixels -2, -1 and the ones past
 // the row's end are zero: the padding columns). The matrix operand of lane (n, g) for column chunk c -- pixels 64c + 4n -
 // 2 + 2g and + 1 -- is then one aligned 16-byte LDS read per kernel row. LDS instructions of one wave execute in order, so
 // the wave needs no barrier between its lanes' writes and reads. The loads run four input rows ahead of the
 // quantization in a ring of registers; the matrix instructions of a row run under the quantization of the next one, its
 // epilogue follows that. Rows outside the image or past the strip read zero through the buffer descriptor.
-template <int S, int EPI, int NL>
+template <int S, int EPI, int NL, int KS>
 __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* __restrict__ x, const int8_t* __restrict__ wa,
                                                                void* __restrict__ out, ConvGeom g, Epilogue ep,
                                                                const float* __restrict__ in_scale_p, float in_half, DwGrid dg,
                                                                int n_strips, int rps, unsigned in_bytes, unsigned out_bytes) {
-    constexpr int RL = 4, PF = 4;      // LDS lines / register stages per wave
+    constexpr int RL = KS == 3 ? 4 : 8, PF = 4;  // LDS lines / register stages per wave
     constexpr int NCH = (NL + 1) / 2;  // column chunks of 64 pixels (a matrix operand covers 4 x 16 of them)
     const float in_scale = in_scale_p[0];
     constexpr int T = S == 1 ? 2 : 1;  // A sets
@@ -395,12 +395,12 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
     const int oy0 = strip * rps;
     const int nrows = min(rps, g.OH - oy0);
     const int iy0 = oy0 * S - g.ph;
-    const int nq = (nrows - 1) * S + 3;  // input rows this strip reads
+    const int nq = (nrows - 1) * S + KS;  // input rows this strip reads
     // Odd strips walk UP: a strip and its neighbour below then read the rows they share at the same end of their walks
     // (both last, or both first), i.e. at about the same time, and the second reader finds them in the XCD's L2 instead
     // of fetching them from memory again (the strips of a plane run side by side on one XCD). Walking up only mirrors
     // the row indices: input row j of the walk is row iy0 + nq - 1 - j, output row r of the walk is the strip's row
-    // nrows - 1 - r, and kernel row dy meets the line that holds walk row 2 - dy (the weights are loaded mirrored).
+    // nrows - 1 - r, and kernel row dy meets the line that holds walk row KS - 1 - dy (the weights are loaded mirrored).
     const bool up = (strip & 1) != 0;  // wave-uniform
     auto issue = [&](int j, v4i (&dst)[NL]) {  // j: input row of the walk
         const int iy = up ? iy0 + nq - 1 - j : iy0 + j;
@@ -432,13 +432,13 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
         for (int k = 0; k < NL; ++k) *reinterpret_cast<int*>(lds + line * LINE + 16 + 256 * k + 4 * lane) = quant4(src[k]);
     };
 
-    v4i a[3][T];  // a[k]: the kernel row that meets the k-th of an output row's three lines
+    v4i a[KS][T];  // a[k]: the kernel row that meets the k-th of an output row's lines
     {
-        const v4i* ap = reinterpret_cast<const v4i*>(wa) + (size_t)o * 3 * T * 64 + lane;
+        const v4i* ap = reinterpret_cast<const v4i*>(wa) + (size_t)o * KS * T * 64 + lane;
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
+        for (int k = 0; k < KS; ++k)
 #pragma unroll
-            for (int t = 0; t < T; ++t) a[k][t] = ap[((up ? 2 - k : k) * T + t) * 64];
+            for (int t = 0; t < T; ++t) a[k][t] = ap[((up ? KS - 1 - k : k) * T + t) * 64];
     }
     // (requested before any input row: loads return in order, so the wait for these in front of the first matrix
     // instruction -- which sits inside the loop and is executed on every pass -- then never reaches past a row's loads)
@@ -515,24 +515,24 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
             }
         }
     };
-    auto row_mfma = [&](int line0) {  // the three input rows of an output row sit in lines line0, +1, +2 (mod RL)
+    auto row_mfma = [&](int line0) {  // the input rows of an output row sit in lines line0, +1, .. (mod RL)
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            v4i b[3];
+            v4i b[KS];
 #pragma unroll
-            for (int dy = 0; dy < 3; ++dy)
+            for (int dy = 0; dy < KS; ++dy)
                 b[dy] = *reinterpret_cast<const v4i*>(lds + ((line0 + dy) % RL) * LINE + (64 * c + 4 * n + 2 * q) * 8);
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 cur[c][t] = v4i{0, 0, 0, 0};
 #pragma unroll
-                for (int dy = 0; dy < 3; ++dy) cur[c][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[dy][t], b[dy], cur[c][t], 0, 0, 0);
+                for (int dy = 0; dy < KS; ++dy) cur[c][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[dy][t], b[dy], cur[c][t], 0, 0, 0);
             }
         }
     };
 
-    // Input row j of the walk sits in line and register stage j % 4 and completes output row (j - 2) / S when that is
-    // whole. Rows 0..2 (everything up to the first output row) run in front of the loop, so that every pass of the loop
+    // Input row j of the walk sits in line j % RL and register stage j % 4 and completes output row (j - KS + 1) / S when that is
+    // whole. Rows 0..KS - 1 (everything up to the first output row) run in front of the loop, so that every pass of the loop
     // issues the same loads and stores on every path: the waits for a row's loads are counted back from the youngest
     // request, and a path with fewer requests would pull them (and with them the loads in flight) closer.
     // (where the rows in front of the loop have no output row to store yet they issue stores that go nowhere -- an
@@ -552,42 +552,64 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
             }
         }
     };
-    auto input_row = [&](int j, int jj, bool store_prev) {  // jj = j modulo 4; both a compile-time constant at every call
+    auto input_row = [&](int j, int jj, bool store_prev) {  // jj = j modulo 8; both a compile-time constant at every call
         quant_write(jj % RL, ld[jj % PF]);
         issue(j + PF, ld[jj % PF]);
-        if ((jj - 2 + 4) % S == 0) {
-            if (store_prev) epilogue_store((j - 2) / S - 1);
+        if ((jj - (KS - 1) + 8) % S == 0) {
+            if (store_prev) epilogue_store((j - (KS - 1)) / S - 1);
             else no_store(j);
-            row_mfma((jj - 2 + 4) % RL);
+            row_mfma((jj - (KS - 1) + 8) % RL);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    no_store(3);
-    input_row(0, 0, false);
-    input_row(1, 1, false);
-    input_row(2, 2, false);
+    no_store(KS);
+#pragma unroll
+    for (int i = 0; i < KS; ++i) input_row(i, i, false);
     // (eight rows per pass: the waits the compiler places in the first rows of a pass reach a row or two further back
     // than the ring needs, so the passes are long)
     constexpr int UNR = 8;
-    const int steps = (nq - 3) / UNR;
-    int jb = 3;
+    const int steps = (nq - KS) / UNR;
+    int jb = KS;
     for (int st = 0; st < steps; ++st, jb += UNR) {
 #pragma unroll
-        for (int i = 0; i < UNR; ++i) input_row(jb + i, 3 + i, true);
+        for (int i = 0; i < UNR; ++i) input_row(jb + i, KS + i, true);
     }
 #pragma unroll
     for (int i = 0; i < UNR - 1; ++i)
-        if (jb + i < nq) input_row(jb + i, 3 + i, true);  // wave-uniform
+        if (jb + i < nq) input_row(jb + i, KS + i, true);  // wave-uniform
     epilogue_store(nrows - 1);
 }
 
 // true when the fused fp32 -> depthwise launch takes this layer and blob (Float8 input; the caller has checked
 // dw_mfma_applicable)
 bool dw_f32in_applicable(const ConvGeom& g, int in_layout) {
-    if (in_layout != OTTER_HIP_F32_P8 || g.kh != 3 || g.kw != 3) return false;
-    if (g.W > 128 || g.W < 17 || g.C % 8 != 0) return false;
+    if (in_layout != OTTER_HIP_F32_P8) return false;
+    if (g.W > 128 || g.C % 8 != 0) return false;
     if ((size_t)g.N * g.C * g.H * g.W * 4 >= ((size_t)1 << 31)) return false;  // 32-bit buffer offsets
     return (long)g.N * (g.C / 8) <= 65535;
+}
+
+// strips of equal height, about two waves per SIMD over the chip (as in run_conv_dw_mfma)
+static int dw_f32in_rows(const ConvGeom& g) {
+    const long planes = (long)g.N * (g.C / 8);
+    int ns = 1;
+    while (ns < g.OH && ns * planes < 2048) ++ns;
+    return (g.OH + ns - 1) / ns;
+}
+
+// Whether this launch is faster than a quantize pass and the int8 kernel: 3x3 on 17 columns and more, wherever it can run (0.80 of the time over 2800
+// drawn layers); narrower images, of whose rows a wave fills a part of its lanes, and 5x5, which reads four rows more for a strip, by models of the
+// two (us, launches replayed from graphs; fitted to 3670 drawn layers, half within 6 and 3 %, nine in ten within 16 and 8 %). Over 1100 other such layers
+// the rule takes 88 % and gives 0.89 of the time (the faster of both each time: 0.88), of calls one by one, which the host bounds, 0.67; 51 are over 5 %
+// slower, the worst 1.31. 32 channels 5x5 @111x111 b6 8.8 us as two; 360 5x5 @22x22 b2 6.0; 120 3x3 @13x13 b10 5.0.
+bool dw_f32in_faster(const ConvGeom& g, int out_bytes) {
+    if (g.kh == 3 && g.W >= 17) return true;
+    const int rps = dw_f32in_rows(g), NL = (g.W + 31) / 32, T = g.sh == 1 ? 2 : 1;
+    const float planes = (float)g.N * (g.C / 8), in = planes * (float)(g.H * g.W) * 8e-6f, res = planes * (float)(g.OH * g.OW) * 8e-6f;
+    const float m = std::max(planes * (float)((g.OH + rps - 1) / rps) / 1024.f, 1.f), rows = (float)((rps - 1) * g.sh + g.kh);
+    const float one = 4.63f + m * (0.0235f * rows * NL + (float)(rps * ((NL + 1) / 2) * T) * (g.kh == 5 ? 0.1506f : 0.087f)) + 0.415f * in + 0.0193f * res * out_bytes;
+    const float two = 5.99f + 0.858f * in + (g.kh == 5 ? 0.143f * res : 0.f) + 0.4f * planes * (float)(g.OH * ((g.OW + 3) / 4 * 4)) * 8e-6f + 2.5e-5f * std::max(0.f, planes - 2048.f);
+    return one < two;
 }
 
 hipError_t run_conv_dw_f32in(const float* x, const int8_t* wa, void* out, const ConvGeom& g, const Epilogue& ep, int epi,
@@ -596,31 +618,30 @@ hipError_t run_conv_dw_f32in(const float* x, const int8_t* wa, void* out, const 
     const int C8 = g.C / 8;
     const long planes = (long)g.N * C8;
     if (planes > 65535) return hipErrorInvalidValue;
-    // strips of equal height, about two waves per SIMD over the chip (as in run_conv_dw_mfma)
-    int rps;
-    if (strip_rows > 0) {
-        rps = std::min(strip_rows, g.OH);
-    } else {
-        int ns = 1;
-        while (ns < g.OH && ns * planes < 2048) ++ns;
-        rps = (g.OH + ns - 1) / ns;
-    }
+    const int rps = strip_rows > 0 ? std::min(strip_rows, g.OH) : dw_f32in_rows(g);
     const int n_strips = (g.OH + rps - 1) / rps;
     const int wpb = n_strips % 4 == 0 ? 4 : (n_strips % 2 == 0 ? 2 : 1);
     const dim3 grid((unsigned)(n_strips / wpb), (unsigned)planes), block(64 * wpb);
     const float in_half = in_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     // A grid of a few workgroups per CU is resident all at once, and the dispatcher is free to give one CU three of them
     // and another one: the kernel then lasts as long as the fullest CU. Reserving a share of the CU's 160 KB of LDS per
-    // workgroup (beyond the 17 KB of lines the kernel uses) caps the workgroups per CU at the even share.
+    // workgroup (beyond the 17 KB of lines the kernel uses, 35 with a 5x5 window) caps the workgroups per CU at the even share.
     const long wgs = (long)grid.x * grid.y, per_cu = (wgs + 255) / 256;
     unsigned lds_reserve = 0;
-    if (wpb == 4 && per_cu >= 2 && per_cu <= 3) lds_reserve = (unsigned)(160 * 1024 / per_cu - 18 * 1024) / 1024 * 1024;
-    if (lds_reserve > 46 * 1024) lds_reserve = 46 * 1024;  // static + dynamic stay within the default 64 KB limit
+    const unsigned lines = (g.kh == 3 ? 18 : 36) * 1024;
+    if (wpb == 4 && per_cu >= 2 && per_cu <= 3) lds_reserve = (unsigned)(160 * 1024 / per_cu - lines) / 1024 * 1024;
+    if (lds_reserve > 64 * 1024 - lines) lds_reserve = 64 * 1024 - lines;  // static + dynamic stay within the default 64 KB limit
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W * 4);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW * (epi == EPI_F32_P4 || epi == EPI_F32_P8 ? 4 : 1));
 #define OHIP_DWF_L(S_, E_, L_)                                                                                           \
-    launch((conv_dw3x3_f32in_kernel<S_, E_, L_>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
-                       DwGrid::of(grid.x, grid.y, (unsigned)C8, wpb), n_strips, rps, in_bytes, out_bytes)
+    do {                                                                                                                 \
+        if (g.kh == 3)                                                                                                   \
+            launch((conv_dw3x3_f32in_kernel<S_, E_, L_, 3>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
+                   DwGrid::of(grid.x, grid.y, (unsigned)C8, wpb), n_strips, rps, in_bytes, out_bytes);                   \
+        else                                                                                                             \
+            launch((conv_dw3x3_f32in_kernel<S_, E_, L_, 5>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
+                   DwGrid::of(grid.x, grid.y, (unsigned)C8, wpb), n_strips, rps, in_bytes, out_bytes);                   \
+    } while (0)
 #define OHIP_DWF_N(S_, E_)                       \
     do {                                         \
         switch ((g.W + 31) / 32) {               \

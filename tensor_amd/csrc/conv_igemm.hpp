@@ -122,6 +122,7 @@ bool xdw_applicable(const ConvGeom& gx, const Epilogue& epx, int epi_x, bool sox
 hipError_t run_conv_xdw(const int8_t* x, const int8_t* wx, const int8_t* wa, void* out, const ConvGeom& gx, const Epilogue& epx,
                         const ConvGeom& g, const Epilogue& ep, int epi_d, int strip_rows, hipStream_t stream);
 bool dw_f32in_applicable(const ConvGeom& g, int in_layout);
+bool dw_f32in_faster(const ConvGeom& g, int out_bytes);  // out_bytes: of a value
 hipError_t run_conv_dw_f32in(const float* x, const int8_t* wa, void* out, const ConvGeom& g, const Epilogue& ep, int epi,
                              const float* in_scale, int in_round_mode, int strip_rows, hipStream_t stream);
 hipError_t run_conv_dw_mfma(const int8_t* x, const int8_t* wa, void* out, const ConvGeom& g, const Epilogue& ep, int epi,
