@@ -906,7 +906,7 @@ int otter_hip_conv_rows_plan(const otter_hip_conv_desc* desc, int n, int in_h, i
 static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout, int n, int in_h, int in_w, void* out,
                         int out_layout, void* workspace, size_t workspace_bytes, void* stream_, int8_t* twin,
                         float twin_scale, int twin_round, const float* residual = nullptr,
-                        otter_hip_workspace_fn make_workspace = nullptr, void* make_ctx = nullptr) {
+                        otter_hip_workspace_fn make_workspace = nullptr, void* make_ctx = nullptr, bool shared_workspace = false) {
     // the caller's workspace, or one that it makes now: most launches on an fp32 blob quantize for themselves and need none
     auto workspace_of = [&](size_t need) {
         if (make_workspace && need && (!workspace || workspace_bytes < need)) workspace = make_workspace(make_ctx, need), workspace_bytes = workspace ? need : 0;
@@ -997,7 +997,8 @@ static int conv_forward(const otter_hip_conv_t* h, const void* in, int in_layout
     {
         Epilogue ep = make_epilogue(h, out_layout);
         const bool alone = !twin && !residual, own6 = alone && use_pw_f32in(h, in_layout, g, ep), own1 = !own6 && use_igemm_f32in(h, in_layout, g, ep);
-        if (alone && (own6 || own1) && pw_quantized_apart(h, g, ep, own6 ? 6 : 1) && workspace_of((size_t)n * g.C * in_h * in_w)) {
+        // (not with the workspace that every call of the GPU shares: such a layer has never touched it, and may overlap with others)
+        if (alone && (own6 || own1) && !shared_workspace && pw_quantized_apart(h, g, ep, own6 ? 6 : 1) && workspace_of((size_t)n * g.C * in_h * in_w)) {
             // as two launches, below
         } else if (own6) {
             OHIP_CHECK(run_conv_pw_f32in((const float*)in, h->w_igemm, h->clamp_hi, out, g, ep, h->in_scale, d.in_round_mode,
@@ -1114,7 +1115,7 @@ int otter_hip_conv_forward_static(const otter_hip_conv_t* h, const void* in, int
     int rc = OTTER_HIP_OK;
     void* ws = need ? static_workspace(&rc) : nullptr;
     if (rc != OTTER_HIP_OK) return rc;
-    return conv_forward(h, in, in_layout, n, in_h, in_w, out, out_layout, ws, need, stream, nullptr, 0.f, 0);
+    return conv_forward(h, in, in_layout, n, in_h, in_w, out, out_layout, ws, need, stream, nullptr, 0.f, 0, nullptr, nullptr, nullptr, true);
 }
 
 // ---- a chain of layers -------------------------------------------------------------------------------------------
