@@ -170,7 +170,7 @@ int otter_hip_conv_forward(const otter_hip_conv_t* handle, const void* in, int i
                            void* out, int out_layout, void* workspace, size_t workspace_bytes, void* stream);
 
 /* otter_hip_conv_forward with the workspace made by the call, at most once and only where the chosen launches use one: make returns
- * device memory of at least that many bytes, on the calling thread, or null (the call then fails as without a workspace). It is the
+ * device memory of at least that many bytes, on the calling thread, or null (the call then does what it does without a workspace). It is the
  * caller's to free, after the stream's work up to here; make must not throw. */
 typedef void* (*otter_hip_workspace_fn)(void* ctx, size_t bytes);
 int otter_hip_conv_forward_making(const otter_hip_conv_t* handle, const void* in, int in_layout, int n, int in_h, int in_w, void* out,
@@ -401,8 +401,9 @@ int otter_hip_conv_block_set_plan(otter_hip_conv_t* expand, int rows_per_band, i
 /* Which kernel family forward() would launch for this input: 0 direct (scalar fallback), 1 MFMA implicit
  * GEMM, 2 depthwise, 3 MFMA 3x3 halo kernel, 4 few-channel 3x3 kernel (an image stem read straight from the unpacked
  * blob), 5 streamed 1x1 kernel (int8 -> int8 over at most 64 input channels), 6 pointwise layer on an fp32 Float8 blob
- * of 64..256 channels, quantize and convolution in one launch that reads the blob once. (Other pointwise and depthwise 3x3
- * layers on an fp32 Float8 blob also quantize inside the convolution's launch; they report 1 and 2. Families 1, 3, 5 and 6
+ * of 64..256 channels, quantize and convolution in one launch that reads the blob once. (Other pointwise layers and depthwise 3x3 and 5x5
+ * layers on an fp32 Float8 blob also quantize inside the convolution's launch, where that is faster; they report 1 and 2. Pointwise layers on
+ * many fp32 values are a quantize pass and an int8 launch where that is faster and there is a workspace. Families 1, 3, 5 and 6
  * have other kernels for layers that those are faster on, see otter_hip_conv_launch_choice; the family stays what is
  * reported.) For tests and profiling. */
 int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w,

@@ -472,10 +472,7 @@ static size_t dwpw_lds_bytes(const ConvGeom& gd, const ConvGeom& g0, const ConvG
 }
 static DwPwStage dwpw_staged(const ConvGeom& gd, int groups) {
     if (gd.sh != 1 || gd.sw != 1 || gd.OH != gd.H || gd.OW != gd.W) return {};
-    DwPwStage st = dwpw_stage(gd.C, gd.H, gd.W, gd.kh, gd.ph, gd.pw, gd.dh, gd.dw, 16 * groups);
-    const FastDiv f = fast_div(st.image);
-    st.image_m = f.m, st.image_s = f.s;
-    return st;
+    return dwpw_stage(gd.C, gd.H, gd.W, gd.kh, gd.ph, gd.pw, gd.dh, gd.dw, 16 * groups);  // (without the division by an image)
 }
 
 bool dwpw_front_applicable(const ConvGeom& gd, const Epilogue& ed) {
@@ -519,48 +516,49 @@ bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom
 // a wave walks nd pairs of octets and n0 and n1 pairs of row tiles one behind the other, once if every workgroup is resident, and the more
 // often the more waves there are for a compute unit than it holds; with staged pixels it issues its share of the copies in front of that.
 struct DwPwShape {
-    double px;  // output pixels
+    float px, mac, wide;  // output pixels; 10^9 multiply-adds of the pointwise layers; 10^6 values past the 256th channel
+    int octets;
     int pairs_d, pairs[2], steps[2];
     bool k5, f32, adds;
     DwPwShape(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1)
-        : px((double)g0.N * g0.H * g0.W), pairs_d((gd.C / 8 + 1) / 2),
+        : px((float)g0.N * g0.H * g0.W), mac(1e-9f * px * g0.K * (float)(gd.C + (g1 ? g1->K : 0))), wide(1e-6f * px * (float)std::max(0, gd.C - 256)), octets(gd.C / 8), pairs_d((gd.C / 8 + 1) / 2),
           pairs{(g0.K + 31) / 32, g1 ? (g1->K + 31) / 32 : 0}, steps{igemm_channel_groups(g0.C), g1 ? igemm_channel_groups(g1->C) : 0},
           k5(gd.kh == 5), f32(e0.out_kind == OTTER_HIP_OUT_F32), adds(e0.residual || e0.join) {}
 };
-static double dwpw_cost(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1, int waves, int groups, const DwPwStage& st, size_t lds) {
+static float dwpw_cost(const DwPwShape& s, float mb, int waves, int groups, const DwPwStage& st, size_t lds) {
     static const struct {
-        double once[10], more[10], byte, mac, wide;  // for 10^6 bytes, 10^9 multiply-adds of the pointwise layers, 10^6 values past the 256th channel
+        float once[10], more[10], byte, mac, wide;  // for 10^6 bytes, 10^9 multiply-adds of the pointwise layers, 10^6 values past the 256th channel
     } table[4] = {  // four and eight waves, without and with staged pixels
-        {{3.11, 0.394, 0.726, 0.319, 0.082, 0.438, 0.0434, 0.166, 0.26}, {0.637, 0.334, 1.12, 0.408, 0.00861, 0.347, 0, 0, 0}, 0.11, 0.878, 0.081},
-        {{3.12, 0.416, 0.885, 0.46, 0.104, 0.563, 0.0802, 0.177, 0.24}, {0.702, 0.283, 1.5, 0.309, 0.0625, 0.344, 0, 0.0807, 0.00366}, 0.105, 0.69, 0},
-        {{3.38, 0.161, 0.305, 0.359, 0.0646, 0.445, 0.0341, 0.16, 0.218, 0.1}, {1.02, 0.226, 0.92, 0.186, 0.0325, 0.328, 0, 0, 0, 0.00464}, 0.12, 1.14, 1.44},
-        {{3.12, 0.267, 0.474, 0.552, 0.0722, 0.597, 0.0785, 0.154, 0.192, 0.139}, {0.945, 0.174, 1.37, 0.283, 0.0383, 0.365, 0, 0.00306, 0, 0.03}, 0.114, 0.558, 0.558}};
-    const int stride = waves / groups, nd = (s.pairs_d + stride - 1) / stride;
+        {{3.11f, 0.394f, 0.726f, 0.319f, 0.082f, 0.438f, 0.0434f, 0.166f, 0.26f}, {0.637f, 0.334f, 1.12f, 0.408f, 0.00861f, 0.347f, 0, 0, 0}, 0.11f, 0.878f, 0.081f},
+        {{3.12f, 0.416f, 0.885f, 0.46f, 0.104f, 0.563f, 0.0802f, 0.177f, 0.24f}, {0.702f, 0.283f, 1.5f, 0.309f, 0.0625f, 0.344f, 0, 0.0807f, 0.00366f}, 0.105f, 0.69f, 0},
+        {{3.38f, 0.161f, 0.305f, 0.359f, 0.0646f, 0.445f, 0.0341f, 0.16f, 0.218f, 0.1f}, {1.02f, 0.226f, 0.92f, 0.186f, 0.0325f, 0.328f, 0, 0, 0, 0.00464f}, 0.12f, 1.14f, 1.44f},
+        {{3.12f, 0.267f, 0.474f, 0.552f, 0.0722f, 0.597f, 0.0785f, 0.154f, 0.192f, 0.139f}, {0.945f, 0.174f, 1.37f, 0.283f, 0.0383f, 0.365f, 0, 0.00306f, 0, 0.03f}, 0.114f, 0.558f, 0.558f}};
+    const int stride = waves / groups, nd = (s.pairs_d + stride - 1) / stride, n0 = (s.pairs[0] + stride - 1) / stride, n1 = (s.pairs[1] + stride - 1) / stride;
     const auto& k = table[(st.pitch ? 2 : 0) + (waves == 8)];
-    const double n0 = (s.pairs[0] + stride - 1) / stride, n1 = (s.pairs[1] + stride - 1) / stride;
-    const double copies = st.pitch ? (double)((st.units + 63) / 64) * ((gd.C / 8 + (64 >> st.lg_lanes) - 1) >> (6 - st.lg_lanes)) / waves : 0.;
-    const double f[10] = {1, s.k5 ? 0. : nd, s.k5 ? (double)nd : 0, n0, n0 * s.steps[0], n1, n1 * s.steps[1], s.f32 ? n0 : 0, s.adds ? n0 : 0, copies};
-    const double held = st.pitch ? std::min(8., (double)waves * (163840 / lds)) : 8.;
-    const double rounds = std::max(0., s.px / (16 * groups) * waves / (256 * held) - 1);
-    double t = 0;
+    const float copies = st.pitch ? (float)((st.units + 63) / 64 * ((s.octets + (64 >> st.lg_lanes) - 1) >> (6 - st.lg_lanes))) / (float)waves : 0.f;
+    const float f[10] = {1, s.k5 ? 0.f : (float)nd, s.k5 ? (float)nd : 0.f, (float)n0, (float)(n0 * s.steps[0]), (float)n1, (float)(n1 * s.steps[1]), s.f32 ? (float)n0 : 0.f,
+                         s.adds ? (float)n0 : 0.f, copies};
+    const float held = st.pitch ? std::min(8.f, (float)(waves * (int)(163840 / lds))) : 8.f;
+    const float rounds = std::max(0.f, s.px * (float)waves / (4096.f * (float)groups * held) - 1.f);
+    float t = k.byte * mb + k.mac * s.mac + k.wide * s.wide;
     for (int i = 0; i < 10; ++i) t += f[i] * (k.once[i] + rounds * k.more[i]);
-    const double mb = 1e-6 * s.px * ((double)gd.C * gd.sh * gd.sw + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (g1 ? g1->K : 0));
-    return t + k.byte * mb + 1e-9 * s.px * g0.K * (gd.C + (g1 ? g1->K : 0.)) * k.mac + 1e-6 * s.px * std::max(0, gd.C - 256) * k.wide;
+    return t;
 }
 // the layers by themselves, the pointwise ones as a pair where that is a launch
-static double dwpw_cost_apart(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1) {
-    const double mbd = 1e-6 * s.px * gd.C * (gd.sh * gd.sw + 1.);
-    const double mb0 = 1e-6 * s.px * (gd.C + (double)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (s.f32 ? g0.K : 0));
-    double t = 4.86 + (0.299 + (s.k5 ? 0.051 : 0)) * mbd + 0.173 * mb0 + 2.396e-9 * s.px * g0.C * g0.K + 1.193e-3 * gd.C + 0.213e-3 * g0.K;
-    if (g1) t += 1.91 + 0.379e-6 * s.px * ((double)g0.K + g1->K) + 1.007e-9 * s.px * g0.K * g1->K + 1.519e-3 * g1->K + (g0.K > 256 ? 0.54 : 0);
+static float dwpw_cost_apart(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1) {
+    const float mbd = 1e-6f * s.px * gd.C * (gd.sh * gd.sw + 1.f);
+    const float mb0 = 1e-6f * s.px * (gd.C + (float)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (s.f32 ? g0.K : 0));
+    float t = 4.86f + (0.299f + (s.k5 ? 0.051f : 0)) * mbd + 0.173f * mb0 + 2.396e-9f * s.px * g0.C * g0.K + 1.193e-3f * gd.C + 0.213e-3f * g0.K;
+    if (g1) t += 1.91f + 0.379e-6f * s.px * ((float)g0.K + g1->K) + 1.007e-9f * s.px * g0.K * g1->K + 1.519e-3f * g1->K + (g0.K > 256 ? 0.54f : 0);
     return t;
 }
 
 // Groups of 16 pixels for a workgroup, + 16 for one of four waves: those have fewer idle waves where there are many pixels and few
 // channels (88 -> 88 -> 88 @52x52 b16 with a shuffle: eight waves and four groups 17.6 us, four and four 15.6), eight a shorter chain;
 // + 32 with staged pixels (15.3): not where the input's address is no multiple of their eight bytes.
-static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, bool aligned, double* cost) {
+static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, bool aligned, float* cost) {
     const DwPwShape s(gd, g0, e0, g1);
+    const float mb = 1e-6f * s.px * ((float)gd.C * gd.sh * gd.sw + (float)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (g1 ? g1->K : 0));
     int best = 0;
     for (int waves = 8; waves >= 4; waves -= 4)
         for (int g = 1; g <= waves; g *= 2)
@@ -568,19 +566,19 @@ static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0,
                 const DwPwStage st = staged ? dwpw_staged(gd, g) : DwPwStage{};
                 const size_t lds = dwpw_lds_bytes(gd, g0, g1, g, st);
                 if (lds > 65536 || (staged && !st.pitch)) continue;
-                const double c = dwpw_cost(s, gd, g0, g1, waves, g, st, lds);
+                const float c = dwpw_cost(s, mb, waves, g, st, lds);
                 if (!best || c < *cost) best = g + (waves == 4 ? 16 : 0) + 32 * staged, *cost = c;
             }
     return best;
 }
-// Over 2330 layers beside the fit the rule takes 67 % and gives 0.88 of the time (the faster of both each time: 0.868); 42 of them are over 5 %
+// Over 2330 layers beside the fit the rule takes 67 % and gives 0.88 of the time (the faster of both each time: 0.868); 39 of them are over 5 %
 // slower than apart, the worst 1.38. Of 88 with 640 channels and more on 4096 pixels and more, where both models are further off, those
 // under 0.75 take 0.80 of the time and none is slower; 664 -> 664 -> 40 on 17340 pixels, 0.78 by the models, is level.
 bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
-    double cost = 0;
+    float cost = 0;
     dwpw_plan(gd, g0, e0, g1, true, &cost);
     const DwPwShape s(gd, g0, e0, g1);
-    return cost < (gd.C >= 640 && s.px >= 4096 ? 0.75 : 0.92) * dwpw_cost_apart(s, gd, g0, g1);
+    return cost < (gd.C >= 640 && s.px >= 4096 ? 0.75f : 0.92f) * dwpw_cost_apart(s, gd, g0, g1);
 }
 
 template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>
@@ -614,12 +612,14 @@ hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const
     pa.HW = g0.H * g0.W, pa.OW = g0.W, pa.H = gd.H, pa.W = gd.W, pa.total_pix = (unsigned)g0.N * (unsigned)pa.HW;
     pa.in_bytes = (unsigned)((size_t)gd.N * gd.C * gd.H * gd.W);
     pa.sh = gd.sh, pa.sw = gd.sw, pa.ph = gd.ph, pa.pw = gd.pw, pa.dh = gd.dh, pa.dw = gd.dw, pa.C8 = gd.C / 8;
-    double cost = 0;
+    float cost = 0;
     const int plan = force ? force : dwpw_plan(gd, g0, e0, g1, (uintptr_t)x % 8 == 0, &cost), groups = plan & 15, waves = plan & 16 ? 4 : 8;
     if (groups > waves) return hipErrorInvalidValue;
     if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return hipErrorInvalidValue;
     if (plan & 32) pa.st = dwpw_staged(gd, groups);
     if ((plan & 32) && (!pa.st.pitch || (uintptr_t)x % 8)) return hipErrorInvalidValue;
+    const FastDiv image = fast_div(pa.st.image);
+    pa.st.image_m = image.m, pa.st.image_s = image.s;
     pa.between = (unsigned)dwpw_between(gd, g1, groups, pa.st);
     const size_t lds = dwpw_lds_bytes(gd, g0, g1, groups, pa.st);
     if (lds > 65536) return hipErrorInvalidValue;
