@@ -573,12 +573,16 @@ static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0,
 }
 // Over 2330 layers beside the fit the rule takes 67 % and gives 0.88 of the time (the faster of both each time: 0.868); 39 of them are over 5 %
 // slower than apart, the worst 1.38. Of 88 with 640 channels and more on 4096 pixels and more, where both models are further off, those
-// under 0.75 take 0.80 of the time and none is slower; 664 -> 664 -> 40 on 17340 pixels, 0.78 by the models, is level.
+// under 0.75 take 0.80 of the time and none is slower; 664 -> 664 -> 40 on 17340 pixels, 0.78 by the models, is level. So it is with ten million values and more of a
+// layer without a stride: apart they find each other's blobs in the caches, which the fits' operands are not in. In 2650 drawn blocks whose depthwise and project layers
+// the rule without this line takes, the whole block takes 0.93 to 0.97 of its time below ten million (stride 2: 0.87 to 0.95 at any size), 1.03 from there, 1.17 from
+// thirty million.
 bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
     float cost = 0;
     dwpw_plan(gd, g0, e0, g1, true, &cost);
     const DwPwShape s(gd, g0, e0, g1);
-    return cost < (gd.C >= 640 && s.px >= 4096 ? 0.75f : 0.92f) * dwpw_cost_apart(s, gd, g0, g1);
+    const bool far = (gd.C >= 640 && s.px >= 4096) || (gd.sh == 1 && gd.sw == 1 && s.px * gd.C >= 1e7f);
+    return cost < (far ? 0.75f : 0.92f) * dwpw_cost_apart(s, gd, g0, g1);
 }
 
 template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>

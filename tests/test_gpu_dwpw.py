@@ -190,6 +190,7 @@ def test_a_blob_at_an_odd_address(hip):
     (120, 3, 1, 32, 0, 6, 24, "i8", 0.71), (128, 5, 1, 128, 112, 16, 13, "i8", 0.75),
     (952, 3, 2, 952, 0, 2, 8, "f32", 3.47), (600, 5, 2, 600, 0, 1, 10, "i8", 2.99), (848, 3, 1, 848, 848, 3, 10, "i8", 2.56),
     # many channels and many pixels, where the models are too kind to the launch
+    (384, 3, 1, 32, 0, 29, 76, "f32", 1.3), (144, 3, 1, 32, 0, 49, 80, "f32", 1.3),  # ten million values and more, in a block with its expand layer
     (664, 3, 1, 664, 32, 7, 49, "f32", 1.50), (696, 3, 1, 696, 120, 4, 75, "i8", 1.47), (904, 3, 2, 904, 904, 3, 78, "f32", 1.19),
 ])
 def test_the_launch_is_taken_where_it_is_faster(hip, C, k, stride, K, K2, n, side, form, ratio):
