@@ -50,9 +50,10 @@ struct DwPwArgs {
     unsigned hw_s, ow_s;
     int lg, dw_lrelu, dw_nonneg;     // lg: log2 of the pixel groups
     unsigned first_pack;             // channels of an element of a shuffle's first half
-    DwPwStage st;                    // the pixels that a workgroup stages, st.pitch 0: none
     unsigned between;                // bytes of LDS between the first layer's pixels and the constants
 };
+template <bool STAGED>
+using DwPwStaged = std::conditional_t<STAGED, DwPwStage, NoJoin>;  // the pixels that a workgroup stages
 
 // the fp32 blob whose elements an epilogue reads
 template <class A>
@@ -98,11 +99,14 @@ void dwpw_pack_weights(const int8_t* w, int C, int ks, int8_t* dst) {
 
 // TAPS: 9 or 25. EPI: the first pointwise layer's epilogue: EPI_I8_P8; EPI_F32_P4_FUSED (with or without a residual and a twin; without
 // a second layer this is the plain fp32 result as well), EPI_F32_P4_PARTS, EPI_F32_SHUFFLE. KIND1: the second layer's result or DP_NONE.
-// DFULL: the depthwise layer ends as EPI_I8_P8_FULL says (else any int8 end).
+// DFULL: the depthwise layer ends as EPI_I8_P8_FULL says (else any int8 end). STAGED: the plans that copy the windows' pixels into LDS.
+// (An instance of its own: with both ways in one kernel either carried the other's registers, 3x3 102 to 114 of them for 80 to 94, 5x5 154 to
+// 166 for 106 to 122, a wave a SIMD less. The plans without staged pixels, the best one of each of 700 drawn layers, half of them with a stride,
+// then took up to 1.14 of their time before there were staged ones, 5x5 up to 1.17 and 1.02 on average; now 3x3 0.97, 5x5 0.995, at most 1.04.)
 // out: the last layer's result; sum: with a second layer, the first one's fp32 result (null: not wanted).
-template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>
+template <int NW, int TAPS, int EPI, int KIND1, bool DFULL, bool STAGED>
 __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __restrict__ x, void* __restrict__ out, float* __restrict__ sum,
-                                                                  DwPwArgs pa, PwAdd<EPI> ja) {
+                                                                  DwPwArgs pa, PwAdd<EPI> ja, DwPwStaged<STAGED> st) {
     constexpr bool SHUF = EPI == EPI_F32_SHUFFLE, I8 = EPI == EPI_I8_P8, PARTS = EPI == EPI_F32_P4_PARTS, FUSED = EPI == EPI_F32_P4_FUSED || PARTS;
     constexpr bool NEXT = KIND1 != DP_NONE;
     constexpr int KS = TAPS == 9 ? 3 : 5, M = (TAPS + 3) / 4, PK = TAPS == 9 ? 2 : 4;
@@ -180,11 +184,15 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
         const unsigned oy = div_by(pix, FastDiv{pa.ow_m, pa.ow_s, (unsigned)pa.OW}), ox = pix - oy * pa.OW;
         const int y0 = (int)oy * pa.sh - pa.ph, x0 = (int)ox * pa.sw - pa.pw;
         // a tap's place in units of 8 bytes: in the blob, or among the staged pixels (one outside the image: the zeros behind them)
-        const bool st = pa.st.pitch != 0;  // (uniform)
-        const unsigned t_first = (unsigned)(tile * PIX), n_first = div_by(t_first, FastDiv{pa.hw_m, pa.hw_s, HW});
-        const int s_first = dwpw_run(pa.st, HW, t_first, n_first);
-        const int base = st ? (int)((q >> 1) * pa.st.pitch) + dwpw_window(pa.st, n, pix) - s_first : (int)((n * C8 + (q >> 1)) * HWi) + y0 * pa.W + x0;
-        const unsigned none = st ? ((q >> 1) * pa.st.pitch + pa.st.slots) * 8u : PR_OOB;
+        int base, s_first = 0;  // (s_first: where the tile's run begins)
+        unsigned none;
+        if constexpr (STAGED) {
+            const unsigned t_first = (unsigned)(tile * PIX);
+            s_first = dwpw_run(st, HW, t_first, div_by(t_first, FastDiv{pa.hw_m, pa.hw_s, HW}));
+            base = (int)((q >> 1) * st.pitch) + dwpw_window(st, n, pix) - s_first, none = ((q >> 1) * st.pitch + st.slots) * 8u;
+        } else {
+            base = (int)((n * C8 + (q >> 1)) * HWi) + y0 * pa.W + x0, none = PR_OOB;
+        }
         // the taps inside the image as bits, shifted to the lane's own
         unsigned columns = 0, taps = 0;
 #pragma unroll
@@ -220,37 +228,33 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
 #pragma unroll
             for (int i = 0; i < PK; ++i) w[i] = t[i];
         };
+        [[maybe_unused]] int8_t* staged_w = nullptr;
+        if constexpr (STAGED) staged_w = staged + st.octets * st.pitch * 8u;
         auto load = [&](int op) {
-            const unsigned s = (unsigned)op * 16u * HWi;
+            const auto pixel = [&](unsigned v) {
+                if constexpr (STAGED) return *reinterpret_cast<const v2i*>(staged + (unsigned)op * 16u * st.pitch + v);
+                else return load8(rin, v, (unsigned)op * 16u * HWi);
+            };
 #pragma unroll
             for (int m = 0; m < M; ++m) {
-                const v2i lo = load8(rin, v[m][0], s), hi = 4 * m + 1 < TAPS ? load8(rin, v[m][1], s) : v2i{0, 0};
+                const v2i lo = pixel(v[m][0]), hi = 4 * m + 1 < TAPS ? pixel(v[m][1]) : v2i{0, 0};
                 b[m] = v4i{lo[0], lo[1], hi[0], hi[1]};
             }
-            if constexpr (PK == 2) weights(load8(rw, lane * 8, (unsigned)op * 512u));
+            if constexpr (STAGED) weights(*reinterpret_cast<const Weights*>(staged_w + (op * 64 + (int)lane) * 4 * PK));
+            else if constexpr (PK == 2) weights(load8(rw, lane * 8, (unsigned)op * 512u));
             else weights(load16(rw, lane * 16, (unsigned)op * 1024u));
         };
-        int8_t* const staged_w = staged + pa.st.octets * pa.st.pitch * 8u;
-        auto load_staged = [&](int op) {
-            const int8_t* const from = staged + (unsigned)op * 16u * pa.st.pitch;
-#pragma unroll
-            for (int m = 0; m < M; ++m) {
-                const v2i lo = *reinterpret_cast<const v2i*>(from + v[m][0]), hi = 4 * m + 1 < TAPS ? *reinterpret_cast<const v2i*>(from + v[m][1]) : v2i{0, 0};
-                b[m] = v4i{lo[0], lo[1], hi[0], hi[1]};
-            }
-            weights(*reinterpret_cast<const Weights*>(staged_w + (op * 64 + (int)lane) * 4 * PK));
-        };
 
-        if (st) {
+        if constexpr (STAGED) {
             // ---- the pixels that the tile's windows touch, octet by octet, and the weights into LDS: two pixels a lane -------------------------
-            const unsigned lg = pa.st.lg_lanes, unit = lane & ((1u << lg) - 1), sub = lane >> lg, sets = 64u >> lg;  // sets: octets of a copy
-            for (unsigned c = 0; c < pa.st.units; c += 64) {
+            const unsigned lg = st.lg_lanes, unit = lane & ((1u << lg) - 1), sub = lane >> lg, sets = 64u >> lg;  // sets: octets of a copy
+            for (unsigned c = 0; c < st.units; c += 64) {
                 const int at = s_first + 2 * (int)(c + unit);
-                const unsigned im = div_by((unsigned)at, FastDiv{pa.st.image_m, pa.st.image_s, pa.st.image});
-                const bool in = at >= 0 && 2 * (c + unit) < pa.st.slots && im * HW < pa.total_pix;
-                const unsigned from = in ? dwpw_copied(pa.st, HW, C8, im, sub, (unsigned)at) : PR_OOB;
-                if (c + unit < pa.st.units)
-                    for (unsigned o = wave * sets; o < C8; o += NW * sets) copy16(rin, staged + (o * pa.st.pitch + 2 * c) * 8, from, o * HW * 8u);
+                const unsigned im = div_by((unsigned)at, FastDiv{st.image_m, st.image_s, st.image});
+                const bool in = at >= 0 && 2 * (c + unit) < st.slots && im * HW < pa.total_pix;
+                const unsigned from = in ? dwpw_copied(st, HW, C8, im, sub, (unsigned)at) : PR_OOB;
+                if (c + unit < st.units)
+                    for (unsigned o = wave * sets; o < C8; o += NW * sets) copy16(rin, staged + (o * st.pitch + 2 * c) * 8, from, o * HW * 8u);
             }
             for (unsigned i = wave; i < ((unsigned)pairs * PK + 3) / 4; i += NW) copy16(rw, staged_w + i * 1024, lane * 16, i * 1024);
         } else {
@@ -283,7 +287,7 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
         Epilogue epd{};
         epd.act_p0 = pa.dw_p0, epd.lrelu = pa.dw_lrelu != 0;
         const ohip_v2s top = __builtin_bit_cast(ohip_v2s, pa.dw_qh), bottom = __builtin_bit_cast(ohip_v2s, pa.dw_nonneg ? 0u : 0xff81ff81u);
-        auto walk = [&](auto load) {
+        if constexpr (STAGED) load(min(first, pairs - 1));
         for (int op = first; op < pairs;) {
             v4i acc = {0, 0, 0, 0};
 #pragma unroll
@@ -317,13 +321,6 @@ __global__ void __launch_bounds__(64 * NW) conv_dwpw_kernel(const int8_t* __rest
                 bytes = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, hi), __builtin_bit_cast(unsigned, lo), 0x06040200u);
             }
             if (2u * now + (q >> 1) < C8) *reinterpret_cast<unsigned*>(px0 + row0 + 16 * now + 4 * q) = bytes;
-        }
-        };
-        if (st) {
-            load_staged(min(first, pairs - 1));
-            walk(load_staged);
-        } else {
-            walk(load);
         }
     }
     __syncthreads();
@@ -586,17 +583,20 @@ bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0
 }
 
 template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>
-static hipError_t launch_dwpw_waves(const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
-    launch((conv_dwpw_kernel<NW, TAPS, EPI, KIND1, DFULL>), dim3((pa.tiles + 7) / 8 * 8), dim3(64 * NW), lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0));
+static hipError_t launch_dwpw_waves(const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const DwPwStage& st, const Epilogue& e0, size_t lds, hipStream_t stream) {
+    const dim3 grid((pa.tiles + 7) / 8 * 8), block(64 * NW);
+    if (st.pitch) launch((conv_dwpw_kernel<NW, TAPS, EPI, KIND1, DFULL, true>), grid, block, lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0), st);
+    else launch((conv_dwpw_kernel<NW, TAPS, EPI, KIND1, DFULL, false>), grid, block, lds, stream, x, out, sum, pa, PwAdd<EPI>::of(e0), NoJoin{});
     return hipGetLastError();
 }
 template <int TAPS, int EPI, int KIND1>
-static hipError_t launch_dwpw(int waves, bool dfull, const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const Epilogue& e0, size_t lds, hipStream_t stream) {
+static hipError_t launch_dwpw(int waves, bool dfull, const int8_t* x, void* out, float* sum, const DwPwArgs& pa, const DwPwStage& st, const Epilogue& e0, size_t lds,
+                              hipStream_t stream) {
     if (dfull)
-        return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1, true>(x, out, sum, pa, e0, lds, stream)
-                          : launch_dwpw_waves<8, TAPS, EPI, KIND1, true>(x, out, sum, pa, e0, lds, stream);
-    return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1, false>(x, out, sum, pa, e0, lds, stream)
-                      : launch_dwpw_waves<8, TAPS, EPI, KIND1, false>(x, out, sum, pa, e0, lds, stream);
+        return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1, true>(x, out, sum, pa, st, e0, lds, stream)
+                          : launch_dwpw_waves<8, TAPS, EPI, KIND1, true>(x, out, sum, pa, st, e0, lds, stream);
+    return waves == 4 ? launch_dwpw_waves<4, TAPS, EPI, KIND1, false>(x, out, sum, pa, st, e0, lds, stream)
+                      : launch_dwpw_waves<8, TAPS, EPI, KIND1, false>(x, out, sum, pa, st, e0, lds, stream);
 }
 
 hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const ConvGeom& gd, const Epilogue& ed, const int8_t* const w[2],
@@ -620,12 +620,13 @@ hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const
     const int plan = force ? force : dwpw_plan(gd, g0, e0, g1, (uintptr_t)x % 8 == 0, &cost), groups = plan & 15, waves = plan & 16 ? 4 : 8;
     if (groups > waves) return hipErrorInvalidValue;
     if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return hipErrorInvalidValue;
-    if (plan & 32) pa.st = dwpw_staged(gd, groups);
-    if ((plan & 32) && (!pa.st.pitch || (uintptr_t)x % 8)) return hipErrorInvalidValue;
-    const FastDiv image = fast_div(pa.st.image);
-    pa.st.image_m = image.m, pa.st.image_s = image.s;
-    pa.between = (unsigned)dwpw_between(gd, g1, groups, pa.st);
-    const size_t lds = dwpw_lds_bytes(gd, g0, g1, groups, pa.st);
+    DwPwStage st{};
+    if (plan & 32) st = dwpw_staged(gd, groups);
+    if ((plan & 32) && (!st.pitch || (uintptr_t)x % 8)) return hipErrorInvalidValue;
+    const FastDiv image = fast_div(st.image);
+    st.image_m = image.m, st.image_s = image.s;
+    pa.between = (unsigned)dwpw_between(gd, g1, groups, st);
+    const size_t lds = dwpw_lds_bytes(gd, g0, g1, groups, st);
     if (lds > 65536) return hipErrorInvalidValue;
     pa.first_pack = e0.join ? (unsigned)e0.join->sh_pack0 : 8u;
     pa.lg = groups == 1 ? 0 : groups == 2 ? 1 : groups == 4 ? 2 : 3;
@@ -635,7 +636,7 @@ hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const
     const bool dfull = pa.dw_nonneg && ed.so_full;
     if (dfull) pa.dw_scale += pa.dw_scale;
     const bool shuffle = e0.join && e0.join->other;
-#define OHIP_DP(T_, E_, N_) return launch_dwpw<T_, E_, N_>(waves, dfull, x, out, sum, pa, e0, lds, stream)
+#define OHIP_DP(T_, E_, N_) return launch_dwpw<T_, E_, N_>(waves, dfull, x, out, sum, pa, st, e0, lds, stream)
 #define OHIP_DPN(T_, E_)                             \
     do {                                             \
         if (next == PP_I8) OHIP_DP(T_, E_, PP_I8);   \
