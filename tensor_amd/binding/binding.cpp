@@ -6,6 +6,7 @@
 // geometry queries the rest). Tensors come from torch's allocator on the current stream, as before; the GIL is released
 // around the C ABI call, as ctypes does.
 #include <Python.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/Context.h>
@@ -86,6 +87,7 @@ struct Workspace {
     long device;
     at::Tensor made;
     std::string error;
+    bool no_memory = false;  // the error is the lack of memory: a layer may do without
     static void* make(void* self_, size_t bytes) {
         auto* self = static_cast<Workspace*>(self_);
         const PyGILState_STATE lock = PyGILState_Ensure();  // (a dispatch mode runs Python)
@@ -93,12 +95,25 @@ struct Workspace {
         try {
             self->made = device_empty((int64_t)bytes, at::kChar, self->device);
             p = self->made.data_ptr();
+        } catch (const c10::OutOfMemoryError& e) {
+            self->fails(e.what(), true);
+        } catch (python_error& e) {
+            e.persist();  // (out of the interpreter, where it would outlive a call that does without)
+            self->fails(e.what(), lack_of_memory(e.type));
         } catch (const std::exception& e) {
-            self->error = e.what();
+            self->fails(e.what(), false);
         }
         PyGILState_Release(lock);
         return p;
     }
+    static bool lack_of_memory(PyObject* type) {  // torch.OutOfMemoryError, the form that it has behind a dispatch mode
+        PyObject* const torch = PyImport_ImportModule("torch");
+        PyObject* const of = torch ? PyObject_GetAttrString(torch, "OutOfMemoryError") : nullptr;
+        const bool is = of && type && PyErr_GivenExceptionMatches(type, of);
+        Py_XDECREF(of), Py_XDECREF(torch), PyErr_Clear();
+        return is;
+    }
+    void fails(const char* what, bool memory) { error = *what ? what : "no workspace", no_memory = memory; }
 };
 
 #define NEED(n)                                                                 \
@@ -144,7 +159,7 @@ PyObject* conv_forward(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
         rc = ws ? otter_hip_conv_forward(h, px, in_layout, n, ih, iw, po, out_layout, pw, wb, stream)
                 : otter_hip_conv_forward_making(h, px, in_layout, n, ih, iw, po, out_layout, Workspace::make, &made_ws, stream);
         Py_END_ALLOW_THREADS
-        if (rc && !made_ws.error.empty()) throw std::runtime_error(made_ws.error);
+        if (!made_ws.error.empty() && (rc || !made_ws.no_memory)) throw std::runtime_error(made_ws.error);
         if (rc) return raise_status(rc);
         return result(a[8], *out);
     } catch (const std::exception& e) {

@@ -62,3 +62,65 @@ def test_a_pointwise_layer_on_many_fp32_values(hip, C, K, n, h, w, kind, act, ma
     conv.set_tile(-6, 0)
     assert hip.torch.equal(got, conv.forward(x, capi.F32_P8, n, h, w))
     conv.close()
+
+
+def _pointwise_on_many_values(hip):
+    """(layer, blob, batch, height, width, result) of a layer that is two launches where there is room for a workspace"""
+    C, K, n, h, w = 520, 264, 24, 37, 53  # (a workspace of 24 MB: more than the allocator keeps beside what is in use)
+    rng = np.random.default_rng(3)
+    conv = hip.conv(wq=rng.integers(-127, 128, (K, C, 1, 1)).astype(np.int8), scale_in=host_scale_in(np.full(K, 60.0, np.float32), 20.0),
+                    bias=rng.normal(0, 1, K).astype(np.float32), in_scale=20.0, act=3, out_kind=capi.OUT_I8, out_scale=[0.07])
+    x = hip.to_device(rng.normal(0, 2, n * C * h * w).astype(np.float32))
+    return conv, x, n, h, w, hip.empty(n * K * h * w, np.int8)
+
+
+def test_an_error_of_the_workspace_allocation_is_the_calls(hip):
+    """A workspace that such a layer could do without: an error that is not the lack of memory is raised, and none stays behind the call."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    conv, x, n, h, w, out = _pointwise_on_many_values(hip)
+
+    class Refusing(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if "empty" in str(func):
+                raise KeyError("no new tensors here")
+            return func(*args, **(kwargs or {}))
+
+    with Refusing(), pytest.raises(RuntimeError, match="no new tensors here"):
+        conv.forward(x, capi.F32_P8, n, h, w, out=out)
+    conv.forward(x, capi.F32_P8, n, h, w, out=out)
+    conv.close()
+
+
+@pytest.mark.parametrize("mode", [False, True])
+def test_without_memory_for_a_workspace_it_is_one_launch(hip, mode):
+    """Where there is no memory for a workspace that the layer can do without, the call does without it, also where a dispatch mode reports that."""
+    import contextlib
+
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    torch = hip.torch
+    conv, x, n, h, w, out = _pointwise_on_many_values(hip)
+    want = conv.forward(x, capi.F32_P8, n, h, w)
+    refused = []
+
+    class Full(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if "empty" in str(func):
+                refused.append(func)
+                raise torch.OutOfMemoryError("no memory")
+            return func(*args, **(kwargs or {}))
+
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_stats()["num_ooms"]
+    try:
+        if not mode:
+            torch.cuda.set_per_process_memory_fraction(1e-9)  # (what is allocated stays; nothing more is given)
+        with Full() if mode else contextlib.nullcontext():
+            conv.forward(x, capi.F32_P8, n, h, w, out=out)
+        assert len(refused) == mode and torch.cuda.memory_stats()["num_ooms"] - before == (not mode)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(out, want)
+    conv.close()
