@@ -507,46 +507,59 @@ bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom
     return true;
 }
 
-// Cost models in us, fitted to launches replayed from captured graphs behind a copy that leaves the L2 caches cold, over 7000 drawn layers
-// (16 to 720 channels, 5x5 to 112x112 pixels, batches of 1 to 64, every end) and every plan of them: half of the times within 4 %, nine in ten within
-// 12 %, and so over 2300 other layers; the plan that they choose takes 1.017 of the fastest one's time there. The launch:
+// Cost models in us, fitted to launches replayed from captured graphs behind a copy that leaves the L2 caches cold, over 11700 drawn layers
+// (16 to 720 channels, 5x5 to 112x112 pixels, batches of 1 to 64, every end) and every plan of them: half of the times within 5 %, nine in ten within
+// 12 % (13 % over 15700 other layers, where the plan that they choose takes 1.014 of the fastest one's time). The launch:
 // a wave walks nd pairs of octets and n0 and n1 pairs of row tiles one behind the other, once if every workgroup is resident, and the more
-// often the more waves there are for a compute unit than it holds; with staged pixels it issues its share of the copies in front of that.
+// often the more waves there are for a compute unit than it holds (the mean of all compute units and the fullest one); with staged pixels it issues
+// its share of the copies in front of that.
 struct DwPwShape {
     float px, mac, wide;  // output pixels; 10^9 multiply-adds of the pointwise layers; 10^6 values past the 256th channel
+    float end, mb;        // bytes that a pointwise end reads and writes beside its input, for a channel of a pixel; 10^6 bytes of the launch
     int octets;
     int pairs_d, pairs[2], steps[2];
     bool k5, f32, adds;
     DwPwShape(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1)
-        : px((float)g0.N * g0.H * g0.W), mac(1e-9f * px * g0.K * (float)(gd.C + (g1 ? g1->K : 0))), wide(1e-6f * px * (float)std::max(0, gd.C - 256)), octets(gd.C / 8), pairs_d((gd.C / 8 + 1) / 2),
+        : px((float)g0.N * g0.H * g0.W), mac(1e-9f * px * g0.K * (float)(gd.C + (g1 ? g1->K : 0))), wide(1e-6f * px * (float)std::max(0, gd.C - 256)), end(ends(e0, g1)),
+          mb(1e-6f * px * ((float)(gd.C * gd.sh * gd.sw) + (float)g0.K * end + (float)(g1 ? g1->K : 0))), octets(gd.C / 8), pairs_d((gd.C / 8 + 1) / 2),
           pairs{(g0.K + 31) / 32, g1 ? (g1->K + 31) / 32 : 0}, steps{igemm_channel_groups(g0.C), g1 ? igemm_channel_groups(g1->C) : 0},
           k5(gd.kh == 5), f32(e0.out_kind == OTTER_HIP_OUT_F32), adds(e0.residual || e0.join) {}
+    static float ends(const Epilogue& e0, const ConvGeom* g1) {
+        if (e0.out_kind != OTTER_HIP_OUT_F32) return g1 ? 0.f : 1.f;
+        if (!e0.join || !e0.join->other) return (e0.residual || e0.join ? 8.f : 4.f) + (e0.twin ? 1.f : 0.f);
+        const JoinArgs& j = *e0.join;
+        return 4.f + (j.sh_out0 ? 4.f : 0.f) + (j.sh_out1 ? 4.f : 0.f) + (j.sh_q0 ? 1.f : 0.f) + (j.sh_q1 ? 1.f : 0.f);
+    }
 };
-static float dwpw_cost(const DwPwShape& s, float mb, int waves, int groups, const DwPwStage& st, size_t lds) {
+static float dwpw_cost(const DwPwShape& s, int waves, int groups, const DwPwStage& st, size_t lds) {
     static const struct {
         float once[10], more[10], byte, mac, wide;  // for 10^6 bytes, 10^9 multiply-adds of the pointwise layers, 10^6 values past the 256th channel
     } table[4] = {  // four and eight waves, without and with staged pixels
-        {{3.11f, 0.394f, 0.726f, 0.319f, 0.082f, 0.438f, 0.0434f, 0.166f, 0.26f}, {0.637f, 0.334f, 1.12f, 0.408f, 0.00861f, 0.347f, 0, 0, 0}, 0.11f, 0.878f, 0.081f},
-        {{3.12f, 0.416f, 0.885f, 0.46f, 0.104f, 0.563f, 0.0802f, 0.177f, 0.24f}, {0.702f, 0.283f, 1.5f, 0.309f, 0.0625f, 0.344f, 0, 0.0807f, 0.00366f}, 0.105f, 0.69f, 0},
-        {{3.38f, 0.161f, 0.305f, 0.359f, 0.0646f, 0.445f, 0.0341f, 0.16f, 0.218f, 0.1f}, {1.02f, 0.226f, 0.92f, 0.186f, 0.0325f, 0.328f, 0, 0, 0, 0.00464f}, 0.12f, 1.14f, 1.44f},
-        {{3.12f, 0.267f, 0.474f, 0.552f, 0.0722f, 0.597f, 0.0785f, 0.154f, 0.192f, 0.139f}, {0.945f, 0.174f, 1.37f, 0.283f, 0.0383f, 0.365f, 0, 0.00306f, 0, 0.03f}, 0.114f, 0.558f, 0.558f}};
+        {{2.85f, 0.386f, 0.711f, 0.381f, 0.0708f, 0.385f, 0.0661f, 0.198f, 0.154f, 0}, {0.572f, 0.252f, 0.78f, 0.19f, 0.0315f, 0.201f, 0.0298f, 0, 0, 0}, 0.0929f, 0.89f, 0.165f},
+        {{2.92f, 0.397f, 0.91f, 0.435f, 0.0943f, 0.514f, 0.102f, 0.262f, 0.169f, 0}, {0.62f, 0.287f, 0.738f, 0.169f, 0.0626f, 0.18f, 0.0679f, 0.116f, 0.0493f, 0}, 0.0832f, 0.476f, 0.0247f},
+        {{3.45f, 0.132f, 0.341f, 0.367f, 0.0546f, 0.369f, 0.0726f, 0.193f, 0.159f, 0.0592f}, {0.682f, 0.171f, 0.556f, 0.11f, 0.0498f, 0.247f, 0.00552f, 0, 0, 0.0638f}, 0.0926f, 1.13f, 1.65f},
+        {{3.24f, 0.25f, 0.561f, 0.432f, 0.0621f, 0.486f, 0.0934f, 0.239f, 0.144f, 0.0525f}, {0.829f, 0.161f, 0.377f, 0.238f, 0, 0.201f, 0.0645f, 0, 0, 0.0838f}, 0.0913f, 0.33f, 0.726f}};
     const int stride = waves / groups, nd = (s.pairs_d + stride - 1) / stride, n0 = (s.pairs[0] + stride - 1) / stride, n1 = (s.pairs[1] + stride - 1) / stride;
     const auto& k = table[(st.pitch ? 2 : 0) + (waves == 8)];
     const float copies = st.pitch ? (float)((st.units + 63) / 64 * ((s.octets + (64 >> st.lg_lanes) - 1) >> (6 - st.lg_lanes))) / (float)waves : 0.f;
     const float f[10] = {1, s.k5 ? 0.f : (float)nd, s.k5 ? (float)nd : 0.f, (float)n0, (float)(n0 * s.steps[0]), (float)n1, (float)(n1 * s.steps[1]), s.f32 ? (float)n0 : 0.f,
                          s.adds ? (float)n0 : 0.f, copies};
-    const float held = st.pitch ? std::min(8.f, (float)(waves * (int)(163840 / lds))) : 8.f;
-    const float rounds = std::max(0.f, s.px * (float)waves / (4096.f * (float)groups * held) - 1.f);
-    float t = k.byte * mb + k.mac * s.mac + k.wide * s.wide;
+    // workgroups for a compute unit, on average and on the fullest one, in rounds of those that run side by side at full speed: eight waves, or what the
+    // LDS with staged pixels has room for, which is whole workgroups
+    const int per_cu = ((int)((s.px + (float)(16 * groups - 1)) / (float)(16 * groups)) + 255) / 256, room = (int)(163840 / lds);
+    const bool few = st.pitch && room * waves <= 8;
+    const float held = few ? (float)room : 8.f / (float)waves;
+    const float fullest = few ? (float)((per_cu + room - 1) / room) : (float)per_cu / held;
+    const float rounds = std::max(0.f, 0.5f * (fullest + s.px / (4096.f * (float)groups * held)) - 1.f);
+    float t = k.byte * s.mb + k.mac * s.mac + k.wide * s.wide;
     for (int i = 0; i < 10; ++i) t += f[i] * (k.once[i] + rounds * k.more[i]);
     return t;
 }
 // the layers by themselves, the pointwise ones as a pair where that is a launch
 static float dwpw_cost_apart(const DwPwShape& s, const ConvGeom& gd, const ConvGeom& g0, const ConvGeom* g1) {
-    const float mbd = 1e-6f * s.px * gd.C * (gd.sh * gd.sw + 1.f);
-    const float mb0 = 1e-6f * s.px * (gd.C + (float)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (s.f32 ? g0.K : 0));
-    float t = 4.86f + (0.299f + (s.k5 ? 0.051f : 0)) * mbd + 0.173f * mb0 + 2.396e-9f * s.px * g0.C * g0.K + 1.193e-3f * gd.C + 0.213e-3f * g0.K;
-    if (g1) t += 1.91f + 0.379e-6f * s.px * ((float)g0.K + g1->K) + 1.007e-9f * s.px * g0.K * g1->K + 1.519e-3f * g1->K + (g0.K > 256 ? 0.54f : 0);
+    const float mbd = 1e-6f * s.px * gd.C * (gd.sh * gd.sw + 1.f), mb0 = 1e-6f * s.px * (gd.C + g0.K * s.end);
+    float t = 4.7f + (0.266f + (s.k5 ? 0.0437f : 0)) * mbd + 0.175f * mb0 + 1.68e-9f * s.px * g0.C * g0.K + 1.35e-3f * gd.C + 0.261e-3f * g0.K;
+    if (g1) t += 1.74f + 0.308e-6f * s.px * ((float)g0.K + g1->K) + 1.34e-9f * s.px * g0.K * g1->K + 1.44e-3f * g1->K + (g0.K > 256 ? 0.827f : 0);
     return t;
 }
 
@@ -555,7 +568,6 @@ static float dwpw_cost_apart(const DwPwShape& s, const ConvGeom& gd, const ConvG
 // + 32 with staged pixels (15.3): not where the input's address is no multiple of their eight bytes.
 static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, bool aligned, float* cost) {
     const DwPwShape s(gd, g0, e0, g1);
-    const float mb = 1e-6f * s.px * ((float)gd.C * gd.sh * gd.sw + (float)g0.K * (s.f32 ? 4 : 1) * (s.adds ? 2 : 1) + (g1 ? g1->K : 0));
     int best = 0;
     for (int waves = 8; waves >= 4; waves -= 4)
         for (int g = 1; g <= waves; g *= 2)
@@ -563,23 +575,26 @@ static int dwpw_plan(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0,
                 const DwPwStage st = staged ? dwpw_staged(gd, g) : DwPwStage{};
                 const size_t lds = dwpw_lds_bytes(gd, g0, g1, g, st);
                 if (lds > 65536 || (staged && !st.pitch)) continue;
-                const float c = dwpw_cost(s, mb, waves, g, st, lds);
+                const float c = dwpw_cost(s, waves, g, st, lds);
                 if (!best || c < *cost) best = g + (waves == 4 ? 16 : 0) + 32 * staged, *cost = c;
             }
     return best;
 }
-// Over 2330 layers beside the fit the rule takes 67 % and gives 0.88 of the time (the faster of both each time: 0.868); 39 of them are over 5 %
-// slower than apart, the worst 1.38. Of 88 with 640 channels and more on 4096 pixels and more, where both models are further off, those
-// under 0.75 take 0.80 of the time and none is slower; 664 -> 664 -> 40 on 17340 pixels, 0.78 by the models, is level. So it is with ten million values and more of a
-// layer without a stride: apart they find each other's blobs in the caches, which the fits' operands are not in. In 2650 drawn blocks whose depthwise and project layers
-// the rule without this line takes, the whole block takes 0.93 to 0.97 of its time below ten million (stride 2: 0.87 to 0.95 at any size), 1.03 from there, 1.17 from
-// thirty million.
+// Over 15684 layers beside the fit the rule takes 58 %, which then take 0.805 of their time apart, and gives 0.886 of the time of all (the faster of both each
+// time: 0.869); 69 are over 5 % slower than apart, the worst 1.29. In each band of pixels, windows and layers behind, nine in ten of those that it takes are at
+// most level with the layers apart (but for ten 5x5 layers alone on 32768 pixels and more: 1.03). Three kinds stay apart whatever the models say:
+//  * 200 MB and more (5x5: 60 MB), which the caches do not hold: both models are a third below the times there, and what 0.92 would take is 1.03 (1.0 to 1.08)
+//    of the time, the worst 1.34.
+//  * 640 channels and more on 4096 pixels and more: 0.92 would take 27 of 207, up to 1.16.
+//  * ten million values and more without a stride: 34 of the 238 that 0.92 would take are over 5 % slower; and apart they find each other's blobs in the caches,
+//    which the fits' operands are not in: in 2650 drawn blocks whose depthwise and project layers ran as one launch, the whole block took 0.93 to 0.97 of
+//    its time below ten million (stride 2: 0.87 to 0.95 at any size), 1.03 from there, 1.17 from thirty million.
 bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1) {
+    const DwPwShape s(gd, g0, e0, g1);
+    if (s.mb >= (s.k5 ? 60.f : 200.f) || (gd.C >= 640 && s.px >= 4096) || (gd.sh == 1 && gd.sw == 1 && s.px * gd.C >= 1e7f)) return false;
     float cost = 0;
     dwpw_plan(gd, g0, e0, g1, true, &cost);
-    const DwPwShape s(gd, g0, e0, g1);
-    const bool far = (gd.C >= 640 && s.px >= 4096) || (gd.sh == 1 && gd.sw == 1 && s.px * gd.C >= 1e7f);
-    return cost < (far ? 0.75f : 0.92f) * dwpw_cost_apart(s, gd, g0, g1);
+    return cost < 0.92f * dwpw_cost_apart(s, gd, g0, g1);
 }
 
 template <int NW, int TAPS, int EPI, int KIND1, bool DFULL>

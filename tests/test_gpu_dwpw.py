@@ -191,6 +191,9 @@ def test_a_blob_at_an_odd_address(hip):
     (952, 3, 2, 952, 0, 2, 8, "f32", 3.47), (600, 5, 2, 600, 0, 1, 10, "i8", 2.99), (848, 3, 1, 848, 848, 3, 10, "i8", 2.56),
     # many channels and many pixels, where the models are too kind to the launch
     (384, 3, 1, 32, 0, 29, 76, "f32", 1.3), (144, 3, 1, 32, 0, 49, 80, "f32", 1.3),  # ten million values and more, in a block with its expand layer
+    # 5x5 in a last round of workgroups that few of them fill; more bytes than the caches hold
+    (136, 5, 1, 136, 136, 4, 65, "i8", 1.33), (256, 5, 1, 24, 112, 43, 20, "i8", 1.31), (512, 5, 2, 512, 0, 42, 40, "sum", 1.39), (168, 5, 1, 168, 168, 8, 48, "i8", 1.33),
+    (600, 3, 1, 600, 0, 12, 28, "f32", 1.22), (520, 3, 1, 520, 32, 11, 81, "shuffle", 1.23), (48, 5, 1, 416, 0, 50, 32, "sum", 1.34),
     (664, 3, 1, 664, 32, 7, 49, "f32", 1.50), (696, 3, 1, 696, 120, 4, 75, "i8", 1.47), (904, 3, 2, 904, 904, 3, 78, "f32", 1.19),
 ])
 def test_the_launch_is_taken_where_it_is_faster(hip, C, k, stride, K, K2, n, side, form, ratio):
