@@ -28,7 +28,7 @@ def quantize_weights(wf):
     return wq, ws
 
 
-def make_block(hip, rng, cin, ce, cout, act, f32_out, stride=1, out_round=capi.ROUND_SSE, dw_pad=1):
+def make_block(hip, rng, cin, ce, cout, act, f32_out, stride=1, out_round=capi.ROUND_SSE, dw_pad=1, scales=None):
     """The three layers as a MobileNetV2 block has them: expand and depthwise with `act` and int8 results, a linear
     project layer with an fp32 or int8 result."""
     layers = []
@@ -37,7 +37,7 @@ def make_block(hip, rng, cin, ce, cout, act, f32_out, stride=1, out_round=capi.R
     for (ci, co, k, s, pad, groups, a, i8) in specs:
         wq, ws = quantize_weights(rng.normal(0, 0.3 if groups > 1 else 2.0 / np.sqrt(ci), (co, ci // groups, k, k)).astype(np.float32))
         bias = rng.normal(0, 0.05, co).astype(np.float32)
-        out_scale = np.float32(rng.uniform(15, 40))
+        out_scale = np.float32(rng.uniform(15, 40) if scales is None else scales[len(layers)])
         si = (np.float32(1.0) / (in_scale * ws)).astype(np.float32)
         conv = hip.conv(wq=wq, scale_in=si, bias=bias, in_scale=float(in_scale), out_scale=[out_scale] if i8 else None,
                         stride=(s, s), pad=(pad, pad), groups=groups, act=a,
@@ -123,6 +123,32 @@ def test_block_equals_the_three_layers(hip, oracle, cin, ce, cout, N, H, W, act,
         assert (out == cur).all()
     for l in layers:
         l["conv"].close()
+
+
+# output scales of the expand and the depthwise layer: with clip the upper clamp is 6 times that, 127 at most
+CLIP_SCALES = [(20.0, 30.0), (30.0, 20.0), (20.0, 15.0), (30.0, 25.0)]
+
+
+def clipped_blobs(layers, xd, n, h, w):
+    """whether both int8 blobs between the layers reach their clamps"""
+    (e, d), (a, b) = (l["conv"] for l in layers[:2]), (min(127, 6 * l["out_scale"]) for l in layers[:2])
+    t = e.forward(xd, capi.I8_P8, n, h, w, capi.I8_P8)
+    return t.max() == a and d.forward(t, capi.I8_P8, n, h, w, capi.I8_P8).max() == b
+
+
+@pytest.mark.parametrize("scales", CLIP_SCALES)
+@pytest.mark.parametrize("cin,ce,cout,N,H", [(64, 384, 64, 2, 14), (160, 960, 160, 2, 7), (24, 144, 24, 1, 28)])
+def test_block_with_clamps_below_the_bytes_end(hip, cin, ce, cout, N, H, scales):
+    """Clip with an upper clamp below 127 in one of the first two layers, in both and in neither."""
+    rng = np.random.default_rng(cin + int(scales[0]))
+    layers = make_block(hip, rng, cin, ce, cout, 3, True, scales=scales + (30.0,))
+    e, d, p = (l["conv"] for l in layers)
+    xd = hip.to_device(rng.integers(-127, 128, N * cin * H * H).astype(np.int8))
+    assert clipped_blobs(layers, xd, N, H, H)
+    assert hip.conv_block_launches(e, d, p, N, H, H) == 1
+    got, got_q = hip.conv_block(e, d, p, xd, N, H, H, q_scale=21.5)
+    want, want_q = one_by_one(hip, layers, xd, N, H, H, None, 21.5)
+    assert hip.torch.equal(got, want) and hip.torch.equal(got_q, want_q)
 
 
 @pytest.mark.parametrize("act,f32_out", [(3, True), (0, False)])

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from tensor_amd import capi
-from test_gpu_block import FP32_RTOL, make_block, one_by_one
+from test_gpu_block import CLIP_SCALES, FP32_RTOL, clipped_blobs, make_block, one_by_one
 
 pytestmark = pytest.mark.gpu
 
@@ -86,6 +86,21 @@ def test_pair_launch_equals_the_three_layers(hip, oracle, cin, ce, cout, N, H, W
         assert (out == cur).all()
     for l in layers:
         l["conv"].close()
+
+
+@pytest.mark.parametrize("scales", CLIP_SCALES)
+@pytest.mark.parametrize("cin,ce,cout,H,W,stride", [(16, 96, 24, 56, 56, 2), (24, 144, 24, 40, 17, 1), (96, 576, 160, 14, 14, 2)])
+def test_pair_launch_with_clamps_below_the_bytes_end(hip, cin, ce, cout, H, W, stride, scales):
+    """Clip with an upper clamp below 127 in one of the first two layers, in both and in neither."""
+    rng = np.random.default_rng(cin + int(scales[0]))
+    layers = make_block(hip, rng, cin, ce, cout, 3, True, stride=stride, scales=scales + (30.0,))
+    e, d, p = (l["conv"] for l in layers)
+    N = 2
+    xd = hip.to_device(rng.integers(-127, 128, N * cin * H * W).astype(np.int8))
+    assert clipped_blobs(layers, xd, N, H, W)
+    want, want_q = one_by_one(hip, layers, xd, N, H, W, None, 21.5)
+    got, got_q = hip.conv_block_form(2, e, d, p, xd, N, H, W, q_scale=21.5)
+    assert hip.torch.equal(got, want) and hip.torch.equal(got_q, want_q)
 
 
 def test_pair_launch_with_the_exact_rounding_mode(hip):

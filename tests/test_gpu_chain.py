@@ -26,13 +26,13 @@ def quantize_weights(wf):
     return wq, ws
 
 
-def _layers(hip, rng, chans, k=3, pad=1, act=1, stride=1):
+def _layers(hip, rng, chans, k=3, pad=1, act=1, stride=1, scales=None, spread=0.05):
     convs, params = [], []
     in_scale = np.float32(127.0)
-    for cin, cout in zip(chans[:-1], chans[1:]):
-        wq, ws = quantize_weights(rng.normal(0, 0.05, (cout, cin, k, k)).astype(np.float32))
+    for i, (cin, cout) in enumerate(zip(chans[:-1], chans[1:])):
+        wq, ws = quantize_weights(rng.normal(0, spread, (cout, cin, k, k)).astype(np.float32))
         bias = rng.normal(0, 0.02, cout).astype(np.float32)
-        out_scale = np.float32(rng.uniform(20, 60))
+        out_scale = np.float32(rng.uniform(20, 60) if scales is None else scales[i])
         si = (np.float32(1.0) / (in_scale * ws)).astype(np.float32)
         convs.append(hip.conv(wq=wq, scale_in=si, bias=bias, out_scale=[out_scale], stride=(stride, stride), pad=(pad, pad),
                               act=act, out_kind=capi.OUT_I8, out_round=capi.ROUND_SSE))
@@ -79,6 +79,23 @@ def test_same_shape_chain_is_one_launch_and_equals_the_layers_one_by_one(hip, or
                                             top_scale=p["out_scale"], int8_out=True, act_type=act)
         got_n = capi.unpack_np(got.cpu().numpy(), 8, (N, C, H, W))[n:n + 1]
         np.testing.assert_array_equal(got_n, cur)
+
+
+@pytest.mark.parametrize("scales", [(9.0, 12.0, 20.5), (60.0, 9.0, 40.0), (60.0, 40.0, 9.0)])  # clip: the clamp is 6 times that, 127 at most
+@pytest.mark.parametrize("C,N,H,W", [(72, 3, 13, 26), (64, 4, 28, 28)])
+def test_chain_with_clamps_below_the_bytes_end(hip, C, N, H, W, scales):
+    """Clip with an upper clamp below 127 in every layer of the launch and in one of them."""
+    rng = np.random.default_rng(C + int(scales[0]))
+    convs, _ = _layers(hip, rng, [C] * 4, act=3, scales=scales, spread=0.3)
+    xd = hip.to_device(rng.integers(-127, 128, N * C * H * W, dtype=np.int8))
+    cur = xd
+    for conv, scale in zip(convs, scales):
+        cur = conv.forward(cur, capi.I8_P8, N, H, W, capi.I8_P8)
+        assert scale > 9 or cur.max() == 6 * scale
+    assert hip.conv_chain_launches(convs, N, H, W) == 1
+    for _ in range(2):
+        assert hip.torch.equal(hip.conv_chain(convs, xd, N, H, W), cur)
+    assert not hip.conv_chain_gave_up()
 
 
 def test_other_chains_run_layer_by_layer(hip, oracle):

@@ -30,15 +30,15 @@ def weights(rng, K, C, k):
     return rng.integers(-127, 128, (K, C, k, k)).astype(np.int8), rng.uniform(40, 400, K).astype(np.float32) * np.float32(np.sqrt(C * k * k))
 
 
-def layer(hip, rng, C, K, act, f32, half=capi.ROUND_SSE):
+def layer(hip, rng, C, K, act, f32, half=capi.ROUND_SSE, scale=23.0, gain=1):
     w, ws = weights(rng, K, C, 1)
-    return hip.conv(wq=w, scale_in=host_scale_in(ws, 31.0), bias=rng.normal(0, 0.4, K).astype(np.float32), in_scale=31.0,
-                    out_scale=None if f32 else [23.0], act=act, act_p0=0.1, out_kind=capi.OUT_F32 if f32 else capi.OUT_I8, out_round=half)
+    return hip.conv(wq=w, scale_in=host_scale_in(ws / np.float32(gain), 31.0), bias=rng.normal(0, 0.4, K).astype(np.float32), in_scale=31.0,
+                    out_scale=None if f32 else [scale], act=act, act_p0=0.1, out_kind=capi.OUT_F32 if f32 else capi.OUT_I8, out_round=half)
 
 
-def depthwise(hip, rng, C, k, stride, pad, dil, act, half=capi.ROUND_SSE):
+def depthwise(hip, rng, C, k, stride, pad, dil, act, half=capi.ROUND_SSE, scale=37.0):
     w, ws = weights(rng, C, 1, k)
-    return hip.conv(wq=w, scale_in=host_scale_in(ws, 29.0), bias=rng.normal(0, 0.4, C).astype(np.float32), in_scale=29.0, out_scale=[37.0], act=act,
+    return hip.conv(wq=w, scale_in=host_scale_in(ws, 29.0), bias=rng.normal(0, 0.4, C).astype(np.float32), in_scale=29.0, out_scale=[scale], act=act,
                     act_p0=0.2, groups=C, stride=(stride, stride), pad=(pad, pad), dil=(dil, dil), out_kind=capi.OUT_I8, out_round=half)
 
 
@@ -133,6 +133,20 @@ def test_one_launch_equals_the_layers(hip, C, k, stride, pad, dil, act, K, K2, n
             pw.close()
 
 
+def staged_lds(C, k, pad, dil, K, K2, H, W, groups):
+    """Bytes of LDS of a plan with staged pixels: rows of a tile's pixels, what is staged (or the second layer's rows), the constants."""
+    up = lambda v, to: -(-v // to) * to
+    pixels = 16 * groups
+    places = pixels + (k - 1) * (dil * W + dil) + (max(0, (pixels + H * W - 2) // (H * W)) if H * W % 2 else 0)
+    units = up(1 + places, 2) // 2 + 1
+    lanes = min(64, 1 << (units - 1).bit_length())
+    octets, pitch = up(up(C // 8, 2), 64 // lanes), 2 * units if units > 64 else 2 * lanes
+    weights = up(up(C // 8, 2) // 2 * 256 * (2 if k == 3 else 4), 1024)
+    row = lambda c: up(c, 64) + 16
+    return (pixels * row(C) + max(8 * octets * pitch + weights, pixels * row(K) if K2 else 0) + 256 * (up(K, 32) + up(K2, 32)) // 32
+            + 128 * (up(C // 8, 2) // 2))
+
+
 @pytest.mark.parametrize("C,k,pad,dil,act,K,K2,N,H,W", [
     (88, 3, 1, 1, 0, 88, 88, 3, 13, 13),     # an odd count of octets, images of an odd count of pixels that begin inside a tile
     (16, 3, 1, 1, 3, 24, 16, 9, 3, 3),       # several images in a tile, octets that share a copy
@@ -149,7 +163,6 @@ def test_staged_pixels(hip, C, k, pad, dil, act, K, K2, N, H, W):
     rng = np.random.default_rng(C + K + W)
     x = hip.to_device(rng.integers(-127, 128, N * C * H * W).astype(np.int8))
     dw = depthwise(hip, rng, C, k, 1, pad, dil, act)
-    ran = 0
     for last in (None, "nonneg"):
         nx = layer(hip, rng, K, K2, 3, False) if last else None
         for form, how in forms(k, last):
@@ -157,15 +170,37 @@ def test_staged_pixels(hip, C, k, pad, dil, act, K, K2, N, H, W):
             for plan in (33, 34, 36, 40, 49, 50, 52):
                 dw.force = (-12, plan)
                 dw.set_tile(-12, plan)
-                try:
-                    got, want = one_and_two(hip, rng, form, how, dw, pw, nx, x, N, H, W)
-                except capi.HipError:  # (more LDS than a launch has)
-                    assert plan > 34
+                if staged_lds(C, k, pad, dil, K, K2 if nx else 0, H, W, plan & 15) > 65536:
+                    assert C > 16  # (the smaller ones run every plan)
+                    with pytest.raises(capi.HipError):
+                        one_and_two(hip, rng, form, how, dw, pw, nx, x, N, H, W)
                     continue
-                ran += 1
+                got, want = one_and_two(hip, rng, form, how, dw, pw, nx, x, N, H, W)
+                assert len(got) == len(want)
                 for i, (g, v) in enumerate(zip(got, want)):
                     assert hip.torch.equal(g, v), (last, form, how, plan, i)
-    assert ran
+
+
+@pytest.mark.parametrize("scale,next_scale", [(9.0, 23.0), (37.0, 9.0), (21.0, 9.0)])  # clip: 6 * 9 and 6 * 21 are below 127
+@pytest.mark.parametrize("C,k,stride,K,K2,n,h,w", [(88, 3, 1, 88, 88, 2, 13, 13), (40, 3, 2, 24, 40, 2, 17, 12), (128, 5, 1, 128, 112, 1, 13, 13)])
+def test_clamps_below_the_bytes_end(hip, C, k, stride, K, K2, n, h, w, scale, next_scale):
+    """Clip with an upper clamp below 127, in the depthwise layer, the last one or both."""
+    rng = np.random.default_rng(C + k)
+    x = hip.to_device(rng.integers(-127, 128, n * C * h * w).astype(np.int8))
+    dw = depthwise(hip, rng, C, k, stride, k // 2, 1, 3, scale=scale)
+    mid = dw.forward(x, capi.I8_P8, n, h, w, capi.I8_P8)
+    assert mid.max() == min(127, 6 * scale) and mid.min() == 0
+    for last in (False, True):
+        nx = layer(hip, rng, K, K2, 3, False, scale=next_scale, gain=16) if last else None
+        for form, how in forms(k, last):
+            pw = layer(hip, rng, C, K, 2 if form != "sum" else 0, form != "i8")
+            for plan in (2, 18) + ((34, 50) if stride == 1 else ()):
+                dw.force = (-12, plan)
+                dw.set_tile(-12, plan)
+                got, want = one_and_two(hip, rng, form, how, dw, pw, nx, x, n, h, w)
+                assert not last or want[0].max() == min(127, 6 * next_scale)
+                for i, (g, v) in enumerate(zip(got, want)):
+                    assert hip.torch.equal(g, v), (last, form, how, plan, i)
 
 
 def test_a_blob_at_an_odd_address(hip):

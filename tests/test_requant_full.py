@@ -80,3 +80,24 @@ def test_ties_and_clamps(hip, oracle, C, K, k, stride, groups, N, H, W, f32, act
                                      int8_out=True, act_type=act)
     assert got.max() >= (6 if act == 3 and scale == 1.0 else 100)
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [21.25, 21.0])  # upper clamps of 127 and 126
+@pytest.mark.parametrize("act", [1, 3])
+@pytest.mark.parametrize("C,K,k,stride,groups,N,H,W,f32", LAYERS)
+def test_results_beyond_the_range(hip, oracle, C, K, k, stride, groups, N, H, W, f32, act, scale):
+    """Biases that are infinite, beyond every scale or not a number: the clamps, and zero, whichever way the bytes are made."""
+    rng = np.random.default_rng(C + K + k)
+    x = rng.integers(-60, 61, (N, C, H, W)).astype(np.float32 if f32 else np.int8)
+    wq = rng.integers(-3, 4, (K, C // groups, k, k)).astype(np.int8)
+    bias = np.resize(np.array([np.inf, -np.inf, np.nan, 3e38, -3e38, 0.5, 1e30], np.float32), K)
+    got, _ = run_conv(hip, oracle, x, wq, np.full(K, 32.0, np.float32), 1.0, stride=stride, pad=k // 2, groups=groups, bias=bias, top_scale=scale,
+                      out_kind=capi.OUT_I8, act=act)
+    top = int(6 * scale) if act == 3 and scale == 21.0 else 127
+    for first, want in ((0, top), (1, 0), (2, 0), (3, top), (4, 0), (6, top)):
+        assert (got[:, first::7] == want).all(), first
+    zero = np.where(np.isfinite(bias), bias, np.float32(0))
+    want = oracle.conv_layer_forward(x, wq, np.full(K, 32.0, np.float32), 1.0, stride=(stride, stride), pad=(k // 2,) * 2, groups=groups, bias=zero,
+                                     top_scale=scale, int8_out=True, act_type=act)
+    np.testing.assert_array_equal(got[:, 5::7], want[:, 5::7])
