@@ -45,6 +45,27 @@ def test_the_rule_for_every_float(tmp_path):
     assert subprocess.run([exe], capture_output=True, text=True).stdout.strip() == "0"
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("half,out_round", [(0.5, capi.ROUND_SSE), (0.49999997, capi.ROUND_EXACT)])
+def test_the_rule_on_the_gpu(hip, half, out_round):
+    """The conversion itself: every quarter step from -1 to 129 and the three floats on either side, as the biases of a layer without weights."""
+    values = [np.arange(-4, 517, dtype=np.float32) / np.float32(4)]
+    for way in (-np.inf, np.inf):
+        beside = values[0]
+        for _ in range(3):
+            beside = np.nextafter(beside, np.float32(way))
+            values.append(beside)
+    bias = np.concatenate(values + [np.zeros(1, np.float32)])
+    K, C, s = bias.size, 64, 4
+    assert K % 8 == 0
+    conv = hip.conv(wq=np.zeros((K, C, 1, 1), np.int8), scale_in=np.ones(K, np.float32), bias=bias, in_scale=1.0, out_scale=[1.0], out_kind=capi.OUT_I8, act=1,
+                    out_round=out_round)
+    x = hip.to_device(np.ones(C * s * s, np.int8))
+    got = capi.unpack_np(conv.forward(x, capi.I8_P8, 1, s, s, capi.I8_P8).cpu().numpy(), 8, (1, K, s, s))
+    want = np.clip((bias + np.float32(half)).astype(np.int32), 0, 127).astype(np.int8)
+    np.testing.assert_array_equal(got, np.broadcast_to(want[None, :, None, None], got.shape))
+
+
 LAYERS = [
     # C, K, kernel, stride, groups, N, H, W, fp32 input
     (64, 128, 3, 1, 1, 8, 28, 28, False),   # LDS-halo kernel
