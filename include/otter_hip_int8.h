@@ -430,13 +430,15 @@ int otter_hip_conv_kernel_kind(const otter_hip_conv_t* handle, int in_layout, in
  * among the waves of a workgroup (1: over 64 input channels; 0: at most 256, and four groups only for a result without a sum, a twin
  * or a shuffle) and the pairs of 16 output channels a wave walks. tn = 0: all three automatic. tm == -12 on a depthwise layer:
  * otter_hip_conv_dwpw_launches says 1 wherever that launch can run, tn = 1, 2, 4 or 8 its groups of 16 pixels,
- * + 16 with four waves to a workgroup (0 = automatic). tm == -13
+ * + 16 with four waves to a workgroup, + 32 with its pixels staged in LDS (stride 1 on a blob at a multiple of eight bytes, where the
+ * LDS has room; 0 = automatic). tm == -13
  * on an image stem: tn pooled rows a workgroup in the launch with its max pooling (1, 2, 4; 0 = automatic). */
 int otter_hip_conv_set_tile(otter_hip_conv_t* handle, int tm, int tn);
 
 /* Test hook with no counterpart in the reference: which of the launches of its family a dense or grouped layer takes on a packed
  * blob (no sum, no twin): choice = { 8, 9 or 10 as set_tile(-8, ...), set_tile(-9, ...) and set_tile(-10, ...) name them, or 0, the family's own launch (on
- * an fp32 blob that may also be a quantize pass and the choice for its int8 copy), tile }. */
+ * an fp32 blob that may also be a quantize pass and the choice for its int8 copy; whether a pointwise layer on many fp32 values is one, which
+ * hangs on the workspace too, is not said), tile }. */
 int otter_hip_conv_launch_choice(const otter_hip_conv_t* handle, int in_layout, int n, int in_h, int in_w, int out_layout,
                                  int choice[2]);
 

@@ -20,10 +20,10 @@
 //    from memory in a ring of four reduction steps that is refilled across pairs and layers: the first ones are requested before the
 //    depthwise layer begins, as are the elements of a residual or of a shuffle's other blob.
 //  * Behind a barrier they do the same for the second pointwise layer.
-// Waits are half of the waves' time (47 to 59 %), vector issue 47, 35 and 16 % of the kernel's and the address unit 53, 51 and 30 % at 2.3, 2.3 and 1.2
-// waves a SIMD (88 channels @52x52, 176 @26x26 and 352 @13x13 with a shuffle and a layer behind). In the detection model, 16 images, us as two
-// or three launches / as one, with the unit's shuffle and the next unit's first layer: 88 channels @52x52 5.1 + 14.3 / 15.8, 176 @26x26
-// 4.1 + 10.0 / 12.5, 352 @13x13 3.7 + 6.1 + 4.9 / 11.7; 5x5 with two pointwise layers, 64 @13x13 3.4 + 4.7 / 6.5.
+// Waits are 40, 50 and 57 % of the waves' time, vector issue 53, 34 and 17 % of the kernel's and the address unit 41, 52 and 26 % at 2.3, 2.3 and 1.2
+// waves a SIMD (88 channels @52x52 with staged pixels, 176 @26x26 without and 352 @13x13 with, each with a shuffle and a layer behind). In traces of the
+// detection model, 16 images, us as two or three launches / as one, with the unit's shuffle and the next unit's first layer: 88 channels @52x52
+// 5.1 + 14.3 / 16.4, 176 @26x26 4.1 + 10.0 / 12.4, 352 @13x13 3.7 + 6.1 + 4.9 / 12.1; 5x5 with two pointwise layers, 64 @13x13 3.4 + 4.7 / 6.0.
 #include "conv_dwpw.hpp"
 
 #include "conv_pwpw_common.hpp"

@@ -14,7 +14,8 @@ bool conv_dwpw_applicable(const ConvGeom& gd, const Epilogue& ed, const ConvGeom
 // whether the launch is faster than the layers by themselves (the pointwise ones as a pair where that is a launch)
 bool conv_dwpw_faster(const ConvGeom& gd, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1);
 // w, so: packed weights and the output scale of every channel of the pointwise layers; sum: the first one's fp32 result in front of a
-// second layer, or null; force: 0 = automatic, else groups of 16 pixels of a workgroup (1, 2, 4, 8), + 16 with four waves to it
+// second layer, or null; force: 0 = automatic, else groups of 16 pixels of a workgroup (1, 2, 4, 8), + 16 with four waves to it,
+// + 32 with staged pixels
 hipError_t run_conv_dwpw(const int8_t* x, const int8_t* dw_w, float dw_so, const ConvGeom& gd, const Epilogue& ed, const int8_t* const w[2],
                          const float so[2], void* out, float* sum, const ConvGeom& g0, const Epilogue& e0, const ConvGeom* g1, const Epilogue* e1,
                          int force, hipStream_t stream);
