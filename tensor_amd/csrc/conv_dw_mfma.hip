@@ -336,6 +336,9 @@ __global__ void __launch_bounds__(64) conv_dw3x3_mfma_kernel(const int8_t* __res
     }
 }
 
+constexpr int dwf_lines(int ks) { return ks == 3 ? 4 : 8; }  // a wave's ring of LDS lines
+constexpr int dwf_line_bytes(int loads) { return (64 * ((loads + 1) / 2) + 8) * 8; }  // (of loads of 32 pixels each)
+
 // ---------------------------------------------------------------------------------------------------------------------
 // The same layer (3x3 or 5x5) straight from an fp32 blob: quantize_to_int8 (Tensor/ConvolutionLayer.cpp:770-775,
 // Tensor/QuantizeX86.cpp:402-490) and the depthwise convolution in ONE launch, for a Float8 input ([N][C/8][H*W][8
@@ -359,13 +362,13 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
                                                                void* __restrict__ out, ConvGeom g, Epilogue ep,
                                                                const float* __restrict__ in_scale_p, float in_half, DwGrid dg,
                                                                int n_strips, int rps, unsigned in_bytes, unsigned out_bytes) {
-    constexpr int RL = KS == 3 ? 4 : 8, PF = 4;  // LDS lines / register stages per wave
+    constexpr int RL = dwf_lines(KS), PF = 4;  // LDS lines / register stages per wave
     constexpr int NCH = (NL + 1) / 2;  // column chunks of 64 pixels (a matrix operand covers 4 x 16 of them)
     const float in_scale = in_scale_p[0];
     constexpr int T = S == 1 ? 2 : 1;  // A sets
     constexpr int PH = 4 / S;          // output pixels per lane column
-    constexpr int LINE = (64 * NCH + 8) * 8;
-    __shared__ __attribute__((aligned(16))) int8_t lds_all[4][RL][LINE];
+    constexpr int LINE = dwf_line_bytes(NL);
+    extern __shared__ __attribute__((aligned(16))) int8_t dwf_lds[];  // [waves][RL][LINE]
     const int C8 = g.C / 8;
     unsigned bx, o_u, img_u;
     dg.locate(&bx, &o_u, &img_u);
@@ -374,7 +377,9 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
     const int strip = __builtin_amdgcn_readfirstlane(bx * dg.wpb + wave);
     if (strip >= n_strips) return;  // whole wave
     const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
-    int8_t* const lds = &lds_all[wave][0][0];
+    int8_t* const lds = dwf_lds + wave * (RL * LINE);
+    // where this lane writes and reads in a line (as offsets: worked out from the pointer, one instance has a register too many)
+    const unsigned to = (unsigned)wave * (unsigned)(RL * LINE) + 16u + 4u * lane, from = (unsigned)wave * (unsigned)(RL * LINE) + (4u * n + 2u * q) * 8u;
 
     // the padding slots of every line: pixels -2, -1 and 32 NL .. 64 NCH + 5 (the row's own pixels from W on are written
     // as zeros with every row)
@@ -429,7 +434,7 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
     // lane l of load k holds pixel 32 k + l / 2, channels 4 (l & 1) ..: byte (pixel + 2) * 8 + 4 (l & 1) = 16 + 256 k + 4 l
     auto quant_write = [&](int line, const v4i (&src)[NL]) {
 #pragma unroll
-        for (int k = 0; k < NL; ++k) *reinterpret_cast<int*>(lds + line * LINE + 16 + 256 * k + 4 * lane) = quant4(src[k]);
+        for (int k = 0; k < NL; ++k) *reinterpret_cast<int*>(dwf_lds + to + line * LINE + 256 * k) = quant4(src[k]);
     };
 
     v4i a[KS][T];  // a[k]: the kernel row that meets the k-th of an output row's lines
@@ -521,7 +526,7 @@ __global__ void __launch_bounds__(256, 3) conv_dw3x3_f32in_kernel(const float* _
             v4i b[KS];
 #pragma unroll
             for (int dy = 0; dy < KS; ++dy)
-                b[dy] = *reinterpret_cast<const v4i*>(lds + ((line0 + dy) % RL) * LINE + (64 * c + 4 * n + 2 * q) * 8);
+                b[dy] = *reinterpret_cast<const v4i*>(dwf_lds + from + ((line0 + dy) % RL) * LINE + 512 * c);
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 cur[c][t] = v4i{0, 0, 0, 0};
@@ -599,9 +604,9 @@ static int dw_f32in_rows(const ConvGeom& g) {
 
 // Whether this launch is faster than a quantize pass and the int8 kernel: 3x3 on 17 columns and more, wherever it can run (0.80 of the time over 2800
 // drawn layers); narrower images, of whose rows a wave fills a part of its lanes, and 5x5, which reads four rows more for a strip, by models of the
-// two (us, launches replayed from graphs; fitted to 3670 drawn layers, half within 6 and 3 %, nine in ten within 16 and 8 %). Over 1100 other such layers
-// the rule takes 88 % and gives 0.89 of the time (the faster of both each time: 0.88), of calls one by one, which the host bounds, 0.67; 51 are over 5 %
-// slower, the worst 1.31. 32 channels 5x5 @111x111 b6 8.8 us as two; 360 5x5 @22x22 b2 6.0; 120 3x3 @13x13 b10 5.0.
+// two (us, launches replayed from graphs; fitted to 3670 drawn layers while every workgroup had four waves' LDS lines, half within 6 and 3 %, nine in ten within
+// 16 and 8 %). Of 31780 drawn layers that the rule takes one launch needs 0.80 of the time of two, the faster of both each time 0.80; 234 are over 5 % slower, the worst 1.19. Of
+// calls one by one, which the host bounds: 0.67. 360 channels 5x5 @22x22 b2 6.0 us as two; 120 3x3 @13x13 b10 5.0.
 bool dw_f32in_faster(const ConvGeom& g, int out_bytes) {
     if (g.kh == 3 && g.W >= 17) return true;
     const int rps = dw_f32in_rows(g), NL = (g.W + 31) / 32, T = g.sh == 1 ? 2 : 1;
@@ -625,21 +630,21 @@ hipError_t run_conv_dw_f32in(const float* x, const int8_t* wa, void* out, const 
     const float in_half = in_round_mode == OTTER_HIP_ROUND_SSE ? 0.5f : 0.49999997f;
     // A grid of a few workgroups per CU is resident all at once, and the dispatcher is free to give one CU three of them
     // and another one: the kernel then lasts as long as the fullest CU. Reserving a share of the CU's 160 KB of LDS per
-    // workgroup (beyond the 17 KB of lines the kernel uses, 35 with a 5x5 window) caps the workgroups per CU at the even share.
+    // workgroup (beyond its waves' lines) caps the workgroups per CU at the even share.
+    // (The lines are those of the waves that there are: with four waves' for every workgroup, 35 KB with a 5x5 window, a CU held four of the one-wave
+    // workgroups of an odd number of strips, and more than 1024 of them were two rounds: 120 channels 5x5 @80x80 b4 11.4 -> 8.5 us, as two launches 9.6)
     const long wgs = (long)grid.x * grid.y, per_cu = (wgs + 255) / 256;
-    unsigned lds_reserve = 0;
-    const unsigned lines = (g.kh == 3 ? 18 : 36) * 1024;
-    if (wpb == 4 && per_cu >= 2 && per_cu <= 3) lds_reserve = (unsigned)(160 * 1024 / per_cu - lines) / 1024 * 1024;
-    if (lds_reserve > 64 * 1024 - lines) lds_reserve = 64 * 1024 - lines;  // static + dynamic stay within the default 64 KB limit
+    unsigned lds = (unsigned)(wpb * dwf_lines(g.kh) * dwf_line_bytes((g.W + 31) / 32));
+    if (wpb == 4 && per_cu >= 2 && per_cu <= 3) lds = std::max(lds, std::min(63u * 1024, (unsigned)(160 * 1024 / per_cu - 1024) / 1024 * 1024));  // (within the default 64 KB limit)
     const unsigned in_bytes = (unsigned)((size_t)g.N * g.C * g.H * g.W * 4);
     const unsigned out_bytes = (unsigned)((size_t)g.N * g.K * g.OH * g.OW * (epi == EPI_F32_P4 || epi == EPI_F32_P8 ? 4 : 1));
 #define OHIP_DWF_L(S_, E_, L_)                                                                                           \
     do {                                                                                                                 \
         if (g.kh == 3)                                                                                                   \
-            launch((conv_dw3x3_f32in_kernel<S_, E_, L_, 3>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
+            launch((conv_dw3x3_f32in_kernel<S_, E_, L_, 3>), grid, block, lds, stream, x, wa, out, g, ep, in_scale, in_half, \
                    DwGrid::of(grid.x, grid.y, (unsigned)C8, wpb), n_strips, rps, in_bytes, out_bytes);                   \
         else                                                                                                             \
-            launch((conv_dw3x3_f32in_kernel<S_, E_, L_, 5>), grid, block, lds_reserve, stream, x, wa, out, g, ep, in_scale, in_half, \
+            launch((conv_dw3x3_f32in_kernel<S_, E_, L_, 5>), grid, block, lds, stream, x, wa, out, g, ep, in_scale, in_half, \
                    DwGrid::of(grid.x, grid.y, (unsigned)C8, wpb), n_strips, rps, in_bytes, out_bytes);                   \
     } while (0)
 #define OHIP_DWF_N(S_, E_)                       \
