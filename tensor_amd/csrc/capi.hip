@@ -838,7 +838,9 @@ static AltKernel alt_kernel(const otter_hip_conv* h, const ConvGeom& g, const Ep
 // 256 -> 512 @28x28 b32 17.0 / 18.3 and 96 -> 576 @14x14 b4 5.1 / 7.4. The two launches' model is fitted to 4700 drawn layers replayed from graphs (half within
 // 3 %, nine in ten within 8 %), against the family's own, which is a third too kind to the implicit-GEMM launch. Over 1060 others of that family
 // the rule takes 16 % and gives 0.964 of all layers' time (the faster of both each time: 0.954), 15 over 3 % slower, the worst 1.30; over 200 of the
-// other 0.98 (0.966) and none. Without room for the int8 blob it is one launch.
+// other 0.98 (0.966) and none. Of 24871 layers that it takes, behind a copy that leaves L2 cold, two launches need 0.76 of the time of one (the faster of both each time
+// 0.754); 2060 are over 5 % slower, the worst 1.39, 1628 of them below eight million values: the one launch's time there hangs on its tiles in a way that models by
+// tile do not foresee either (fitted to these layers they leave 642 of 842). Without room for the int8 blob it is one launch.
 static bool pw_quantized_apart(const otter_hip_conv* h, const ConvGeom& g, const Epilogue& ep, int family) {
     if (h->force_tm != 0 || !h->so_same || !conv_pw_reg_applicable(g, ep)) return false;
     const float px = (float)g.N * g.H * g.W * 1e-6f, C = (float)g.C, K = (float)g.K;
